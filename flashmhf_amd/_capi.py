@@ -1,17 +1,19 @@
-"""ctypes binding of libmhffn_hip.so (declared in include/mhffn.h).
+"""Bindings of libmhffn_hip.so (declared in include/mhffn.h): ``lib()`` is the C ABI through ctypes, for benchmarks and
+tests that hand over raw pointers; ``native()`` is the extension module the torch operators call.
 
-torch only supplies device memory and the current stream: tensors are passed as raw device pointers, the
-stream as ``torch.cuda.current_stream().cuda_stream`` -- the same launch discipline as the reference's
+torch only supplies device memory and the current stream -- the same launch discipline as the reference's
 launcher (kernels/thunderkittens/flash_ffn_moe.cu:991).  There is no CPU fallback: if the library has not
 been built, loading raises and every operator that needs it fails loudly.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "libmhffn_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "_lib", "_native.so")
 
 DTYPE_BF16, DTYPE_F32 = 0, 1
 OK = 0
@@ -65,6 +67,22 @@ def lib():
         L.mhffn_gate_bwd.argtypes = [vp, vp, ctypes.c_float, vp, vp, ctypes.c_int, vp, vp, vp, vp, dp, vp]
         _lib = L
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The torch side of the operators (csrc/mhffn_torch.cpp), loaded once.  Raises ImportError when it is missing."""
+    global _native
+    if _native is None:
+        if not os.path.exists(NATIVE_PATH):
+            raise ImportError(f"{NATIVE_PATH} not found: build it with `python -m flashmhf_amd.build`. "
+                              "flashmhf_amd has no CPU or eager fallback.")
+        spec = importlib.util.spec_from_file_location("flashmhf_amd._lib._native", NATIVE_PATH)
+        _native = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_native)
+    return _native
 
 
 def strerror(code):

@@ -1,8 +1,9 @@
-"""Builds libmhffn_hip.so (the C-ABI library) in-tree with hipcc for gfx950.
+"""Builds libmhffn_hip.so (the C-ABI library) in-tree with hipcc for gfx950, and the torch extension module over it.
 
     python -m flashmhf_amd.build
 
-One code object, one architecture; no CUDA headers, no torch headers, links only libamdhip64.
+One code object, one architecture; no CUDA headers, no torch headers, links only libamdhip64.  Beside it _native.so, the torch
+operators' host side on top of that C ABI (g++, torch's headers).
 """
 import os
 import subprocess
@@ -14,6 +15,9 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(LIBDIR, "libmhffn_hip.so")
 SOURCES = ["mhffn_capi.hip", "mhffn_fwd.hip", "mhffn_bwd.hip", "mhffn_f32.hip", "mhffn_gate.hip"]
+# the torch side: an extension module on top of the C ABI, plain C++
+NATIVE_LIB = os.path.join(LIBDIR, "_native.so")
+NATIVE_SOURCE = "mhffn_torch.cpp"
 # benchmark-only object: a register-resident matrix-instruction loop bench.py times beside the kernels
 PROBE_LIB = os.path.join(LIBDIR, "libmhffn_probe.so")
 PROBE_SOURCE = "mhffn_probe.hip"
@@ -56,11 +60,26 @@ def build_lib(verbose=False, jobs=4):
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)
+    subprocess.check_call(native_command())
     with open(os.path.join(LIBDIR, "resource_usage.txt"), "w") as f:     # registers, scratch, occupancy per kernel
         for name in sorted(usage):
             f.write(name + "  " + "  ".join(f"{k}={v}" for k, v in usage[name].items()) + "\n")
     check_no_scratch(usage)
     return LIB
+
+
+def native_command():
+    """g++ line of the extension module: torch's headers and libraries, libmhffn_hip.so beside it."""
+    import sysconfig
+    import torch
+    t = os.path.dirname(torch.__file__)
+    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-attributes",
+            *(f"-isystem{i}" for i in inc), os.path.join(CSRC, NATIVE_SOURCE), "-o", NATIVE_LIB,
+            "-L" + LIBDIR, "-lmhffn_hip", "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+            "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
 
 
 def parse_resource_usage(stderr_text):

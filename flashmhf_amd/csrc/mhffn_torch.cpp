@@ -1,0 +1,364 @@
+// Host side of the operator for torch tensors: checks, output and workspace tensors, launches through the C ABI of
+// libmhffn_hip.so, and the autograd nodes.  The same steps written in Python (two autograd.Function nodes, ctypes calls, a
+// dozen attribute look-ups) take 20 us per forward and 100 us per forward + backward of the operator on the host, several
+// times what the kernels of a short sequence take on the GPU.
+//
+// What each function computes and returns is described in flash_mlp_moe.py, head_gate.py and mhffn_layer.py, which call
+// these.  Errors carry the exception types of the reference: TypeError for dtypes, ValueError for the expert and head
+// dims, RuntimeError otherwise (kernels/triton/flash_mlp_moe.py:758-766, kernels/thunderkittens/flash_ffn_moe.cu:943-958).
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/utils/pybind.h>
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include "../../include/mhffn.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+void raise_for_code(int code, const char* what)
+{
+    if (code == MHFFN_OK) return;
+    const char* text = mhffn_strerror(code);
+    TORCH_CHECK_TYPE(code != MHFFN_ERR_DTYPE, what, ": ", text, " (code ", code, ")");
+    TORCH_CHECK_VALUE(code != MHFFN_ERR_EXPERT_DIM && code != MHFFN_ERR_HEAD_DIM, what, ": ", text, " (code ", code, ")");
+    TORCH_CHECK(false, what, ": ", text, " (code ", code, ")");
+}
+
+int dtype_code(at::ScalarType t)
+{
+    return t == at::kBFloat16 ? MHFFN_DTYPE_BF16 : t == at::kFloat ? MHFFN_DTYPE_F32 : -1;
+}
+
+// Workspace bytes of a shape, remembered per thread: the slots of a direct-mapped table.
+struct Plan {
+    mhffn_dims dims;
+    int dtype;
+    size_t fwd_bytes, bwd_bytes;
+};
+const Plan& plan_for(const mhffn_dims& d, int dtype)
+{
+    static thread_local Plan table[64] = {};
+    unsigned h = (unsigned)d.S * 2654435761u ^ (unsigned)d.B * 40503u ^ (unsigned)d.d_e * 97u ^ (unsigned)d.E * 31u ^
+                 (unsigned)d.H * 7u ^ (unsigned)d.Hkuv * 3u ^ (unsigned)d.d_h ^ (unsigned)dtype;
+    Plan& p = table[(h ^ (h >> 13)) & 63];
+    if (memcmp(&p.dims, &d, sizeof d) != 0 || p.dtype != dtype) {
+        raise_for_code(mhffn_check_dims(&d, dtype), "mhffn");
+        p = Plan{d, dtype, mhffn_fwd_workspace_bytes(&d, dtype), mhffn_bwd_workspace_bytes(&d, dtype)};
+    }
+    return p;
+}
+
+// The library launches on the current device: a guard only where the tensors live on another one.
+struct OnDevice {
+    c10::OptionalDeviceGuard guard;
+    explicit OnDevice(const Tensor& t)
+    {
+        if (t.device().index() != c10::hip::current_device()) guard.reset_device(t.device());
+    }
+};
+void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+Tensor empty_like_layout(const Tensor& t) { return at::detail::empty_strided_cuda(t.sizes(), t.strides(), t.scalar_type(), t.device()); }
+Tensor empty_of(at::IntArrayRef sizes, at::ScalarType dtype, const Tensor& on)
+{
+    return at::detail::empty_cuda(sizes, dtype, on.device(), std::nullopt);
+}
+Tensor scratch(size_t bytes, const Tensor& on)
+{
+    return bytes ? empty_of({(int64_t)bytes}, at::kByte, on) : Tensor();
+}
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+bool token_major(const Tensor& t)      // [B, H, S, d] seen through the transposed view of a contiguous [B, S, H, d]
+{
+    const auto s = t.strides(), n = t.sizes();
+    return (s[3] == 1 || n[3] == 1) && (s[1] == n[3] || n[1] == 1) && (s[2] == n[1] * n[3] || n[2] == 1) &&
+           (s[0] == n[2] * n[1] * n[3] || n[0] == 1);
+}
+
+void check_inputs(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R)
+{
+    TORCH_CHECK(Q.dim() == 4 && K.dim() == 4 && R.dim() == 4, "expected Q [B,H,S,d_h], K/U/V [Hkuv,E,d_e,d_h], R [B,H,S,E]");
+    const auto dt = Q.scalar_type();
+    TORCH_CHECK_TYPE((dt == at::kBFloat16 || dt == at::kFloat) && K.scalar_type() == dt && V.scalar_type() == dt && U.scalar_type() == dt,
+                     "FlashMLPFunction expects all inputs in torch.bfloat16 (or all in torch.float32), got Q=", dt, ", K=",
+                     K.scalar_type(), ", V=", V.scalar_type(), ", U=", U.scalar_type());
+    TORCH_CHECK_TYPE(R.scalar_type() == at::kFloat, "R must be float32 (the router gate is computed in fp32), got ", R.scalar_type());
+    TORCH_CHECK(U.sizes() == K.sizes() && V.sizes() == K.sizes(), "K, U, V must share one shape, got ", K.sizes(), ", ", U.sizes(),
+                ", ", V.sizes());
+    TORCH_CHECK(R.size(0) == Q.size(0) && R.size(1) == Q.size(1) && R.size(2) == Q.size(2) && R.size(3) == K.size(1),
+                "R must be [B,H,S,E] = [", Q.size(0), ", ", Q.size(1), ", ", Q.size(2), ", ", K.size(1), "], got ", R.sizes());
+    TORCH_CHECK_VALUE(dt != at::kBFloat16 || K.size(2) % 32 == 0, "Expert dimension ", K.size(2), " must be divisible by 32");
+    TORCH_CHECK(Q.is_cuda(), "flashmhf_amd runs on the GPU only; there is no CPU path");
+    for (const Tensor* t : {&K, &U, &V, &R})
+        TORCH_CHECK(t->device() == Q.device(), "K, U, V and R must be on the device of Q, ", Q.device(), "; one is on ", t->device());
+    TORCH_CHECK(Q.size(3) == K.size(3), "head dim mismatch: Q has ", Q.size(3), ", K has ", K.size(3));
+}
+
+mhffn_dims dims_of(const Tensor& Q, const Tensor& K)
+{
+    return mhffn_dims{(int)Q.size(0), (int)Q.size(1), (int)K.size(0), (int)Q.size(2), (int)Q.size(3), (int)K.size(1), (int)K.size(2)};
+}
+
+// (the tensor to pass, its layout): [B,H,S,d_h] contiguous, or the transposed view of a contiguous [B,S,H,d_h]
+std::pair<Tensor, int> laid_out(const Tensor& Q)
+{
+    if (Q.is_contiguous()) return {Q, MHFFN_TOKENS_BHSD};
+    if (token_major(Q)) return {Q, MHFFN_TOKENS_BSHD};
+    return {Q.contiguous(), MHFFN_TOKENS_BHSD};
+}
+Tensor as_layout(const Tensor& t, int layout)
+{
+    if (layout == MHFFN_TOKENS_BHSD) return t.contiguous();
+    return token_major(t) ? t : t.transpose(1, 2).contiguous().transpose(1, 2);
+}
+Tensor contig(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+
+Tensor op_forward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, const Tensor& V0, const Tensor& R0)
+{
+    check_inputs(Q0, K0, U0, V0, R0);
+    auto [Q, layout] = laid_out(Q0);
+    const Tensor K = contig(K0), U = contig(U0), V = contig(V0), R = contig(R0);
+    const int dt = dtype_code(Q.scalar_type());
+    const Plan& p = plan_for(dims_of(Q, K), dt);
+    OnDevice guard(Q);
+    Tensor O = empty_like_layout(Q), ws = scratch(p.fwd_bytes, Q);
+    raise_for_code(mhffn_fwd_layout(ptr(Q), ptr(K), ptr(U), ptr(V), (const float*)ptr(R), ptr(O), ptr(ws), p.fwd_bytes, &p.dims, dt,
+                                    layout, stream(), MHFFN_FWD_ALL),
+                   "mhffn_fwd");
+    return O;
+}
+
+variable_list op_backward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, const Tensor& V0, const Tensor& R0,
+                          const Tensor& dO0, at::ScalarType grad_w)
+{
+    check_inputs(Q0, K0, U0, V0, R0);
+    TORCH_CHECK(dO0.sizes() == Q0.sizes(), "grad_output shape should be the same as Q");
+    auto [Q, layout] = laid_out(Q0);
+    const Tensor K = contig(K0), U = contig(U0), V = contig(V0), R = contig(R0);
+    const Tensor dO = as_layout(dO0.scalar_type() == Q.scalar_type() ? dO0 : dO0.to(Q.scalar_type()), layout);
+    const int dt = dtype_code(Q.scalar_type()), wdt = dtype_code(grad_w);
+    const Plan& p = plan_for(dims_of(Q, K), dt);
+    OnDevice guard(Q);
+    Tensor dQ = empty_like_layout(Q), dR = empty_of(R.sizes(), at::kFloat, Q), ws = scratch(p.bwd_bytes, Q);
+    Tensor dK = empty_of(K.sizes(), grad_w, Q), dU = empty_of(K.sizes(), grad_w, Q), dV = empty_of(K.sizes(), grad_w, Q);
+    raise_for_code(mhffn_bwd_layout(ptr(Q), ptr(K), ptr(U), ptr(V), (const float*)ptr(R), ptr(dO), ptr(dQ), ptr(dK), ptr(dU), ptr(dV),
+                                    (float*)ptr(dR), wdt, ptr(ws), p.bwd_bytes, &p.dims, dt, layout, stream(), MHFFN_BWD_ALL),
+                   "mhffn_bwd");
+    return {dQ, dK, dU, dV, dR};
+}
+
+bool records_grad(std::initializer_list<const Tensor*> ts)
+{
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor* t : ts)
+        if (t->defined() && t->requires_grad()) return true;
+    return false;
+}
+
+// O = fused(Q, K, U, V, R).  f32_grads: dQ, dK, dU, dV in float32 whatever the inputs are (the ThunderKittens wrapper's
+// convention, kernels/thunderkittens/flash_ffn_moe_torch.py:17-21); otherwise in the inputs' dtypes.
+struct OpNode : torch::autograd::Function<OpNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R,
+                          bool f32_grads)
+    {
+        ctx->save_for_backward({Q, K, U, V, R});
+        ctx->saved_data["f32"] = f32_grads;
+        return op_forward(Q, K, U, V, R);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        const bool f32 = ctx->saved_data["f32"].toBool();
+        auto out = op_backward(s[0], s[1], s[2], s[3], s[4], g[0], f32 ? at::kFloat : s[1].scalar_type());
+        if (f32) out[0] = out[0].to(at::kFloat);
+        out.emplace_back();
+        return out;
+    }
+};
+Tensor op(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, bool f32_grads)
+{
+    if (!records_grad({&Q, &K, &U, &V, &R})) return op_forward(Q, K, U, V, R);
+    return OpNode::apply(Q, K, U, V, R, f32_grads);
+}
+
+// The single-expert operator: Q [B,H,S,d_h], K/U/V [Hkuv, rows, d_h], gate 1.
+Tensor ones_gate(const Tensor& Q) { return at::ones({Q.size(0), Q.size(1), Q.size(2), 1}, Q.options().dtype(at::kFloat)); }
+struct SingleNode : torch::autograd::Function<SingleNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V)
+    {
+        const Tensor R = ones_gate(Q);
+        ctx->save_for_backward({Q, K, U, V, R});
+        return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), R);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        auto out = op_backward(s[0], s[1].unsqueeze(1), s[2].unsqueeze(1), s[3].unsqueeze(1), s[4], g[0], s[1].scalar_type());
+        return {out[0], out[1].squeeze(1), out[2].squeeze(1), out[3].squeeze(1)};
+    }
+};
+Tensor single(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V)
+{
+    if (!records_grad({&Q, &K, &U, &V})) return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones_gate(Q));
+    return SingleNode::apply(Q, K, U, V);
+}
+
+// ---- head prologue -------------------------------------------------------------------------------------------------
+mhffn_dims gate_dims(const Tensor& x4, const Tensor& wn, const Tensor& router)
+{
+    TORCH_CHECK(x4.dim() == 4 && router.dim() == 3, "expected x [B,S,H,d_h] and router [H,d_h,E]");
+    TORCH_CHECK_TYPE(x4.scalar_type() == at::kBFloat16, "head_norm_gate expects bfloat16 heads, got ", x4.scalar_type());
+    const auto n = x4.sizes();
+    TORCH_CHECK(router.size(0) == n[2] && router.size(1) == n[3], "router must be [H,d_h,E] = [", n[2], ",", n[3], ",E], got ",
+                router.sizes());
+    TORCH_CHECK(!wn.defined() || (wn.dim() == 2 && wn.size(0) == n[2] && wn.size(1) == n[3]), "norm_weight must be [H,d_h] = [", n[2],
+                ",", n[3], "], got ", wn.defined() ? wn.sizes() : at::IntArrayRef());
+    TORCH_CHECK(x4.is_cuda(), "flashmhf_amd runs on the GPU only; there is no CPU path");
+    return mhffn_dims{(int)n[0], (int)n[2], (int)n[2], (int)n[1], (int)n[3], (int)router.size(2), 32};
+}
+
+struct GateForward {
+    Tensor x4, wn, wr, q4, R;      // contiguous x, float32 weights, normalised heads [B,S,H,d_h] (x4 without a norm), gate
+};
+GateForward gate_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& router, double eps)
+{
+    const mhffn_dims d = gate_dims(x, norm_weight, router);
+    GateForward f;
+    f.x4 = contig(x);
+    if (norm_weight.defined()) f.wn = contig(norm_weight.to(at::kFloat));
+    f.wr = contig(router.to(at::kFloat));
+    OnDevice guard(f.x4);
+    f.q4 = f.wn.defined() ? empty_of(x.sizes(), at::kBFloat16, f.x4) : f.x4;
+    f.R = empty_of({d.B, d.H, d.S, d.E}, at::kFloat, f.x4);
+    raise_for_code(mhffn_gate_fwd(ptr(f.x4), (const float*)ptr(f.wn), (float)eps, (const float*)ptr(f.wr),
+                                  f.wn.defined() ? ptr(f.q4) : nullptr, (float*)ptr(f.R), &d, stream()),
+                   "mhffn_gate_fwd");
+    return f;
+}
+// {dx, d_norm_weight, d_router}; dQ, dR may be undefined (zero)
+variable_list gate_backward(const Tensor& x4, const Tensor& norm_weight, const Tensor& router, const Tensor& wn, const Tensor& wr,
+                            double eps, Tensor dQ, Tensor dR)
+{
+    const mhffn_dims d = gate_dims(x4, norm_weight, router);
+    OnDevice guard(x4);
+    if (!dQ.defined()) dQ = at::zeros_like(x4).transpose(1, 2);
+    if (!dR.defined()) dR = at::zeros({d.B, d.H, d.S, d.E}, x4.options().dtype(at::kFloat));
+    int layout = MHFFN_TOKENS_BSHD;
+    if (!token_major(dQ)) {
+        layout = MHFFN_TOKENS_BHSD;
+        dQ = dQ.contiguous();
+    }
+    dR = contig(dR.to(at::kFloat));
+    Tensor dx = empty_of(x4.sizes(), at::kBFloat16, x4), dwn, dwr = at::zeros_like(wr);
+    if (wn.defined()) dwn = at::zeros_like(wn);
+    raise_for_code(mhffn_gate_bwd(ptr(x4), (const float*)ptr(wn), (float)eps, (const float*)ptr(wr), ptr(dQ), layout,
+                                  (const float*)ptr(dR), ptr(dx), (float*)ptr(dwn), (float*)ptr(dwr), &d, stream()),
+                   "mhffn_gate_bwd");
+    return {dx, dwn.defined() ? dwn.to(norm_weight.scalar_type()) : dwn, dwr.to(router.scalar_type())};
+}
+
+struct GateNode : torch::autograd::Function<GateNode> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const std::optional<Tensor>& norm_weight, const Tensor& router,
+                                 double eps)
+    {
+        const Tensor nw = norm_weight.value_or(Tensor());
+        GateForward f = gate_forward(x, nw, router, eps);
+        ctx->save_for_backward({f.x4, nw, router, f.wn, f.wr});
+        ctx->saved_data["eps"] = eps;
+        return {f.q4.transpose(1, 2), f.R};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        auto out = gate_backward(s[0], s[1], s[2], s[3], s[4], ctx->saved_data["eps"].toDouble(), g[0], g[1]);
+        out.emplace_back();
+        return out;
+    }
+};
+std::pair<Tensor, Tensor> gate(const Tensor& x, const std::optional<Tensor>& norm_weight, const Tensor& router, double eps)
+{
+    const Tensor nw = norm_weight.value_or(Tensor());
+    if (!records_grad({&x, &nw, &router})) {
+        GateForward f = gate_forward(x, nw, router, eps);
+        return {f.q4.transpose(1, 2), f.R};
+    }
+    auto out = GateNode::apply(x, norm_weight, router, eps);
+    return {out[0], out[1]};
+}
+
+// ---- the whole block: w_self, prologue, operator, w_self_2 ---------------------------------------------------------
+struct BlockForward {
+    GateForward g;
+    Tensor O4, Y;      // operator output [B,S,H,d_h], block output
+};
+BlockForward block_forward(const Tensor& x, const Tensor& w1, const Tensor& norm_weight, const Tensor& router, const Tensor& K,
+                           const Tensor& U, const Tensor& V, const Tensor& w2, double eps)
+{
+    BlockForward f;
+    const int64_t B = x.size(0), S = x.size(1), hid = x.size(2);
+    f.g = gate_forward(at::linear(x, w1).view({B, S, router.size(0), router.size(1)}), norm_weight, router, eps);
+    f.O4 = op_forward(f.g.q4.transpose(1, 2), K, U, V, f.g.R).transpose(1, 2);
+    f.Y = at::linear(f.O4.view({B, S, hid}), w2);
+    return f;
+}
+
+struct BlockNode : torch::autograd::Function<BlockNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight,
+                          const Tensor& router, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& w2, double eps)
+    {
+        const Tensor nw = norm_weight.value_or(Tensor());
+        BlockForward f = block_forward(x, w1, nw, router, K, U, V, w2, eps);
+        ctx->save_for_backward({x, w1, nw, router, K, U, V, w2, f.g.x4, f.g.wn, f.g.wr, f.g.q4, f.g.R, f.O4});
+        ctx->saved_data["eps"] = eps;
+        return f.Y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const auto s = ctx->get_saved_variables();
+        const Tensor &x = s[0], &w1 = s[1], &nw = s[2], &router = s[3], &K = s[4], &U = s[5], &V = s[6], &w2 = s[7], &x4 = s[8],
+                     &wn = s[9], &wr = s[10], &q4 = s[11], &R = s[12], &O4 = s[13];
+        const int64_t hid = x.size(2);
+        // (the products of a linear layer's own backward: d_in = d_out w, d_w = d_out^T in)
+        const Tensor dY = grads[0].reshape({-1, hid});
+        const Tensor dO = at::mm(dY, w2).view(O4.sizes());
+        const Tensor dw2 = at::mm(dY.t(), O4.view({-1, hid}));
+        auto g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type());
+        auto h = gate_backward(x4, nw, router, wn, wr, ctx->saved_data["eps"].toDouble(), g[0], g[4]);
+        const Tensor dp = h[0].view({-1, hid});
+        Tensor dx;
+        if (ctx->needs_input_grad(0)) dx = at::mm(dp, w1).view(x.sizes());
+        const Tensor dw1 = at::mm(dp.t(), x.reshape({-1, hid}));
+        return {dx, dw1, h[1], h[2], g[1], g[2], g[3], dw2, Tensor()};
+    }
+};
+Tensor block(const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight, const Tensor& router, const Tensor& K,
+             const Tensor& U, const Tensor& V, const Tensor& w2, double eps)
+{
+    const Tensor nw = norm_weight.value_or(Tensor());
+    if (!records_grad({&x, &w1, &nw, &router, &K, &U, &V, &w2})) return block_forward(x, w1, nw, router, K, U, V, w2, eps).Y;
+    return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_native, m)
+{
+    // (all without the interpreter lock, as a ctypes call is)
+    m.def("op_forward", torch::wrap_pybind_function_no_gil(op_forward));
+    m.def("op_backward", torch::wrap_pybind_function_no_gil(
+                             [](const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, const Tensor& dO,
+                                bool f32_grad_w) { return op_backward(Q, K, U, V, R, dO, f32_grad_w ? at::kFloat : at::kBFloat16); }));
+    m.def("op", torch::wrap_pybind_function_no_gil(op));
+    m.def("single", torch::wrap_pybind_function_no_gil(single));
+    m.def("gate", torch::wrap_pybind_function_no_gil(gate));
+    m.def("block", torch::wrap_pybind_function_no_gil(block));
+}

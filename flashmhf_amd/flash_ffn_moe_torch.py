@@ -5,6 +5,7 @@ needed here: the HIP kernels read R as [B,H,S,E].
 """
 import torch
 
+from . import _capi
 from .flash_mlp_moe import mhffn_backward, mhffn_forward
 
 
@@ -27,4 +28,4 @@ class FlashFFNMoE(torch.nn.Module):
         super().__init__()
 
     def forward(self, Q, K, U, V, R):
-        return FlashFFNMoEFunction.apply(Q, K, U, V, R)
+        return _capi.native().op(Q, K, U, V, R, True)

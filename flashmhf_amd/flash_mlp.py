@@ -9,7 +9,7 @@ It is the E = 1, R = 1 case of the fused MoE operator (which is what runs), with
 """
 import torch
 
-from .flash_mlp_moe import FlashMLPFunction
+from . import _capi
 
 
 class FlashMLP(torch.nn.Module):
@@ -25,5 +25,4 @@ class FlashMLP(torch.nn.Module):
             raise ValueError("FlashMLP SiLU variant requires up-projection tensor U (got None)")
         if K.dim() != 3:
             raise RuntimeError("expected K/U/V [Hkuv, intermediate, d_h]")
-        ones = torch.ones(*Q.shape[:3], 1, dtype=torch.float32, device=Q.device)
-        return FlashMLPFunction.apply(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones)
+        return _capi.native().single(Q, K, U, V)

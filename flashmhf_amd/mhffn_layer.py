@@ -33,6 +33,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _capi
 from .flash_mlp_moe import FlashMLPMoE
 from .head_gate import head_norm_gate
 
@@ -62,6 +63,15 @@ def router_gate(logits):
     """sigmoid, then divide by the sum over experts clamped at 1e-20 (modeling_mhffnmoe.py:384-386); fp32 in and out."""
     R = logits.sigmoid()
     return R / R.sum(dim=-1, keepdim=True).clamp(min=1e-20)
+
+
+def _unhooked(m):
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
+def _global_hooks():
+    g = nn.modules.module
+    return g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks
 
 
 class MHFFNLayer(nn.Module):
@@ -129,8 +139,25 @@ class MHFFNLayer(nn.Module):
             logits = (x.float() @ self.w_router.float()).view(B, S, H, E).transpose(1, 2)
         return Q, router_gate(logits).contiguous()
 
+    def _one_node(self, x):
+        """Whether the block can run as one native node (projection, prologue, operator, projection: the same kernels and
+        library products as the steps below, a quarter of the host time): bfloat16 on the GPU with the default operator
+        and plain bias-free projections that no hook, subclass or autocast context would have a say in.  (More than 32
+        experts take the prologue's two-tile instances, which heads_and_gate chooses among.)"""
+        m = self._modules
+        return (self.router_input == "q" and self.fused_prologue and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 3
+                and self.num_experts <= 32 and self.head_dim in (64, 96, 128) and type(m["op"]) is FlashMLPMoE
+                and all(type(w) is nn.Linear and w.bias is None and _unhooked(w) for w in (m["w_self"], m["w_self_2"]))
+                and ("q_norm" not in m or type(m["q_norm"]) is RMSNorm and _unhooked(m["q_norm"])) and _unhooked(m["op"])
+                and not torch.is_autocast_enabled("cuda") and not _global_hooks()
+                and self.w_self.weight.dtype == self.w_self_2.weight.dtype == self.K.dtype == self.U.dtype == self.V.dtype
+                == torch.bfloat16)
+
     def forward(self, x):
         B, S, hid = x.shape
+        if self._one_node(x):
+            return _capi.native().block(x, self.w_self.weight, None if self.q_norm is None else self.q_norm.weight, self.router,
+                                        self.K, self.U, self.V, self.w_self_2.weight, self.rms_norm_eps)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
