@@ -53,14 +53,17 @@ def build_lib(verbose=False, jobs=4):
         usage.update(parse_resource_usage(r.stderr))
         return obj
 
+    native_obj = os.path.join(objdir, NATIVE_SOURCE.replace(".cpp", ".o"))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        native = ex.submit(subprocess.check_call, native_compile(native_obj))
         objs = list(ex.map(compile_one, SOURCES + [PROBE_SOURCE]))
+        native.result()
     for out, members in ((LIB, objs[:-1]), (PROBE_LIB, objs[-1:])):
         cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *members]
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)
-    subprocess.check_call(native_command())
+    subprocess.check_call(native_link(native_obj))
     with open(os.path.join(LIBDIR, "resource_usage.txt"), "w") as f:     # registers, scratch, occupancy per kernel
         for name in sorted(usage):
             f.write(name + "  " + "  ".join(f"{k}={v}" for k, v in usage[name].items()) + "\n")
@@ -68,18 +71,23 @@ def build_lib(verbose=False, jobs=4):
     return LIB
 
 
-def native_command():
-    """g++ line of the extension module: torch's headers and libraries, libmhffn_hip.so beside it."""
+def native_compile(obj):
+    """g++ line of the extension module's one source: torch's, Python's and HIP's headers."""
     import sysconfig
     import torch
-    t = os.path.dirname(torch.__file__)
-    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
-           sysconfig.get_paths()["include"]]
-    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    t = os.path.join(os.path.dirname(torch.__file__), "include")
+    inc = [t, os.path.join(t, "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-attributes",
-            *(f"-isystem{i}" for i in inc), os.path.join(CSRC, NATIVE_SOURCE), "-o", NATIVE_LIB,
-            "-L" + LIBDIR, "-lmhffn_hip", "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
-            "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+            *(f"-isystem{i}" for i in inc), "-c", os.path.join(CSRC, NATIVE_SOURCE), "-o", obj]
+
+
+def native_link(obj):
+    """... and of its link: torch's libraries, libmhffn_hip.so beside it."""
+    import torch
+    t = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return [os.environ.get("CXX", "g++"), "-shared", obj, "-o", NATIVE_LIB, "-L" + LIBDIR, "-lmhffn_hip", "-L" + t, "-lc10",
+            "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
 
 
 def parse_resource_usage(stderr_text):

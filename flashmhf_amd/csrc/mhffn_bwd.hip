@@ -1,6 +1,7 @@
 // Fused multi-head FFN backward for gfx950 (bf16 MFMA, fp32 accumulation), two kernels:
 //
-//  (1) dQ/dR kernel -- a workgroup of 8 waves (two per SIMD) owns 256 tokens of one (batch, q-head), 32 per wave, and
+//  (1) dQ/dR kernel -- a workgroup of 8 waves (two per SIMD) owns 256 rows of one K/U/V head (tokens of any batch and
+//      q-head of its group: RowMap), 32 per wave, and all the head's blocks or one part of them (pick_nsplit); it
 //      streams the K, U, V blocks (32 rows at a time) through a ring of LDS stages with LDS-direct loads.  Per block:
 //          M^T = K Q^T, N^T = U Q^T, dA^T = V dO^T            (recomputed, registers only)
 //          dR_e += sum_j dA * silu(M) * N                      (fp32, before any rounding)
@@ -30,8 +31,9 @@ struct DqArgs {
     const float* R;
     bf16_t* dQ;
     float* dR;
-    int H, G, S, E, nbe;
-    int tokmaj;   // Q, dO, dQ token-major ([B, S, H, d_h]) instead of [B, H, S, d_h]
+    float* part;          // [nsplit][Hkuv][rows.n][DH] dQ, then [nsplit][Hkuv][rows.n][E] dR: fp32 partial sums
+    RowMap rows;          // rows of Q, dO, dQ, R, dR that meet one K/U/V head
+    Parts parts;          // ... and the blocks of that head
 };
 
 constexpr int DQ_NST = 4;                  // LDS stages (K | U | V tiles each)
@@ -48,13 +50,14 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x, tb = blockIdx.y, b = blockIdx.z;
-    const int hk = h / p.G;
-    const long rowbase = ((long)b * p.H + h) * p.S;          // rows of R, dR
-    const TokRows qrows = tok_rows(p.tokmaj, b, h, p.H, p.S);   // rows of Q, dO, dQ
-    const int tok0 = tb * BT + wave * 32;
-    const int nblk = p.E * p.nbe;
-    const bf16_t* Kh = p.K + (long)hk * nblk * JB * DH;
+    // blockIdx.x = tile * Hkuv + kv-head: the head index runs fastest, so each head's weights stay in one XCD's L2
+    const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    const int tok0 = tile * BT + wave * 32;                  // this wave's rows of the list (RowMap)
+    const int nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;   // blocks of this workgroup, counted from blk0
+    const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;        // expert of the first, its place in the expert
+    const int nex = p.parts.by_nbe.div(jb0 + nblk + nbe - 1);                // experts they belong to, counted from ex0
+    const bf16_t* Kh = p.K + ((long)hk * E * nbe + blk0) * JB * DH;
     const long offU = p.U - p.K, offV = p.V - p.K;
 
     auto issue_block = [&](int blk) {
@@ -69,13 +72,16 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
             tile_fill_ins<DH>(Kh + toff + roff, DH, st + which * TILE_B, id & 7, lane);
         }
     };
+    const int first = tok0 < p.rows.n ? tok0 : p.rows.n - 1;
+    const RowMap::Run run = p.rows.run(hk, first, 32);
     // The Q and dO rows come from HBM and are the longest wait of the prologue: request them before anything else.
     bf16x8 q[KS], go[KS];
     {
         int t = tok0 + l32;
-        t = t < p.S ? t : p.S - 1;
-        const bf16_t* qr = p.Q + (qrows.base + (long)t * qrows.stride) * DH + 8 * g;
-        const bf16_t* gr = p.dO + (qrows.base + (long)t * qrows.stride) * DH + 8 * g;
+        t = t < p.rows.n ? t : p.rows.n - 1;
+        const long row = p.rows.tok(run, hk, first, t) * DH + 8 * g;
+        const bf16_t* qr = p.Q + row;
+        const bf16_t* gr = p.dO + row;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             q[ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16);
@@ -89,12 +95,12 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
     // them too, and a layer with more experts refills the slots 32 at a time as the block loop leaves them behind.
     const float* rrow;
     {
-        int t = tb * BT + (wave >> 1) * 64 + lane;
-        t = t < p.S ? t : p.S - 1;
-        rrow = p.R + (rowbase + t) * p.E;
+        int t = tile * BT + (wave >> 1) * 64 + lane;
+        t = t < p.rows.n ? t : p.rows.n - 1;
+        rrow = p.R + p.rows.gate(hk, t) * E + ex0;
     }
     auto stage_gates = [&](int e0, int e1) {
-        e1 = e1 < p.E ? e1 : p.E;
+        e1 = e1 < nex ? e1 : nex;
         for (int e = e0 + (wave & 1); e < e1; e += 2)
             __builtin_amdgcn_global_load_lds((gptr_t)(rrow + e), (lptr_t)(sR + (e & 63) * BT + (wave >> 1) * 64), 4, 0, 0);
     };
@@ -193,15 +199,22 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    int e = 0, jb = 0;          // expert and block-in-expert of the block whose element-wise work comes next
+    // where this lane's dR values go: the row of dR itself, or of this part's sums
+    float* drow;
+    {
+        const int t = tok0 + l32 < p.rows.n ? tok0 + l32 : p.rows.n - 1;
+        const long hrows = (long)p.rows.Hkuv * p.rows.n;
+        drow = nsplit == 1 ? p.dR + p.rows.gate(run, hk, first, t) * E
+                           : p.part + nsplit * hrows * DH + (z * hrows + (long)hk * p.rows.n + t) * E + ex0;
+    }
+    int e = 0, jb = jb0;        // expert and block-in-expert of the block whose element-wise work comes next
     auto finish_block = [&](int blk) {
         element_wise(sR[(e & 63) * BT + wave * 32 + l32]);
         second_products(blk);
-        if (++jb == p.nbe) {
+        if (++jb == nbe || blk == nblk - 1) {
             // dR[t, e]: the two lane halves hold disjoint j rows of the same token column.
             const float tot = dr + __shfl_xor(dr, 32);
-            const int t = tok0 + l32;
-            if (g == 0 && t < p.S) p.dR[(rowbase + t) * p.E + e] = tot;
+            if (g == 0 && tok0 + l32 < p.rows.n) drow[e] = tot;
             dr = 0.0f;
             jb = 0;
             ++e;
@@ -209,7 +222,7 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
             // 32k-32 .. 32k-1 with experts 32k+32 .. 32k+63 of its own 64 tokens.  Its partner is in the same interval
             // between two barriers, so at a block of expert 32k or later; the values are first read 31 experts on, and
             // every barrier's wait on the way leaves at most three of this wave's loads outstanding.
-            if (e > 1 && (e & 31) == 1 && e + 31 < p.E) stage_gates(e + 31, e + 63);
+            if (e > 1 && (e & 31) == 1 && e + 31 < nex) stage_gates(e + 31, e + 63);
         }
     };
     // Barrier b: block b has landed for every wave, and every wave is done with block b - 2, whose stage the fill of
@@ -242,6 +255,11 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
     wait_vmcnt<0>();   // drain the phantom prefetches: they write the ring, which the epilogue reuses
     __syncthreads();   // every wave is done reading the ring
 
+    if (nsplit > 1) {     // a part of the blocks leaves its sums as they are, fp32, for the pass that adds the parts
+        store_rows_f32<DH>(smem + wave * TILE_B, p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH,
+                           p.rows.n - tok0, lane, [&](auto ic) -> const f32x16& { return dq[decltype(ic)::value]; });
+        return;
+    }
     // dQ^T registers -> dQ[t][c] through a private 8 KB region of the ring per wave (rows of 256 bytes, 16-byte chunk c16
     // of row r at chunk c16 ^ (r & 15)), so that the stores are whole rows (16 lanes x 16 bytes, 4 rows per instruction)
     // instead of 8-byte pieces scattered over 32 rows.  Register 4a+x of row tile i is c = 32i + 8a + 4g + x.
@@ -257,15 +275,54 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
                 *reinterpret_cast<bf16x4*>(otile + l32 * TILE_ROW_B + (((4 * i + a) ^ (l32 & 15)) << 4) + 8 * g) = v;
             }
         const int c16 = lane & 15;
+        auto store = [&](auto&& address_row) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int row = 4 * k + (lane >> 4);
-            const int t = tok0 + row;
-            if (c16 < DH / 8 && t < p.S) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(otile + row * TILE_ROW_B + ((c16 ^ (row & 15)) << 4));
-                *reinterpret_cast<u32x4*>(p.dQ + (qrows.base + (long)t * qrows.stride) * DH + c16 * 8) = v;
+            for (int k = 0; k < 8; ++k) {
+                const int row = 4 * k + (lane >> 4);
+                if (c16 < DH / 8 && tok0 + row < p.rows.n) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(otile + row * TILE_ROW_B + ((c16 ^ (row & 15)) << 4));
+                    *reinterpret_cast<u32x4*>(p.dQ + address_row(row) * DH + c16 * 8) = v;
+                }
             }
+        };
+        if (run.tok.stride) store([&](int row) { return run.tok.base + (long)row * run.tok.stride; });
+        else store([&](int row) { return p.rows.tok(hk, tok0 + row); });
+    }
+}
+
+// Adds the parts' sums of dQ (in the order of the parts) and rounds once, eight columns per lane; adds the sums of dR over the
+// parts that hold blocks of the expert, one value per lane.  blockIdx.x < dq_blocks: dQ, otherwise dR.
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsigned dq_blocks)
+{
+    const int hk = blockIdx.y;
+    const long hrows = (long)p.rows.Hkuv * p.rows.n;
+    if (blockIdx.x < dq_blocks) {
+        const unsigned i = blockIdx.x * 256 + threadIdx.x;
+        const unsigned r = i / (DH / 8), c = (i % (DH / 8)) * 8;
+        if (r >= (unsigned)p.rows.n) return;
+        const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
+        f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+        for (int z = 1; z < p.parts.nsplit; ++z) {
+            src += hrows * DH;
+            lo += *reinterpret_cast<const f32x4*>(src);
+            hi += *reinterpret_cast<const f32x4*>(src + 4);
         }
+        bf16x8 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) { v[x] = (bf16_t)lo[x]; v[4 + x] = (bf16_t)hi[x]; }
+        *reinterpret_cast<bf16x8*>(p.dQ + p.rows.tok(hk, r) * DH + c) = v;
+    } else {
+        const unsigned i = (blockIdx.x - dq_blocks) * 256 + threadIdx.x;
+        const int E = p.parts.E, nbe = p.parts.nbe;
+        const unsigned r = i / (unsigned)E;
+        const int e = i - r * E;
+        if (r >= (unsigned)p.rows.n) return;
+        const float* src = p.part + p.parts.nsplit * hrows * DH + ((long)hk * p.rows.n + r) * E + e;
+        float sum = 0.0f;
+        for (int z = 0; z < p.parts.nsplit; ++z)
+            if (p.parts.first(z) < (e + 1) * nbe && p.parts.first(z + 1) > e * nbe) sum += src[z * hrows * E];
+        p.dR[p.rows.gate(hk, r) * E + e] = sum;
     }
 }
 
@@ -787,7 +844,6 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // one are worth it only where one slice leaves CUs idle; with one slice the kernel writes dK, dU, dV itself and neither
 // partial sums nor the summing pass exist.  Every further slice adds a set of fp32 partial sums that is written and
 // read back once (priced at the time of a token tile per 2.5 MB: about 4 TB/s against 1.25 us per tile).
-constexpr int DW_CUS = 256;             // compute units of an MI355X
 constexpr long DW_FIXED_TILES = 9;      // prologue + epilogue of a workgroup, in token tiles
 constexpr long DW_BYTES_PER_TILE_TIME = 2500000;
 static int pick_nslice(const Dims& d, size_t ws_bytes)
@@ -799,7 +855,7 @@ static int pick_nslice(const Dims& d, size_t ws_bytes)
     long best = 1, best_cost = -1;
     for (long ns = 1; ns <= 64 && (ns == 1 || ns <= ntile / 8); ++ns) {
         if (ns > 1 && align256((size_t)ns * slice_b) > ws_bytes) break;
-        const long rounds = (cols * ns + DW_CUS - 1) / DW_CUS;
+        const long rounds = (cols * ns + CUS - 1) / CUS;
         const long cost = rounds * ((ntile + ns - 1) / ns + DW_FIXED_TILES) +
                           (ns > 1 ? ns * (long)(slice_b / DW_BYTES_PER_TILE_TIME) : 0);
         if (best_cost < 0 || cost < best_cost) { best = ns; best_cost = cost; }
@@ -807,11 +863,16 @@ static int pick_nslice(const Dims& d, size_t ws_bytes)
     return (int)best;
 }
 
+static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
+
+// The two kernels run one after the other, so the parts of dQ, dR and the token slices of dK, dU, dV share the workspace.
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
     const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
-    const int ns = pick_nslice(d, ~(size_t)0);
-    return ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
+    const int ns = pick_nslice(d, ~(size_t)0), nq = pick_nsplit(d, dq_part_bytes(d), ~(size_t)0);
+    const size_t dw = ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
+    const size_t dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
+    return dw > dq ? dw : dq;
 }
 
 template <int DH>
@@ -825,15 +886,21 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
 
     if (phases & PH_BWD_DQDR) {
         DqArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R,
-                 (bf16_t*)dQ, dR, d.H, G, d.S, d.E, nbe, d.tokmaj};
+                 (bf16_t*)dQ, dR, part, RowMap(d),
+                 Parts(d.E, nbe, pick_nsplit(d, dq_part_bytes(d), ws && !(phases & PH_ONE_PART) ? ws_bytes : 0))};
         const int tokw = 256;
         const int smem = DQ_NST * DQ_STAGE_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
         if (smem > 160 * 1024) return hipErrorInvalidValue;
         static LdsOptIn optin;
         err = ensure_dynamic_lds(optin, (const void*)mhffn_bwd_dqdr_kernel<DH>, smem);
         if (err != hipSuccess) return err;
-        dim3 grid((unsigned)d.H, (unsigned)((d.S + tokw - 1) / tokw), (unsigned)d.B);
+        dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
         hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
+        if (a.parts.nsplit > 1) {
+            const unsigned qb = (unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256);
+            const unsigned rb = (unsigned)(((long)a.rows.n * d.E + 255) / 256);
+            hipLaunchKernelGGL((mhffn_bwd_dqdr_sum_kernel<DH>), dim3(qb + rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, qb);
+        }
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }

@@ -107,7 +107,7 @@ int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V,
     const int rc = check_dims_impl(dims, dtype);
     if (rc != MHFFN_OK) return rc;
     if (token_layout != MHFFN_TOKENS_BHSD && token_layout != MHFFN_TOKENS_BSHD) return MHFFN_ERR_SHAPE;
-    if (phases & ~MHFFN_FWD_ALL) return MHFFN_ERR_SHAPE;       // a bit this build does not define: refuse, do not ignore
+    if (phases & ~(MHFFN_FWD_ALL | MHFFN_ONE_PART)) return MHFFN_ERR_SHAPE;       // a bit this build does not define: refuse, do not ignore
     if (!Q || !K || !U || !V || !R || !O) return MHFFN_ERR_NULL_POINTER;
     if (!aligned16(Q) || !aligned16(K) || !aligned16(U) || !aligned16(V) || !aligned16(R) || !aligned16(O) ||
         !aligned16(workspace))
@@ -117,9 +117,7 @@ int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V,
         if (!(phases & MHFFN_FWD_MAIN)) return MHFFN_OK;
         return mhffn::launch_fwd_f32(Q, K, U, V, R, O, d, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
     }
-    const size_t need = mhffn::fwd_workspace_bytes_bf16(d);
-    if (need > 0 && (!workspace || workspace_bytes < need)) return MHFFN_ERR_WORKSPACE;
-    const hipError_t err = mhffn::launch_fwd_bf16(Q, K, U, V, R, O, workspace, d, (hipStream_t)stream, phases);
+    const hipError_t err = mhffn::launch_fwd_bf16(Q, K, U, V, R, O, workspace, workspace_bytes, d, (hipStream_t)stream, phases);
     return err == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
 }
 
@@ -145,7 +143,7 @@ int mhffn_bwd_layout(const void* Q, const void* K, const void* U, const void* V,
     if (rc != MHFFN_OK) return rc;
     if (token_layout != MHFFN_TOKENS_BHSD && token_layout != MHFFN_TOKENS_BSHD) return MHFFN_ERR_SHAPE;
     if (grad_w_dtype != MHFFN_DTYPE_BF16 && grad_w_dtype != MHFFN_DTYPE_F32) return MHFFN_ERR_DTYPE;
-    if (phases & ~MHFFN_BWD_ALL) return MHFFN_ERR_SHAPE;       // a bit this build does not define: refuse, do not ignore
+    if (phases & ~(MHFFN_BWD_ALL | MHFFN_ONE_PART)) return MHFFN_ERR_SHAPE;       // a bit this build does not define: refuse, do not ignore
     if (!Q || !K || !U || !V || !R || !dO || !dQ || !dK || !dU || !dV || !dR) return MHFFN_ERR_NULL_POINTER;
     const void* ptrs[] = {Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, workspace};
     for (const void* p : ptrs)

@@ -275,6 +275,40 @@ __device__ __forceinline__ bf16x8 tr_value(const TrOperand& t)
     return __builtin_bit_cast(bf16x8, v);
 }
 
+// Stores 32 rows of DH fp32 values held as accumulator tiles of a transposed product (acc(i), row tile i: register 4a + x of
+// lane (l32, g) is column 32i + 8a + 4g + x of row l32) to dst[row][DH], rows below nrows.  Stored straight from the registers
+// these would be 32-byte pieces of 32 rows per instruction (23 MB of partial sums of the forward took 10 us longer that
+// way); they go 64 columns at a time through 8 KB of LDS private to the wave (256-byte rows, 16-byte chunk c of row r at
+// c ^ (r & 15)) and leave as 256-byte runs, 4 rows per instruction.  LDS operations of one wave complete in order.
+template <int DH, class Acc>
+__device__ __forceinline__ void store_rows_f32(unsigned char* region, float* dst, int nrows, int lane, Acc&& acc)
+{
+    constexpr int CT = DH / 32;
+    const int l32 = lane & 31, g = lane >> 5, c16 = lane & 15;
+    if (nrows <= 0) return;
+    static_for<(CT + 1) / 2>([&](auto hc) {
+        constexpr int h = decltype(hc)::value, NT = 2 * h + 1 < CT ? 2 : 1;
+        static_for<NT>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            const f32x16& v16 = acc(std::integral_constant<int, 2 * h + i>{});
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                f32x4 v;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[x] = v16[4 * a + x];
+                *reinterpret_cast<f32x4*>(region + l32 * 256 + (((8 * i + 2 * a + g) ^ (l32 & 15)) << 4)) = v;
+            }
+        });
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int row = 4 * k + (lane >> 4);
+            if (c16 < 8 * NT && row < nrows)
+                *reinterpret_cast<f32x4*>(dst + row * DH + 64 * h + 4 * c16) =
+                    *reinterpret_cast<const f32x4*>(region + row * 256 + ((c16 ^ (row & 15)) << 4));
+        }
+    });
+}
+
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt[3:0] at bits 3:0, vmcnt[5:4] at bits 15:14; other counters unconstrained).
 template <int N>
 __device__ __forceinline__ void wait_vmcnt()
@@ -317,11 +351,123 @@ __host__ __device__ inline TokRows tok_rows(int tokmaj, int b, int h, int H, int
     return tokmaj ? TokRows{(long)b * S * H + h, H} : TokRows{((long)b * H + h) * S, 1};
 }
 
-size_t fwd_workspace_bytes_bf16(const Dims& d);
+// Unsigned division by a fixed divisor, exact for dividends below 2^31 (the round-up method of Granlund and Montgomery,
+// "Division by invariant integers using multiplication", 1994): q = (mulhi(n, m) + n) >> l with l = ceil(log2 d).
+struct FastDiv {
+    unsigned m, l;
+    FastDiv() = default;
+    explicit FastDiv(unsigned d)
+    {
+        l = 0;
+        while ((1ull << l) < d) ++l;
+        m = (unsigned)(((1ull << 32) * ((1ull << l) - d)) / d + 1);
+    }
+    __device__ __forceinline__ unsigned div(unsigned n) const { return (__umulhi(n, m) + n) >> l; }
+};
+
+// The rows that meet one K/U/V head: the B * S tokens of its G q-heads, numbered so that a tile of consecutive rows is as
+// contiguous in memory as the layout allows ([B, H, S]: batch, then head of the group, then token; [B, S, H]: token,
+// then head of the group).  The forward and the dQ/dR kernel tile this list instead of the tokens of one (batch, q-head):
+// short sequences, decoded tokens and the heads of a group then share a tile and one pass over the weights.
+struct RowMap {
+    int tokmaj, H, Hkuv, G, S;
+    int n;            // rows of the list: G * B * S
+    FastDiv by_g, by_s, by_gs, by_hkuv;
+    RowMap() = default;
+    explicit RowMap(const Dims& d)
+        : tokmaj(d.tokmaj), H(d.H), Hkuv(d.Hkuv), G(d.H / d.Hkuv), S(d.S), n(d.H / d.Hkuv * d.B * d.S), by_g(d.H / d.Hkuv), by_s(d.S),
+          by_gs((unsigned)(d.H / d.Hkuv) * d.S), by_hkuv(d.Hkuv)
+    {
+    }
+    // row of Q, O, dO, dQ (units of d_h elements)
+    __device__ __forceinline__ long tok(int hk, unsigned r) const
+    {
+        if (tokmaj) {
+            const unsigned t = by_g.div(r);
+            return (long)t * H + hk * G + (r - t * G);
+        }
+        return head_major(hk, r);
+    }
+    // row of R, dR (units of E elements; always [B, H, S])
+    __device__ __forceinline__ long gate(int hk, unsigned r) const
+    {
+        if (tokmaj) {
+            const unsigned t = by_g.div(r), b = by_s.div(t);
+            return ((long)b * H + hk * G + (r - t * G)) * S + (t - b * S);
+        }
+        return head_major(hk, r);
+    }
+    // The rows first .. first + count - 1 (those of the list; first < n) as base + i * stride where they are such a run of
+    // Q, O, dO, dQ (tok) and of R, dR (gate); stride 0 where they are not.  Wave-uniform arguments: the kernels take the
+    // addresses of a run without a division per lane and stored row, which a tile needs only where it mixes batches
+    // (always divided, the twenty divisions of a wave cost the forward 1 % at 16,384 tokens).
+    struct Run {
+        TokRows tok, gate;
+    };
+    __device__ __forceinline__ Run run(int hk, unsigned first, unsigned count) const
+    {
+        const unsigned last = first + count <= (unsigned)n ? first + count - 1 : n - 1;
+        const FastDiv& d = tokmaj ? by_s : by_gs;
+        const bool one_batch = d.div(first) == d.div(last), ungrouped = !tokmaj || G == 1;
+        return Run{TokRows{tok(hk, first), tokmaj ? (ungrouped ? H : 0) : one_batch},
+                   TokRows{gate(hk, first), one_batch && ungrouped}};
+    }
+    __device__ __forceinline__ long tok(const Run& u, int hk, unsigned first, unsigned r) const
+    {
+        return u.tok.stride ? u.tok.base + (long)(r - first) * u.tok.stride : tok(hk, r);
+    }
+    __device__ __forceinline__ long gate(const Run& u, int hk, unsigned first, unsigned r) const
+    {
+        return u.gate.stride ? u.gate.base + (r - first) : gate(hk, r);
+    }
+    __device__ __forceinline__ long head_major(int hk, unsigned r) const
+    {
+        const unsigned b = by_gs.div(r);
+        return ((long)b * Hkuv + hk) * ((long)G * S) + (r - b * (unsigned)(G * S));
+    }
+};
+
+// The E * nbe blocks of a head (nbe = d_e / 32 per expert) in nsplit parts of consecutive blocks.
+struct Parts {
+    int E, nbe, nsplit;
+    FastDiv by_nbe, by_nsplit;
+    Parts() = default;
+    Parts(int E_, int nbe_, int nsplit_) : E(E_), nbe(nbe_), nsplit(nsplit_), by_nbe(nbe_), by_nsplit(nsplit_) {}
+    // first block of part z (z = nsplit: the end); E * nbe * nsplit < 2^31
+    __device__ __forceinline__ int first(int z) const { return by_nsplit.div(E * nbe * z); }
+};
+
+// Into how many parts the forward and the dQ/dR kernel cut the E * d_e / 32 blocks of a head.  One part needs no partial
+// sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute units a part per idle unit
+// shortens the serial walk over the blocks (one token of the 370M layer: 8 tiles of 121 blocks, 122 us with one part, 15
+// with 32), and every part costs a set of fp32 sums that is written and read back.  Priced in block steps (about 1 us):
+// rounds of CUS workgroups x (blocks of a part + 3 for prologue and epilogue) + 2 for the summing pass + 1 per 1.7 MB of
+// sums; over 29 shapes of 1 to 8,192 rows the pick is within 1 % of the fastest count measured on average, 11 % at worst.
+// Not cut: more experts than one LDS window of gate values holds; and 16,384 rows per head or more, where a head fills
+// a quarter of the chip alone and its results do not depend on how many other heads run beside it.
+constexpr int CUS = 256;                     // compute units of an MI355X
+constexpr long SPLIT_FIXED_STEPS = 3, SPLIT_SUM_STEPS = 2, SPLIT_BYTES_PER_STEP = 1700000;
+constexpr long SPLIT_ROWS_BELOW = 16384;
+inline int pick_nsplit(const Dims& d, size_t part_bytes, size_t ws_bytes)
+{
+    const long rows = (long)(d.H / d.Hkuv) * d.B * d.S, tiles = (rows + 255) / 256 * d.Hkuv;
+    const long blocks = (long)d.E * (d.d_e / JB);
+    if (d.E > GATE_WIN || rows >= SPLIT_ROWS_BELOW || blocks >= (1 << 24)) return 1;
+    long best = 1, best_cost = (tiles + CUS - 1) / CUS * (blocks + SPLIT_FIXED_STEPS);
+    for (long ns = 2; ns <= blocks && ns <= 64 && ns * part_bytes <= ws_bytes; ++ns) {
+        const long cost = (tiles * ns + CUS - 1) / CUS * ((blocks + ns - 1) / ns + SPLIT_FIXED_STEPS) + SPLIT_SUM_STEPS +
+                          (long)(ns * part_bytes) / SPLIT_BYTES_PER_STEP;
+        if (cost < best_cost) { best = ns; best_cost = cost; }
+    }
+    return (int)best;
+}
+
+size_t fwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one part);
+                                                      // with less it runs fewer parts
 size_t bwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one token
                                                       // slice, no partial sums); with less it runs fewer slices
 hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
-                           void* ws, const Dims& d, hipStream_t st, int phases);
+                           void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases);
 hipError_t launch_bwd_bf16(const void* Q, const void* K, const void* U, const void* V, const float* R, const void* dO,
                            void* dQ, void* dK, void* dU, void* dV, float* dR, int grad_w_f32,
                            void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases);
@@ -340,7 +486,8 @@ hipError_t launch_gate_fwd(const void* X, const float* Wn, float eps, const floa
 hipError_t launch_gate_bwd(const void* X, const float* Wn, float eps, const float* Wr, const void* dQ, int dq_tokmaj,
                            const float* dR, void* dX, float* dWn, float* dWr, const Dims& d, hipStream_t st);
 
-// Bits of the `phases` argument of the launch functions (the values of MHFFN_FWD_* / MHFFN_BWD_* in include/mhffn.h).
-constexpr int PH_FWD_MAIN = 1, PH_BWD_DQDR = 1, PH_BWD_DKDUDV = 2, PH_BWD_REDUCE = 4;
+// Bits of the `phases` argument of the launch functions (the values of MHFFN_FWD_*, MHFFN_BWD_*, MHFFN_ONE_PART in
+// include/mhffn.h).
+constexpr int PH_FWD_MAIN = 1, PH_BWD_DQDR = 1, PH_BWD_DKDUDV = 2, PH_BWD_REDUCE = 4, PH_ONE_PART = 256;
 
 }  // namespace mhffn

@@ -1,7 +1,8 @@
 // Fused multi-head FFN forward for gfx950 (bf16 MFMA, fp32 accumulation).
 //
-// One workgroup (4 waves, one per SIMD, 512 registers each) owns 256 tokens of one (batch, q-head); a wave owns 64 tokens
-// (two column tiles of 32).  The workgroup streams the K, U, V blocks (32 rows of the E*d_e axis at a time) straight
+// One workgroup (4 waves, one per SIMD, 512 registers each) owns 256 rows of one K/U/V head (tokens of any batch and q-head
+// of its group: RowMap) and all the head's blocks or one part of them (pick_nsplit); a wave owns 64 rows (two column tiles
+// of 32), "tokens" below.  The workgroup streams the K, U, V blocks (32 rows of the E*d_e axis at a time) straight
 // from the weight tensors into a ring of LDS stages with asynchronous LDS-direct loads.  Per block and wave:
 //     M^T = K Q^T, N^T = U Q^T               (A = rows of the K/U tiles, B = Q^T held in AGPRs for the whole kernel)
 //     P^T = silu(M^T) * N^T * r_e             (fp32 in the accumulator registers, rounded once to bf16)
@@ -29,8 +30,9 @@ struct FwdArgs {
     const bf16_t* V;
     const float* R;
     bf16_t* O;
-    int H, G, S, E, nbe;  // G = H / Hkuv, nbe = d_e / 32 blocks per expert
-    int tokmaj;           // Q, O token-major ([B, S, H, d_h]) instead of [B, H, S, d_h]
+    float* part;          // [nsplit][Hkuv][rows.n][DH] fp32 partial sums (more parts than one)
+    RowMap rows;          // rows of Q, O, R that meet one K/U/V head
+    Parts parts;          // ... and the blocks of that head
 };
 
 // LDS ring of FWD_NST stages, laid out as three regions (all V tiles, all K tiles, all U tiles).  The block loop is
@@ -68,13 +70,14 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x, tb = blockIdx.y, b = blockIdx.z;
-    const int hk = h / p.G;
-    const long rowbase = ((long)b * p.H + h) * p.S;          // rows of R
-    const TokRows qrows = tok_rows(p.tokmaj, b, h, p.H, p.S);   // rows of Q and O
-    const int tok0 = tb * BT + wave * 64;
-    const int nblk = p.E * p.nbe;
-    const long wbase = (long)hk * nblk * JB * DH;
+    // blockIdx.x = tile * Hkuv + kv-head: the head index runs fastest, so each head's weights stay in one XCD's L2
+    const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    const int tok0 = tile * BT + wave * 64;                  // this wave's rows of the list (RowMap)
+    const int nbe = p.parts.nbe, E = p.parts.E;
+    const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;   // blocks of this workgroup, counted from blk0
+    const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;        // expert of the first, its place in the expert
+    const int nex = p.parts.by_nbe.div(jb0 + nblk + nbe - 1);                // experts they belong to, counted from ex0
+    const long wbase = ((long)hk * E * nbe + blk0) * JB * DH;
     const bf16_t* Kh = p.K + wbase;
     const long offU = p.U - p.K, offV = p.V - p.K;
 
@@ -90,13 +93,15 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
             tile_fill_ins<DH>(Kh + toff + roff, DH, smem + region + stage * TILE_B, id & 7, lane);
         }
     };
+    const int first = tok0 < p.rows.n ? tok0 : p.rows.n - 1;
+    const RowMap::Run run = p.rows.run(hk, first, 64);
     // The Q rows come from HBM and are the longest wait of the prologue: request them before anything else.
     bf16x8 q[2][KS];
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) {
         int t = tok0 + ct * 32 + l32;
-        t = t < p.S ? t : p.S - 1;
-        const bf16_t* qr = p.Q + (qrows.base + (long)t * qrows.stride) * DH + 8 * g;
+        t = t < p.rows.n ? t : p.rows.n - 1;
+        const bf16_t* qr = p.Q + p.rows.tok(run, hk, first, t) * DH + 8 * g;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) q[ct][ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16);
     }
@@ -108,11 +113,11 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
     const float* rrow;
     {
         int t = tok0 + lane;
-        t = t < p.S ? t : p.S - 1;
-        rrow = p.R + (rowbase + t) * p.E;
+        t = t < p.rows.n ? t : p.rows.n - 1;
+        rrow = p.R + p.rows.gate(run, hk, first, t) * E + ex0;
     }
     auto stage_gates = [&](int e0) {
-        const int e1 = e0 + GATE_WIN < p.E ? e0 + GATE_WIN : p.E;
+        const int e1 = e0 + GATE_WIN < nex ? e0 + GATE_WIN : nex;
         for (int e = e0; e < e1; ++e)
             __builtin_amdgcn_global_load_lds((gptr_t)(rrow + e), (lptr_t)(sR + (e - e0) * BT + wave * 64), 4, 0, 0);
     };
@@ -271,19 +276,20 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
     using S1 = std::integral_constant<int, 1>;
     using S2 = std::integral_constant<int, 2>;
     using S3 = std::integral_constant<int, 3>;
-    int e = 0, jb = 0, blk = 0;
+    int e = 0, jb = jb0, blk = 0;
     auto advance = [&]() {
-        if (++jb == p.nbe) { jb = 0; ++e; }
+        if (++jb == nbe) { jb = 0; ++e; }
     };
-    // (A window of GATE_WIN experts is a multiple of four blocks, so every window starts on stage 0 and register set A.)
-    for (int e0 = 0; e0 < p.E; e0 += GATE_WIN) {
+    // (A window of GATE_WIN experts is a multiple of four blocks, so every window starts on stage 0 and register set A.
+    // The launcher cuts the blocks only where one window holds all experts: a part then has just this first window.)
+    for (int e0 = 0; e0 < nex; e0 += GATE_WIN) {
         if (e0 > 0) {
             __syncthreads();      // every wave has read its gate values of the window before
             stage_gates(e0);
             wait_vmcnt<0>();      // (also lands the two blocks in flight; the next step's wait then passes at once)
             __syncthreads();
         }
-        const int wend = (e0 + GATE_WIN) * p.nbe < nblk ? (e0 + GATE_WIN) * p.nbe : nblk;
+        const int wend = (e0 + GATE_WIN) * nbe < nblk ? (e0 + GATE_WIN) * nbe : nblk;
         for (; blk + 4 <= wend; blk += 4) {
             step(S0{}, blk, e, mA, nA, mB, nB);
             advance();
@@ -307,6 +313,14 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
     wait_vmcnt<0>();      // drain the phantom prefetches: they write the ring, which the epilogue reuses
     __syncthreads();      // every wave is done reading the ring
 
+    if (p.parts.nsplit > 1) {     // a part of the blocks leaves its sums as they are, fp32, for the pass that adds the parts
+        float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH;
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+            store_rows_f32<DH>(smem + wave * TILE_B, prow + ct * 32 * DH, p.rows.n - tok0 - ct * 32, lane,
+                               [&](auto ic) -> const f32x16& { return oacc[decltype(ic)::value][ct]; });
+        return;
+    }
     // O^T registers -> O[t][c].  Register 4a+b of row tile i is c = 32i + 8a + 4g + b: a lane owns runs of 4 c of one
     // token, which stored directly would be 8-byte pieces scattered over 32 rows per instruction.  Instead each wave
     // writes its 64 x d_h tile into a private 16 KB region of the ring (rows of 256 bytes, 16-byte chunk c16 of row r at
@@ -326,17 +340,44 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
                     *reinterpret_cast<bf16x4*>(otile + (ct * 32 + l32) * TILE_ROW_B + (((4 * i + a) ^ (l32 & 15)) << 4) + 8 * g) = v;
                 }
         const int c16 = lane & 15;
+        auto store = [&](auto&& address_row) {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int row = 4 * k + (lane >> 4);
-            const int t = tok0 + row;
-            if (c16 < DH / 8 && t < p.S) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(otile + row * TILE_ROW_B + ((c16 ^ (row & 15)) << 4));
-                *reinterpret_cast<u32x4*>(p.O + (qrows.base + (long)t * qrows.stride) * DH + c16 * 8) = v;
+            for (int k = 0; k < 16; ++k) {
+                const int row = 4 * k + (lane >> 4);
+                if (c16 < DH / 8 && tok0 + row < p.rows.n) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(otile + row * TILE_ROW_B + ((c16 ^ (row & 15)) << 4));
+                    *reinterpret_cast<u32x4*>(p.O + address_row(row) * DH + c16 * 8) = v;
+                }
             }
-        }
+        };
+        if (run.tok.stride) store([&](int row) { return run.tok.base + (long)row * run.tok.stride; });
+        else store([&](int row) { return p.rows.tok(hk, tok0 + row); });
     }
 }
+
+// Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, eight columns per lane.
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
+{
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    const unsigned r = i / (DH / 8), c = (i % (DH / 8)) * 8;
+    const int hk = blockIdx.y;
+    if (r >= (unsigned)p.rows.n) return;
+    const long step = (long)p.rows.Hkuv * p.rows.n * DH;
+    const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
+    f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+    for (int z = 1; z < p.parts.nsplit; ++z) {
+        src += step;
+        lo += *reinterpret_cast<const f32x4*>(src);
+        hi += *reinterpret_cast<const f32x4*>(src + 4);
+    }
+    bf16x8 v;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) { v[x] = (bf16_t)lo[x]; v[4 + x] = (bf16_t)hi[x]; }
+    *reinterpret_cast<bf16x8*>(p.O + p.rows.tok(hk, r) * DH + c) = v;
+}
+
+static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 
 template <int DH>
 static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, hipStream_t st)
@@ -347,21 +388,28 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, hipStream_t st)
     static LdsOptIn optin;
     const hipError_t e = ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem);
     if (e != hipSuccess) return e;
-    dim3 grid((unsigned)d.H, (unsigned)((d.S + tokw - 1) / tokw), (unsigned)d.B);
+    dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
     hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
+    if (a.parts.nsplit > 1) {
+        dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256), (unsigned)d.Hkuv);
+        hipLaunchKernelGGL((mhffn_fwd_sum_kernel<DH>), sgrid, dim3(256), 0, st, a);
+    }
     return hipGetLastError();
 }
 
-size_t fwd_workspace_bytes_bf16(const Dims&) { return 0; }
+size_t fwd_workspace_bytes_bf16(const Dims& d)
+{
+    const int ns = pick_nsplit(d, fwd_part_bytes(d), ~(size_t)0);
+    return ns > 1 ? ns * fwd_part_bytes(d) : 0;
+}
 
 hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
-                           void* ws, const Dims& d, hipStream_t st, int phases)
+                           void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases)
 {
-    (void)ws;
     if (!(phases & PH_FWD_MAIN)) return hipSuccess;
-    FwdArgs a{(const bf16_t*)Q, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, (bf16_t*)O,
-              d.H,              d.H / d.Hkuv,     d.S,              d.E,              d.d_e / JB,
-              d.tokmaj};
+    const int nsplit = pick_nsplit(d, fwd_part_bytes(d), ws && !(phases & PH_ONE_PART) ? ws_bytes : 0);
+    FwdArgs a{(const bf16_t*)Q, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V,           R,
+              (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, nsplit)};
     switch (d.d_h) {
         case 64: return launch_fwd_t<64>(a, d, st);
         case 96: return launch_fwd_t<96>(a, d, st);

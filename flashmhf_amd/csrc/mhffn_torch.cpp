@@ -122,7 +122,7 @@ Tensor as_layout(const Tensor& t, int layout)
 }
 Tensor contig(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
 
-Tensor op_forward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, const Tensor& V0, const Tensor& R0)
+Tensor op_forward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, const Tensor& V0, const Tensor& R0, bool one_part)
 {
     check_inputs(Q0, K0, U0, V0, R0);
     auto [Q, layout] = laid_out(Q0);
@@ -130,15 +130,15 @@ Tensor op_forward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, const Te
     const int dt = dtype_code(Q.scalar_type());
     const Plan& p = plan_for(dims_of(Q, K), dt);
     OnDevice guard(Q);
-    Tensor O = empty_like_layout(Q), ws = scratch(p.fwd_bytes, Q);
+    Tensor O = empty_like_layout(Q), ws = scratch(one_part ? 0 : p.fwd_bytes, Q);
     raise_for_code(mhffn_fwd_layout(ptr(Q), ptr(K), ptr(U), ptr(V), (const float*)ptr(R), ptr(O), ptr(ws), p.fwd_bytes, &p.dims, dt,
-                                    layout, stream(), MHFFN_FWD_ALL),
+                                    layout, stream(), MHFFN_FWD_ALL | (one_part ? MHFFN_ONE_PART : 0)),
                    "mhffn_fwd");
     return O;
 }
 
 variable_list op_backward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, const Tensor& V0, const Tensor& R0,
-                          const Tensor& dO0, at::ScalarType grad_w)
+                          const Tensor& dO0, at::ScalarType grad_w, bool one_part)
 {
     check_inputs(Q0, K0, U0, V0, R0);
     TORCH_CHECK(dO0.sizes() == Q0.sizes(), "grad_output shape should be the same as Q");
@@ -151,7 +151,8 @@ variable_list op_backward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, 
     Tensor dQ = empty_like_layout(Q), dR = empty_of(R.sizes(), at::kFloat, Q), ws = scratch(p.bwd_bytes, Q);
     Tensor dK = empty_of(K.sizes(), grad_w, Q), dU = empty_of(K.sizes(), grad_w, Q), dV = empty_of(K.sizes(), grad_w, Q);
     raise_for_code(mhffn_bwd_layout(ptr(Q), ptr(K), ptr(U), ptr(V), (const float*)ptr(R), ptr(dO), ptr(dQ), ptr(dK), ptr(dU), ptr(dV),
-                                    (float*)ptr(dR), wdt, ptr(ws), p.bwd_bytes, &p.dims, dt, layout, stream(), MHFFN_BWD_ALL),
+                                    (float*)ptr(dR), wdt, ptr(ws), p.bwd_bytes, &p.dims, dt, layout, stream(),
+                                    MHFFN_BWD_ALL | (one_part ? MHFFN_ONE_PART : 0)),
                    "mhffn_bwd");
     return {dQ, dK, dU, dV, dR};
 }
@@ -168,26 +169,29 @@ bool records_grad(std::initializer_list<const Tensor*> ts)
 // convention, kernels/thunderkittens/flash_ffn_moe_torch.py:17-21); otherwise in the inputs' dtypes.
 struct OpNode : torch::autograd::Function<OpNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R,
-                          bool f32_grads)
+                          bool f32_grads, bool one_part)
     {
         ctx->save_for_backward({Q, K, U, V, R});
         ctx->saved_data["f32"] = f32_grads;
-        return op_forward(Q, K, U, V, R);
+        ctx->saved_data["one_part"] = one_part;
+        return op_forward(Q, K, U, V, R, one_part);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
     {
         const auto s = ctx->get_saved_variables();
         const bool f32 = ctx->saved_data["f32"].toBool();
-        auto out = op_backward(s[0], s[1], s[2], s[3], s[4], g[0], f32 ? at::kFloat : s[1].scalar_type());
+        auto out = op_backward(s[0], s[1], s[2], s[3], s[4], g[0], f32 ? at::kFloat : s[1].scalar_type(),
+                               ctx->saved_data["one_part"].toBool());
         if (f32) out[0] = out[0].to(at::kFloat);
-        out.emplace_back();
+        out.resize(7);
         return out;
     }
 };
-Tensor op(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, bool f32_grads)
+Tensor op(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, bool f32_grads,
+          bool one_part)
 {
-    if (!records_grad({&Q, &K, &U, &V, &R})) return op_forward(Q, K, U, V, R);
-    return OpNode::apply(Q, K, U, V, R, f32_grads);
+    if (!records_grad({&Q, &K, &U, &V, &R})) return op_forward(Q, K, U, V, R, one_part);
+    return OpNode::apply(Q, K, U, V, R, f32_grads, one_part);
 }
 
 // The single-expert operator: Q [B,H,S,d_h], K/U/V [Hkuv, rows, d_h], gate 1.
@@ -197,18 +201,18 @@ struct SingleNode : torch::autograd::Function<SingleNode> {
     {
         const Tensor R = ones_gate(Q);
         ctx->save_for_backward({Q, K, U, V, R});
-        return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), R);
+        return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), R, false);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
     {
         const auto s = ctx->get_saved_variables();
-        auto out = op_backward(s[0], s[1].unsqueeze(1), s[2].unsqueeze(1), s[3].unsqueeze(1), s[4], g[0], s[1].scalar_type());
+        auto out = op_backward(s[0], s[1].unsqueeze(1), s[2].unsqueeze(1), s[3].unsqueeze(1), s[4], g[0], s[1].scalar_type(), false);
         return {out[0], out[1].squeeze(1), out[2].squeeze(1), out[3].squeeze(1)};
     }
 };
 Tensor single(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V)
 {
-    if (!records_grad({&Q, &K, &U, &V})) return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones_gate(Q));
+    if (!records_grad({&Q, &K, &U, &V})) return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones_gate(Q), false);
     return SingleNode::apply(Q, K, U, V);
 }
 
@@ -301,24 +305,26 @@ struct BlockForward {
     Tensor O4, Y;      // operator output [B,S,H,d_h], block output
 };
 BlockForward block_forward(const Tensor& x, const Tensor& w1, const Tensor& norm_weight, const Tensor& router, const Tensor& K,
-                           const Tensor& U, const Tensor& V, const Tensor& w2, double eps)
+                           const Tensor& U, const Tensor& V, const Tensor& w2, double eps, bool one_part)
 {
     BlockForward f;
     const int64_t B = x.size(0), S = x.size(1), hid = x.size(2);
     f.g = gate_forward(at::linear(x, w1).view({B, S, router.size(0), router.size(1)}), norm_weight, router, eps);
-    f.O4 = op_forward(f.g.q4.transpose(1, 2), K, U, V, f.g.R).transpose(1, 2);
+    f.O4 = op_forward(f.g.q4.transpose(1, 2), K, U, V, f.g.R, one_part).transpose(1, 2);
     f.Y = at::linear(f.O4.view({B, S, hid}), w2);
     return f;
 }
 
 struct BlockNode : torch::autograd::Function<BlockNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight,
-                          const Tensor& router, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& w2, double eps)
+                          const Tensor& router, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& w2, double eps,
+                          bool one_part)
     {
         const Tensor nw = norm_weight.value_or(Tensor());
-        BlockForward f = block_forward(x, w1, nw, router, K, U, V, w2, eps);
+        BlockForward f = block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part);
         ctx->save_for_backward({x, w1, nw, router, K, U, V, w2, f.g.x4, f.g.wn, f.g.wr, f.g.q4, f.g.R, f.O4});
         ctx->saved_data["eps"] = eps;
+        ctx->saved_data["one_part"] = one_part;
         return f.Y;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads)
@@ -331,21 +337,22 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor dY = grads[0].reshape({-1, hid});
         const Tensor dO = at::mm(dY, w2).view(O4.sizes());
         const Tensor dw2 = at::mm(dY.t(), O4.view({-1, hid}));
-        auto g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type());
+        auto g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type(), ctx->saved_data["one_part"].toBool());
         auto h = gate_backward(x4, nw, router, wn, wr, ctx->saved_data["eps"].toDouble(), g[0], g[4]);
         const Tensor dp = h[0].view({-1, hid});
         Tensor dx;
         if (ctx->needs_input_grad(0)) dx = at::mm(dp, w1).view(x.sizes());
         const Tensor dw1 = at::mm(dp.t(), x.reshape({-1, hid}));
-        return {dx, dw1, h[1], h[2], g[1], g[2], g[3], dw2, Tensor()};
+        return {dx, dw1, h[1], h[2], g[1], g[2], g[3], dw2, Tensor(), Tensor()};
     }
 };
 Tensor block(const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight, const Tensor& router, const Tensor& K,
-             const Tensor& U, const Tensor& V, const Tensor& w2, double eps)
+             const Tensor& U, const Tensor& V, const Tensor& w2, double eps, bool one_part)
 {
     const Tensor nw = norm_weight.value_or(Tensor());
-    if (!records_grad({&x, &w1, &nw, &router, &K, &U, &V, &w2})) return block_forward(x, w1, nw, router, K, U, V, w2, eps).Y;
-    return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps);
+    if (!records_grad({&x, &w1, &nw, &router, &K, &U, &V, &w2}))
+        return block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part).Y;
+    return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps, one_part);
 }
 
 }  // namespace
@@ -356,7 +363,9 @@ PYBIND11_MODULE(_native, m)
     m.def("op_forward", torch::wrap_pybind_function_no_gil(op_forward));
     m.def("op_backward", torch::wrap_pybind_function_no_gil(
                              [](const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, const Tensor& dO,
-                                bool f32_grad_w) { return op_backward(Q, K, U, V, R, dO, f32_grad_w ? at::kFloat : at::kBFloat16); }));
+                                bool f32_grad_w, bool one_part) {
+                                 return op_backward(Q, K, U, V, R, dO, f32_grad_w ? at::kFloat : at::kBFloat16, one_part);
+                             }));
     m.def("op", torch::wrap_pybind_function_no_gil(op));
     m.def("single", torch::wrap_pybind_function_no_gil(single));
     m.def("gate", torch::wrap_pybind_function_no_gil(gate));

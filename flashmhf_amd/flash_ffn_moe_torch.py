@@ -28,4 +28,4 @@ class FlashFFNMoE(torch.nn.Module):
         super().__init__()
 
     def forward(self, Q, K, U, V, R):
-        return _capi.native().op(Q, K, U, V, R, True)
+        return _capi.native().op(Q, K, U, V, R, True, False)

@@ -18,18 +18,19 @@ import torch
 from . import _capi
 
 
-def mhffn_forward(Q, K, U, V, R):
-    """Launches the fused forward on the current stream and returns O (same shape and dtype as Q)."""
-    return _capi.native().op_forward(Q, K, U, V, R)
+def mhffn_forward(Q, K, U, V, R, one_part=False):
+    """Launches the fused forward on the current stream and returns O (same shape and dtype as Q).
+    ``one_part``: sum over the experts in one fixed order whatever the number of tokens (MHFFN_ONE_PART in include/mhffn.h)."""
+    return _capi.native().op_forward(Q, K, U, V, R, one_part)
 
 
-def mhffn_backward(Q, K, U, V, R, dO, grad_w_dtype=torch.bfloat16):
+def mhffn_backward(Q, K, U, V, R, dO, grad_w_dtype=torch.bfloat16, one_part=False):
     """Launches the fused backward; returns (dQ, dK, dU, dV, dR).  dQ has Q's dtype, dR is fp32,
     dK/dU/dV have ``grad_w_dtype`` (bf16 as flash_mlp_moe.py:808-810, or fp32 as flash_ffn_moe_torch.py:18-20)."""
     assert dO.shape == Q.shape, "grad_output shape should be the same as Q"
     if grad_w_dtype not in (torch.bfloat16, torch.float32):
         _capi.raise_for_code(_capi.ERR_DTYPE, "mhffn_bwd")
-    return tuple(_capi.native().op_backward(Q, K, U, V, R, dO, grad_w_dtype == torch.float32))
+    return tuple(_capi.native().op_backward(Q, K, U, V, R, dO, grad_w_dtype == torch.float32, one_part))
 
 
 class FlashMLPFunction(torch.autograd.Function):
@@ -51,10 +52,12 @@ class FlashMLPFunction(torch.autograd.Function):
 
 
 class FlashMLPMoE(torch.nn.Module):
-    """Stateless module, ``forward(Q, K, U, V, R) -> O``.  Mirrors kernels/triton/flash_mlp_moe.py:871-903."""
+    """Stateless module, ``forward(Q, K, U, V, R) -> O``.  Mirrors kernels/triton/flash_mlp_moe.py:871-903.
+    ``one_part``: see ``mhffn_forward``; O, dQ and dR of a token then do not depend on the other tokens of the call."""
 
-    def __init__(self):
+    def __init__(self, one_part=False):
         super().__init__()
+        self.one_part = one_part
 
     def forward(self, Q, K, U, V, R):
-        return _capi.native().op(Q, K, U, V, R, False)
+        return _capi.native().op(Q, K, U, V, R, False, self.one_part)

@@ -157,7 +157,7 @@ class MHFFNLayer(nn.Module):
         B, S, hid = x.shape
         if self._one_node(x):
             return _capi.native().block(x, self.w_self.weight, None if self.q_norm is None else self.q_norm.weight, self.router,
-                                        self.K, self.U, self.V, self.w_self_2.weight, self.rms_norm_eps)
+                                        self.K, self.U, self.V, self.w_self_2.weight, self.rms_norm_eps, self.op.one_part)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
@@ -210,6 +210,10 @@ class MHFFNDecoder(nn.Module):
     def __init__(self, vocab_size, hidden_size, num_layers, attn_heads, ffn_heads, num_experts, expert_dim, eps=1e-6,
                  **layer_kw):
         super().__init__()
+        # One fixed order of summation: what a sequence gets from the model, and what it gives to the gradients, does not
+        # depend on the rest of its batch.  (Rounding differences of the operator grow from block to block: another order
+        # moves the gradients of a four-block model by 1 % of their norm.)
+        layer_kw.setdefault("op", FlashMLPMoE(one_part=True))
         self.embed = nn.Embedding(vocab_size, hidden_size)
         self.blocks = nn.ModuleList(
             MHFFNDecoderBlock(hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps, **layer_kw)

@@ -16,8 +16,8 @@
  *   - the library never allocates, never synchronises and never throws; work is enqueued on `stream`
  *     (a hipStream_t passed as void*, NULL = the default stream).
  *   - return value: MHFFN_OK or a negative MHFFN_ERR_* code; all argument checks happen before any launch.
- *   - `workspace` is caller-provided device scratch of at least the size the matching *_workspace_bytes()
- *     call reports (16-byte aligned).  Its contents are undefined after the call.
+ *   - `workspace` is caller-provided device scratch of the size the matching *_workspace_bytes() call reports
+ *     (16-byte aligned).  Its contents are undefined after the call.
  */
 #ifndef MHFFN_H_
 #define MHFFN_H_
@@ -40,7 +40,7 @@ enum {
     MHFFN_ERR_HEAD_DIM     = -3,  /* reference: assert head_dim == 128, flash_ffn_moe.cu:956 */
     MHFFN_ERR_EXPERT_DIM   = -4,  /* reference: ValueError, flash_mlp_moe.py:758-759; assert flash_ffn_moe.cu:958 */
     MHFFN_ERR_SHAPE        = -5,  /* non-positive extent, H not a multiple of Hkuv, gate kernels with E > 64 */
-    MHFFN_ERR_WORKSPACE    = -6,  /* workspace missing or smaller than *_workspace_bytes() */
+    MHFFN_ERR_WORKSPACE    = -6,  /* backward: workspace missing or smaller than mhffn_bwd_workspace_bytes() */
     MHFFN_ERR_LAUNCH       = -7,  /* hipGetLastError() after a launch */
     MHFFN_ERR_ALIGNMENT    = -8,  /* a tensor or workspace pointer is not 16-byte aligned */
     MHFFN_ERR_STATIC_SCRATCH = -9 /* mhffn_bwd_static only: the problem needs more than MHFFN_STATIC_SCRATCH_BYTES */
@@ -68,9 +68,12 @@ int mhffn_is_supported(int d_h, int d_e, int dtype);
 /* Checks extents and dtype only (no pointers, no GPU).  Returns MHFFN_OK or the error the launch would return. */
 int mhffn_check_dims(const mhffn_dims* dims, int dtype);
 
-/* Scratch bytes needed by mhffn_fwd / mhffn_bwd for these extents.  0 is a valid answer, not only the answer for invalid
- * extents (ask mhffn_check_dims for those): the forward never needs scratch, and the bfloat16 backward needs none where
- * its dK/dU/dV kernel runs as one token slice (e.g. the 370M and 1.3B layers); `workspace` may then be NULL. */
+/* Scratch bytes of mhffn_fwd / mhffn_bwd for these extents.  0 is a valid answer, not only the answer for invalid extents
+ * (ask mhffn_check_dims for those): the bfloat16 kernels need none where their row tiles and weight columns fill the GPU by
+ * themselves (e.g. the 370M and 1.3B layers at their benchmark sizes); `workspace` may then be NULL.
+ *   - forward: the bytes are those of the fp32 partial sums with which a small number of tokens is computed fastest.  Any
+ *     smaller workspace, NULL included, is accepted: the same result (up to fp32 summation order), with less of the GPU busy.
+ *   - backward: the workspace is required. */
 size_t mhffn_fwd_workspace_bytes(const mhffn_dims* dims, int dtype);
 size_t mhffn_bwd_workspace_bytes(const mhffn_dims* dims, int dtype);
 
@@ -99,10 +102,15 @@ int mhffn_bwd(const void* Q, const void* K, const void* U, const void* V, const 
  * mhffn_bwd == mhffn_bwd_phases(..., MHFFN_BWD_ALL).  They exist so a benchmark can bracket one kernel with HIP
  * events on the launch stream; the reference has no counterpart (its kernels are launched one per Python call,
  * flash_mlp_moe.py:832-866).  A mask with a bit outside MHFFN_FWD_ALL / MHFFN_BWD_ALL returns MHFFN_ERR_SHAPE (the bit
- * values are not stable across versions of this header: pass the names, not numbers). */
+ * values are not stable across versions of this header: pass the names, not numbers).  MHFFN_BWD_REDUCE alone needs the last
+ * call on the workspace to have run MHFFN_BWD_DKDUDV: the kernels of MHFFN_BWD_DQDR use the same bytes. */
 enum {
     MHFFN_FWD_MAIN = 1, MHFFN_FWD_ALL = 1,
-    MHFFN_BWD_DQDR = 1, MHFFN_BWD_DKDUDV = 2, MHFFN_BWD_REDUCE = 4, MHFFN_BWD_ALL = 7
+    MHFFN_BWD_DQDR = 1, MHFFN_BWD_DKDUDV = 2, MHFFN_BWD_REDUCE = 4, MHFFN_BWD_ALL = 7,
+    /* May be added to any mask (bfloat16): O, dQ and dR are summed over the experts' rows in one fixed order, so that a token's
+     * values do not depend, to the last bit, on how many other tokens the call holds.  Without it a call with few tokens
+     * adds the partial sums of several workgroups (see mhffn_fwd_workspace_bytes), which is faster. */
+    MHFFN_ONE_PART = 256
 };
 int mhffn_fwd_phases(const void* Q, const void* K, const void* U, const void* V, const float* R,
                      void* O, void* workspace, size_t workspace_bytes,

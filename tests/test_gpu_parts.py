@@ -1,0 +1,58 @@
+"""Few rows per head: the forward and the dQ/dR kernel cut the blocks of a head into parts whose fp32 sums a second pass adds
+(pick_nsplit in csrc/mhffn_common.hpp).  Row counts around the 32- and 256-row tiles, tiles that mix batches, q-heads of a
+group and ragged ends, parts that begin and end inside an expert, against the fp64 oracle; and MHFFN_ONE_PART, whose
+results for a token do not depend on the call's other tokens."""
+import pytest
+import torch
+
+from oracle import mhffn_oracle as orc
+from tests.helpers import assert_bf16_parity, make_inputs
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+CASES = [
+    # B, H, S, dh, E, de, Hk, token_major
+    (1, 2, 1, 64, 1, 32, 2, False),       # one block: nothing to cut
+    (1, 3, 1, 128, 5, 96, 3, True),       # one row, a part per block
+    (5, 4, 1, 96, 2, 64, 2, True),        # decoded tokens of five sequences share a tile with the heads of their group
+    (1, 2, 255, 128, 3, 224, 2, False),
+    (3, 4, 43, 64, 7, 96, 1, False),      # 516 rows of one K/U/V head: tiles across batches and heads
+    (2, 2, 257, 96, 64, 32, 2, False),    # as many experts as one LDS window of gate values holds
+]
+
+
+def _run(case, seed=3):
+    B, H, S, dh, E, de, Hk, tm = case
+    ins = make_inputs(B, H, S, dh, E, de, Hk, seed=seed, dtype=torch.bfloat16)
+    dev = [t.to(DEV) for t in ins]
+    if tm:
+        dev[0], dev[5] = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (dev[0], dev[5]))
+    return ins, dev
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_parts_match_the_oracle(case):
+    from flashmhf_amd import _capi, mhffn_backward, mhffn_forward
+    print("case", case, flush=True)
+    B, H, S, dh, E, de, Hk, _ = case
+    blocks = E * de // 32
+    assert (_capi.lib().mhffn_fwd_workspace_bytes(_capi.Dims(B, H, Hk, S, dh, E, de), 0) > 0) == (blocks > 1)
+    ins, dev = _run(case)
+    O = mhffn_forward(*dev[:5])
+    g = mhffn_backward(*dev, grad_w_dtype=torch.float32)
+    torch.cuda.synchronize()
+    ref = (orc.mhffn_forward(*ins[:5], compute_dtype=torch.float64), *orc.mhffn_backward(*ins, compute_dtype=torch.float64))
+    for name, got, r in zip(("O", "dQ", "dK", "dU", "dV", "dR"), (O, *g), ref):
+        assert_bf16_parity(name, got.float().cpu(), r, case)
+
+
+def test_one_part_does_not_depend_on_the_other_tokens():
+    from flashmhf_amd import mhffn_backward, mhffn_forward
+    _, (Q, K, U, V, R, dO) = _run((2, 4, 300, 128, 5, 96, 2, False))
+    O, g = mhffn_forward(Q, K, U, V, R, one_part=True), mhffn_backward(Q, K, U, V, R, dO, one_part=True)
+    few = slice(37, 40)
+    q, r, d = (t[1:, :, few].contiguous() for t in (Q, R, dO))
+    o, h = mhffn_forward(q, K, U, V, r, one_part=True), mhffn_backward(q, K, U, V, r, d, one_part=True)
+    for a, b in ((o, O), (h[0], g[0]), (h[4], g[4])):
+        assert torch.equal(a, b[1:, :, few])
