@@ -89,7 +89,7 @@ int mhffn_check_dims(const mhffn_dims* dims, int dtype) { return check_dims_impl
 size_t mhffn_fwd_workspace_bytes(const mhffn_dims* dims, int dtype)
 {
     if (check_dims_impl(dims, dtype) != MHFFN_OK) return 0;
-    if (dtype == MHFFN_DTYPE_F32) return 0;
+    if (dtype == MHFFN_DTYPE_F32) return mhffn::fwd_workspace_bytes_f32(to_dims(dims));
     return mhffn::fwd_workspace_bytes_bf16(to_dims(dims));
 }
 
@@ -115,7 +115,9 @@ int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V,
     const mhffn::Dims d = to_dims(dims, token_layout);
     if (dtype == MHFFN_DTYPE_F32) {
         if (!(phases & MHFFN_FWD_MAIN)) return MHFFN_OK;
-        return mhffn::launch_fwd_f32(Q, K, U, V, R, O, d, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
+        return mhffn::launch_fwd_f32(Q, K, U, V, R, O, workspace, workspace_bytes, d, (hipStream_t)stream, phases) == hipSuccess
+                   ? MHFFN_OK
+                   : MHFFN_ERR_LAUNCH;
     }
     const hipError_t err = mhffn::launch_fwd_bf16(Q, K, U, V, R, O, workspace, workspace_bytes, d, (hipStream_t)stream, phases);
     return err == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
@@ -152,8 +154,8 @@ int mhffn_bwd_layout(const void* Q, const void* K, const void* U, const void* V,
     const size_t need = dtype == MHFFN_DTYPE_F32 ? mhffn::bwd_workspace_bytes_f32(d) : mhffn::bwd_workspace_bytes_bf16(d);
     if (need > 0 && (!workspace || workspace_bytes < need)) return MHFFN_ERR_WORKSPACE;
     if (dtype == MHFFN_DTYPE_F32)
-        return mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, workspace, d,
-                                     (hipStream_t)stream, phases) == hipSuccess
+        return mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, workspace,
+                                     need, d, (hipStream_t)stream, phases) == hipSuccess
                    ? MHFFN_OK
                    : MHFFN_ERR_LAUNCH;
     const hipError_t err = mhffn::launch_bwd_bf16(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR,
@@ -183,7 +185,7 @@ int mhffn_bwd_static(const void* Q, const void* K, const void* U, const void* V,
     if (static_scratch_of_current_device(&ws) != hipSuccess) return MHFFN_ERR_LAUNCH;
     hipError_t err;
     if (dtype == MHFFN_DTYPE_F32)
-        err = mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, ws, d,
+        err = mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, ws, need, d,
                                     (hipStream_t)stream, MHFFN_BWD_ALL);
     else
         err = mhffn::launch_bwd_bf16(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, ws,

@@ -420,6 +420,14 @@ struct RowMap {
     {
         return u.gate.stride ? u.gate.base + (r - first) : gate(hk, r);
     }
+    // The same rows in [B, H, S] order whatever the layout (sums over rows then have one order): row of Q, dO; the row of R
+    // is head_major(hk, r).
+    __device__ __forceinline__ long tok_head_major(int hk, unsigned r) const
+    {
+        if (!tokmaj) return head_major(hk, r);
+        const unsigned b = by_gs.div(r), rem = r - b * (unsigned)(G * S), gi = by_s.div(rem);
+        return ((long)b * S + (rem - gi * S)) * H + hk * G + gi;
+    }
     __device__ __forceinline__ long head_major(int hk, unsigned r) const
     {
         const unsigned b = by_gs.div(r);
@@ -446,20 +454,27 @@ struct Parts {
 // Not cut: more experts than one LDS window of gate values holds; and 16,384 rows per head or more, where a head fills
 // a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X
-constexpr long SPLIT_FIXED_STEPS = 3, SPLIT_SUM_STEPS = 2, SPLIT_BYTES_PER_STEP = 1700000;
-constexpr long SPLIT_ROWS_BELOW = 16384;
-inline int pick_nsplit(const Dims& d, size_t part_bytes, size_t ws_bytes)
+struct SplitCost {
+    long tile_rows, fixed_steps, sum_steps, bytes_per_step;
+};
+inline int cheapest_nsplit(const SplitCost& c, const Dims& d, long blocks, size_t part_bytes, size_t ws_bytes)
 {
-    const long rows = (long)(d.H / d.Hkuv) * d.B * d.S, tiles = (rows + 255) / 256 * d.Hkuv;
-    const long blocks = (long)d.E * (d.d_e / JB);
-    if (d.E > GATE_WIN || rows >= SPLIT_ROWS_BELOW || blocks >= (1 << 24)) return 1;
-    long best = 1, best_cost = (tiles + CUS - 1) / CUS * (blocks + SPLIT_FIXED_STEPS);
+    const long tiles = ((long)(d.H / d.Hkuv) * d.B * d.S + c.tile_rows - 1) / c.tile_rows * d.Hkuv;
+    if (tiles >= CUS || blocks >= (1 << 24)) return 1;
+    long best = 1, best_cost = blocks + c.fixed_steps;
     for (long ns = 2; ns <= blocks && ns <= 64 && ns * part_bytes <= ws_bytes; ++ns) {
-        const long cost = (tiles * ns + CUS - 1) / CUS * ((blocks + ns - 1) / ns + SPLIT_FIXED_STEPS) + SPLIT_SUM_STEPS +
-                          (long)(ns * part_bytes) / SPLIT_BYTES_PER_STEP;
+        const long cost = (tiles * ns + CUS - 1) / CUS * ((blocks + ns - 1) / ns + c.fixed_steps) + c.sum_steps +
+                          (long)(ns * part_bytes) / c.bytes_per_step;
         if (cost < best_cost) { best = ns; best_cost = cost; }
     }
     return (int)best;
+}
+constexpr SplitCost BF16_COST = {256, 3, 2, 1700000};
+constexpr long SPLIT_ROWS_BELOW = 16384;
+inline int pick_nsplit(const Dims& d, size_t part_bytes, size_t ws_bytes)
+{
+    if (d.E > GATE_WIN || (long)(d.H / d.Hkuv) * d.B * d.S >= SPLIT_ROWS_BELOW) return 1;
+    return cheapest_nsplit(BF16_COST, d, (long)d.E * (d.d_e / JB), part_bytes, ws_bytes);
 }
 
 size_t fwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one part);
@@ -473,12 +488,13 @@ hipError_t launch_bwd_bf16(const void* Q, const void* K, const void* U, const vo
                            void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases);
 
 // fp32 instantiation (mhffn_f32.hip): d_h a multiple of 8 up to 128, any d_e, any E.
+size_t fwd_workspace_bytes_f32(const Dims& d);        // as fwd_workspace_bytes_bf16
 size_t bwd_workspace_bytes_f32(const Dims& d);
 hipError_t launch_fwd_f32(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
-                          const Dims& d, hipStream_t st);
+                          void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases);
 hipError_t launch_bwd_f32(const void* Q, const void* K, const void* U, const void* V, const float* R, const void* dO,
-                          void* dQ, void* dK, void* dU, void* dV, float* dR, int grad_w_f32, void* ws, const Dims& d,
-                          hipStream_t st, int phases);
+                          void* dQ, void* dK, void* dU, void* dV, float* dR, int grad_w_f32, void* ws, size_t ws_bytes,
+                          const Dims& d, hipStream_t st, int phases);
 
 // Head prologue (mhffn_gate.hip): per-head RMSNorm + expert gate over [B, S, H, d_h] bf16 rows; d_h 64/96/128, E <= 64.
 hipError_t launch_gate_fwd(const void* X, const float* Wn, float eps, const float* Wr, void* Qn, float* R, const Dims& d,

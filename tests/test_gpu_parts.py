@@ -56,3 +56,24 @@ def test_one_part_does_not_depend_on_the_other_tokens():
     o, h = mhffn_forward(q, K, U, V, r, one_part=True), mhffn_backward(q, K, U, V, r, d, one_part=True)
     for a, b in ((o, O), (h[0], g[0]), (h[4], g[4])):
         assert torch.equal(a, b[1:, :, few])
+
+
+@pytest.mark.parametrize("case", [
+    # B, H, S, dh, E, de, Hk, token_major: rows around the 128-row tile, weight rows around the 32-row block, every tile width
+    (1, 2, 1, 8, 1, 1, 2, False), (1, 2, 127, 32, 2, 31, 1, True), (1, 1, 129, 72, 3, 33, 1, False),
+    (2, 2, 64, 128, 5, 65, 2, True), (1, 4, 385, 96, 2, 64, 2, True),
+])
+def test_float32_parts_and_slices_match_the_oracle(case):
+    from flashmhf_amd import mhffn_backward, mhffn_forward
+    print("case", case, flush=True)
+    B, H, S, dh, E, de, Hk, tm = case
+    ins = make_inputs(B, H, S, dh, E, de, Hk, seed=9)
+    dev = [t.to(DEV) for t in ins]
+    if tm:
+        dev[0], dev[5] = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (dev[0], dev[5]))
+    got = (mhffn_forward(*dev[:5]), *mhffn_backward(*dev, grad_w_dtype=torch.float32))
+    torch.cuda.synchronize()
+    ref = (orc.mhffn_forward(*ins[:5], compute_dtype=torch.float64), *orc.mhffn_backward(*ins, compute_dtype=torch.float64))
+    for name, a, r in zip(("O", "dQ", "dK", "dU", "dV", "dR"), got, ref):
+        err = (a.double().cpu() - r).abs().max().item()
+        assert err <= 1e-5 * max(1.0, r.abs().max().item()), (name, case, err)
