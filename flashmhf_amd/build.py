@@ -68,6 +68,10 @@ def build_lib(verbose=False, jobs=4):
         for name in sorted(usage):
             f.write(name + "  " + "  ".join(f"{k}={v}" for k, v in usage[name].items()) + "\n")
     check_no_scratch(usage)
+    for frag, count in VARIANT_KERNELS:
+        found = [n for n in usage if frag in n]
+        if len(found) != count or any(int(usage[n]["ScratchSize"]) for n in found):
+            raise RuntimeError(f"expected {count} instantiations of {frag} without scratch memory, found {found}")
     return LIB
 
 
@@ -110,6 +114,8 @@ EXPECTED_KERNELS = (
     ("mhffn_fwd_kernel", 3), ("mhffn_bwd_dqdr_kernel", 3), ("mhffn_bwd_dkdudv_kernel", 6),
     ("mhffn_gate_fwd_kernel", 12), ("mhffn_gate_bwd_kernel", 12),
 )
+# Variants of those kernels for smaller problems, under the same rule.
+VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3),)
 # The one instantiation known to spill: head prologue backward for d_h = 128 with more than 32 experts and RMSNorm
 # (<128, 2, true>).  It is correct but slow; the block (MHFFNLayer.heads_and_gate) does not route that case to it.
 ALLOWED_SCRATCH = ("mhffn_gate_bwd_kernelILi128ELi2ELb1E",)

@@ -1,7 +1,7 @@
 // Fused multi-head FFN backward for gfx950 (bf16 MFMA, fp32 accumulation), two kernels:
 //
 //  (1) dQ/dR kernel -- a workgroup of 8 waves (two per SIMD) owns 256 rows of one K/U/V head (tokens of any batch and
-//      q-head of its group: RowMap), 32 per wave, and all the head's blocks or one part of them (pick_nsplit); it
+//      q-head of its group: RowMap), 32 per wave, and all the head's blocks or one part of them (pick_parts); it
 //      streams the K, U, V blocks (32 rows at a time) through a ring of LDS stages with LDS-direct loads.  Per block:
 //          M^T = K Q^T, N^T = U Q^T, dA^T = V dO^T            (recomputed, registers only)
 //          dR_e += sum_j dA * silu(M) * N                      (fp32, before any rounding)
@@ -865,11 +865,17 @@ static int pick_nslice(const Dims& d, size_t ws_bytes)
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
+constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33}};
+static int dq_nsplit(const Dims& d, size_t ws_bytes)
+{
+    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), ws_bytes).nsplit;
+}
+
 // The two kernels run one after the other, so the parts of dQ, dR and the token slices of dK, dU, dV share the workspace.
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
     const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
-    const int ns = pick_nslice(d, ~(size_t)0), nq = pick_nsplit(d, dq_part_bytes(d), ~(size_t)0);
+    const int ns = pick_nslice(d, ~(size_t)0), nq = dq_nsplit(d, ~(size_t)0);
     const size_t dw = ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
     const size_t dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
     return dw > dq ? dw : dq;
@@ -887,7 +893,7 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     if (phases & PH_BWD_DQDR) {
         DqArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R,
                  (bf16_t*)dQ, dR, part, RowMap(d),
-                 Parts(d.E, nbe, pick_nsplit(d, dq_part_bytes(d), ws && !(phases & PH_ONE_PART) ? ws_bytes : 0))};
+                 Parts(d.E, nbe, dq_nsplit(d, ws && !(phases & PH_ONE_PART) ? ws_bytes : 0))};
         const int tokw = 256;
         const int smem = DQ_NST * DQ_STAGE_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
         if (smem > 160 * 1024) return hipErrorInvalidValue;

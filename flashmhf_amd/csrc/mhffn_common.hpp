@@ -109,6 +109,10 @@ __device__ __forceinline__ void mfma_result_fence(f32x16& a, f32x16& b, f32x16& 
     // are operands of the statement, so no read of them can be scheduled above it.
     asm volatile("s_nop 15\n\ts_nop 15" : "+v"(a), "+v"(b), "+v"(c));
 }
+__device__ __forceinline__ void mfma_result_fence(f32x16& a, f32x16& b)
+{
+    asm volatile("s_nop 15\n\ts_nop 15" : "+v"(a), "+v"(b));
+}
 // Never pass the same object twice to one fence: the compiler would materialise the extra operands as register copies
 // of the result, and those copies are VALU reads issued before the wait states have passed.
 __device__ __forceinline__ void mfma_result_fence(f32x16& a)
@@ -242,11 +246,18 @@ __device__ __forceinline__ u32x4 lds_read16_async(unsigned addr)
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(IMM));
     return v;
 }
-// Two 4-byte values per lane, 128 bytes apart (one instruction, one LDS operation).
-__device__ __forceinline__ u32x2 lds_read2x4_async(unsigned addr)
+// N 4-byte values per lane, 128 bytes apart (one instruction, one LDS operation).
+template <int N>
+__device__ __forceinline__ u32x2 lds_read_apart_async(unsigned addr)
 {
     u32x2 v;
-    asm volatile("ds_read2_b32 %0, %1 offset1:32" : "=v"(v) : "v"(addr));
+    if constexpr (N == 2) {
+        asm volatile("ds_read2_b32 %0, %1 offset1:32" : "=v"(v) : "v"(addr));
+    } else {
+        unsigned x;
+        asm volatile("ds_read_b32 %0, %1" : "=v"(x) : "v"(addr));
+        v = u32x2{x, 0u};
+    }
     return v;
 }
 // At most N LDS operations of this wave still outstanding; the operands cannot be used above it.  Same conditions as
@@ -445,36 +456,44 @@ struct Parts {
     __device__ __forceinline__ int first(int z) const { return by_nsplit.div(E * nbe * z); }
 };
 
-// Into how many parts the forward and the dQ/dR kernel cut the E * d_e / 32 blocks of a head.  One part needs no partial
-// sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute units a part per idle unit
-// shortens the serial walk over the blocks (one token of the 370M layer: 8 tiles of 121 blocks, 122 us with one part, 15
-// with 32), and every part costs a set of fp32 sums that is written and read back.  Priced in block steps (about 1 us):
-// rounds of CUS workgroups x (blocks of a part + 3 for prologue and epilogue) + 2 for the summing pass + 1 per 1.7 MB of
-// sums; over 29 shapes of 1 to 8,192 rows the pick is within 1 % of the fastest count measured on average, 11 % at worst.
-// Not cut: more experts than one LDS window of gate values holds; and 16,384 rows per head or more, where a head fills
-// a quarter of the chip alone and its results do not depend on how many other heads run beside it.
+// Into how many parts the forward and the dQ/dR kernel cut the blocks of a head, and which of a kernel's tile heights runs.
+// One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute
+// units a part per idle unit shortens the serial walk over the blocks (one token of the 370M layer: 8 tiles of 121 blocks,
+// 122 us with one part, 15 with 32), and every part costs a set of fp32 sums that is written and read back.  Time of a
+// launch in us: rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing
+// pass + 0.6 per MB of sums; a step slows by up to `full` as the chip fills (power).  Over 36 shapes of 1 to 16,384 rows the
+// pick is within 1.5 % of the fastest measured on average, 14 % at worst.
+// Not cut: more experts than one LDS window of gate values holds (bfloat16); and 16,384 rows per head or more, where a head
+// fills a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X
-struct SplitCost {
-    long tile_rows, fixed_steps, sum_steps, bytes_per_step;
-};
-inline int cheapest_nsplit(const SplitCost& c, const Dims& d, long blocks, size_t part_bytes, size_t ws_bytes)
-{
-    const long tiles = ((long)(d.H / d.Hkuv) * d.B * d.S + c.tile_rows - 1) / c.tile_rows * d.Hkuv;
-    if (tiles >= CUS || blocks >= (1 << 24)) return 1;
-    long best = 1, best_cost = blocks + c.fixed_steps;
-    for (long ns = 2; ns <= blocks && ns <= 64 && ns * part_bytes <= ws_bytes; ++ns) {
-        const long cost = (tiles * ns + CUS - 1) / CUS * ((blocks + ns - 1) / ns + c.fixed_steps) + c.sum_steps +
-                          (long)(ns * part_bytes) / c.bytes_per_step;
-        if (cost < best_cost) { best = ns; best_cost = cost; }
-    }
-    return (int)best;
-}
-constexpr SplitCost BF16_COST = {256, 3, 2, 1700000};
 constexpr long SPLIT_ROWS_BELOW = 16384;
-inline int pick_nsplit(const Dims& d, size_t part_bytes, size_t ws_bytes)
+struct Variant {
+    int tile_rows;
+    double step, full;
+};
+struct Pick {
+    int tile_rows, nsplit;
+};
+template <int N>
+inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, bool may_cut, size_t part_bytes, size_t ws_bytes)
 {
-    if (d.E > GATE_WIN || (long)(d.H / d.Hkuv) * d.B * d.S >= SPLIT_ROWS_BELOW) return 1;
-    return cheapest_nsplit(BF16_COST, d, (long)d.E * (d.d_e / JB), part_bytes, ws_bytes);
+    const long rows = (long)(d.H / d.Hkuv) * d.B * d.S;
+    const int most = may_cut && rows < SPLIT_ROWS_BELOW && blocks < (1 << 24) ? (blocks < 64 ? blocks : 64) : 1;
+    const double part_us = part_bytes * 0.6e-6;
+    Pick best{variants[0].tile_rows, 1};
+    double best_us = 0;
+    for (const Variant& v : variants) {
+        const long tiles = (rows + v.tile_rows - 1) / v.tile_rows * d.Hkuv;
+        for (int ns = 1; ns <= most; ++ns) {
+            if (ns > 1 && (ns * part_bytes > ws_bytes || tiles * (ns - 1) >= 2 * CUS)) break;
+            const long wgs = tiles * ns;
+            const double load = wgs <= CUS / 2 ? 0 : wgs >= CUS ? 1 : (wgs - CUS / 2) / (double)(CUS / 2);
+            const double us = (double)((wgs + CUS - 1) / CUS) * ((blocks + ns - 1) / ns * v.step * (1 + v.full * load) + 3) +
+                              (ns > 1 ? 2 + ns * part_us : 0);
+            if (best_us == 0 || us < best_us) { best_us = us; best = Pick{v.tile_rows, ns}; }
+        }
+    }
+    return best;
 }
 
 size_t fwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one part);

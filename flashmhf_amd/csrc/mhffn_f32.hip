@@ -480,15 +480,14 @@ __global__ __launch_bounds__(256) void reduce_f32_kernel(const float* __restrict
     }
 }
 
-// How the work is spread, in block steps of 128 rows (about 5 us): parts of the blocks for the forward and dQ/dR as for
-// bfloat16 (pick_nsplit), 1 step of prologue and epilogue, 1 for the summing pass, 1 per 8 MB of partial sums.
-constexpr SplitCost F32_COST = {128, 1, 1, 8000000};
+// Parts of the blocks for the forward and dQ/dR as for bfloat16 (pick_parts).
+constexpr Variant F32_VARIANTS[] = {{128, 5.0, 0.0}};
 int nbe_of(const Dims& d) { return (d.d_e + JB - 1) / JB; }
 size_t o_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 int parts_of(const Dims& d, size_t part_bytes, size_t ws_bytes)
 {
-    return cheapest_nsplit(F32_COST, d, (long)d.E * nbe_of(d), part_bytes, ws_bytes);
+    return pick_parts(F32_VARIANTS, d, d.E * nbe_of(d), true, part_bytes, ws_bytes).nsplit;
 }
 
 // Token slices of dK/dU/dV: only where the workgroups (two blocks of weight rows each) leave compute units idle.

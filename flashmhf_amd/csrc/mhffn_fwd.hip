@@ -1,8 +1,8 @@
 // Fused multi-head FFN forward for gfx950 (bf16 MFMA, fp32 accumulation).
 //
 // One workgroup (4 waves, one per SIMD, 512 registers each) owns 256 rows of one K/U/V head (tokens of any batch and q-head
-// of its group: RowMap) and all the head's blocks or one part of them (pick_nsplit); a wave owns 64 rows (two column tiles
-// of 32), "tokens" below.  The workgroup streams the K, U, V blocks (32 rows of the E*d_e axis at a time) straight
+// of its group: RowMap) and all the head's blocks or one part of them (pick_parts); a wave owns 64 rows (NT = 2 column tiles
+// of 32), "tokens" below.  With few rows the same code runs on 128 of them, one column tile per wave (FWD_VARIANTS).  The workgroup streams the K, U, V blocks (32 rows of the E*d_e axis at a time) straight
 // from the weight tensors into a ring of LDS stages with asynchronous LDS-direct loads.  Per block and wave:
 //     M^T = K Q^T, N^T = U Q^T               (A = rows of the K/U tiles, B = Q^T held in AGPRs for the whole kernel)
 //     P^T = silu(M^T) * N^T * r_e             (fp32 in the accumulator registers, rounded once to bf16)
@@ -55,24 +55,25 @@ __host__ __device__ constexpr int fwd_younger_reads(int ks, int KS, int CT)
     return n;
 }
 
-template <int DH>
-__global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
+template <int DH, int NT>
+__device__ __forceinline__ void fwd_body(const FwdArgs& p)
 {
-    constexpr int KS = DH / 16, CT = DH / 32, NW = 4, BT = NW * 64;
+    constexpr int KS = DH / 16, CT = DH / 32, NW = 4, WT = 32 * NT, BT = NW * WT;
     constexpr int FILL = 24 / NW;
-    constexpr int NG1 = 4 * KS, NG2 = 4 * CT, NSLOT = NG1 + NG2;   // MFMAs per step
+    constexpr int NG1 = 2 * NT * KS, NG2 = 2 * NT * CT, NSLOT = NG1 + NG2;   // MFMAs per step
     // The first products of a step are written by inline-assembly MFMAs whose results the next step's element-wise code
     // reads without a fence of its own: the NG2 second-product MFMAs issued in between (32 matrix-pipe cycles each) are
     // what covers the 18 wait states an MFMA result needs before a VALU read.
-    static_assert(NG2 >= 8, "the second-product MFMAs of a step must cover the hazard window of its first products");
+    static_assert(NG2 >= 4, "the second-product MFMAs of a step must cover the hazard window of its first products");
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    float* sR = reinterpret_cast<float*>(smem + FWD_RING_B);   // [min(E, GATE_WIN)][BT]: gate values of one expert window
+    // gate values of one expert window: [min(E, GATE_WIN)][NW][64], a wave's WT rows (repeated where that is 32)
+    float* sR = reinterpret_cast<float*>(smem + FWD_RING_B);
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blockIdx.x = tile * Hkuv + kv-head: the head index runs fastest, so each head's weights stay in one XCD's L2
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
-    const int tok0 = tile * BT + wave * 64;                  // this wave's rows of the list (RowMap)
+    const int tok0 = tile * BT + wave * WT;                  // this wave's rows of the list (RowMap)
     const int nbe = p.parts.nbe, E = p.parts.E;
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;   // blocks of this workgroup, counted from blk0
     const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;        // expert of the first, its place in the expert
@@ -94,11 +95,11 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         }
     };
     const int first = tok0 < p.rows.n ? tok0 : p.rows.n - 1;
-    const RowMap::Run run = p.rows.run(hk, first, 64);
+    const RowMap::Run run = p.rows.run(hk, first, WT);
     // The Q rows come from HBM and are the longest wait of the prologue: request them before anything else.
-    bf16x8 q[2][KS];
+    bf16x8 q[NT][KS];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
+    for (int ct = 0; ct < NT; ++ct) {
         int t = tok0 + ct * 32 + l32;
         t = t < p.rows.n ? t : p.rows.n - 1;
         const bf16_t* qr = p.Q + p.rows.tok(run, hk, first, t) * DH + 8 * g;
@@ -106,30 +107,30 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         for (int ks = 0; ks < KS; ++ks) q[ct][ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16);
     }
     issue_block(0, 0);
-    // Gate values of the workgroup's 256 tokens, expert-major [E][BT]: one asynchronous 4-byte LDS-direct load per expert
+    // Gate values of the workgroup's tokens, expert-major: one asynchronous 4-byte LDS-direct load per expert
     // and wave (lane = token, so the 64 values of an instruction are contiguous in LDS).  LDS holds a window of GATE_WIN
     // experts at a time; the first window is issued between block 0 and block 1, so that the wait for block 0 below
     // covers it too, and a layer with more experts restages the tile between two steps of the block loop.
     const float* rrow;
     {
-        int t = tok0 + lane;
+        int t = tok0 + lane % WT;
         t = t < p.rows.n ? t : p.rows.n - 1;
         rrow = p.R + p.rows.gate(run, hk, first, t) * E + ex0;
     }
     auto stage_gates = [&](int e0) {
         const int e1 = e0 + GATE_WIN < nex ? e0 + GATE_WIN : nex;
         for (int e = e0; e < e1; ++e)
-            __builtin_amdgcn_global_load_lds((gptr_t)(rrow + e), (lptr_t)(sR + (e - e0) * BT + wave * 64), 4, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(rrow + e), (lptr_t)(sR + ((e - e0) * NW + wave) * 64), 4, 0, 0);
     };
     stage_gates(0);
     issue_block(1, 1);
     issue_block(2, 2);
 
-    f32x16 oacc[CT][2];
+    f32x16 oacc[CT][NT];
 #pragma unroll
     for (int i = 0; i < CT; ++i)
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
+        for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
             for (int x = 0; x < 16; ++x) oacc[i][ct][x] = 0.0f;
 
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
     const unsigned smem0 = lds_addr(smem);
 
     // consumes M/N of block blk (mc, nc), produces M/N of block blk+1 (mn, nn); ST = blk % FWD_NST
-    auto step = [&](auto st_, int blk, int e, f32x16 (&mc)[2], f32x16 (&nc)[2], f32x16 (&mn)[2], f32x16 (&nn)[2]) {
+    auto step = [&](auto st_, int blk, int e, f32x16 (&mc)[NT], f32x16 (&nc)[NT], f32x16 (&mn)[NT], f32x16 (&nn)[NT]) {
         constexpr int ST = decltype(st_)::value, STN = (ST + 1) % FWD_NST;
         wait_vmcnt<FILL>();   // blocks <= blk+1 have landed (only block blk+2's loads may be in flight)
         __syncthreads();      // ... for every wave; and every wave is done with the stage about to be refilled
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         // ks - 1 (for the second product, long after) and the K/U operands of k-step ks + 2.  LDS operations complete in
         // order, so "at most younger(ks) outstanding" means the operands of k-step ks have arrived; the V^T operands
         // have a full wait of their own in front of the second product, by when they have long landed.
-        u32x2 rvu = lds_read2x4_async(lds_addr(sR + (e & (GATE_WIN - 1)) * BT + wave * 64 + l32));
+        u32x2 rvu = lds_read_apart_async<NT>(lds_addr(sR + ((e & (GATE_WIN - 1)) * NW + wave) * 64 + l32));
         TrOperand av[CT][2];
         u32x4 ak[3], au[3];   // K/U operand ring, two k-steps ahead
         auto request = [&](auto kc) {
@@ -174,12 +175,12 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         // instructions pass while those reads are on their way
         __builtin_amdgcn_sched_barrier(0);
         issue_block(blk + 3, (ST + 3) % FWD_NST);
-        float rinv[2];
-        bf16x8 pt[2][2];
+        float rinv[NT];
+        bf16x8 pt[NT][2];
         float e0 = 0, e1 = 0, xn0 = 0, xn1 = 0;   // carried between the chunks of one element pair
         __builtin_amdgcn_sched_barrier(0);
 
-        // chunk c: third c%3 of element pair c/3; pairs ordered (tile 0, s 0), (tile 1, s 0), (tile 0, s 1), (tile 1, s 1)
+        // chunk c: third c%3 of element pair c/3; pairs ordered s-major ((tile 0, s 0), (tile 1, s 0), (tile 0, s 1), ...)
         // so that each second-product operand P^T[ct][s] is complete well before the slot that consumes it.  The thirds
         // are cut so that their issue times are about equal (a transcendental instruction costs a lone wave about 10
         // cycles, a plain one about 6): 3 plain + 1 transcendental, 2 + 2, 4 + 1.
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         auto chunk = [&](auto c_) {
             constexpr int c = decltype(c_)::value;
             constexpr int pi = c / 3, third = c % 3;
-            constexpr int ct = (pi / 4) % 2, pp = (pi % 4) + 4 * (pi / 8), i0 = 2 * pp, i1 = i0 + 1;
+            constexpr int ct = (pi / 4) % NT, pp = (pi % 4) + 4 * (pi / (4 * NT)), i0 = 2 * pp, i1 = i0 + 1;
             if constexpr (third == 0) {
                 const float t0 = -LOG2E * mc[ct][i0];
                 t1 = -LOG2E * mc[ct][i1];
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         static_for<NSLOT>([&](auto k_) {
             constexpr int k = decltype(k_)::value;
             if constexpr (k < NG1) {
-                constexpr int ks = k / 4, w = k % 4, ct = w >> 1;
+                constexpr int ks = k / (2 * NT), w = k % (2 * NT), ct = w >> 1;
                 if constexpr (w == 0) {
                     if constexpr (ks >= 1 && ks <= CT) request_v(std::integral_constant<int, ks - 1>{});
                     if constexpr (ks + 2 < KS) request(std::integral_constant<int, ks + 2>{});
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
                         // fewer per element.  1/r is clamped to the largest finite float, so a zero gate makes the
                         // denominator at least FLT_MAX, whose reciprocal the hardware flushes to exactly 0.
 #pragma unroll
-                        for (int c2 = 0; c2 < 2; ++c2) {
+                        for (int c2 = 0; c2 < NT; ++c2) {
                             const unsigned bits = rvu[c2];    // (a scalar copy: the cast below must not see a vector element)
                             rinv[c2] = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(__builtin_bit_cast(float, bits)),
                                                                -FLT_MAX_F, FLT_MAX_F);
@@ -234,27 +235,29 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
                     else mfma32_vgpr_acc_bacc(nn[ct], __builtin_bit_cast(bf16x8, au[ks % 3]), q[ct][ks]);
                 }
             } else {
-                constexpr int g2 = k - NG1, s = g2 / (2 * CT), ct = (g2 / CT) % 2, i = g2 % CT;
+                constexpr int g2 = k - NG1, s = g2 / (NT * CT), ct = (g2 / CT) % NT, i = g2 % CT;
                 if constexpr (g2 == 0) {
 #pragma unroll
                     for (int ii = 0; ii < CT; ++ii) lds_tr_wait(av[ii][0], av[ii][1]);
                 }
                 oacc[i][ct] = mfma32(tr_value(av[i][s]), pt[ct][s], oacc[i][ct]);
             }
-            // element-wise chunks: chunk c goes behind slot c * (NSLOT - CT) / 48, so the last one is done before the
-            // CT slots that consume P^T[1][1]
-            static_for<48>([&](auto c_) {
-                if constexpr (decltype(c_)::value * (NSLOT - CT) / 48 == k) chunk(c_);
+            // element-wise chunks: chunk c goes behind slot c * (NSLOT - CT) / NCHUNK, so the last one is done before the
+            // CT slots that consume P^T of the last tile's s = 1
+            constexpr int NCHUNK = 24 * NT;
+            static_for<NCHUNK>([&](auto c_) {
+                if constexpr (decltype(c_)::value * (NSLOT - CT) / NCHUNK == k) chunk(c_);
             });
             __builtin_amdgcn_sched_barrier(0);
         });
         // The first products are written by the matrix pipe long after their instruction has issued.  Keep their
         // registers allocated to the end of the step even when nothing reads them (the phantom block behind an odd
         // count): otherwise the compiler hands them to other values, which the late write then overwrites.
-        asm volatile("" :: "v"(mn[0]), "v"(mn[1]), "v"(nn[0]), "v"(nn[1]));
+        if constexpr (NT == 2) asm volatile("" :: "v"(mn[0]), "v"(mn[NT - 1]), "v"(nn[0]), "v"(nn[NT - 1]));
+        else asm volatile("" :: "v"(mn[0]), "v"(nn[0]));
     };
 
-    f32x16 mA[2], nA[2], mB[2], nB[2];
+    f32x16 mA[NT], nA[NT], mB[NT], nB[NT];
     wait_vmcnt<2 * FILL>();   // all but the fills of blocks 1 and 2: block 0 and the gate values have landed
     __syncthreads();
     {
@@ -262,13 +265,14 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         for (int ks = 0; ks < KS; ++ks) {
             const bf16x8 a = tile_read_rows(smem + FWD_K0, krow, ks, g), u = tile_read_rows(smem + FWD_U0, krow, ks, g);
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct) {
+            for (int ct = 0; ct < NT; ++ct) {
                 if (ks == 0) { mfma32_vgpr_first_bacc(mA[ct], a, q[ct][0]); mfma32_vgpr_first_bacc(nA[ct], u, q[ct][0]); }
                 else { mfma32_vgpr_acc_bacc(mA[ct], a, q[ct][ks]); mfma32_vgpr_acc_bacc(nA[ct], u, q[ct][ks]); }
             }
         }
-        mfma_result_fence(mA[0], nA[0], mA[1]);   // the element-wise code of step 0 reads these results
-        mfma_result_fence(nA[1]);
+        // the element-wise code of step 0 reads these results
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) mfma_result_fence(mA[ct], nA[ct]);
     }
     // Four blocks per trip (one per LDS stage; the two M/N register sets alternate), then the last one to three.  (The
     // step of the last block still computes first products, of the block its prefetch clamped to; nothing reads them.)
@@ -316,20 +320,20 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
     if (p.parts.nsplit > 1) {     // a part of the blocks leaves its sums as they are, fp32, for the pass that adds the parts
         float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH;
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
+        for (int ct = 0; ct < NT; ++ct)
             store_rows_f32<DH>(smem + wave * TILE_B, prow + ct * 32 * DH, p.rows.n - tok0 - ct * 32, lane,
                                [&](auto ic) -> const f32x16& { return oacc[decltype(ic)::value][ct]; });
         return;
     }
     // O^T registers -> O[t][c].  Register 4a+b of row tile i is c = 32i + 8a + 4g + b: a lane owns runs of 4 c of one
     // token, which stored directly would be 8-byte pieces scattered over 32 rows per instruction.  Instead each wave
-    // writes its 64 x d_h tile into a private 16 KB region of the ring (rows of 256 bytes, 16-byte chunk c16 of row r at
+    // writes its rows x d_h tile into a private region of the ring (rows of 256 bytes, 16-byte chunk c16 of row r at
     // chunk c16 ^ (r & 15)), reads it back row-wise and stores whole rows: 16 lanes x 16 bytes per row, 4 rows per
     // instruction.  Only this wave touches the region, and LDS operations of one wave complete in order.
     {
-        unsigned char* otile = smem + wave * (64 * TILE_ROW_B);
+        unsigned char* otile = smem + wave * (WT * TILE_ROW_B);
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
+        for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
             for (int i = 0; i < CT; ++i)
 #pragma unroll
@@ -342,7 +346,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         const int c16 = lane & 15;
         auto store = [&](auto&& address_row) {
 #pragma unroll
-            for (int k = 0; k < 16; ++k) {
+            for (int k = 0; k < 8 * NT; ++k) {
                 const int row = 4 * k + (lane >> 4);
                 if (c16 < DH / 8 && tok0 + row < p.rows.n) {
                     const u32x4 v = *reinterpret_cast<const u32x4*>(otile + row * TILE_ROW_B + ((c16 ^ (row & 15)) << 4));
@@ -354,6 +358,11 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p)
         else store([&](int row) { return p.rows.tok(hk, tok0 + row); });
     }
 }
+
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p) { fwd_body<DH, 2>(p); }
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_fwd_rows128_kernel(FwdArgs p) { fwd_body<DH, 1>(p); }
 
 // Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, eight columns per lane.
 template <int DH>
@@ -377,19 +386,29 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
     *reinterpret_cast<bf16x8*>(p.O + p.rows.tok(hk, r) * DH + c) = v;
 }
 
+// Tiles of 256 rows (64 per wave) where they fill the chip; of 128 (32 per wave) below that: a step then takes 0.6 us
+// instead of 1.0, with 20 % less throughput once every compute unit has one (16,384 tokens of the 370M layer: 342 us with 256
+// rows, 407 with 128; 1,500 tokens in one part: 131 and 85; 733 tokens: 33 and 32 us at each one's best number of parts,
+// of the 128M layer 25.5 and 21.4).  Rows have the same sums, bit for bit, in either.
+constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2}, {128, 0.6, 0.33}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
+static Pick fwd_pick(const Dims& d, size_t ws_bytes)
+{
+    return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), ws_bytes);
+}
 
 template <int DH>
-static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, hipStream_t st)
+static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, hipStream_t st)
 {
-    const int tokw = 256;
-    const int smem = FWD_RING_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
+    const int smem = FWD_RING_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * 256 * (int)sizeof(float);
     if (smem > 160 * 1024) return hipErrorInvalidValue;
-    static LdsOptIn optin;
-    const hipError_t e = ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem);
+    static LdsOptIn optin, optin128;
+    const hipError_t e = tile_rows == 256 ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
+                                          : ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem);
     if (e != hipSuccess) return e;
-    dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
-    hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
+    dim3 grid((unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv), (unsigned)a.parts.nsplit);
+    if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
+    else hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
         dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256), (unsigned)d.Hkuv);
         hipLaunchKernelGGL((mhffn_fwd_sum_kernel<DH>), sgrid, dim3(256), 0, st, a);
@@ -399,7 +418,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, hipStream_t st)
 
 size_t fwd_workspace_bytes_bf16(const Dims& d)
 {
-    const int ns = pick_nsplit(d, fwd_part_bytes(d), ~(size_t)0);
+    const int ns = fwd_pick(d, ~(size_t)0).nsplit;
     return ns > 1 ? ns * fwd_part_bytes(d) : 0;
 }
 
@@ -407,13 +426,13 @@ hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const vo
                            void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases)
 {
     if (!(phases & PH_FWD_MAIN)) return hipSuccess;
-    const int nsplit = pick_nsplit(d, fwd_part_bytes(d), ws && !(phases & PH_ONE_PART) ? ws_bytes : 0);
+    const Pick pick = fwd_pick(d, ws && !(phases & PH_ONE_PART) ? ws_bytes : 0);
     FwdArgs a{(const bf16_t*)Q, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V,           R,
-              (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, nsplit)};
+              (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, pick.nsplit)};
     switch (d.d_h) {
-        case 64: return launch_fwd_t<64>(a, d, st);
-        case 96: return launch_fwd_t<96>(a, d, st);
-        case 128: return launch_fwd_t<128>(a, d, st);
+        case 64: return launch_fwd_t<64>(a, d, pick.tile_rows, st);
+        case 96: return launch_fwd_t<96>(a, d, pick.tile_rows, st);
+        case 128: return launch_fwd_t<128>(a, d, pick.tile_rows, st);
     }
     return hipErrorInvalidValue;
 }
