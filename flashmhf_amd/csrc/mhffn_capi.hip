@@ -220,15 +220,44 @@ static int check_gate_dims(const mhffn_dims* d)
     return MHFFN_OK;
 }
 
-int mhffn_gate_fwd(const void* X, const float* norm_weight, float eps, const float* router, void* Qn, float* R,
-                   const mhffn_dims* dims, void* stream)
+static bool param_dtypes_ok(int norm_dtype, int router_dtype)
+{
+    return (norm_dtype == MHFFN_DTYPE_BF16 || norm_dtype == MHFFN_DTYPE_F32) &&
+           (router_dtype == MHFFN_DTYPE_BF16 || router_dtype == MHFFN_DTYPE_F32);
+}
+
+int mhffn_gate_fwd_typed(const void* X, const void* norm_weight, int norm_dtype, float eps, const void* router, int router_dtype,
+                         void* Qn, float* R, const mhffn_dims* dims, void* stream)
 {
     const int rc = check_gate_dims(dims);
     if (rc != MHFFN_OK) return rc;
+    if (!param_dtypes_ok(norm_dtype, router_dtype)) return MHFFN_ERR_DTYPE;
     if (!X || !router || !R || (norm_weight && !Qn)) return MHFFN_ERR_NULL_POINTER;
     if (!aligned16(X) || !aligned16(Qn) || !aligned16(R) || !aligned16(router) || !aligned16(norm_weight))
         return MHFFN_ERR_ALIGNMENT;
-    return mhffn::launch_gate_fwd(X, norm_weight, eps, router, Qn, R, to_dims(dims), (hipStream_t)stream) == hipSuccess
+    return mhffn::launch_gate_fwd(X, norm_weight, norm_dtype == MHFFN_DTYPE_BF16, eps, router, router_dtype == MHFFN_DTYPE_BF16, Qn, R,
+                                  to_dims(dims), (hipStream_t)stream) == hipSuccess
+               ? MHFFN_OK
+               : MHFFN_ERR_LAUNCH;
+}
+
+int mhffn_gate_fwd(const void* X, const float* norm_weight, float eps, const float* router, void* Qn, float* R,
+                   const mhffn_dims* dims, void* stream)
+{
+    return mhffn_gate_fwd_typed(X, norm_weight, MHFFN_DTYPE_F32, eps, router, MHFFN_DTYPE_F32, Qn, R, dims, stream);
+}
+
+static int gate_bwd(const void* X, const void* norm_weight, int norm_dtype, float eps, const void* router, int router_dtype,
+                    const void* dQ, int dq_token_layout, const float* dR, void* dX, void* d_norm_weight, void* d_router, void* workspace,
+                    const mhffn_dims* dims, void* stream)
+{
+    if (dq_token_layout != MHFFN_TOKENS_BHSD && dq_token_layout != MHFFN_TOKENS_BSHD) return MHFFN_ERR_SHAPE;
+    if (!X || !router || !dQ || !dR || !dX || !d_router || (norm_weight && !d_norm_weight)) return MHFFN_ERR_NULL_POINTER;
+    const void* ptrs[] = {X, norm_weight, router, dQ, dR, dX, d_norm_weight, d_router, workspace};
+    for (const void* p : ptrs)
+        if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
+    return mhffn::launch_gate_bwd(X, norm_weight, norm_dtype == MHFFN_DTYPE_BF16, eps, router, router_dtype == MHFFN_DTYPE_BF16, dQ,
+                                  dq_token_layout, dR, dX, d_norm_weight, d_router, workspace, to_dims(dims), (hipStream_t)stream) == hipSuccess
                ? MHFFN_OK
                : MHFFN_ERR_LAUNCH;
 }
@@ -239,15 +268,25 @@ int mhffn_gate_bwd(const void* X, const float* norm_weight, float eps, const flo
 {
     const int rc = check_gate_dims(dims);
     if (rc != MHFFN_OK) return rc;
-    if (dq_token_layout != MHFFN_TOKENS_BHSD && dq_token_layout != MHFFN_TOKENS_BSHD) return MHFFN_ERR_SHAPE;
-    if (!X || !router || !dQ || !dR || !dX || !d_router || (norm_weight && !d_norm_weight)) return MHFFN_ERR_NULL_POINTER;
-    const void* ptrs[] = {X, norm_weight, router, dQ, dR, dX, d_norm_weight, d_router};
-    for (const void* p : ptrs)
-        if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
-    return mhffn::launch_gate_bwd(X, norm_weight, eps, router, dQ, dq_token_layout, dR, dX, d_norm_weight, d_router,
-                                  to_dims(dims), (hipStream_t)stream) == hipSuccess
-               ? MHFFN_OK
-               : MHFFN_ERR_LAUNCH;
+    return gate_bwd(X, norm_weight, MHFFN_DTYPE_F32, eps, router, MHFFN_DTYPE_F32, dQ, dq_token_layout, dR, dX, d_norm_weight, d_router,
+                    nullptr, dims, stream);
+}
+
+size_t mhffn_gate_bwd_workspace_bytes(const mhffn_dims* dims)
+{
+    return check_gate_dims(dims) == MHFFN_OK ? mhffn::gate_bwd_workspace_bytes(to_dims(dims)) : 0;
+}
+
+int mhffn_gate_bwd_into(const void* X, const void* norm_weight, int norm_dtype, float eps, const void* router, int router_dtype,
+                        const void* dQ, int dq_token_layout, const float* dR, void* dX, void* d_norm_weight, void* d_router, void* workspace,
+                        size_t workspace_bytes, const mhffn_dims* dims, void* stream)
+{
+    const int rc = check_gate_dims(dims);
+    if (rc != MHFFN_OK) return rc;
+    if (!param_dtypes_ok(norm_dtype, router_dtype)) return MHFFN_ERR_DTYPE;
+    if (!workspace || workspace_bytes < mhffn::gate_bwd_workspace_bytes(to_dims(dims))) return MHFFN_ERR_WORKSPACE;
+    return gate_bwd(X, norm_weight, norm_dtype, eps, router, router_dtype, dQ, dq_token_layout, dR, dX, d_norm_weight, d_router,
+                    workspace, dims, stream);
 }
 
 }  // extern "C"

@@ -516,10 +516,13 @@ hipError_t launch_bwd_f32(const void* Q, const void* K, const void* U, const voi
                           const Dims& d, hipStream_t st, int phases);
 
 // Head prologue (mhffn_gate.hip): per-head RMSNorm + expert gate over [B, S, H, d_h] bf16 rows; d_h 64/96/128, E <= 64.
-hipError_t launch_gate_fwd(const void* X, const float* Wn, float eps, const float* Wr, void* Qn, float* R, const Dims& d,
-                           hipStream_t st);
-hipError_t launch_gate_bwd(const void* X, const float* Wn, float eps, const float* Wr, const void* dQ, int dq_tokmaj,
-                           const float* dR, void* dX, float* dWn, float* dWr, const Dims& d, hipStream_t st);
+// Wn, Wr (and dWn, dWr where there is a workspace) are float or, with wn_bf16, wr_bf16, bfloat16.  Without a workspace the backward adds
+// to float dWn, dWr; with one (gate_bwd_workspace_bytes) it overwrites them.
+hipError_t launch_gate_fwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, void* Qn, float* R,
+                           const Dims& d, hipStream_t st);
+size_t gate_bwd_workspace_bytes(const Dims& d);
+hipError_t launch_gate_bwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, const void* dQ,
+                           int dq_tokmaj, const float* dR, void* dX, void* dWn, void* dWr, void* ws, const Dims& d, hipStream_t st);
 
 // Bits of the `phases` argument of the launch functions (the values of MHFFN_FWD_*, MHFFN_BWD_*, MHFFN_ONE_PART in
 // include/mhffn.h).

@@ -14,36 +14,53 @@
 //   * backward: dy += dz router^T (B = dz straight from the logits' registers: the router rows are fed in row_perm32
 //     order, exactly as the main kernels chain their products) and d_router += y^T dz (contraction over tokens = lanes:
 //     y and dz go through a wave-private LDS tile and come back with transposing reads).
-// d_router and d_norm_weight are summed over all tokens: per-wave partial sums in registers, one atomic add per wave
-// and element at the end (the caller passes zero-filled or to-be-accumulated buffers).
+// d_router and d_norm_weight are summed over all tokens: partial sums per wave, added up per workgroup, then either one atomic
+// add per workgroup and element (mhffn_gate_bwd: the caller passes zero-filled or to-be-accumulated buffers) or a partial
+// sum in memory that a second pass adds in order and writes in the parameters' type (mhffn_gate_bwd_into).
 #include "mhffn_common.hpp"
 
 namespace mhffn {
 
 struct GateArgs {
     const bf16_t* X;     // [B, S, H, DH]
-    const float* Wn;     // [H, DH] (NORM only)
-    const float* Wr;     // [H, DH, E]
+    const void* Wn;      // [H, DH] (NORM only), float or bfloat16 (wn_bf16)
+    const void* Wr;      // [H, DH, E], float or bfloat16 (wr_bf16)
     bf16_t* Qn;          // [B, S, H, DH] (NORM only)
     float* R;            // [B, H, S, E]
     const bf16_t* dQ;    // gradient of y, rows addressed through dq_tokmaj
     const float* dR;     // [B, H, S, E]
     bf16_t* dX;          // [B, S, H, DH]
-    float* dWn;          // [H, DH], accumulated
-    float* dWr;          // [H, DH, E], accumulated
-    int B, H, S, E, tpw, dq_tokmaj;
+    float* dWn;          // [H, DH] and
+    float* dWr;          // [H, DH, E], accumulated by atomic adds, or (part != null) not used:
+    float* part;         // [H][workgroups of a head][DH * E + DH] sums of d_router, d_norm_weight over a workgroup's tokens
+    int B, H, S, E, tpw, dq_tokmaj, wn_bf16, wr_bf16;
     float eps;
 };
 
+__device__ __forceinline__ float param(const void* p, long i, int bf16)
+{
+    return bf16 ? (float)static_cast<const bf16_t*>(p)[i] : static_cast<const float*>(p)[i];
+}
 __device__ __forceinline__ float bf_even(unsigned w) { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float bf_odd(unsigned w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 __device__ __forceinline__ float bf_at(const u32x4& v, int j) { return (j & 1) ? bf_odd(v[j >> 1]) : bf_even(v[j >> 1]); }
+
+template <int DH, int NT, typename T>
+__device__ void stage_router_rows(const T* Wr, int E, unsigned char* dst);
+template <int DH, int NT, typename T>
+__device__ void stage_router_cols(const T* Wr, int E, unsigned char* dst);
 
 // Router slice of head h as MFMA A operands in LDS.
 //   part 0/1 (hi/lo), expert tile nt, k-step ks, lane (rho, g): router[(2ks+g)*8 + j][nt*32 + row_perm32(rho)], j = 0..7
 // so that register 8s + kk of lane half g of the product holds expert nt*32 + 16s + 8g + kk.
 template <int DH, int NT>
-__device__ __forceinline__ void stage_router_rows(const float* Wr, int E, unsigned char* dst)
+__device__ __forceinline__ void stage_router_rows(const void* Wr, long w0, int bf16, int E, unsigned char* dst)
+{
+    if (bf16) stage_router_rows<DH, NT>(static_cast<const bf16_t*>(Wr) + w0, E, dst);
+    else stage_router_rows<DH, NT>(static_cast<const float*>(Wr) + w0, E, dst);
+}
+template <int DH, int NT, typename T>
+__device__ __forceinline__ void stage_router_rows(const T* Wr, int E, unsigned char* dst)
 {
     constexpr int KS = DH / 16;
     for (int idx = threadIdx.x; idx < NT * KS * 64; idx += blockDim.x) {
@@ -52,7 +69,7 @@ __device__ __forceinline__ void stage_router_rows(const float* Wr, int E, unsign
         bf16x8 hi, lo;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float v = e < E ? Wr[(long)(k0 + j) * E + e] : 0.0f;
+            const float x = (float)Wr[(long)(k0 + j) * E + (e < E ? e : 0)], v = e < E ? x : 0.0f;
             hi[j] = (bf16_t)v;
             lo[j] = (bf16_t)(v - (float)hi[j]);
         }
@@ -64,7 +81,13 @@ __device__ __forceinline__ void stage_router_rows(const float* Wr, int E, unsign
 // Router slice as A operands of dy^T [d_h x tokens] = router [d_h x E] dz^T: column tile ct, k-step q = 2nt + s,
 // lane (rho, g): router[ct*32 + row_perm32(rho)][nt*32 + 16s + 8g + j]  (bf16, high part only: dy is rounded to bf16).
 template <int DH, int NT>
-__device__ __forceinline__ void stage_router_cols(const float* Wr, int E, unsigned char* dst)
+__device__ __forceinline__ void stage_router_cols(const void* Wr, long w0, int bf16, int E, unsigned char* dst)
+{
+    if (bf16) stage_router_cols<DH, NT>(static_cast<const bf16_t*>(Wr) + w0, E, dst);
+    else stage_router_cols<DH, NT>(static_cast<const float*>(Wr) + w0, E, dst);
+}
+template <int DH, int NT, typename T>
+__device__ __forceinline__ void stage_router_cols(const T* Wr, int E, unsigned char* dst)
 {
     constexpr int CT = DH / 32;
     for (int idx = threadIdx.x; idx < CT * 2 * NT * 64; idx += blockDim.x) {
@@ -72,7 +95,10 @@ __device__ __forceinline__ void stage_router_cols(const float* Wr, int E, unsign
         const int col = ct * 32 + row_perm32(ln & 31), e0 = q * 16 + 8 * (ln >> 5);
         bf16x8 v;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (bf16_t)(e0 + j < E ? Wr[(long)col * E + e0 + j] : 0.0f);
+        for (int j = 0; j < 8; ++j) {
+            const float x = (float)Wr[(long)col * E + (e0 + j < E ? e0 + j : 0)];
+            v[j] = (bf16_t)(e0 + j < E ? x : 0.0f);
+        }
         *reinterpret_cast<bf16x8*>(dst + idx * 16) = v;
     }
 }
@@ -93,6 +119,8 @@ struct GateTile {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) xr[ks] = *reinterpret_cast<const u32x4*>(xrow + (2 * ks + g) * 8);
     }
+    // FENCED: one k-step's LDS reads at a time (the backward has no registers for all of them at once)
+    template <bool FENCED>
     __device__ __forceinline__ void normalise(const float* sW, int g)
     {
         if constexpr (NORM) {
@@ -113,6 +141,7 @@ struct GateTile {
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
                     y[ks][j] = (bf16_t)((bf_at(xr[ks], j) * rstd) * (j < 4 ? w0[j & 3] : w1[j & 3]));
+                if constexpr (FENCED) __builtin_amdgcn_sched_barrier(0);
             }
         } else {
             rstd = 1.0f;
@@ -120,6 +149,7 @@ struct GateTile {
             for (int ks = 0; ks < KS; ++ks) y[ks] = __builtin_bit_cast(bf16x8, xr[ks]);
         }
     }
+    template <bool FENCED>
     __device__ __forceinline__ void gate(const unsigned char* sA, int lane, int g, int E)
     {
         f32x16 acc[NT];
@@ -128,13 +158,17 @@ struct GateTile {
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[nt][i] = 0.0f;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+        for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 const unsigned char* a = sA + ((nt * KS + ks) * 64 + lane) * 16;
                 acc[nt] = mfma32(*reinterpret_cast<const bf16x8*>(a), y[ks], acc[nt]);
                 acc[nt] = mfma32(*reinterpret_cast<const bf16x8*>(a + NT * KS * 1024), y[ks], acc[nt]);
             }
+            if constexpr (FENCED) {
+                if (ks % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         sum = 0.0f;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
@@ -165,9 +199,9 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
     float* rtile = sW + DH + wave * (TILE_B / 4);
     const int h = blockIdx.y, b = blockIdx.z;
 
-    stage_router_rows<DH, NT>(p.Wr + (long)h * DH * p.E, p.E, smem);
+    stage_router_rows<DH, NT>(p.Wr, (long)h * DH * p.E, p.wr_bf16, p.E, smem);
     if constexpr (NORM)
-        for (int i = threadIdx.x; i < DH; i += blockDim.x) sW[i] = p.Wn[h * DH + i];
+        for (int i = threadIdx.x; i < DH; i += blockDim.x) sW[i] = param(p.Wn, h * DH + i, p.wn_bf16);
     __syncthreads();
 
     const int ntiles = (p.S + 31) / 32;
@@ -180,7 +214,7 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
         GateTile<DH, NT, NORM> T;
         T.eps_ = p.eps;
         T.load(p.X + row, g);
-        T.normalise(sW, g);
+        T.template normalise<false>(sW, g);
         if constexpr (NORM) {
             if (valid) {
 #pragma unroll
@@ -188,7 +222,7 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
                     *reinterpret_cast<bf16x8*>(p.Qn + row + (2 * ks + g) * 8) = T.y[ks];
             }
         }
-        T.gate(smem, lane, g, p.E);
+        T.template gate<false>(smem, lane, g, p.E);
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -204,18 +238,30 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 
 // ---- backward -------------------------------------------------------------------------------------------------------
 // LDS: router rows (hi, lo) | router columns | norm weight | per wave: y tile (8 KB) + dz tile (8 KB), both in the
-// swizzled 32 x 256-byte tile layout of the main kernels so the transposing reads can be shared.
-// One wave per SIMD (the register partial sums leave no room for a second), so the next tile's rows are requested
-// before the current tile's arithmetic starts; a wave takes enough consecutive tiles that the launch is one wave per
-// SIMD of the chip where the problem allows, which also bounds the number of atomic adds per element.
-// The per-wave region doubles as the staging area of the end-of-kernel reductions over the four waves: one expert
-// tile of d_router partials ((d_h/32) x 16 x 64 floats <= 16 KB) or a 64 x 65 float transpose of the d_norm_weight
-// partials; a [4][128] float array for the latter's cross-wave sums follows the regions.
-constexpr int GATE_WAVE_REGION_B = 2 * TILE_B + 1024;
-constexpr size_t gate_bwd_smem(int DH, int NT)
+// swizzled 32 x 256-byte tile layout of the main kernels so the transposing reads can be shared | [waves][128] floats for
+// the sums across waves.  A wave takes enough consecutive tiles that the launch fills the chip once, which also bounds
+// the number of partial sums.
+//
+// Up to 32 experts (NT = 1) eight waves, two per SIMD, and nothing but sums in few registers lives across tiles: the waves'
+// y and dz tiles are contracted together, each wave keeping one column tile of d_router (16 registers) over the tokens
+// of several waves, two barriers per tile; the products d * u of d_norm_weight pass through the wave's LDS region a half at a
+// time and are added up down the columns (4 values per 64 columns).  What that frees holds the next tile's rows of x, requested
+// behind the contraction, while dR and dQ of a tile are requested at its top and used half a trip later.  One wave per SIMD
+// with all sums in registers, ~2,400 instructions per tile, a quarter of them register moves, took 150 us on 32,768 tokens of
+// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 128 us
+// (3.5 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
+// More experts (NT = 2) have twice the d_router operands: four waves, one per SIMD, all sums in registers, and the next
+// tile's rows requested before the current tile's arithmetic starts.
+template <int NT>
+constexpr int gate_bwd_waves() { return NT == 1 ? 8 : 4; }
+constexpr int GATE_WAVE_REGION_B = 2 * TILE_B + 1024;      // NT = 2: also a 64 x 65 float transpose; NT = 1: 2 * TILE_B
+template <int NT>
+constexpr int gate_bwd_region() { return NT == 1 ? 2 * TILE_B : GATE_WAVE_REGION_B; }
+template <int NT>
+constexpr size_t gate_bwd_smem(int DH)
 {
-    return (size_t)2 * NT * (DH / 16) * 1024 + (size_t)(DH / 32) * 2 * NT * 1024 + DH * 4 + 4 * GATE_WAVE_REGION_B +
-           4 * 128 * 4;
+    return (size_t)2 * NT * (DH / 16) * 1024 + (size_t)(DH / 32) * 2 * NT * 1024 + DH * 4 +
+           gate_bwd_waves<NT>() * (gate_bwd_region<NT>() + 128 * 4);
 }
 
 // Transposed operand (column tile ct, k-half s) of a swizzled tile.  Only column tile 0's two lane offsets are kept in
@@ -236,9 +282,14 @@ __device__ __forceinline__ bf16x8 tile_cols(const unsigned char* tile, const TrL
 }
 
 template <int DH, int NT, bool NORM>
-__global__ __launch_bounds__(256) void mhffn_gate_bwd_kernel(GateArgs p)
+__global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
 {
-    constexpr int KS = DH / 16, CT = DH / 32;
+    constexpr int KS = DH / 16, CT = DH / 32, NW = gate_bwd_waves<NT>(), REGION_B = gate_bwd_region<NT>();
+    constexpr bool AHEAD = NT > 1;                              // rows requested one tile ahead; d_norm_weight in registers
+    constexpr int NHALF = (DH + 63) / 64;
+    // NT = 1: wave w sums column tile w % CT of d_router over the TPG token tiles of its group w / CT of the workgroup's
+    // waves (waves beyond GROUPS * CT none); NT = 2: a wave sums all of it over its own tiles
+    constexpr int GROUPS = NW / CT, TPG = NW / GROUPS, WCT = AHEAD ? CT : 1;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* sA = smem;                                   // logits operands
     unsigned char* sC = sA + 2 * NT * KS * 1024;                // dy operands
@@ -246,61 +297,106 @@ __global__ __launch_bounds__(256) void mhffn_gate_bwd_kernel(GateArgs p)
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: tile counters and tile bases stay scalar
     unsigned char* regions = reinterpret_cast<unsigned char*>(sW + DH);
-    unsigned char* ytile = regions + wave * GATE_WAVE_REGION_B;
+    unsigned char* ytile = regions + wave * REGION_B;
     unsigned char* ztile = ytile + TILE_B;
     const int h = blockIdx.y, b = blockIdx.z;
 
-    stage_router_rows<DH, NT>(p.Wr + (long)h * DH * p.E, p.E, sA);
-    stage_router_cols<DH, NT>(p.Wr + (long)h * DH * p.E, p.E, sC);
+    stage_router_rows<DH, NT>(p.Wr, (long)h * DH * p.E, p.wr_bf16, p.E, sA);
+    stage_router_cols<DH, NT>(p.Wr, (long)h * DH * p.E, p.wr_bf16, p.E, sC);
     if constexpr (NORM)
-        for (int i = threadIdx.x; i < DH; i += blockDim.x) sW[i] = p.Wn[h * DH + i];
+        for (int i = threadIdx.x; i < DH; i += blockDim.x) sW[i] = param(p.Wn, h * DH + i, p.wn_bf16);
     // the dz tile's chunks beyond the experts in use are read by nobody, but columns e >= E inside a used chunk are:
     // they are written as zeros every tile, so nothing needs clearing here
     __syncthreads();
 
-    const TrLane<1> trl = make_tr_lane<1, 8, 4>(lane);
     const TokRows dqrows = tok_rows(p.dq_tokmaj, b, h, p.H, p.S);
-    f32x16 wacc[CT][NT];            // d_router partial: rows = columns of y, cols = experts
-    float dwacc[KS][8];             // d_norm_weight partial for the lane's own columns
+    f32x16 wacc[WCT][NT];           // d_router partial: rows = columns of y, cols = experts
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < WCT; ++ct)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) wacc[ct][nt][i] = 0.0f;
+    // d_norm_weight partial: for the lane's own columns, or columns 64 h + 4 (lane % 16) .. +3 over rows lane / 16 + 4k
+    [[maybe_unused]] float dwacc[KS][8];
+    [[maybe_unused]] f32x4 dwcol[NHALF];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
         for (int j = 0; j < 8; ++j) dwacc[ks][j] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NHALF; ++i) dwcol[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     const int ntiles = (p.S + 31) / 32;
-    const int tile0 = (blockIdx.x * 4 + wave) * p.tpw;
+    const int tile0 = (blockIdx.x * NW + wave) * p.tpw;
     const int tile1 = min(tile0 + p.tpw, ntiles);
-    // rows of the tile after the current one, requested one iteration ahead
     u32x4 nx[KS], ndq[KS];
     float ngr[NT * 16];
-    auto request = [&](int tile) {
-        const int t = tile * 32 + l32;
+    auto request_x = [&](int tile, int lane) {
+        const int l32 = lane & 31, g = lane >> 5, t = tile * 32 + l32;
+        const bf16_t* xrow = p.X + (((long)b * p.S + (t < p.S ? t : p.S - 1)) * p.H + h) * DH;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) nx[ks] = *reinterpret_cast<const u32x4*>(xrow + (2 * ks + g) * 8);
+    };
+    auto request = [&](int tile, int lane) {
+        const int l32 = lane & 31, g = lane >> 5, t = tile * 32 + l32;
         const bool valid = t < p.S;
         const int tc = valid ? t : p.S - 1;
-        const bf16_t* xrow = p.X + (((long)b * p.S + tc) * p.H + h) * DH;
         const bf16_t* dqrow = p.dQ + (dqrows.base + (long)tc * dqrows.stride) * DH;
         const float* dblock = p.dR + (((long)b * p.H + h) * p.S + tile * 32) * p.E;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            nx[ks] = *reinterpret_cast<const u32x4*>(xrow + (2 * ks + g) * 8);
-            ndq[ks] = *reinterpret_cast<const u32x4*>(dqrow + (2 * ks + g) * 8);
-        }
         // the tile's [32][E] block of dR is contiguous: dword k*64 + lane of it, zero past the last token
         const int lim = min(32, p.S - tile * 32) * p.E;
 #pragma unroll
-        for (int k = 0; k < NT * 16; ++k) ngr[k] = k * 64 + lane < lim ? dblock[k * 64 + lane] : 0.0f;
+        for (int k = 0; k < NT * 16; ++k) {
+            const float v = dblock[min(k * 64 + lane, lim - 1)];
+            ngr[k] = k * 64 + lane < lim ? v : 0.0f;
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) ndq[ks] = *reinterpret_cast<const u32x4*>(dqrow + (2 * ks + g) * 8);
     };
-    if (tile0 < tile1) request(tile0);
-    for (int tile = tile0; tile < tile1; ++tile) {
+    if (tile0 < tile1) {
+        request_x(tile0, lane);
+        if (AHEAD) request(tile0, lane);
+    }
+    for (int tile = tile0; tile < (AHEAD ? tile1 : tile0 + p.tpw); ++tile) {
+        // (The lane number of this trip is hidden from the compiler, or it keeps the dozens of addresses below, which cost
+        // an instruction or two each, in registers across the loop: with two waves per SIMD there are none to spare.)
+        int lane = threadIdx.x & 63;
+        if constexpr (!AHEAD) asm volatile("" : "+v"(lane));
+        const int l32 = lane & 31, g = lane >> 5;
+        const TrLane<1> trl = make_tr_lane<1, 8, 4>(lane);
+        // Lane parts of the LDS addresses: row l32 of the y and dz tiles, of the product tile, and this lane's reads of the
+        // latter (16 bytes of row lane / 16); the rest of an address is a constant that the swizzle's exclusive-or and the
+        // row pitch leave alone.
+        const int yrow = l32 * TILE_ROW_B + ((g ^ swz16(l32)) << 4), prow = l32 * TILE_ROW_B + (((2 * g) ^ (l32 & 15)) << 4);
+        const int pread = (lane >> 4) * TILE_ROW_B + (((lane & 15) ^ (lane >> 4)) << 4);
+        // NT = 1: this tile's token contraction, two barriers around it (every wave of the workgroup passes them p.tpw times)
+        auto contract = [&]() {
+            __syncthreads();
+            const int grp = wave / CT, ct = wave - grp * CT;
+            if (grp < GROUPS) {
+                for (int k = 0; k < TPG; ++k) {
+                    const unsigned char* yt = regions + (grp * TPG + k) * REGION_B;
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+                        wacc[0][0] = mfma32(tile_cols(yt, trl, ct, s), tile_cols(yt + TILE_B, trl, 0, s), wacc[0][0]);
+                }
+            }
+            __syncthreads();
+        };
+        if (!AHEAD && tile >= tile1) {      // no tile left for this wave: it adds zeros
+            const u32x4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<u32x4*>(ytile + (yrow ^ (ks << 5))) = zero;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) *reinterpret_cast<u32x4*>(ztile + (yrow ^ (s << 5))) = zero;
+            contract();
+            continue;
+        }
         const int t = tile * 32 + l32;
         const bool valid = t < p.S;
         const long row = (((long)b * p.S + (valid ? t : p.S - 1)) * p.H + h) * DH;
+        if (!AHEAD) request(tile, lane);
         GateTile<DH, NT, NORM> T;
         T.eps_ = p.eps;
         u32x4 dqr[KS];
@@ -311,7 +407,7 @@ __global__ __launch_bounds__(256) void mhffn_gate_bwd_kernel(GateArgs p)
             dqr[ks] = ndq[ks];
         }
         // dR goes lane-major -> token-major through the (currently idle) dz tile
-        {
+        auto exchange_dr = [&]() {
             float* rt = reinterpret_cast<float*>(ztile);
 #pragma unroll
             for (int k = 0; k < NT * 16; ++k) rt[k * 64 + lane] = ngr[k];
@@ -320,19 +416,26 @@ __global__ __launch_bounds__(256) void mhffn_gate_bwd_kernel(GateArgs p)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const int e = nt * 32 + 16 * (i >> 3) + 8 * g + (i & 7);
-                    gr[nt][i] = e < p.E ? rt[l32 * p.E + e] : 0.0f;
+                    const float v = rt[min(l32 * p.E + e, 1024 * NT - 1)];
+                    gr[nt][i] = e < p.E ? v : 0.0f;
                 }
+        };
+        if (AHEAD) exchange_dr();
+        if (AHEAD && tile + 1 < tile1) {
+            request_x(tile + 1, lane);
+            request(tile + 1, lane);
         }
-        if (tile + 1 < tile1) request(tile + 1);
-        T.normalise(sW, g);
+        if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);
+        T.template normalise<!AHEAD>(sW, g);
         if (!valid) {   // rows past the end contribute nothing to the sums over tokens
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) T.y[ks] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            *reinterpret_cast<bf16x8*>(ytile + l32 * TILE_ROW_B + (((2 * ks + g) ^ swz16(l32)) << 4)) = T.y[ks];
-        T.gate(sA, lane, g, p.E);
+            *reinterpret_cast<bf16x8*>(ytile + (yrow ^ (ks << 5))) = T.y[ks];
+        T.template gate<!AHEAD>(sA, lane, g, p.E);
+        if (!AHEAD) exchange_dr();      // (requested at the top of the trip)
 
         // R = s * inv; d s = (dR - [sum >= 1e-20] sum_e dR R) * inv; d z = d s * s (1 - s)
         float dot = 0.0f;
@@ -354,41 +457,88 @@ __global__ __launch_bounds__(256) void mhffn_gate_bwd_kernel(GateArgs p)
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int s = 0; s < 2; ++s)
-                *reinterpret_cast<bf16x8*>(ztile + l32 * TILE_ROW_B + (((4 * nt + 2 * s + g) ^ swz16(l32)) << 4)) =
-                    dzb[nt][s];
+                *reinterpret_cast<bf16x8*>(ztile + (yrow ^ ((4 * nt + 2 * s) << 4))) = dzb[nt][s];
 
-        // dy^T = router dz^T, then the RMSNorm backward on the lane's own half row
-        f32x16 dy[CT];
+        // The phases of a tile are fenced, and each unpacks the rows of x anew: left to itself the compiler keeps the 64
+        // unpacked values (and their products with rstd) from one phase to the next, which two waves per SIMD have no
+        // registers for.
+        auto next_phase = [&]() {
+            if constexpr (!AHEAD) {
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
+                for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(T.xr[ks]));
+            }
+        };
+        next_phase();
+        // d_router += y^T dz over this tile's tokens
+        if constexpr (!AHEAD) {
+            contract();
+            request_x(min(tile + 1, ntiles - 1), lane);     // (always: behind a branch the waits for dq below would be for x too)
+        } else
 #pragma unroll
-            for (int i = 0; i < 16; ++i) dy[ct][i] = 0.0f;
+        for (int s = 0; s < 2; ++s) {
+            bf16x8 bz[NT];
 #pragma unroll
-            for (int q = 0; q < 2 * NT; ++q)
-                dy[ct] = mfma32(*reinterpret_cast<const bf16x8*>(sC + ((ct * 2 * NT + q) * 64 + lane) * 16),
-                                dzb[q >> 1][q & 1], dy[ct]);
+            for (int nt = 0; nt < NT; ++nt) bz[nt] = tile_cols(ztile, trl, nt, s);
+#pragma unroll
+            for (int ct = 0; ct < WCT; ++ct) {
+                const bf16x8 ay = tile_cols(ytile, trl, ct, s);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) wacc[ct][nt] = mfma32(ay, bz[nt], wacc[ct][nt]);
+            }
         }
+
+        next_phase();
+        // dy^T = router dz^T, then the RMSNorm backward on the lane's own half row
+        // (one column tile of dy at a time)
+        f32x16 dy;
         float du[KS][8];
         float cpart = 0.0f;
+        static_for<KS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value, ct = ks / 2;
+            if constexpr (ks % 2 == 0) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            [[maybe_unused]] f32x4 w0, w1;
+                for (int i = 0; i < 16; ++i) dy[i] = 0.0f;
+#pragma unroll
+                for (int q = 0; q < 2 * NT; ++q)
+                    dy = mfma32(*reinterpret_cast<const bf16x8*>(sC + ((ct * 2 * NT + q) * 64 + lane) * 16), dzb[q >> 1][q & 1], dy);
+            }
+            [[maybe_unused]] f32x4 w0, w1, prod[2];
             if constexpr (NORM) {
                 w0 = *reinterpret_cast<const f32x4*>(sW + (2 * ks + g) * 8);
                 w1 = *reinterpret_cast<const f32x4*>(sW + (2 * ks + g) * 8 + 4);
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                float d = dy[ks >> 1][8 * (ks & 1) + j] + bf_at(dqr[ks], j);
+                float d = dy[8 * (ks & 1) + j] + bf_at(dqr[ks], j);
                 if constexpr (NORM) {
                     const float u = bf_at(T.xr[ks], j) * T.rstd;
-                    if (valid) dwacc[ks][j] = fmaf(d, u, dwacc[ks][j]);
+                    if constexpr (AHEAD) {
+                        if (valid) dwacc[ks][j] = fmaf(d, u, dwacc[ks][j]);
+                    } else {
+                        prod[j >> 2][j & 3] = valid ? d * u : 0.0f;
+                    }
                     d *= (j < 4 ? w0[j & 3] : w1[j & 3]);
                     cpart = fmaf(d, u, cpart);
                 }
                 du[ks][j] = d;
             }
-        }
+            if constexpr (NORM && !AHEAD) {
+                // 64 columns of the products (chunk c of row r at c ^ (r % 16)) to each half of the region, whose y and dz
+                // tiles have been read, and down the columns
+                constexpr int half = ks / 4, c0 = 4 * (ks % 4);
+                unsigned char* ptile = ytile + half * TILE_B;
+#pragma unroll
+                for (int q = 0; q < 2; ++q) *reinterpret_cast<f32x4*>(ptile + (prow ^ ((c0 + q) << 4))) = prod[q];
+                if constexpr (ks % 4 == 3 || ks == KS - 1) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)      // (lanes of columns beyond d_h add up what nobody reads)
+                        dwcol[half] += *reinterpret_cast<const f32x4*>(ptile + k * 1024 + (pread ^ ((k & 3) << 6)));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+        next_phase();
         if constexpr (NORM) {
             cpart += __shfl_xor(cpart, 32);
             const float c = cpart / (float)DH;
@@ -407,97 +557,153 @@ __global__ __launch_bounds__(256) void mhffn_gate_bwd_kernel(GateArgs p)
                 *reinterpret_cast<bf16x8*>(p.dX + row + (2 * ks + g) * 8) = o;
             }
         }
-
-        // d_router += y^T dz over this tile's tokens
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            bf16x8 bz[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) bz[nt] = tile_cols(ztile, trl, nt, s);
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const bf16x8 ay = tile_cols(ytile, trl, ct, s);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) wacc[ct][nt] = mfma32(ay, bz[nt], wacc[ct][nt]);
-            }
-        }
     }
 
-    // ---- sums over tokens: the four waves' partials meet in LDS, then one atomic add per workgroup and element ------
+    // ---- sums over tokens: the waves' partials meet in LDS, then leave as one atomic add or one partial sum per workgroup
+    // and element --------------------------------------------------------------------------------------------------------
     __syncthreads();   // every wave is past its last tile: the per-wave regions are free
-    float* mine = reinterpret_cast<float*>(regions + wave * GATE_WAVE_REGION_B);
+    float* mine = reinterpret_cast<float*>(ytile);
+    float* part = p.part ? p.part + (((long)h * gridDim.z + b) * gridDim.x + blockIdx.x) * (DH * p.E + DH) : nullptr;
     float* dWr = p.dWr + (long)h * DH * p.E;
+    auto put = [&](int nt, int idx, float v) {      // value idx of expert tile nt: lane idx % 64, register idx / 64 % 16, column tile
+        const int ln = idx & 63, i = (idx >> 6) & 15, ct = idx >> 10;
+        const int e = nt * 32 + (ln & 31), col = ct * 32 + 8 * (i >> 2) + 4 * (ln >> 5) + (i & 3);
+        if (e >= p.E) return;
+        if (part) part[col * p.E + e] = v;
+        else unsafeAtomicAdd(dWr + (long)col * p.E + e, v);
+    };
+    if constexpr (!AHEAD) {
+        float* sums = reinterpret_cast<float*>(regions);      // [GROUPS][CT][16][64]
+        if (wave < GROUPS * CT)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) mine[(ct * 16 + i) * 64 + lane] = wacc[ct][nt][i];
+            for (int i = 0; i < 16; ++i) sums[(wave * 16 + i) * 64 + lane] = wacc[0][0][i];
         __syncthreads();
-        for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 256) {
+        for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 64 * NW) {
             float v = 0.0f;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) v += reinterpret_cast<const float*>(regions + w * GATE_WAVE_REGION_B)[idx];
-            const int ln = idx & 63, i = (idx >> 6) & 15, ct = idx >> 10;
-            const int e = nt * 32 + (ln & 31), col = ct * 32 + 8 * (i >> 2) + 4 * (ln >> 5) + (i & 3);
-            if (e < p.E) unsafeAtomicAdd(dWr + (long)col * p.E + e, v);
+            for (int q = 0; q < GROUPS; ++q) v += sums[q * CT * 1024 + idx];
+            put(0, idx, v);
         }
         __syncthreads();
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+            for (int ct = 0; ct < WCT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) mine[(ct * 16 + i) * 64 + lane] = wacc[ct][nt][i];
+            __syncthreads();
+            for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 64 * NW) {
+                float v = 0.0f;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) v += reinterpret_cast<const float*>(regions + w * REGION_B)[idx];
+                put(nt, idx, v);
+            }
+            __syncthreads();
+        }
     }
     if constexpr (NORM) {
-        // transpose inside the wave: value v = 8 ks + j of every lane goes to row v (row stride 65 floats keeps both the
-        // writes and the row-wise reads conflict-free), then lane v adds up each lane half of its row
+        float* cross = reinterpret_cast<float*>(regions + NW * REGION_B);   // [NW waves][128 columns]
+        if constexpr (AHEAD) {
+            // transpose inside the wave: value v = 8 ks + j of every lane goes to row v (row stride 65 floats keeps both
+            // the writes and the row-wise reads conflict-free), then lane v adds up each lane half of its row
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+            for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) mine[(ks * 8 + j) * 65 + lane] = dwacc[ks][j];
-        float* cross = reinterpret_cast<float*>(regions + 4 * GATE_WAVE_REGION_B);   // [4 waves][128 columns]
-        if (lane < KS * 8) {
-            float s0 = 0.0f, s1 = 0.0f;
-            for (int i = 0; i < 32; ++i) {
-                s0 += mine[lane * 65 + i];
-                s1 += mine[lane * 65 + 32 + i];
+                for (int j = 0; j < 8; ++j) mine[(ks * 8 + j) * 65 + lane] = dwacc[ks][j];
+            if (lane < KS * 8) {
+                float s0 = 0.0f, s1 = 0.0f;
+                for (int i = 0; i < 32; ++i) {
+                    s0 += mine[lane * 65 + i];
+                    s1 += mine[lane * 65 + 32 + i];
+                }
+                const int ks = lane >> 3, j = lane & 7;
+                cross[wave * 128 + (2 * ks) * 8 + j] = s0;
+                cross[wave * 128 + (2 * ks + 1) * 8 + j] = s1;
             }
-            const int ks = lane >> 3, j = lane & 7;
-            cross[wave * 128 + (2 * ks) * 8 + j] = s0;
-            cross[wave * 128 + (2 * ks + 1) * 8 + j] = s1;
+        } else {
+#pragma unroll
+            for (int i = 0; i < NHALF; ++i) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    float v = dwcol[i][x];
+                    v += __shfl_xor(v, 16);
+                    v += __shfl_xor(v, 32);
+                    if (lane < 16 && 64 * i + 4 * lane < DH) cross[wave * 128 + 64 * i + 4 * lane + x] = v;
+                }
+            }
         }
         __syncthreads();
-        if (threadIdx.x < DH)
-            unsafeAtomicAdd(p.dWn + h * DH + threadIdx.x, cross[threadIdx.x] + cross[128 + threadIdx.x] +
-                                                              cross[256 + threadIdx.x] + cross[384 + threadIdx.x]);
+        if (threadIdx.x < DH) {
+            float v = 0.0f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v += cross[w * 128 + threadIdx.x];
+            if (part) part[DH * p.E + threadIdx.x] = v;
+            else unsafeAtomicAdd(p.dWn + h * DH + threadIdx.x, v);
+        }
     }
+}
+
+// Adds the workgroups' sums of a head (in order) and writes d_router and d_norm_weight in the parameters' types.
+__global__ __launch_bounds__(256) void mhffn_gate_sum_kernel(const float* part, void* dWn, int wn_bf16, void* dWr, int wr_bf16, int dh,
+                                                             int E, int wgs)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, nr = dh * E, n = nr + dh;
+    if (i >= n || (i >= nr && !dWn)) return;
+    const float* src = part + (long)h * wgs * n + i;
+    float v = 0.0f;
+    int w = 0;
+    for (; w + 8 <= wgs; w += 8) {      // (eight loads in flight)
+        float x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = src[(long)(w + k) * n];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v += x[k];
+    }
+    for (; w < wgs; ++w) v += src[(long)w * n];
+    const bool r = i < nr;
+    void* dst = r ? dWr : dWn;
+    const long at = r ? (long)h * nr + i : (long)h * dh + i - nr;
+    if (r ? wr_bf16 : wn_bf16) static_cast<bf16_t*>(dst)[at] = (bf16_t)v;
+    else static_cast<float*>(dst)[at] = v;
 }
 
 // ---- launch ---------------------------------------------------------------------------------------------------------
 namespace {
 
-int tiles_per_wave(const GateArgs& a, bool backward)
+// Tiles a wave takes.  Forward: several waves per SIMD hide the latency, so a wave only takes several tiles once there
+// are at least 8 waves per SIMD; backward: as many waves (and partial sums) as fill the chip once.
+int tiles_per_wave(int B, int H, int S, int waves, long cap)
 {
-    const long total = (long)a.B * a.H * ((a.S + 31) / 32);
-    // forward: several waves per SIMD hide the latency, so a wave only takes several tiles once there are at least 8 waves
-    // per SIMD; backward: one wave per SIMD with its own prefetch, as few waves (= atomic adds) as fill the chip once
-    const long tpw = backward ? total / 1024 : total / 8192;
-    const long cap = backward ? 64 : 16;
+    const long total = (long)B * H * ((S + 31) / 32);
+    const long tpw = total / waves;
     return (int)(tpw < 1 ? 1 : tpw > cap ? cap : tpw);
+}
+template <int NT>
+dim3 gate_bwd_grid(int B, int H, int S, int& tpw)
+{
+    constexpr int NW = gate_bwd_waves<NT>();
+    tpw = tiles_per_wave(B, H, S, NW * CUS, 64);
+    const int ntiles = (S + 31) / 32;
+    return dim3((ntiles + NW * tpw - 1) / (NW * tpw), H, B);
 }
 
 template <int DH, int NT, bool NORM>
 hipError_t launch_gate(GateArgs a, bool backward, hipStream_t st)
 {
     static LdsOptIn optin_fwd, optin_bwd;
-    a.tpw = tiles_per_wave(a, backward);
-    const int ntiles = (a.S + 31) / 32;
-    const dim3 grid((ntiles + 4 * a.tpw - 1) / (4 * a.tpw), a.H, a.B);
     if (backward) {
-        const size_t smem = gate_bwd_smem(DH, NT);
+        const size_t smem = gate_bwd_smem<NT>(DH);
         const hipError_t e = ensure_dynamic_lds(optin_bwd, (const void*)mhffn_gate_bwd_kernel<DH, NT, NORM>, (int)smem);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((mhffn_gate_bwd_kernel<DH, NT, NORM>), grid, dim3(256), smem, st, a);
+        const dim3 grid = gate_bwd_grid<NT>(a.B, a.H, a.S, a.tpw);
+        hipLaunchKernelGGL((mhffn_gate_bwd_kernel<DH, NT, NORM>), grid, dim3(64 * gate_bwd_waves<NT>()), smem, st, a);
     } else {
         const size_t smem = gate_fwd_smem(DH, NT);
         const hipError_t e = ensure_dynamic_lds(optin_fwd, (const void*)mhffn_gate_fwd_kernel<DH, NT, NORM>, (int)smem);
         if (e != hipSuccess) return e;
+        a.tpw = tiles_per_wave(a.B, a.H, a.S, 8192, 16);
+        const dim3 grid(((a.S + 31) / 32 + 4 * a.tpw - 1) / (4 * a.tpw), a.H, a.B);
         hipLaunchKernelGGL((mhffn_gate_fwd_kernel<DH, NT, NORM>), grid, dim3(256), smem, st, a);
     }
     return hipGetLastError();
@@ -521,36 +727,60 @@ hipError_t launch_gate_any(const GateArgs& a, int d_h, bool backward, hipStream_
     return hipErrorInvalidValue;
 }
 
+int gate_bwd_workgroups(const Dims& d)      // of one head
+{
+    int tpw;
+    const dim3 g = d.E <= 32 ? gate_bwd_grid<1>(d.B, d.H, d.S, tpw) : gate_bwd_grid<2>(d.B, d.H, d.S, tpw);
+    return (int)(g.x * g.z);
+}
+
 }  // namespace
 
-hipError_t launch_gate_fwd(const void* X, const float* Wn, float eps, const float* Wr, void* Qn, float* R, const Dims& d,
-                           hipStream_t st)
+hipError_t launch_gate_fwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, void* Qn, float* R,
+                           const Dims& d, hipStream_t st)
 {
     GateArgs a{};
     a.X = (const bf16_t*)X;
     a.Wn = Wn;
     a.Wr = Wr;
+    a.wn_bf16 = wn_bf16;
+    a.wr_bf16 = wr_bf16;
     a.Qn = (bf16_t*)Qn;
     a.R = R;
     a.B = d.B, a.H = d.H, a.S = d.S, a.E = d.E, a.eps = eps;
     return launch_gate_any(a, d.d_h, false, st);
 }
 
-hipError_t launch_gate_bwd(const void* X, const float* Wn, float eps, const float* Wr, const void* dQ, int dq_tokmaj,
-                           const float* dR, void* dX, float* dWn, float* dWr, const Dims& d, hipStream_t st)
+size_t gate_bwd_workspace_bytes(const Dims& d)
+{
+    return (size_t)d.H * gate_bwd_workgroups(d) * (d.d_h * d.E + d.d_h) * sizeof(float);
+}
+
+hipError_t launch_gate_bwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, const void* dQ,
+                           int dq_tokmaj, const float* dR, void* dX, void* dWn, void* dWr, void* ws, const Dims& d, hipStream_t st)
 {
     GateArgs a{};
     a.X = (const bf16_t*)X;
     a.Wn = Wn;
     a.Wr = Wr;
+    a.wn_bf16 = wn_bf16;
+    a.wr_bf16 = wr_bf16;
     a.dQ = (const bf16_t*)dQ;
     a.dR = dR;
     a.dX = (bf16_t*)dX;
-    a.dWn = dWn;
-    a.dWr = dWr;
+    a.part = (float*)ws;
+    if (!ws) {
+        a.dWn = (float*)dWn;
+        a.dWr = (float*)dWr;
+    }
     a.dq_tokmaj = dq_tokmaj;
     a.B = d.B, a.H = d.H, a.S = d.S, a.E = d.E, a.eps = eps;
-    return launch_gate_any(a, d.d_h, true, st);
+    hipError_t err = launch_gate_any(a, d.d_h, true, st);
+    if (err != hipSuccess || !ws) return err;
+    const dim3 grid((d.d_h * d.E + d.d_h + 255) / 256, d.H);
+    const int wgs = gate_bwd_workgroups(d);
+    hipLaunchKernelGGL(mhffn_gate_sum_kernel, grid, dim3(256), 0, st, a.part, Wn ? dWn : nullptr, wn_bf16, dWr, wr_bf16, d.d_h, d.E, wgs);
+    return hipGetLastError();
 }
 
 }  // namespace mhffn

@@ -165,33 +165,29 @@ bool records_grad(std::initializer_list<const Tensor*> ts)
     return false;
 }
 
-// O = fused(Q, K, U, V, R).  f32_grads: dQ, dK, dU, dV in float32 whatever the inputs are (the ThunderKittens wrapper's
-// convention, kernels/thunderkittens/flash_ffn_moe_torch.py:17-21); otherwise in the inputs' dtypes.
+// O = fused(Q, K, U, V, R), gradients in the inputs' types.  (The ThunderKittens wrapper returns float32 gradients,
+// kernels/thunderkittens/flash_ffn_moe_torch.py:17-21, which autograd rounds to the inputs' types before anyone sees
+// them: the same values, so the kernels write those at once.)
 struct OpNode : torch::autograd::Function<OpNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R,
-                          bool f32_grads, bool one_part)
+                          bool one_part)
     {
         ctx->save_for_backward({Q, K, U, V, R});
-        ctx->saved_data["f32"] = f32_grads;
         ctx->saved_data["one_part"] = one_part;
         return op_forward(Q, K, U, V, R, one_part);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
     {
         const auto s = ctx->get_saved_variables();
-        const bool f32 = ctx->saved_data["f32"].toBool();
-        auto out = op_backward(s[0], s[1], s[2], s[3], s[4], g[0], f32 ? at::kFloat : s[1].scalar_type(),
-                               ctx->saved_data["one_part"].toBool());
-        if (f32) out[0] = out[0].to(at::kFloat);
-        out.resize(7);
+        auto out = op_backward(s[0], s[1], s[2], s[3], s[4], g[0], s[1].scalar_type(), ctx->saved_data["one_part"].toBool());
+        out.emplace_back();
         return out;
     }
 };
-Tensor op(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, bool f32_grads,
-          bool one_part)
+Tensor op(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& R, bool one_part)
 {
     if (!records_grad({&Q, &K, &U, &V, &R})) return op_forward(Q, K, U, V, R, one_part);
-    return OpNode::apply(Q, K, U, V, R, f32_grads, one_part);
+    return OpNode::apply(Q, K, U, V, R, one_part);
 }
 
 // The single-expert operator: Q [B,H,S,d_h], K/U/V [Hkuv, rows, d_h], gate 1.
@@ -231,20 +227,26 @@ mhffn_dims gate_dims(const Tensor& x4, const Tensor& wn, const Tensor& router)
 }
 
 struct GateForward {
-    Tensor x4, wn, wr, q4, R;      // contiguous x, float32 weights, normalised heads [B,S,H,d_h] (x4 without a norm), gate
+    Tensor x4, wn, wr, q4, R;      // contiguous x and weights, normalised heads [B,S,H,d_h] (x4 without a norm), gate
 };
+Tensor gate_param(const Tensor& w)      // contiguous, float32 or bfloat16
+{
+    if (!w.defined()) return w;
+    return contig(w.scalar_type() == at::kBFloat16 || w.scalar_type() == at::kFloat ? w : w.to(at::kFloat));
+}
+int param_code(const Tensor& w) { return w.defined() ? dtype_code(w.scalar_type()) : MHFFN_DTYPE_F32; }
 GateForward gate_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& router, double eps)
 {
     const mhffn_dims d = gate_dims(x, norm_weight, router);
     GateForward f;
     f.x4 = contig(x);
-    if (norm_weight.defined()) f.wn = contig(norm_weight.to(at::kFloat));
-    f.wr = contig(router.to(at::kFloat));
+    f.wn = gate_param(norm_weight);
+    f.wr = gate_param(router);
     OnDevice guard(f.x4);
     f.q4 = f.wn.defined() ? empty_of(x.sizes(), at::kBFloat16, f.x4) : f.x4;
     f.R = empty_of({d.B, d.H, d.S, d.E}, at::kFloat, f.x4);
-    raise_for_code(mhffn_gate_fwd(ptr(f.x4), (const float*)ptr(f.wn), (float)eps, (const float*)ptr(f.wr),
-                                  f.wn.defined() ? ptr(f.q4) : nullptr, (float*)ptr(f.R), &d, stream()),
+    raise_for_code(mhffn_gate_fwd_typed(ptr(f.x4), ptr(f.wn), param_code(f.wn), (float)eps, ptr(f.wr), param_code(f.wr),
+                                        f.wn.defined() ? ptr(f.q4) : nullptr, (float*)ptr(f.R), &d, stream()),
                    "mhffn_gate_fwd");
     return f;
 }
@@ -261,11 +263,13 @@ variable_list gate_backward(const Tensor& x4, const Tensor& norm_weight, const T
         layout = MHFFN_TOKENS_BHSD;
         dQ = dQ.contiguous();
     }
-    dR = contig(dR.to(at::kFloat));
-    Tensor dx = empty_of(x4.sizes(), at::kBFloat16, x4), dwn, dwr = at::zeros_like(wr);
-    if (wn.defined()) dwn = at::zeros_like(wn);
-    raise_for_code(mhffn_gate_bwd(ptr(x4), (const float*)ptr(wn), (float)eps, (const float*)ptr(wr), ptr(dQ), layout,
-                                  (const float*)ptr(dR), ptr(dx), (float*)ptr(dwn), (float*)ptr(dwr), &d, stream()),
+    dR = contig(dR.scalar_type() == at::kFloat ? dR : dR.to(at::kFloat));
+    Tensor dx = empty_of(x4.sizes(), at::kBFloat16, x4), dwn, dwr = empty_of(wr.sizes(), wr.scalar_type(), x4);
+    if (wn.defined()) dwn = empty_of(wn.sizes(), wn.scalar_type(), x4);
+    const size_t ws_bytes = mhffn_gate_bwd_workspace_bytes(&d);
+    Tensor ws = scratch(ws_bytes, x4);
+    raise_for_code(mhffn_gate_bwd_into(ptr(x4), ptr(wn), param_code(wn), (float)eps, ptr(wr), param_code(wr), ptr(dQ), layout,
+                                       (const float*)ptr(dR), ptr(dx), ptr(dwn), ptr(dwr), ptr(ws), ws_bytes, &d, stream()),
                    "mhffn_gate_bwd");
     return {dx, dwn.defined() ? dwn.to(norm_weight.scalar_type()) : dwn, dwr.to(router.scalar_type())};
 }

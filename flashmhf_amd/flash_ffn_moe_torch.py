@@ -1,7 +1,8 @@
 """Drop-in for the reference's ``kernels/thunderkittens/flash_ffn_moe_torch.py`` (``FlashFFNMoEFunction`` :5-24,
-``FlashFFNMoE`` :27-31): same call signature, and -- as that wrapper does (:17-21) -- gradients of the bf16
-weights and of Q are returned in float32.  The R transpose the ThunderKittens kernel needs (:9, :23) is not
-needed here: the HIP kernels read R as [B,H,S,E].
+``FlashFFNMoE`` :27-31): same call signature.  That wrapper returns the gradients of the bf16 weights and of Q in float32
+(:17-21), and autograd hands each on in its tensor's own dtype: ``FlashFFNMoEFunction`` does as the wrapper does, the
+module's native node writes those values without the float32 copies.  The R transpose the ThunderKittens kernel needs
+(:9, :23) is not needed here: the HIP kernels read R as [B,H,S,E].
 """
 import torch
 
@@ -28,4 +29,4 @@ class FlashFFNMoE(torch.nn.Module):
         super().__init__()
 
     def forward(self, Q, K, U, V, R):
-        return _capi.native().op(Q, K, U, V, R, True, False)
+        return _capi.native().op(Q, K, U, V, R, False)

@@ -60,4 +60,4 @@ class FlashMLPMoE(torch.nn.Module):
         self.one_part = one_part
 
     def forward(self, Q, K, U, V, R):
-        return _capi.native().op(Q, K, U, V, R, False, self.one_part)
+        return _capi.native().op(Q, K, U, V, R, self.one_part)

@@ -186,6 +186,18 @@ int mhffn_gate_bwd(const void* X, const float* norm_weight, float eps, const flo
                    const void* dQ, int dq_token_layout, const float* dR,
                    void* dX, float* d_norm_weight, float* d_router, const mhffn_dims* dims, void* stream);
 
+/* The same prologue with norm_weight and router, and the gradients of both, each in a type of its own (norm_dtype,
+ * router_dtype: MHFFN_DTYPE_*), so that a bfloat16 model needs no float32 copies.  mhffn_gate_bwd_into overwrites
+ * d_norm_weight and d_router (no zero fill) and is deterministic: the workgroups' sums go to the workspace
+ * (mhffn_gate_bwd_workspace_bytes) and are added in a fixed order. */
+int mhffn_gate_fwd_typed(const void* X, const void* norm_weight, int norm_dtype, float eps,
+                         const void* router, int router_dtype, void* Qn, float* R, const mhffn_dims* dims, void* stream);
+size_t mhffn_gate_bwd_workspace_bytes(const mhffn_dims* dims);
+int mhffn_gate_bwd_into(const void* X, const void* norm_weight, int norm_dtype, float eps,
+                        const void* router, int router_dtype, const void* dQ, int dq_token_layout, const float* dR,
+                        void* dX, void* d_norm_weight, void* d_router,
+                        void* workspace, size_t workspace_bytes, const mhffn_dims* dims, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
