@@ -25,7 +25,7 @@ EXPORTS = (
     "mhffn_strerror", "mhffn_is_supported", "mhffn_check_dims", "mhffn_fwd_workspace_bytes",
     "mhffn_bwd_workspace_bytes", "mhffn_fwd", "mhffn_bwd", "mhffn_fwd_phases", "mhffn_bwd_phases",
     "mhffn_fwd_layout", "mhffn_bwd_layout", "mhffn_bwd_static", "mhffn_gate_fwd", "mhffn_gate_bwd",
-    "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into",
+    "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into", "mhffn_rope_fwd", "mhffn_rope_bwd",
 )
 TOKENS_BHSD, TOKENS_BSHD = 0, 1     # layout of Q, O, dO, dQ
 FWD_MAIN, FWD_ALL = 1, 1

@@ -289,4 +289,36 @@ int mhffn_gate_bwd_into(const void* X, const void* norm_weight, int norm_dtype, 
                     workspace, dims, stream);
 }
 
+static int check_rope_dims(int B, int S, int H, int d)
+{
+    if (B <= 0 || S <= 0 || H <= 0 || d <= 0 || (double)B * S * H * (d / 16) >= 2147483648.0) return MHFFN_ERR_SHAPE;
+    return d % 16 == 0 ? MHFFN_OK : MHFFN_ERR_HEAD_DIM;
+}
+
+int mhffn_rope_fwd(const void* qkv, const void* cos, const void* sin, void* q, void* k, int B, int S, int H, int d, void* stream)
+{
+    const int rc = check_rope_dims(B, S, H, d);
+    if (rc != MHFFN_OK) return rc;
+    const void* ptrs[] = {qkv, cos, sin, q, k};
+    for (const void* p : ptrs) {
+        if (!p) return MHFFN_ERR_NULL_POINTER;
+        if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
+    }
+    return mhffn::launch_rope_fwd(qkv, cos, sin, q, k, B, S, H, d, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
+}
+
+int mhffn_rope_bwd(const void* dq, const void* dk, const void* dv, const long* strides, const void* cos, const void* sin, void* dqkv,
+                   int B, int S, int H, int d, void* stream)
+{
+    const int rc = check_rope_dims(B, S, H, d);
+    if (rc != MHFFN_OK) return rc;
+    if (!dq || !dk || !dv || !strides || !cos || !sin || !dqkv) return MHFFN_ERR_NULL_POINTER;
+    if (!aligned16(cos) || !aligned16(sin) || !aligned16(dqkv)) return MHFFN_ERR_ALIGNMENT;
+    const void* grads[3] = {dq, dk, dv};
+    return mhffn::launch_rope_bwd(grads, reinterpret_cast<const long(*)[3]>(strides), cos, sin, dqkv, B, S, H, d,
+                                  (hipStream_t)stream) == hipSuccess
+               ? MHFFN_OK
+               : MHFFN_ERR_LAUNCH;
+}
+
 }  // extern "C"

@@ -524,6 +524,12 @@ size_t gate_bwd_workspace_bytes(const Dims& d);
 hipError_t launch_gate_bwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, const void* dQ,
                            int dq_tokmaj, const float* dR, void* dX, void* dWn, void* dWr, void* ws, const Dims& d, hipStream_t st);
 
+// Rotary positions of the decoder's attention (mhffn_rope.hip); d a multiple of 16, B * S * H * d / 16 below 2^31.
+hipError_t launch_rope_fwd(const void* qkv, const void* cos, const void* sin, void* q, void* k, int B, int S, int H, int dh,
+                           hipStream_t st);
+hipError_t launch_rope_bwd(const void* const d[3], const long (*stride)[3], const void* cos, const void* sin, void* dqkv, int B, int S,
+                           int H, int dh, hipStream_t st);
+
 // Bits of the `phases` argument of the launch functions (the values of MHFFN_FWD_*, MHFFN_BWD_*, MHFFN_ONE_PART in
 // include/mhffn.h).
 constexpr int PH_FWD_MAIN = 1, PH_BWD_DQDR = 1, PH_BWD_DKDUDV = 2, PH_BWD_REDUCE = 4, PH_ONE_PART = 256;

@@ -359,6 +359,65 @@ Tensor block(const Tensor& x, const Tensor& w1, const std::optional<Tensor>& nor
     return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps, one_part);
 }
 
+// ---- the decoder's rotary positions --------------------------------------------------------------------------------
+struct RopeForward {
+    Tensor q, k, v;      // [B, H, S, d] views: q, k of [B, S, H, d] memory, v of qkv itself
+};
+RopeForward rope_forward(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
+{
+    TORCH_CHECK(qkv.dim() == 3 && qkv.is_contiguous() && qkv.is_cuda() && cos.is_contiguous() && sin.is_contiguous() &&
+                    cos.sizes() == sin.sizes() && cos.dim() == 2 && cos.size(0) == qkv.size(1) && qkv.size(2) == 3 * H * cos.size(1),
+                "expected qkv [B,S,3*H*d] contiguous on the GPU and cos, sin [S,d]");
+    for (const Tensor* t : {&qkv, &cos, &sin}) TORCH_CHECK_TYPE(t->scalar_type() == at::kBFloat16, "rotary positions are bfloat16 here");
+    const int64_t B = qkv.size(0), S = qkv.size(1), d = cos.size(1);
+    OnDevice guard(qkv);
+    RopeForward f;
+    f.q = empty_of({B, S, H, d}, at::kBFloat16, qkv);
+    f.k = empty_of({B, S, H, d}, at::kBFloat16, qkv);
+    raise_for_code(mhffn_rope_fwd(ptr(qkv), ptr(cos), ptr(sin), ptr(f.q), ptr(f.k), (int)B, (int)S, (int)H, (int)d, stream()), "mhffn_rope");
+    f.q = f.q.transpose(1, 2);
+    f.k = f.k.transpose(1, 2);
+    f.v = qkv.view({B, S, 3, H, d}).select(2, 2).transpose(1, 2);
+    return f;
+}
+struct RopeNode : torch::autograd::Function<RopeNode> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
+    {
+        RopeForward f = rope_forward(qkv, cos, sin, H);
+        ctx->save_for_backward({cos, sin});
+        return {f.q, f.k, f.v};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        long strides[9];
+        Tensor any;
+        for (Tensor& t : g)
+            if (t.defined()) any = t;
+        for (int w = 0; w < 3; ++w) {
+            if (!g[w].defined()) g[w] = at::zeros_like(any);
+            if (g[w].stride(3) != 1) g[w] = g[w].contiguous();
+            for (int i = 0; i < 3; ++i) strides[3 * w + i] = g[w].stride(i);
+        }
+        const int64_t B = any.size(0), H = any.size(1), S = any.size(2), d = any.size(3);
+        OnDevice guard(any);
+        Tensor dqkv = empty_of({B, S, 3 * H * d}, at::kBFloat16, any);
+        raise_for_code(mhffn_rope_bwd(ptr(g[0]), ptr(g[1]), ptr(g[2]), strides, ptr(s[0]), ptr(s[1]), ptr(dqkv), (int)B, (int)S, (int)H,
+                                      (int)d, stream()),
+                       "mhffn_rope");
+        return {dqkv, Tensor(), Tensor(), Tensor()};
+    }
+};
+std::tuple<Tensor, Tensor, Tensor> rope(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
+{
+    if (!records_grad({&qkv})) {
+        RopeForward f = rope_forward(qkv, cos, sin, H);
+        return {f.q, f.k, f.v};
+    }
+    auto out = RopeNode::apply(qkv, cos, sin, H);
+    return {out[0], out[1], out[2]};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m)
@@ -373,5 +432,6 @@ PYBIND11_MODULE(_native, m)
     m.def("op", torch::wrap_pybind_function_no_gil(op));
     m.def("single", torch::wrap_pybind_function_no_gil(single));
     m.def("gate", torch::wrap_pybind_function_no_gil(gate));
+    m.def("rope", torch::wrap_pybind_function_no_gil(rope));
     m.def("block", torch::wrap_pybind_function_no_gil(block));
 }

@@ -186,9 +186,13 @@ class CausalSelfAttention(nn.Module):
 
     def forward(self, x, rope=None):
         B, S, hid = x.shape
-        q, k, v = self.qkv(x).view(B, S, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
         cos, sin = rope if rope is not None else _rotary(S, self.head_dim, self.rope_base, x.device, x.dtype)
-        q, k = _apply_rotary(q, cos, sin), _apply_rotary(k, cos, sin)
+        qkv = self.qkv(x)
+        if qkv.is_cuda and qkv.dtype == cos.dtype == torch.bfloat16 and self.head_dim % 16 == 0:
+            q, k, v = _capi.native().rope(qkv.contiguous(), cos, sin, self.num_heads)     # one pass, the same roundings
+        else:
+            q, k, v = qkv.view(B, S, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
+            q, k = _apply_rotary(q, cos, sin), _apply_rotary(k, cos, sin)
         y = F.scaled_dot_product_attention(q, k, v, is_causal=True)
         return self.out(y.transpose(1, 2).reshape(B, S, hid))
 
@@ -225,10 +229,25 @@ class MHFFNDecoder(nn.Module):
             if isinstance(m, nn.Linear):
                 nn.init.normal_(m.weight, std=0.02 if m is not self.lm_head else 1.0 / math.sqrt(hidden_size))
 
+    def _rope_tables(self, seq_len, device, dtype):
+        """The rotary tables of one sequence length, kept for the next call of that length on the same stream (a dozen small
+        launches).  Tables made while a graph is captured belong to the graph, inference tensors cannot be saved for a
+        backward: neither are kept."""
+        attn = self.blocks[0].attn
+        on_gpu = device.type == "cuda"
+        key = (seq_len, attn.head_dim, attn.rope_base, device, dtype,
+               torch.cuda.current_stream(device).cuda_stream if on_gpu else None)
+        kept = self.__dict__.get("_rope_kept")
+        if kept is not None and kept[0] == key:
+            return kept[1]
+        tables = _rotary(seq_len, attn.head_dim, attn.rope_base, device, dtype)
+        if not torch.is_inference_mode_enabled() and not (on_gpu and torch.cuda.is_current_stream_capturing()):
+            self.__dict__["_rope_kept"] = (key, tables)
+        return tables
+
     def forward(self, ids, labels=None):
         x = self.embed(ids)
-        attn = self.blocks[0].attn
-        rope = _rotary(ids.shape[1], attn.head_dim, attn.rope_base, x.device, x.dtype)   # one table for every block
+        rope = self._rope_tables(ids.shape[1], x.device, x.dtype)   # one table for every block
         for blk in self.blocks:
             x = blk(x, rope)
         logits = self.lm_head(self.norm(x))

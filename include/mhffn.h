@@ -198,6 +198,15 @@ int mhffn_gate_bwd_into(const void* X, const void* norm_weight, int norm_dtype, 
                         void* dX, void* d_norm_weight, void* d_router,
                         void* workspace, size_t workspace_bytes, const mhffn_dims* dims, void* stream);
 
+/* Rotary positions of the decoder shell's attention (models/flashmhf/modeling_mhffnmoe.py applies them as
+ * x cos + rotate_half(x) sin), with every product and sum rounded to bfloat16 as those element-wise operations round them.
+ *   qkv, dqkv   [B, S, 3, H, d] bfloat16: the projection's memory;  cos, sin [S, d] bfloat16;  q, k [B, S, H, d]
+ *   dq, dk, dv  bfloat16, element (b, h, s, c) at b * stride[0] + h * stride[1] + s * stride[2] + c of its own strides
+ *               (strides: 9 numbers, of dq, dk, dv);  d a multiple of 16 */
+int mhffn_rope_fwd(const void* qkv, const void* cos, const void* sin, void* q, void* k, int B, int S, int H, int d, void* stream);
+int mhffn_rope_bwd(const void* dq, const void* dk, const void* dv, const long* strides, const void* cos, const void* sin,
+                   void* dqkv, int B, int S, int H, int d, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
