@@ -10,6 +10,7 @@ import importlib.util
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "libmhffn_hip.so")
@@ -84,6 +85,18 @@ def native():
         _native = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(_native)
     return _native
+
+
+def native_nodes():
+    """Whether the operators may record the native autograd nodes.  A trace keeps only calls that it knows (the native ones
+    would become constants), and functorch transforms and forward mode have to meet a torch.autograd.Function, which runs
+    or refuses them: under these the operators go through their Python Functions."""
+    return not (torch._C._is_tracing() or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0)
+
+
+def traced(t):
+    """`t`, an output of a native call inside a Function's forward, as a tensor that a running trace knows."""
+    return t.clone() if torch._C._is_tracing() else t
 
 
 def strerror(code):

@@ -223,16 +223,24 @@ mhffn_dims gate_dims(const Tensor& x4, const Tensor& wn, const Tensor& router)
     TORCH_CHECK(!wn.defined() || (wn.dim() == 2 && wn.size(0) == n[2] && wn.size(1) == n[3]), "norm_weight must be [H,d_h] = [", n[2],
                 ",", n[3], "], got ", wn.defined() ? wn.sizes() : at::IntArrayRef());
     TORCH_CHECK(x4.is_cuda(), "flashmhf_amd runs on the GPU only; there is no CPU path");
+    TORCH_CHECK(router.device() == x4.device() && (!wn.defined() || wn.device() == x4.device()),
+                "router and norm_weight must be on the device of x, ", x4.device());
     return mhffn_dims{(int)n[0], (int)n[2], (int)n[2], (int)n[1], (int)n[3], (int)router.size(2), 32};
 }
 
 struct GateForward {
     Tensor x4, wn, wr, q4, R;      // contiguous x and weights, normalised heads [B,S,H,d_h] (x4 without a norm), gate
 };
-Tensor gate_param(const Tensor& w)      // contiguous, float32 or bfloat16
+// `t` contiguous on a 16-byte boundary (a view into a flat buffer of parameters may start anywhere)
+Tensor on_boundary(const Tensor& t)
+{
+    const Tensor c = contig(t);
+    return (reinterpret_cast<uintptr_t>(c.data_ptr()) & 15) == 0 ? c : c.clone();
+}
+Tensor gate_param(const Tensor& w)      // contiguous and on a boundary, float32 or bfloat16
 {
     if (!w.defined()) return w;
-    return contig(w.scalar_type() == at::kBFloat16 || w.scalar_type() == at::kFloat ? w : w.to(at::kFloat));
+    return on_boundary(w.scalar_type() == at::kBFloat16 || w.scalar_type() == at::kFloat ? w : w.to(at::kFloat));
 }
 int param_code(const Tensor& w) { return w.defined() ? dtype_code(w.scalar_type()) : MHFFN_DTYPE_F32; }
 GateForward gate_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& router, double eps)
@@ -319,6 +327,14 @@ BlockForward block_forward(const Tensor& x, const Tensor& w1, const Tensor& norm
     return f;
 }
 
+Tensor stepwise_O4(const Tensor& x, const Tensor& w1, const Tensor& nw, const Tensor& router, const Tensor& K, const Tensor& U,
+                   const Tensor& V, double eps, bool one_part)
+{
+    auto [Q, R] = gate(at::linear(x, w1).view({x.size(0), x.size(1), router.size(0), router.size(1)}),
+                       nw.defined() ? std::optional<Tensor>(nw) : std::nullopt, router, eps);
+    return op(Q, K, U, V, R, one_part).transpose(1, 2);
+}
+
 struct BlockNode : torch::autograd::Function<BlockNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight,
                           const Tensor& router, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& w2, double eps,
@@ -335,12 +351,15 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
     {
         const auto s = ctx->get_saved_variables();
         const Tensor &x = s[0], &w1 = s[1], &nw = s[2], &router = s[3], &K = s[4], &U = s[5], &V = s[6], &w2 = s[7], &x4 = s[8],
-                     &wn = s[9], &wr = s[10], &q4 = s[11], &R = s[12], &O4 = s[13];
+                     &wn = s[9], &wr = s[10], &q4 = s[11], &R = s[12];
         const int64_t hid = x.size(2);
+        Tensor O4 = s[13];
+        if (at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
+            O4 = stepwise_O4(x, w1, nw, router, K, U, V, ctx->saved_data["eps"].toDouble(), ctx->saved_data["one_part"].toBool());
         // (the products of a linear layer's own backward: d_in = d_out w, d_w = d_out^T in)
         const Tensor dY = grads[0].reshape({-1, hid});
         const Tensor dO = at::mm(dY, w2).view(O4.sizes());
-        const Tensor dw2 = at::mm(dY.t(), O4.view({-1, hid}));
+        const Tensor dw2 = at::mm(dY.t(), O4.reshape({-1, hid}));
         auto g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type(), ctx->saved_data["one_part"].toBool());
         auto h = gate_backward(x4, nw, router, wn, wr, ctx->saved_data["eps"].toDouble(), g[0], g[4]);
         const Tensor dp = h[0].view({-1, hid});
@@ -368,13 +387,17 @@ RopeForward rope_forward(const Tensor& qkv, const Tensor& cos, const Tensor& sin
     TORCH_CHECK(qkv.dim() == 3 && qkv.is_contiguous() && qkv.is_cuda() && cos.is_contiguous() && sin.is_contiguous() &&
                     cos.sizes() == sin.sizes() && cos.dim() == 2 && cos.size(0) == qkv.size(1) && qkv.size(2) == 3 * H * cos.size(1),
                 "expected qkv [B,S,3*H*d] contiguous on the GPU and cos, sin [S,d]");
-    for (const Tensor* t : {&qkv, &cos, &sin}) TORCH_CHECK_TYPE(t->scalar_type() == at::kBFloat16, "rotary positions are bfloat16 here");
+    for (const Tensor* t : {&qkv, &cos, &sin}) {
+        TORCH_CHECK_TYPE(t->scalar_type() == at::kBFloat16, "rotary positions are bfloat16 here");
+        TORCH_CHECK(t->device() == qkv.device(), "cos and sin must be on the device of qkv, ", qkv.device());
+    }
     const int64_t B = qkv.size(0), S = qkv.size(1), d = cos.size(1);
     OnDevice guard(qkv);
     RopeForward f;
     f.q = empty_of({B, S, H, d}, at::kBFloat16, qkv);
     f.k = empty_of({B, S, H, d}, at::kBFloat16, qkv);
-    raise_for_code(mhffn_rope_fwd(ptr(qkv), ptr(cos), ptr(sin), ptr(f.q), ptr(f.k), (int)B, (int)S, (int)H, (int)d, stream()), "mhffn_rope");
+    const Tensor src = on_boundary(qkv), c = on_boundary(cos), s = on_boundary(sin);
+    raise_for_code(mhffn_rope_fwd(ptr(src), ptr(c), ptr(s), ptr(f.q), ptr(f.k), (int)B, (int)S, (int)H, (int)d, stream()), "mhffn_rope");
     f.q = f.q.transpose(1, 2);
     f.k = f.k.transpose(1, 2);
     f.v = qkv.view({B, S, 3, H, d}).select(2, 2).transpose(1, 2);
@@ -384,7 +407,7 @@ struct RopeNode : torch::autograd::Function<RopeNode> {
     static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
     {
         RopeForward f = rope_forward(qkv, cos, sin, H);
-        ctx->save_for_backward({cos, sin});
+        ctx->save_for_backward({on_boundary(cos), on_boundary(sin)});
         return {f.q, f.k, f.v};
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
@@ -432,6 +455,14 @@ PYBIND11_MODULE(_native, m)
     m.def("op", torch::wrap_pybind_function_no_gil(op));
     m.def("single", torch::wrap_pybind_function_no_gil(single));
     m.def("gate", torch::wrap_pybind_function_no_gil(gate));
+    m.def("gate_backward", torch::wrap_pybind_function_no_gil(
+                               [](const Tensor& x, const std::optional<Tensor>& norm_weight, const Tensor& router, double eps,
+                                  const std::optional<Tensor>& dQ, const std::optional<Tensor>& dR) {
+                                   const Tensor nw = norm_weight.value_or(Tensor());
+                                   variable_list g = gate_backward(contig(x), nw, router, gate_param(nw), gate_param(router), eps,
+                                                                   dQ.value_or(Tensor()), dR.value_or(Tensor()));
+                                   return std::make_tuple(g[0], g[1].defined() ? std::optional<Tensor>(g[1]) : std::nullopt, g[2]);
+                               }));
     m.def("rope", torch::wrap_pybind_function_no_gil(rope));
     m.def("block", torch::wrap_pybind_function_no_gil(block));
 }

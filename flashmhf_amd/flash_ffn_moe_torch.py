@@ -13,7 +13,7 @@ from .flash_mlp_moe import mhffn_backward, mhffn_forward
 class FlashFFNMoEFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, Q, K, U, V, R):
-        O = mhffn_forward(Q, K, U, V, R)
+        O = _capi.traced(mhffn_forward(Q, K, U, V, R))
         ctx.save_for_backward(Q, K, U, V, R)
         return O
 
@@ -29,4 +29,6 @@ class FlashFFNMoE(torch.nn.Module):
         super().__init__()
 
     def forward(self, Q, K, U, V, R):
+        if not _capi.native_nodes():
+            return FlashFFNMoEFunction.apply(Q, K, U, V, R)
         return _capi.native().op(Q, K, U, V, R, False)

@@ -10,6 +10,7 @@ It is the E = 1, R = 1 case of the fused MoE operator (which is what runs), with
 import torch
 
 from . import _capi
+from .flash_mlp_moe import FlashMLPFunction
 
 
 class FlashMLP(torch.nn.Module):
@@ -25,4 +26,7 @@ class FlashMLP(torch.nn.Module):
             raise ValueError("FlashMLP SiLU variant requires up-projection tensor U (got None)")
         if K.dim() != 3:
             raise RuntimeError("expected K/U/V [Hkuv, intermediate, d_h]")
+        if not _capi.native_nodes():
+            ones = torch.ones(*Q.shape[:3], 1, dtype=torch.float32, device=Q.device)
+            return FlashMLPFunction.apply(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones)
         return _capi.native().single(Q, K, U, V)

@@ -36,28 +36,34 @@ def mhffn_backward(Q, K, U, V, R, dO, grad_w_dtype=torch.bfloat16, one_part=Fals
 class FlashMLPFunction(torch.autograd.Function):
     """forward(ctx, Q, K, U, V, R) -> O ; backward(ctx, dO) -> (dQ, dK, dU, dV, dR).
     Mirrors kernels/triton/flash_mlp_moe.py:739-868.  (The modules record the same node natively, with a tenth of the host
-    time; this class is the boundary for callers that use the reference's ``FlashMLPFunction.apply``.)"""
+    time, where ``_capi.native_nodes()`` allows it; this class is for the other cases and for callers that use the
+    reference's ``FlashMLPFunction.apply``.)"""
 
     @staticmethod
-    def forward(ctx, Q, K, U, V, R):
-        O = mhffn_forward(Q, K, U, V, R)
+    def forward(ctx, Q, K, U, V, R, one_part=False):
+        O = _capi.traced(mhffn_forward(Q, K, U, V, R, one_part))
         ctx.save_for_backward(Q, K, U, V, R)
+        ctx.one_part = one_part
         return O
 
     @staticmethod
     def backward(ctx, grad_output):
         Q, K, U, V, R = ctx.saved_tensors
         assert grad_output.shape == Q.shape, "grad_output shape should be the same as Q"
-        return mhffn_backward(Q, K, U, V, R, grad_output, grad_w_dtype=K.dtype)
+        return (*mhffn_backward(Q, K, U, V, R, grad_output, grad_w_dtype=K.dtype, one_part=ctx.one_part), None)
 
 
 class FlashMLPMoE(torch.nn.Module):
     """Stateless module, ``forward(Q, K, U, V, R) -> O``.  Mirrors kernels/triton/flash_mlp_moe.py:871-903.
     ``one_part``: see ``mhffn_forward``; O, dQ and dR of a token then do not depend on the other tokens of the call."""
 
+    one_part = False        # (of modules saved before there was a choice)
+
     def __init__(self, one_part=False):
         super().__init__()
         self.one_part = one_part
 
     def forward(self, Q, K, U, V, R):
+        if not _capi.native_nodes():
+            return FlashMLPFunction.apply(Q, K, U, V, R, self.one_part)
         return _capi.native().op(Q, K, U, V, R, self.one_part)

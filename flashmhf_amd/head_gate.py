@@ -9,13 +9,29 @@ and ``R`` is [B,H,S,E] float32.  With ``norm_weight=None`` no normalisation happ
 The backward takes dQ (either layout) and dR and returns dx4, d_norm_weight and d_router, recomputing the forward from
 ``x4``: nothing but the inputs is saved.  bfloat16 only, d_h in {64, 96, 128}, E <= 64; no CPU path.
 """
+import torch
+
 from . import _capi
 
 
+class HeadNormGateFunction(torch.autograd.Function):
+    """The node of ``head_norm_gate`` as a torch.autograd.Function, for where the native one cannot run
+    (``_capi.native_nodes``)."""
+
+    @staticmethod
+    def forward(ctx, x4, norm_weight, router, eps):
+        ctx.save_for_backward(x4, norm_weight, router)
+        ctx.eps = float(eps)
+        Q, R = _capi.native().gate(x4, norm_weight, router, ctx.eps)
+        return _capi.traced(Q), _capi.traced(R)
+
+    @staticmethod
+    def backward(ctx, dQ, dR):
+        x4, norm_weight, router = ctx.saved_tensors
+        return (*_capi.native().gate_backward(x4, norm_weight, router, ctx.eps, dQ, dR), None)
+
+
 def head_norm_gate(x4, norm_weight, router, eps=1e-6):
+    if not _capi.native_nodes():
+        return HeadNormGateFunction.apply(x4, norm_weight, router, eps)
     return _capi.native().gate(x4, norm_weight, router, float(eps))
-
-
-class HeadNormGateFunction:
-    """The autograd node of ``head_norm_gate`` under the name and call of a torch.autograd.Function."""
-    apply = staticmethod(head_norm_gate)

@@ -149,7 +149,8 @@ class MHFFNLayer(nn.Module):
                 and self.num_experts <= 32 and self.head_dim in (64, 96, 128) and type(m["op"]) is FlashMLPMoE
                 and all(type(w) is nn.Linear and w.bias is None and _unhooked(w) for w in (m["w_self"], m["w_self_2"]))
                 and ("q_norm" not in m or type(m["q_norm"]) is RMSNorm and _unhooked(m["q_norm"])) and _unhooked(m["op"])
-                and not torch.is_autocast_enabled("cuda") and not _global_hooks()
+                and not torch.is_autocast_enabled("cuda") and not _global_hooks() and _capi.native_nodes()
+                and not torch.overrides.has_torch_function((x, self.w_self.weight, self.w_self_2.weight))
                 and self.w_self.weight.dtype == self.w_self_2.weight.dtype == self.K.dtype == self.U.dtype == self.V.dtype
                 == torch.bfloat16)
 
@@ -188,8 +189,11 @@ class CausalSelfAttention(nn.Module):
         B, S, hid = x.shape
         cos, sin = rope if rope is not None else _rotary(S, self.head_dim, self.rope_base, x.device, x.dtype)
         qkv = self.qkv(x)
-        if qkv.is_cuda and qkv.dtype == cos.dtype == torch.bfloat16 and self.head_dim % 16 == 0:
-            q, k, v = _capi.native().rope(qkv.contiguous(), cos, sin, self.num_heads)     # one pass, the same roundings
+        if (qkv.is_cuda and qkv.dtype == cos.dtype == sin.dtype == torch.bfloat16 and self.head_dim % 16 == 0 and qkv.numel()
+                and all(t.shape == (S, self.head_dim) and t.device == qkv.device and not t.requires_grad for t in (cos, sin))
+                and _capi.native_nodes()):
+            # one pass, the same roundings
+            q, k, v = _capi.native().rope(qkv.contiguous(), cos.contiguous(), sin.contiguous(), self.num_heads)
         else:
             q, k, v = qkv.view(B, S, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
             q, k = _apply_rotary(q, cos, sin), _apply_rotary(k, cos, sin)
@@ -231,19 +235,27 @@ class MHFFNDecoder(nn.Module):
 
     def _rope_tables(self, seq_len, device, dtype):
         """The rotary tables of one sequence length, kept for the next call of that length on the same stream (a dozen small
-        launches).  Tables made while a graph is captured belong to the graph, inference tensors cannot be saved for a
-        backward: neither are kept."""
+        launches).  A captured graph makes tables of its own: it outlives the kept ones, and what it makes belongs to it.
+        Inference tensors cannot be saved for a backward, and under a trace, a transform or a fake-tensor mode the tables
+        are not plain tensors: none of these are kept."""
         attn = self.blocks[0].attn
         on_gpu = device.type == "cuda"
+        if on_gpu and torch.cuda.is_current_stream_capturing() or not _capi.native_nodes():
+            return _rotary(seq_len, attn.head_dim, attn.rope_base, device, dtype)
         key = (seq_len, attn.head_dim, attn.rope_base, device, dtype,
                torch.cuda.current_stream(device).cuda_stream if on_gpu else None)
         kept = self.__dict__.get("_rope_kept")
         if kept is not None and kept[0] == key:
             return kept[1]
         tables = _rotary(seq_len, attn.head_dim, attn.rope_base, device, dtype)
-        if not torch.is_inference_mode_enabled() and not (on_gpu and torch.cuda.is_current_stream_capturing()):
+        if type(tables[0]) is torch.Tensor and not tables[0].is_inference():
             self.__dict__["_rope_kept"] = (key, tables)
         return tables
+
+    def __getstate__(self):
+        state = super().__getstate__()
+        state.pop("_rope_kept", None)       # (not of the module: copies and files go without)
+        return state
 
     def forward(self, ids, labels=None):
         x = self.embed(ids)
