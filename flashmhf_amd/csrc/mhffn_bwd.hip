@@ -302,27 +302,21 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsig
         const unsigned r = i / (DH / 8), c = (i % (DH / 8)) * 8;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
-        f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
-        for (int z = 1; z < p.parts.nsplit; ++z) {
-            src += hrows * DH;
-            lo += *reinterpret_cast<const f32x4*>(src);
-            hi += *reinterpret_cast<const f32x4*>(src + 4);
-        }
+        auto load = [&](int z) { return *reinterpret_cast<const f32x8*>(src + z * hrows * DH); };
+        const f32x8 sum = sum_in_order(load(0), 1, p.parts.nsplit, load);
         bf16x8 v;
 #pragma unroll
-        for (int x = 0; x < 4; ++x) { v[x] = (bf16_t)lo[x]; v[4 + x] = (bf16_t)hi[x]; }
+        for (int x = 0; x < 8; ++x) v[x] = (bf16_t)sum[x];
         *reinterpret_cast<bf16x8*>(p.dQ + p.rows.tok(hk, r) * DH + c) = v;
     } else {
         const unsigned i = (blockIdx.x - dq_blocks) * 256 + threadIdx.x;
-        const int E = p.parts.E, nbe = p.parts.nbe;
+        const int E = p.parts.E;
         const unsigned r = i / (unsigned)E;
         const int e = i - r * E;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + p.parts.nsplit * hrows * DH + ((long)hk * p.rows.n + r) * E + e;
-        float sum = 0.0f;
-        for (int z = 0; z < p.parts.nsplit; ++z)
-            if (p.parts.first(z) < (e + 1) * nbe && p.parts.first(z + 1) > e * nbe) sum += src[z * hrows * E];
-        p.dR[p.rows.gate(hk, r) * E + e] = sum;
+        p.dR[p.rows.gate(hk, r) * E + e] =
+            sum_in_order(0.0f, p.parts.part_lo(e), p.parts.part_hi(e), [&](int z) { return src[z * hrows * E]; });
     }
 }
 
@@ -815,24 +809,22 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     }
 }
 
-// Sums the token-slice partials and converts to the output dtype.  HBM-bound: reads nslice*3*|W| fp32 once.
+// Sums the token-slice partials of dK, dU or dV (blockIdx.y) and converts to the output dtype, four values per lane.
 template <typename OutT>
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ part, OutT* dK, OutT* dU, OutT* dV,
                                                               long wsz, int nslice)
 {
+    typedef OutT OutT4 __attribute__((ext_vector_type(4)));
     const long i4 = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i4 >= wsz) return;
-    OutT* outs[3] = {dK, dU, dV};
+    const int w = blockIdx.y;
+    const float* src = part + w * wsz + i4;
+    auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + 3 * z * wsz); };
+    const f32x4 sum = sum_in_order(load(0), 1, nslice, load);
+    OutT4 v;
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
-        f32x4 acc = *reinterpret_cast<const f32x4*>(part + w * wsz + i4);
-        for (int z = 1; z < nslice; ++z) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(part + ((long)z * 3 + w) * wsz + i4);
-            acc += v;
-        }
-#pragma unroll
-        for (int x = 0; x < 4; ++x) outs[w][i4 + x] = (OutT)acc[x];
-    }
+    for (int x = 0; x < 4; ++x) v[x] = (OutT)sum[x];
+    *reinterpret_cast<OutT4*>((w == 0 ? dK : w == 1 ? dU : dV) + i4) = v;
 }
 
 // ------------------------------------------------------------------------------------------------ host side
@@ -932,10 +924,10 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
         const long wsz = (long)d.Hkuv * d.E * d.d_e * d.d_h;
         const unsigned rblocks = (unsigned)((wsz / 4 + 255) / 256);
         if (grad_w_f32)
-            hipLaunchKernelGGL((reduce_partials_kernel<float>), dim3(rblocks), dim3(256), 0, st, part, (float*)dK,
+            hipLaunchKernelGGL((reduce_partials_kernel<float>), dim3(rblocks, 3), dim3(256), 0, st, part, (float*)dK,
                                (float*)dU, (float*)dV, wsz, nslice);
         else
-            hipLaunchKernelGGL((reduce_partials_kernel<bf16_t>), dim3(rblocks), dim3(256), 0, st, part, (bf16_t*)dK,
+            hipLaunchKernelGGL((reduce_partials_kernel<bf16_t>), dim3(rblocks, 3), dim3(256), 0, st, part, (bf16_t*)dK,
                                (bf16_t*)dU, (bf16_t*)dV, wsz, nslice);
         err = hipGetLastError();
     }

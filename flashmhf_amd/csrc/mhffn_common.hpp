@@ -26,6 +26,7 @@ typedef __bf16 bf16_t;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));   // 16-byte copy unit (native vector: stays in registers)
 
@@ -454,7 +455,40 @@ struct Parts {
     Parts(int E_, int nbe_, int nsplit_) : E(E_), nbe(nbe_), nsplit(nsplit_), by_nbe(nbe_), by_nsplit(nsplit_) {}
     // first block of part z (z = nsplit: the end); E * nbe * nsplit < 2^31
     __device__ __forceinline__ int first(int z) const { return by_nsplit.div(E * nbe * z); }
+    // the parts that hold blocks of expert e: part_lo(e) .. part_hi(e) - 1 (every part has a block: nsplit <= E * nbe)
+    __host__ __device__ __forceinline__ int part_lo(int e) const
+    {
+        const unsigned t = (unsigned)E * nbe;
+        return (((unsigned)e * nbe + 1u) * nsplit + t - 1) / t - 1;
+    }
+    __host__ __device__ __forceinline__ int part_hi(int e) const { return ((e + 1u) * nsplit + E - 1) / E; }
 };
+
+// acc + load(z0) + load(z0 + 1) + .. + load(z1 - 1), added in this order, with up to eight loads in flight: a summing pass
+// has few lanes and a load of partial sums takes 0.1 us or more, so one load per addition made such a pass a chain of
+// latencies.  z0, z1 wave-uniform or not.
+template <int N, class T, class Load>
+__device__ __forceinline__ void add_batch(T& acc, int z, Load&& load)
+{
+    T x[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) x[k] = load(z + k);
+#pragma unroll
+    for (int k = 0; k < N; ++k) acc += x[k];
+}
+template <class T, class Load>
+__device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
+{
+    int z = z0;
+    for (; z + 8 <= z1; z += 8) add_batch<8>(acc, z, load);
+    if (z + 4 <= z1) { add_batch<4>(acc, z, load); z += 4; }
+    switch (z1 - z) {
+        case 3: add_batch<3>(acc, z, load); break;
+        case 2: add_batch<2>(acc, z, load); break;
+        case 1: add_batch<1>(acc, z, load); break;
+    }
+    return acc;
+}
 
 // Into how many parts the forward and the dQ/dR kernel cut the blocks of a head, and which of a kernel's tile heights runs.
 // One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute

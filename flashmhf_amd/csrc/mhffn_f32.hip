@@ -451,18 +451,15 @@ __global__ __launch_bounds__(256) void sum_f32_kernel(F32Args p, float* dst, uns
         const int c = (i - r * (DH / 4)) * 4;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
-        f32x4 sum = *reinterpret_cast<const f32x4*>(src);
-        for (int z = 1; z < p.parts.nsplit; ++z) sum += *reinterpret_cast<const f32x4*>(src + z * hrows * DH);
-        *reinterpret_cast<f32x4*>(dst + p.rows.tok(hk, r) * DH + c) = sum;
+        auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + z * hrows * DH); };
+        *reinterpret_cast<f32x4*>(dst + p.rows.tok(hk, r) * DH + c) = sum_in_order(load(0), 1, p.parts.nsplit, load);
     } else {
         const unsigned i = (blockIdx.x - row_blocks) * 256 + threadIdx.x, r = i / (unsigned)E;
-        const int e = i - r * E, nbe = p.parts.nbe;
+        const int e = i - r * E;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + p.parts.nsplit * hrows * DH + ((long)hk * p.rows.n + r) * E + e;
-        float sum = 0.0f;
-        for (int z = 0; z < p.parts.nsplit; ++z)
-            if (p.parts.first(z) < (e + 1) * nbe && p.parts.first(z + 1) > e * nbe) sum += src[z * hrows * E];
-        p.dR[p.rows.gate(hk, r) * E + e] = sum;
+        p.dR[p.rows.gate(hk, r) * E + e] =
+            sum_in_order(0.0f, p.parts.part_lo(e), p.parts.part_hi(e), [&](int z) { return src[z * hrows * E]; });
     }
 }
 
@@ -474,9 +471,7 @@ __global__ __launch_bounds__(256) void reduce_f32_kernel(const float* __restrict
     if (i >= wsz) return;
     OutT* outs[3] = {dK, dU, dV};
     for (int w = 0; w < 3; ++w) {
-        float acc = 0.0f;
-        for (int z = 0; z < nslice; ++z) acc += part[((long)z * 3 + w) * wsz + i];
-        outs[w][i] = (OutT)acc;
+        outs[w][i] = (OutT)sum_in_order(0.0f, 0, nslice, [&](int z) { return part[((long)z * 3 + w) * wsz + i]; });
     }
 }
 

@@ -374,15 +374,11 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
     if (r >= (unsigned)p.rows.n) return;
     const long step = (long)p.rows.Hkuv * p.rows.n * DH;
     const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
-    f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
-    for (int z = 1; z < p.parts.nsplit; ++z) {
-        src += step;
-        lo += *reinterpret_cast<const f32x4*>(src);
-        hi += *reinterpret_cast<const f32x4*>(src + 4);
-    }
+    auto load = [&](int z) { return *reinterpret_cast<const f32x8*>(src + z * step); };
+    const f32x8 sum = sum_in_order(load(0), 1, p.parts.nsplit, load);
     bf16x8 v;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) { v[x] = (bf16_t)lo[x]; v[4 + x] = (bf16_t)hi[x]; }
+    for (int x = 0; x < 8; ++x) v[x] = (bf16_t)sum[x];
     *reinterpret_cast<bf16x8*>(p.O + p.rows.tok(hk, r) * DH + c) = v;
 }
 

@@ -651,16 +651,7 @@ __global__ __launch_bounds__(256) void mhffn_gate_sum_kernel(const float* part, 
     const int i = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, nr = dh * E, n = nr + dh;
     if (i >= n || (i >= nr && !dWn)) return;
     const float* src = part + (long)h * wgs * n + i;
-    float v = 0.0f;
-    int w = 0;
-    for (; w + 8 <= wgs; w += 8) {      // (eight loads in flight)
-        float x[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) x[k] = src[(long)(w + k) * n];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v += x[k];
-    }
-    for (; w < wgs; ++w) v += src[(long)w * n];
+    const float v = sum_in_order(0.0f, 0, wgs, [&](int w) { return src[(long)w * n]; });
     const bool r = i < nr;
     void* dst = r ? dWr : dWn;
     const long at = r ? (long)h * nr + i : (long)h * dh + i - nr;
