@@ -115,7 +115,7 @@ EXPECTED_KERNELS = (
     ("mhffn_gate_fwd_kernel", 12), ("mhffn_gate_bwd_kernel", 12),
 )
 # Variants of those kernels for smaller problems, under the same rule.
-VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3),)
+VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3))
 # The one instantiation known to spill: head prologue backward for d_h = 128 with more than 32 experts and RMSNorm
 # (<128, 2, true>).  It is correct but slow; the block (MHFFNLayer.heads_and_gate) does not route that case to it.
 ALLOWED_SCRATCH = ("mhffn_gate_bwd_kernelILi128ELi2ELb1E",)

@@ -290,6 +290,210 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
     }
 }
 
+// 32 rows, four blocks a trip: the same products, element-wise formulas and order of sums as the kernel above.  K and U tiles
+// are read by all waves to the end of a trip, V only by its own wave's first products.  K tiles have two sets; LDS has no
+// room for a second set of U too, whose next tile waits in registers instead.  dR is one running sum over the elements of an
+// expert's blocks: wave k adds those of its block to what wave k - 1 left, in the k-th of the four phases in which all
+// waves take the second products of block k (an exchange of the terms would take another 32 KB of LDS; the phases cost 0.35 of
+// a trip's 2.7 us).  All three tiles through registers: 2.95 us a trip without the phases.
+constexpr int DQ32_U0 = 2 * QUAD * TILE_B, DQ32_V0 = DQ32_U0 + QUAD * TILE_B, DQ32_D0 = DQ32_V0 + QUAD * TILE_B,
+              DQ32_E0 = DQ32_D0 + QUAD * 4096, DQ32_R0 = DQ32_E0 + 256;
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
+{
+    constexpr int KS = DH / 16, CT = DH / 32;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    float* sR = reinterpret_cast<float*>(smem + DQ32_R0);                 // [E][32]
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
+    const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
+    const int nex = p.parts.by_nbe.div(jb0 + nblk + nbe - 1);
+    const bf16_t* Kh = p.K + ((long)hk * E * nbe + blk0) * JB * DH;
+    const long offU = p.U - p.K, offV = p.V - p.K;
+    unsigned char *ownU = smem + DQ32_U0 + wave * TILE_B, *ownV = smem + DQ32_V0 + wave * TILE_B;
+    auto row_of = [&](int t) { return tok0 + t < p.rows.n ? tok0 + t : p.rows.n - 1; };
+    auto block = [&](int b0) { return Kh + (long)(b0 + wave < nblk ? b0 + wave : nblk - 1) * JB * DH; };
+    auto fill_k = [&](int b0, int set) { quad_fill<DH>(block(b0), smem + (set * QUAD + wave) * TILE_B, lane); };
+    // U through registers, coalesced as the fills are: row lane / 16 of every group of four, 16-byte chunk lane % 16 (a narrow
+    // row's unused chunks take chunk 0)
+    u32x4 un[8];
+    auto load_u = [&](int b0) {
+        const int c = (lane & 15) < DH / 8 ? lane & 15 : 0;
+        const bf16_t* src = block(b0) + offU + (lane >> 4) * DH + c * 8;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) un[i] = *reinterpret_cast<const u32x4*>(src + 4 * i * DH);
+    };
+    auto store_u = [&]() {
+        static_for<8>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            const int r = 4 * i + (lane >> 4);
+            lds_write16<0>(lds_addr(ownU) + r * TILE_ROW_B + (((lane & 15) ^ swz16(r)) << 4), un[i]);
+        });
+    };
+
+    bf16x8 q[KS], go[KS];
+    {
+        const long row = p.rows.tok(hk, row_of(l32)) * DH + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            q[ks] = *reinterpret_cast<const bf16x8*>(p.Q + row + ks * 16);
+            go[ks] = *reinterpret_cast<const bf16x8*>(p.dO + row + ks * 16);
+        }
+    }
+    quad_stage_gates(sR, p.R + ex0, nex, tid, [&](int t) { return p.rows.gate(hk, row_of(t)) * E; });
+    // (from here to the end of the loop the vmcnt events are the fills, the loads of U and the stores of dR)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]), "+v"(go[ks]));
+    __syncthreads();          // the gate values
+    load_u(0);
+    fill_k(0, 0);
+    quad_fill<DH>(block(0) + offV, ownV, lane);
+    float* drow;
+    {
+        const int t = row_of(l32);
+        const long hrows = (long)p.rows.Hkuv * p.rows.n;
+        drow = nsplit == 1 ? p.dR + p.rows.gate(hk, t) * E
+                           : p.part + nsplit * hrows * DH + (z * hrows + (long)hk * p.rows.n + t) * E + ex0;
+    }
+    f32x16 dq;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) dq[x] = 0.0f;
+    const int krow = row_perm32(l32);
+    const TrLane<CT> trl = make_tr_lane<CT, 8, 4>(lane);
+    TrLane<1> tr{};                           // this wave's column tile
+#pragma unroll
+    for (int i = 0; i < CT; ++i)
+        if (i == wave) { tr.off[0][0] = trl.off[i][0]; tr.off[0][1] = trl.off[i][1]; }
+    const unsigned smem0 = lds_addr(smem), rowoff = krow * TILE_ROW_B, sw = swz16(krow), ra = lds_addr(sR) + 4 * l32;
+    const unsigned sD = smem0 + DQ32_D0 + lane * 16, sE = smem0 + DQ32_E0 + lane * 4;
+
+    auto trip = [&](auto set_, int b0) {
+        constexpr int SET = decltype(set_)::value;
+        const unsigned sK = smem0 + SET * QUAD * TILE_B;
+        __builtin_amdgcn_sched_barrier(0);
+        store_u();            // (the barrier before was every wave's last use of the tile)
+        load_u(b0 + QUAD);
+        fill_k(b0 + QUAD, 1 - SET);
+        // this wave's K and V of the trip have landed: the sixteen loads just issued are younger (stores of dR in between only
+        // make the wait longer)
+        wait_vmcnt<16>();
+        __builtin_amdgcn_sched_barrier(0);
+        u32x2 rv = lds_read_apart_async<1>(ra + 128 * p.parts.by_nbe.div(jb0 + (b0 + wave < nblk ? b0 + wave : nblk - 1)));
+        QuadRows<KS, 3> a;
+        static_for<KS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            const unsigned at = rowoff + (((2 * ks + g) ^ sw) << 4);
+            a.template request<0, ks>(sK + wave * TILE_B + at);
+            a.template request<1, ks>(lds_addr(ownU) + at);
+            a.template request<2, ks>(lds_addr(ownV) + at);
+        });
+        f32x16 m, n, da;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) { m[x] = 0.0f; n[x] = 0.0f; da[x] = 0.0f; }
+        static_for<KS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            a.template wait<ks>();
+            m = mfma32(a.get(0, ks), q[ks], m);
+            n = mfma32(a.get(1, ks), q[ks], n);
+            da = mfma32(a.get(2, ks), go[ks], da);
+        });
+        asm volatile("" : "+v"(rv));
+        __builtin_amdgcn_sched_barrier(0);
+        quad_fill<DH>(block(b0 + QUAD) + offV, ownV, lane);      // (every read of the tile has returned)
+        bf16x8 dmt[2], dnt[2];
+        f32x16 as;            // the first factors of dR's terms (n holds the second ones)
+        {
+            const unsigned rbits = rv[0];
+            const float r = __builtin_bit_cast(float, rbits);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float x = m[i], nn = n[i], a = da[i];
+                const float sg = fast_sigmoid(x);
+                const float sl = x * sg;                 // silu(m)
+                as[i] = a * sl;
+                const float w = __builtin_fmaf(sl, 1.0f - sg, sg);    // silu'(m)
+                dnt[i >> 3][i & 7] = (bf16_t)(r * as[i]);
+                dmt[i >> 3][i & 7] = (bf16_t)((r * a) * (nn * w));
+            }
+        }
+        lds_write16<0>(sD + wave * 4096, dmt[0]);
+        lds_write16<1024>(sD + wave * 4096, dmt[1]);
+        lds_write16<2048>(sD + wave * 4096, dnt[0]);
+        lds_write16<3072>(sD + wave * 4096, dnt[1]);
+        quad_barrier();       // the four blocks' operands and tiles
+        const int nb = nblk - b0 < QUAD ? nblk - b0 : QUAD;     // (a block that is not there is the last one again, and not used)
+        // a block's operands (twelve LDS operations) are requested one block ahead of their use
+        u32x4 d[2][4];        // dM s 0, 1, dN s 0, 1
+        TrOperand tk[2][2], tu[2][2];
+        auto request = [&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            const unsigned aK = sK + k * TILE_B, aU = smem0 + DQ32_U0 + k * TILE_B;
+            tk[k & 1][0] = tile_read_cols_async<0>(aK, tr, 0);
+            tu[k & 1][0] = tile_read_cols_async<0>(aU, tr, 0);
+            tk[k & 1][1] = tile_read_cols_async<4096>(aK, tr, 0);
+            tu[k & 1][1] = tile_read_cols_async<4096>(aU, tr, 0);
+            d[k & 1][0] = lds_read16_async<k * 4096>(sD);
+            d[k & 1][1] = lds_read16_async<k * 4096 + 1024>(sD);
+            d[k & 1][2] = lds_read16_async<k * 4096 + 2048>(sD);
+            d[k & 1][3] = lds_read16_async<k * 4096 + 3072>(sD);
+        };
+        request(std::integral_constant<int, 0>{});
+        static_for<QUAD>([&](auto kc) {
+            constexpr int k = decltype(kc)::value, c = k & 1;
+            if (k == wave && k < nb) {
+                const int at = jb0 + b0 + k, e = p.parts.by_nbe.div(at), jb = at - e * nbe;
+                u32x2 in = lds_read_apart_async<1>(sE);
+                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(in));
+                const unsigned bits = in[0];
+                float dr = jb == 0 || b0 + k == 0 ? 0.0f : __builtin_bit_cast(float, bits);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) dr = __builtin_fmaf(as[i], n[i], dr);
+                lds_write4(sE, dr);
+                if (jb == nbe - 1 || b0 + k == nblk - 1) {
+                    const float tot = dr + __shfl_xor(dr, 32);      // the lane halves hold disjoint j rows of one token column
+                    if (g == 0 && tok0 + l32 < p.rows.n) drow[e] = tot;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (k + 1 < QUAD) request(std::integral_constant<int, k + 1>{});
+            constexpr int younger = k + 1 < QUAD ? 12 : 0;
+            lds_tr_wait_n<younger>(tk[c][0], tu[c][0]);
+            lds_tr_wait_n<younger>(tk[c][1], tu[c][1]);
+            asm volatile("" : "+v"(d[c][0]), "+v"(d[c][1]), "+v"(d[c][2]), "+v"(d[c][3]));
+            if (k < nb && wave < CT)
+                static_for<2>([&](auto sc) {
+                    constexpr int s = decltype(sc)::value;
+                    dq = mfma32(tr_value(tk[c][s]), __builtin_bit_cast(bf16x8, d[c][s]), dq);
+                    dq = mfma32(tr_value(tu[c][s]), __builtin_bit_cast(bf16x8, d[c][2 + s]), dq);
+                });
+            // the next wave's running sum; behind the last phase, every wave is done with the tiles and the operands
+            if constexpr (k + 1 < QUAD) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (k == wave) lds_wait_n<0>();
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            } else quad_barrier();
+        });
+    };
+    for (int b0 = 0; b0 < nblk; b0 += 2 * QUAD) {
+        trip(std::integral_constant<int, 0>{}, b0);
+        if (b0 + QUAD < nblk) trip(std::integral_constant<int, 1>{}, b0 + QUAD);
+    }
+    wait_vmcnt<0>();          // the fills of blocks that are not there write this wave's tiles, which the epilogue reuses
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave >= CT) return;
+    const int nrows = p.rows.n - tok0;
+    if (nsplit > 1) {
+        float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH + 32 * wave;
+        quad_store_f32(ownV, dq, nrows, lane, [&](int row) { return prow + row * DH; });
+    } else {
+        quad_store_bf16(ownV, dq, nrows, lane, [&](int row) { return p.dQ + p.rows.tok(hk, tok0 + row) * DH + 32 * wave; });
+    }
+}
+
 // Adds the parts' sums of dQ (in the order of the parts) and rounds once, eight columns per lane; adds the sums of dR over the
 // parts that hold blocks of the expert, one value per lane.  blockIdx.x < dq_blocks: dQ, otherwise dR.
 template <int DH>
@@ -857,17 +1061,20 @@ static int pick_nslice(const Dims& d, size_t ws_bytes)
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
-constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33}};
-static int dq_nsplit(const Dims& d, size_t ws_bytes)
+// Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.7 us (four steps of the
+// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 512 rows: 204 us with 256 rows, 87 with
+// 32; 2,048 rows: 204 and 172 (two rounds); with parts, one row 15 and 12.7 us.
+constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33, 1}, {32, 2.7, 0.05, QUAD}};
+static Pick dq_pick(const Dims& d, size_t ws_bytes)
 {
-    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), ws_bytes).nsplit;
+    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), ws_bytes);
 }
 
 // The two kernels run one after the other, so the parts of dQ, dR and the token slices of dK, dU, dV share the workspace.
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
     const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
-    const int ns = pick_nslice(d, ~(size_t)0), nq = dq_nsplit(d, ~(size_t)0);
+    const int ns = pick_nslice(d, ~(size_t)0), nq = dq_pick(d, ~(size_t)0).nsplit;
     const size_t dw = ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
     const size_t dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
     return dw > dq ? dw : dq;
@@ -883,17 +1090,21 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     const int nbe = d.d_e / JB, G = d.H / d.Hkuv;
 
     if (phases & PH_BWD_DQDR) {
+        const Pick pick = dq_pick(d, ws && !(phases & PH_ONE_PART) ? ws_bytes : 0);
         DqArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R,
                  (bf16_t*)dQ, dR, part, RowMap(d),
-                 Parts(d.E, nbe, dq_nsplit(d, ws && !(phases & PH_ONE_PART) ? ws_bytes : 0))};
-        const int tokw = 256;
-        const int smem = DQ_NST * DQ_STAGE_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
+                 Parts(d.E, nbe, pick.nsplit)};
+        const int tokw = pick.tile_rows;
+        const int smem = (tokw == 32 ? DQ32_R0 : DQ_NST * DQ_STAGE_B) +
+                         (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
         if (smem > 160 * 1024) return hipErrorInvalidValue;
-        static LdsOptIn optin;
-        err = ensure_dynamic_lds(optin, (const void*)mhffn_bwd_dqdr_kernel<DH>, smem);
+        static LdsOptIn optin, optin32;
+        err = tokw == 32 ? ensure_dynamic_lds(optin32, (const void*)mhffn_bwd_dqdr_rows32_kernel<DH>, smem)
+                         : ensure_dynamic_lds(optin, (const void*)mhffn_bwd_dqdr_kernel<DH>, smem);
         if (err != hipSuccess) return err;
         dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
-        hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
+        if (tokw == 32) hipLaunchKernelGGL((mhffn_bwd_dqdr_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
+        else hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
         if (a.parts.nsplit > 1) {
             const unsigned qb = (unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256);
             const unsigned rb = (unsigned)(((long)a.rows.n * d.E + 255) / 256);

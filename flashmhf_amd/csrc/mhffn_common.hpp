@@ -321,6 +321,102 @@ __device__ __forceinline__ void store_rows_f32(unsigned char* region, float* dst
     });
 }
 
+// ---- tiles of 32 rows, four blocks at a time ------------------------------------------------------------------------
+// With few rows the tiles of 128 and 256 rows leave most of the chip idle, and a workgroup walks a head's blocks one after
+// the other.  The rows32 kernels put the four waves of a workgroup on four consecutive blocks of the same 32 rows instead:
+// a wave takes the first products and the element-wise work of its own block, hands the rounded result to the others
+// through LDS, and then adds all four blocks, in their order, to the 32 output columns it owns: the sums are those of the
+// kernels with larger tiles bit for bit.
+// Every LDS access of their loops is inline assembly and every wait counted by hand: the compiler would put a wait for all
+// outstanding LDS-direct loads in front of each access.
+constexpr int QUAD = 4;                      // waves of a workgroup = blocks of a trip
+
+// Asynchronous fill of one 32-row tile by one wave: eight vmcnt events.
+template <int DH>
+__device__ __forceinline__ void quad_fill(const bf16_t* src, unsigned char* tile, int lane)
+{
+#pragma unroll
+    for (int i = 0; i < 8; ++i) tile_fill_ins<DH>(src, DH, tile, i, lane);
+}
+template <int IMM, class T>
+__device__ __forceinline__ void lds_write16(unsigned addr, const T& v)
+{
+    asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(__builtin_bit_cast(u32x4, v)), "n"(IMM));
+}
+__device__ __forceinline__ void lds_write4(unsigned addr, float v) { asm volatile("ds_write_b32 %0, %1" ::"v"(addr), "v"(v)); }
+// This wave's LDS operations are done, then the workgroup's; loads in flight stay in flight.
+__device__ __forceinline__ void quad_barrier()
+{
+    __builtin_amdgcn_sched_barrier(0);
+    lds_wait_n<0>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+}
+// Row-major operands of every k-step of up to three tiles (16-byte LDS reads, all requested before the first is used: the
+// wave is alone on its SIMD), and the wait for k-step KSI of the N tiles.
+template <int KS, int N>
+struct QuadRows {
+    u32x4 v[N][KS];
+    template <int T, int KSI>
+    __device__ __forceinline__ void request(unsigned rowaddr)      // address of the row's k-step 0 chunk position
+    {
+        v[T][KSI] = lds_read16_async<0>(rowaddr);
+    }
+    template <int KSI>
+    __device__ __forceinline__ void wait()
+    {
+        constexpr int younger = (KS - 1 - KSI) * N < 15 ? (KS - 1 - KSI) * N : 15;
+        lds_wait_n<younger>();
+#pragma unroll
+        for (int t = 0; t < N; ++t) asm volatile("" : "+v"(v[t][KSI]));
+    }
+    __device__ __forceinline__ bf16x8 get(int t, int ks) const { return __builtin_bit_cast(bf16x8, v[t][ks]); }
+};
+// Gate values of 32 rows, expert-major [nex][32]: R row address(t) of every row t (clamped by the caller), eight lanes per row.
+template <class Row>
+__device__ __forceinline__ void quad_stage_gates(float* sR, const float* R, int nex, int tid, Row&& address)
+{
+    const int t = tid >> 3;
+    const float* src = R + address(t);
+    for (int e = tid & 7; e < nex; e += 8) sR[e * 32 + t] = src[e];
+}
+// Stores a 32 x 32 tile held as an accumulator of a transposed product (register 4a + x of lane (l32, g): column 8a + 4g + x of
+// row l32) through 4 KB of LDS private to the wave, rows below nrows: fp32 to dst(row), or rounded to bf16.
+template <class Dst>
+__device__ __forceinline__ void quad_store_f32(unsigned char* region, const f32x16& acc, int nrows, int lane, Dst&& dst)
+{
+    const int l32 = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        f32x4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = acc[4 * a + x];
+        *reinterpret_cast<f32x4*>(region + l32 * 128 + (((2 * a + g) ^ (l32 & 7)) << 4)) = v;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int row = 8 * k + (lane >> 3), c = lane & 7;
+        if (row < nrows) *reinterpret_cast<f32x4*>(dst(row) + 4 * c) = *reinterpret_cast<const f32x4*>(region + row * 128 + ((c ^ (row & 7)) << 4));
+    }
+}
+template <class Dst>
+__device__ __forceinline__ void quad_store_bf16(unsigned char* region, const f32x16& acc, int nrows, int lane, Dst&& dst)
+{
+    const int l32 = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        bf16x4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = (bf16_t)acc[4 * a + x];
+        *reinterpret_cast<bf16x4*>(region + l32 * 64 + ((a ^ (l32 & 3)) << 4) + 8 * g) = v;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int row = 16 * k + (lane >> 2), c = lane & 3;
+        if (row < nrows) *reinterpret_cast<u32x4*>(dst(row) + 8 * c) = *reinterpret_cast<const u32x4*>(region + row * 64 + ((c ^ (row & 3)) << 4));
+    }
+}
+
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt[3:0] at bits 3:0, vmcnt[5:4] at bits 15:14; other counters unconstrained).
 template <int N>
 __device__ __forceinline__ void wait_vmcnt()
@@ -491,6 +587,7 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 }
 
 // Into how many parts the forward and the dQ/dR kernel cut the blocks of a head, and which of a kernel's tile heights runs.
+// The steps are measured times of each kernel on half a chip; a rows32 step is a trip of four blocks.
 // One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute
 // units a part per idle unit shortens the serial walk over the blocks (one token of the 370M layer: 8 tiles of 121 blocks,
 // 122 us with one part, 15 with 32), and every part costs a set of fp32 sums that is written and read back.  Time of a
@@ -504,6 +601,7 @@ constexpr long SPLIT_ROWS_BELOW = 16384;
 struct Variant {
     int tile_rows;
     double step, full;
+    int unit;             // blocks of a step
 };
 struct Pick {
     int tile_rows, nsplit;
@@ -517,12 +615,13 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
     Pick best{variants[0].tile_rows, 1};
     double best_us = 0;
     for (const Variant& v : variants) {
+        if (v.unit > 1 && !may_cut) continue;      // (the rows32 kernels keep all gate values of a tile in LDS)
         const long tiles = (rows + v.tile_rows - 1) / v.tile_rows * d.Hkuv;
         for (int ns = 1; ns <= most; ++ns) {
             if (ns > 1 && (ns * part_bytes > ws_bytes || tiles * (ns - 1) >= 2 * CUS)) break;
             const long wgs = tiles * ns;
             const double load = wgs <= CUS / 2 ? 0 : wgs >= CUS ? 1 : (wgs - CUS / 2) / (double)(CUS / 2);
-            const double us = (double)((wgs + CUS - 1) / CUS) * ((blocks + ns - 1) / ns * v.step * (1 + v.full * load) + 3) +
+            const double us = (double)((wgs + CUS - 1) / CUS) * (((blocks + ns - 1) / ns + v.unit - 1) / v.unit * v.step * (1 + v.full * load) + 3) +
                               (ns > 1 ? 2 + ns * part_us : 0);
             if (best_us == 0 || us < best_us) { best_us = us; best = Pick{v.tile_rows, ns}; }
         }

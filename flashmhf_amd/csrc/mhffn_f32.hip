@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256) void reduce_f32_kernel(const float* __restrict
 }
 
 // Parts of the blocks for the forward and dQ/dR as for bfloat16 (pick_parts).
-constexpr Variant F32_VARIANTS[] = {{128, 5.0, 0.0}};
+constexpr Variant F32_VARIANTS[] = {{128, 5.0, 0.0, 1}};
 int nbe_of(const Dims& d) { return (d.d_e + JB - 1) / JB; }
 size_t o_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }

@@ -364,6 +364,139 @@ __global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p) { fwd_body<DH
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_fwd_rows128_kernel(FwdArgs p) { fwd_body<DH, 1>(p); }
 
+// 32 rows, four blocks a trip: the same products, element-wise formula and order of sums as fwd_body.  One barrier a trip: P^T
+// operands and V tiles (which all waves read) have two sets, K and U tiles (which only their wave reads) are refilled as
+// soon as the first products have read them.  A trip is 1.43 us, bound by the issue of a lone wave and LDS; with the tiles loaded
+// to registers and written to LDS it was 2.15 (0.58 us of it the writes, 0.45 waiting for the loads).
+constexpr int FWD32_V0 = QUAD * 2 * TILE_B, FWD32_P0 = FWD32_V0 + 2 * QUAD * TILE_B, FWD32_R0 = FWD32_P0 + 2 * QUAD * 2048;
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_fwd_rows32_kernel(FwdArgs p)
+{
+    constexpr int KS = DH / 16, CT = DH / 32;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    float* sR = reinterpret_cast<float*>(smem + FWD32_R0);                       // [E][32]
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
+    const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
+    const int nex = p.parts.by_nbe.div(jb0 + nblk + nbe - 1);
+    const bf16_t* Kh = p.K + ((long)hk * E * nbe + blk0) * JB * DH;
+    const long offU = p.U - p.K, offV = p.V - p.K;
+    unsigned char* own = smem + wave * 2 * TILE_B;      // K | U of this wave's block
+    auto row_of = [&](int t) { return tok0 + t < p.rows.n ? tok0 + t : p.rows.n - 1; };
+    auto block = [&](int b0) { return Kh + (long)(b0 + wave < nblk ? b0 + wave : nblk - 1) * JB * DH; };
+    auto fill_v = [&](int b0, int set) { quad_fill<DH>(block(b0) + offV, smem + FWD32_V0 + (set * QUAD + wave) * TILE_B, lane); };
+    auto fill_ku = [&](int b0) {
+        quad_fill<DH>(block(b0), own, lane);
+        quad_fill<DH>(block(b0) + offU, own + TILE_B, lane);
+    };
+
+    bf16x8 q[KS];
+    {
+        const bf16_t* qr = p.Q + p.rows.tok(hk, row_of(l32)) * DH + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) q[ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16);
+    }
+    quad_stage_gates(sR, p.R + ex0, nex, tid, [&](int t) { return p.rows.gate(hk, row_of(t)) * E; });
+    // (the compiler's own loads and stores end here; from the next line on the vmcnt events are the fills)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]));
+    __syncthreads();          // the gate values
+    fill_ku(0);
+    fill_v(0, 0);
+    f32x16 o;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) o[x] = 0.0f;
+    const int krow = row_perm32(l32);
+    const TrLane<CT> trl = make_tr_lane<CT, 8, 4>(lane);
+    TrLane<1> tr{};                           // this wave's column tile
+#pragma unroll
+    for (int i = 0; i < CT; ++i)
+        if (i == wave) { tr.off[0][0] = trl.off[i][0]; tr.off[0][1] = trl.off[i][1]; }
+    const unsigned own_row = lds_addr(own) + krow * TILE_ROW_B, sw = swz16(krow);
+    const unsigned smem0 = lds_addr(smem), ra = lds_addr(sR) + 4 * l32;
+
+    auto trip = [&](auto set_, int b0) {
+        constexpr int SET = decltype(set_)::value;
+        bf16x8 pt[2];
+        wait_vmcnt<8>();      // this wave's K and U of the trip have landed, its V (issued behind them) may be in flight
+        __builtin_amdgcn_sched_barrier(0);
+        u32x2 rv = lds_read_apart_async<1>(ra + 128 * p.parts.by_nbe.div(jb0 + (b0 + wave < nblk ? b0 + wave : nblk - 1)));
+        QuadRows<KS, 2> a;
+        static_for<KS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            const unsigned at = own_row + (((2 * ks + g) ^ sw) << 4);
+            a.template request<0, ks>(at);
+            a.template request<1, ks>(at + TILE_B);
+        });
+        f32x16 m, n;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) { m[x] = 0.0f; n[x] = 0.0f; }
+        static_for<KS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            a.template wait<ks>();
+            m = mfma32(a.get(0, ks), q[ks], m);
+            n = mfma32(a.get(1, ks), q[ks], n);
+        });
+        asm volatile("" : "+v"(rv));
+        __builtin_amdgcn_sched_barrier(0);
+        fill_ku(b0 + QUAD);   // (every read of the two tiles has returned)
+        const unsigned rbits = rv[0];
+        const float rinv = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(__builtin_bit_cast(float, rbits)), -FLT_MAX_F, FLT_MAX_F);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float ex = __builtin_amdgcn_exp2f(-LOG2E * m[i]);
+            const float xn = m[i] * n[i];
+            pt[i >> 3][i & 7] = (bf16_t)(xn * __builtin_amdgcn_rcpf(__builtin_fmaf(ex, rinv, rinv)));
+        }
+        const unsigned sP = smem0 + FWD32_P0 + SET * QUAD * 2048 + lane * 16;
+        lds_write16<0>(sP + wave * 2048, pt[0]);
+        lds_write16<1024>(sP + wave * 2048, pt[1]);
+        wait_vmcnt<16>();     // this wave's V has landed, the next K and U may be in flight
+        quad_barrier();       // the four blocks' P^T and V tiles; and every wave is done with the trip before
+        fill_v(b0 + QUAD, 1 - SET);
+        if (wave < CT) {
+            // (a block that is not there is the last one again, and not used)
+            const int nb = nblk - b0 < QUAD ? nblk - b0 : QUAD;
+            u32x4 pv[QUAD][2];
+            TrOperand v[QUAD][2];
+            static_for<QUAD>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const unsigned sV = smem0 + FWD32_V0 + (SET * QUAD + k) * TILE_B;
+                pv[k][0] = lds_read16_async<k * 2048>(sP);
+                pv[k][1] = lds_read16_async<k * 2048 + 1024>(sP);
+                v[k][0] = tile_read_cols_async<0>(sV, tr, 0);
+                v[k][1] = tile_read_cols_async<4096>(sV, tr, 0);
+            });
+            static_for<QUAD>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                lds_tr_wait_n<(QUAD - 1 - k) * 6 < 15 ? (QUAD - 1 - k) * 6 : 15>(v[k][0], v[k][1]);
+                asm volatile("" : "+v"(pv[k][0]), "+v"(pv[k][1]));
+                if (k < nb) {
+                    o = mfma32(tr_value(v[k][0]), __builtin_bit_cast(bf16x8, pv[k][0]), o);
+                    o = mfma32(tr_value(v[k][1]), __builtin_bit_cast(bf16x8, pv[k][1]), o);
+                }
+            });
+        }
+    };
+    for (int b0 = 0; b0 < nblk; b0 += 2 * QUAD) {
+        trip(std::integral_constant<int, 0>{}, b0);
+        if (b0 + QUAD < nblk) trip(std::integral_constant<int, 1>{}, b0 + QUAD);
+    }
+    wait_vmcnt<0>();          // the fills of blocks that are not there write this wave's tiles, which the epilogue reuses
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave >= CT) return;
+    const int nrows = p.rows.n - tok0;
+    if (nsplit > 1) {
+        float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH + 32 * wave;
+        quad_store_f32(own, o, nrows, lane, [&](int row) { return prow + row * DH; });
+    } else {
+        quad_store_bf16(own, o, nrows, lane, [&](int row) { return p.O + p.rows.tok(hk, tok0 + row) * DH + 32 * wave; });
+    }
+}
+
 // Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, eight columns per lane.
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
@@ -385,8 +518,10 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // Tiles of 256 rows (64 per wave) where they fill the chip; of 128 (32 per wave) below that: a step then takes 0.6 us
 // instead of 1.0, with 20 % less throughput once every compute unit has one (16,384 tokens of the 370M layer: 342 us with 256
 // rows, 407 with 128; 1,500 tokens in one part: 131 and 85; 733 tokens: 33 and 32 us at each one's best number of parts,
-// of the 128M layer 25.5 and 21.4).  Rows have the same sums, bit for bit, in either.
-constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2}, {128, 0.6, 0.33}};
+// of the 128M layer 25.5 and 21.4).  Of 32, four blocks a trip of 1.43 us, below that: one token of the 370M layer 12.7 -> 10.3
+// us, 16 tokens of the 1.3B layer 21.2 -> 17.8 us (95 MB of weights, 5.3 TB/s), 512 rows in one part 84 -> 49 us.  Rows have
+// the same sums, bit for bit, in all three.
+constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 static Pick fwd_pick(const Dims& d, size_t ws_bytes)
 {
@@ -396,15 +531,19 @@ static Pick fwd_pick(const Dims& d, size_t ws_bytes)
 template <int DH>
 static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, hipStream_t st)
 {
-    const int smem = FWD_RING_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * 256 * (int)sizeof(float);
+    const int gates = d.E < GATE_WIN ? d.E : GATE_WIN;
+    const int smem = tile_rows == 32 ? FWD32_R0 + gates * 32 * (int)sizeof(float)
+                                     : FWD_RING_B + gates * 256 * (int)sizeof(float);
     if (smem > 160 * 1024) return hipErrorInvalidValue;
-    static LdsOptIn optin, optin128;
-    const hipError_t e = tile_rows == 256 ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
-                                          : ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem);
+    static LdsOptIn optin, optin128, optin32;
+    const hipError_t e = tile_rows == 256   ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
+                         : tile_rows == 128 ? ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem)
+                                            : ensure_dynamic_lds(optin32, (const void*)mhffn_fwd_rows32_kernel<DH>, smem);
     if (e != hipSuccess) return e;
     dim3 grid((unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv), (unsigned)a.parts.nsplit);
     if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
-    else hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(256), smem, st, a);
+    else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(256), smem, st, a);
+    else hipLaunchKernelGGL((mhffn_fwd_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
         dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256), (unsigned)d.Hkuv);
         hipLaunchKernelGGL((mhffn_fwd_sum_kernel<DH>), sgrid, dim3(256), 0, st, a);

@@ -48,15 +48,22 @@ def test_parts_match_the_oracle(case):
         assert_bf16_parity(name, got.float().cpu(), r, case)
 
 
-def test_one_part_does_not_depend_on_the_other_tokens():
+@pytest.mark.parametrize("case", [
+    (2, 4, 300, 128, 5, 96, 2, False),        # tiles of 32 rows, four blocks a trip, for all and for few
+    (2, 16, 2000, 128, 5, 96, 16, False),     # 256-row tiles against 32-row ones
+    (2, 16, 2000, 96, 3, 32, 16, True),       # ... three blocks: a trip that is not full
+    (2, 16, 1999, 64, 9, 32, 8, True),        # ... a ragged last tile of two q-heads; a trip of one block
+    (1, 8, 1500, 128, 3, 256, 8, False),
+])
+def test_one_part_does_not_depend_on_the_other_tokens(case):
     from flashmhf_amd import mhffn_backward, mhffn_forward
-    _, (Q, K, U, V, R, dO) = _run((2, 4, 300, 128, 5, 96, 2, False))
+    _, (Q, K, U, V, R, dO) = _run(case)
     O, g = mhffn_forward(Q, K, U, V, R, one_part=True), mhffn_backward(Q, K, U, V, R, dO, one_part=True)
     few = slice(37, 40)
-    q, r, d = (t[1:, :, few].contiguous() for t in (Q, R, dO))
+    q, r, d = (t[-1:, :, few].contiguous() for t in (Q, R, dO))
     o, h = mhffn_forward(q, K, U, V, r, one_part=True), mhffn_backward(q, K, U, V, r, d, one_part=True)
     for a, b in ((o, O), (h[0], g[0]), (h[4], g[4])):
-        assert torch.equal(a, b[1:, :, few])
+        assert torch.equal(a, b[-1:, :, few])
 
 
 @pytest.mark.parametrize("case", [
