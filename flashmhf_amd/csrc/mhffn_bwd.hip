@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
     }
 }
 
-// Adds the parts' sums of dQ (in the order of the parts) and rounds once, eight columns per lane; adds the sums of dR over the
+// Adds the parts' sums of dQ (in the order of the parts) and rounds once, four columns per lane; adds the sums of dR over the
 // parts that hold blocks of the expert, one value per lane.  blockIdx.x < dq_blocks: dQ, otherwise dR.
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsigned dq_blocks)
@@ -503,15 +503,15 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsig
     const long hrows = (long)p.rows.Hkuv * p.rows.n;
     if (blockIdx.x < dq_blocks) {
         const unsigned i = blockIdx.x * 256 + threadIdx.x;
-        const unsigned r = i / (DH / 8), c = (i % (DH / 8)) * 8;
+        const unsigned r = i / (DH / 4), c = (i % (DH / 4)) * 4;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
-        auto load = [&](int z) { return *reinterpret_cast<const f32x8*>(src + z * hrows * DH); };
-        const f32x8 sum = sum_in_order(load(0), 1, p.parts.nsplit, load);
-        bf16x8 v;
+        auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + z * hrows * DH); };
+        const f32x4 sum = sum_in_order(load(0), 1, p.parts.nsplit, load);
+        bf16x4 v;
 #pragma unroll
-        for (int x = 0; x < 8; ++x) v[x] = (bf16_t)sum[x];
-        *reinterpret_cast<bf16x8*>(p.dQ + p.rows.tok(hk, r) * DH + c) = v;
+        for (int x = 0; x < 4; ++x) v[x] = (bf16_t)sum[x];
+        *reinterpret_cast<bf16x4*>(p.dQ + p.rows.tok(hk, r) * DH + c) = v;
     } else {
         const unsigned i = (blockIdx.x - dq_blocks) * 256 + threadIdx.x;
         const int E = p.parts.E;
@@ -1106,7 +1106,7 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
         if (tokw == 32) hipLaunchKernelGGL((mhffn_bwd_dqdr_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
         else hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
         if (a.parts.nsplit > 1) {
-            const unsigned qb = (unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256);
+            const unsigned qb = (unsigned)(((long)a.rows.n * (DH / 4) + 255) / 256);
             const unsigned rb = (unsigned)(((long)a.rows.n * d.E + 255) / 256);
             hipLaunchKernelGGL((mhffn_bwd_dqdr_sum_kernel<DH>), dim3(qb + rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, qb);
         }

@@ -26,7 +26,6 @@ typedef __bf16 bf16_t;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));   // 16-byte copy unit (native vector: stays in registers)
 
@@ -560,28 +559,31 @@ struct Parts {
     __host__ __device__ __forceinline__ int part_hi(int e) const { return ((e + 1u) * nsplit + E - 1) / E; }
 };
 
-// acc + load(z0) + load(z0 + 1) + .. + load(z1 - 1), added in this order, with up to eight loads in flight: a summing pass
-// has few lanes and a load of partial sums takes 0.1 us or more, so one load per addition made such a pass a chain of
-// latencies.  z0, z1 wave-uniform or not.
+// acc + load(z0) + load(z0 + 1) + .. + load(z1 - 1), added in this order, with up to sixteen loads in flight: a summing pass
+// has few lanes and a load of partial sums takes half a microsecond, so one load per addition made such a pass a chain of
+// latencies.  A last batch of more than four is filled up with loads of the last element, which are not added (31 parts: two
+// latencies instead of the five of batches of 8, 8, 8, 4, 2).
 template <int N, class T, class Load>
-__device__ __forceinline__ void add_batch(T& acc, int z, Load&& load)
+__device__ __forceinline__ void add_batch(T& acc, int z, int z1, Load&& load)
 {
     T x[N];
 #pragma unroll
-    for (int k = 0; k < N; ++k) x[k] = load(z + k);
+    for (int k = 0; k < N; ++k) x[k] = load(z + k < z1 ? z + k : z1 - 1);
 #pragma unroll
-    for (int k = 0; k < N; ++k) acc += x[k];
+    for (int k = 0; k < N; ++k)
+        if (z + k < z1) acc += x[k];
 }
 template <class T, class Load>
 __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 {
     int z = z0;
-    for (; z + 8 <= z1; z += 8) add_batch<8>(acc, z, load);
-    if (z + 4 <= z1) { add_batch<4>(acc, z, load); z += 4; }
+    for (; z + 8 < z1; z += 16) add_batch<16>(acc, z, z1, load);
     switch (z1 - z) {
-        case 3: add_batch<3>(acc, z, load); break;
-        case 2: add_batch<2>(acc, z, load); break;
-        case 1: add_batch<1>(acc, z, load); break;
+        case 8: case 7: case 6: case 5: add_batch<8>(acc, z, z1, load); break;
+        case 4: add_batch<4>(acc, z, z1, load); break;
+        case 3: add_batch<3>(acc, z, z1, load); break;
+        case 2: add_batch<2>(acc, z, z1, load); break;
+        case 1: add_batch<1>(acc, z, z1, load); break;
     }
     return acc;
 }

@@ -497,22 +497,22 @@ __global__ __launch_bounds__(256) void mhffn_fwd_rows32_kernel(FwdArgs p)
     }
 }
 
-// Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, eight columns per lane.
+// Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, four columns per lane.
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 {
     const unsigned i = blockIdx.x * 256 + threadIdx.x;
-    const unsigned r = i / (DH / 8), c = (i % (DH / 8)) * 8;
+    const unsigned r = i / (DH / 4), c = (i % (DH / 4)) * 4;
     const int hk = blockIdx.y;
     if (r >= (unsigned)p.rows.n) return;
     const long step = (long)p.rows.Hkuv * p.rows.n * DH;
     const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
-    auto load = [&](int z) { return *reinterpret_cast<const f32x8*>(src + z * step); };
-    const f32x8 sum = sum_in_order(load(0), 1, p.parts.nsplit, load);
-    bf16x8 v;
+    auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + z * step); };
+    const f32x4 sum = sum_in_order(load(0), 1, p.parts.nsplit, load);
+    bf16x4 v;
 #pragma unroll
-    for (int x = 0; x < 8; ++x) v[x] = (bf16_t)sum[x];
-    *reinterpret_cast<bf16x8*>(p.O + p.rows.tok(hk, r) * DH + c) = v;
+    for (int x = 0; x < 4; ++x) v[x] = (bf16_t)sum[x];
+    *reinterpret_cast<bf16x4*>(p.O + p.rows.tok(hk, r) * DH + c) = v;
 }
 
 // Tiles of 256 rows (64 per wave) where they fill the chip; of 128 (32 per wave) below that: a step then takes 0.6 us
@@ -545,7 +545,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, h
     else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(256), smem, st, a);
     else hipLaunchKernelGGL((mhffn_fwd_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
-        dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 8) + 255) / 256), (unsigned)d.Hkuv);
+        dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 4) + 255) / 256), (unsigned)d.Hkuv);
         hipLaunchKernelGGL((mhffn_fwd_sum_kernel<DH>), sgrid, dim3(256), 0, st, a);
     }
     return hipGetLastError();
