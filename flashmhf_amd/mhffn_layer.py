@@ -69,6 +69,12 @@ def _unhooked(m):
     return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
 
 
+def _runs_own_forward(m, cls):
+    """Whether calling `m` runs the `forward` that `cls` was defined with and nothing else: not a subclass's, the instance's or
+    a patched one, no hooks.  A fused path may stand in for such a call only."""
+    return type(m) is cls and cls.forward is _FORWARD[cls] and "forward" not in m.__dict__ and _unhooked(m)
+
+
 def _global_hooks():
     g = nn.modules.module
     return g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks
@@ -125,9 +131,11 @@ class MHFFNLayer(nn.Module):
         H, dh, E = self.num_heads, self.head_dim, self.num_experts
         q = self.w_self(x).view(B, S, H, dh)
         # (d_h = 128 with more than 32 experts and RMSNorm is left to torch: that instantiation of the prologue's backward
-        # kernel does not fit the register file and runs several times slower than it should)
+        # kernel does not fit the register file and runs several times slower than it should; so is a q_norm with code of its
+        # own, which the kernel would pass by)
         if (self.fused_prologue and self.router_input == "q" and q.dtype == torch.bfloat16 and q.is_cuda
-                and E <= 64 and dh in (64, 96, 128) and not (dh == 128 and E > 32 and self.q_norm is not None)):
+                and E <= 64 and dh in (64, 96, 128)
+                and (self.q_norm is None or _runs_own_forward(self.q_norm, RMSNorm) and not (dh == 128 and E > 32))):
             return head_norm_gate(q, None if self.q_norm is None else self.q_norm.weight, self.router,
                                   self.rms_norm_eps)
         if self.q_norm is not None:
@@ -139,20 +147,29 @@ class MHFFNLayer(nn.Module):
             logits = (x.float() @ self.w_router.float()).view(B, S, H, E).transpose(1, 2)
         return Q, router_gate(logits).contiguous()
 
+    def _stock_steps(self):
+        """Whether every step of the block is this module's own: heads_and_gate, and plain bias-free projections, RMSNorm and
+        operator, with no override in a subclass, on an instance or on a patched class and no hook that would have a say;
+        K, U, V and the router plain parameters (a parametrization computes them anew on every access)."""
+        m, p = self._modules, self._parameters
+        return (type(self).heads_and_gate is _HEADS_AND_GATE and "heads_and_gate" not in self.__dict__
+                and _runs_own_forward(m.get("op"), FlashMLPMoE)
+                and all(_runs_own_forward(w, nn.Linear) and w.bias is None for w in (m.get("w_self"), m.get("w_self_2")))
+                and (self.q_norm is None or _runs_own_forward(self.q_norm, RMSNorm))
+                and all(p.get(n) is not None for n in ("K", "U", "V", "router")) and not _global_hooks())
+
     def _one_node(self, x):
         """Whether the block can run as one native node (projection, prologue, operator, projection: the same kernels and
-        library products as the steps below, a quarter of the host time): bfloat16 on the GPU with the default operator
-        and plain bias-free projections that no hook, subclass or autocast context would have a say in.  (More than 32
-        experts take the prologue's two-tile instances, which heads_and_gate chooses among.)"""
-        m = self._modules
-        return (self.router_input == "q" and self.fused_prologue and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 3
-                and self.num_experts <= 32 and self.head_dim in (64, 96, 128) and type(m["op"]) is FlashMLPMoE
-                and all(type(w) is nn.Linear and w.bias is None and _unhooked(w) for w in (m["w_self"], m["w_self_2"]))
-                and ("q_norm" not in m or type(m["q_norm"]) is RMSNorm and _unhooked(m["q_norm"])) and _unhooked(m["op"])
-                and not torch.is_autocast_enabled("cuda") and not _global_hooks() and _capi.native_nodes()
-                and not torch.overrides.has_torch_function((x, self.w_self.weight, self.w_self_2.weight))
-                and self.w_self.weight.dtype == self.w_self_2.weight.dtype == self.K.dtype == self.U.dtype == self.V.dtype
-                == torch.bfloat16)
+        library products as the steps below, a quarter of the host time): bfloat16 on the GPU, with steps that are all its
+        own and no autocast context or tensor subclass that would change them.  (More than 32 experts take the prologue's
+        two-tile instances, which heads_and_gate chooses among.)"""
+        if not (self.router_input == "q" and self.fused_prologue and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 3
+                and self.num_experts <= 32 and self.head_dim in (64, 96, 128) and self._stock_steps()
+                and not torch.is_autocast_enabled("cuda") and _capi.native_nodes()):
+            return False
+        weights = (self.w_self.weight, self.w_self_2.weight, self.K, self.U, self.V)
+        return (all(w.dtype == torch.bfloat16 for w in weights)
+                and not torch.overrides.has_torch_function((x, *weights, self.router)))
 
     def forward(self, x):
         B, S, hid = x.shape
@@ -162,6 +179,11 @@ class MHFFNLayer(nn.Module):
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
+
+
+# what _stock_steps compares with: the code as it is defined here
+_FORWARD = {c: c.forward for c in (nn.Linear, RMSNorm, FlashMLPMoE)}
+_HEADS_AND_GATE = MHFFNLayer.heads_and_gate
 
 
 def _rotary(seq_len, head_dim, base, device, dtype):
