@@ -403,6 +403,41 @@ RopeForward rope_forward(const Tensor& qkv, const Tensor& cos, const Tensor& sin
     f.v = qkv.view({B, S, 3, H, d}).select(2, 2).transpose(1, 2);
     return f;
 }
+// dqkv [B,S,3*H*d] of gradients of q, k, v [B,H,S,d] of any strides
+Tensor rope_backward(Tensor dq, Tensor dk, Tensor dv, const Tensor& cos, const Tensor& sin)
+{
+    long strides[9];
+    Tensor* g[3] = {&dq, &dk, &dv};
+    for (int w = 0; w < 3; ++w) {
+        if (g[w]->stride(3) != 1) *g[w] = g[w]->contiguous();
+        for (int i = 0; i < 3; ++i) strides[3 * w + i] = g[w]->stride(i);
+    }
+    const int64_t B = dq.size(0), H = dq.size(1), S = dq.size(2), d = dq.size(3);
+    OnDevice guard(dq);
+    Tensor dqkv = empty_of({B, S, 3 * H * d}, at::kBFloat16, dq);
+    raise_for_code(mhffn_rope_bwd(ptr(dq), ptr(dk), ptr(dv), strides, ptr(cos), ptr(sin), ptr(dqkv), (int)B, (int)S, (int)H, (int)d,
+                                  stream()),
+                   "mhffn_rope");
+    return dqkv;
+}
+std::tuple<Tensor, Tensor, Tensor> rope(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H);
+
+// The backward as a node of its own, for create_graph: the map is linear in dq, dk, dv and its transpose is the forward.
+struct RopeBackNode : torch::autograd::Function<RopeBackNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& cos, const Tensor& sin)
+    {
+        ctx->save_for_backward({cos, sin});
+        ctx->saved_data["H"] = dq.size(1);
+        return rope_backward(dq, dk, dv, cos, sin);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        auto [q, k, v] = rope(contig(g[0]), s[0], s[1], ctx->saved_data["H"].toInt());
+        return {q, k, v, Tensor(), Tensor()};
+    }
+};
+
 struct RopeNode : torch::autograd::Function<RopeNode> {
     static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
     {
@@ -413,21 +448,13 @@ struct RopeNode : torch::autograd::Function<RopeNode> {
     static variable_list backward(AutogradContext* ctx, variable_list g)
     {
         const auto s = ctx->get_saved_variables();
-        long strides[9];
         Tensor any;
-        for (Tensor& t : g)
+        for (const Tensor& t : g)
             if (t.defined()) any = t;
-        for (int w = 0; w < 3; ++w) {
-            if (!g[w].defined()) g[w] = at::zeros_like(any);
-            if (g[w].stride(3) != 1) g[w] = g[w].contiguous();
-            for (int i = 0; i < 3; ++i) strides[3 * w + i] = g[w].stride(i);
-        }
-        const int64_t B = any.size(0), H = any.size(1), S = any.size(2), d = any.size(3);
-        OnDevice guard(any);
-        Tensor dqkv = empty_of({B, S, 3 * H * d}, at::kBFloat16, any);
-        raise_for_code(mhffn_rope_bwd(ptr(g[0]), ptr(g[1]), ptr(g[2]), strides, ptr(s[0]), ptr(s[1]), ptr(dqkv), (int)B, (int)S, (int)H,
-                                      (int)d, stream()),
-                       "mhffn_rope");
+        for (Tensor& t : g)
+            if (!t.defined()) t = at::zeros_like(any);
+        const Tensor dqkv = records_grad({&g[0], &g[1], &g[2]}) ? RopeBackNode::apply(g[0], g[1], g[2], s[0], s[1])
+                                                                : rope_backward(g[0], g[1], g[2], s[0], s[1]);
         return {dqkv, Tensor(), Tensor(), Tensor()};
     }
 };

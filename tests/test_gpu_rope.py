@@ -29,3 +29,50 @@ def test_rope_is_the_element_wise_form(B, S, H, d, strided):
         assert all(torch.equal(x, y) for x, y in zip(_capi.native().rope(a, cos, sin, H), out))
     only_v = torch.autograd.grad(_capi.native().rope(a, cos, sin, H)[2], a, grads[2])[0].view(B, S, 3, H, d)
     assert torch.equal(only_v[:, :, 2], grads[2].transpose(1, 2)) and not only_v[:, :, :2].any()
+
+
+@pytest.mark.parametrize("B,S,H,d", [(1, 1, 1, 16), (2, 37, 3, 96)])
+def test_derivatives_of_the_gradient_are_the_element_wise_forms(B, S, H, d):
+    """create_graph: the gradient is a function of the outputs' gradients, and so on to any order (the map is linear)."""
+    from flashmhf_amd import _capi
+    dev = "cuda:0"
+    torch.manual_seed(S)
+    qkv = torch.randn(B, S, 3 * H * d, device=dev).bfloat16()
+    cos, sin = _rotary(S, d, 10000.0, torch.device(dev), torch.bfloat16)
+    grads = [torch.randn(B, H, S, d, device=dev).bfloat16() for _ in range(3)]
+    v2, v3 = torch.randn_like(qkv), [torch.randn(B, H, S, d, device=dev).bfloat16() for _ in range(3)]
+    results = []
+    for native in (True, False):
+        x, g = qkv.clone().requires_grad_(), [t.clone().requires_grad_() for t in grads]
+        if native:
+            out = _capi.native().rope(x, cos, sin, H)
+        else:
+            q, k, v = x.view(B, S, 3, H, d).permute(2, 0, 3, 1, 4)
+            out = _apply_rotary(q, cos, sin), _apply_rotary(k, cos, sin), v
+        dx, = torch.autograd.grad(out, x, g, create_graph=True)
+        w = v2.clone().requires_grad_()
+        dg = torch.autograd.grad(dx, g, w, create_graph=True)
+        dw, = torch.autograd.grad(dg, w, v3)
+        results.append([dx, *dg, dw])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
+def test_gradient_penalty_through_attention(monkeypatch):
+    """All terms of a second derivative, those behind q, k and v among them, against the element-wise rotary form (which tables
+    of another shape bring back).  The attention itself is a stand-in of element-wise products: which of torch's attention
+    kernels has a second derivative is not this module's business."""
+    from flashmhf_amd import mhffn_layer
+    from flashmhf_amd.mhffn_layer import CausalSelfAttention
+    monkeypatch.setattr(mhffn_layer.F, "scaled_dot_product_attention", lambda q, k, v, is_causal: torch.tanh(q) * k * v)
+    B, S, H, d = 2, 24, 2, 64
+    torch.manual_seed(0)
+    attn = CausalSelfAttention(H * d, H).to("cuda:0").to(torch.bfloat16)
+    x = torch.randn(B, S, H * d, device="cuda:0").bfloat16().requires_grad_()
+    cos, sin = _rotary(S, d, 10000.0, x.device, x.dtype)
+    results = []
+    for tables in ((cos, sin), (cos[None], sin[None])):
+        dx, = torch.autograd.grad(attn(x, rope=tables).float().sum(), x, create_graph=True)
+        results.append([dx, *torch.autograd.grad(dx.float().square().sum(), [x, *attn.parameters()])])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
