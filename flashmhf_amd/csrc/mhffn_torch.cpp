@@ -335,6 +335,7 @@ Tensor stepwise_O4(const Tensor& x, const Tensor& w1, const Tensor& nw, const Te
     return op(Q, K, U, V, R, one_part).transpose(1, 2);
 }
 
+// Only where every parameter takes a gradient (block() below): what it saves is then what the steps' own nodes would.
 struct BlockNode : torch::autograd::Function<BlockNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight,
                           const Tensor& router, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& w2, double eps,
@@ -352,20 +353,39 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const auto s = ctx->get_saved_variables();
         const Tensor &x = s[0], &w1 = s[1], &nw = s[2], &router = s[3], &K = s[4], &U = s[5], &V = s[6], &w2 = s[7], &x4 = s[8],
                      &wn = s[9], &wr = s[10], &q4 = s[11], &R = s[12];
+        const double eps = ctx->saved_data["eps"].toDouble();
+        const bool one_part = ctx->saved_data["one_part"].toBool();
         const int64_t hid = x.size(2);
-        Tensor O4 = s[13];
-        if (at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
-            O4 = stepwise_O4(x, w1, nw, router, K, U, V, ctx->saved_data["eps"].toDouble(), ctx->saved_data["one_part"].toBool());
+        // What this pass asks for (torch.autograd.grad may name a few inputs): a step whose results nobody asked for is left
+        // out, as the engine leaves out a node of its own.  The numbers count the tensors that went in: x, w1, nw if there is
+        // one, router, K, U, V, w2.
+        const size_t after_nw = nw.defined() ? 3 : 2;
+        auto asked = [&](size_t from, size_t to) {
+            for (size_t i = from; i < to; ++i)
+                if (ctx->needs_input_grad(i)) return true;
+            return false;
+        };
+        const bool prologue = asked(0, after_nw + 1), experts = asked(after_nw + 1, after_nw + 4);
+        Tensor dx, dw1, dw2;
+        variable_list g(5), h(3);
         // (the products of a linear layer's own backward: d_in = d_out w, d_w = d_out^T in)
         const Tensor dY = grads[0].reshape({-1, hid});
-        const Tensor dO = at::mm(dY, w2).view(O4.sizes());
-        const Tensor dw2 = at::mm(dY.t(), O4.reshape({-1, hid}));
-        auto g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type(), ctx->saved_data["one_part"].toBool());
-        auto h = gate_backward(x4, nw, router, wn, wr, ctx->saved_data["eps"].toDouble(), g[0], g[4]);
-        const Tensor dp = h[0].view({-1, hid});
-        Tensor dx;
-        if (ctx->needs_input_grad(0)) dx = at::mm(dp, w1).view(x.sizes());
-        const Tensor dw1 = at::mm(dp.t(), x.reshape({-1, hid}));
+        if (asked(after_nw + 4, after_nw + 5)) {
+            Tensor O4 = s[13];
+            if (at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
+                O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part);
+            dw2 = at::mm(dY.t(), O4.reshape({-1, hid}));
+        }
+        if (prologue || experts) {
+            const Tensor dO = at::mm(dY, w2).view(s[13].sizes());
+            g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type(), one_part);
+        }
+        if (prologue) {
+            h = gate_backward(x4, nw, router, wn, wr, eps, g[0], g[4]);
+            const Tensor dp = h[0].view({-1, hid});
+            if (ctx->needs_input_grad(0)) dx = at::mm(dp, w1).view(x.sizes());
+            if (ctx->needs_input_grad(1)) dw1 = at::mm(dp.t(), x.reshape({-1, hid}));
+        }
         return {dx, dw1, h[1], h[2], g[1], g[2], g[3], dw2, Tensor(), Tensor()};
     }
 };
@@ -375,6 +395,11 @@ Tensor block(const Tensor& x, const Tensor& w1, const std::optional<Tensor>& nor
     const Tensor nw = norm_weight.value_or(Tensor());
     if (!records_grad({&x, &w1, &nw, &router, &K, &U, &V, &w2}))
         return block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part).Y;
+    // With anything frozen (adapters, training of the experts alone) the steps record their own nodes: each saves what its
+    // own gradients need, and what nobody asks for is neither kept nor computed.
+    for (const Tensor* t : {&x, &w1, &nw, &router, &K, &U, &V, &w2})
+        if (t->defined() && !t->requires_grad())
+            return at::linear(stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part).reshape(x.sizes()), w2);
     return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps, one_part);
 }
 
