@@ -24,7 +24,7 @@ STATIC_SCRATCH_BYTES = 96 << 20
 
 EXPORTS = (
     "mhffn_strerror", "mhffn_is_supported", "mhffn_check_dims", "mhffn_fwd_workspace_bytes",
-    "mhffn_bwd_workspace_bytes", "mhffn_fwd", "mhffn_bwd", "mhffn_fwd_phases", "mhffn_bwd_phases",
+    "mhffn_bwd_workspace_bytes", "mhffn_bwd_workspace_min_bytes", "mhffn_fwd", "mhffn_bwd", "mhffn_fwd_phases", "mhffn_bwd_phases",
     "mhffn_fwd_layout", "mhffn_bwd_layout", "mhffn_bwd_static", "mhffn_gate_fwd", "mhffn_gate_bwd",
     "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into", "mhffn_rope_fwd", "mhffn_rope_bwd",
 )
@@ -54,7 +54,7 @@ def lib():
         L.mhffn_strerror.argtypes = [ctypes.c_int]
         L.mhffn_is_supported.argtypes = [ctypes.c_int] * 3
         L.mhffn_check_dims.argtypes = [dp, ctypes.c_int]
-        for f in (L.mhffn_fwd_workspace_bytes, L.mhffn_bwd_workspace_bytes):
+        for f in (L.mhffn_fwd_workspace_bytes, L.mhffn_bwd_workspace_bytes, L.mhffn_bwd_workspace_min_bytes):
             f.restype = ctypes.c_size_t
             f.argtypes = [dp, ctypes.c_int]
         L.mhffn_fwd.argtypes = [vp] * 6 + [vp, ctypes.c_size_t, dp, ctypes.c_int, vp]

@@ -1070,12 +1070,18 @@ static Pick dq_pick(const Dims& d, size_t ws_bytes)
     return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), ws_bytes);
 }
 
+size_t bwd_min_workspace_bytes_bf16(const Dims& d)
+{
+    const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
+    const int ns = pick_nslice(d, ~(size_t)0);
+    return ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
+}
+
 // The two kernels run one after the other, so the parts of dQ, dR and the token slices of dK, dU, dV share the workspace.
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
-    const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
-    const int ns = pick_nslice(d, ~(size_t)0), nq = dq_pick(d, ~(size_t)0).nsplit;
-    const size_t dw = ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
+    const int nq = dq_pick(d, ~(size_t)0).nsplit;
+    const size_t dw = bwd_min_workspace_bytes_bf16(d);
     const size_t dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
     return dw > dq ? dw : dq;
 }

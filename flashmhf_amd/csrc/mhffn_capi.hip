@@ -100,6 +100,12 @@ size_t mhffn_bwd_workspace_bytes(const mhffn_dims* dims, int dtype)
     return mhffn::bwd_workspace_bytes_bf16(to_dims(dims));
 }
 
+size_t mhffn_bwd_workspace_min_bytes(const mhffn_dims* dims, int dtype)
+{
+    if (check_dims_impl(dims, dtype) != MHFFN_OK) return 0;
+    return dtype == MHFFN_DTYPE_F32 ? mhffn::bwd_min_workspace_bytes_f32(to_dims(dims)) : mhffn::bwd_min_workspace_bytes_bf16(to_dims(dims));
+}
+
 int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
                      void* workspace, size_t workspace_bytes, const mhffn_dims* dims, int dtype, int token_layout,
                      void* stream, int phases)
@@ -151,15 +157,15 @@ int mhffn_bwd_layout(const void* Q, const void* K, const void* U, const void* V,
     for (const void* p : ptrs)
         if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
     const mhffn::Dims d = to_dims(dims, token_layout);
-    const size_t need = dtype == MHFFN_DTYPE_F32 ? mhffn::bwd_workspace_bytes_f32(d) : mhffn::bwd_workspace_bytes_bf16(d);
-    if (need > 0 && (!workspace || workspace_bytes < need)) return MHFFN_ERR_WORKSPACE;
+    const size_t ws_bytes = workspace ? workspace_bytes : 0;
+    if (ws_bytes < mhffn_bwd_workspace_min_bytes(dims, dtype)) return MHFFN_ERR_WORKSPACE;
     if (dtype == MHFFN_DTYPE_F32)
         return mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, workspace,
-                                     need, d, (hipStream_t)stream, phases) == hipSuccess
+                                     ws_bytes, d, (hipStream_t)stream, phases) == hipSuccess
                    ? MHFFN_OK
                    : MHFFN_ERR_LAUNCH;
     const hipError_t err = mhffn::launch_bwd_bf16(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR,
-                                                  grad_w_dtype == MHFFN_DTYPE_F32, workspace, need, d,
+                                                  grad_w_dtype == MHFFN_DTYPE_F32, workspace, ws_bytes, d,
                                                   (hipStream_t)stream, phases);
     return err == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
 }

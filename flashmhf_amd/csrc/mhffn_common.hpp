@@ -633,8 +633,10 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
 
 size_t fwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one part);
                                                       // with less it runs fewer parts
-size_t bwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one token
-                                                      // slice, no partial sums); with less it runs fewer slices
+size_t bwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely: the token slices of
+                                                      // dK, dU, dV and the parts of dQ, dR (0: one of each); with less it
+                                                      // runs fewer
+size_t bwd_min_workspace_bytes_bf16(const Dims& d);   // those of the token slices alone
 hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
                            void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases);
 hipError_t launch_bwd_bf16(const void* Q, const void* K, const void* U, const void* V, const float* R, const void* dO,
@@ -643,7 +645,8 @@ hipError_t launch_bwd_bf16(const void* Q, const void* K, const void* U, const vo
 
 // fp32 instantiation (mhffn_f32.hip): d_h a multiple of 8 up to 128, any d_e, any E.
 size_t fwd_workspace_bytes_f32(const Dims& d);        // as fwd_workspace_bytes_bf16
-size_t bwd_workspace_bytes_f32(const Dims& d);
+size_t bwd_workspace_bytes_f32(const Dims& d);        // as bwd_workspace_bytes_bf16, but the token slices are fixed:
+size_t bwd_min_workspace_bytes_f32(const Dims& d);    // the launch needs these
 hipError_t launch_fwd_f32(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
                           void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases);
 hipError_t launch_bwd_f32(const void* Q, const void* K, const void* U, const void* V, const float* R, const void* dO,

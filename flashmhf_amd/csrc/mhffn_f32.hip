@@ -562,11 +562,17 @@ size_t fwd_workspace_bytes_f32(const Dims& d)
     return ns > 1 ? ns * o_part_bytes(d) : 0;
 }
 
-// (at least one copy of dK, dU, dV, which the launch needs only where it slices the tokens: the size callers of
-// earlier versions reserve, and room for the parts of dQ, dR)
+// (at least one copy of dK, dU, dV, which the launch needs only where it slices the tokens: what callers of earlier versions
+// reserve)
+size_t bwd_min_workspace_bytes_f32(const Dims& d)
+{
+    return (size_t)f32_nslice(d) * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float);
+}
+
+// ... and room for the parts of dQ, dR
 size_t bwd_workspace_bytes_f32(const Dims& d)
 {
-    const size_t dw = (size_t)f32_nslice(d) * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float);
+    const size_t dw = bwd_min_workspace_bytes_f32(d);
     const int nq = parts_of(d, dq_part_bytes(d), ~(size_t)0);
     const size_t dq = nq > 1 ? nq * dq_part_bytes(d) : 0;
     return dw > dq ? dw : dq;

@@ -41,7 +41,7 @@ int dtype_code(at::ScalarType t)
 struct Plan {
     mhffn_dims dims;
     int dtype;
-    size_t fwd_bytes, bwd_bytes;
+    size_t fwd_bytes, bwd_bytes, bwd_min_bytes;
 };
 const Plan& plan_for(const mhffn_dims& d, int dtype)
 {
@@ -51,7 +51,8 @@ const Plan& plan_for(const mhffn_dims& d, int dtype)
     Plan& p = table[(h ^ (h >> 13)) & 63];
     if (memcmp(&p.dims, &d, sizeof d) != 0 || p.dtype != dtype) {
         raise_for_code(mhffn_check_dims(&d, dtype), "mhffn");
-        p = Plan{d, dtype, mhffn_fwd_workspace_bytes(&d, dtype), mhffn_bwd_workspace_bytes(&d, dtype)};
+        p = Plan{d, dtype, mhffn_fwd_workspace_bytes(&d, dtype), mhffn_bwd_workspace_bytes(&d, dtype),
+                 mhffn_bwd_workspace_min_bytes(&d, dtype)};
     }
     return p;
 }
@@ -148,10 +149,11 @@ variable_list op_backward(const Tensor& Q0, const Tensor& K0, const Tensor& U0, 
     const int dt = dtype_code(Q.scalar_type()), wdt = dtype_code(grad_w);
     const Plan& p = plan_for(dims_of(Q, K), dt);
     OnDevice guard(Q);
-    Tensor dQ = empty_like_layout(Q), dR = empty_of(R.sizes(), at::kFloat, Q), ws = scratch(p.bwd_bytes, Q);
+    const size_t ws_bytes = one_part ? p.bwd_min_bytes : p.bwd_bytes;
+    Tensor dQ = empty_like_layout(Q), dR = empty_of(R.sizes(), at::kFloat, Q), ws = scratch(ws_bytes, Q);
     Tensor dK = empty_of(K.sizes(), grad_w, Q), dU = empty_of(K.sizes(), grad_w, Q), dV = empty_of(K.sizes(), grad_w, Q);
     raise_for_code(mhffn_bwd_layout(ptr(Q), ptr(K), ptr(U), ptr(V), (const float*)ptr(R), ptr(dO), ptr(dQ), ptr(dK), ptr(dU), ptr(dV),
-                                    (float*)ptr(dR), wdt, ptr(ws), p.bwd_bytes, &p.dims, dt, layout, stream(),
+                                    (float*)ptr(dR), wdt, ptr(ws), ws_bytes, &p.dims, dt, layout, stream(),
                                     MHFFN_BWD_ALL | (one_part ? MHFFN_ONE_PART : 0)),
                    "mhffn_bwd");
     return {dQ, dK, dU, dV, dR};

@@ -40,7 +40,7 @@ enum {
     MHFFN_ERR_HEAD_DIM     = -3,  /* reference: assert head_dim == 128, flash_ffn_moe.cu:956 */
     MHFFN_ERR_EXPERT_DIM   = -4,  /* reference: ValueError, flash_mlp_moe.py:758-759; assert flash_ffn_moe.cu:958 */
     MHFFN_ERR_SHAPE        = -5,  /* non-positive extent, H not a multiple of Hkuv, gate kernels with E > 64 */
-    MHFFN_ERR_WORKSPACE    = -6,  /* backward: workspace missing or smaller than mhffn_bwd_workspace_bytes() */
+    MHFFN_ERR_WORKSPACE    = -6,  /* backward: workspace missing or smaller than mhffn_bwd_workspace_min_bytes() */
     MHFFN_ERR_LAUNCH       = -7,  /* hipGetLastError() after a launch */
     MHFFN_ERR_ALIGNMENT    = -8,  /* a tensor or workspace pointer is not 16-byte aligned */
     MHFFN_ERR_STATIC_SCRATCH = -9 /* mhffn_bwd_static only: the problem needs more than MHFFN_STATIC_SCRATCH_BYTES */
@@ -73,9 +73,13 @@ int mhffn_check_dims(const mhffn_dims* dims, int dtype);
  * themselves (e.g. the 370M and 1.3B layers at their benchmark sizes); `workspace` may then be NULL.
  *   - forward: the bytes are those of the fp32 partial sums with which a small number of tokens is computed fastest.  Any
  *     smaller workspace, NULL included, is accepted: the same result (up to fp32 summation order), with less of the GPU busy.
- *   - backward: the workspace is required. */
+ *   - backward: the bytes are the larger of the partial sums of dQ, dR (few tokens, as in the forward) and those of dK, dU, dV
+ *     (token slices).  The second are required and what mhffn_bwd_workspace_min_bytes reports; between the two sizes dQ and dR
+ *     are computed with less of the GPU busy, to the same result up to fp32 summation order.  A smaller workspace returns
+ *     MHFFN_ERR_WORKSPACE. */
 size_t mhffn_fwd_workspace_bytes(const mhffn_dims* dims, int dtype);
 size_t mhffn_bwd_workspace_bytes(const mhffn_dims* dims, int dtype);
+size_t mhffn_bwd_workspace_min_bytes(const mhffn_dims* dims, int dtype);
 
 /* Forward.  Replaces the launch in FlashMLPFunction.forward (flash_mlp_moe.py:777-790) and
  * flashffn_moe_forward (flash_ffn_moe.cu:938-1007).  O is written, nothing else. */

@@ -80,6 +80,24 @@ def test_backward_workspace_follows_the_token_slice_policy(L):
         assert L.mhffn_bwd_workspace_bytes(d, _capi.DTYPE_BF16) == want, (dims, slices)
 
 
+@pytest.mark.parametrize("dtype", [_capi.DTYPE_BF16, _capi.DTYPE_F32])
+def test_backward_needs_no_more_than_the_token_slices(L, dtype):
+    """The parts of dQ and dR are optional: what a backward call cannot do without is the token slices of dK, dU, dV, 0 where
+    those are one slice, and does not grow when there are few tokens."""
+    for H, Hk, dh, E, de in ((8, 8, 128, 11, 352), (16, 16, 128, 22, 352), (8, 2, 96, 8, 256), (2, 1, 64, 64, 32)):
+        slices = set()
+        for S in (1, 37, 300, 512, 733, 2048, 16384):
+            d = _capi.Dims(1, H, Hk, S, dh, E, de)
+            need, most = L.mhffn_bwd_workspace_min_bytes(d, dtype), L.mhffn_bwd_workspace_bytes(d, dtype)
+            slices.add(need // (3 * 4 * Hk * E * de * dh))
+            assert need <= most and need % (3 * 4 * Hk * E * de * dh) == 0
+        assert min(slices) == dtype and max(slices) <= 64
+        if dtype == _capi.DTYPE_BF16 and Hk * E * de // 128 >= 256 * 3 // 4:
+            assert slices == {0}        # the weight columns fill the chip: mhffn_bwd takes a NULL workspace at any S
+    assert L.mhffn_bwd_workspace_bytes(_capi.Dims(1, 8, 8, 512, 128, 11, 352), _capi.DTYPE_BF16) > 0
+    assert L.mhffn_bwd_workspace_min_bytes(_capi.Dims(1, 8, 3, 512, 128, 11, 352), dtype) == 0
+
+
 def test_entry_points_validate_before_touching_the_gpu(L):
     d = _capi.Dims(1, 2, 2, 64, 128, 2, 64)
     null = ctypes.c_void_p(0)
