@@ -183,16 +183,16 @@ int mhffn_bwd_static(const void* Q, const void* K, const void* U, const void* V,
     for (const void* p : ptrs)
         if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
     const mhffn::Dims d = to_dims(dims, token_layout);
-    // The float32 kernels take exactly the workspace they ask for.  The bfloat16 launch runs with as many token slices
-    // as the array holds partial sums for (with one slice it needs none), so it never exceeds the array.
-    const size_t need = dtype == MHFFN_DTYPE_F32 ? mhffn::bwd_workspace_bytes_f32(d) : 0;
+    // The bfloat16 launch runs with as many token slices and parts as the array holds partial sums for (with one it needs
+    // none), so it never exceeds the array.  So does the float32 launch with its parts; its token slices are fixed.
+    const size_t need = dtype == MHFFN_DTYPE_F32 ? mhffn::bwd_min_workspace_bytes_f32(d) : 0;
     if (need > MHFFN_STATIC_SCRATCH_BYTES) return MHFFN_ERR_STATIC_SCRATCH;
     void* ws = nullptr;
     if (static_scratch_of_current_device(&ws) != hipSuccess) return MHFFN_ERR_LAUNCH;
     hipError_t err;
     if (dtype == MHFFN_DTYPE_F32)
-        err = mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, ws, need, d,
-                                    (hipStream_t)stream, MHFFN_BWD_ALL);
+        err = mhffn::launch_bwd_f32(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, ws,
+                                    (size_t)MHFFN_STATIC_SCRATCH_BYTES, d, (hipStream_t)stream, MHFFN_BWD_ALL);
     else
         err = mhffn::launch_bwd_bf16(Q, K, U, V, R, dO, dQ, dK, dU, dV, dR, grad_w_dtype == MHFFN_DTYPE_F32, ws,
                                      (size_t)MHFFN_STATIC_SCRATCH_BYTES, d, (hipStream_t)stream, MHFFN_BWD_ALL);

@@ -74,6 +74,16 @@ def test_static_scratch_backward_with_fewer_token_slices_than_the_workspace_back
         assert torch.equal(a, b), name
 
 
+def test_static_scratch_backward_in_float32_with_fewer_parts_than_the_workspace_backward():
+    from flashmhf_amd import _capi
+    # 512 rows against 1,000 experts: the token slices take 0.1 MiB, the parts of dQ, dR that mhffn_bwd asks for more than the array
+    ref, got, ws_bytes = _run_both((1, 1, 512, 8, 1000, 1, 1), 47, torch.float32, torch.float32)
+    assert ws_bytes > _capi.STATIC_SCRATCH_BYTES, "this case is meant to need fewer parts than mhffn_bwd uses"
+    for name, a, b in zip(("dQ", "dK", "dU", "dV", "dR"), got, ref):
+        assert not torch.isnan(a).any() and (a - b).abs().max().item() <= 1e-5 * b.abs().max().item(), name
+    assert all(torch.equal(a, b) for a, b in zip(got[1:4], ref[1:4]))
+
+
 def test_static_scratch_backward_rejects_what_does_not_fit_before_any_launch():
     from flashmhf_amd import _capi
     L = _capi.lib()
