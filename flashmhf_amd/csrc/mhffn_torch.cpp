@@ -195,23 +195,25 @@ Tensor op(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, co
 // The single-expert operator: Q [B,H,S,d_h], K/U/V [Hkuv, rows, d_h], gate 1.
 Tensor ones_gate(const Tensor& Q) { return at::ones({Q.size(0), Q.size(1), Q.size(2), 1}, Q.options().dtype(at::kFloat)); }
 struct SingleNode : torch::autograd::Function<SingleNode> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V)
+    static Tensor forward(AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, bool one_part)
     {
         const Tensor R = ones_gate(Q);
         ctx->save_for_backward({Q, K, U, V, R});
-        return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), R, false);
+        ctx->saved_data["one_part"] = one_part;
+        return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), R, one_part);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
     {
         const auto s = ctx->get_saved_variables();
-        auto out = op_backward(s[0], s[1].unsqueeze(1), s[2].unsqueeze(1), s[3].unsqueeze(1), s[4], g[0], s[1].scalar_type(), false);
-        return {out[0], out[1].squeeze(1), out[2].squeeze(1), out[3].squeeze(1)};
+        auto out = op_backward(s[0], s[1].unsqueeze(1), s[2].unsqueeze(1), s[3].unsqueeze(1), s[4], g[0], s[1].scalar_type(),
+                               ctx->saved_data["one_part"].toBool());
+        return {out[0], out[1].squeeze(1), out[2].squeeze(1), out[3].squeeze(1), Tensor()};
     }
 };
-Tensor single(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V)
+Tensor single(const Tensor& Q, const Tensor& K, const Tensor& U, const Tensor& V, bool one_part)
 {
-    if (!records_grad({&Q, &K, &U, &V})) return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones_gate(Q), false);
-    return SingleNode::apply(Q, K, U, V);
+    if (!records_grad({&Q, &K, &U, &V})) return op_forward(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones_gate(Q), one_part);
+    return SingleNode::apply(Q, K, U, V, one_part);
 }
 
 // ---- head prologue -------------------------------------------------------------------------------------------------

@@ -12,23 +12,29 @@ from .flash_mlp_moe import mhffn_backward, mhffn_forward
 
 class FlashFFNMoEFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, Q, K, U, V, R):
-        O = _capi.traced(mhffn_forward(Q, K, U, V, R))
+    def forward(ctx, Q, K, U, V, R, one_part=False):
+        O = _capi.traced(mhffn_forward(Q, K, U, V, R, one_part))
         ctx.save_for_backward(Q, K, U, V, R)
+        ctx.one_part = one_part
         return O
 
     @staticmethod
     def backward(ctx, grad_output):
         Q, K, U, V, R = ctx.saved_tensors
-        dQ, dK, dU, dV, dR = mhffn_backward(Q, K, U, V, R, grad_output, grad_w_dtype=torch.float32)
-        return dQ.float(), dK, dU, dV, dR
+        dQ, dK, dU, dV, dR = mhffn_backward(Q, K, U, V, R, grad_output, grad_w_dtype=torch.float32, one_part=ctx.one_part)
+        return dQ.float(), dK, dU, dV, dR, None
 
 
 class FlashFFNMoE(torch.nn.Module):
-    def __init__(self):
+    """``one_part``: as in ``FlashMLPMoE``."""
+
+    one_part = False        # (of modules saved before there was a choice)
+
+    def __init__(self, one_part=False):
         super().__init__()
+        self.one_part = one_part
 
     def forward(self, Q, K, U, V, R):
         if not _capi.native_nodes():
-            return FlashFFNMoEFunction.apply(Q, K, U, V, R)
-        return _capi.native().op(Q, K, U, V, R, False)
+            return FlashFFNMoEFunction.apply(Q, K, U, V, R, self.one_part)
+        return _capi.native().op(Q, K, U, V, R, self.one_part)

@@ -14,8 +14,13 @@ from .flash_mlp_moe import FlashMLPFunction
 
 
 class FlashMLP(torch.nn.Module):
-    def __init__(self):
+    """``one_part``: as in ``FlashMLPMoE``."""
+
+    one_part = False        # (of modules saved before there was a choice)
+
+    def __init__(self, one_part=False):
         super().__init__()
+        self.one_part = one_part
 
     def forward(self, Q, K, U, V, apply_dot_scaling=False, head_scaling=1.0, up_scaling=1.0, activation_fn="silu"):
         if activation_fn != "silu":
@@ -28,5 +33,5 @@ class FlashMLP(torch.nn.Module):
             raise RuntimeError("expected K/U/V [Hkuv, intermediate, d_h]")
         if not _capi.native_nodes():
             ones = torch.ones(*Q.shape[:3], 1, dtype=torch.float32, device=Q.device)
-            return FlashMLPFunction.apply(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones)
-        return _capi.native().single(Q, K, U, V)
+            return FlashMLPFunction.apply(Q, K.unsqueeze(1), U.unsqueeze(1), V.unsqueeze(1), ones, self.one_part)
+        return _capi.native().single(Q, K, U, V, self.one_part)

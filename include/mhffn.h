@@ -111,7 +111,7 @@ int mhffn_bwd(const void* Q, const void* K, const void* U, const void* V, const 
 enum {
     MHFFN_FWD_MAIN = 1, MHFFN_FWD_ALL = 1,
     MHFFN_BWD_DQDR = 1, MHFFN_BWD_DKDUDV = 2, MHFFN_BWD_REDUCE = 4, MHFFN_BWD_ALL = 7,
-    /* May be added to any mask (bfloat16): O, dQ and dR are summed over the experts' rows in one fixed order, so that a token's
+    /* May be added to any mask: O, dQ and dR are summed over the experts' rows in one fixed order, so that a token's
      * values do not depend, to the last bit, on how many other tokens the call holds.  Without it a call with few tokens
      * adds the partial sums of several workgroups (see mhffn_fwd_workspace_bytes), which is faster. */
     MHFFN_ONE_PART = 256

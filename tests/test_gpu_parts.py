@@ -66,6 +66,27 @@ def test_one_part_does_not_depend_on_the_other_tokens(case):
         assert torch.equal(a, b[-1:, :, few])
 
 
+@pytest.mark.parametrize("entry", ["moe", "ffn", "mlp", "moe function", "ffn function"])
+def test_every_operator_offers_one_part(entry):
+    from flashmhf_amd import FlashFFNMoE, FlashMLP, FlashMLPMoE
+    from flashmhf_amd.flash_ffn_moe_torch import FlashFFNMoEFunction
+    from flashmhf_amd.flash_mlp_moe import FlashMLPFunction
+    _, (Q, K, U, V, R, dO) = _run((1, 8, 1500, 128, 1 if entry == "mlp" else 11, 352, 8, False))
+    op = {"moe": FlashMLPMoE(one_part=True), "ffn": FlashFFNMoE(one_part=True), "mlp": FlashMLP(one_part=True),
+          "moe function": lambda *a: FlashMLPFunction.apply(*a, True), "ffn function": lambda *a: FlashFFNMoEFunction.apply(*a, True)}[entry]
+    if entry == "mlp":
+        K, U, V = (w[:, 0].contiguous() for w in (K, U, V))
+
+    def run(rows):
+        leaves = [t[:, :, rows].contiguous().requires_grad_() for t in ([Q] if entry == "mlp" else [Q, R])]
+        o = op(leaves[0], K, U, V, *leaves[1:])
+        return [o, *torch.autograd.grad(o, leaves, dO[:, :, rows].contiguous())]
+
+    few = slice(37, 40)
+    for a, b in zip(run(few), run(slice(None))):
+        assert torch.equal(a, b[:, :, few])
+
+
 @pytest.mark.parametrize("case", [
     # B, H, S, dh, E, de, Hk, token_major: rows around the 128-row tile, weight rows around the 32-row block, every tile width
     (1, 2, 1, 8, 1, 1, 2, False), (1, 2, 127, 32, 2, 31, 1, True), (1, 1, 129, 72, 3, 33, 1, False),
