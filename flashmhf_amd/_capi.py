@@ -67,6 +67,13 @@ def lib():
         L.mhffn_bwd_static.argtypes = [vp] * 6 + [vp] * 5 + [ctypes.c_int, dp, ctypes.c_int, ctypes.c_int, vp]
         L.mhffn_gate_fwd.argtypes = [vp, vp, ctypes.c_float, vp, vp, vp, dp, vp]
         L.mhffn_gate_bwd.argtypes = [vp, vp, ctypes.c_float, vp, vp, ctypes.c_int, vp, vp, vp, vp, dp, vp]
+        L.mhffn_gate_fwd_typed.argtypes = [vp, vp, ctypes.c_int, ctypes.c_float, vp, ctypes.c_int, vp, vp, dp, vp]
+        L.mhffn_gate_bwd_workspace_bytes.restype = ctypes.c_size_t
+        L.mhffn_gate_bwd_workspace_bytes.argtypes = [dp]
+        L.mhffn_gate_bwd_into.argtypes = [vp, vp, ctypes.c_int, ctypes.c_float, vp, ctypes.c_int, vp, ctypes.c_int, vp, vp, vp, vp,
+                                          vp, ctypes.c_size_t, dp, vp]
+        L.mhffn_rope_fwd.argtypes = [vp] * 5 + [ctypes.c_int] * 4 + [vp]
+        L.mhffn_rope_bwd.argtypes = [vp] * 3 + [ctypes.POINTER(ctypes.c_long)] + [vp] * 3 + [ctypes.c_int] * 4 + [vp]
         _lib = L
     return _lib
 

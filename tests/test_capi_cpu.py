@@ -29,6 +29,23 @@ def test_every_declared_symbol_is_exported(L):
         assert getattr(L, name) is not None
 
 
+def test_every_binding_has_the_types_of_its_declaration(L):
+    """Unbound, ctypes passes pointers and returns sizes as 32-bit ints."""
+    header = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "mhffn.h")).read(), flags=re.S)
+    scalar = {"int": ctypes.c_int, "float": ctypes.c_float, "size_t": ctypes.c_size_t, "const char*": ctypes.c_char_p}
+    pointers = {"const mhffn_dims*": [ctypes.POINTER(_capi.Dims)], "const long*": [ctypes.POINTER(ctypes.c_long)]}
+    found = re.findall(r"^(int|size_t|const char\*) (mhffn_[a-z_]+)\((.*?)\);", header, flags=re.S | re.M)
+    assert {name for _, name, _ in found} == set(_capi.EXPORTS)
+    for result, name, args in found:
+        f = getattr(L, name)
+        assert f.restype is scalar[result], name
+        want = [re.sub(r"\s+", " ", a).strip() for a in args.split(",")]
+        assert f.argtypes is not None and len(f.argtypes) == len(want), name
+        for got, a in zip(f.argtypes, want):
+            kind = a[:a.rindex("*") + 1] if "*" in a else a.rsplit(" ", 1)[0]
+            assert got in ([scalar[kind]] if "*" not in a else pointers.get(kind, [ctypes.c_void_p])), (name, a, got)
+
+
 def test_strerror_and_is_supported(L):
     assert _capi.strerror(0) == "ok"
     for code in range(-8, 0):
