@@ -68,10 +68,7 @@ def build_lib(verbose=False, jobs=4):
         for name in sorted(usage):
             f.write(name + "  " + "  ".join(f"{k}={v}" for k, v in usage[name].items()) + "\n")
     check_no_scratch(usage)
-    for frag, count in VARIANT_KERNELS:
-        found = [n for n in usage if frag in n]
-        if len(found) != count or any(int(usage[n]["ScratchSize"]) for n in found):
-            raise RuntimeError(f"expected {count} instantiations of {frag} without scratch memory, found {found}")
+    check_variants(usage)
     return LIB
 
 
@@ -114,8 +111,9 @@ EXPECTED_KERNELS = (
     ("mhffn_fwd_kernel", 3), ("mhffn_bwd_dqdr_kernel", 3), ("mhffn_bwd_dkdudv_kernel", 6),
     ("mhffn_gate_fwd_kernel", 12), ("mhffn_gate_bwd_kernel", 12),
 )
-# Variants of those kernels for smaller problems, under the same rule.
-VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3))
+# Variants of those kernels for smaller problems and for float32, under the same rule.
+VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
+                   ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 4))
 # The one instantiation known to spill: head prologue backward for d_h = 128 with more than 32 experts and RMSNorm
 # (<128, 2, true>).  It is correct but slow; the block (MHFFNLayer.heads_and_gate) does not route that case to it.
 ALLOWED_SCRATCH = ("mhffn_gate_bwd_kernelILi128ELi2ELb1E",)
@@ -135,6 +133,14 @@ def check_no_scratch(usage):
             if any(a in name for a in ALLOWED_SCRATCH):
                 continue
             raise RuntimeError(f"{name} uses {u['ScratchSize']} bytes of scratch per lane: a spill in a hand-scheduled kernel")
+
+
+def check_variants(usage):
+    """check_no_scratch's rule for VARIANT_KERNELS, none of which may spill."""
+    for frag, count in VARIANT_KERNELS:
+        found = [n for n in usage if frag in n and "ScratchSize" in usage[n]]
+        if len(found) != count or any(int(usage[n]["ScratchSize"]) for n in found):
+            raise RuntimeError(f"expected {count} instantiations of {frag} without scratch memory, found {found}")
 
 
 if __name__ == "__main__":

@@ -326,69 +326,75 @@ __global__ __launch_bounds__(256, 1) void dkdudv_f32_kernel(F32Args p)
     constexpr int STAGE_B = 2 * T::BYTES;      // Q and dO tile
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     float* sR = reinterpret_cast<float*>(lds + 4 * STAGE_B);      // [stage][wave][32] gate values
-    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
-    const int hk = blockIdx.y, z = blockIdx.z, DH = p.DH, E = p.parts.E, nblk = E * p.parts.nbe;
+    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
     const int blk = blockIdx.x * 2 + bw;
     const Block b(p, hk, blk < nblk ? blk : nblk - 1);
-    const bool active = blk < nblk, live = l32 < b.rows;
-    const long wrow = b.wrow + (live ? l32 : b.rows - 1);
 
-    const int ntile = (p.rows.n + 31) / 32;
-    const int t0 = (int)((long)ntile * z / p.nslice), t1 = (int)((long)ntile * (z + 1) / p.nslice);
-    const int steps = (t1 - t0 + 1) / 2;
-    auto fill = [&](int s) {
-        const int t = t0 + 2 * s + half;
-        const int row0 = 32 * (t < ntile ? t : ntile - 1);
-        unsigned char* stage = lds + (half * 2 + (s & 1)) * STAGE_B;
-        int lane = threadIdx.x & 63;
-        asm volatile("" : "+v"(lane));      // (the fills' addresses are not worth a register each)
-        auto row = [&](const float* W) {
-            return [&, W](int r) { return W + p.rows.tok_head_major(hk, row0 + r < p.rows.n ? row0 + r : p.rows.n - 1) * DH; };
-        };
-#pragma unroll
-        for (int k = 0; k < FI; ++k) {
-            T::fill(stage, bw * FI + k, lane, DH, row(p.Q));
-            T::fill(stage + T::BYTES, bw * FI + k, lane, DH, row(p.dO));
-        }
-        // gate values of this wave's expert; 0 for the rows that a tile lacks, which removes them from every product
-        if (g == 0) {
-            const bool ok = t < t1 && row0 + l32 < p.rows.n;
-            sR[((s & 1) * 4 + wave) * 32 + l32] = ok ? p.R[p.rows.head_major(hk, ok ? row0 + l32 : 0) * E + b.e] : 0.0f;
-        }
-    };
-    fill(0);
-    f32x4 kB[4 * CT], uB[4 * CT], vB[4 * CT];
-    load_row<CT>(kB, p.K + wrow * DH, g, DH);
-    load_row<CT>(uB, p.U + wrow * DH, g, DH);
-    load_row<CT>(vB, p.V + wrow * DH, g, DH);
     f32x16 dk[CT], du[CT], dv[CT];
+    {
+        const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5, DH = p.DH;
+        const int ntile = (p.rows.n + 31) / 32;
+        const int t0 = (int)((long)ntile * z / p.nslice), t1 = (int)((long)ntile * (z + 1) / p.nslice);
+        const int steps = (t1 - t0 + 1) / 2;
+        auto fill = [&](int s) {
+            const int t = t0 + 2 * s + half;
+            const int row0 = 32 * (t < ntile ? t : ntile - 1);
+            unsigned char* stage = lds + (half * 2 + (s & 1)) * STAGE_B;
+            int lane = threadIdx.x & 63;
+            asm volatile("" : "+v"(lane));      // (the fills' addresses are not worth a register each)
+            auto row = [&](const float* W) {
+                return [&, W](int r) { return W + p.rows.tok_head_major(hk, row0 + r < p.rows.n ? row0 + r : p.rows.n - 1) * DH; };
+            };
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) { dk[ct] = zero16(); du[ct] = zero16(); dv[ct] = zero16(); }
+            for (int k = 0; k < FI; ++k) {
+                T::fill(stage, bw * FI + k, lane, DH, row(p.Q));
+                T::fill(stage + T::BYTES, bw * FI + k, lane, DH, row(p.dO));
+            }
+            // gate values of this wave's expert; 0 for the rows that a tile lacks, which removes them from every product
+            if (g == 0) {
+                const bool ok = t < t1 && row0 + l32 < p.rows.n;
+                sR[((s & 1) * 4 + wave) * 32 + l32] = ok ? p.R[p.rows.head_major(hk, ok ? row0 + l32 : 0) * E + b.e] : 0.0f;
+            }
+        };
+        fill(0);
+        f32x4 kB[4 * CT], uB[4 * CT], vB[4 * CT];
+        const long wrow = b.wrow + (l32 < b.rows ? l32 : b.rows - 1);
+        load_row<CT>(kB, p.K + wrow * DH, g, DH);
+        load_row<CT>(uB, p.U + wrow * DH, g, DH);
+        load_row<CT>(vB, p.V + wrow * DH, g, DH);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) { dk[ct] = zero16(); du[ct] = zero16(); dv[ct] = zero16(); }
 
-    for (int s = 0; s < steps; ++s) {
-        const unsigned char *sQ = lds + (half * 2 + (s & 1)) * STAGE_B, *sG = sQ + T::BYTES;
-        wait_vmcnt<0>();
-        __syncthreads();
-        if (s + 1 < steps) fill(s + 1);
-        f32x16 mna[3];
-        const typename T::Lane l(l32, g);
-        first_products<CT, 3>(mna, {sQ, sQ, sG}, {kB, uB, vB}, l);
-        f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
-        const float* rw = sR + ((s & 1) * 4 + wave) * 32;
+        for (int s = 0; s < steps; ++s) {
+            const unsigned char *sQ = lds + (half * 2 + (s & 1)) * STAGE_B, *sG = sQ + T::BYTES;
+            wait_vmcnt<0>();
+            __syncthreads();
+            if (s + 1 < steps) fill(s + 1);
+            f32x16 mna[3];
+            const typename T::Lane l(l32, g);
+            first_products<CT, 3>(mna, {sQ, sQ, sG}, {kB, uB, vB}, l);
+            f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
+            const float* rw = sR + ((s & 1) * 4 + wave) * 32;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const float r = rw[reg_row(i, g)], sg = sigmoid_exact(m[i]), sl = m[i] * sg, a = da[i], nn = n[i];
-            m[i] = r * a * nn * (sg + sl * (1.0f - sg));      // dM
-            n[i] = r * a * sl;                                // dN
-            da[i] = r * sl * nn;                              // P
+            for (int i = 0; i < 16; ++i) {
+                const float r = rw[reg_row(i, g)], sg = sigmoid_exact(m[i]), sl = m[i] * sg, a = da[i], nn = n[i];
+                m[i] = r * a * nn * (sg + sl * (1.0f - sg));      // dM
+                n[i] = r * a * sl;                                // dN
+                da[i] = r * sl * nn;                              // P
+            }
+            second_product<CT>(dk, sQ, m, l);
+            second_product<CT>(du, sQ, n, l);
+            second_product<CT>(dv, sG, da, l);
         }
-        second_product<CT>(dk, sQ, m, l);
-        second_product<CT>(du, sQ, n, l);
-        second_product<CT>(dv, sG, da, l);
     }
     // The odd tiles' sums to the wave with the even ones, one gradient at a time (64 lanes x 16 CT floats, lane-private).
+    // (This lane's row and the bounds of its columns are worked out again, out of the compiler's sight: kept over the loop they
+    // are the few registers too many that made it spill for d_h > 96.)
     __syncthreads();
+    int lane = threadIdx.x & 63, DH = p.DH;
+    asm volatile("" : "+v"(lane), "+s"(DH));
+    const int l32 = lane & 31, g = lane >> 5;
     float* xch = reinterpret_cast<float*>(lds) + bw * (3 * CT * 16 * 64) + lane;
     if (half == 1) {
 #pragma unroll
@@ -401,7 +407,7 @@ __global__ __launch_bounds__(256, 1) void dkdudv_f32_kernel(F32Args p)
             }
     }
     __syncthreads();
-    if (half == 1 || !active || !live) return;
+    if (half == 1 || blk >= nblk || l32 >= b.rows) return;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -410,7 +416,7 @@ __global__ __launch_bounds__(256, 1) void dkdudv_f32_kernel(F32Args p)
             du[ct][i] += xch[((CT + ct) * 16 + i) * 64];
             dv[ct][i] += xch[((2 * CT + ct) * 16 + i) * 64];
         }
-    const long wsz = (long)p.rows.Hkuv * E * p.de * DH;
+    const long wrow = b.wrow + l32, wsz = (long)p.rows.Hkuv * E * p.de * DH;
     auto store_bf16 = [&](const f32x16(&acc)[CT], void* out) {
         bf16_t* dst = static_cast<bf16_t*>(out) + wrow * DH;
 #pragma unroll

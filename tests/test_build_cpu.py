@@ -68,3 +68,27 @@ def test_the_committed_resource_listing_is_clean():
         name, *fields = line.split("  ")
         usage[name] = dict(f.strip().split("=", 1) for f in fields if "=" in f)
     build.check_no_scratch(usage)
+
+
+def _listing():
+    path = os.path.join(build.LIBDIR, "resource_usage.txt")
+    if not os.path.exists(path):
+        pytest.skip("library not built")
+    usage = {}
+    for line in open(path):
+        name, *fields = line.split("  ")
+        usage[name] = dict(f.strip().split("=", 1) for f in fields if "=" in f)
+    return usage
+
+
+@pytest.mark.parametrize("frag,count", build.VARIANT_KERNELS)
+def test_no_variant_and_no_float32_kernel_spills(frag, count):
+    usage = _listing()
+    build.check_variants(usage)
+    found = [n for n in usage if frag in n]
+    assert len(found) == count
+    for n in found:
+        with pytest.raises(RuntimeError, match="scratch"):
+            build.check_variants({**usage, n: {**usage[n], "ScratchSize": "16"}})
+        with pytest.raises(RuntimeError, match="scratch"):
+            build.check_variants({k: v for k, v in usage.items() if k != n})
