@@ -23,7 +23,7 @@ OK = 0
 STATIC_SCRATCH_BYTES = 96 << 20
 
 EXPORTS = (
-    "mhffn_strerror", "mhffn_is_supported", "mhffn_check_dims", "mhffn_fwd_workspace_bytes",
+    "mhffn_strerror", "mhffn_is_supported", "mhffn_check_dims", "mhffn_launch_plan", "mhffn_fwd_workspace_bytes",
     "mhffn_bwd_workspace_bytes", "mhffn_bwd_workspace_min_bytes", "mhffn_fwd", "mhffn_bwd", "mhffn_fwd_phases", "mhffn_bwd_phases",
     "mhffn_fwd_layout", "mhffn_bwd_layout", "mhffn_bwd_static", "mhffn_gate_fwd", "mhffn_gate_bwd",
     "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into", "mhffn_rope_fwd", "mhffn_rope_bwd",
@@ -31,10 +31,15 @@ EXPORTS = (
 TOKENS_BHSD, TOKENS_BSHD = 0, 1     # layout of Q, O, dO, dQ
 FWD_MAIN, FWD_ALL = 1, 1
 BWD_DQDR, BWD_DKDUDV, BWD_REDUCE, BWD_ALL = 1, 2, 4, 7
+ONE_PART = 256
 
 
 class Dims(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int) for n in ("B", "H", "Hkuv", "S", "d_h", "E", "d_e")]
+
+
+class Plan(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("fwd_tile_rows", "fwd_parts", "dqdr_tile_rows", "dqdr_parts", "dkdudv_slices")]
 
 
 _lib = None
@@ -57,6 +62,7 @@ def lib():
         for f in (L.mhffn_fwd_workspace_bytes, L.mhffn_bwd_workspace_bytes, L.mhffn_bwd_workspace_min_bytes):
             f.restype = ctypes.c_size_t
             f.argtypes = [dp, ctypes.c_int]
+        L.mhffn_launch_plan.argtypes = [dp, ctypes.c_int, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int, ctypes.POINTER(Plan)]
         L.mhffn_fwd.argtypes = [vp] * 6 + [vp, ctypes.c_size_t, dp, ctypes.c_int, vp]
         L.mhffn_bwd.argtypes = [vp] * 6 + [vp] * 5 + [ctypes.c_int, vp, ctypes.c_size_t, dp, ctypes.c_int, vp]
         L.mhffn_fwd_phases.argtypes = L.mhffn_fwd.argtypes + [ctypes.c_int]
@@ -104,6 +110,15 @@ def native_nodes():
 def traced(t):
     """`t`, an output of a native call inside a Function's forward, as a tensor that a running trace knows."""
     return t.clone() if torch._C._is_tracing() else t
+
+
+def launch_plan(dims, dtype, one_part=False):
+    """What the operators run for these extents (they hand over the workspaces that are asked for)."""
+    p = Plan()
+    raise_for_code(lib().mhffn_launch_plan(dims, dtype, lib().mhffn_fwd_workspace_bytes(dims, dtype),
+                                           lib().mhffn_bwd_workspace_bytes(dims, dtype), ONE_PART if one_part else 0, p),
+                   "mhffn_launch_plan")
+    return p
 
 
 def strerror(code):

@@ -1042,7 +1042,7 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // read back once (priced at the time of a token tile per 2.5 MB: about 4 TB/s against 1.25 us per tile).
 constexpr long DW_FIXED_TILES = 9;      // prologue + epilogue of a workgroup, in token tiles
 constexpr long DW_BYTES_PER_TILE_TIME = 2500000;
-static int pick_nslice(const Dims& d, size_t ws_bytes)
+int dw_slices_bf16(const Dims& d, size_t ws_bytes)
 {
     const int nblk = d.E * (d.d_e / JB);
     const long cols = (long)((nblk + 3) / 4) * d.Hkuv;
@@ -1065,22 +1065,22 @@ static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d
 // large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 512 rows: 204 us with 256 rows, 87 with
 // 32; 2,048 rows: 204 and 172 (two rounds); with parts, one row 15 and 12.7 us.
 constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33, 1}, {32, 2.7, 0.05, QUAD}};
-static Pick dq_pick(const Dims& d, size_t ws_bytes)
+Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
-    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), ws_bytes);
+    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
 }
 
 size_t bwd_min_workspace_bytes_bf16(const Dims& d)
 {
     const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
-    const int ns = pick_nslice(d, ~(size_t)0);
+    const int ns = dw_slices_bf16(d, ~(size_t)0);
     return ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
 }
 
 // The two kernels run one after the other, so the parts of dQ, dR and the token slices of dK, dU, dV share the workspace.
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
-    const int nq = dq_pick(d, ~(size_t)0).nsplit;
+    const int nq = dq_pick_bf16(d, ~(size_t)0, 0).nsplit;
     const size_t dw = bwd_min_workspace_bytes_bf16(d);
     const size_t dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
     return dw > dq ? dw : dq;
@@ -1096,7 +1096,7 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     const int nbe = d.d_e / JB, G = d.H / d.Hkuv;
 
     if (phases & PH_BWD_DQDR) {
-        const Pick pick = dq_pick(d, ws && !(phases & PH_ONE_PART) ? ws_bytes : 0);
+        const Pick pick = dq_pick_bf16(d, ws ? ws_bytes : 0, phases);
         DqArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R,
                  (bf16_t*)dQ, dR, part, RowMap(d),
                  Parts(d.E, nbe, pick.nsplit)};
@@ -1119,7 +1119,7 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
-    const int nslice = pick_nslice(d, ws_bytes);
+    const int nslice = dw_slices_bf16(d, ws_bytes);
     if (phases & PH_BWD_DKDUDV) {
         DwArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, part,
                  {dK, dU, dV}, grad_w_f32, d.B, d.H, G, d.S, d.E, nbe, nslice, d.tokmaj};

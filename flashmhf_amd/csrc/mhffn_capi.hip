@@ -106,6 +106,23 @@ size_t mhffn_bwd_workspace_min_bytes(const mhffn_dims* dims, int dtype)
     return dtype == MHFFN_DTYPE_F32 ? mhffn::bwd_min_workspace_bytes_f32(to_dims(dims)) : mhffn::bwd_min_workspace_bytes_bf16(to_dims(dims));
 }
 
+int mhffn_launch_plan(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases,
+                      mhffn_plan* plan)
+{
+    const int rc = check_dims_impl(dims, dtype);
+    if (rc != MHFFN_OK) return rc;
+    if (!plan) return MHFFN_ERR_NULL_POINTER;
+    if (phases & ~(MHFFN_BWD_ALL | MHFFN_ONE_PART)) return MHFFN_ERR_SHAPE;
+    if (bwd_workspace_bytes < mhffn_bwd_workspace_min_bytes(dims, dtype)) return MHFFN_ERR_WORKSPACE;
+    const mhffn::Dims d = to_dims(dims);
+    const bool f32 = dtype == MHFFN_DTYPE_F32;
+    const mhffn::Pick f = f32 ? mhffn::fwd_pick_f32(d, fwd_workspace_bytes, phases) : mhffn::fwd_pick_bf16(d, fwd_workspace_bytes, phases);
+    const mhffn::Pick q = f32 ? mhffn::dq_pick_f32(d, bwd_workspace_bytes, phases) : mhffn::dq_pick_bf16(d, bwd_workspace_bytes, phases);
+    *plan = mhffn_plan{f.tile_rows, f.nsplit, q.tile_rows, q.nsplit,
+                       f32 ? mhffn::dw_slices_f32(d) : mhffn::dw_slices_bf16(d, bwd_workspace_bytes)};
+    return MHFFN_OK;
+}
+
 int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
                      void* workspace, size_t workspace_bytes, const mhffn_dims* dims, int dtype, int token_layout,
                      void* stream, int phases)

@@ -631,6 +631,14 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
     return best;
 }
 
+// What a launch with this workspace (0: none) and these phases runs.
+Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases);
+Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases);
+int dw_slices_bf16(const Dims& d, size_t ws_bytes);
+Pick fwd_pick_f32(const Dims& d, size_t ws_bytes, int phases);
+Pick dq_pick_f32(const Dims& d, size_t ws_bytes, int phases);
+int dw_slices_f32(const Dims& d);
+
 size_t fwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely (0: one part);
                                                       // with less it runs fewer parts
 size_t bwd_workspace_bytes_bf16(const Dims& d);       // what the launch uses when it may choose freely: the token slices of

@@ -486,20 +486,9 @@ constexpr Variant F32_VARIANTS[] = {{128, 5.0, 0.0, 1}};
 int nbe_of(const Dims& d) { return (d.d_e + JB - 1) / JB; }
 size_t o_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
-int parts_of(const Dims& d, size_t part_bytes, size_t ws_bytes)
+Pick pick_f32(const Dims& d, size_t part_bytes, size_t ws_bytes, int phases)
 {
-    return pick_parts(F32_VARIANTS, d, d.E * nbe_of(d), true, part_bytes, ws_bytes).nsplit;
-}
-
-// Token slices of dK/dU/dV: only where the workgroups (two blocks of weight rows each) leave compute units idle.
-int f32_nslice(const Dims& d)
-{
-    const long groups = ((long)d.E * nbe_of(d) + 1) / 2 * d.Hkuv;
-    const long ntile = ((long)(d.H / d.Hkuv) * d.B * d.S + 31) / 32;
-    long ns = CUS / groups;
-    if (ns > ntile / 2) ns = ntile / 2;
-    if (ns > 64) ns = 64;
-    return ns < 1 ? 1 : (int)ns;
+    return pick_parts(F32_VARIANTS, d, d.E * nbe_of(d), true, part_bytes, phases & PH_ONE_PART ? 0 : ws_bytes);
 }
 
 F32Args f32_args(const void* Q, const void* K, const void* U, const void* V, const float* R, const Dims& d, int nsplit)
@@ -562,9 +551,23 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
 
 }  // namespace
 
+Pick fwd_pick_f32(const Dims& d, size_t ws_bytes, int phases) { return pick_f32(d, o_part_bytes(d), ws_bytes, phases); }
+Pick dq_pick_f32(const Dims& d, size_t ws_bytes, int phases) { return pick_f32(d, dq_part_bytes(d), ws_bytes, phases); }
+
+// Token slices of dK/dU/dV: only where the workgroups (two blocks of weight rows each) leave compute units idle.
+int dw_slices_f32(const Dims& d)
+{
+    const long groups = ((long)d.E * nbe_of(d) + 1) / 2 * d.Hkuv;
+    const long ntile = ((long)(d.H / d.Hkuv) * d.B * d.S + 31) / 32;
+    long ns = CUS / groups;
+    if (ns > ntile / 2) ns = ntile / 2;
+    if (ns > 64) ns = 64;
+    return ns < 1 ? 1 : (int)ns;
+}
+
 size_t fwd_workspace_bytes_f32(const Dims& d)
 {
-    const int ns = parts_of(d, o_part_bytes(d), ~(size_t)0);
+    const int ns = fwd_pick_f32(d, ~(size_t)0, 0).nsplit;
     return ns > 1 ? ns * o_part_bytes(d) : 0;
 }
 
@@ -572,14 +575,14 @@ size_t fwd_workspace_bytes_f32(const Dims& d)
 // reserve)
 size_t bwd_min_workspace_bytes_f32(const Dims& d)
 {
-    return (size_t)f32_nslice(d) * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float);
+    return (size_t)dw_slices_f32(d) * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float);
 }
 
 // ... and room for the parts of dQ, dR
 size_t bwd_workspace_bytes_f32(const Dims& d)
 {
     const size_t dw = bwd_min_workspace_bytes_f32(d);
-    const int nq = parts_of(d, dq_part_bytes(d), ~(size_t)0);
+    const int nq = dq_pick_f32(d, ~(size_t)0, 0).nsplit;
     const size_t dq = nq > 1 ? nq * dq_part_bytes(d) : 0;
     return dw > dq ? dw : dq;
 }
@@ -587,7 +590,7 @@ size_t bwd_workspace_bytes_f32(const Dims& d)
 hipError_t launch_fwd_f32(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O, void* ws,
                           size_t ws_bytes, const Dims& d, hipStream_t st, int phases)
 {
-    F32Args a = f32_args(Q, K, U, V, R, d, parts_of(d, o_part_bytes(d), ws && !(phases & PH_ONE_PART) ? ws_bytes : 0));
+    F32Args a = f32_args(Q, K, U, V, R, d, fwd_pick_f32(d, ws ? ws_bytes : 0, phases).nsplit);
     a.O = (float*)O;
     a.part = (float*)ws;
     switch ((d.d_h + 31) / 32) {
@@ -602,10 +605,10 @@ hipError_t launch_bwd_f32(const void* Q, const void* K, const void* U, const voi
                           void* dQ, void* dK, void* dU, void* dV, float* dR, int grad_w_f32, void* ws, size_t ws_bytes,
                           const Dims& d, hipStream_t st, int phases)
 {
-    F32Args a = f32_args(Q, K, U, V, R, d, parts_of(d, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes));
+    F32Args a = f32_args(Q, K, U, V, R, d, dq_pick_f32(d, ws_bytes, phases).nsplit);
     a.dO = (const float*)dO; a.dQ = (float*)dQ; a.dR = dR; a.part = (float*)ws;
     a.out[0] = dK; a.out[1] = dU; a.out[2] = dV; a.out_f32 = grad_w_f32;
-    a.nslice = f32_nslice(d);
+    a.nslice = dw_slices_f32(d);
     hipError_t err;
     switch ((d.d_h + 31) / 32) {
         case 1: err = launch_bwd_f32_t<1>(a, d, st, phases); break;

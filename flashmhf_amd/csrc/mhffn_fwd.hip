@@ -523,9 +523,9 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // the same sums, bit for bit, in all three.
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
-static Pick fwd_pick(const Dims& d, size_t ws_bytes)
+Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
-    return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), ws_bytes);
+    return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
 }
 
 template <int DH>
@@ -553,7 +553,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, h
 
 size_t fwd_workspace_bytes_bf16(const Dims& d)
 {
-    const int ns = fwd_pick(d, ~(size_t)0).nsplit;
+    const int ns = fwd_pick_bf16(d, ~(size_t)0, 0).nsplit;
     return ns > 1 ? ns * fwd_part_bytes(d) : 0;
 }
 
@@ -561,7 +561,7 @@ hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const vo
                            void* ws, size_t ws_bytes, const Dims& d, hipStream_t st, int phases)
 {
     if (!(phases & PH_FWD_MAIN)) return hipSuccess;
-    const Pick pick = fwd_pick(d, ws && !(phases & PH_ONE_PART) ? ws_bytes : 0);
+    const Pick pick = fwd_pick_bf16(d, ws ? ws_bytes : 0, phases);
     FwdArgs a{(const bf16_t*)Q, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V,           R,
               (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, pick.nsplit)};
     switch (d.d_h) {

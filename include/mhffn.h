@@ -126,6 +126,17 @@ int mhffn_bwd_phases(const void* Q, const void* K, const void* U, const void* V,
                      void* workspace, size_t workspace_bytes,
                      const mhffn_dims* dims, int dtype, void* stream, int phases);
 
+/* What mhffn_fwd and mhffn_bwd would run for these extents with workspaces of these sizes: the tile heights name the kernels
+ * (forward 256, 128 or 32 rows, dQ/dR 256 or 32; float32: 128).  For tests that are meant for one kernel and for benchmarks;
+ * no GPU is needed.  Only MHFFN_ONE_PART of `phases` matters.  Errors as the launches'. */
+typedef struct mhffn_plan {
+    int fwd_tile_rows, fwd_parts;
+    int dqdr_tile_rows, dqdr_parts;
+    int dkdudv_slices;
+} mhffn_plan;
+int mhffn_launch_plan(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases,
+                      mhffn_plan* plan);
+
 /* Token-major variants: Q, O, dO, dQ are [B, S, H, d_h] (MHFFN_TOKENS_BSHD) -- the layout the caller's projections
  * produce and consume -- instead of [B, H, S, d_h] (MHFFN_TOKENS_BHSD, what the calls above use).  K, U, V, R, dR and all
  * other conventions are unchanged; results are identical to the [B, H, S, d_h] calls on the transposed tensors.

@@ -33,7 +33,8 @@ def test_every_binding_has_the_types_of_its_declaration(L):
     """Unbound, ctypes passes pointers and returns sizes as 32-bit ints."""
     header = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "mhffn.h")).read(), flags=re.S)
     scalar = {"int": ctypes.c_int, "float": ctypes.c_float, "size_t": ctypes.c_size_t, "const char*": ctypes.c_char_p}
-    pointers = {"const mhffn_dims*": [ctypes.POINTER(_capi.Dims)], "const long*": [ctypes.POINTER(ctypes.c_long)]}
+    pointers = {"const mhffn_dims*": [ctypes.POINTER(_capi.Dims)], "mhffn_plan*": [ctypes.POINTER(_capi.Plan)],
+                "const long*": [ctypes.POINTER(ctypes.c_long)]}
     found = re.findall(r"^(int|size_t|const char\*) (mhffn_[a-z_]+)\((.*?)\);", header, flags=re.S | re.M)
     assert {name for _, name, _ in found} == set(_capi.EXPORTS)
     for result, name, args in found:

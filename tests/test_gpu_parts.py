@@ -18,8 +18,8 @@ CASES = [
     (5, 4, 1, 96, 2, 256, 2, True),       # decoded tokens of five sequences share a tile with the heads of their group
     (1, 2, 255, 128, 3, 224, 2, False),
     (3, 4, 43, 64, 7, 96, 1, False),      # 516 rows of one K/U/V head: tiles across batches and heads
-    (1, 8, 1300, 64, 3, 320, 8, True),    # enough rows that the tile height is open
-    (1, 1, 129, 128, 2, 64, 1, False),    # 128-row tiles: a row beyond the first
+    (1, 8, 1300, 64, 3, 320, 8, True),    # 128-row tiles in two parts
+    (1, 1, 129, 128, 2, 64, 1, False),    # a row beyond four 32-row tiles
     (2, 2, 257, 96, 64, 32, 2, False),    # as many experts as one LDS window of gate values holds
 ]
 

@@ -1,0 +1,97 @@
+"""Which kernel a call runs (mhffn_launch_plan), and one case per kernel: the forward's tiles of 256, 128 and 32 rows and those of
+dQ/dR of 256 and 32, each in one part and in several, dK/dU/dV in one token slice and in several, for every head width.  The
+plan is asserted without a GPU, so that a case whose kernel is no longer picked for it fails instead of testing another one."""
+import ctypes
+
+import pytest
+import torch
+
+from flashmhf_amd import _capi
+from tests.helpers import assert_bf16_parity, make_inputs
+
+DEV = "cuda:0"
+
+# (B, H, S, E, de, Hk): rows of the forward's tile, several parts, rows of dQ/dR's tile, several parts, several token slices
+KERNELS = {
+    dh: [((1, 1, 129, 1, 32, 1), (128, False, 256, False, False)),
+         ((1, 1, 129, 3, 64, 1), (128, True, 256, True, False)),
+         ((1, 1, 129, 3, 32, 1), (32, False, 32, False, False)),
+         ((1, 1, 300, 9, 256, 1), (32, True, 32, True, False)),
+         ((2, 1, 255, 7, 96, 1), (32, True, 32, True, True)),
+         ((2, 4, 4097, 1, 32, 2), (256, False, 256, False, True)),
+         ((1, 64, 129, 9, 96 if dh == 64 else 256, 64), (256, True, 256, True, False))]
+    for dh in (64, 96, 128)
+}
+CASES = [(dh, dims, want) for dh, cases in KERNELS.items() for dims, want in cases]
+
+
+def _dims(dh, dims):
+    B, H, S, E, de, Hk = dims
+    return _capi.Dims(B, H, Hk, S, dh, E, de)
+
+
+def _plan(d, dtype=_capi.DTYPE_BF16, one_part=False):
+    p = _capi.launch_plan(d, dtype, one_part)
+    return p.fwd_tile_rows, p.fwd_parts > 1, p.dqdr_tile_rows, p.dqdr_parts > 1, p.dkdudv_slices > 1
+
+
+@pytest.mark.parametrize("dh,dims,want", CASES)
+def test_the_case_runs_the_kernels_it_is_for(dh, dims, want):
+    assert _plan(_dims(dh, dims)) == want
+
+
+def test_the_cases_cover_every_kernel():
+    for cases in KERNELS.values():
+        plans = [want for _, want in cases]
+        assert {p[:2] for p in plans} == {(r, s) for r in (256, 128, 32) for s in (False, True)}
+        assert {p[2:4] for p in plans} == {(r, s) for r in (256, 32) for s in (False, True)}
+        assert {p[4] for p in plans} == {False, True}
+
+
+def test_one_part_cases_compare_two_kernels():
+    """The cases of test_gpu_parts.test_one_part_does_not_depend_on_the_other_tokens: tile heights of the large call and of the
+    small one."""
+    from tests.test_gpu_parts import test_one_part_does_not_depend_on_the_other_tokens as t
+    cases = [m for m in t.pytestmark if m.name == "parametrize"][0].args[1]
+    want = [(32, 32), (256, 256), (256, 256), (256, 256), (128, 32)]
+    for (B, H, S, dh, E, de, Hk, _), (fwd, dq) in zip(cases, want, strict=True):
+        assert _plan(_capi.Dims(B, H, Hk, S, dh, E, de), one_part=True)[:4] == (fwd, False, dq, False)
+        assert _plan(_capi.Dims(1, H, Hk, 3, dh, E, de), one_part=True)[:4] == (32, False, 32, False)
+
+
+def test_less_workspace_and_one_part_mean_fewer_parts():
+    L, p = _capi.lib(), _capi.Plan()
+    d = _capi.Dims(1, 8, 8, 512, 128, 11, 352)
+    fwd, bwd = (f(d, 0) for f in (L.mhffn_fwd_workspace_bytes, L.mhffn_bwd_workspace_bytes))
+    seen = []
+    for f in (0, fwd // 2, fwd, 2 * fwd):
+        assert L.mhffn_launch_plan(d, 0, f, bwd * f // fwd, 0, p) == 0
+        seen.append((p.fwd_parts, p.dqdr_parts))
+        assert p.fwd_parts * 4 * 512 * 8 * 128 <= f or p.fwd_parts == 1
+        assert L.mhffn_launch_plan(d, 0, f, bwd * f // fwd, _capi.ONE_PART, p) == 0 and p.fwd_parts == p.dqdr_parts == 1
+    assert seen[0] == (1, 1) and seen[2] == seen[3] and min(seen[2]) > 1 and seen == sorted(seen)
+    sliced = _capi.Dims(2, 8, 2, 300, 96, 8, 256)
+    assert L.mhffn_launch_plan(sliced, 0, 0, 0, 0, p) == _capi.ERR_WORKSPACE
+    assert L.mhffn_launch_plan(d, 0, 0, 0, 512, p) == _capi.ERR_SHAPE
+    assert L.mhffn_launch_plan(d, 7, 0, 0, 0, p) == _capi.ERR_DTYPE
+    assert L.mhffn_launch_plan(d, 0, 0, 0, 0, ctypes.POINTER(_capi.Plan)()) == _capi.ERR_NULL_POINTER
+    many = _plan(_capi.Dims(1, 8, 8, 33, 128, 65, 32))      # more experts than one LDS window holds: one part, no 32-row tiles
+    assert many[:4] == (128, False, 256, False)
+    f32 = _capi.launch_plan(_capi.Dims(2, 8, 8, 128, 96, 8, 256), _capi.DTYPE_F32)
+    assert f32.fwd_tile_rows == f32.dqdr_tile_rows == 128 and f32.fwd_parts > 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dh,dims,want", CASES)
+def test_each_kernel_matches_the_oracle(dh, dims, want):
+    from flashmhf_amd import mhffn_backward, mhffn_forward
+    from oracle import mhffn_oracle as orc
+    print("case", dh, dims, flush=True)
+    B, H, S, E, de, Hk = dims
+    ins = make_inputs(B, H, S, dh, E, de, Hk, seed=5, dtype=torch.bfloat16)
+    dev = [t.to(DEV) for t in ins]
+    got = (mhffn_forward(*dev[:5]), *mhffn_backward(*dev, grad_w_dtype=torch.float32))
+    torch.cuda.synchronize()
+    ref = (orc.mhffn_forward(*ins[:5], compute_dtype=torch.float64), *orc.mhffn_backward(*ins, compute_dtype=torch.float64))
+    for name, a, r in zip(("O", "dQ", "dK", "dU", "dV", "dR"), got, ref):
+        assert_bf16_parity(name, a.float().cpu(), r, (dh, dims))
