@@ -1062,8 +1062,8 @@ int dw_slices_bf16(const Dims& d, size_t ws_bytes)
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
 // Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.7 us (four steps of the
-// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 512 rows: 204 us with 256 rows, 87 with
-// 32; 2,048 rows: 204 and 172 (two rounds); with parts, one row 15 and 12.7 us.
+// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 400 rows: 199 us with 256 rows, 85 with
+// 32; 2,048 rows: 202 and 173 (two rounds); one row in 32 parts of 32-row tiles 10.3 us.
 constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33, 1}, {32, 2.7, 0.05, QUAD}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {

@@ -517,10 +517,10 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 
 // Tiles of 256 rows (64 per wave) where they fill the chip; of 128 (32 per wave) below that: a step then takes 0.6 us
 // instead of 1.0, with 20 % less throughput once every compute unit has one (16,384 tokens of the 370M layer: 342 us with 256
-// rows, 407 with 128; 1,500 tokens in one part: 131 and 85; 733 tokens: 33 and 32 us at each one's best number of parts,
-// of the 128M layer 25.5 and 21.4).  Of 32, four blocks a trip of 1.43 us, below that: one token of the 370M layer 12.7 -> 10.3
-// us, 16 tokens of the 1.3B layer 21.2 -> 17.8 us (95 MB of weights, 5.3 TB/s), 512 rows in one part 84 -> 49 us.  Rows have
-// the same sums, bit for bit, in all three.
+// rows, 407 with 128; 1,500 tokens in one part: 130 and 84; 733 tokens: 33 and 32 us at each one's best number of parts,
+// of the 128M layer 25.6 and 22.0).  Of 32, four blocks a trip of 1.43 us, below that, where 128-row tiles take, at each one's best
+// number of parts: one token of the 370M layer 7.8 us against 10.0, 16 tokens of the 1.3B layer 20.3 against 22.5 (95 MB of
+// weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)

@@ -53,7 +53,7 @@ typedef struct mhffn_dims {
     int Hkuv;   /* K/U/V heads; H % Hkuv == 0 (grouped "GQ-FFN", flash_mlp_moe.py:194,222) */
     int S;      /* tokens per (batch, head) */
     int d_h;    /* head dim */
-    int E;      /* experts (sub-networks) per head (bf16: at most 64) */
+    int E;      /* experts (sub-networks) per head */
     int d_e;    /* rows of K/U/V per expert */
 } mhffn_dims;
 
@@ -61,7 +61,7 @@ typedef struct mhffn_dims {
 const char* mhffn_strerror(int code);
 
 /* 1 if kernels exist for (d_h, d_e, dtype), else 0.  bf16 (MFMA kernels): d_h in {64, 96, 128}, d_e % 32 == 0, any E.
- * float32 (correctness instantiation, plain FMA): d_h a multiple of 8 up to 128, any d_e, any E.
+ * float32 (correctness instantiation, fp32 matrix instructions): d_h a multiple of 8 up to 128, any d_e, any E.
  * Replaces the reference's shape gates (flash_mlp_moe.py:758, flash_ffn_moe.cu:956-958, 1037). */
 int mhffn_is_supported(int d_h, int d_e, int dtype);
 
