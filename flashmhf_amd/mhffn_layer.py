@@ -148,34 +148,46 @@ class MHFFNLayer(nn.Module):
         return Q, router_gate(logits).contiguous()
 
     def _stock_steps(self):
-        """Whether every step of the block is this module's own: heads_and_gate, and plain bias-free projections, RMSNorm and
-        operator, with no override in a subclass, on an instance or on a patched class and no hook that would have a say;
-        K, U, V and the router plain parameters (a parametrization computes them anew on every access)."""
+        """The tensors of the block (projection, head norm's weight or None, router, K, U, V, output projection) where every
+        step is this module's own, else None: heads_and_gate, and plain bias-free projections, RMSNorm and operator, with no
+        override in a subclass, on an instance or on a patched class and no hook that would have a say; all of them plain
+        parameters (a parametrization computes a tensor anew on every access)."""
         m, p = self._modules, self._parameters
-        return (type(self).heads_and_gate is _HEADS_AND_GATE and "heads_and_gate" not in self.__dict__
-                and _runs_own_forward(m.get("op"), FlashMLPMoE)
-                and all(_runs_own_forward(w, nn.Linear) and w.bias is None for w in (m.get("w_self"), m.get("w_self_2")))
-                and (self.q_norm is None or _runs_own_forward(self.q_norm, RMSNorm))
-                and all(p.get(n) is not None for n in ("K", "U", "V", "router")) and not _global_hooks())
+        w1, w2, q_norm = m.get("w_self"), m.get("w_self_2"), m["q_norm"] if "q_norm" in m else self.q_norm
+        if not (type(self).heads_and_gate is _HEADS_AND_GATE and "heads_and_gate" not in self.__dict__
+                and _runs_own_forward(m.get("op"), FlashMLPMoE) and _runs_own_forward(w1, nn.Linear)
+                and _runs_own_forward(w2, nn.Linear) and (q_norm is None or _runs_own_forward(q_norm, RMSNorm))
+                and w1._parameters.get("bias", w1) is None and w2._parameters.get("bias", w2) is None and not _global_hooks()):
+            return None
+        weights = [w1._parameters.get("weight"), p.get("router"), p.get("K"), p.get("U"), p.get("V"), w2._parameters.get("weight")]
+        if q_norm is not None:
+            weights.append(q_norm._parameters.get("weight"))
+        if any(w is None for w in weights):
+            return None
+        return weights[0], None if q_norm is None else weights[6], *weights[1:6]
 
     def _one_node(self, x):
-        """Whether the block can run as one native node (projection, prologue, operator, projection: the same kernels and
-        library products as the steps below, a quarter of the host time): bfloat16 on the GPU, with steps that are all its
-        own and no autocast context or tensor subclass that would change them.  (More than 32 experts take the prologue's
-        two-tile instances, which heads_and_gate chooses among.)"""
+        """The block's tensors where it can run as one native node (projection, prologue, operator, projection: the same kernels
+        and library products as the steps below, a quarter of the host time), else None: bfloat16 on the GPU, with steps that
+        are all its own and no autocast context or tensor subclass that would change them.  (More than 32 experts take the
+        prologue's two-tile instances, which heads_and_gate chooses among.)"""
         if not (self.router_input == "q" and self.fused_prologue and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() == 3
-                and self.num_experts <= 32 and self.head_dim in (64, 96, 128) and self._stock_steps()
-                and not torch.is_autocast_enabled("cuda") and _capi.native_nodes()):
-            return False
-        weights = (self.w_self.weight, self.w_self_2.weight, self.K, self.U, self.V)
-        return (all(w.dtype == torch.bfloat16 for w in weights)
-                and not torch.overrides.has_torch_function((x, *weights, self.router)))
+                and self.num_experts <= 32 and self.head_dim in (64, 96, 128)):
+            return None
+        weights = self._stock_steps()
+        if weights is None or torch.is_autocast_enabled("cuda") or not _capi.native_nodes():
+            return None
+        w1, norm, router, K, U, V, w2 = weights
+        if not (w1.dtype == w2.dtype == K.dtype == U.dtype == V.dtype == torch.bfloat16
+                and not torch.overrides.has_torch_function((x, w1, w2, K, U, V, router, norm))):
+            return None
+        return weights
 
     def forward(self, x):
         B, S, hid = x.shape
-        if self._one_node(x):
-            return _capi.native().block(x, self.w_self.weight, None if self.q_norm is None else self.q_norm.weight, self.router,
-                                        self.K, self.U, self.V, self.w_self_2.weight, self.rms_norm_eps, self.op.one_part)
+        weights = self._one_node(x)
+        if weights is not None:
+            return _capi.native().block(x, *weights, self.rms_norm_eps, self._modules["op"].one_part)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
