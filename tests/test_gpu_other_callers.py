@@ -69,6 +69,23 @@ def test_second_derivative_of_the_block_is_the_stepwise_one():
     assert torch.equal(*out)
 
 
+@pytest.mark.parametrize("frozen", [(), ("w_self.weight",), ("w_self_2.weight", "K")])
+def test_every_second_derivative_of_the_block_is_the_stepwise_one(frozen):
+    """All first gradients under create_graph, and what they hand back to every tensor."""
+    layer, x, dY = _layer(), _x(0, grad=True), _x(1, grad=True)
+    params = {n: p.requires_grad_(n not in frozen) for n, p in layer.named_parameters()}
+    leaves = [x, *(p for n, p in params.items() if n not in frozen)]
+    out = []
+    for stepwise in (False, True):
+        if stepwise:
+            layer.w_self.register_forward_hook(lambda *a: None)
+        first = torch.autograd.grad(layer(x), leaves, dY, create_graph=True)
+        loss = sum(g.float().square().mean() for g in first if g.requires_grad)
+        out.append([*first, *torch.autograd.grad(loss, [*leaves, dY], allow_unused=True)])
+    for i, (a, b) in enumerate(zip(*out)):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b)), i
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_parameters_at_any_place_of_a_flat_buffer(dtype):
     x4 = _x(0).view(B, S, H, dh)
