@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(LIBDIR, "libmhffn_hip.so")
-SOURCES = ["mhffn_capi.hip", "mhffn_fwd.hip", "mhffn_bwd.hip", "mhffn_f32.hip", "mhffn_gate.hip", "mhffn_rope.hip"]
+SOURCES = ["mhffn_capi.hip", "mhffn_fwd.hip", "mhffn_bwd.hip", "mhffn_f32.hip", "mhffn_gate.hip", "mhffn_rope.hip", "mhffn_product.hip"]
 # the torch side: an extension module on top of the C ABI, plain C++
 NATIVE_LIB = os.path.join(LIBDIR, "_native.so")
 NATIVE_SOURCE = "mhffn_torch.cpp"
@@ -111,9 +111,10 @@ EXPECTED_KERNELS = (
     ("mhffn_fwd_kernel", 3), ("mhffn_bwd_dqdr_kernel", 3), ("mhffn_bwd_dkdudv_kernel", 6),
     ("mhffn_gate_fwd_kernel", 12), ("mhffn_gate_bwd_kernel", 12),
 )
-# Variants of those kernels for smaller problems and for float32, under the same rule.
+# Variants of those kernels for smaller problems and for float32, and the products, under the same rule.
 VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
-                   ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 4))
+                   ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 4),
+                   ("mhffn_product_kernel", 9), ("mhffn_product_split_kernel", 2))
 # The one instantiation known to spill: head prologue backward for d_h = 128 with more than 32 experts and RMSNorm
 # (<128, 2, true>).  It is correct but slow; the block (MHFFNLayer.heads_and_gate) does not route that case to it.
 ALLOWED_SCRATCH = ("mhffn_gate_bwd_kernelILi128ELi2ELb1E",)

@@ -1,6 +1,7 @@
 // C ABI of libmhffn_hip.so: argument validation, error codes, dispatch.  No torch, no pybind, no allocation.
 #include "../../include/mhffn.h"
 #include "mhffn_common.hpp"
+#include "mhffn_product.hpp"
 
 // Scratch of mhffn_bwd_static: device memory that belongs to this code object, so the call needs no allocation.  Every
 // GPU the library is loaded on holds its own copy at its own address until the process ends.  In host code the array's
@@ -342,6 +343,35 @@ int mhffn_rope_bwd(const void* dq, const void* dk, const void* dv, const long* s
                                   (hipStream_t)stream) == hipSuccess
                ? MHFFN_OK
                : MHFFN_ERR_LAUNCH;
+}
+
+int mhffn_product_preferred(int M, int N) { return M > 0 && N > 0 && mhffn::product_preferred(M, N); }
+
+static int check_product(int form, int M, int N, int K)
+{
+    if (form != MHFFN_PRODUCT_NT && form != MHFFN_PRODUCT_NN && form != MHFFN_PRODUCT_TN) return MHFFN_ERR_SHAPE;
+    const int ld = form == MHFFN_PRODUCT_TN ? M : K;      // with N the lengths of the rows in memory
+    if (M <= 0 || N <= 0 || K <= 0 || N % 8 != 0 || ld % 8 != 0) return MHFFN_ERR_SHAPE;
+    // (a stage's lane offsets, at most 128 rows, are 32-bit, and so is the number of tiles)
+    if (N > (1 << 22) || ld > (1 << 22) || (double)M * N >= 1024.0 * 2147483648.0) return MHFFN_ERR_SHAPE;
+    return MHFFN_OK;
+}
+
+int mhffn_product_tile(int form, int M, int N, int K)
+{
+    return check_product(form, M, N, K) == MHFFN_OK ? mhffn::product_tile(form, M, N, K) : 0;
+}
+
+int mhffn_product(int form, const void* A, const void* B, void* C, int M, int N, int K, void* stream)
+{
+    const int rc = check_product(form, M, N, K);
+    if (rc != MHFFN_OK) return rc;
+    const void* ptrs[] = {A, B, C};
+    for (const void* p : ptrs) {
+        if (!p) return MHFFN_ERR_NULL_POINTER;
+        if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
+    }
+    return mhffn::launch_product(form, A, B, C, M, N, K, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
 }
 
 }  // extern "C"

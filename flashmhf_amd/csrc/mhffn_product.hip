@@ -1,0 +1,522 @@
+// The block's projections: C = A B over bfloat16 matrices, fp32 sums rounded once, in the three forms that a linear layer and
+// its backward need.
+//
+//     NT   C[M,N] = A[M,K]   B[N,K]^T    x w^T       both operands have the summed index running fastest ("rows")
+//     NN   C[M,N] = A[M,K]   B[K,N]      dy w        A rows, B the summed index slowest ("cols")
+//     TN   C[M,N] = A[K,M]^T B[K,N]      dy^T x      both cols
+//
+// They stand beside the library's products, which are made for matrices large enough to fill the chip with tiles of 256: at one
+// round of smaller tiles (product_preferred) these are faster.  us per product in a captured graph of 20, library / here:
+//     hidden 1024, tokens    64         512        1,024       2,048       4,096
+//         NT             6.6 / 3.9   6.4 / 5.0   7.7 / 6.8  10.0 / 8.8  13.1 / 12.9
+//         NN             8.7 / 6.2   7.9 / 6.4   9.2 / 6.6  11.2 / 8.7  14.8 / 13.1
+//         TN             4.7 / 3.9   8.4 / 5.0  11.2 / 6.6  16.1 / 9.5  27.9 / 16.4
+//     hidden 2048, 16 tokens: NT 5.3 / 4.8.
+// About 3 us of each are the launch, the first loads and the last stores; the rest is the rate at which a compute unit's LDS is
+// filled from L2 (65 to 80 GB/s in these kernels; 115 in a loop of nothing but fills), not the matrix pipe (a third busy).
+//
+// LDS units are 32 rows of 128 bytes: 32 rows of C x 64 of the summed index (rows), or 32 of the summed index x 64 rows of C
+// (cols), filled by global_load_lds_dwordx4, read by 16-byte row reads or transposing 8-byte reads.  Chunk c (16 bytes) of row r
+// sits at c ^ prod_swz(r), which makes both kinds of read free of bank conflicts (16 consecutive rows at one chunk, and 4
+// consecutive rows at 4 aligned chunks, each cover 256 bytes once).
+#include "mhffn_common.hpp"
+#include "mhffn_product.hpp"
+
+namespace mhffn {
+
+constexpr int PROD_UNIT_B = 4096;
+constexpr int FILLERS = 4;          // waves of a tile kernel's workgroup that do nothing but fill
+__device__ __forceinline__ int prod_swz(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
+
+struct ProductArgs {
+    const bf16_t* A;
+    const bf16_t* B;
+    bf16_t* C;
+    int M, N, K;
+    int mtiles, ntiles;
+};
+
+// (what lanes of a fill read where the summed index or the columns end)
+static __device__ __align__(16) const unsigned prod_zeros[4] = {0u, 0u, 0u, 0u};
+
+// Workgroup i runs on XCD i % 8: each XCD takes a run of consecutive tiles, counted in columns four tiles of rows high, so that what
+// it reads fits its L2.
+__device__ __forceinline__ void prod_tile(const ProductArgs& p, int& mt, int& nt)
+{
+    const unsigned total = p.mtiles * p.ntiles, xcd = blockIdx.x & 7, q = total >> 3, rem = total & 7;
+    const unsigned t = (blockIdx.x >> 3) + xcd * q + (xcd < rem ? xcd : rem);
+    const unsigned band = t / (4u * p.ntiles), in = t - band * 4u * p.ntiles;
+    const unsigned high = min(4u, p.mtiles - 4u * band);
+    mt = 4 * band + in % high;
+    nt = in / high;
+}
+
+// One operand's share of a stage: BR rows of C, KU units of 64 of the summed index, filled by WAVES waves: COUNT instructions each
+// per stage, at a uniform base plus a lane offset that does not change from stage to stage.  Rows of C that are not there are
+// the last one again (nothing stores what they give); where the summed index ends, zeros.
+template <bool COLS, int BR, int KU, int WAVES>
+struct ProductFill {
+    static constexpr int COUNT = BR * KU / (8 * WAVES), REGION_B = BR * KU * 128;
+    const unsigned char* base;     // wave-uniform
+    unsigned off[COUNT];
+    int lim[COUNT];                // the lane has something to read while stage * KU * 64 < lim
+    long inc;
+    __device__ __forceinline__ void init(const bf16_t* X, int row0, int rows, int K, int wave, int lane)
+    {
+        const long ld = COLS ? rows : K;
+        base = reinterpret_cast<const unsigned char*>(X + (COLS ? row0 : row0 * ld));
+        inc = 2 * (COLS ? KU * 64 * ld : KU * 64);
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i) {
+            const int id = wave * COUNT + i, unit = id >> 2, r = 8 * (id & 3) + (lane >> 3), c = (lane & 7) ^ prod_swz(r);
+            if constexpr (COLS) {
+                const int kr = unit / (BR / 64), cu = unit % (BR / 64);
+                const int k = 32 * kr + r, col = 64 * cu + 8 * c;
+                off[i] = 2 * (unsigned)(k * ld + col);
+                lim[i] = row0 + col < rows ? K - k : 0;
+            } else {
+                const int ku = unit / (BR / 32), rg = unit % (BR / 32);
+                const int k = 64 * ku + 8 * c, row = 32 * rg + r;
+                off[i] = 2 * (unsigned)((row0 + row < rows ? row : rows - 1 - row0) * ld + k);
+                lim[i] = K - k;
+            }
+        }
+    }
+    // CHECK: a stage that reaches beyond the end of the summed index or a tile that reaches beyond the last column
+    template <int I, bool CHECK>
+    __device__ __forceinline__ void issue(unsigned char* region, int k0, int wave) const
+    {
+        const unsigned char* p = base + off[I];
+        if constexpr (CHECK) p = k0 < lim[I] ? p : reinterpret_cast<const unsigned char*>(prod_zeros);
+        __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(region + (wave * COUNT + I) * 1024), 16, 0, 0);
+    }
+    __device__ __forceinline__ void skip(int stages) { base += stages * inc; }
+};
+
+template <int IMM>
+__device__ __forceinline__ TrOperand prod_read_cols(unsigned lo, unsigned hi)
+{
+    TrOperand t;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(t.lo) : "v"(lo), "n"(IMM));
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(t.hi) : "v"(hi), "n"(IMM));
+    return t;
+}
+
+// One operand's reads of a wave: TR tiles of 32 rows of C from tile t0 on, of KGS k-groups the k-steps (16 each) of group kg.
+// (The reads are inline assembly and in flight only inside one basic block: nothing can copy their registers before they arrive.)
+template <bool COLS, int BR, int KU, int TR, int KGS>
+struct ProductRead {
+    static constexpr int KSW = 4 * KU / KGS;
+    unsigned off[COLS ? 2 * TR : KSW];
+    struct Set {
+        u32x4 row[COLS ? 1 : TR][COLS ? 1 : KSW];
+        TrOperand col[COLS ? TR : 1][COLS ? KSW : 1];
+    };
+    __device__ __forceinline__ void init(int t0, int kg, int lane)
+    {
+        const int l32 = lane & 31, g = lane >> 5;
+        if constexpr (COLS) {
+            const int lam = lane & 15;
+#pragma unroll
+            for (int i = 0; i < TR; ++i)
+#pragma unroll
+                for (int hi = 0; hi < 2; ++hi) {
+                    const int r = 8 * g + 4 * hi + (lam >> 2), ct = t0 + i;
+                    const int chunk = 4 * (ct & 1) + 2 * (l32 >> 4) + ((lam & 3) >> 1);
+                    off[2 * i + hi] = (kg * (KSW / 2) * ((BR + 63) / 64) + (ct >> 1)) * PROD_UNIT_B + r * 128 + ((chunk ^ prod_swz(r)) << 4) + (lam & 1) * 8;
+                }
+        } else {
+#pragma unroll
+            for (int j = 0; j < KSW; ++j) {
+                const int ks = kg * KSW + j;
+                off[j] = ((ks >> 2) * (BR / 32) + t0) * PROD_UNIT_B + l32 * 128 + (((2 * (ks & 3) + g) ^ prod_swz(l32)) << 4);
+            }
+        }
+    }
+    template <int J, int I>
+    __device__ __forceinline__ void request(unsigned base, Set& s) const      // k-step J of tile I
+    {
+        if constexpr (COLS) {
+            constexpr int IMM = (J >> 1) * ((BR + 63) / 64) * PROD_UNIT_B + (J & 1) * 2048;
+            s.col[I][J] = prod_read_cols<IMM>(base + off[2 * I], base + off[2 * I + 1]);
+        } else {
+            s.row[I][J] = lds_read16_async<I * PROD_UNIT_B>(base + off[J]);
+        }
+    }
+    // behind a wait: no use of the operands above it
+    static __device__ __forceinline__ void arrived(Set& s, int j)
+    {
+#pragma unroll
+        for (int i = 0; i < TR; ++i) {
+            if constexpr (COLS) asm volatile("" : "+v"(s.col[i][j].lo), "+v"(s.col[i][j].hi));
+            else asm volatile("" : "+v"(s.row[i][j]));
+        }
+    }
+    static __device__ __forceinline__ bf16x8 get(const Set& s, int i, int j)
+    {
+        if constexpr (COLS) return tr_value(s.col[i][j]);
+        else return __builtin_bit_cast(bf16x8, s.row[i][j]);
+    }
+};
+
+// BM x BN of C per workgroup.  Four waves fill a ring of NST stages of KU * 64 of the summed index.  Eight multiply: two k-groups
+// (each takes half of a stage's k-steps; their sums are added at the end) of 2 x 2 waves with BM/2 x BN/2 of the tile each, one
+// wave of each group per SIMD, half a stage apart: one reads its operands while the other multiplies.
+// The waves that multiply do not fill: a fill instruction holds its wave for 30 ns and more, and in the same wave it held up the
+// products behind it (TN of 1,024 x 1,024 x 2,048: 11.1 us with every wave filling, 12.2 with the fills between the products, 9.5
+// so; with all eight waves reading, then multiplying together 10.0 to 11.1).
+template <bool ACOLS, bool BCOLS, int BM, int BN, int KU, int NST>
+__global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(ProductArgs p)
+{
+    constexpr int TM = BM / 64, TN = BN / 64;
+    using FA = ProductFill<ACOLS, BM, KU, FILLERS>;
+    using FB = ProductFill<BCOLS, BN, KU, FILLERS>;
+    constexpr int FILLS = FA::COUNT + FB::COUNT, STAGE_B = FA::REGION_B + FB::REGION_B, KSW = 2 * KU;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+
+    int mt, nt;
+    prod_tile(p, mt, nt);
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int nst = (p.K + 64 * KU - 1) / (64 * KU);
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Barriers 2st + 1 and 2st + 2 of a stage, counted from the first as 0: group 0 reads stage st before 2st + 1 and multiplies
+    // before 2st + 2, group 1 one barrier later; fillers refill the slot of stage st - 1 behind barrier 2st, when both have read it,
+    // and have seen stage st + 1 land before barrier 2st + 2.
+    if (wave >= 8) {
+        const int pw = wave - 8;
+        FA fa;
+        FB fb;
+        fa.init(p.A, m0, p.M, p.K, pw, lane);
+        fb.init(p.B, n0, p.N, p.K, pw, lane);
+        const bool inside = (!ACOLS || m0 + BM <= p.M) && (!BCOLS || n0 + BN <= p.N);
+        auto issue = [&](int st, int slot) {
+            unsigned char* s = smem + slot * STAGE_B;
+            auto all = [&](auto check_) {
+                constexpr bool CHECK = decltype(check_)::value;
+                static_for<FA::COUNT>([&](auto ic) { fa.template issue<decltype(ic)::value, CHECK>(s, st * KU * 64, pw); });
+                static_for<FB::COUNT>([&](auto ic) { fb.template issue<decltype(ic)::value, CHECK>(s + FA::REGION_B, st * KU * 64, pw); });
+            };
+            if (inside && (st + 1) * KU * 64 <= p.K) all(std::false_type{});
+            else all(std::true_type{});
+            fa.skip(1);
+            fb.skip(1);
+        };
+        // this wave's fills of all stages up to `st` have landed, those of younger ones (up to NST - 2) may be in flight
+        auto landed = [&](int st, int issued) {
+            const int younger = issued - 1 - st;
+            static_assert((NST - 2) * FILLS < 64, "the counter has six bits");
+            static_for<NST - 1>([&](auto yc) {
+                constexpr int y = decltype(yc)::value;
+                if (younger == y) wait_vmcnt<y * FILLS>();
+            });
+        };
+#pragma unroll
+        for (int s = 0; s < NST - 1; ++s)
+            if (s < nst) issue(s, s);
+        landed(0, NST - 1 < nst ? NST - 1 : nst);
+        barrier();
+        int prev = NST - 1;
+        for (int st = 0; st < nst; ++st) {
+            if (st + NST - 1 < nst) issue(st + NST - 1, prev);
+            barrier();
+            if (st + 1 < nst) landed(st + 1, st + NST < nst ? st + NST : nst);
+            barrier();
+            prev = prev + 1 == NST ? 0 : prev + 1;
+        }
+        barrier();
+        __syncthreads();
+        __syncthreads();
+        __syncthreads();
+        return;
+    }
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int x = 0; x < 16; ++x) acc[i][j][x] = 0.0f;
+    using RA = ProductRead<ACOLS, BM, KU, TM, 2>;
+    using RB = ProductRead<BCOLS, BN, KU, TN, 2>;
+    RA ra;
+    RB rb;
+    ra.init(wm * TM, kg, lane);
+    rb.init(wn * TN, kg, lane);
+    const unsigned smem0 = lds_addr(smem);
+    barrier();
+    if (kg == 1) barrier();
+    int slot = 0;
+    for (int st = 0; st < nst; ++st) {
+        const unsigned sa = smem0 + slot * STAGE_B, sb = sa + FA::REGION_B;
+        typename RA::Set a;
+        typename RB::Set b;
+        static_for<KSW>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            static_for<TM>([&](auto ic) { ra.template request<j, decltype(ic)::value>(sa, a); });
+            static_for<TN>([&](auto ic) { rb.template request<j, decltype(ic)::value>(sb, b); });
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        lds_wait_n<0>();
+        static_for<KSW>([&](auto jc) {
+            RA::arrived(a, decltype(jc)::value);
+            RB::arrived(b, decltype(jc)::value);
+        });
+        barrier();
+        static_for<KSW>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int n = 0; n < TN; ++n)
+                    acc[i][n] = mfma32(RB::get(b, n, j), RA::get(a, i, j), acc[i][n]);   // (lanes: rows of C)
+        });
+        barrier();
+        slot = slot + 1 == NST ? 0 : slot + 1;
+    }
+    if (kg == 0) barrier();
+    __syncthreads();
+    // The second k-group's sums go to the first through LDS (16 bytes per lane and register quad), then the tile leaves as whole rows.
+    f32x4* xch = reinterpret_cast<f32x4*>(smem) + (wave & 3) * (TM * TN * 4 * 64) + lane;
+    if (kg == 1) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int n = 0; n < TN; ++n)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    f32x4 v;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = acc[i][n][4 * a + x];
+                    xch[((i * TN + n) * 4 + a) * 64] = v;
+                }
+    }
+    __syncthreads();
+    // rows of BN * 2 bytes, 16-byte chunk c of row r at c ^ (r % 8)
+    unsigned char* out = smem + BM * BN * 4;
+    if (kg == 0) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int n = 0; n < TN; ++n)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4 other = xch[((i * TN + n) * 4 + a) * 64];
+                    bf16x4 v;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = (bf16_t)(acc[i][n][4 * a + x] + other[x]);
+                    const int r = (wm * TM + i) * 32 + l32, c = (wn * TN + n) * 4 + a;
+                    *reinterpret_cast<bf16x4*>(out + r * (BN * 2) + ((c ^ (r & 7)) << 4) + 8 * g) = v;
+                }
+    }
+    __syncthreads();
+    constexpr int CH = BN / 8;
+#pragma unroll
+    for (int k = 0; k < BM * CH / 512; ++k) {
+        const int id = k * 512 + threadIdx.x, r = id / CH, c = id % CH;
+        if (m0 + r < p.M && n0 + 8 * c < p.N)
+            *reinterpret_cast<u32x4*>(p.C + (long)(m0 + r) * p.N + n0 + 8 * c) =
+                *reinterpret_cast<const u32x4*>(out + r * (BN * 2) + ((c ^ (r & 7)) << 4));
+    }
+}
+
+// NT with few tiles: 32 TM x 32 TN of C per workgroup.  Its eight waves take every eighth chunk of 64 of the summed index each, through
+// LDS of their own (Q chunks in flight, no barrier before the end), and their sums are added at the end, in the waves' order.
+// (512 x 1,024 x 1,024: 5.0 us with 64 x 32 against 6.4 with the tiles of 64 above; 64 x 64 this way 6.7.)
+template <int TM, int TN, int Q>
+__global__ __launch_bounds__(512) void mhffn_product_split_kernel(ProductArgs p)
+{
+    constexpr int BM = 32 * TM, BN = 32 * TN;
+    using FA = ProductFill<false, BM, 1, 1>;
+    using FB = ProductFill<false, BN, 1, 1>;
+    using RA = ProductRead<false, BM, 1, TM, 1>;
+    using RB = ProductRead<false, BN, 1, TN, 1>;
+    constexpr int FILLS = FA::COUNT + FB::COUNT, CHUNK_B = FA::REGION_B + FB::REGION_B;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int mt, nt;
+    prod_tile(p, mt, nt);
+    const int m0 = mt * BM, n0 = nt * BN;
+    unsigned char* own = smem + wave * Q * CHUNK_B;
+    FA fa;
+    FB fb;
+    fa.init(p.A, m0, p.M, p.K, 0, lane);
+    fb.init(p.B, n0, p.N, p.K, 0, lane);
+    fa.skip(wave);
+    fb.skip(wave);
+    const int chunks = (p.K + 63) / 64;
+    auto fill = [&](int ch, int buf) {
+        unsigned char* s = own + buf * CHUNK_B;
+        auto all = [&](auto check_) {
+            constexpr bool CHECK = decltype(check_)::value;
+            static_for<FA::COUNT>([&](auto ic) { fa.template issue<decltype(ic)::value, CHECK>(s, 64 * ch, 0); });
+            static_for<FB::COUNT>([&](auto ic) { fb.template issue<decltype(ic)::value, CHECK>(s + FA::REGION_B, 64 * ch, 0); });
+        };
+        if (64 * ch + 64 <= p.K) all(std::false_type{});
+        else all(std::true_type{});
+        fa.skip(8);
+        fb.skip(8);
+    };
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+        if (wave + 8 * q < chunks) fill(wave + 8 * q, q);
+    RA ra;
+    RB rb;
+    ra.init(0, 0, lane);
+    rb.init(0, 0, lane);
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int x = 0; x < 16; ++x) acc[i][j][x] = 0.0f;
+    int buf = 0;
+    for (int ch = wave; ch < chunks; ch += 8) {
+        if (Q > 1 && ch + 8 < chunks) wait_vmcnt<(Q - 1) * FILLS>();
+        else wait_vmcnt<0>();
+        static_assert(Q <= 2, "the wait above");
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned t = lds_addr(own) + buf * CHUNK_B;
+        typename RA::Set a;
+        typename RB::Set b;
+        static_for<4>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            static_for<TM>([&](auto ic) { ra.template request<j, decltype(ic)::value>(t, a); });
+            static_for<TN>([&](auto ic) { rb.template request<j, decltype(ic)::value>(t + FA::REGION_B, b); });
+        });
+        lds_wait_n<0>();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            RA::arrived(a, j);
+            RB::arrived(b, j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (ch + 8 * Q < chunks) fill(ch + 8 * Q, buf);      // (this wave alone reads what it fills)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int n = 0; n < TN; ++n) acc[i][n] = mfma32(RB::get(b, n, j), RA::get(a, i, j), acc[i][n]);   // (lanes: rows of C)
+        buf = buf + 1 == Q ? 0 : buf + 1;
+    }
+    __syncthreads();
+    f32x4* sums = reinterpret_cast<f32x4*>(smem);
+    constexpr int QUADS = TM * TN * 4;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                f32x4 v;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[x] = acc[i][n][4 * q + x];
+                sums[(wave * QUADS + (i * TN + n) * 4 + q) * 64 + lane] = v;
+            }
+    __syncthreads();
+    for (int k = wave; k < QUADS; k += 8) {
+        f32x4 s = sums[k * 64 + lane];
+#pragma unroll
+        for (int v = 1; v < 8; ++v) s += sums[(v * QUADS + k) * 64 + lane];
+        bf16x4 o;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) o[x] = (bf16_t)s[x];
+        const int m = m0 + 32 * (k / (4 * TN)) + l32, n = n0 + 32 * (k / 4 % TN) + 8 * (k % 4) + 4 * g;
+        if (m < p.M && n < p.N) *reinterpret_cast<bf16x4*>(p.C + (long)m * p.N + n) = o;
+    }
+}
+
+template <bool ACOLS, bool BCOLS, int BM, int BN, int KU, int NST>
+static hipError_t launch_tiles(ProductArgs a, hipStream_t st)
+{
+    constexpr int ring = (BM + BN) * KU * 128 * NST, tail = BM * BN * 6, smem = ring > tail ? ring : tail;
+    static_assert(smem <= 160 * 1024, "LDS of a compute unit");
+    static LdsOptIn optin;
+    auto* fn = mhffn_product_kernel<ACOLS, BCOLS, BM, BN, KU, NST>;
+    const hipError_t e = ensure_dynamic_lds(optin, (const void*)fn, smem);
+    if (e != hipSuccess) return e;
+    a.mtiles = (a.M + BM - 1) / BM;
+    a.ntiles = (a.N + BN - 1) / BN;
+    hipLaunchKernelGGL(fn, dim3((unsigned)a.mtiles * a.ntiles), dim3(512 + 64 * FILLERS), smem, st, a);
+    return hipGetLastError();
+}
+template <int TM, int TN, int Q>
+static hipError_t launch_split(ProductArgs a, hipStream_t st)
+{
+    constexpr int smem = 8 * PROD_UNIT_B * (TM + TN) * Q;      // (holds the sums, 8 * TM * TN units, too)
+    static_assert(TM * TN <= (TM + TN) * Q && smem <= 160 * 1024, "LDS of a compute unit");
+    static LdsOptIn optin;
+    auto* fn = mhffn_product_split_kernel<TM, TN, Q>;
+    const hipError_t e = ensure_dynamic_lds(optin, (const void*)fn, smem);
+    if (e != hipSuccess) return e;
+    a.mtiles = (a.M + 32 * TM - 1) / (32 * TM);
+    a.ntiles = (a.N + 32 * TN - 1) / (32 * TN);
+    hipLaunchKernelGGL(fn, dim3((unsigned)a.mtiles * a.ntiles), dim3(512), smem, st, a);
+    return hipGetLastError();
+}
+
+// Time of a launch in us: base + rounds of CUS workgroups x (stages of 64 of the summed index x step, slower by up to `full` as the
+// chip fills) + again for every round after the first.  Fitted to the three forms at hidden 768, 1024 and 2048 with 16 to 8,192
+// tokens; the pick is the fastest or within 0.4 us of it at each of these where one round suffices.
+struct ProductVariant {
+    int bm, bn;
+    double base, step, full, again;
+};
+constexpr ProductVariant PRODUCT_VARIANTS[] = {{64, 64, 3.2, 0.19, 0.1, 2.4},  {128, 64, 3.6, 0.28, 0.15, 2.5}, {128, 128, 4.0, 0.38, 0.45, 3.0},
+                                               {32, 32, 2.4, 0.08, 0.2, 1.3},  {64, 32, 3.0, 0.115, 0.1, 1.6}};     // (the last two: NT)
+static int product_variant(int form, int M, int N, int K)
+{
+    int best = 0;
+    double best_us = 0;
+    for (int v = 0; v < (form == PRODUCT_NT ? 5 : 3); ++v) {
+        const ProductVariant& p = PRODUCT_VARIANTS[v];
+        const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), rounds = (tiles + CUS - 1) / CUS;
+        const double load = tiles <= CUS / 2 ? 0 : tiles >= CUS ? 1 : (tiles - CUS / 2) / (double)(CUS / 2);
+        const double us = p.base + (rounds - 1) * p.again + rounds * ((K + 63) / 64) * p.step * (1 + p.full * load);
+        if (best_us == 0 || us < best_us) { best_us = us; best = v; }
+    }
+    return best;
+}
+int product_tile(int form, int M, int N, int K)
+{
+    const ProductVariant& p = PRODUCT_VARIANTS[product_variant(form, M, N, K)];
+    return 65536 * p.bm + p.bn;
+}
+// One round of the largest tiles: there these kernels are as fast as the library's or faster (NT of 3,000 x 1,024 x 1,024 11.3 us
+// against 11.4, of 2,048^3 21.6 against 22.6; TN of the latter 22.3 against 26.6); with more its larger tiles win in NT and NN
+// (8,192 x 1,024 x 1,024: 25.0 against 21.9).
+bool product_preferred(int M, int N) { return (long)((M + 127) / 128) * ((N + 127) / 128) <= CUS; }
+
+template <bool ACOLS, bool BCOLS>
+static hipError_t launch_form(const ProductArgs& a, int variant, hipStream_t st)
+{
+    switch (variant) {
+        case 0: return launch_tiles<ACOLS, BCOLS, 64, 64, 2, 4>(a, st);
+        case 1: return launch_tiles<ACOLS, BCOLS, 128, 64, 2, 3>(a, st);
+        case 2: return launch_tiles<ACOLS, BCOLS, 128, 128, 1, 4>(a, st);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_product(int form, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st)
+{
+    const ProductArgs a{(const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, M, N, K, 0, 0};
+    const int v = product_variant(form, M, N, K);
+    switch (form) {
+        case PRODUCT_NT: return v == 3 ? launch_split<1, 1, 2>(a, st) : v == 4 ? launch_split<2, 1, 1>(a, st) : launch_form<false, false>(a, v, st);
+        case PRODUCT_NN: return launch_form<false, true>(a, v, st);
+        case PRODUCT_TN: return launch_form<true, true>(a, v, st);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace mhffn

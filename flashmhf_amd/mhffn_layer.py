@@ -65,6 +65,19 @@ def router_gate(logits):
     return R / R.sum(dim=-1, keepdim=True).clamp(min=1e-20)
 
 
+class Projection(nn.Linear):
+    """nn.Linear whose products, forward and backward, run in the framework's kernels where these are faster than the library's
+    (csrc/mhffn_product.hip): bfloat16 on the GPU, without bias, called as the plain layer; else nn.Linear's own forward."""
+
+    def forward(self, x):
+        w = self.weight
+        if (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and self.bias is None and nn.Linear.forward is _FORWARD[nn.Linear]
+                and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling() and _capi.native_nodes()
+                and not torch.overrides.has_torch_function((x, w))):
+            return _capi.native().linear(x, w)
+        return super().forward(x)
+
+
 def _unhooked(m):
     return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
 
@@ -75,6 +88,11 @@ def _runs_own_forward(m, cls):
     return type(m) is cls and cls.forward is _FORWARD[cls] and "forward" not in m.__dict__ and _unhooked(m)
 
 
+def _plain_linear(m):
+    """A Projection, or the nn.Linear that a program or a saved module has in its place, which keeps the library's products."""
+    return _runs_own_forward(m, Projection if type(m) is Projection else nn.Linear) and nn.Linear.forward is _FORWARD[nn.Linear]
+
+
 def _global_hooks():
     g = nn.modules.module
     return g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks
@@ -82,7 +100,7 @@ def _global_hooks():
 
 class MHFFNLayer(nn.Module):
     def __init__(self, hidden_size, num_heads, num_experts, expert_dim, num_kuv_heads=None, *, apply_rmsnorm=False,
-                 rms_norm_eps=1e-6, bias=False, router_input="q", op=None, fused_prologue=True):
+                 rms_norm_eps=1e-6, bias=False, router_input="q", op=None, fused_prologue=True, linear=Projection):
         super().__init__()
         if hidden_size % num_heads:
             raise ValueError("hidden_size must be a multiple of num_heads")
@@ -95,8 +113,8 @@ class MHFFNLayer(nn.Module):
         self.router_input = router_input
         self.fused_prologue = fused_prologue
         self.rms_norm_eps = rms_norm_eps
-        self.w_self = nn.Linear(hidden_size, hidden_size, bias=bias)
-        self.w_self_2 = nn.Linear(hidden_size, hidden_size, bias=bias)
+        self.w_self = linear(hidden_size, hidden_size, bias=bias)
+        self.w_self_2 = linear(hidden_size, hidden_size, bias=bias)
         wshape = (self.num_kuv_heads, num_experts, expert_dim, self.head_dim)
         std = self.head_dim ** -0.5
         self.K = nn.Parameter(torch.randn(wshape) * std)
@@ -155,8 +173,8 @@ class MHFFNLayer(nn.Module):
         m, p = self._modules, self._parameters
         w1, w2, q_norm = m.get("w_self"), m.get("w_self_2"), m["q_norm"] if "q_norm" in m else self.q_norm
         if not (type(self).heads_and_gate is _HEADS_AND_GATE and "heads_and_gate" not in self.__dict__
-                and _runs_own_forward(m.get("op"), FlashMLPMoE) and _runs_own_forward(w1, nn.Linear)
-                and _runs_own_forward(w2, nn.Linear) and (q_norm is None or _runs_own_forward(q_norm, RMSNorm))
+                and _runs_own_forward(m.get("op"), FlashMLPMoE) and _plain_linear(w1) and _plain_linear(w2)
+                and (q_norm is None or _runs_own_forward(q_norm, RMSNorm))
                 and w1._parameters.get("bias", w1) is None and w2._parameters.get("bias", w2) is None and not _global_hooks()):
             return None
         weights = [w1._parameters.get("weight"), p.get("router"), p.get("K"), p.get("U"), p.get("V"), w2._parameters.get("weight")]
@@ -187,14 +205,16 @@ class MHFFNLayer(nn.Module):
         B, S, hid = x.shape
         weights = self._one_node(x)
         if weights is not None:
-            return _capi.native().block(x, *weights, self.rms_norm_eps, self._modules["op"].one_part)
+            m = self._modules
+            own = type(m["w_self"]) is type(m["w_self_2"]) is Projection
+            return _capi.native().block(x, *weights, self.rms_norm_eps, m["op"].one_part, own)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
 
 
 # what _stock_steps compares with: the code as it is defined here
-_FORWARD = {c: c.forward for c in (nn.Linear, RMSNorm, FlashMLPMoE)}
+_FORWARD = {c: c.forward for c in (nn.Linear, Projection, RMSNorm, FlashMLPMoE)}
 _HEADS_AND_GATE = MHFFNLayer.heads_and_gate
 
 
@@ -256,6 +276,9 @@ class MHFFNDecoder(nn.Module):
         # depend on the rest of its batch.  (Rounding differences of the operator grow from block to block: another order
         # moves the gradients of a four-block model by 1 % of their norm.)
         layer_kw.setdefault("op", FlashMLPMoE(one_part=True))
+        # The library's products in the blocks as in the attention and the output head, for the same reason: sums taken another
+        # way (Projection) move single gradients of a four-block model by half of their root mean square.
+        layer_kw.setdefault("linear", nn.Linear)
         self.embed = nn.Embedding(vocab_size, hidden_size)
         self.blocks = nn.ModuleList(
             MHFFNDecoderBlock(hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps, **layer_kw)

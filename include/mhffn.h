@@ -222,6 +222,20 @@ int mhffn_rope_fwd(const void* qkv, const void* cos, const void* sin, void* q, v
 int mhffn_rope_bwd(const void* dq, const void* dk, const void* dv, const long* strides, const void* cos, const void* sin,
                    void* dqkv, int B, int S, int H, int d, void* stream);
 
+/* Products of row-major bfloat16 matrices with float32 sums, rounded once: the block's projections (modeling_mhffnmoe.py:371,
+ * :410) and their backward.
+ *   MHFFN_PRODUCT_NT   C[M,N] = A[M,K] B[N,K]^T     MHFFN_PRODUCT_NN   C[M,N] = A[M,K] B[K,N]
+ *   MHFFN_PRODUCT_TN   C[M,N] = A[K,M]^T B[K,N]
+ * Extents positive; N, and K (NT, NN) or M (TN), multiples of 8 (MHFFN_ERR_SHAPE otherwise).  mhffn_product_preferred() is 1
+ * where these kernels are meant for the size of the result, 0 where a BLAS library's larger tiles are faster;
+ * mhffn_product_tile() is the tile a product runs in, 65536 * rows + columns (0: extents refused). */
+#define MHFFN_PRODUCT_NT 0
+#define MHFFN_PRODUCT_NN 1
+#define MHFFN_PRODUCT_TN 2
+int mhffn_product_preferred(int M, int N);
+int mhffn_product_tile(int form, int M, int N, int K);
+int mhffn_product(int form, const void* A, const void* B, void* C, int M, int N, int K, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
