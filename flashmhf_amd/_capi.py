@@ -83,8 +83,8 @@ def lib():
         L.mhffn_rope_fwd.argtypes = [vp] * 5 + [ctypes.c_int] * 4 + [vp]
         L.mhffn_rope_bwd.argtypes = [vp] * 3 + [ctypes.POINTER(ctypes.c_long)] + [vp] * 3 + [ctypes.c_int] * 4 + [vp]
         L.mhffn_product_preferred.argtypes = [ctypes.c_int] * 2
-        L.mhffn_product_tile.argtypes = [ctypes.c_int] * 4
-        L.mhffn_product.argtypes = [ctypes.c_int] + [vp] * 3 + [ctypes.c_int] * 3 + [vp]
+        L.mhffn_product_tile.argtypes = [ctypes.c_int] * 5
+        L.mhffn_product.argtypes = [ctypes.c_int] * 2 + [vp] * 3 + [ctypes.c_int] * 3 + [vp]
         _lib = L
     return _lib
 

@@ -357,12 +357,12 @@ static int check_product(int form, int M, int N, int K)
     return MHFFN_OK;
 }
 
-int mhffn_product_tile(int form, int M, int N, int K)
+int mhffn_product_tile(int form, int in_order, int M, int N, int K)
 {
-    return check_product(form, M, N, K) == MHFFN_OK ? mhffn::product_tile(form, M, N, K) : 0;
+    return check_product(form, M, N, K) == MHFFN_OK ? mhffn::product_tile(form, in_order != 0, M, N, K) : 0;
 }
 
-int mhffn_product(int form, const void* A, const void* B, void* C, int M, int N, int K, void* stream)
+int mhffn_product(int form, int in_order, const void* A, const void* B, void* C, int M, int N, int K, void* stream)
 {
     const int rc = check_product(form, M, N, K);
     if (rc != MHFFN_OK) return rc;
@@ -371,7 +371,7 @@ int mhffn_product(int form, const void* A, const void* B, void* C, int M, int N,
         if (!p) return MHFFN_ERR_NULL_POINTER;
         if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
     }
-    return mhffn::launch_product(form, A, B, C, M, N, K, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
+    return mhffn::launch_product(form, in_order != 0, A, B, C, M, N, K, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
 }
 
 }  // extern "C"

@@ -8,12 +8,16 @@
 // They stand beside the library's products, which are made for matrices large enough to fill the chip with tiles of 256: at one
 // round of smaller tiles (product_preferred) these are faster.  us per product in a captured graph of 20, library / here:
 //     hidden 1024, tokens    64         512        1,024       2,048       4,096
-//         NT             6.6 / 3.9   6.4 / 5.0   7.7 / 6.8  10.0 / 8.8  13.1 / 12.9
-//         NN             8.7 / 6.2   7.9 / 6.4   9.2 / 6.6  11.2 / 8.7  14.8 / 13.1
-//         TN             4.7 / 3.9   8.4 / 5.0  11.2 / 6.6  16.1 / 9.5  27.9 / 16.4
+//         NT             6.6 / 3.9   6.5 / 5.1   8.0 / 7.5  10.3 / 9.1  13.5 / 12.5
+//         NN             8.7 / 6.8   8.0 / 6.9   9.3 / 7.2  11.2 / 8.8  14.3 / 12.7
+//         TN             4.7 / 3.8   8.5 / 5.2  11.3 / 6.8  16.1 / 10.1 27.5 / 17.6
 //     hidden 2048, 16 tokens: NT 5.3 / 4.8.
 // About 3 us of each are the launch, the first loads and the last stores; the rest is the rate at which a compute unit's LDS is
 // filled from L2 (65 to 80 GB/s in these kernels; 115 in a loop of nothing but fills), not the matrix pipe (a third busy).
+//
+// The tile kernels add the terms of an element in the order of the summed index, one accumulator from the first to the last (a tile
+// whose k-steps two groups of waves shared took 6.3 instead of 6.9 us for 64 x 64 of K = 1,024, as long or longer in larger ones).
+// The library's do, too, wherever it does not split the summed index: the same bits.  Only the split kernel (NT, few tiles) does not.
 //
 // LDS units are 32 rows of 128 bytes: 32 rows of C x 64 of the summed index (rows), or 32 of the summed index x 64 rows of C
 // (cols), filled by global_load_lds_dwordx4, read by 16-byte row reads or transposing 8-byte reads.  Chunk c (16 bytes) of row r
@@ -102,45 +106,47 @@ __device__ __forceinline__ TrOperand prod_read_cols(unsigned lo, unsigned hi)
     return t;
 }
 
-// One operand's reads of a wave: TR tiles of 32 rows of C from tile t0 on, of KGS k-groups the k-steps (16 each) of group kg.
-// (The reads are inline assembly and in flight only inside one basic block: nothing can copy their registers before they arrive.)
-template <bool COLS, int BR, int KU, int TR, int KGS>
+// One operand's reads of a wave: TR tiles of TH rows of C from tile t0 on, the steps of a stage: 16 of the summed index each for the
+// 32-row instruction, 32 for the 16-row one.  (The reads are inline assembly and in flight only inside one basic block: nothing
+// can copy their registers before they arrive.)
+template <bool COLS, int BR, int KU, int TH, int TR>
 struct ProductRead {
-    static constexpr int KSW = 4 * KU / KGS;
-    unsigned off[COLS ? 2 * TR : KSW];
+    static constexpr int STEPS = KU * (TH == 32 ? 4 : 2), ACROSS = (BR + 63) / 64;
+    unsigned off[COLS ? 2 * TR : STEPS];
     struct Set {
-        u32x4 row[COLS ? 1 : TR][COLS ? 1 : KSW];
-        TrOperand col[COLS ? TR : 1][COLS ? KSW : 1];
+        u32x4 row[COLS ? 1 : TR][COLS ? 1 : STEPS];
+        TrOperand col[COLS ? TR : 1][COLS ? STEPS : 1];
     };
-    __device__ __forceinline__ void init(int t0, int kg, int lane)
+    __device__ __forceinline__ void init(int t0, int lane)
     {
-        const int l32 = lane & 31, g = lane >> 5;
         if constexpr (COLS) {
             const int lam = lane & 15;
 #pragma unroll
             for (int i = 0; i < TR; ++i)
 #pragma unroll
                 for (int hi = 0; hi < 2; ++hi) {
-                    const int r = 8 * g + 4 * hi + (lam >> 2), ct = t0 + i;
-                    const int chunk = 4 * (ct & 1) + 2 * (l32 >> 4) + ((lam & 3) >> 1);
-                    off[2 * i + hi] = (kg * (KSW / 2) * ((BR + 63) / 64) + (ct >> 1)) * PROD_UNIT_B + r * 128 + ((chunk ^ prod_swz(r)) << 4) + (lam & 1) * 8;
+                    const int r = 8 * (lane / TH) + 4 * hi + (lam >> 2), col = (t0 + i) * TH + (lane % TH & 16);      // 16 columns from `col` on
+                    const int chunk = ((col & 63) >> 3) + ((lam & 3) >> 1);
+                    off[2 * i + hi] = (col >> 6) * PROD_UNIT_B + r * 128 + ((chunk ^ prod_swz(r)) << 4) + (lam & 1) * 8;
                 }
         } else {
+            const int r = t0 * TH + lane % TH;
 #pragma unroll
-            for (int j = 0; j < KSW; ++j) {
-                const int ks = kg * KSW + j;
-                off[j] = ((ks >> 2) * (BR / 32) + t0) * PROD_UNIT_B + l32 * 128 + (((2 * (ks & 3) + g) ^ prod_swz(l32)) << 4);
+            for (int j = 0; j < STEPS; ++j) {
+                constexpr int PER = TH == 32 ? 4 : 2;      // steps of a unit
+                const int chunk = 8 / PER * (j % PER) + lane / TH;
+                off[j] = (j / PER * (BR / 32) + (r >> 5)) * PROD_UNIT_B + (r & 31) * 128 + ((chunk ^ prod_swz(r & 31)) << 4);
             }
         }
     }
     template <int J, int I>
-    __device__ __forceinline__ void request(unsigned base, Set& s) const      // k-step J of tile I
+    __device__ __forceinline__ void request(unsigned base, Set& s) const      // step J of tile I
     {
         if constexpr (COLS) {
-            constexpr int IMM = (J >> 1) * ((BR + 63) / 64) * PROD_UNIT_B + (J & 1) * 2048;
+            constexpr int IMM = TH == 32 ? (J >> 1) * ACROSS * PROD_UNIT_B + (J & 1) * 2048 : J * ACROSS * PROD_UNIT_B;
             s.col[I][J] = prod_read_cols<IMM>(base + off[2 * I], base + off[2 * I + 1]);
         } else {
-            s.row[I][J] = lds_read16_async<I * PROD_UNIT_B>(base + off[J]);
+            s.row[I][J] = lds_read16_async<I * (TH == 32 ? PROD_UNIT_B : 2048)>(base + off[J]);
         }
     }
     // behind a wait: no use of the operands above it
@@ -158,24 +164,26 @@ struct ProductRead {
         else return __builtin_bit_cast(bf16x8, s.row[i][j]);
     }
 };
+__device__ __forceinline__ f32x16 prod_mfma(bf16x8 a, bf16x8 b, f32x16 c) { return mfma32(a, b, c); }
+__device__ __forceinline__ f32x4 prod_mfma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
-// BM x BN of C per workgroup.  Four waves fill a ring of NST stages of KU * 64 of the summed index.  Eight multiply: two k-groups
-// (each takes half of a stage's k-steps; their sums are added at the end) of 2 x 2 waves with BM/2 x BN/2 of the tile each, one
-// wave of each group per SIMD, half a stage apart: one reads its operands while the other multiplies.
+// BM x BN of C per workgroup.  Four waves fill a ring of NST stages of KU * 64 of the summed index.  Eight multiply, WM of them side by
+// side along the rows of the tile, with instructions of TH x TH; four of them (one per SIMD) run half a stage behind the other
+// four: one wave of a SIMD reads its operands while the other multiplies.
 // The waves that multiply do not fill: a fill instruction holds its wave for 30 ns and more, and in the same wave it held up the
 // products behind it (TN of 1,024 x 1,024 x 2,048: 11.1 us with every wave filling, 12.2 with the fills between the products, 9.5
-// so; with all eight waves reading, then multiplying together 10.0 to 11.1).
-template <bool ACOLS, bool BCOLS, int BM, int BN, int KU, int NST>
+// with waves of their own for them; all eight waves reading and then multiplying together were between these).
+template <bool ACOLS, bool BCOLS, int BM, int BN, int TH, int WM, int KU, int NST>
 __global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(ProductArgs p)
 {
-    constexpr int TM = BM / 64, TN = BN / 64;
+    constexpr int TM = BM / WM / TH, TN = BN / (8 / WM) / TH;      // tiles of a wave
     using FA = ProductFill<ACOLS, BM, KU, FILLERS>;
     using FB = ProductFill<BCOLS, BN, KU, FILLERS>;
-    constexpr int FILLS = FA::COUNT + FB::COUNT, STAGE_B = FA::REGION_B + FB::REGION_B, KSW = 2 * KU;
+    constexpr int FILLS = FA::COUNT + FB::COUNT, STAGE_B = FA::REGION_B + FB::REGION_B;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int late = wave >> 2, wm = wave % WM, wn = wave / WM;
 
     int mt, nt;
     prod_tile(p, mt, nt);
@@ -186,8 +194,8 @@ __global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(Produ
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
-    // Barriers 2st + 1 and 2st + 2 of a stage, counted from the first as 0: group 0 reads stage st before 2st + 1 and multiplies
-    // before 2st + 2, group 1 one barrier later; fillers refill the slot of stage st - 1 behind barrier 2st, when both have read it,
+    // Barriers 2st + 1 and 2st + 2 of a stage, counted from the first as 0: the early waves read stage st before 2st + 1 and multiply
+    // before 2st + 2, the late ones one barrier later; fillers refill the slot of stage st - 1 behind barrier 2st, when both have read it,
     // and have seen stage st + 1 land before barrier 2st + 2.
     if (wave >= 8) {
         const int pw = wave - 8;
@@ -233,110 +241,89 @@ __global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(Produ
         barrier();
         __syncthreads();
         __syncthreads();
-        __syncthreads();
         return;
     }
-    f32x16 acc[TM][TN];
+    using RA = ProductRead<ACOLS, BM, KU, TH, TM>;
+    using RB = ProductRead<BCOLS, BN, KU, TH, TN>;
+    using Acc = std::conditional_t<TH == 32, f32x16, f32x4>;
+    constexpr int STEPS = RA::STEPS, QUADS = TH == 32 ? 4 : 1;
+    Acc acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int x = 0; x < 16; ++x) acc[i][j][x] = 0.0f;
-    using RA = ProductRead<ACOLS, BM, KU, TM, 2>;
-    using RB = ProductRead<BCOLS, BN, KU, TN, 2>;
+            for (int x = 0; x < 4 * QUADS; ++x) acc[i][j][x] = 0.0f;
     RA ra;
     RB rb;
-    ra.init(wm * TM, kg, lane);
-    rb.init(wn * TN, kg, lane);
+    ra.init(wm * TM, lane);
+    rb.init(wn * TN, lane);
     const unsigned smem0 = lds_addr(smem);
     barrier();
-    if (kg == 1) barrier();
+    if (late) barrier();
     int slot = 0;
     for (int st = 0; st < nst; ++st) {
         const unsigned sa = smem0 + slot * STAGE_B, sb = sa + FA::REGION_B;
         typename RA::Set a;
         typename RB::Set b;
-        static_for<KSW>([&](auto jc) {
+        static_for<STEPS>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
             static_for<TM>([&](auto ic) { ra.template request<j, decltype(ic)::value>(sa, a); });
             static_for<TN>([&](auto ic) { rb.template request<j, decltype(ic)::value>(sb, b); });
         });
         __builtin_amdgcn_sched_barrier(0);
         lds_wait_n<0>();
-        static_for<KSW>([&](auto jc) {
+        static_for<STEPS>([&](auto jc) {
             RA::arrived(a, decltype(jc)::value);
             RB::arrived(b, decltype(jc)::value);
         });
         barrier();
-        static_for<KSW>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
+#pragma unroll
+        for (int j = 0; j < STEPS; ++j)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int n = 0; n < TN; ++n)
-                    acc[i][n] = mfma32(RB::get(b, n, j), RA::get(a, i, j), acc[i][n]);   // (lanes: rows of C)
-        });
+                for (int n = 0; n < TN; ++n) acc[i][n] = prod_mfma(RB::get(b, n, j), RA::get(a, i, j), acc[i][n]);   // (lanes: rows of C)
         barrier();
         slot = slot + 1 == NST ? 0 : slot + 1;
     }
-    if (kg == 0) barrier();
+    if (!late) barrier();
     __syncthreads();
-    // The second k-group's sums go to the first through LDS (16 bytes per lane and register quad), then the tile leaves as whole rows.
-    f32x4* xch = reinterpret_cast<f32x4*>(smem) + (wave & 3) * (TM * TN * 4 * 64) + lane;
-    if (kg == 1) {
+    // the tile leaves as whole rows, by way of LDS: rows of BN * 2 bytes, 16-byte chunk c of row r at c ^ (r % 8)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int n = 0; n < TN; ++n)
+        for (int n = 0; n < TN; ++n)
 #pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    f32x4 v;
+            for (int a = 0; a < QUADS; ++a) {
+                bf16x4 v;
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = acc[i][n][4 * a + x];
-                    xch[((i * TN + n) * 4 + a) * 64] = v;
-                }
-    }
-    __syncthreads();
-    // rows of BN * 2 bytes, 16-byte chunk c of row r at c ^ (r % 8)
-    unsigned char* out = smem + BM * BN * 4;
-    if (kg == 0) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int n = 0; n < TN; ++n)
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const f32x4 other = xch[((i * TN + n) * 4 + a) * 64];
-                    bf16x4 v;
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = (bf16_t)(acc[i][n][4 * a + x] + other[x]);
-                    const int r = (wm * TM + i) * 32 + l32, c = (wn * TN + n) * 4 + a;
-                    *reinterpret_cast<bf16x4*>(out + r * (BN * 2) + ((c ^ (r & 7)) << 4) + 8 * g) = v;
-                }
-    }
+                for (int x = 0; x < 4; ++x) v[x] = (bf16_t)acc[i][n][4 * a + x];
+                const int r = (wm * TM + i) * TH + lane % TH, col = (wn * TN + n) * TH + (TH == 32 ? 8 * a : 0) + 4 * (lane / TH);
+                *reinterpret_cast<bf16x4*>(smem + r * (BN * 2) + (((col >> 3) ^ (r & 7)) << 4) + (col & 4) * 2) = v;
+            }
     __syncthreads();
     constexpr int CH = BN / 8;
 #pragma unroll
-    for (int k = 0; k < BM * CH / 512; ++k) {
-        const int id = k * 512 + threadIdx.x, r = id / CH, c = id % CH;
+    for (int id = threadIdx.x; id < BM * CH; id += 512) {
+        const int r = id / CH, c = id % CH;
         if (m0 + r < p.M && n0 + 8 * c < p.N)
             *reinterpret_cast<u32x4*>(p.C + (long)(m0 + r) * p.N + n0 + 8 * c) =
-                *reinterpret_cast<const u32x4*>(out + r * (BN * 2) + ((c ^ (r & 7)) << 4));
+                *reinterpret_cast<const u32x4*>(smem + r * (BN * 2) + ((c ^ (r & 7)) << 4));
     }
 }
 
 // NT with few tiles: 32 TM x 32 TN of C per workgroup.  Its eight waves take every eighth chunk of 64 of the summed index each, through
 // LDS of their own (Q chunks in flight, no barrier before the end), and their sums are added at the end, in the waves' order.
-// (512 x 1,024 x 1,024: 5.0 us with 64 x 32 against 6.4 with the tiles of 64 above; 64 x 64 this way 6.7.)
+// (512 x 1,024 x 1,024: 5.1 us with 64 x 32 against 6.0 with 32 x 64 above; 64 x 64 this way 6.7.)
 template <int TM, int TN, int Q>
 __global__ __launch_bounds__(512) void mhffn_product_split_kernel(ProductArgs p)
 {
     constexpr int BM = 32 * TM, BN = 32 * TN;
     using FA = ProductFill<false, BM, 1, 1>;
     using FB = ProductFill<false, BN, 1, 1>;
-    using RA = ProductRead<false, BM, 1, TM, 1>;
-    using RB = ProductRead<false, BN, 1, TN, 1>;
+    using RA = ProductRead<false, BM, 1, 32, TM>;
+    using RB = ProductRead<false, BN, 1, 32, TN>;
     constexpr int FILLS = FA::COUNT + FB::COUNT, CHUNK_B = FA::REGION_B + FB::REGION_B;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
@@ -369,8 +356,8 @@ __global__ __launch_bounds__(512) void mhffn_product_split_kernel(ProductArgs p)
         if (wave + 8 * q < chunks) fill(wave + 8 * q, q);
     RA ra;
     RB rb;
-    ra.init(0, 0, lane);
-    rb.init(0, 0, lane);
+    ra.init(0, lane);
+    rb.init(0, lane);
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -435,13 +422,13 @@ __global__ __launch_bounds__(512) void mhffn_product_split_kernel(ProductArgs p)
     }
 }
 
-template <bool ACOLS, bool BCOLS, int BM, int BN, int KU, int NST>
+template <bool ACOLS, bool BCOLS, int BM, int BN, int TH, int WM, int KU, int NST>
 static hipError_t launch_tiles(ProductArgs a, hipStream_t st)
 {
-    constexpr int ring = (BM + BN) * KU * 128 * NST, tail = BM * BN * 6, smem = ring > tail ? ring : tail;
-    static_assert(smem <= 160 * 1024, "LDS of a compute unit");
+    constexpr int smem = (BM + BN) * KU * 128 * NST;      // (holds the tile of C, too)
+    static_assert(BM * BN * 2 <= smem && smem <= 160 * 1024, "LDS of a compute unit");
     static LdsOptIn optin;
-    auto* fn = mhffn_product_kernel<ACOLS, BCOLS, BM, BN, KU, NST>;
+    auto* fn = mhffn_product_kernel<ACOLS, BCOLS, BM, BN, TH, WM, KU, NST>;
     const hipError_t e = ensure_dynamic_lds(optin, (const void*)fn, smem);
     if (e != hipSuccess) return e;
     a.mtiles = (a.M + BM - 1) / BM;
@@ -471,13 +458,14 @@ struct ProductVariant {
     int bm, bn;
     double base, step, full, again;
 };
-constexpr ProductVariant PRODUCT_VARIANTS[] = {{64, 64, 3.2, 0.19, 0.1, 2.4},  {128, 64, 3.6, 0.28, 0.15, 2.5}, {128, 128, 4.0, 0.38, 0.45, 3.0},
-                                               {32, 32, 2.4, 0.08, 0.2, 1.3},  {64, 32, 3.0, 0.115, 0.1, 1.6}};     // (the last two: NT)
-static int product_variant(int form, int M, int N, int K)
+constexpr ProductVariant PRODUCT_VARIANTS[] = {{64, 64, 3.2, 0.23, 0.0, 2.8}, {128, 64, 3.4, 0.285, 0.12, 2.9}, {128, 128, 3.6, 0.4, 0.3, 1.0},
+                                               {32, 64, 2.8, 0.18, 0.1, 1.6},                                       // NT in order
+                                               {32, 32, 2.4, 0.08, 0.2, 1.3}, {64, 32, 3.0, 0.115, 0.1, 1.6}};      // NT in any order
+static int product_variant(int form, bool in_order, int M, int N, int K)
 {
     int best = 0;
     double best_us = 0;
-    for (int v = 0; v < (form == PRODUCT_NT ? 5 : 3); ++v) {
+    for (int v = 0; v < (form != PRODUCT_NT ? 3 : in_order ? 4 : 6); ++v) {
         const ProductVariant& p = PRODUCT_VARIANTS[v];
         const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), rounds = (tiles + CUS - 1) / CUS;
         const double load = tiles <= CUS / 2 ? 0 : tiles >= CUS ? 1 : (tiles - CUS / 2) / (double)(CUS / 2);
@@ -486,33 +474,38 @@ static int product_variant(int form, int M, int N, int K)
     }
     return best;
 }
-int product_tile(int form, int M, int N, int K)
+int product_tile(int form, bool in_order, int M, int N, int K)
 {
-    const ProductVariant& p = PRODUCT_VARIANTS[product_variant(form, M, N, K)];
+    const ProductVariant& p = PRODUCT_VARIANTS[product_variant(form, in_order, M, N, K)];
     return 65536 * p.bm + p.bn;
 }
 // One round of the largest tiles: there these kernels are as fast as the library's or faster (NT of 3,000 x 1,024 x 1,024 11.3 us
-// against 11.4, of 2,048^3 21.6 against 22.6; TN of the latter 22.3 against 26.6); with more its larger tiles win in NT and NN
-// (8,192 x 1,024 x 1,024: 25.0 against 21.9).
+// against 11.7, of 2,048^3 20.3 against 20.4; TN of the latter 21.2 against 25.3); with more its larger tiles win in NT and NN
+// (8,192 x 1,024 x 1,024: 25 against 22).
 bool product_preferred(int M, int N) { return (long)((M + 127) / 128) * ((N + 127) / 128) <= CUS; }
 
 template <bool ACOLS, bool BCOLS>
 static hipError_t launch_form(const ProductArgs& a, int variant, hipStream_t st)
 {
     switch (variant) {
-        case 0: return launch_tiles<ACOLS, BCOLS, 64, 64, 2, 4>(a, st);
-        case 1: return launch_tiles<ACOLS, BCOLS, 128, 64, 2, 3>(a, st);
-        case 2: return launch_tiles<ACOLS, BCOLS, 128, 128, 1, 4>(a, st);
+        case 0: return launch_tiles<ACOLS, BCOLS, 64, 64, 16, 4, 2, 4>(a, st);
+        case 1: return launch_tiles<ACOLS, BCOLS, 128, 64, 32, 4, 2, 3>(a, st);
+        case 2: return launch_tiles<ACOLS, BCOLS, 128, 128, 32, 4, 1, 4>(a, st);
+    }
+    if constexpr (!ACOLS && !BCOLS) switch (variant) {
+        case 3: return launch_tiles<ACOLS, BCOLS, 32, 64, 16, 2, 2, 4>(a, st);
+        case 4: return launch_split<1, 1, 2>(a, st);
+        case 5: return launch_split<2, 1, 1>(a, st);
     }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_product(int form, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st)
+hipError_t launch_product(int form, bool in_order, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st)
 {
     const ProductArgs a{(const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, M, N, K, 0, 0};
-    const int v = product_variant(form, M, N, K);
+    const int v = product_variant(form, in_order, M, N, K);
     switch (form) {
-        case PRODUCT_NT: return v == 3 ? launch_split<1, 1, 2>(a, st) : v == 4 ? launch_split<2, 1, 1>(a, st) : launch_form<false, false>(a, v, st);
+        case PRODUCT_NT: return launch_form<false, false>(a, v, st);
         case PRODUCT_NN: return launch_form<false, true>(a, v, st);
         case PRODUCT_TN: return launch_form<true, true>(a, v, st);
     }

@@ -5,8 +5,8 @@ namespace mhffn {
 
 // Products of bfloat16 matrices (mhffn_product.hip), forms as MHFFN_PRODUCT_* in include/mhffn.h; N and K (TN: M and N) multiples of 8.
 constexpr int PRODUCT_NT = 0, PRODUCT_NN = 1, PRODUCT_TN = 2;
-int product_tile(int form, int M, int N, int K);      // 65536 * rows + columns of the tiles that a launch runs in
+int product_tile(int form, bool in_order, int M, int N, int K);      // 65536 * rows + columns of the tiles that a launch runs in
 bool product_preferred(int M, int N);
-hipError_t launch_product(int form, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st);
+hipError_t launch_product(int form, bool in_order, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st);
 
 }  // namespace mhffn

@@ -323,75 +323,87 @@ bool plain(const Tensor& t)
 {
     return t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.is_cuda() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
+// Whose products: the library's, these kernels', or these kernels' where both take each element's sum in the order of the summed index
+// and so have the same bits (a model's layers amplify a different rounding, see MHFFNDecoder in mhffn_layer.py).  The library splits the
+// summed index for 16 rows and fewer, and in NN with more than 1,024 of it and no more than 2^18 results (found by comparing
+// bits: 2,370 products of hidden 768 and 1024, 1 to 2,048 rows).
+enum Whose { LIBRARY = 0, OWN = 1, OWN_IN_ORDER = 2 };
+bool library_in_order(int form, int64_t M, int64_t N, int64_t K)
+{
+    return (form == MHFFN_PRODUCT_TN ? K : M) > 16 && (form != MHFFN_PRODUCT_NN || K <= 1024 || M * N > (1 << 18));
+}
 // M x N with inner extent K into `out_sizes`, or an undefined tensor where the product is the library's: outside the kernels'
 // sizes, under a dispatch mode (which is to see the call), or where autograd is to record the call.
-Tensor own_product(int form, const Tensor& a, const Tensor& b, int64_t M, int64_t N, int64_t K, at::IntArrayRef out_sizes)
+Tensor own_product(int form, Whose whose, const Tensor& a, const Tensor& b, int64_t M, int64_t N, int64_t K, at::IntArrayRef out_sizes)
 {
+    if (whose == LIBRARY || (whose == OWN_IN_ORDER && !library_in_order(form, M, N, K))) return {};
     if (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) return {};
     if (!plain(a) || !plain(b) || a.device() != b.device() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return {};
-    if (std::max({M, N, K}) > INT_MAX || !mhffn_product_preferred((int)M, (int)N) || !mhffn_product_tile(form, (int)M, (int)N, (int)K)) return {};
+    if (std::max({M, N, K}) > INT_MAX || !mhffn_product_preferred((int)M, (int)N)) return {};
+    const int in_order = whose == OWN_IN_ORDER;
+    if (!mhffn_product_tile(form, in_order, (int)M, (int)N, (int)K)) return {};
     RECORD_FUNCTION("mhffn::product", std::vector<c10::IValue>());
     OnDevice on_device(a);
     Tensor c = empty_of(out_sizes, at::kBFloat16, a);
-    raise_for_code(mhffn_product(form, ptr(a), ptr(b), ptr(c), (int)M, (int)N, (int)K, stream()), "mhffn_product");
+    raise_for_code(mhffn_product(form, in_order, ptr(a), ptr(b), ptr(c), (int)M, (int)N, (int)K, stream()), "mhffn_product");
     return c;
 }
 // x w^T, x [.., in], w [out, in]
-Tensor project(const Tensor& x, const Tensor& w, bool own)
+Tensor project(const Tensor& x, const Tensor& w, Whose whose)
 {
-    if (own && x.dim() > 0 && w.dim() == 2 && x.size(-1) == w.size(1) && w.size(1) > 0) {
+    if (x.dim() > 0 && w.dim() == 2 && x.size(-1) == w.size(1) && w.size(1) > 0) {
         at::DimVector sizes(x.sizes());
         sizes.back() = w.size(0);
-        Tensor y = own_product(MHFFN_PRODUCT_NT, x, w, x.numel() / w.size(1), w.size(0), w.size(1), sizes);
+        Tensor y = own_product(MHFFN_PRODUCT_NT, whose, x, w, x.numel() / w.size(1), w.size(0), w.size(1), sizes);
         if (y.defined()) return y;
     }
     return at::linear(x, w);
 }
 // dy w and dy^T x of matrices
-Tensor product_nn(const Tensor& a, const Tensor& b, bool own = true)
+Tensor product_nn(const Tensor& a, const Tensor& b, Whose whose)
 {
-    Tensor c;
-    if (own) c = own_product(MHFFN_PRODUCT_NN, a, b, a.size(0), b.size(1), a.size(1), {a.size(0), b.size(1)});
+    Tensor c = own_product(MHFFN_PRODUCT_NN, whose, a, b, a.size(0), b.size(1), a.size(1), {a.size(0), b.size(1)});
     return c.defined() ? c : at::mm(a, b);
 }
-Tensor product_tn(const Tensor& a, const Tensor& b, bool own = true)
+Tensor product_tn(const Tensor& a, const Tensor& b, Whose whose)
 {
-    Tensor c;
-    if (own) c = own_product(MHFFN_PRODUCT_TN, a, b, a.size(1), b.size(1), a.size(0), {a.size(1), b.size(1)});
+    Tensor c = own_product(MHFFN_PRODUCT_TN, whose, a, b, a.size(1), b.size(1), a.size(0), {a.size(1), b.size(1)});
     return c.defined() ? c : at::mm(a.t(), b);
 }
 
-// A linear layer without bias.  (own: with the kernels above, see Projection in mhffn_layer.py)
+// A linear layer without bias (Projection in mhffn_layer.py).
 struct LinearNode : torch::autograd::Function<LinearNode> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w)
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, int64_t whose)
     {
+        ctx->saved_data["whose"] = whose;
         // (each gradient needs the other factor)
         ctx->save_for_backward({w.requires_grad() ? x : Tensor(), x.requires_grad() ? w : Tensor()});
-        return project(x, w, true);
+        return project(x, w, Whose(whose));
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
     {
         const auto s = ctx->get_saved_variables();
         const Tensor &x = s[0], &w = s[1];
+        const Whose whose = Whose(ctx->saved_data["whose"].toInt());
         const Tensor dy = g[0].reshape({-1, g[0].size(-1)});
         Tensor dx, dw;
         if (ctx->needs_input_grad(0)) {
             at::DimVector sizes(g[0].sizes());
             sizes.back() = w.size(1);
-            dx = product_nn(dy, w).view(sizes);
+            dx = product_nn(dy, w, whose).view(sizes);
         }
-        if (ctx->needs_input_grad(1)) dw = product_tn(dy, x.reshape({-1, x.size(-1)}));
-        return {dx, dw};
+        if (ctx->needs_input_grad(1)) dw = product_tn(dy, x.reshape({-1, x.size(-1)}), whose);
+        return {dx, dw, Tensor()};
     }
 };
-Tensor linear(const Tensor& x, const Tensor& w, bool own)
+Tensor linear(const Tensor& x, const Tensor& w, Whose whose)
 {
-    if (!own || !records_grad({&x, &w})) return project(x, w, own);
-    // (the library's node where its products would run both ways, and where a dispatch mode is to see them)
-    if (x.dim() == 0 || w.dim() != 2 || x.numel() == 0 || x.size(-1) != w.size(1) || !plain(x) || !plain(w) ||
+    if (!records_grad({&x, &w})) return project(x, w, whose);
+    // (torch's node where the products are the library's, and where a dispatch mode is to see them)
+    if (whose == LIBRARY || x.dim() == 0 || w.dim() != 2 || x.numel() == 0 || x.size(-1) != w.size(1) || !plain(x) || !plain(w) ||
         c10::impl::TorchDispatchModeTLS::any_modes_set())
         return at::linear(x, w);
-    return LinearNode::apply(x, w);
+    return LinearNode::apply(x, w, (int64_t)whose);
 }
 
 // ---- the whole block: w_self, prologue, operator, w_self_2 ---------------------------------------------------------
@@ -400,20 +412,20 @@ struct BlockForward {
     Tensor O4, Y;      // operator output [B,S,H,d_h], block output
 };
 BlockForward block_forward(const Tensor& x, const Tensor& w1, const Tensor& norm_weight, const Tensor& router, const Tensor& K,
-                           const Tensor& U, const Tensor& V, const Tensor& w2, double eps, bool one_part, bool own)
+                           const Tensor& U, const Tensor& V, const Tensor& w2, double eps, bool one_part, Whose whose)
 {
     BlockForward f;
     const int64_t B = x.size(0), S = x.size(1), hid = x.size(2);
-    f.g = gate_forward(project(x, w1, own).view({B, S, router.size(0), router.size(1)}), norm_weight, router, eps);
+    f.g = gate_forward(project(x, w1, whose).view({B, S, router.size(0), router.size(1)}), norm_weight, router, eps);
     f.O4 = op_forward(f.g.q4.transpose(1, 2), K, U, V, f.g.R, one_part).transpose(1, 2);
-    f.Y = project(f.O4.view({B, S, hid}), w2, own);
+    f.Y = project(f.O4.view({B, S, hid}), w2, whose);
     return f;
 }
 
 Tensor stepwise_O4(const Tensor& x, const Tensor& w1, const Tensor& nw, const Tensor& router, const Tensor& K, const Tensor& U,
-                   const Tensor& V, double eps, bool one_part, bool own)
+                   const Tensor& V, double eps, bool one_part, Whose whose)
 {
-    auto [Q, R] = gate(linear(x, w1, own).view({x.size(0), x.size(1), router.size(0), router.size(1)}),
+    auto [Q, R] = gate(linear(x, w1, whose).view({x.size(0), x.size(1), router.size(0), router.size(1)}),
                        nw.defined() ? std::optional<Tensor>(nw) : std::nullopt, router, eps);
     return op(Q, K, U, V, R, one_part).transpose(1, 2);
 }
@@ -422,14 +434,15 @@ Tensor stepwise_O4(const Tensor& x, const Tensor& w1, const Tensor& nw, const Te
 struct BlockNode : torch::autograd::Function<BlockNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight,
                           const Tensor& router, const Tensor& K, const Tensor& U, const Tensor& V, const Tensor& w2, double eps,
-                          bool one_part, bool own)
+                          bool one_part, int64_t whose_)
     {
+        const Whose whose = Whose(whose_);
         const Tensor nw = norm_weight.value_or(Tensor());
-        BlockForward f = block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part, own);
+        BlockForward f = block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part, whose);
         ctx->save_for_backward({x, w1, nw, router, K, U, V, w2, f.g.x4, f.g.wn, f.g.wr, f.g.q4, f.g.R, f.O4});
         ctx->saved_data["eps"] = eps;
         ctx->saved_data["one_part"] = one_part;
-        ctx->saved_data["own"] = own;
+        ctx->saved_data["whose"] = whose_;
         return f.Y;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads)
@@ -438,7 +451,8 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor &x = s[0], &w1 = s[1], &nw = s[2], &router = s[3], &K = s[4], &U = s[5], &V = s[6], &w2 = s[7], &x4 = s[8],
                      &wn = s[9], &wr = s[10], &q4 = s[11], &R = s[12];
         const double eps = ctx->saved_data["eps"].toDouble();
-        const bool one_part = ctx->saved_data["one_part"].toBool(), own = ctx->saved_data["own"].toBool();
+        const bool one_part = ctx->saved_data["one_part"].toBool();
+        const Whose whose = Whose(ctx->saved_data["whose"].toInt());
         const int64_t hid = x.size(2);
         // What this pass asks for (torch.autograd.grad may name a few inputs): a step whose results nobody asked for is left
         // out, as the engine leaves out a node of its own.  The numbers count the tensors that went in: x, w1, nw if there is
@@ -457,34 +471,35 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         if (asked(after_nw + 4, after_nw + 5)) {
             Tensor O4 = s[13];
             if (at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
-                O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, own);
-            dw2 = product_tn(dY, O4.reshape({-1, hid}), own);
+                O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose);
+            dw2 = product_tn(dY, O4.reshape({-1, hid}), whose);
         }
         if (prologue || experts) {
-            const Tensor dO = product_nn(dY, w2, own).view(s[13].sizes());
+            const Tensor dO = product_nn(dY, w2, whose).view(s[13].sizes());
             g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type(), one_part);
         }
         if (prologue) {
             h = gate_backward(x4, nw, router, wn, wr, eps, g[0], g[4]);
             const Tensor dp = h[0].view({-1, hid});
-            if (ctx->needs_input_grad(0)) dx = product_nn(dp, w1, own).view(x.sizes());
-            if (ctx->needs_input_grad(1)) dw1 = product_tn(dp, x.reshape({-1, hid}), own);
+            if (ctx->needs_input_grad(0)) dx = product_nn(dp, w1, whose).view(x.sizes());
+            if (ctx->needs_input_grad(1)) dw1 = product_tn(dp, x.reshape({-1, hid}), whose);
         }
         return {dx, dw1, h[1], h[2], g[1], g[2], g[3], dw2, Tensor(), Tensor(), Tensor()};
     }
 };
 Tensor block(const Tensor& x, const Tensor& w1, const std::optional<Tensor>& norm_weight, const Tensor& router, const Tensor& K,
-             const Tensor& U, const Tensor& V, const Tensor& w2, double eps, bool one_part, bool own)
+             const Tensor& U, const Tensor& V, const Tensor& w2, double eps, bool one_part, int64_t whose_)
 {
+    const Whose whose = Whose(whose_);
     const Tensor nw = norm_weight.value_or(Tensor());
     if (!records_grad({&x, &w1, &nw, &router, &K, &U, &V, &w2}))
-        return block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part, own).Y;
+        return block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part, whose).Y;
     // With anything frozen (adapters, training of the experts alone) the steps record their own nodes: each saves what its
     // own gradients need, and what nobody asks for is neither kept nor computed.
     for (const Tensor* t : {&x, &w1, &nw, &router, &K, &U, &V, &w2})
         if (t->defined() && !t->requires_grad())
-            return linear(stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, own).reshape(x.sizes()), w2, own);
-    return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps, one_part, own);
+            return linear(stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose).reshape(x.sizes()), w2, whose);
+    return BlockNode::apply(x, w1, norm_weight, router, K, U, V, w2, eps, one_part, whose_);
 }
 
 // ---- the decoder's rotary positions --------------------------------------------------------------------------------
@@ -599,7 +614,7 @@ PYBIND11_MODULE(_native, m)
                                                                    dQ.value_or(Tensor()), dR.value_or(Tensor()));
                                    return std::make_tuple(g[0], g[1].defined() ? std::optional<Tensor>(g[1]) : std::nullopt, g[2]);
                                }));
-    m.def("linear", torch::wrap_pybind_function_no_gil([](const Tensor& x, const Tensor& w) { return linear(x, w, true); }));
+    m.def("linear", torch::wrap_pybind_function_no_gil([](const Tensor& x, const Tensor& w, int64_t whose) { return linear(x, w, Whose(whose)); }));
     m.def("rope", torch::wrap_pybind_function_no_gil(rope));
     m.def("block", torch::wrap_pybind_function_no_gil(block));
 }

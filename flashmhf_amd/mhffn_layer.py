@@ -68,14 +68,20 @@ def router_gate(logits):
 class Projection(nn.Linear):
     """nn.Linear whose products, forward and backward, run in the framework's kernels where these are faster than the library's
     (csrc/mhffn_product.hip): bfloat16 on the GPU, without bias, called as the plain layer; else nn.Linear's own forward."""
+    products = 1        # `Whose` in csrc/mhffn_torch.cpp
 
     def forward(self, x):
         w = self.weight
         if (x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and self.bias is None and nn.Linear.forward is _FORWARD[nn.Linear]
                 and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling() and _capi.native_nodes()
                 and not torch.overrides.has_torch_function((x, w))):
-            return _capi.native().linear(x, w)
+            return _capi.native().linear(x, w, self.products)
         return super().forward(x)
+
+
+class OrderedProjection(Projection):
+    """... where they also have the library's bits: both take every sum in the order of its terms."""
+    products = 2
 
 
 def _unhooked(m):
@@ -90,7 +96,8 @@ def _runs_own_forward(m, cls):
 
 def _plain_linear(m):
     """A Projection, or the nn.Linear that a program or a saved module has in its place, which keeps the library's products."""
-    return _runs_own_forward(m, Projection if type(m) is Projection else nn.Linear) and nn.Linear.forward is _FORWARD[nn.Linear]
+    cls = type(m)
+    return cls in _LINEAR and _runs_own_forward(m, cls) and nn.Linear.forward is _FORWARD[nn.Linear]
 
 
 def _global_hooks():
@@ -206,15 +213,17 @@ class MHFFNLayer(nn.Module):
         weights = self._one_node(x)
         if weights is not None:
             m = self._modules
-            own = type(m["w_self"]) is type(m["w_self_2"]) is Projection
-            return _capi.native().block(x, *weights, self.rms_norm_eps, m["op"].one_part, own)
+            cls = type(m["w_self"])
+            products = cls.products if cls is type(m["w_self_2"]) and cls is not nn.Linear else 0
+            return _capi.native().block(x, *weights, self.rms_norm_eps, m["op"].one_part, products)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
 
 
 # what _stock_steps compares with: the code as it is defined here
-_FORWARD = {c: c.forward for c in (nn.Linear, Projection, RMSNorm, FlashMLPMoE)}
+_LINEAR = (nn.Linear, Projection, OrderedProjection)
+_FORWARD = {c: c.forward for c in (*_LINEAR, RMSNorm, FlashMLPMoE)}
 _HEADS_AND_GATE = MHFFNLayer.heads_and_gate
 
 
@@ -236,8 +245,8 @@ class CausalSelfAttention(nn.Module):
     def __init__(self, hidden_size, num_heads, rope_base=10000.0):
         super().__init__()
         self.num_heads, self.head_dim, self.rope_base = num_heads, hidden_size // num_heads, rope_base
-        self.qkv = nn.Linear(hidden_size, 3 * hidden_size, bias=False)
-        self.out = nn.Linear(hidden_size, hidden_size, bias=False)
+        self.qkv = OrderedProjection(hidden_size, 3 * hidden_size, bias=False)
+        self.out = OrderedProjection(hidden_size, hidden_size, bias=False)
 
     def forward(self, x, rope=None):
         B, S, hid = x.shape
@@ -276,15 +285,15 @@ class MHFFNDecoder(nn.Module):
         # depend on the rest of its batch.  (Rounding differences of the operator grow from block to block: another order
         # moves the gradients of a four-block model by 1 % of their norm.)
         layer_kw.setdefault("op", FlashMLPMoE(one_part=True))
-        # The library's products in the blocks as in the attention and the output head, for the same reason: sums taken another
-        # way (Projection) move single gradients of a four-block model by half of their root mean square.
-        layer_kw.setdefault("linear", nn.Linear)
+        # Products in one order of summation, too, the library's: in another (Projection) single gradients of a four-block model
+        # move by half of their root mean square.
+        layer_kw.setdefault("linear", OrderedProjection)
         self.embed = nn.Embedding(vocab_size, hidden_size)
         self.blocks = nn.ModuleList(
             MHFFNDecoderBlock(hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps, **layer_kw)
             for _ in range(num_layers))
         self.norm = RMSNorm((hidden_size,), eps)
-        self.lm_head = nn.Linear(hidden_size, vocab_size, bias=False)
+        self.lm_head = OrderedProjection(hidden_size, vocab_size, bias=False)
         nn.init.normal_(self.embed.weight, std=0.02)
         for m in self.modules():
             if isinstance(m, nn.Linear):

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 NT, NN, TN = _capi.PRODUCT_NT, _capi.PRODUCT_NN, _capi.PRODUCT_TN
 
 
-def _case(form, M, N, K, seed=0):
+def _case(form, M, N, K, in_order, seed=0):
     dev = "cuda:0"
     g = torch.Generator(device=dev).manual_seed(seed)
     shapes = {NT: ((M, K), (N, K)), NN: ((M, K), (K, N)), TN: ((K, M), (K, N))}[form]
@@ -18,7 +18,7 @@ def _case(form, M, N, K, seed=0):
     # (behind the result and the operands lies what must not be touched or read)
     out = torch.full((M * N + 64,), 7.0, device=dev, dtype=torch.bfloat16)
     pad = [torch.cat([t.reshape(-1), torch.full((64,), float("nan"), device=dev, dtype=torch.bfloat16)]) for t in (a, b)]
-    rc = _capi.lib().mhffn_product(form, pad[0].data_ptr(), pad[1].data_ptr(), out.data_ptr(), M, N, K,
+    rc = _capi.lib().mhffn_product(form, in_order, pad[0].data_ptr(), pad[1].data_ptr(), out.data_ptr(), M, N, K,
                                    torch.cuda.current_stream().cuda_stream)
     assert rc == _capi.OK
     assert (out[M * N:] == 7.0).all()
@@ -36,26 +36,47 @@ SIZES = [(8, 8), (24, 40), (72, 96), (136, 128), (264, 192), (496, 1000), (1000,
 
 
 # rows x columns of every tile, with edges inside a tile, one and several rounds of workgroups
-@pytest.mark.parametrize("form", [NT, NN, TN])
+@pytest.mark.parametrize("form,in_order", [(NT, 0), (NT, 1), (NN, 0), (TN, 0)])
 @pytest.mark.parametrize("M,N", SIZES)
 # one chunk of 64 and less, the stages' edges, fewer chunks than waves, more stages than the ring holds
 @pytest.mark.parametrize("K", [8, 64, 72, 136, 512, 1096])
-def test_products(form, M, N, K):
-    print(f"form {form} M={M} N={N} K={K}", flush=True)
-    _case(form, M, N, K, seed=M + N + K)
+def test_products(form, in_order, M, N, K):
+    print(f"form {form} M={M} N={N} K={K} in_order={in_order}", flush=True)
+    _case(form, M, N, K, in_order, seed=M + N + K)
 
 
 @pytest.mark.parametrize("form,M,N,K", [(NT, 1, 768, 768), (NT, 17, 2048, 2048), (NT, 733, 768, 768), (NN, 1, 64, 64), (NN, 37, 96, 96),
                                         (TN, 64, 64, 1), (TN, 96, 96, 37), (TN, 768, 768, 1025)])
 def test_products_of_odd_token_counts(form, M, N, K):
-    _case(form, M, N, K, seed=K)
+    for in_order in (0, 1):
+        _case(form, M, N, K, in_order, seed=K)
 
 
 def test_every_tile_is_one_of_the_cases():
-    tiles = {form: {divmod(_capi.lib().mhffn_product_tile(form, M, N, 512), 65536) for M, N in SIZES} for form in (NT, NN, TN)}
+    tile = _capi.lib().mhffn_product_tile
+    tiles = {(form, o): {divmod(tile(form, o, M, N, 512), 65536) for M, N in SIZES} for form in (NT, NN, TN) for o in (0, 1)}
     large = {(64, 64), (128, 64), (128, 128)}
-    assert tiles == {NT: large | {(32, 32), (64, 32)}, NN: large, TN: large}
-    assert not _capi.lib().mhffn_product_tile(NT, 8, 8, 12) and not _capi.lib().mhffn_product_tile(TN, 12, 8, 8)
+    assert tiles == {(NT, 0): large | {(32, 32), (64, 32)}, (NT, 1): large | {(32, 64)}, **{(f, o): large for f in (NN, TN) for o in (0, 1)}}
+    assert not tile(NT, 0, 8, 8, 12) and not tile(TN, 0, 12, 8, 8)
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 192, 192), (64, 1024, 1024), (300, 768, 768), (512, 3072, 1024), (1000, 1024, 1024), (2048, 768, 768)])
+def test_sums_in_order_have_the_library_s_bits(M, N, K):
+    """OrderedProjection, values and gradients, against nn.Linear."""
+    from flashmhf_amd.mhffn_layer import OrderedProjection
+    dev = "cuda:0"
+    torch.manual_seed(M)
+    own = OrderedProjection(K, N, bias=False, device=dev, dtype=torch.bfloat16)
+    lib = torch.nn.Linear(K, N, bias=False, device=dev, dtype=torch.bfloat16)
+    lib.load_state_dict(own.state_dict())
+    x, dy = torch.randn(M, K, device=dev).bfloat16(), torch.randn(M, N, device=dev).bfloat16()
+    results = []
+    for m in (own, lib):
+        xi = x.clone().requires_grad_(True)
+        y = m(xi)
+        results.append((y, *torch.autograd.grad(y, [xi, m.weight], dy)))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("T", [1, 16, 300, 2048])
