@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -17,3 +18,11 @@ def scalar_oracle():
     from oracle import scalar
     scalar.build()
     return scalar
+
+
+@pytest.fixture(autouse=True)
+def _no_garbage_of_earlier_tests(request):
+    """Tests that compare the allocator's counters around a call begin without reference cycles of earlier tests, whose tensors the
+    collector may free in between."""
+    if "no_alloc" in request.node.nodeid:
+        gc.collect()
