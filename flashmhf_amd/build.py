@@ -6,8 +6,10 @@ One code object, one architecture; no CUDA headers, no torch headers, links only
 operators' host side on top of that C ABI (g++, torch's headers).
 """
 import os
+import re
 import subprocess
 import sys
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -15,6 +17,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(LIBDIR, "libmhffn_hip.so")
 SOURCES = ["mhffn_capi.hip", "mhffn_fwd.hip", "mhffn_bwd.hip", "mhffn_f32.hip", "mhffn_gate.hip", "mhffn_rope.hip", "mhffn_product.hip"]
+# those that read LDS from inline assembly and wait by count (reads_touched_in_flight)
+ASYNC_READ_SOURCES = ["mhffn_bwd.hip", "mhffn_fwd.hip", "mhffn_product.hip"]
 # the torch side: an extension module on top of the C ABI, plain C++
 NATIVE_LIB = os.path.join(LIBDIR, "_native.so")
 NATIVE_SOURCE = "mhffn_torch.cpp"
@@ -29,13 +33,13 @@ FLAGS = [
 ]
 
 
-def build_lib(verbose=False, jobs=4):
+def build_lib(verbose=False, jobs=8):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(LIBDIR, exist_ok=True)
     objdir = os.path.join(LIBDIR, "obj")
     os.makedirs(objdir, exist_ok=True)
 
-    usage = {}
+    usage, touched = {}, {}
 
     def compile_one(src):
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
@@ -53,11 +57,25 @@ def build_lib(verbose=False, jobs=4):
         usage.update(parse_resource_usage(r.stderr))
         return obj
 
+    def check_assembly(src):
+        with tempfile.TemporaryDirectory() as tmp:
+            out = os.path.join(tmp, "kernels.s")
+            subprocess.check_call([hipcc, *FLAGS, "--offload-device-only", "-S", os.path.join(CSRC, src), "-o", out],
+                                  stderr=subprocess.DEVNULL)
+            with open(out) as f:
+                lines = f.readlines()
+        if not any("ds_read" in line for line in lines):
+            raise RuntimeError(f"no LDS reads found in the assembly of {src}")
+        touched.update(reads_touched_in_flight(lines))
+
     native_obj = os.path.join(objdir, NATIVE_SOURCE.replace(".cpp", ".o"))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         native = ex.submit(subprocess.check_call, native_compile(native_obj))
+        checks = [ex.submit(check_assembly, src) for src in ASYNC_READ_SOURCES]
         objs = list(ex.map(compile_one, SOURCES + [PROBE_SOURCE]))
         native.result()
+        for check in checks:
+            check.result()
     for out, members in ((LIB, objs[:-1]), (PROBE_LIB, objs[-1:])):
         cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *members]
         if verbose:
@@ -69,6 +87,8 @@ def build_lib(verbose=False, jobs=4):
             f.write(name + "  " + "  ".join(f"{k}={v}" for k, v in usage[name].items()) + "\n")
     check_no_scratch(usage)
     check_variants(usage)
+    if touched:
+        raise RuntimeError(f"registers used before the LDS read that fills them has returned: {touched}")
     return LIB
 
 
@@ -93,7 +113,6 @@ def native_link(obj):
 
 def parse_resource_usage(stderr_text):
     """{kernel symbol: {field: value}} from hipcc's -Rpass-analysis=kernel-resource-usage remarks."""
-    import re
     usage, cur = {}, None
     for line in stderr_text.splitlines():
         m = re.search(r"remark:\s+Function Name: (\S+)", line)
@@ -142,6 +161,46 @@ def check_variants(usage):
         found = [n for n in usage if frag in n and "ScratchSize" in usage[n]]
         if len(found) != count or any(int(usage[n]["ScratchSize"]) for n in found):
             raise RuntimeError(f"expected {count} instantiations of {frag} without scratch memory, found {found}")
+
+
+def _registers(operand):
+    m = re.match(r"([va])(?:(\d+)|\[(\d+):(\d+)\])$", operand)
+    if not m:
+        return set()
+    lo, hi = (m[2], m[2]) if m[2] else (m[3], m[4])
+    return {(m[1], k) for k in range(int(lo), int(hi) + 1)}
+
+
+def reads_touched_in_flight(assembly):
+    """{kernel symbol: first such instruction} where an instruction uses a register that an LDS read in front of it (in the order of the
+    text) is still to fill.  LDS reads issued from inline assembly are waited for by count in inline assembly, too; between the two the
+    compiler may copy their registers, which it takes for filled: wrong values, depending on timing."""
+    found, kernel, in_flight = {}, None, []
+    for line in assembly:
+        m = re.match(r"(_Z\S+):", line)
+        if m:
+            kernel, in_flight = m[1], []
+        elif line.startswith(".Lfunc_end"):
+            kernel = None
+        code = line.split(";")[0].strip()
+        if kernel is None or not code or code.startswith(".") or code.endswith(":"):
+            continue
+        op, _, rest = code.partition(" ")
+        if op == "s_waitcnt":
+            m = re.search(r"lgkmcnt\((\d+)\)", rest)
+            if m:                                   # LDS operations return in order
+                in_flight = in_flight[max(0, len(in_flight) - int(m[1])):]
+            continue
+        if op in ("s_branch", "s_endpgm"):
+            in_flight = []
+            continue
+        operands = [t.strip().split(" ")[0] for t in rest.split(",")]
+        used = set().union(*(_registers(t) for t in operands))
+        if any(r & used for r in in_flight):
+            found.setdefault(kernel, code)
+        if op.startswith("ds_"):
+            in_flight.append(_registers(operands[0]) if op.startswith("ds_read") else set())
+    return found
 
 
 if __name__ == "__main__":

@@ -246,18 +246,13 @@ __device__ __forceinline__ u32x4 lds_read16_async(unsigned addr)
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(IMM));
     return v;
 }
-// N 4-byte values per lane, 128 bytes apart (one instruction, one LDS operation).
+// N 4-byte values per lane, 128 bytes apart (one instruction, one LDS operation); for N = 1 the same one twice, so that the read fills
+// both registers of the result: put together from a single one, the compiler copied that one before the read had returned.
 template <int N>
 __device__ __forceinline__ u32x2 lds_read_apart_async(unsigned addr)
 {
     u32x2 v;
-    if constexpr (N == 2) {
-        asm volatile("ds_read2_b32 %0, %1 offset1:32" : "=v"(v) : "v"(addr));
-    } else {
-        unsigned x;
-        asm volatile("ds_read_b32 %0, %1" : "=v"(x) : "v"(addr));
-        v = u32x2{x, 0u};
-    }
+    asm volatile("ds_read2_b32 %0, %1 offset1:%2" : "=v"(v) : "v"(addr), "n"(32 * (N - 1)));
     return v;
 }
 // At most N LDS operations of this wave still outstanding; the operands cannot be used above it.  Same conditions as

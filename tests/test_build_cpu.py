@@ -92,3 +92,24 @@ def test_no_variant_and_no_float32_kernel_spills(frag, count):
             build.check_variants({**usage, n: {**usage[n], "ScratchSize": "16"}})
         with pytest.raises(RuntimeError, match="scratch"):
             build.check_variants({k: v for k, v in usage.items() if k != n})
+
+
+READ = """_Z6kernelv:
+	ds_read_b32 v50, v50
+	ds_read_b128 v[54:57], v186 offset:0x2000
+	v_mov_b64_e32 v[60:61], v[62:63]
+{}	;;#ASMSTART
+	s_waitcnt lgkmcnt({})
+	;;#ASMEND
+	v_mov_b64_e32 v[52:53], v[50:51]
+	v_add_f32_e32 v1, v2, v3
+.Lfunc_end0:
+	v_mov_b32_e32 v1, v54
+"""
+
+
+@pytest.mark.parametrize("between,left,found", [("", 0, False), ("", 1, False), ("", 2, True), ("\tv_mov_b64_e32 v[52:53], v[50:51]\n", 0, True),
+                                                ("\tv_mov_b32_e32 v56, 0\n", 0, True), ("\ts_branch .LBB0_1\n", 2, False)])
+def test_registers_of_reads_in_flight_are_found(between, left, found):
+    got = build.reads_touched_in_flight(READ.format(between, left).splitlines())
+    assert bool(got) is found and (not found or list(got) == ["_Z6kernelv"])
