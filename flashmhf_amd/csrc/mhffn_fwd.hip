@@ -2,7 +2,8 @@
 //
 // One workgroup (4 waves, one per SIMD, 512 registers each) owns 256 rows of one K/U/V head (tokens of any batch and q-head
 // of its group: RowMap) and all the head's blocks or one part of them (pick_parts); a wave owns 64 rows (NT = 2 column tiles
-// of 32), "tokens" below.  With few rows the same code runs on 128 of them, one column tile per wave (FWD_VARIANTS).  The workgroup streams the K, U, V blocks (32 rows of the E*d_e axis at a time) straight
+// of 32), "tokens" below.  With few rows the same code runs on 128 of them, one column tile per wave, and four more waves do the
+// filling (FWD_VARIANTS, fwd_body).  The workgroup streams the K, U, V blocks (32 rows of the E*d_e axis at a time) straight
 // from the weight tensors into a ring of LDS stages with asynchronous LDS-direct loads.  Per block and wave:
 //     M^T = K Q^T, N^T = U Q^T               (A = rows of the K/U tiles, B = Q^T held in AGPRs for the whole kernel)
 //     P^T = silu(M^T) * N^T * r_e             (fp32 in the accumulator registers, rounded once to bf16)
@@ -55,7 +56,24 @@ __host__ __device__ constexpr int fwd_younger_reads(int ks, int KS, int CT)
     return n;
 }
 
-template <int DH, int NT>
+// One matrix instruction of the first products, Q^T in accumulation registers or (QV) in ordinary ones: with two waves per SIMD a wave
+// has 256 of both together, and the compiler would split them in half.
+template <bool QV, bool FIRST>
+__device__ __forceinline__ void first_product(f32x16& d, bf16x8 a, bf16x8 q)
+{
+    if constexpr (QV) {
+        if constexpr (FIRST) mfma32_vgpr_first(d, a, q);
+        else mfma32_vgpr_acc(d, a, q);
+    } else {
+        if constexpr (FIRST) mfma32_vgpr_first_bacc(d, a, q);
+        else mfma32_vgpr_acc_bacc(d, a, q);
+    }
+}
+
+// FILLERS: waves 4 to 7 do nothing but fill the ring, for waves 0 to 3.  A fill instruction holds its wave for 30 ns and more, six of
+// them a third of a step of one column tile: a block takes 0.53 us instead of 0.60 (d_h 96; 0.60 instead of 0.67 with 128), 733 tokens of the
+// 128M layer 19.5 us instead of 21.2.  With two column tiles a wave needs more than the 256 registers that two waves per SIMD leave it.
+template <int DH, int NT, bool FILLERS>
 __device__ __forceinline__ void fwd_body(const FwdArgs& p)
 {
     constexpr int KS = DH / 16, CT = DH / 32, NW = 4, WT = 32 * NT, BT = NW * WT;
@@ -87,13 +105,41 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
         const long roff = (long)bc * JB * DH;
 #pragma unroll
         for (int k = 0; k < FILL; ++k) {
-            const int id = wave + NW * k;
+            const int id = (wave & (NW - 1)) + NW * k;
             const int which = id >> 3;
             const long toff = which == 0 ? 0 : (which == 1 ? offU : offV);
             const int region = which == 0 ? FWD_K0 : (which == 1 ? FWD_U0 : FWD_V0);
             tile_fill_ins<DH>(Kh + toff + roff, DH, smem + region + stage * TILE_B, id & 7, lane);
         }
     };
+    if (FILLERS && wave >= NW) {
+        // One barrier of the workgroup for each of the others': behind the landing of blocks 0, and of b + 1 before step b.
+        auto barrier = [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        issue_block(0, 0);
+        issue_block(1, 1);
+        issue_block(2, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<2 * FILL>();
+        barrier();
+        const int window = GATE_WIN * nbe;
+        for (int b = 0; b < nblk; ++b) {
+            if (b > 0 && b % window == 0) {      // (the others restage the gate values)
+                barrier();
+                barrier();
+            }
+            wait_vmcnt<FILL>();
+            barrier();
+            issue_block(b + 3, (b + 3) % FWD_NST);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        wait_vmcnt<0>();
+        barrier();
+        return;
+    }
     const int first = tok0 < p.rows.n ? tok0 : p.rows.n - 1;
     const RowMap::Run run = p.rows.run(hk, first, WT);
     // The Q rows come from HBM and are the longest wait of the prologue: request them before anything else.
@@ -106,7 +152,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) q[ct][ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16);
     }
-    issue_block(0, 0);
+    if (!FILLERS) issue_block(0, 0);
     // Gate values of the workgroup's tokens, expert-major: one asynchronous 4-byte LDS-direct load per expert
     // and wave (lane = token, so the 64 values of an instruction are contiguous in LDS).  LDS holds a window of GATE_WIN
     // experts at a time; the first window is issued between block 0 and block 1, so that the wait for block 0 below
@@ -123,8 +169,10 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
             __builtin_amdgcn_global_load_lds((gptr_t)(rrow + e), (lptr_t)(sR + ((e - e0) * NW + wave) * 64), 4, 0, 0);
     };
     stage_gates(0);
-    issue_block(1, 1);
-    issue_block(2, 2);
+    if (!FILLERS) {
+        issue_block(1, 1);
+        issue_block(2, 2);
+    }
 
     f32x16 oacc[CT][NT];
 #pragma unroll
@@ -147,7 +195,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
     // consumes M/N of block blk (mc, nc), produces M/N of block blk+1 (mn, nn); ST = blk % FWD_NST
     auto step = [&](auto st_, int blk, int e, f32x16 (&mc)[NT], f32x16 (&nc)[NT], f32x16 (&mn)[NT], f32x16 (&nn)[NT]) {
         constexpr int ST = decltype(st_)::value, STN = (ST + 1) % FWD_NST;
-        wait_vmcnt<FILL>();   // blocks <= blk+1 have landed (only block blk+2's loads may be in flight)
+        if (!FILLERS) wait_vmcnt<FILL>();   // blocks <= blk+1 have landed (only block blk+2's loads may be in flight)
         __syncthreads();      // ... for every wave; and every wave is done with the stage about to be refilled
 
         // LDS reads of the step, all issued from inline assembly and waited for by count (the compiler's own waits are
@@ -174,7 +222,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
         // the fill of the stage that has just come free is issued behind the first reads: its address arithmetic and six
         // instructions pass while those reads are on their way
         __builtin_amdgcn_sched_barrier(0);
-        issue_block(blk + 3, (ST + 3) % FWD_NST);
+        if (!FILLERS) issue_block(blk + 3, (ST + 3) % FWD_NST);
         float rinv[NT];
         bf16x8 pt[NT][2];
         float e0 = 0, e1 = 0, xn0 = 0, xn1 = 0;   // carried between the chunks of one element pair
@@ -227,13 +275,8 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
                         lds_wait_n<fwd_younger_reads(ks, KS, CT)>();     // (consumed by asm matrix instructions only)
                     }
                 }
-                if constexpr ((w & 1) == 0) {
-                    if constexpr (ks == 0) mfma32_vgpr_first_bacc(mn[ct], __builtin_bit_cast(bf16x8, ak[0]), q[ct][0]);
-                    else mfma32_vgpr_acc_bacc(mn[ct], __builtin_bit_cast(bf16x8, ak[ks % 3]), q[ct][ks]);
-                } else {
-                    if constexpr (ks == 0) mfma32_vgpr_first_bacc(nn[ct], __builtin_bit_cast(bf16x8, au[0]), q[ct][0]);
-                    else mfma32_vgpr_acc_bacc(nn[ct], __builtin_bit_cast(bf16x8, au[ks % 3]), q[ct][ks]);
-                }
+                const bf16x8 a = __builtin_bit_cast(bf16x8, (w & 1) == 0 ? ak[ks % 3] : au[ks % 3]);
+                first_product<FILLERS, ks == 0>((w & 1) == 0 ? mn[ct] : nn[ct], a, q[ct][ks]);
             } else {
                 constexpr int g2 = k - NG1, s = g2 / (NT * CT), ct = (g2 / CT) % NT, i = g2 % CT;
                 if constexpr (g2 == 0) {
@@ -258,7 +301,8 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
     };
 
     f32x16 mA[NT], nA[NT], mB[NT], nB[NT];
-    wait_vmcnt<2 * FILL>();   // all but the fills of blocks 1 and 2: block 0 and the gate values have landed
+    if (FILLERS) wait_vmcnt<0>();
+    else wait_vmcnt<2 * FILL>();   // all but the fills of blocks 1 and 2: block 0 and the gate values have landed
     __syncthreads();
     {
 #pragma unroll
@@ -266,8 +310,8 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
             const bf16x8 a = tile_read_rows(smem + FWD_K0, krow, ks, g), u = tile_read_rows(smem + FWD_U0, krow, ks, g);
 #pragma unroll
             for (int ct = 0; ct < NT; ++ct) {
-                if (ks == 0) { mfma32_vgpr_first_bacc(mA[ct], a, q[ct][0]); mfma32_vgpr_first_bacc(nA[ct], u, q[ct][0]); }
-                else { mfma32_vgpr_acc_bacc(mA[ct], a, q[ct][ks]); mfma32_vgpr_acc_bacc(nA[ct], u, q[ct][ks]); }
+                if (ks == 0) { first_product<FILLERS, true>(mA[ct], a, q[ct][0]); first_product<FILLERS, true>(nA[ct], u, q[ct][0]); }
+                else { first_product<FILLERS, false>(mA[ct], a, q[ct][ks]); first_product<FILLERS, false>(nA[ct], u, q[ct][ks]); }
             }
         }
         // the element-wise code of step 0 reads these results
@@ -360,9 +404,9 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
 }
 
 template <int DH>
-__global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p) { fwd_body<DH, 2>(p); }
+__global__ __launch_bounds__(256) void mhffn_fwd_kernel(FwdArgs p) { fwd_body<DH, 2, false>(p); }
 template <int DH>
-__global__ __launch_bounds__(256) void mhffn_fwd_rows128_kernel(FwdArgs p) { fwd_body<DH, 1>(p); }
+__global__ __launch_bounds__(512) void mhffn_fwd_rows128_kernel(FwdArgs p) { fwd_body<DH, 1, true>(p); }
 
 // 32 rows, four blocks a trip: the same products, element-wise formula and order of sums as fwd_body.  One barrier a trip: P^T
 // operands and V tiles (which all waves read) have two sets, K and U tiles (which only their wave reads) are refilled as
@@ -515,10 +559,9 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
     *reinterpret_cast<bf16x4*>(p.O + p.rows.tok(hk, r) * DH + c) = v;
 }
 
-// Tiles of 256 rows (64 per wave) where they fill the chip; of 128 (32 per wave) below that: a step then takes 0.6 us
-// instead of 1.0, with 20 % less throughput once every compute unit has one (16,384 tokens of the 370M layer: 342 us with 256
-// rows, 407 with 128; 1,500 tokens in one part: 130 and 84; 733 tokens: 33 and 32 us at each one's best number of parts,
-// of the 128M layer 25.6 and 22.0).  Of 32, four blocks a trip of 1.43 us, below that, where 128-row tiles take, at each one's best
+// Tiles of 256 rows (64 per wave) where they fill the chip; of 128 (32 per wave) below that: a step then takes 0.53 to 0.6 us
+// instead of 1.0 (1,500 tokens of the 370M layer in one part: 130 us with 256 rows, 74 with 128; 733 tokens at each one's best number of
+// parts 32.6 and 29.8, of the 128M layer 25.2 and 20.6), and the two are level where every compute unit has one.  Of 32, four blocks a trip of 1.43 us, below that, where 128-row tiles take, at each one's best
 // number of parts: one token of the 370M layer 7.8 us against 10.0, 16 tokens of the 1.3B layer 20.3 against 22.5 (95 MB of
 // weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
@@ -542,7 +585,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, h
     if (e != hipSuccess) return e;
     dim3 grid((unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv), (unsigned)a.parts.nsplit);
     if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
-    else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(256), smem, st, a);
+    else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(512), smem, st, a);
     else hipLaunchKernelGGL((mhffn_fwd_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
         dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 4) + 255) / 256), (unsigned)d.Hkuv);
