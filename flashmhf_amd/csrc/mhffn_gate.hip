@@ -237,31 +237,32 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 }
 
 // ---- backward -------------------------------------------------------------------------------------------------------
-// LDS: router rows (hi, lo) | router columns | norm weight | per wave: y tile (8 KB) + dz tile (8 KB), both in the
-// swizzled 32 x 256-byte tile layout of the main kernels so the transposing reads can be shared | [waves][128] floats for
+// LDS: router rows (hi, lo) | router columns | norm weight | per wave: y tile (8 KB, the swizzled 32 x 256-byte layout of the
+// main kernels so the transposing reads can be shared) + dz tile (NT = 2: the same; NT = 1: 4 KB) | [waves][128] floats for
 // the sums across waves.  A wave takes enough consecutive tiles that the launch fills the chip once, which also bounds
 // the number of partial sums.
 //
-// Up to 32 experts (NT = 1) eight waves, two per SIMD, and nothing but sums in few registers lives across tiles: the waves'
-// y and dz tiles are contracted together, each wave keeping one column tile of d_router (16 registers) over the tokens
+// Up to 32 experts (NT = 1) eight waves, two per SIMD (with few tokens four: gate_bwd_waves), and nothing but sums in few
+// registers lives across tiles: the waves' y and dz tiles are contracted together, each wave keeping one column tile of d_router (16 registers) over the tokens
 // of several waves, two barriers per tile; the products d * u of d_norm_weight pass through the wave's LDS region a half at a
 // time and are added up down the columns (4 values per 64 columns).  What that frees holds the next tile's rows of x, requested
 // behind the contraction, while dR and dQ of a tile are requested at its top and used half a trip later.  One wave per SIMD
 // with all sums in registers, ~2,400 instructions per tile, a quarter of them register moves, took 150 us on 32,768 tokens of
-// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 128 us
-// (3.5 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
+// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 109 us
+// (4.1 TB/s; 128 us traced).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
 // More experts (NT = 2) have twice the d_router operands: four waves, one per SIMD, all sums in registers, and the next
 // tile's rows requested before the current tile's arithmetic starts.
+constexpr int GATE_Z_ROW_B = 64;                           // NT = 1: row of the dz tile
+constexpr int GATE_WAVE_REGION_B = 2 * TILE_B + 1024;      // NT = 2: also a 64 x 65 float transpose
 template <int NT>
-constexpr int gate_bwd_waves() { return NT == 1 ? 8 : 4; }
-constexpr int GATE_WAVE_REGION_B = 2 * TILE_B + 1024;      // NT = 2: also a 64 x 65 float transpose; NT = 1: 2 * TILE_B
+constexpr int gate_bwd_max_waves() { return NT == 1 ? 8 : 4; }
 template <int NT>
-constexpr int gate_bwd_region() { return NT == 1 ? 2 * TILE_B : GATE_WAVE_REGION_B; }
+constexpr int gate_bwd_region() { return NT == 1 ? TILE_B + 32 * 32 * 4 : GATE_WAVE_REGION_B; }      // (dR passes through the dz tile as fp32)
 template <int NT>
-constexpr size_t gate_bwd_smem(int DH)
+constexpr size_t gate_bwd_smem(int DH, int waves)
 {
     return (size_t)2 * NT * (DH / 16) * 1024 + (size_t)(DH / 32) * 2 * NT * 1024 + DH * 4 +
-           gate_bwd_waves<NT>() * (gate_bwd_region<NT>() + 128 * 4);
+           waves * (gate_bwd_region<NT>() + 128 * 4);
 }
 
 // Transposed operand (column tile ct, k-half s) of a swizzled tile.  Only column tile 0's two lane offsets are kept in
@@ -281,15 +282,34 @@ __device__ __forceinline__ bf16x8 tile_cols(const unsigned char* tile, const TrL
     return r;
 }
 
-template <int DH, int NT, bool NORM>
-__global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
+// The same of the dz tile of NT = 1: rows of 32 experts, chunk c of row r at c ^ (r / 4 % 4).
+__device__ __forceinline__ bf16x8 z_cols(const unsigned char* tile, int lane, int s)
 {
-    constexpr int KS = DH / 16, CT = DH / 32, NW = gate_bwd_waves<NT>(), REGION_B = gate_bwd_region<NT>();
+    typedef __attribute__((address_space(3))) v4bf16_t* lds_v4;
+    const int lam = lane & 15, l32 = lane & 31, g = lane >> 5, r = 8 * g + (lam >> 2), c = 2 * (l32 >> 4) + ((lam & 3) >> 1);
+    const int at = r * GATE_Z_ROW_B + ((c ^ (r >> 2 & 3)) << 4) + (lam & 1) * 8;
+    const v4bf16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4)(tile + at + 16 * GATE_Z_ROW_B * s));
+    const v4bf16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4)(tile + (at ^ 16) + (16 * s + 4) * GATE_Z_ROW_B));
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[j] = lo[j];
+        v[4 + j] = hi[j];
+    }
+    return v;
+}
+
+template <int DH, int NT, bool NORM>
+__global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
+{
+    const int NW = NT == 1 ? (int)blockDim.x / 64 : 4;
+    constexpr int KS = DH / 16, CT = DH / 32, REGION_B = gate_bwd_region<NT>();
     constexpr bool AHEAD = NT > 1;                              // rows requested one tile ahead; d_norm_weight in registers
     constexpr int NHALF = (DH + 63) / 64;
     // NT = 1: wave w sums column tile w % CT of d_router over the TPG token tiles of its group w / CT of the workgroup's
     // waves (waves beyond GROUPS * CT none); NT = 2: a wave sums all of it over its own tiles
-    constexpr int GROUPS = NW / CT, TPG = NW / GROUPS, WCT = AHEAD ? CT : 1;
+    constexpr int TPG = CT == 2 ? 2 : 4, WCT = AHEAD ? CT : 1;
+    const int GROUPS = NW / TPG;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* sA = smem;                                   // logits operands
     unsigned char* sC = sA + 2 * NT * KS * 1024;                // dy operands
@@ -369,6 +389,7 @@ __global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kern
         // latter (16 bytes of row lane / 16); the rest of an address is a constant that the swizzle's exclusive-or and the
         // row pitch leave alone.
         const int yrow = l32 * TILE_ROW_B + ((g ^ swz16(l32)) << 4), prow = l32 * TILE_ROW_B + (((2 * g) ^ (l32 & 15)) << 4);
+        const int zrow = AHEAD ? yrow : l32 * GATE_Z_ROW_B + ((g ^ (l32 >> 2 & 3)) << 4);
         const int pread = (lane >> 4) * TILE_ROW_B + (((lane & 15) ^ (lane >> 4)) << 4);
         // NT = 1: this tile's token contraction, two barriers around it (every wave of the workgroup passes them p.tpw times)
         auto contract = [&]() {
@@ -379,7 +400,7 @@ __global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kern
                     const unsigned char* yt = regions + (grp * TPG + k) * REGION_B;
 #pragma unroll
                     for (int s = 0; s < 2; ++s)
-                        wacc[0][0] = mfma32(tile_cols(yt, trl, ct, s), tile_cols(yt + TILE_B, trl, 0, s), wacc[0][0]);
+                        wacc[0][0] = mfma32(tile_cols(yt, trl, ct, s), z_cols(yt + TILE_B, lane, s), wacc[0][0]);
                 }
             }
             __syncthreads();
@@ -389,7 +410,7 @@ __global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kern
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<u32x4*>(ytile + (yrow ^ (ks << 5))) = zero;
 #pragma unroll
-            for (int s = 0; s < 2; ++s) *reinterpret_cast<u32x4*>(ztile + (yrow ^ (s << 5))) = zero;
+            for (int s = 0; s < 2; ++s) *reinterpret_cast<u32x4*>(ztile + (zrow ^ (s << 5))) = zero;
             contract();
             continue;
         }
@@ -457,7 +478,7 @@ __global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kern
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int s = 0; s < 2; ++s)
-                *reinterpret_cast<bf16x8*>(ztile + (yrow ^ ((4 * nt + 2 * s) << 4))) = dzb[nt][s];
+                *reinterpret_cast<bf16x8*>(ztile + (zrow ^ ((4 * nt + 2 * s) << 4))) = dzb[nt][s];
 
         // The phases of a tile are fenced, and each unpacks the rows of x anew: left to itself the compiler keeps the 64
         // unpacked values (and their products with rstd) from one phase to the next, which two waves per SIMD have no
@@ -524,10 +545,10 @@ __global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kern
                 du[ks][j] = d;
             }
             if constexpr (NORM && !AHEAD) {
-                // 64 columns of the products (chunk c of row r at c ^ (r % 16)) to each half of the region, whose y and dz
-                // tiles have been read, and down the columns
+                // 64 columns of the products at a time (chunk c of row r at c ^ (r % 16)) into the y tile, which has been
+                // read, and down the columns
                 constexpr int half = ks / 4, c0 = 4 * (ks % 4);
-                unsigned char* ptile = ytile + half * TILE_B;
+                unsigned char* ptile = ytile;
 #pragma unroll
                 for (int q = 0; q < 2; ++q) *reinterpret_cast<f32x4*>(ptile + (prow ^ ((c0 + q) << 4))) = prod[q];
                 if constexpr (ks % 4 == 3 || ks == KS - 1) {
@@ -572,76 +593,88 @@ __global__ __launch_bounds__(64 * gate_bwd_waves<NT>()) void mhffn_gate_bwd_kern
         if (part) part[col * p.E + e] = v;
         else unsafeAtomicAdd(dWr + (long)col * p.E + e, v);
     };
-    if constexpr (!AHEAD) {
-        float* sums = reinterpret_cast<float*>(regions);      // [GROUPS][CT][16][64]
-        if (wave < GROUPS * CT)
+    auto leave = [&](auto nw) {      // (for either number of waves: the loops over them are unrolled)
+        constexpr int NW = decltype(nw)::value;
+        [[maybe_unused]] constexpr int GROUPS = NW / TPG;
+        if constexpr (!AHEAD) {
+            if constexpr (GROUPS == 1) {      // (a wave's sums are those of the workgroup)
+                if (wave < CT)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sums[(wave * 16 + i) * 64 + lane] = wacc[0][0][i];
-        __syncthreads();
-        for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 64 * NW) {
-            float v = 0.0f;
+                    for (int i = 0; i < 16; ++i) put(0, (wave * 16 + i) * 64 + lane, wacc[0][0][i]);
+            } else {
+                float* sums = reinterpret_cast<float*>(regions);      // [GROUPS][CT][16][64]
+                if (wave < GROUPS * CT)
 #pragma unroll
-            for (int q = 0; q < GROUPS; ++q) v += sums[q * CT * 1024 + idx];
-            put(0, idx, v);
-        }
-        __syncthreads();
-    } else {
+                    for (int i = 0; i < 16; ++i) sums[(wave * 16 + i) * 64 + lane] = wacc[0][0][i];
+                __syncthreads();
+                for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 64 * NW) {
+                    float v = 0.0f;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-            for (int ct = 0; ct < WCT; ++ct)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) mine[(ct * 16 + i) * 64 + lane] = wacc[ct][nt][i];
-            __syncthreads();
-            for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 64 * NW) {
-                float v = 0.0f;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) v += reinterpret_cast<const float*>(regions + w * REGION_B)[idx];
-                put(nt, idx, v);
-            }
-            __syncthreads();
-        }
-    }
-    if constexpr (NORM) {
-        float* cross = reinterpret_cast<float*>(regions + NW * REGION_B);   // [NW waves][128 columns]
-        if constexpr (AHEAD) {
-            // transpose inside the wave: value v = 8 ks + j of every lane goes to row v (row stride 65 floats keeps both
-            // the writes and the row-wise reads conflict-free), then lane v adds up each lane half of its row
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) mine[(ks * 8 + j) * 65 + lane] = dwacc[ks][j];
-            if (lane < KS * 8) {
-                float s0 = 0.0f, s1 = 0.0f;
-                for (int i = 0; i < 32; ++i) {
-                    s0 += mine[lane * 65 + i];
-                    s1 += mine[lane * 65 + 32 + i];
+                    for (int q = 0; q < GROUPS; ++q) v += sums[q * CT * 1024 + idx];
+                    put(0, idx, v);
                 }
-                const int ks = lane >> 3, j = lane & 7;
-                cross[wave * 128 + (2 * ks) * 8 + j] = s0;
-                cross[wave * 128 + (2 * ks + 1) * 8 + j] = s1;
+                __syncthreads();
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < NHALF; ++i) {
+            for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    float v = dwcol[i][x];
-                    v += __shfl_xor(v, 16);
-                    v += __shfl_xor(v, 32);
-                    if (lane < 16 && 64 * i + 4 * lane < DH) cross[wave * 128 + 64 * i + 4 * lane + x] = v;
+                for (int ct = 0; ct < WCT; ++ct)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) mine[(ct * 16 + i) * 64 + lane] = wacc[ct][nt][i];
+                __syncthreads();
+                for (int idx = threadIdx.x; idx < CT * 16 * 64; idx += 64 * NW) {
+                    float v = 0.0f;
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) v += reinterpret_cast<const float*>(regions + w * REGION_B)[idx];
+                    put(nt, idx, v);
                 }
+                __syncthreads();
             }
         }
-        __syncthreads();
-        if (threadIdx.x < DH) {
-            float v = 0.0f;
+        if constexpr (NORM) {
+            float* cross = reinterpret_cast<float*>(regions + NW * REGION_B);   // [NW waves][128 columns]
+            if constexpr (AHEAD) {
+                // transpose inside the wave: value v = 8 ks + j of every lane goes to row v (row stride 65 floats keeps both
+                // the writes and the row-wise reads conflict-free), then lane v adds up each lane half of its row
 #pragma unroll
-            for (int w = 0; w < NW; ++w) v += cross[w * 128 + threadIdx.x];
-            if (part) part[DH * p.E + threadIdx.x] = v;
-            else unsafeAtomicAdd(p.dWn + h * DH + threadIdx.x, v);
+                for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) mine[(ks * 8 + j) * 65 + lane] = dwacc[ks][j];
+                if (lane < KS * 8) {
+                    float s0 = 0.0f, s1 = 0.0f;
+                    for (int i = 0; i < 32; ++i) {
+                        s0 += mine[lane * 65 + i];
+                        s1 += mine[lane * 65 + 32 + i];
+                    }
+                    const int ks = lane >> 3, j = lane & 7;
+                    cross[wave * 128 + (2 * ks) * 8 + j] = s0;
+                    cross[wave * 128 + (2 * ks + 1) * 8 + j] = s1;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NHALF; ++i) {
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        float v = dwcol[i][x];
+                        v += __shfl_xor(v, 16);
+                        v += __shfl_xor(v, 32);
+                        if (lane < 16 && 64 * i + 4 * lane < DH) cross[wave * 128 + 64 * i + 4 * lane + x] = v;
+                    }
+                }
+            }
+            __syncthreads();
+            if (threadIdx.x < DH) {
+                float v = 0.0f;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) v += cross[w * 128 + threadIdx.x];
+                if (part) part[DH * p.E + threadIdx.x] = v;
+                else unsafeAtomicAdd(p.dWn + h * DH + threadIdx.x, v);
+            }
         }
-    }
+    };
+    if (NT == 1 && NW == 8) leave(std::integral_constant<int, 8>{});
+    else leave(std::integral_constant<int, 4>{});
 }
 
 // Adds the workgroups' sums of a head (in order) and writes d_router and d_norm_weight in the parameters' types.
@@ -670,25 +703,29 @@ int tiles_per_wave(int B, int H, int S, int waves, long cap)
     const long tpw = total / waves;
     return (int)(tpw < 1 ? 1 : tpw > cap ? cap : tpw);
 }
-template <int NT>
-dim3 gate_bwd_grid(int B, int H, int S, int& tpw)
+// Waves of a backward workgroup.  Few tokens run with four also where up to 32 experts leave room for eight: with eight they fill
+// less than half the chip, and a workgroup's tiles share its barriers and its LDS.  The backward's two kernels, us, with eight and with
+// four waves: 16 tiles of 8 heads of 128 (11 experts) 16.3, 13.1; 64 tiles of 8 heads 17.2, 13.9; 20 tiles of 8 heads of 96 15.1, 12.6;
+// 63 of 16 heads of 128 (22 experts) 18.9, 16.6; one tile 12.1, 11.9.  With more the second set of partial sums costs more than it
+// gives: 122 tiles of 16 heads 21.3, 22.9.
+int gate_bwd_waves(const Dims& d) { return d.E > 32 || (long)d.B * d.H * ((d.S + 31) / 32) < 4 * CUS ? 4 : 8; }
+dim3 gate_bwd_grid(const Dims& d, int& tpw)
 {
-    constexpr int NW = gate_bwd_waves<NT>();
-    tpw = tiles_per_wave(B, H, S, NW * CUS, 64);
-    const int ntiles = (S + 31) / 32;
-    return dim3((ntiles + NW * tpw - 1) / (NW * tpw), H, B);
+    const int nw = gate_bwd_waves(d), ntiles = (d.S + 31) / 32;
+    tpw = tiles_per_wave(d.B, d.H, d.S, nw * CUS, 64);
+    return dim3((ntiles + nw * tpw - 1) / (nw * tpw), d.H, d.B);
 }
 
 template <int DH, int NT, bool NORM>
-hipError_t launch_gate(GateArgs a, bool backward, hipStream_t st)
+hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
 {
     static LdsOptIn optin_fwd, optin_bwd;
     if (backward) {
-        const size_t smem = gate_bwd_smem<NT>(DH);
-        const hipError_t e = ensure_dynamic_lds(optin_bwd, (const void*)mhffn_gate_bwd_kernel<DH, NT, NORM>, (int)smem);
+        const int most = (int)gate_bwd_smem<NT>(DH, gate_bwd_max_waves<NT>()), waves = gate_bwd_waves(d);
+        const hipError_t e = ensure_dynamic_lds(optin_bwd, (const void*)mhffn_gate_bwd_kernel<DH, NT, NORM>, most);
         if (e != hipSuccess) return e;
-        const dim3 grid = gate_bwd_grid<NT>(a.B, a.H, a.S, a.tpw);
-        hipLaunchKernelGGL((mhffn_gate_bwd_kernel<DH, NT, NORM>), grid, dim3(64 * gate_bwd_waves<NT>()), smem, st, a);
+        const dim3 grid = gate_bwd_grid(d, a.tpw);
+        hipLaunchKernelGGL((mhffn_gate_bwd_kernel<DH, NT, NORM>), grid, dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
     } else {
         const size_t smem = gate_fwd_smem(DH, NT);
         const hipError_t e = ensure_dynamic_lds(optin_fwd, (const void*)mhffn_gate_fwd_kernel<DH, NT, NORM>, (int)smem);
@@ -701,19 +738,19 @@ hipError_t launch_gate(GateArgs a, bool backward, hipStream_t st)
 }
 
 template <int DH>
-hipError_t launch_gate_dh(const GateArgs& a, bool backward, hipStream_t st)
+hipError_t launch_gate_dh(const GateArgs& a, const Dims& d, bool backward, hipStream_t st)
 {
     const bool norm = a.Wn != nullptr;
-    if (a.E <= 32) return norm ? launch_gate<DH, 1, true>(a, backward, st) : launch_gate<DH, 1, false>(a, backward, st);
-    return norm ? launch_gate<DH, 2, true>(a, backward, st) : launch_gate<DH, 2, false>(a, backward, st);
+    if (a.E <= 32) return norm ? launch_gate<DH, 1, true>(a, d, backward, st) : launch_gate<DH, 1, false>(a, d, backward, st);
+    return norm ? launch_gate<DH, 2, true>(a, d, backward, st) : launch_gate<DH, 2, false>(a, d, backward, st);
 }
 
-hipError_t launch_gate_any(const GateArgs& a, int d_h, bool backward, hipStream_t st)
+hipError_t launch_gate_any(const GateArgs& a, const Dims& d, bool backward, hipStream_t st)
 {
-    switch (d_h) {
-        case 64: return launch_gate_dh<64>(a, backward, st);
-        case 96: return launch_gate_dh<96>(a, backward, st);
-        case 128: return launch_gate_dh<128>(a, backward, st);
+    switch (d.d_h) {
+        case 64: return launch_gate_dh<64>(a, d, backward, st);
+        case 96: return launch_gate_dh<96>(a, d, backward, st);
+        case 128: return launch_gate_dh<128>(a, d, backward, st);
     }
     return hipErrorInvalidValue;
 }
@@ -721,7 +758,7 @@ hipError_t launch_gate_any(const GateArgs& a, int d_h, bool backward, hipStream_
 int gate_bwd_workgroups(const Dims& d)      // of one head
 {
     int tpw;
-    const dim3 g = d.E <= 32 ? gate_bwd_grid<1>(d.B, d.H, d.S, tpw) : gate_bwd_grid<2>(d.B, d.H, d.S, tpw);
+    const dim3 g = gate_bwd_grid(d, tpw);
     return (int)(g.x * g.z);
 }
 
@@ -739,7 +776,7 @@ hipError_t launch_gate_fwd(const void* X, const void* Wn, int wn_bf16, float eps
     a.Qn = (bf16_t*)Qn;
     a.R = R;
     a.B = d.B, a.H = d.H, a.S = d.S, a.E = d.E, a.eps = eps;
-    return launch_gate_any(a, d.d_h, false, st);
+    return launch_gate_any(a, d, false, st);
 }
 
 size_t gate_bwd_workspace_bytes(const Dims& d)
@@ -766,7 +803,7 @@ hipError_t launch_gate_bwd(const void* X, const void* Wn, int wn_bf16, float eps
     }
     a.dq_tokmaj = dq_tokmaj;
     a.B = d.B, a.H = d.H, a.S = d.S, a.E = d.E, a.eps = eps;
-    hipError_t err = launch_gate_any(a, d.d_h, true, st);
+    hipError_t err = launch_gate_any(a, d, true, st);
     if (err != hipSuccess || !ws) return err;
     const dim3 grid((d.d_h * d.E + d.d_h + 255) / 256, d.H);
     const int wgs = gate_bwd_workgroups(d);
