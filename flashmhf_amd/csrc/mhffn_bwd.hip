@@ -293,11 +293,12 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
 // 32 rows, four blocks a trip: the same products, element-wise formulas and order of sums as the kernel above.  K and U tiles
 // are read by all waves to the end of a trip, V only by its own wave's first products.  K tiles have two sets; LDS has no
 // room for a second set of U too, whose next tile waits in registers instead.  dR is one running sum over the elements of an
-// expert's blocks: wave k adds those of its block to what wave k - 1 left, in the k-th of the four phases in which all
-// waves take the second products of block k (an exchange of the terms would take another 32 KB of LDS; the phases cost 0.35 of
-// a trip's 2.7 us).  All three tiles through registers: 2.95 us a trip without the phases.
+// expert's blocks: wave k adds those of its block to what wave k - 1 left (an exchange of the terms would take another 32 KB of
+// LDS).  A number in LDS says whose turn it is -- the blocks added so far; a wave looks for its own in front of its second products of
+// its own block, by when the wave before has had the time of one block's products, and nobody else waits: 2.45 us a trip, against
+// 2.7 with a barrier behind each of the four.  (Wave 0's number is there since the trip before, so every wait ends.)
 constexpr int DQ32_U0 = 2 * QUAD * TILE_B, DQ32_V0 = DQ32_U0 + QUAD * TILE_B, DQ32_D0 = DQ32_V0 + QUAD * TILE_B,
-              DQ32_E0 = DQ32_D0 + QUAD * 4096, DQ32_R0 = DQ32_E0 + 256;
+              DQ32_E0 = DQ32_D0 + QUAD * 4096, DQ32_T0 = DQ32_E0 + 256, DQ32_R0 = DQ32_T0 + 256;
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
 {
@@ -344,6 +345,7 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
         }
     }
     quad_stage_gates(sR, p.R + ex0, nex, tid, [&](int t) { return p.rows.gate(hk, row_of(t)) * E; });
+    if (tid == 0) *reinterpret_cast<int*>(smem + DQ32_T0) = 0;
     // (from here to the end of the loop the vmcnt events are the fills, the loads of U and the stores of dR)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]), "+v"(go[ks]));
@@ -368,7 +370,7 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
     for (int i = 0; i < CT; ++i)
         if (i == wave) { tr.off[0][0] = trl.off[i][0]; tr.off[0][1] = trl.off[i][1]; }
     const unsigned smem0 = lds_addr(smem), rowoff = krow * TILE_ROW_B, sw = swz16(krow), ra = lds_addr(sR) + 4 * l32;
-    const unsigned sD = smem0 + DQ32_D0 + lane * 16, sE = smem0 + DQ32_E0 + lane * 4;
+    const unsigned sD = smem0 + DQ32_D0 + lane * 16, sE = smem0 + DQ32_E0 + lane * 4, sT = smem0 + DQ32_T0;
 
     auto trip = [&](auto set_, int b0) {
         constexpr int SET = decltype(set_)::value;
@@ -445,13 +447,20 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
             constexpr int k = decltype(kc)::value, c = k & 1;
             if (k == wave && k < nb) {
                 const int at = jb0 + b0 + k, e = p.parts.by_nbe.div(at), jb = at - e * nbe;
-                u32x2 in = lds_read_apart_async<1>(sE);
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(in));
+                u32x2 in;      // (the sum is read behind the number that is checked, and written in front of it)
+                int done;
+                do {
+                    u32x2 tag = lds_read_apart_async<1>(sT);
+                    in = lds_read_apart_async<1>(sE);
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tag), "+v"(in));
+                    done = __builtin_amdgcn_readfirstlane((int)tag[0]);
+                } while (done != b0 + k);
                 const unsigned bits = in[0];
                 float dr = jb == 0 || b0 + k == 0 ? 0.0f : __builtin_bit_cast(float, bits);
 #pragma unroll
                 for (int i = 0; i < 16; ++i) dr = __builtin_fmaf(as[i], n[i], dr);
                 lds_write4(sE, dr);
+                lds_write4(sT, __builtin_bit_cast(float, b0 + k + 1));
                 if (jb == nbe - 1 || b0 + k == nblk - 1) {
                     const float tot = dr + __shfl_xor(dr, 32);      // the lane halves hold disjoint j rows of one token column
                     if (g == 0 && tok0 + l32 < p.rows.n) drow[e] = tot;
@@ -469,14 +478,9 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
                     dq = mfma32(tr_value(tk[c][s]), __builtin_bit_cast(bf16x8, d[c][s]), dq);
                     dq = mfma32(tr_value(tu[c][s]), __builtin_bit_cast(bf16x8, d[c][2 + s]), dq);
                 });
-            // the next wave's running sum; behind the last phase, every wave is done with the tiles and the operands
-            if constexpr (k + 1 < QUAD) {
-                __builtin_amdgcn_sched_barrier(0);
-                if (k == wave) lds_wait_n<0>();
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-            } else quad_barrier();
+            __builtin_amdgcn_sched_barrier(0);
         });
+        quad_barrier();       // every wave is done with the tiles and the operands
     };
     for (int b0 = 0; b0 < nblk; b0 += 2 * QUAD) {
         trip(std::integral_constant<int, 0>{}, b0);
@@ -1061,9 +1065,10 @@ int dw_slices_bf16(const Dims& d, size_t ws_bytes)
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
-// Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.7 us (four steps of the
-// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 400 rows: 199 us with 256 rows, 85 with
-// 32; 2,048 rows: 202 and 173 (two rounds); one row in 32 parts of 32-row tiles 10.3 us.
+// Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.45 us (four steps of the
+// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 400 rows: 199 us with 256 rows, 79 with
+// 32; 2,048 rows: 202 and (at 2.7 us a trip, two rounds) 173; one row in 32 parts of 32-row tiles 10.1 us.  (Priced at 2.7, as the sweep
+// behind pick_parts measured it: the line between the two kernels lies where it did.)
 constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33, 1}, {32, 2.7, 0.05, QUAD}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
