@@ -297,6 +297,8 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
 // LDS).  A number in LDS says whose turn it is -- the blocks added so far; a wave looks for its own in front of its second products of
 // its own block, by when the wave before has had the time of one block's products, and nobody else waits: 2.45 us a trip, against
 // 2.7 with a barrier behind each of the four.  (Wave 0's number is there since the trip before, so every wait ends.)
+// A lone wave stands still while the loads that it has issued wait for the path to LDS: the next trip's K and U are requested one
+// instruction of each behind a k-step of the first products, V two behind four elements, instead of in bursts: 2.39 us.
 constexpr int DQ32_U0 = 2 * QUAD * TILE_B, DQ32_V0 = DQ32_U0 + QUAD * TILE_B, DQ32_D0 = DQ32_V0 + QUAD * TILE_B,
               DQ32_E0 = DQ32_D0 + QUAD * 4096, DQ32_T0 = DQ32_E0 + 256, DQ32_R0 = DQ32_T0 + 256;
 template <int DH>
@@ -317,15 +319,12 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
     unsigned char *ownU = smem + DQ32_U0 + wave * TILE_B, *ownV = smem + DQ32_V0 + wave * TILE_B;
     auto row_of = [&](int t) { return tok0 + t < p.rows.n ? tok0 + t : p.rows.n - 1; };
     auto block = [&](int b0) { return Kh + (long)(b0 + wave < nblk ? b0 + wave : nblk - 1) * JB * DH; };
-    auto fill_k = [&](int b0, int set) { quad_fill<DH>(block(b0), smem + (set * QUAD + wave) * TILE_B, lane); };
     // U through registers, coalesced as the fills are: row lane / 16 of every group of four, 16-byte chunk lane % 16 (a narrow
     // row's unused chunks take chunk 0)
     u32x4 un[8];
-    auto load_u = [&](int b0) {
+    auto load_u = [&](int b0, int i) {
         const int c = (lane & 15) < DH / 8 ? lane & 15 : 0;
-        const bf16_t* src = block(b0) + offU + (lane >> 4) * DH + c * 8;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) un[i] = *reinterpret_cast<const u32x4*>(src + 4 * i * DH);
+        un[i] = *reinterpret_cast<const u32x4*>(block(b0) + offU + (lane >> 4) * DH + c * 8 + 4 * i * DH);
     };
     auto store_u = [&]() {
         static_for<8>([&](auto ic) {
@@ -350,8 +349,9 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]), "+v"(go[ks]));
     __syncthreads();          // the gate values
-    load_u(0);
-    fill_k(0, 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) load_u(0, i);
+    quad_fill<DH>(block(0), smem + wave * TILE_B, lane);
     quad_fill<DH>(block(0) + offV, ownV, lane);
     float* drow;
     {
@@ -377,13 +377,10 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
         const unsigned sK = smem0 + SET * QUAD * TILE_B;
         __builtin_amdgcn_sched_barrier(0);
         store_u();            // (the barrier before was every wave's last use of the tile)
-        load_u(b0 + QUAD);
-        fill_k(b0 + QUAD, 1 - SET);
-        // this wave's K and V of the trip have landed: the sixteen loads just issued are younger (stores of dR in between only
-        // make the wait longer)
-        wait_vmcnt<16>();
+        wait_vmcnt<0>();      // this wave's K and V of the trip have landed
         __builtin_amdgcn_sched_barrier(0);
         u32x2 rv = lds_read_apart_async<1>(ra + 128 * p.parts.by_nbe.div(jb0 + (b0 + wave < nblk ? b0 + wave : nblk - 1)));
+        const bf16_t* next = block(b0 + QUAD);
         QuadRows<KS, 3> a;
         static_for<KS>([&](auto kc) {
             constexpr int ks = decltype(kc)::value;
@@ -401,24 +398,38 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
             m = mfma32(a.get(0, ks), q[ks], m);
             n = mfma32(a.get(1, ks), q[ks], n);
             da = mfma32(a.get(2, ks), go[ks], da);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = ks * 8 / KS; i < (ks + 1) * 8 / KS; ++i) {
+                load_u(b0 + QUAD, i);
+                tile_fill_ins<DH>(next, DH, smem + ((1 - SET) * QUAD + wave) * TILE_B, i, lane);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         });
         asm volatile("" : "+v"(rv));
         __builtin_amdgcn_sched_barrier(0);
-        quad_fill<DH>(block(b0 + QUAD) + offV, ownV, lane);      // (every read of the tile has returned)
         bf16x8 dmt[2], dnt[2];
         f32x16 as;            // the first factors of dR's terms (n holds the second ones)
         {
             const unsigned rbits = rv[0];
             const float r = __builtin_bit_cast(float, rbits);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float x = m[i], nn = n[i], a = da[i];
-                const float sg = fast_sigmoid(x);
-                const float sl = x * sg;                 // silu(m)
-                as[i] = a * sl;
-                const float w = __builtin_fmaf(sl, 1.0f - sg, sg);    // silu'(m)
-                dnt[i >> 3][i & 7] = (bf16_t)(r * as[i]);
-                dmt[i >> 3][i & 7] = (bf16_t)((r * a) * (nn * w));
+            for (int i4 = 0; i4 < 4; ++i4) {
+#pragma unroll
+                for (int i = 4 * i4; i < 4 * i4 + 4; ++i) {
+                    const float x = m[i], nn = n[i], a = da[i];
+                    const float sg = fast_sigmoid(x);
+                    const float sl = x * sg;                 // silu(m)
+                    as[i] = a * sl;
+                    const float w = __builtin_fmaf(sl, 1.0f - sg, sg);    // silu'(m)
+                    dnt[i >> 3][i & 7] = (bf16_t)(r * as[i]);
+                    dmt[i >> 3][i & 7] = (bf16_t)((r * a) * (nn * w));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 2 * i4; k < 2 * i4 + 2; ++k)      // (every read of the tile has returned)
+                    tile_fill_ins<DH>(next + offV, DH, ownV, k, lane);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         lds_write16<0>(sD + wave * 4096, dmt[0]);
@@ -1065,8 +1076,8 @@ int dw_slices_bf16(const Dims& d, size_t ws_bytes)
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
-// Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.45 us (four steps of the
-// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 400 rows: 199 us with 256 rows, 79 with
+// Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.4 us (four steps of the
+// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 400 rows: 199 us with 256 rows, 77 with
 // 32; 2,048 rows: 202 and (at 2.7 us a trip, two rounds) 173; one row in 32 parts of 32-row tiles 10.1 us.  (Priced at 2.7, as the sweep
 // behind pick_parts measured it: the line between the two kernels lies where it did.)
 constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33, 1}, {32, 2.7, 0.05, QUAD}};
