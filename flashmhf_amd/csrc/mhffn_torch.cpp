@@ -318,10 +318,11 @@ std::pair<Tensor, Tensor> gate(const Tensor& x, const std::optional<Tensor>& nor
 }
 
 // ---- products of the block's projections ----------------------------------------------------------------------------
-// A plain matrix that the product kernels read as it lies.
+// A plain matrix that the product kernels read as it lies; one with a tangent (forward mode, which may be entered for the backward alone)
+// is more than that.
 bool plain(const Tensor& t)
 {
-    return t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.is_cuda() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+    return !t._fw_grad(0).defined() && t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.is_cuda() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 // Whose products: the library's, these kernels', or these kernels' where both take each element's sum in the order of the summed index
 // and so have the same bits (a model's layers amplify a different rounding, see MHFFNDecoder in mhffn_layer.py).  The library splits the
