@@ -318,11 +318,20 @@ std::pair<Tensor, Tensor> gate(const Tensor& x, const std::optional<Tensor>& nor
 }
 
 // ---- products of the block's projections ----------------------------------------------------------------------------
-// A plain matrix that the product kernels read as it lies; one with a tangent (forward mode, which may be entered for the backward alone)
-// is more than that.
+// Whether a tensor on the GPU is its memory and nothing more: no code of a subclass, a transform (batches) or a lazy view (negation) is
+// to run for it, and no tangent goes with it (forward mode, which may be entered for the backward alone).  Asked before its pointer:
+// some of the others have none.
+bool memory_alone(const Tensor& t)
+{
+    using Key = c10::DispatchKey;
+    constexpr c10::DispatchKeySet plain_keys({Key::CUDA, Key::AutogradCUDA, Key::ADInplaceOrView, Key::AutocastCUDA});
+    return (t.key_set().raw_repr() & ~plain_keys.raw_repr()) == 0 && !t._fw_grad(0).defined();
+}
+// A plain matrix that the product kernels read as it lies.
 bool plain(const Tensor& t)
 {
-    return !t._fw_grad(0).defined() && t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.is_cuda() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+    return memory_alone(t) && t.is_contiguous() && t.scalar_type() == at::kBFloat16 &&
+           (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 // Whose products: the library's, these kernels', or these kernels' where both take each element's sum in the order of the summed index
 // and so have the same bits (a model's layers amplify a different rounding, see MHFFNDecoder in mhffn_layer.py).  The library splits the

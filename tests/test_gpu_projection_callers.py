@@ -1,4 +1,7 @@
-"""What meets the projections' own products as it meets torch's linear layer: forward mode in the backward alone."""
+"""What meets the projections' own products as it meets torch's linear layer: forward mode, batched gradients and tensors with code
+of their own, in the forward call and in the backward alone."""
+import warnings
+
 import pytest
 import torch
 from torch.autograd import forward_ad
@@ -70,3 +73,75 @@ def test_the_block_s_last_weight_keeps_its_gradient_s_tangent():
         g = forward_ad.unpack_dual(g)
     want, = torch.autograd.grad(y, [layer.w_self_2.weight], t)
     assert g.tangent is not None and _near(g.tangent, want)
+
+
+def test_gradients_in_batches(projection):
+    x, dys = _normal(0, B, S, H * dh).requires_grad_(), _normal(1, 3, B, S, projection.out_features)
+    y = projection(x)
+    got = torch.autograd.grad(y, [x, projection.weight], dys, is_grads_batched=True, retain_graph=True)
+    for i, dy in enumerate(dys):
+        assert all(_near(a[i], b) for a, b in zip(got, torch.autograd.grad(y, [x, projection.weight], dy, retain_graph=True)))
+
+
+class Seen(torch.Tensor):
+    """Records what is dispatched on it; `Wrapper` has no memory of its own, `Memory` has."""
+    __torch_function__ = torch._C._disabled_torch_function_impl
+    names = []
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        Seen.names.append(str(func))
+        tree = torch.utils._pytree
+        plain = tree.tree_map_only(Seen, lambda t: t.plain, (args, kwargs or {}))
+        return tree.tree_map_only(torch.Tensor, cls.of, func(*plain[0], **plain[1]))
+
+
+class Wrapper(Seen):
+    @staticmethod
+    def of(t):
+        r = torch.Tensor._make_wrapper_subclass(Wrapper, t.shape, strides=t.stride(), dtype=t.dtype, device=t.device,
+                                                requires_grad=t.requires_grad)
+        r.plain = t.detach()
+        return r
+
+
+class Memory(Seen):
+    @staticmethod
+    def of(t):
+        r = torch.Tensor._make_subclass(Memory, t.detach(), t.requires_grad)
+        r.plain = t.detach()
+        return r
+
+
+@pytest.mark.parametrize("cls", [Wrapper, Memory])
+@pytest.mark.parametrize("where", ["x", "weight", "dy"])
+def test_code_of_a_tensor_runs(projection, cls, where):
+    x, dy = _normal(0, B, S, H * dh).requires_grad_(), _normal(1, B, S, projection.out_features)
+    want = [projection(x)]
+    want += torch.autograd.grad(want[0], [x, projection.weight], dy)
+    if where == "x":
+        x = cls.of(x)
+    if where == "weight":
+        projection.weight = torch.nn.Parameter(cls.of(projection.weight))
+    Seen.names.clear()
+    y = projection(x)
+    assert where == "dy" or any("mm" in n for n in Seen.names) and isinstance(y, cls)
+    Seen.names.clear()
+    got = [y, *torch.autograd.grad(y, [x, projection.weight], cls.of(dy) if where == "dy" or isinstance(y, cls) else dy)]
+    assert sum("mm" in n for n in Seen.names) == 2 and all(isinstance(t, cls) for t in got[1:])
+    with torch.no_grad():
+        assert all(_near(getattr(a, "plain", a), b) for a, b in zip(got, want))
+
+
+def test_fake_tensors(projection):
+    from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    x = mode.from_tensor(_normal(0, B, S, H * dh)).requires_grad_()
+    with warnings.catch_warnings():
+        warnings.filterwarnings("error", message=".*data.pointer")
+        for inside in (False, True):
+            with mode if inside else torch.enable_grad():
+                y = projection(x)
+                dx, dw = torch.autograd.grad(y, [x, projection.weight], torch.ones_like(y))
+            assert all(type(t) is FakeTensor for t in (y, dx, dw)), inside
+            assert y.shape == (B, S, projection.out_features) and dx.shape == x.shape and dw.shape == projection.weight.shape
