@@ -556,6 +556,26 @@ Tensor rope_backward(Tensor dq, Tensor dk, Tensor dv, const Tensor& cos, const T
 }
 std::tuple<Tensor, Tensor, Tensor> rope(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H);
 
+// The same in torch's operations, for tensors that are more than their memory.
+std::tuple<Tensor, Tensor, Tensor> rope_by_elements(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
+{
+    const int64_t d = cos.size(1), half = d / 2;
+    auto rotate = [&](const Tensor& x) {
+        return x * cos + at::cat({-x.narrow(-1, half, half), x.narrow(-1, 0, half)}, -1) * sin;
+    };
+    const Tensor x = qkv.view({qkv.size(0), qkv.size(1), 3, H, d}).permute({2, 0, 3, 1, 4});
+    return {rotate(x.select(0, 0)), rotate(x.select(0, 1)), x.select(0, 2)};
+}
+Tensor rope_backward_by_elements(const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& cos, const Tensor& sin)
+{
+    const int64_t half = cos.size(1) / 2;
+    auto back = [&](const Tensor& g) {
+        const Tensor s = g * sin;
+        return g * cos + at::cat({s.narrow(-1, half, half), -s.narrow(-1, 0, half)}, -1);
+    };
+    return at::stack({back(dq), back(dk), dv}, 0).permute({1, 3, 0, 2, 4}).reshape({dq.size(0), dq.size(2), 3 * dq.size(1) * dq.size(3)});
+}
+
 // The backward as a node of its own, for create_graph: the map is linear in dq, dk, dv and its transpose is the forward.
 struct RopeBackNode : torch::autograd::Function<RopeBackNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& cos, const Tensor& sin)
@@ -583,10 +603,15 @@ struct RopeNode : torch::autograd::Function<RopeNode> {
     {
         const auto s = ctx->get_saved_variables();
         Tensor any;
+        bool memory = true;
         for (const Tensor& t : g)
-            if (t.defined()) any = t;
+            if (t.defined()) {
+                any = t;
+                memory = memory && memory_alone(t);
+            }
         for (Tensor& t : g)
             if (!t.defined()) t = at::zeros_like(any);
+        if (!memory) return {rope_backward_by_elements(g[0], g[1], g[2], s[0], s[1]), Tensor(), Tensor(), Tensor()};
         const Tensor dqkv = records_grad({&g[0], &g[1], &g[2]}) ? RopeBackNode::apply(g[0], g[1], g[2], s[0], s[1])
                                                                 : rope_backward(g[0], g[1], g[2], s[0], s[1]);
         return {dqkv, Tensor(), Tensor(), Tensor()};
@@ -594,6 +619,7 @@ struct RopeNode : torch::autograd::Function<RopeNode> {
 };
 std::tuple<Tensor, Tensor, Tensor> rope(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t H)
 {
+    if (!memory_alone(qkv) || !memory_alone(cos) || !memory_alone(sin)) return rope_by_elements(qkv, cos, sin, H);
     if (!records_grad({&qkv})) {
         RopeForward f = rope_forward(qkv, cos, sin, H);
         return {f.q, f.k, f.v};

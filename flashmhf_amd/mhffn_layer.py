@@ -254,7 +254,7 @@ class CausalSelfAttention(nn.Module):
         qkv = self.qkv(x)
         if (qkv.is_cuda and qkv.dtype == cos.dtype == sin.dtype == torch.bfloat16 and self.head_dim % 16 == 0 and qkv.numel()
                 and all(t.shape == (S, self.head_dim) and t.device == qkv.device and not t.requires_grad for t in (cos, sin))
-                and _capi.native_nodes()):
+                and _capi.native_nodes() and not torch.overrides.has_torch_function((qkv, cos, sin))):
             # one pass, the same roundings
             q, k, v = _capi.native().rope(qkv.contiguous(), cos.contiguous(), sin.contiguous(), self.num_heads)
         else:

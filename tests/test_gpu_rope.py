@@ -3,7 +3,8 @@ product and sum rounded): the same values, forward and backward, also for gradie
 import pytest
 import torch
 
-from flashmhf_amd.mhffn_layer import _apply_rotary, _rotary
+from flashmhf_amd.mhffn_layer import CausalSelfAttention, _apply_rotary, _rotary
+from tests.test_gpu_projection_callers import Memory, Wrapper
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +77,53 @@ def test_gradient_penalty_through_attention(monkeypatch):
         results.append([dx, *torch.autograd.grad(dx.float().square().sum(), [x, *attn.parameters()])])
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+def _both(x, tables, H, d):
+    """The native call and the element-wise form."""
+    from flashmhf_amd import _capi
+    B, S, _ = x.shape
+    q, k, v = x.view(B, S, 3, H, d).permute(2, 0, 3, 1, 4)
+    return _capi.native().rope(x, *tables, H), (_apply_rotary(q, *tables), _apply_rotary(k, *tables), v)
+
+
+@pytest.mark.parametrize("asked", [(0, 1, 2), (0,), (2,)])
+def test_gradients_that_are_more_than_their_memory(asked):
+    """Tangents (forward mode for the backward alone), batches, subclasses with code of their own: what the element-wise form gives."""
+    from torch.autograd import forward_ad
+    dev, (B, S, H, d) = "cuda:0", (2, 9, 3, 32)
+    torch.manual_seed(0)
+    tables = _rotary(S, d, 10000.0, torch.device(dev), torch.bfloat16)
+    x = torch.randn(B, S, 3 * H * d, device=dev).bfloat16().requires_grad_()
+    outs = [[o[i] for i in asked] for o in _both(x, tables, H, d)]
+    dys, ts = ([torch.randn(B, H, S, d, device=dev).bfloat16() for _ in asked] for _ in range(2))
+    with forward_ad.dual_level():
+        got, want = (forward_ad.unpack_dual(torch.autograd.grad(o, x, [forward_ad.make_dual(*p) for p in zip(dys, ts)], retain_graph=True)[0])
+                     for o in outs)
+        assert torch.equal(got.primal, want.primal) and torch.equal(got.tangent, want.tangent)
+    got, want = (torch.autograd.grad(o, x, [torch.stack(p) for p in zip(dys, ts)], is_grads_batched=True, retain_graph=True)[0] for o in outs)
+    assert torch.equal(got, want)
+    for cls in (Wrapper, Memory):
+        got, want = (torch.autograd.grad(o, x, [cls.of(t) for t in dys], retain_graph=True)[0] for o in outs)
+        assert isinstance(got, cls) and torch.equal(got.plain, want.plain)
+
+
+@pytest.mark.parametrize("cls", [Wrapper, Memory])
+def test_code_of_a_tensor_runs(cls):
+    dev, (B, S, H, d) = "cuda:0", (2, 9, 3, 32)
+    torch.manual_seed(0)
+    tables = _rotary(S, d, 10000.0, torch.device(dev), torch.bfloat16)
+    x = torch.randn(B, S, 3 * H * d, device=dev).bfloat16()
+    _, want = _both(x, tables, H, d)
+    got, _ = _both(cls.of(x), tables, H, d)
+    assert all(isinstance(a, cls) and torch.equal(a.plain, b) for a, b in zip(got, want))
+
+
+def test_a_subclass_is_carried_through():
+    class Named(torch.Tensor):
+        pass
+    dev, (S, H, d) = "cuda:0", (9, 3, 32)
+    attn = CausalSelfAttention(H * d, H).to(dev).to(torch.bfloat16)
+    x = torch.randn(2, S, H * d, device=dev).bfloat16()
+    y = attn(x.as_subclass(Named))
+    assert type(y) is Named and torch.equal(y.as_subclass(torch.Tensor), attn(x))
