@@ -333,14 +333,20 @@ bool plain(const Tensor& t)
     return memory_alone(t) && t.is_contiguous() && t.scalar_type() == at::kBFloat16 &&
            (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
-// Whose products: the library's, these kernels', or these kernels' where both take each element's sum in the order of the summed index
-// and so have the same bits (a model's layers amplify a different rounding, see MHFFNDecoder in mhffn_layer.py).  The library splits the
-// summed index for 16 rows and fewer, and in NN with more than 1,024 of it and no more than 2^18 results (found by comparing
-// bits: 2,370 products of hidden 768 and 1024, 1 to 2,048 rows).
+// Whose products: the library's, these kernels', or these kernels' where the library was found to take each element's sum in the order
+// of the summed index, as the tile kernels do, so that both have the same bits (a model's layers amplify a different rounding, see
+// MHFFNDecoder in mhffn_layer.py).  Found by comparing bits, 11,700 products of 512 to 4,096 columns and summed indexes to 8,192, of
+// 17 to 8,192 rows: the library splits the summed index, or adds in another order,
+//   NT  below 32 rows, and with more than 1,024 of the summed index only where there are no more than 2^18 results
+//   NN  at 16 rows and fewer, and with more than 1,024 of the summed index only where there are no more than 2^18 results
+//   TN  for 16 rows and fewer, and for more than 16,384.  Above them the sum stays in order here: the gradient of a weight goes into
+//       no other layer's (hidden 1024, 32,768 rows: 128 us, the library's 198).
+// It is a table of another library's choices, not a promise of it: tests/test_gpu_product.py compares.
 enum Whose { LIBRARY = 0, OWN = 1, OWN_IN_ORDER = 2 };
 bool library_in_order(int form, int64_t M, int64_t N, int64_t K)
 {
-    return (form == MHFFN_PRODUCT_TN ? K : M) > 16 && (form != MHFFN_PRODUCT_NN || K <= 1024 || M * N > (1 << 18));
+    if (form == MHFFN_PRODUCT_TN) return K > 16;
+    return M > (form == MHFFN_PRODUCT_NT ? 31 : 16) && (K <= 1024 || M * N > (1 << 18));
 }
 // M x N with inner extent K into `out_sizes`, or an undefined tensor where the product is the library's: outside the kernels'
 // sizes, under a dispatch mode (which is to see the call), or where autograd is to record the call.

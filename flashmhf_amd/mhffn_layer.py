@@ -80,7 +80,7 @@ class Projection(nn.Linear):
 
 
 class OrderedProjection(Projection):
-    """... where they also have the library's bits: both take every sum in the order of its terms."""
+    """... with every sum in the order of its terms, and only at sizes at which the library was found to take it so, too."""
     products = 2
 
 
@@ -285,8 +285,9 @@ class MHFFNDecoder(nn.Module):
         # depend on the rest of its batch.  (Rounding differences of the operator grow from block to block: another order
         # moves the gradients of a four-block model by 1 % of their norm.)
         layer_kw.setdefault("op", FlashMLPMoE(one_part=True))
-        # Products in one order of summation, too, the library's: in another (Projection) single gradients of a four-block model
-        # move by half of their root mean square.
+        # Products, too: every sum in the order of its terms where they are the framework's own, which is where the library was
+        # found to take it so (OrderedProjection); the others are the library's.  In another order (Projection) single gradients of
+        # a four-block model move by half of their root mean square.
         layer_kw.setdefault("linear", OrderedProjection)
         self.embed = nn.Embedding(vocab_size, hidden_size)
         self.blocks = nn.ModuleList(

@@ -79,6 +79,13 @@ def test_sums_in_order_have_the_library_s_bits(M, N, K):
         assert torch.equal(a, b)
 
 
+# sizes at which the library sums in another order: nothing but its own products has its bits
+@pytest.mark.parametrize("M,N,K", [(17, 1024, 1024), (24, 768, 768), (31, 2048, 768), (128, 1024, 4096), (96, 1280, 1280), (80, 1536, 1536),
+                                   (64, 2048, 2048), (144, 1792, 1792)])
+def test_ordered_projections_of_few_rows_have_the_library_s_bits(M, N, K):
+    test_sums_in_order_have_the_library_s_bits(M, N, K)
+
+
 @pytest.mark.parametrize("T", [1, 16, 300, 2048])
 def test_the_block_projects_as_a_linear_layer_does(T):
     """A captured graph of the block, replayed with the program's own work between, gives what an eager call gives, and a dispatch
