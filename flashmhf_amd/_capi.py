@@ -27,7 +27,7 @@ EXPORTS = (
     "mhffn_bwd_workspace_bytes", "mhffn_bwd_workspace_min_bytes", "mhffn_fwd", "mhffn_bwd", "mhffn_fwd_phases", "mhffn_bwd_phases",
     "mhffn_fwd_layout", "mhffn_bwd_layout", "mhffn_bwd_static", "mhffn_gate_fwd", "mhffn_gate_bwd",
     "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into", "mhffn_rope_fwd", "mhffn_rope_bwd",
-    "mhffn_product_preferred", "mhffn_product_tile", "mhffn_product",
+    "mhffn_product_preferred", "mhffn_product_faster", "mhffn_product_tile", "mhffn_product",
 )
 PRODUCT_NT, PRODUCT_NN, PRODUCT_TN = 0, 1, 2
 TOKENS_BHSD, TOKENS_BSHD = 0, 1     # layout of Q, O, dO, dQ
@@ -83,6 +83,7 @@ def lib():
         L.mhffn_rope_fwd.argtypes = [vp] * 5 + [ctypes.c_int] * 4 + [vp]
         L.mhffn_rope_bwd.argtypes = [vp] * 3 + [ctypes.POINTER(ctypes.c_long)] + [vp] * 3 + [ctypes.c_int] * 4 + [vp]
         L.mhffn_product_preferred.argtypes = [ctypes.c_int] * 2
+        L.mhffn_product_faster.argtypes = [ctypes.c_int] * 5
         L.mhffn_product_tile.argtypes = [ctypes.c_int] * 5
         L.mhffn_product.argtypes = [ctypes.c_int] * 2 + [vp] * 3 + [ctypes.c_int] * 3 + [vp]
         _lib = L

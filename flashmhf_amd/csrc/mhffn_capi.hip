@@ -362,6 +362,11 @@ int mhffn_product_tile(int form, int in_order, int M, int N, int K)
     return check_product(form, M, N, K) == MHFFN_OK ? mhffn::product_tile(form, in_order != 0, M, N, K) : 0;
 }
 
+int mhffn_product_faster(int form, int in_order, int M, int N, int K)
+{
+    return check_product(form, M, N, K) == MHFFN_OK && mhffn::product_faster(form, in_order != 0, M, N, K);
+}
+
 int mhffn_product(int form, int in_order, const void* A, const void* B, void* C, int M, int N, int K, void* stream)
 {
     const int rc = check_product(form, M, N, K);

@@ -6,7 +6,7 @@
 //     TN   C[M,N] = A[K,M]^T B[K,N]      dy^T x      both cols
 //
 // They stand beside the library's products, which are made for matrices large enough to fill the chip with tiles of 256: at one
-// round of smaller tiles (product_preferred) these are faster.  us per product in a captured graph of 20, library / here:
+// round of smaller tiles these are faster but for the exceptions at product_faster.  us per product in a captured graph of 20, library / here:
 //     hidden 1024, tokens    64         512        1,024       2,048       4,096
 //         NT             6.6 / 3.9   6.5 / 5.1   8.0 / 7.5  10.3 / 9.1  13.5 / 12.5
 //         NN             8.7 / 6.8   8.0 / 6.9   9.3 / 7.2  11.2 / 8.8  14.3 / 12.7
@@ -461,13 +461,15 @@ struct ProductVariant {
 constexpr ProductVariant PRODUCT_VARIANTS[] = {{64, 64, 3.2, 0.23, 0.0, 2.8}, {128, 64, 3.4, 0.285, 0.12, 2.9}, {128, 128, 3.6, 0.4, 0.3, 1.0},
                                                {32, 64, 2.8, 0.18, 0.1, 1.6},                                       // NT in order
                                                {32, 32, 2.4, 0.08, 0.2, 1.3}, {64, 32, 3.0, 0.115, 0.1, 1.6}};      // NT in any order
+constexpr int FIRST_SPLIT = 4;
+static long product_tiles(const ProductVariant& p, int M, int N) { return (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn); }
 static int product_variant(int form, bool in_order, int M, int N, int K)
 {
     int best = 0;
     double best_us = 0;
     for (int v = 0; v < (form != PRODUCT_NT ? 3 : in_order ? 4 : 6); ++v) {
         const ProductVariant& p = PRODUCT_VARIANTS[v];
-        const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), rounds = (tiles + CUS - 1) / CUS;
+        const long tiles = product_tiles(p, M, N), rounds = (tiles + CUS - 1) / CUS;
         const double load = tiles <= CUS / 2 ? 0 : tiles >= CUS ? 1 : (tiles - CUS / 2) / (double)(CUS / 2);
         const double us = p.base + (rounds - 1) * p.again + rounds * ((K + 63) / 64) * p.step * (1 + p.full * load);
         if (best_us == 0 || us < best_us) { best_us = us; best = v; }
@@ -483,6 +485,25 @@ int product_tile(int form, bool in_order, int M, int N, int K)
 // against 11.7, of 2,048^3 20.3 against 20.4; TN of the latter 21.2 against 25.3); with more its larger tiles win in NT and NN
 // (8,192 x 1,024 x 1,024: 25 against 22).
 bool product_preferred(int M, int N) { return (long)((M + 127) / 128) * ((N + 127) / 128) <= CUS; }
+
+// ... but for what the form and the length of the sum add to that.  us here / library, in a graph of ten:
+//   TN  faster at every length of the sum: hidden 1024 with 2,048 tokens 10.9 / 16.8, 16,384 59.6 / 101.6, 32,768 128 / 198; hidden 2048
+//       23 / 28, 151 / 168 and 292 / 292; 1,024 x 3,072 of 16,384 tokens 127 / 148.
+//   NN  for few rows the library splits the sum, and here it is one wave's chain: 8 rows of hidden 320 5.0 / 5.8, 384 5.0 / 4.6, 768
+//       6.4 / 5.2, 2048 11.0 / 7.0; 24 rows of hidden 1024 7.3 / 8.2, 1280 8.2 / 6.0, 2048 11.0 / 7.6; 64 rows of hidden 2048 11.0 / 13.1.
+//   NT  a long sum in the tile kernels takes longer than in the library's deeper tiles: 733 rows of hidden 2048 14.4 / 13.5, but 1,024 rows
+//       15.4 / 16.5; of 2560 19.2 / 18.1 and 22.4 / 21.9; of 4096 33.6 / 28.9 and 38.0 / 35.7.  One round of the split kernel is faster
+//       at any length: 64 rows of hidden 4096 9.2 / 12.5.
+bool product_faster(int form, bool in_order, int M, int N, int K)
+{
+    if (!product_preferred(M, N)) return false;
+    if (form == PRODUCT_NN) return M > 16 ? K <= 1024 || M >= 64 : K < 384;
+    if (form == PRODUCT_NT && K > 2048) {
+        const int v = product_variant(form, in_order, M, N, K);
+        return v >= FIRST_SPLIT && product_tiles(PRODUCT_VARIANTS[v], M, N) <= CUS;
+    }
+    return true;
+}
 
 template <bool ACOLS, bool BCOLS>
 static hipError_t launch_form(const ProductArgs& a, int variant, hipStream_t st)

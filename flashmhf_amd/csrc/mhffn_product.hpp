@@ -6,7 +6,8 @@ namespace mhffn {
 // Products of bfloat16 matrices (mhffn_product.hip), forms as MHFFN_PRODUCT_* in include/mhffn.h; N and K (TN: M and N) multiples of 8.
 constexpr int PRODUCT_NT = 0, PRODUCT_NN = 1, PRODUCT_TN = 2;
 int product_tile(int form, bool in_order, int M, int N, int K);      // 65536 * rows + columns of the tiles that a launch runs in
-bool product_preferred(int M, int N);
+bool product_preferred(int M, int N);                                 // the result is one round of tiles or less
+bool product_faster(int form, bool in_order, int M, int N, int K);    // faster than the library's product
 hipError_t launch_product(int form, bool in_order, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st);
 
 }  // namespace mhffn

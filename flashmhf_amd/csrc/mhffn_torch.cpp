@@ -348,16 +348,15 @@ bool library_in_order(int form, int64_t M, int64_t N, int64_t K)
     if (form == MHFFN_PRODUCT_TN) return K > 16;
     return M > (form == MHFFN_PRODUCT_NT ? 31 : 16) && (K <= 1024 || M * N > (1 << 18));
 }
-// M x N with inner extent K into `out_sizes`, or an undefined tensor where the product is the library's: outside the kernels'
-// sizes, under a dispatch mode (which is to see the call), or where autograd is to record the call.
+// M x N with inner extent K into `out_sizes`, or an undefined tensor where the product is the library's: where it is
+// faster or outside the kernels' sizes, under a dispatch mode (which is to see the call), or where autograd is to record the call.
 Tensor own_product(int form, Whose whose, const Tensor& a, const Tensor& b, int64_t M, int64_t N, int64_t K, at::IntArrayRef out_sizes)
 {
     if (whose == LIBRARY || (whose == OWN_IN_ORDER && !library_in_order(form, M, N, K))) return {};
     if (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) return {};
     if (!plain(a) || !plain(b) || a.device() != b.device() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return {};
-    if (std::max({M, N, K}) > INT_MAX || !mhffn_product_preferred((int)M, (int)N)) return {};
     const int in_order = whose == OWN_IN_ORDER;
-    if (!mhffn_product_tile(form, in_order, (int)M, (int)N, (int)K)) return {};
+    if (std::max({M, N, K}) > INT_MAX || !mhffn_product_faster(form, in_order, (int)M, (int)N, (int)K)) return {};
     RECORD_FUNCTION("mhffn::product", std::vector<c10::IValue>());
     OnDevice on_device(a);
     Tensor c = empty_of(out_sizes, at::kBFloat16, a);

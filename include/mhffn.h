@@ -229,11 +229,13 @@ int mhffn_rope_bwd(const void* dq, const void* dk, const void* dv, const long* s
  * Extents positive; N, and K (NT, NN) or M (TN), multiples of 8 (MHFFN_ERR_SHAPE otherwise).  in_order: nonzero for sums taken
  * in the order of the summed index whatever the size; zero leaves the order to the size.  mhffn_product_preferred() is 1
  * where these kernels are meant for the size of the result, 0 where a BLAS library's larger tiles are faster;
+ * mhffn_product_faster() is 1 where they also are for this form and length of the sum (0: slower, or extents refused);
  * mhffn_product_tile() is the tile a product runs in, 65536 * rows + columns (0: extents refused). */
 #define MHFFN_PRODUCT_NT 0
 #define MHFFN_PRODUCT_NN 1
 #define MHFFN_PRODUCT_TN 2
 int mhffn_product_preferred(int M, int N);
+int mhffn_product_faster(int form, int in_order, int M, int N, int K);
 int mhffn_product_tile(int form, int in_order, int M, int N, int K);
 int mhffn_product(int form, int in_order, const void* A, const void* B, void* C, int M, int N, int K, void* stream);
 

@@ -168,3 +168,23 @@ def test_products_that_nobody_asks_for_are_not_taken(trained, products, by):
             torch.autograd.grad(layer(x), asked, torch.ones_like(x))
         counts = {e.key: e.count for e in prof.key_averages()}
         assert (counts.get("mhffn::product"), counts.get("aten::mm", 0)) == (products, 0), stepwise
+
+
+# (own products of: y, dx, dw; the others are the library's)
+@pytest.mark.parametrize("T,hidden,own", [(8, 320, 3), (8, 1024, 2), (32, 1024, 3), (63, 2048, 2), (64, 2048, 3), (160, 3072, 1)])
+def test_few_rows_and_long_sums_take_the_faster_product(T, hidden, own):
+    from flashmhf_amd.mhffn_layer import Projection
+    dev = "cuda:0"
+    torch.manual_seed(T)
+    m = Projection(hidden, hidden, bias=False, device=dev, dtype=torch.bfloat16)
+    x, dy = (torch.randn(T, hidden, device=dev).bfloat16() for _ in range(2))
+    x.requires_grad_()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        y = m(x)
+        dx, dw = torch.autograd.grad(y, [x, m.weight], dy)
+    names = {e.key: e.count for e in prof.key_averages()}
+    assert (names.get("mhffn::product", 0), names.get("aten::mm", 0)) == (own, 3 - own)
+    a, b, w = (t.detach().double() for t in (x, dy, m.weight))
+    for got, p, q, K in ((y, a, w.t().contiguous(), hidden), (dx, b, w, hidden), (dw, b.t().contiguous(), a, T)):
+        ref, mag = p @ q, p.abs() @ q.abs()
+        assert ((got.double() - ref).abs() <= ref.abs() * 2 ** -8 + mag * K * 2 ** -24).all()

@@ -95,3 +95,15 @@ def test_each_kernel_matches_the_oracle(dh, dims, want):
     ref = (orc.mhffn_forward(*ins[:5], compute_dtype=torch.float64), *orc.mhffn_backward(*ins, compute_dtype=torch.float64))
     for name, a, r in zip(("O", "dQ", "dK", "dU", "dV", "dR"), got, ref):
         assert_bf16_parity(name, a.float().cpu(), r, (dh, dims))
+
+
+# (form, in order, M, N, K): both sides of every line of the rule that chooses between the framework's products and the library's
+@pytest.mark.parametrize("product,here", [
+    (("TN", 0, 1024, 1024, 1), True), (("TN", 1, 1024, 1024, 1 << 20), True), (("TN", 0, 2048, 2056, 300), False), (("TN", 0, 12, 64, 64), False),
+    (("NN", 0, 16, 512, 376), True), (("NN", 0, 16, 512, 384), False), (("NN", 0, 17, 512, 1024), True), (("NN", 0, 63, 512, 1032), False),
+    (("NN", 0, 64, 512, 1032), True), (("NN", 0, 64, 512, 8192), True),
+    (("NT", 0, 2048, 2048, 2048), True), (("NT", 0, 2048, 2048, 2056), False), (("NT", 0, 64, 4096, 4096), True), (("NT", 1, 64, 4096, 4096), False),
+    (("NT", 0, 160, 3072, 3072), False), (("NT", 0, 2049, 2048, 64), False), (("NT", 1, 1, 64, 64), True), (("NT", 0, 1, 64, 12), False)])
+def test_whose_products_are_faster(product, here):
+    form = {"NT": _capi.PRODUCT_NT, "NN": _capi.PRODUCT_NN, "TN": _capi.PRODUCT_TN}[product[0]]
+    assert bool(_capi.lib().mhffn_product_faster(form, *product[1:])) is here
