@@ -67,7 +67,8 @@ def router_gate(logits):
 
 class Projection(nn.Linear):
     """nn.Linear whose products, forward and backward, run in the framework's kernels where these are faster than the library's
-    (csrc/mhffn_product.hip): bfloat16 on the GPU, without bias, called as the plain layer; else nn.Linear's own forward."""
+    (csrc/mhffn_product.hip): bfloat16 on the GPU, without bias, called as the plain layer; else nn.Linear's own forward.  Tools
+    that go by the exact type nn.Linear do not take a subclass: `linear=nn.Linear` makes a block or a decoder without any."""
     products = 1        # `Whose` in csrc/mhffn_torch.cpp
 
     def forward(self, x):
@@ -242,11 +243,11 @@ def _apply_rotary(x, cos, sin):
 
 
 class CausalSelfAttention(nn.Module):
-    def __init__(self, hidden_size, num_heads, rope_base=10000.0):
+    def __init__(self, hidden_size, num_heads, rope_base=10000.0, linear=OrderedProjection):
         super().__init__()
         self.num_heads, self.head_dim, self.rope_base = num_heads, hidden_size // num_heads, rope_base
-        self.qkv = OrderedProjection(hidden_size, 3 * hidden_size, bias=False)
-        self.out = OrderedProjection(hidden_size, hidden_size, bias=False)
+        self.qkv = linear(hidden_size, 3 * hidden_size, bias=False)
+        self.out = linear(hidden_size, hidden_size, bias=False)
 
     def forward(self, x, rope=None):
         B, S, hid = x.shape
@@ -265,10 +266,10 @@ class CausalSelfAttention(nn.Module):
 
 
 class MHFFNDecoderBlock(nn.Module):
-    def __init__(self, hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps=1e-6, **layer_kw):
+    def __init__(self, hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps=1e-6, attn_linear=OrderedProjection, **layer_kw):
         super().__init__()
         self.input_norm = RMSNorm((hidden_size,), eps)
-        self.attn = CausalSelfAttention(hidden_size, attn_heads)
+        self.attn = CausalSelfAttention(hidden_size, attn_heads, linear=attn_linear)
         self.post_attn_norm = RMSNorm((hidden_size,), eps)
         self.mlp = MHFFNLayer(hidden_size, ffn_heads, num_experts, expert_dim, rms_norm_eps=eps, **layer_kw)
 
@@ -288,13 +289,13 @@ class MHFFNDecoder(nn.Module):
         # Products, too: every sum in the order of its terms where they are the framework's own, which is where the library was
         # found to take it so (OrderedProjection); the others are the library's.  In another order (Projection) single gradients of
         # a four-block model move by half of their root mean square.
-        layer_kw.setdefault("linear", OrderedProjection)
+        linear = layer_kw.setdefault("linear", OrderedProjection)
         self.embed = nn.Embedding(vocab_size, hidden_size)
         self.blocks = nn.ModuleList(
-            MHFFNDecoderBlock(hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps, **layer_kw)
+            MHFFNDecoderBlock(hidden_size, attn_heads, ffn_heads, num_experts, expert_dim, eps, attn_linear=linear, **layer_kw)
             for _ in range(num_layers))
         self.norm = RMSNorm((hidden_size,), eps)
-        self.lm_head = OrderedProjection(hidden_size, vocab_size, bias=False)
+        self.lm_head = linear(hidden_size, vocab_size, bias=False)
         nn.init.normal_(self.embed.weight, std=0.02)
         for m in self.modules():
             if isinstance(m, nn.Linear):

@@ -188,3 +188,20 @@ def test_few_rows_and_long_sums_take_the_faster_product(T, hidden, own):
     for got, p, q, K in ((y, a, w.t().contiguous(), hidden), (dx, b, w, hidden), (dw, b.t().contiguous(), a, T)):
         ref, mag = p @ q, p.abs() @ q.abs()
         assert ((got.double() - ref).abs() <= ref.abs() * 2 ** -8 + mag * K * 2 ** -24).all()
+
+
+@pytest.mark.parametrize("B,S", [(1, 24), (1, 300), (3, 200)])
+def test_a_decoder_of_linear_layers_has_the_same_bits(B, S):
+    """The decoder's own projections against torch's layers throughout, loss and every gradient."""
+    from flashmhf_amd import MHFFNDecoder
+    dev = "cuda:0"
+    ids = torch.randint(0, 512, (B, S), device=dev, generator=torch.Generator(device=dev).manual_seed(S))
+    results = []
+    for kw in ({}, {"linear": torch.nn.Linear}):
+        torch.manual_seed(0)
+        with torch.device(dev):
+            m = MHFFNDecoder(512, 768, 2, 8, 8, 3, 64, **kw).to(torch.bfloat16)
+        loss = m(ids, labels=ids)
+        results.append((loss, *torch.autograd.grad(loss, list(m.parameters()))))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

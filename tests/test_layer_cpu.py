@@ -104,3 +104,12 @@ def test_decoder_runs_and_trains_on_cpu_with_the_eager_operator():
         ids2[:, -1] = (ids2[:, -1] + 1) % 50
         b = model(ids2)
     assert torch.allclose(a[:, :-1], b[:, :-1], atol=1e-6)
+
+
+@pytest.mark.parametrize("linear", [None, torch.nn.Linear])
+def test_tools_that_go_by_the_exact_type_find_every_projection(linear):
+    """With linear=nn.Linear; without it they are subclasses of it."""
+    model = MHFFNDecoder(50, 32, 2, 4, 4, 2, 8, op=_eager_op, **({} if linear is None else {"linear": linear}))
+    layers = [m for m in model.modules() if isinstance(m, torch.nn.Linear)]
+    assert len(layers) == 2 * 4 + 1
+    assert sum(type(m) is torch.nn.Linear for m in layers) == (0 if linear is None else len(layers))
