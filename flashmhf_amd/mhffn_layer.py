@@ -158,12 +158,12 @@ class MHFFNLayer(nn.Module):
         q = self.w_self(x).view(B, S, H, dh)
         # (d_h = 128 with more than 32 experts and RMSNorm is left to torch: that instantiation of the prologue's backward
         # kernel does not fit the register file and runs several times slower than it should; so is a q_norm with code of its
-        # own, which the kernel would pass by)
+        # own, which the kernel would pass by, or with a weight of another form than [H, d_h], such as one that the heads share)
+        norm = self.q_norm
         if (self.fused_prologue and self.router_input == "q" and q.dtype == torch.bfloat16 and q.is_cuda
                 and E <= 64 and dh in (64, 96, 128)
-                and (self.q_norm is None or _runs_own_forward(self.q_norm, RMSNorm) and not (dh == 128 and E > 32))):
-            return head_norm_gate(q, None if self.q_norm is None else self.q_norm.weight, self.router,
-                                  self.rms_norm_eps)
+                and (norm is None or _runs_own_forward(norm, RMSNorm) and norm.weight.shape == (H, dh) and not (dh == 128 and E > 32))):
+            return head_norm_gate(q, None if norm is None else norm.weight, self.router, self._head_norm_eps())
         if self.q_norm is not None:
             q = self.q_norm(q)
         Q = q.transpose(1, 2)                                       # a view: the kernels read token-major rows
@@ -172,6 +172,10 @@ class MHFFNLayer(nn.Module):
         else:
             logits = (x.float() @ self.w_router.float()).view(B, S, H, E).transpose(1, 2)
         return Q, router_gate(logits).contiguous()
+
+    def _head_norm_eps(self):
+        """That of the norm in place, which may be another than the block was made with."""
+        return self.rms_norm_eps if self.q_norm is None else self.q_norm.eps
 
     def _stock_steps(self):
         """The tensors of the block (projection, head norm's weight or None, router, K, U, V, output projection) where every
@@ -205,6 +209,7 @@ class MHFFNLayer(nn.Module):
             return None
         w1, norm, router, K, U, V, w2 = weights
         if not (w1.dtype == w2.dtype == K.dtype == U.dtype == V.dtype == torch.bfloat16
+                and (norm is None or norm.shape == (self.num_heads, self.head_dim))
                 and not torch.overrides.has_torch_function((x, w1, w2, K, U, V, router, norm))):
             return None
         return weights
@@ -216,7 +221,7 @@ class MHFFNLayer(nn.Module):
             m = self._modules
             cls = type(m["w_self"])
             products = cls.products if cls is type(m["w_self_2"]) and cls is not nn.Linear else 0
-            return _capi.native().block(x, *weights, self.rms_norm_eps, m["op"].one_part, products)
+            return _capi.native().block(x, *weights, self._head_norm_eps(), m["op"].one_part, products)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view

@@ -138,3 +138,28 @@ def test_an_own_head_norm_takes_part():
     layer.q_norm.forward = torch.zeros_like
     with torch.no_grad():
         assert not layer(x).any()       # O = sum_e R_e (silu(0) * 0) V
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("norm", [lambda: RMSNorm((H, dh), 0.5), lambda: RMSNorm((dh,), 0.5), lambda: RMSNorm((dh,)), lambda: RMSNorm((1, dh), 0.5)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_head_norm_in_place_of_the_block_s_is_the_one_that_runs(norm, grad):
+    """Its epsilon (which outweighs the rows here) and its weight, in the block's node and in its steps, as in torch's operations."""
+    dev, (B, S) = "cuda:0", (2, 24)
+    layer = _make()
+    layer.q_norm = norm()
+    with torch.no_grad():
+        layer.q_norm.weight.uniform_(0.5, 1.5, generator=torch.Generator().manual_seed(2))
+    layer = layer.to(dev).to(torch.bfloat16)
+    x = (torch.randn(B, S, H * dh, generator=torch.Generator().manual_seed(1)) * 0.25).bfloat16().to(dev).requires_grad_(grad)
+    results = []
+    for how in ("block", "steps", "torch"):
+        if how == "steps":
+            layer.w_self.register_forward_hook(lambda *a: None)
+        layer.fused_prologue = how != "torch"
+        y = layer(x)
+        results.append([y, *torch.autograd.grad(y, [x, *layer.parameters()], torch.ones_like(y))] if grad else [y])
+    for a, b, ref in zip(*results):
+        for got in (a, b):
+            # the two sides round bfloat16 intermediates at other places (2^-9 each, some ten of them)
+            assert (got - ref).float().norm() <= 2e-2 * ref.float().norm()
