@@ -105,9 +105,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
         const long roff = (long)bc * JB * DH;
 #pragma unroll
         for (int k = 0; k < FILL; ++k) {
-            // (Without fillers `wave` is below NW as it is.  Masked, the compiler knows each instruction's matrix: 0.5 % faster with
-            // d_h 128, 2 x 1,500 tokens 109.6 -> 109.1 us; with 96 its code is 0.45 % slower, 16,384 tokens 148.4 -> 149.1.)
-            const int id = (FILLERS || DH == 128 ? wave & (NW - 1) : wave) + NW * k;
+            const int id = (FILLERS ? wave & (NW - 1) : wave) + NW * k;      // (the filling waves are numbered from NW on)
             const int which = id >> 3;
             const long toff = which == 0 ? 0 : (which == 1 ? offU : offV);
             const int region = which == 0 ? FWD_K0 : (which == 1 ? FWD_U0 : FWD_V0);
