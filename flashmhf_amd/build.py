@@ -171,35 +171,57 @@ def _registers(operand):
     return {(m[1], k) for k in range(int(lo), int(hi) + 1)}
 
 
-def reads_touched_in_flight(assembly):
-    """{kernel symbol: first such instruction} where an instruction uses a register that an LDS read in front of it (in the order of the
-    text) is still to fill.  LDS reads issued from inline assembly are waited for by count in inline assembly, too; between the two the
-    compiler may copy their registers, which it takes for filled: wrong values, depending on timing."""
-    found, kernel, in_flight = {}, None, []
+def _kernels(assembly):
+    """(symbol, [(opcode, operands, text)], {label: index into them}) of every kernel of an assembly listing."""
+    name = None
     for line in assembly:
-        m = re.match(r"(_Z\S+):", line)
-        if m:
-            kernel, in_flight = m[1], []
-        elif line.startswith(".Lfunc_end"):
-            kernel = None
         code = line.split(";")[0].strip()
-        if kernel is None or not code or code.startswith(".") or code.endswith(":"):
-            continue
-        op, _, rest = code.partition(" ")
-        if op == "s_waitcnt":
-            m = re.search(r"lgkmcnt\((\d+)\)", rest)
-            if m:                                   # LDS operations return in order
-                in_flight = in_flight[max(0, len(in_flight) - int(m[1])):]
-            continue
-        if op in ("s_branch", "s_endpgm"):
-            in_flight = []
-            continue
-        operands = [t.strip().split(" ")[0] for t in rest.split(",")]
-        used = set().union(*(_registers(t) for t in operands))
-        if any(r & used for r in in_flight):
-            found.setdefault(kernel, code)
-        if op.startswith("ds_"):
-            in_flight.append(_registers(operands[0]) if op.startswith("ds_read") else set())
+        if m := re.match(r"(_Z\S+):", line):
+            name, code_lines, labels = m[1], [], {}
+        elif name and line.startswith(".Lfunc_end"):
+            yield name, code_lines, labels
+            name = None
+        elif name and (m := re.match(r"(\.L\S+):", code)):
+            labels[m[1]] = len(code_lines)
+        elif name and code and not code.startswith(".") and not code.endswith(":"):
+            op, _, rest = code.partition(" ")
+            code_lines.append((op, rest.strip(), code))
+
+
+def reads_touched_in_flight(assembly):
+    """{kernel symbol: first such instruction} where an instruction uses a register that an LDS read in front of it, on any way through
+    the kernel, is still to fill.  LDS reads issued from inline assembly are waited for by count in inline assembly, too; between the two
+    the compiler may copy their registers, which it takes for filled: wrong values, depending on timing."""
+    found = {}
+    for kernel, code, labels in _kernels(assembly):
+        registers = [[_registers(t.strip().split(" ")[0]) for t in rest.split(",")] for _, rest, _ in code]
+        touched, seen, ways = set(), set(), [(0, ())]        # a way: where it goes on, the registers of each read in flight
+        while ways:
+            at, in_flight = ways.pop()
+            while at < len(code) and (at, in_flight) not in seen:
+                seen.add((at, in_flight))
+                if len(seen) > 1000 * (len(code) + 1):
+                    raise RuntimeError(f"too many ways through {kernel}")
+                op, rest, _ = code[at]
+                at += 1
+                if op == "s_endpgm":
+                    break
+                if op == "s_waitcnt":
+                    m = re.search(r"lgkmcnt\((\d+)\)", rest)
+                    if m:                                    # LDS operations return in order
+                        in_flight = in_flight[max(0, len(in_flight) - int(m[1])):]
+                elif op == "s_branch":
+                    at = labels.get(rest, len(code))
+                elif op.startswith("s_cbranch"):
+                    ways.append((labels.get(rest, len(code)), in_flight))
+                else:
+                    used = set().union(*registers[at - 1])
+                    if any(r & used for r in in_flight):
+                        touched.add(at - 1)
+                    if op.startswith("ds_"):
+                        in_flight = (*in_flight, frozenset(registers[at - 1][0]) if op.startswith("ds_read") else frozenset())[-64:]
+        if touched:
+            found[kernel] = code[min(touched)][2]
     return found
 
 

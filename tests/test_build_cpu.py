@@ -113,3 +113,33 @@ READ = """_Z6kernelv:
 def test_registers_of_reads_in_flight_are_found(between, left, found):
     got = build.reads_touched_in_flight(READ.format(between, left).splitlines())
     assert bool(got) is found and (not found or list(got) == ["_Z6kernelv"])
+
+
+LOOP = """_Z6kernelv:
+	ds_read_b32 v50, v1
+	s_waitcnt lgkmcnt(0)
+.LBB0_1:
+	v_add_f32_e32 v2, v2, v{used}
+	ds_read_b32 v50, v1
+	{wait}
+	s_cbranch_scc1 .LBB0_1
+	s_waitcnt lgkmcnt(0)
+	s_branch .LBB0_3
+.LBB0_2:
+	v_add_f32_e32 v2, v2, v50
+	s_endpgm
+.LBB0_3:
+	ds_read_b32 v50, v1
+	s_branch .LBB0_{target}
+.LBB0_4:
+	s_endpgm
+.Lfunc_end0:
+"""
+
+
+@pytest.mark.parametrize("used,wait,target,found", [(50, "s_nop 0", 4, "v_add_f32_e32 v2, v2, v50"), (51, "s_nop 0", 4, "ds_read_b32 v50, v1"),
+                                                    (50, "s_waitcnt lgkmcnt(0)", 4, None), (50, "s_waitcnt lgkmcnt(0)", 2, "v_add_f32_e32 v2, v2, v50")])
+def test_reads_in_flight_are_followed_over_branches(used, wait, target, found):
+    """Around a loop and through a jump, forwards and backwards in the text."""
+    got = build.reads_touched_in_flight(LOOP.format(used=used, wait=wait, target=target).splitlines())
+    assert got == ({} if found is None else {"_Z6kernelv": found})
