@@ -584,15 +584,16 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 }
 
 // Into how many parts the forward and the dQ/dR kernel cut the blocks of a head, and which of a kernel's tile heights runs.
-// The steps are measured times of each kernel on half a chip; a rows32 step is a trip of four blocks.
+// The steps are times of each kernel on half a chip, two of them of earlier forms of it (at each kernel's variants); a rows32 step is a
+// trip of four blocks.
 // One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute
 // units a part per idle unit shortens the serial walk over the blocks (one token of the 370M layer, 8 tiles of 121 blocks: 46 us
 // in one part, 7.8 in 31), and every part costs a set of fp32 sums that is written and read back.  Time of a launch in us:
 // rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing pass + 0.6 per MB
 // of sums; a step slows by up to `full` as the chip fills (power).  The prices are those of d_h = 128 for every d_h: with it the
-// variants of a kernel get cheaper together.  Against every tile height and 1 to 64 parts, measured on 336 bfloat16 calls (forward
-// and dQ/dR; d_h 64, 96, 128; four layers; 1 to 12,000 rows; profiles/pick_parts_sweep.csv) the pick is 1.3 % slower than
-// the fastest on average and 20 % at worst (dQ/dR of 64 rows of 4 heads of 96, 10.8 us against 8.9); by d_h at most 13, 20, 13 %.
+// variants of a kernel get cheaper nearly together.  Against every tile height and 1 to 64 parts, measured on 336 bfloat16 calls
+// (forward and dQ/dR; d_h 64, 96, 128; four layers; 1 to 12,000 rows; profiles/pick_parts_sweep.csv) the pick is 1.5 % slower than
+// the fastest on average and 23 % at worst (forward of 4,096 rows of 8 heads of 64, 45.8 us against 37.3); by d_h at most 23, 21, 18 %.
 // Not cut: more experts than one LDS window of gate values holds (bfloat16); and 16,384 rows per head or more, where a head
 // fills a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X

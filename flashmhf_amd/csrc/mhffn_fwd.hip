@@ -563,7 +563,8 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // instead of 1.0 (1,500 tokens of the 370M layer in one part: 130 us with 256 rows, 74 with 128; 733 tokens at each one's best number of
 // parts 32.6 and 29.8, of the 128M layer 25.2 and 20.6), and the two are level where every compute unit has one.  Of 32, four blocks a trip of 1.43 us, below that, where 128-row tiles take, at each one's best
 // number of parts: one token of the 370M layer 7.8 us against 10.0, 16 tokens of the 1.3B layer 20.3 against 22.5 (95 MB of
-// weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.
+// weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.  (Priced at 0.6 for 128 rows, as
+// before its filling waves: the line between the two kernels lies where it did.)
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
