@@ -511,6 +511,8 @@ Tensor block(const Tensor& x, const Tensor& w1, const std::optional<Tensor>& nor
         return block_forward(x, w1, nw, router, K, U, V, w2, eps, one_part, whose).Y;
     // With anything frozen (adapters, training of the experts alone) the steps record their own nodes: each saves what its
     // own gradients need, and what nobody asks for is neither kept nor computed.
+    // So with plain data for x: the node would keep w1 as well, which nothing but dx needs.  (17 us of host time on calls of a few rows,
+    // 116 against 99 us of a training call on 32 tokens; from 600 tokens on the GPU takes longer than either.)
     for (const Tensor* t : {&x, &w1, &nw, &router, &K, &U, &V, &w2})
         if (t->defined() && !t->requires_grad())
             return linear(stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose).reshape(x.sizes()), w2, whose);

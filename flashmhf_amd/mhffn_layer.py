@@ -163,7 +163,7 @@ class MHFFNLayer(nn.Module):
         if (self.fused_prologue and self.router_input == "q" and q.dtype == torch.bfloat16 and q.is_cuda
                 and E <= 64 and dh in (64, 96, 128)
                 and (norm is None or _runs_own_forward(norm, RMSNorm) and norm.weight.shape == (H, dh) and not (dh == 128 and E > 32))):
-            return head_norm_gate(q, None if norm is None else norm.weight, self.router, self._head_norm_eps())
+            return head_norm_gate(q, None if norm is None else norm.weight, self.router, self.rms_norm_eps if norm is None else norm.eps)
         if self.q_norm is not None:
             q = self.q_norm(q)
         Q = q.transpose(1, 2)                                       # a view: the kernels read token-major rows
@@ -172,10 +172,6 @@ class MHFFNLayer(nn.Module):
         else:
             logits = (x.float() @ self.w_router.float()).view(B, S, H, E).transpose(1, 2)
         return Q, router_gate(logits).contiguous()
-
-    def _head_norm_eps(self):
-        """That of the norm in place, which may be another than the block was made with."""
-        return self.rms_norm_eps if self.q_norm is None else self.q_norm.eps
 
     def _stock_steps(self):
         """The tensors of the block (projection, head norm's weight or None, router, K, U, V, output projection) where every
@@ -221,7 +217,8 @@ class MHFFNLayer(nn.Module):
             m = self._modules
             cls = type(m["w_self"])
             products = cls.products if cls is type(m["w_self_2"]) and cls is not nn.Linear else 0
-            return _capi.native().block(x, *weights, self._head_norm_eps(), m["op"].one_part, products)
+            eps = self.rms_norm_eps if weights[1] is None else (m["q_norm"] if "q_norm" in m else self.q_norm).eps
+            return _capi.native().block(x, *weights, eps, m["op"].one_part, products)
         Q, R = self.heads_and_gate(x)
         O = self.op(Q, self.K.to(Q.dtype), self.U.to(Q.dtype), self.V.to(Q.dtype), R)
         return self.w_self_2(O.transpose(1, 2).reshape(B, S, hid))  # token-major O: the reshape is a view
