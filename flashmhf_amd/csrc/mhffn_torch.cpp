@@ -339,8 +339,8 @@ bool plain(const Tensor& t)
 // 17 to 8,192 rows: the library splits the summed index, or adds in another order,
 //   NT  below 32 rows, and with more than 1,024 of the summed index only where there are no more than 2^18 results
 //   NN  at 16 rows and fewer, and with more than 1,024 of the summed index only where there are no more than 2^18 results
-//   TN  for 16 rows and fewer, and for more than 16,384.  Above them the sum stays in order here: the gradient of a weight goes into
-//       no other layer's (hidden 1024, 32,768 rows: 128 us, the library's 198).
+//   TN  of 16 rows and fewer, and of more than 16,384 (compared to 32,768).  Those of more stay here, in order: the gradient of a
+//       weight goes into no other layer's (hidden 1024, 32,768 rows: 128 us, the library's 198).
 // It is a table of another library's choices, not a promise of it: tests/test_gpu_product.py compares.
 enum Whose { LIBRARY = 0, OWN = 1, OWN_IN_ORDER = 2 };
 bool library_in_order(int form, int64_t M, int64_t N, int64_t K)
