@@ -1,23 +1,26 @@
-// fp32 instantiation of the fused multi-head FFN (forward, dQ/dR, dK/dU/dV), on the fp32 matrix instructions: operands,
-// products and sums are float32 and the sigmoid is exact, so results track an fp32 eager evaluation to ~1e-6.  Same fusion
-// as the bf16 kernels -- the [tokens, E*d_e] intermediate exists only in registers.  Generic in d_h (multiple of 8, at most
-// 128; CT = 32-column tiles of it), d_e and E.
+// fp32 instantiation of the fused multi-head FFN (forward, dQ/dR, dK/dU/dV): operands, products and sums are float32 and the
+// sigmoid is exact, so results track an fp32 eager evaluation to ~1e-6.  Same fusion as the bf16 kernels -- the
+// [tokens, E*d_e] intermediate exists only in registers.  Generic in d_h (multiple of 8, at most 128; CT = 32-column tiles of
+// it), d_e and E.
 // Formulas: models/flashmhf/modeling_mhffnmoe.py:418-427 (forward), kernels/triton/flash_mlp_moe.py:401-414, 527-542,
 // 720-729 (backward).
 //
-// All products are v_mfma_f32_32x32x2_f32, D = A(32x2) * B(2x32) + C, 64 cycles each:
+// The products run on v_mfma_f32_32x32x16_bf16 with every operand taken apart into three bfloat16 values ("planes", below);
+// operand layouts are those of mhffn_common.hpp.  dK/dU/dV for d_h > 96, whose planes do not fit a wave's registers, keeps
+// v_mfma_f32_32x32x2_f32, D = A(32x2) * B(2x32) + C, 64 cycles each:
 //       A: lane l holds row (l % 32), k = l / 32         B: lane l holds col (l % 32), k = l / 32
 //       C/D: lane l holds col (l % 32), register i holds row 8*(i/4) + 4*(l/32) + (i%4)
 // * First products contract over the head dim.  The order of the k index is free as long as A and B agree: with lane group
 //   g = l / 32 holding columns 8m + 4g .. +3, one 16-byte read of each operand row feeds four instructions.
-// * They are written with rows = j (weight rows) and columns = tokens (in dK/dU/dV: rows = tokens, columns = j), so that
-//   register i of the result is, as it stands, the B operand of the second products' step i: k slot g is row
-//   8*(i/4) + 4g + i%4.  The A operand of that step is one row of V (K, U; Q, dO) per lane group, read along its columns.
+// * They are written with rows = tokens, columns = j, so that register i of the result is, as it stands, the B operand of the
+//   second products' step i: k slot g is row 8*(i/4) + 4g + i%4.  The A operand of that step is one row of Q (dO) per lane
+//   group, read along its columns.
 //
-// What bounds them: the matrix pipe (an instruction moves 2 operand rows per 64 cycles, so LDS and L2 are idle most of the
-// time; 153 TFLOP/s is what a large library product reaches on the card).  256 tokens of the 128M layer, forward + backward:
-// 6.0 ms with plain FMAs on 32-token tiles of one workgroup each, the whole E * d_e axis in series; see the launchers for
-// how the work is spread over the chip now.
+// What bounds them.  256 tokens of the 128M layer took 30 (forward), 45 (dQ/dR) and 61 us (dK/dU/dV) on the fp32 matrix
+// instructions, whose time a kernel's four waves could not go below (15, 26 and 31 us, 153 TFLOP/s over the chip) and under which
+// they issue next to nothing else.  The planes take 2.7 times less matrix time and some VALU instructions per operand and
+// element, put between the matrix instructions where registers allow: 24, 34 and 47 us; per 32 rows of weights (forward, dQ/dR;
+// 128 rows) 5.2 -> 2.2 and 8.2 -> 4.2 us, per 32 tokens (dK/dU/dV, two tiles) 11.2 -> 6.6, the rest is prologue and epilogue.
 #include "mhffn_common.hpp"
 
 namespace mhffn {
@@ -36,7 +39,13 @@ struct F32Args {
 };
 
 __device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + __expf(-x)); }
+// 1 / (1 + e^-x): the reciprocal with one Newton step (an IEEE division takes three times the instructions), at least 2^-126 (the
+// step would make NaN of an infinite e^-x)
+__device__ __forceinline__ float sigmoid_exact(float x)
+{
+    const float d = 1.0f + __builtin_amdgcn_exp2f(fminf(-LOG2E * x, 126.0f)), y = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, y, 1.0f), y, y);
+}
 __device__ __forceinline__ f32x16 zero16()
 {
     f32x16 z;
@@ -163,6 +172,216 @@ __device__ __forceinline__ void store_row(const f32x16 (&acc)[CT], float* dst, i
             }
 }
 
+// ---- float32 operands on the bf16 matrix instructions -----------------------------------------------------------------
+// A float32 value is the exact sum of three bfloat16 values (8 + 8 + 8 bits: the upper half of its pattern, then the rest
+// rounded, then what is left).  Of the nine products of two such sums the six of the largest terms run on
+// v_mfma_f32_32x32x16_bf16, which has sixteen times the rate of v_mfma_f32_32x32x2_f32; the three left out are at most 2^-23
+// of the product, 2^-26 on average and of either sign, below what one float32 addition rounds away.  A sum over k then rounds once
+// per sixteen terms and plane instead of once per two: against 64 bits the results are 10 to 30 % closer than those of the fp32
+// instructions (32 to 1,024 tokens, d_h 24 to 128; O 3.5e-7 -> 2.7e-7, dQ 4.0 -> 3.4, dK, dU, dV 3.4 -> 2.8, dR 3.7 -> 3.0 for
+// 256 tokens of the 128M layer).  The matrix instructions take a plane below 2^-126 for zero, so an operand counts to
+// 2^-126 absolutely (values below 2^-110 lose their last bits).  An infinity or NaN in an operand makes every sum that it enters
+// infinite or NaN; an infinity comes out as NaN where it meets a zero plane.
+constexpr int PLANE_B = TILE_B;                 // one plane of a 32-row tile, in the layout of the bf16 kernels' tiles
+constexpr int PLANES_B = 3 * PLANE_B;
+
+// the pair (x0, x1) as three packed pairs of bfloat16, largest first
+__device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned& m, unsigned& l)
+{
+    typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+    const unsigned b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
+    h = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+    const float r0 = x0 - __uint_as_float(b0 & 0xffff0000u), r1 = x1 - __uint_as_float(b1 & 0xffff0000u);
+    m = __builtin_bit_cast(unsigned, bf16x2{(bf16_t)r0, (bf16_t)r1});
+    asm("" : "+v"(m));      // (or the compiler rounds r0 a second time instead of shifting the pair)
+    l = __builtin_bit_cast(unsigned, bf16x2{(bf16_t)(r0 - __uint_as_float(m << 16)), (bf16_t)(r1 - __uint_as_float(m & 0xffff0000u))});
+}
+struct Split8 {
+    bf16x8 p[3];
+};
+// 16 bytes per lane from src to dst + 16 lane, asynchronously and without the compiler's knowledge, which would put a wait for it in
+// front of every LDS read behind it.
+template <int IMM>
+__device__ __forceinline__ void lds_direct16(const float* src, unsigned char* dst)
+{
+    // (the instruction's offset counts at both ends)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(src), "s"(lds_addr(dst) - IMM), "n"(IMM) : "memory");
+}
+// pair I of eight values: the planes' registers I
+template <int I, class V>
+__device__ __forceinline__ void split8_pair(u32x4 (&v)[3], V&& x)
+{
+    unsigned h, m, l;
+    split2(x(2 * I), x(2 * I + 1), h, m, l);
+    v[0][I] = h; v[1][I] = m; v[2][I] = l;
+}
+__device__ __forceinline__ Split8 split8_of(const u32x4 (&v)[3])
+{
+    return Split8{{__builtin_bit_cast(bf16x8, v[0]), __builtin_bit_cast(bf16x8, v[1]), __builtin_bit_cast(bf16x8, v[2])}};
+}
+template <class V>
+__device__ __forceinline__ Split8 split8(V&& x)      // x(0) .. x(7)
+{
+    u32x4 v[3];
+    static_for<4>([&](auto ic) { split8_pair<decltype(ic)::value>(v, x); });
+    return split8_of(v);
+}
+// the planes of the six products, smallest terms first
+constexpr int SPLIT_A[6] = {2, 0, 1, 1, 0, 0}, SPLIT_B[6] = {0, 2, 1, 0, 1, 0};
+
+// four values taken apart, two at a time
+struct CutPiece {
+    u32x2 h, m, l;
+    template <int I>
+    __device__ __forceinline__ void half(const f32x4& x)
+    {
+        unsigned a, b, c;
+        split2(x[2 * I], x[2 * I + 1], a, b, c);
+        h[I] = a; m[I] = b; l[I] = c;
+    }
+};
+// A thread of a team of 256 that takes 32 rows x 32 CT columns of weights apart: row t / 8, columns 32 k + 4 (t % 8) .. + 3.
+template <int CT>
+struct Cut {
+    int row, col, at;                      // at: byte in a plane, column group 0 (column group k: at ^ (k << 6))
+    __device__ explicit Cut(int t) : row(t >> 3), col(4 * (t & 7)), at((t >> 3) * TILE_ROW_B + ((((t & 7) >> 1) ^ swz16(t >> 3)) << 4) + 8 * (t & 1)) {}
+    // W: first row of the tile, of which `rows` exist; the columns beyond d_h are zero
+    __device__ void load(f32x4 (&x)[CT], const float* W, int rows, int DH) const
+    {
+        const float* src = W + (row < rows ? row : rows - 1) * DH + col;
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+            x[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (32 * k + col < DH) x[k] = *reinterpret_cast<const f32x4*>(src + 32 * k);
+        }
+    }
+    __device__ void store(unsigned char* planes, int k, const f32x4& x) const
+    {
+        CutPiece c;
+        c.half<0>(x);
+        c.half<1>(x);
+        store(planes, k, c);
+    }
+    __device__ void store(unsigned char* planes, int k, const CutPiece& c) const
+    {
+        unsigned char* d = planes + (at ^ (k << 6));
+        *reinterpret_cast<u32x2*>(d) = c.h;
+        *reinterpret_cast<u32x2*>(d + PLANE_B) = c.m;
+        *reinterpret_cast<u32x2*>(d + 2 * PLANE_B) = c.l;
+    }
+};
+// Per-lane byte offsets of the reads of a plane: by rows (k-step ks: row ^ (ks << 5)) and by columns (column tile ct, 16 rows s:
+// (col ^ (ct << 6)) + 4096 s).
+struct PlaneLane {
+    int row, col[2];
+    __device__ explicit PlaneLane(int lane)
+    {
+        const int r = row_perm32(lane & 31);
+        const TrLane<1> t = make_tr_lane<1, 8, 4>(lane);
+        row = r * TILE_ROW_B + (((lane >> 5) ^ swz16(r)) << 4);
+        col[0] = t.off[0][0]; col[1] = t.off[0][1];
+    }
+};
+// row of the weight tile that register i of a first product holds
+__device__ __forceinline__ int split_row(int i, int g) { return 16 * (i >> 3) + 8 * g + (i & 7); }
+
+struct Operand {
+    bf16x8 p[3];
+};
+__device__ __forceinline__ Operand read_rows(const unsigned char* planes, const PlaneLane& l, int ks)
+{
+    Operand a;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) a.p[x] = *reinterpret_cast<const bf16x8*>(planes + (l.row ^ (ks << 5)) + x * PLANE_B);
+    return a;
+}
+__device__ __forceinline__ Operand read_cols(const unsigned char* planes, const PlaneLane& l, int ct, int s)
+{
+    typedef __attribute__((address_space(3))) v4bf16_t* lds_v4;
+    Operand a;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        const v4bf16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4)(planes + (l.col[0] ^ (ct << 6)) + 4096 * s + x * PLANE_B));
+        const v4bf16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4)(planes + (l.col[1] ^ (ct << 6)) + 4096 * s + x * PLANE_B));
+        a.p[x] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    return a;
+}
+// d[k] = rows of the planes of a tile times this lane's row v[k].  The first SHARED products take the first tile (planes), every
+// further one the next.  ACC(k, plane): that plane of v[k] is kept in accumulation registers.  slot(i) runs behind the i-th of the
+// 12 CT N matrix instructions.  The results are architectural registers and need mfma_result_fence before the VALU reads them.
+template <int CT, int N, int SHARED, class Acc, class Slot>
+__device__ __forceinline__ void first_split(f32x16 (&d)[N], const unsigned char* planes, const Split8* const (&v)[N], const PlaneLane& l,
+                                            Acc, Slot&& slot)
+{
+    constexpr int T = N - SHARED + 1;
+    Operand a[2];
+    a[0] = read_rows(planes, l, 0);
+    static_for<2 * CT * T>([&](auto uc) {
+        constexpr int u = decltype(uc)::value, n = u + 1, ks = u / T, k0 = u % T ? u % T + SHARED - 1 : 0, kn = u % T ? 1 : SHARED;
+        if constexpr (n < 2 * CT * T) a[n & 1] = read_rows(planes + (n % T) * PLANES_B, l, n / T);
+        static_for<6 * kn>([&](auto xc) {
+            constexpr int x = decltype(xc)::value / kn, k = k0 + decltype(xc)::value % kn;
+            const bf16x8 w = a[u & 1].p[SPLIT_A[x]], q = v[k][ks].p[SPLIT_B[x]];
+            if constexpr (Acc{}(k, SPLIT_B[x])) {
+                if constexpr (ks == 0 && x == 0) mfma32_vgpr_first_bacc(d[k], w, q);
+                else mfma32_vgpr_acc_bacc(d[k], w, q);
+            } else {
+                if constexpr (ks == 0 && x == 0) mfma32_vgpr_first(d[k], w, q);
+                else mfma32_vgpr_acc(d[k], w, q);
+            }
+            slot(std::integral_constant<int, 6 * (N * ks + k0) + decltype(xc)::value>{});
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+struct NoAcc {
+    constexpr bool operator()(int, int) const { return false; }
+};
+struct AllAcc {
+    constexpr bool operator()(int, int) const { return true; }
+};
+// dK/dU/dV: K and the last plane of U beside the accumulators of the gradients
+struct WeightAcc {
+    constexpr bool operator()(int k, int plane) const { return k == 0 || (k == 1 && plane == 2); }
+};
+// acc[ct] += columns 32 ct + l32 of the planes' rows 16 s .. + 15 times b.  slot(i) runs behind the i-th of the 6 CT matrix
+// instructions.
+template <int CT, class Slot>
+__device__ __forceinline__ void second_split(f32x16 (&acc)[CT], const unsigned char* planes, int s, const Split8& b, const PlaneLane& l,
+                                             Slot&& slot)
+{
+    Operand a[2];
+    a[0] = read_cols(planes, l, 0, s);
+    static_for<CT>([&](auto cc) {
+        constexpr int ct = decltype(cc)::value;
+        if constexpr (ct + 1 < CT) a[(ct + 1) & 1] = read_cols(planes, l, ct + 1, s);
+        static_for<6>([&](auto xc) {
+            constexpr int x = decltype(xc)::value;
+            acc[ct] = mfma32(a[ct & 1].p[SPLIT_A[x]], b.p[SPLIT_B[x]], acc[ct]);
+            slot(std::integral_constant<int, 6 * ct + x>{});
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+// This lane's row as B operands of the first products, zero beyond d_h: its values, then their planes.
+template <int CT>
+__device__ __forceinline__ void load_row_operand(f32x4 (&x)[4 * CT], const float* row, int g, int DH)
+{
+#pragma unroll
+    for (int i = 0; i < 4 * CT; ++i) {
+        const int c = 16 * (i >> 1) + 8 * g;
+        x[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < DH) x[i] = *reinterpret_cast<const f32x4*>(row + c + 4 * (i & 1));
+    }
+}
+template <int CT>
+__device__ __forceinline__ void split_row_operand(Split8 (&v)[2 * CT], const f32x4 (&x)[4 * CT])
+{
+#pragma unroll
+    for (int ks = 0; ks < 2 * CT; ++ks) v[ks] = split8([&](int i) { return x[2 * ks + (i >> 2)][i & 3]; });
+}
+
 // Workgroup of the forward and of dQ/dR: 4 waves of 32 rows of one K/U/V head, one part of the head's blocks.
 struct Place {
     int hk, z, row0, row, blk0, nblk;      // row0: this wave's first row of the list, row: this lane's (clamped into the list)
@@ -192,132 +411,452 @@ struct Block {
     }
 };
 
-// Forward.  LDS: K and U tiles of two blocks, V tile of one (80 KB for d_h > 64, so that two workgroups share a CU and one's
-// element-wise code and barriers lie under the other's matrix instructions).
-template <int CT>
-__global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args p)
+// Forward: 128 rows, GROUPS teams of four waves that take the blocks of the part in turn, their sums added at the end.  A team's
+// threads take the next block's weights apart on their way from memory to LDS, K and U under the second products, V under the first.
+template <int CT, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, GROUPS) void fwd_f32_kernel(F32Args p)
 {
-    using T = Tile<CT>;
-    constexpr int FI = T::INS / 4 > 0 ? T::INS / 4 : 1;      // fill instructions per wave and tile
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Place w(p, wave, l32);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = wave >> 2;
+    const Place w(p, wave & 3, l32);
     const int DH = p.DH;
+    const Cut<CT> cut(threadIdx.x & 255);
+    const PlaneLane pl(lane);
+    unsigned char* planes = lds + group * 3 * PLANES_B;      // K, U, V
 
-    auto fill = [&](const float* W, int blk, unsigned char* tile) {
-        const Block b(p, w.hk, w.blk0 + (blk < w.nblk ? blk : w.nblk - 1));
-#pragma unroll
-        for (int k = 0; k < FI; ++k)
-            T::fill(tile, wave * FI + k, lane, DH, [&](int r) { return W + (b.wrow + (r < b.rows ? r : b.rows - 1)) * DH; });
-    };
-    unsigned char* sV = lds + 4 * T::BYTES;
-    fill(p.K, 0, lds);
-    fill(p.U, 0, lds + T::BYTES);
-    f32x4 q[4 * CT];
-    load_row<CT>(q, p.Q + p.rows.tok(w.hk, w.row) * DH, g, DH);
+    auto block = [&](int it) { return Block(p, w.hk, w.blk0 + (it * GROUPS + group < w.nblk ? it * GROUPS + group : w.nblk - 1)); };
+    f32x4 xk[CT], xu[CT], xv[CT];
+    {
+        const Block b = block(0);
+        cut.load(xk, p.K + b.wrow * DH, b.rows, DH);
+        cut.load(xu, p.U + b.wrow * DH, b.rows, DH);
+        cut.load(xv, p.V + b.wrow * DH, b.rows, DH);
+    }
+    f32x4 qx[4 * CT];
+    load_row_operand<CT>(qx, p.Q + p.rows.tok(w.hk, w.row) * DH, g, DH);
+    Split8 q[2 * CT];
+    split_row_operand<CT>(q, qx);
     const float* rrow = p.R + p.rows.gate(w.hk, w.row) * p.parts.E;
-
     f32x16 o[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) o[ct] = zero16();
-    for (int blk = 0; blk < w.nblk; ++blk) {
-        const Block b(p, w.hk, w.blk0 + blk);
-        const unsigned char *sK = lds + (blk & 1) * 2 * T::BYTES, *sU = sK + T::BYTES;
-        const float r = rrow[b.e];
-        wait_vmcnt<0>();      // K and U of this block have landed
-        __syncthreads();      // ... for every wave, and every wave is done with the block before
-        fill(p.V, blk, sV);
-        fill(p.K, blk + 1, lds + (~blk & 1) * 2 * T::BYTES);
-        fill(p.U, blk + 1, lds + (~blk & 1) * 2 * T::BYTES + T::BYTES);
-        f32x16 mn[2];
-        const typename T::Lane l(l32, g);
-        first_products<CT, 2>(mn, {sK, sU}, {q, q}, l);
-        f32x16 &m = mn[0], &n = mn[1];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            // (computed for the rows that a short block lacks too: hidden from the compiler, or it makes a branch of each element,
-            // and fp32 matrix instructions leave no time under them: 1,024 rows of 8 heads of 128 224 us, now 216)
-            float v = m[i] * sigmoid_exact(m[i]) * n[i] * r;
-            asm volatile("" : "+v"(v));
-            m[i] = reg_row(i, g) < b.rows ? v : 0.0f;
-        }
-        wait_vmcnt<2 * FI>();      // V has landed (the next block's K and U may be in flight)
-        __syncthreads();
-        second_product<CT>(o, sV, m, l);
+    for (int k = 0; k < CT; ++k) {
+        cut.store(planes, k, xk[k]);
+        cut.store(planes + PLANES_B, k, xu[k]);
     }
-    wait_vmcnt<0>();
+    const int iters = (w.nblk + GROUPS - 1) / GROUPS;
+    Block b = block(0);
+    float r = group < w.nblk ? rrow[b.e] : 0.0f;      // (0 removes the block that a team lacks in the last turn)
+    if (group == 1) {
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(2);
+    }
+    for (int it = 0; it < iters; ++it) {
+        const Block next = block(it + 1);
+        __syncthreads();      // K and U are there, and V has been read
+        const float rnext = (it + 1) * GROUPS + group < w.nblk ? rrow[next.e] : 0.0f;
+        cut.load(xk, p.K + next.wrow * DH, next.rows, DH);
+        cut.load(xu, p.U + next.wrow * DH, next.rows, DH);
+        f32x16 mn[2];
+        first_split<CT, 2, 1>(mn, planes, {q, q}, pl, NoAcc{}, [&](auto ic) {
+            constexpr int i = decltype(ic)::value, k = i / 24;      // 24 CT instructions, CT pieces
+            if constexpr (i % 24 == 11) cut.store(planes + 2 * PLANES_B, k, xv[k]);
+        });
+        __syncthreads();      // V is there, and K and U have been read
+        cut.load(xv, p.V + next.wrow * DH, next.rows, DH);
+        f32x16 &m = mn[0], &n = mn[1];
+        mfma_result_fence(m, n);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m[i] *= sigmoid_exact(m[i]) * n[i] * r;
+        if (b.rows < JB) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m[i] = split_row(i, g) < b.rows ? m[i] : 0.0f;
+        }
+        static_for<2>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            const Split8 ps = split8([&](int i) { return m[8 * s + i]; });
+            second_split<CT>(o, planes + 2 * PLANES_B, s, ps, pl, [&](auto ic) {
+                constexpr int i = decltype(ic)::value, k = i / 6;
+                if constexpr (i % 6 == 5) cut.store(planes + s * PLANES_B, k, s ? xu[k] : xk[k]);
+            });
+        });
+        b = next;
+        r = rnext;
+    }
+    if (GROUPS > 1 && group == 0) __syncthreads();
+    if (GROUPS > 1) {
+        __syncthreads();
+        float* xch = reinterpret_cast<float*>(lds) + (wave & 3) * (CT * 16 * 64) + lane;
+        if (group == 1) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) xch[(ct * 16 + i) * 64] = o[ct][i];
+        }
+        __syncthreads();
+        if (group == 1) return;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[ct][i] += xch[(ct * 16 + i) * 64];
+    }
     if (w.valid)
         store_row<CT>(o, p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * DH
                                             : p.O + p.rows.tok(w.hk, w.row) * DH, g, DH);
 }
 
-// dQ and dR.  LDS: K, U and V tiles of one block; the second workgroup of the CU covers the wait for the next.  (d_h > 96
-// takes more than half the register file: one workgroup.)
+// dQ and dR: four waves of 32 rows, alone on their SIMDs.  LDS: the planes of two blocks; the next block's weights are taken apart
+// between the matrix instructions of this block's first products, and the element-wise code of its second half of rows between
+// those of the second products of the first.
 template <int CT>
-__global__ __launch_bounds__(256, CT > 3 ? 1 : 2) void dqdr_f32_kernel(F32Args p)
+__global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
 {
-    using T = Tile<CT>;
-    constexpr int FI = T::INS / 4 > 0 ? T::INS / 4 : 1;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Place w(p, wave, l32);
     const int DH = p.DH, E = p.parts.E;
-    const unsigned char *sK = lds, *sU = lds + T::BYTES, *sV = lds + 2 * T::BYTES;
+    const Cut<CT> cut(threadIdx.x);
+    const PlaneLane pl(lane);
 
+    f32x4 x[3][CT];
+    auto load = [&](int blk) {
+        const Block b(p, w.hk, w.blk0 + (blk < w.nblk ? blk : w.nblk - 1));
+        cut.load(x[0], p.K + b.wrow * DH, b.rows, DH);
+        cut.load(x[1], p.U + b.wrow * DH, b.rows, DH);
+        cut.load(x[2], p.V + b.wrow * DH, b.rows, DH);
+    };
+    load(0);
     const long tok = p.rows.tok(w.hk, w.row) * DH;
-    f32x4 q[4 * CT], go[4 * CT];
-    load_row<CT>(q, p.Q + tok, g, DH);
-    load_row<CT>(go, p.dO + tok, g, DH);
+    Split8 q[2 * CT], go[2 * CT];
+    {
+        f32x4 qx[4 * CT], gx[4 * CT];
+        load_row_operand<CT>(qx, p.Q + tok, g, DH);
+        load_row_operand<CT>(gx, p.dO + tok, g, DH);
+        split_row_operand<CT>(q, qx);
+        split_row_operand<CT>(go, gx);
+    }
+    if (CT < 4) {      // (held there over the loop; with 64 registers more the compiler does better by itself)
+#pragma unroll
+        for (int ks = 0; ks < 2 * CT; ++ks)
+#pragma unroll
+            for (int x = 0; x < 3; ++x) asm volatile("" : "+a"(q[ks].p[x]), "+a"(go[ks].p[x]));
+    }
     const float* rrow = p.R + p.rows.gate(w.hk, w.row) * E;
     const long hrows = (long)p.rows.Hkuv * p.rows.n;
     float* drow = p.parts.nsplit > 1 ? p.part + p.parts.nsplit * hrows * DH + (w.z * hrows + (long)w.hk * p.rows.n + w.row) * E
                                      : p.dR + p.rows.gate(w.hk, w.row) * E;
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int k = 0; k < CT; ++k) cut.store(lds + t * PLANES_B, k, x[t][k]);
+    load(1);
 
     f32x16 dq[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) dq[ct] = zero16();
     float dr = 0.0f;
+    Block b(p, w.hk, w.blk0);
+    float r = rrow[b.e];
     for (int blk = 0; blk < w.nblk; ++blk) {
-        const Block b(p, w.hk, w.blk0 + blk);
-        const float r = rrow[b.e];
-        __syncthreads();      // every wave is done with the block before
-        int lane = threadIdx.x & 63;
-        asm volatile("" : "+v"(lane));      // (the fills' addresses are not worth a register each)
-#pragma unroll
-        for (int k = 0; k < FI; ++k) {
-            auto row = [&](const float* W) {
-                return [&, W](int rr) { return W + (b.wrow + (rr < b.rows ? rr : b.rows - 1)) * DH; };
-            };
-            T::fill(lds, wave * FI + k, lane, DH, row(p.K));
-            T::fill(lds + T::BYTES, wave * FI + k, lane, DH, row(p.U));
-            T::fill(lds + 2 * T::BYTES, wave * FI + k, lane, DH, row(p.V));
-        }
-        wait_vmcnt<0>();
-        __syncthreads();
+        const Block next(p, w.hk, w.blk0 + (blk + 1 < w.nblk ? blk + 1 : blk));
+        const float rnext = rrow[next.e];
+        const unsigned char* planes = lds + (blk & 1) * 3 * PLANES_B;
+        unsigned char* other = lds + (~blk & 1) * 3 * PLANES_B;
+        __syncthreads();      // this block's planes are there, and the other ones have been read
         f32x16 mna[3];
-        const typename T::Lane l(l32, g);
-        first_products<CT, 3>(mna, {sK, sU, sV}, {q, q, go}, l);
+        CutPiece c;
+        first_split<CT, 3, 1>(mna, planes, {q, q, go}, pl, AllAcc{}, [&](auto ic) {
+            constexpr int i = decltype(ic)::value, t = i / 12 / CT, k = i / 12 % CT;      // 36 CT instructions, 3 CT pieces
+            if constexpr (i % 12 == 3) c.half<0>(x[t][k]);
+            if constexpr (i % 12 == 6) c.half<1>(x[t][k]);
+            if constexpr (i % 12 == 9) cut.store(other + t * PLANES_B, k, c);
+        });
+        load(blk + 2);
         f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
+        mfma_result_fence(m, n, da);
+        if (b.rows < JB) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const float sg = sigmoid_exact(m[i]), sl = m[i] * sg;
-            const float a = reg_row(i, g) < b.rows ? da[i] : 0.0f;
-            dr = fmaf(a * sl, n[i], dr);
-            m[i] = r * a * n[i] * (sg + sl * (1.0f - sg));      // dM
-            n[i] = r * a * sl;                                  // dN
+            for (int i = 0; i < 16; ++i) da[i] = split_row(i, g) < b.rows ? da[i] : 0.0f;
         }
-        second_product<CT>(dq, sK, m, l);
-        second_product<CT>(dq, sU, n, l);
-        if (blk + 1 == w.nblk || Block(p, w.hk, w.blk0 + blk + 1).e != b.e) {
+        float sg;
+        auto sigma = [&](int i) { sg = sigmoid_exact(m[i]); };
+        auto element = [&](int i) {
+            const float sl = m[i] * sg, a = da[i] * sl, ra = r * da[i];
+            dr = fmaf(a, n[i], dr);
+            m[i] = ra * n[i] * fmaf(sl, 1.0f - sg, sg);         // dM
+            n[i] = r * a;                                       // dN
+        };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            sigma(i);
+            element(i);
+        }
+        // The second products of the first eight rows; behind their matrix instructions the rest of the element-wise code.
+        u32x4 dm[3], dn[3], dm1[3];
+        static_for<4>([&](auto ic) { split8_pair<decltype(ic)::value>(dm, [&](int i) { return m[i]; }); });
+        second_split<CT>(dq, planes, 0, split8_of(dm), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 4) split8_pair<i>(dn, [&](int j) { return n[j]; });
+            else if constexpr (i < 8 || (i < 16 && CT > 2)) {
+                if constexpr (i & 1) element(8 + (i - 4) / 2);
+                else sigma(8 + (i - 4) / 2);
+            }
+        });
+        constexpr int DONE = CT == 1 ? 9 : CT == 2 ? 10 : 14;      // (6, 12 or 18 instructions and more)
+        second_split<CT>(dq, planes + PLANES_B, 0, split8_of(dn), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 2 * (16 - DONE)) {
+                if constexpr (i & 1) element(DONE + i / 2);
+                else sigma(DONE + i / 2);
+            } else if constexpr (i < 2 * (16 - DONE) + 4) split8_pair<i - 2 * (16 - DONE)>(dm1, [&](int j) { return m[8 + j]; });
+        });
+        static_for<16>([&](auto ic) {      // (what d_h < 96 leaves)
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i >= DONE + 3 * CT) {
+                sigma(i);
+                element(i);
+            }
+        });
+        if constexpr (6 * CT < 2 * (16 - DONE) + 4) static_for<4>([&](auto ic) { split8_pair<decltype(ic)::value>(dm1, [&](int j) { return m[8 + j]; }); });
+        second_split<CT>(dq, planes, 1, split8_of(dm1), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 4) split8_pair<i>(dn, [&](int j) { return n[8 + j]; });
+        });
+        second_split<CT>(dq, planes + PLANES_B, 1, split8_of(dn), pl, [](auto) {});
+        if (blk + 1 == w.nblk || next.e != b.e) {
             const float tot = dr + __shfl_xor(dr, 32);      // the two lane halves hold different rows j of the same token
             if (g == 0 && w.valid) drow[b.e] = tot;
             dr = 0.0f;
         }
+        b = next;
+        r = rnext;
     }
     if (w.valid)
         store_row<CT>(dq, p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * DH : p.dQ + tok, g, DH);
+}
+
+// End of a dK/dU/dV kernel: the odd tiles' sums to the wave with the even ones, one gradient at a time (64 lanes x 16 CT floats,
+// lane-private), then to memory.  (This lane's row and the bounds of its columns are worked out again, out of the compiler's
+// sight: kept over the loop they are the few registers too many that made it spill for d_h > 96.)
+template <int CT>
+__device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned char* lds, f32x16 (&dk)[CT], f32x16 (&du)[CT], f32x16 (&dv)[CT])
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
+    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
+    const int blk = blockIdx.x * 2 + bw;
+    const Block b(p, hk, blk < nblk ? blk : nblk - 1);
+    __syncthreads();
+    int lane = threadIdx.x & 63, DH = p.DH;
+    asm volatile("" : "+v"(lane), "+s"(DH));
+    const int l32 = lane & 31, g = lane >> 5;
+    float* xch = reinterpret_cast<float*>(lds) + bw * (3 * CT * 16 * 64) + lane;
+    if (half == 1) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                xch[(ct * 16 + i) * 64] = dk[ct][i];
+                xch[((CT + ct) * 16 + i) * 64] = du[ct][i];
+                xch[((2 * CT + ct) * 16 + i) * 64] = dv[ct][i];
+            }
+    }
+    __syncthreads();
+    if (half == 1 || blk >= nblk || l32 >= b.rows) return;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            dk[ct][i] += xch[(ct * 16 + i) * 64];
+            du[ct][i] += xch[((CT + ct) * 16 + i) * 64];
+            dv[ct][i] += xch[((2 * CT + ct) * 16 + i) * 64];
+        }
+    const long wrow = b.wrow + l32, wsz = (long)p.rows.Hkuv * E * p.de * DH;
+    auto store_bf16 = [&](const f32x16(&acc)[CT], void* out) {
+        bf16_t* dst = static_cast<bf16_t*>(out) + wrow * DH;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                if (32 * ct + 8 * a < DH) {
+                    bf16x4 v;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = (bf16_t)acc[ct][4 * a + x];
+                    *reinterpret_cast<bf16x4*>(dst + 32 * ct + 8 * a + 4 * g) = v;
+                }
+    };
+    if (p.nslice > 1) {
+        float* dst = p.part + (long)z * 3 * wsz + wrow * DH;
+        store_row<CT>(dk, dst, g, DH);
+        store_row<CT>(du, dst + wsz, g, DH);
+        store_row<CT>(dv, dst + 2 * wsz, g, DH);
+    } else if (p.out_f32) {
+        store_row<CT>(dk, static_cast<float*>(p.out[0]) + wrow * DH, g, DH);
+        store_row<CT>(du, static_cast<float*>(p.out[1]) + wrow * DH, g, DH);
+        store_row<CT>(dv, static_cast<float*>(p.out[2]) + wrow * DH, g, DH);
+    } else {
+        store_bf16(dk, p.out[0]);
+        store_bf16(du, p.out[1]);
+        store_bf16(dv, p.out[2]);
+    }
+}
+
+// dK, dU, dV for d_h <= 96.  A wave owns one block of weight rows (the planes of its rows and the accumulators stay in registers)
+// and every other 32-row tile of its slice of the head's rows: waves 0, 1 take the even tiles of two blocks, waves 2, 3 the odd
+// ones, and their sums meet in LDS at the end.  The two waves of a tile take it apart; its float32 values, requested a step
+// ahead, wait in LDS where the lane that needs them put them (there are no registers for them).
+template <int CT>
+__global__ __launch_bounds__(256, 1) void dkdudv_split_kernel(F32Args p)
+{
+    static_assert(CT <= 3, "");
+    constexpr int RAW = 4 * CT;                // 16-byte loads of a lane and step: Q and dO, two halves of the rows, CT column groups
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
+    unsigned char* planes = lds + half * 2 * PLANES_B;                            // Q, dO
+    unsigned char* raw = lds + 4 * PLANES_B + wave * RAW * 1024;
+    float* sR = reinterpret_cast<float*>(lds + 4 * PLANES_B + 4 * RAW * 1024) + wave * 32;      // gate values of the wave's expert
+    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe, DH = p.DH;
+    const int blk = blockIdx.x * 2 + bw;
+    const Block b(p, hk, blk < nblk ? blk : nblk - 1);
+    const int ntile = (p.rows.n + 31) / 32;
+    const int t0 = (int)((long)ntile * z / p.nslice), t1 = (int)((long)ntile * (z + 1) / p.nslice);
+    const int steps = (t1 - t0 + 1) / 2;
+
+    const Cut<CT> cut(threadIdx.x & 127);      // rows 0 .. 15 of a tile; the same columns of rows 16 .. 31
+    auto request = [&](int s) {
+        const int t = t0 + 2 * s + half, row0 = 32 * (t < ntile ? t : ntile - 1);
+        int col = cut.col;
+        asm volatile("" : "+v"(col));      // (the addresses are not worth a register each)
+        const int last = 32 * (CT - 1) + col < DH ? 32 * (CT - 1) : -col;      // (columns beyond d_h: any; they are replaced by zero below)
+        static_for<4>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            const int r = row0 + 16 * (i & 1) + cut.row;
+            const float* src = (i < 2 ? p.Q : p.dO) + p.rows.tok_head_major(hk, r < p.rows.n ? r : p.rows.n - 1) * DH + col;
+            static_for<CT - 1>([&](auto kc) { lds_direct16<128 * decltype(kc)::value>(src, raw + (i * CT + decltype(kc)::value) * 1024); });
+            lds_direct16<0>(src + last, raw + (i * CT + CT - 1) * 1024);
+        });
+    };
+    // gate value of row l32 of this wave's next tile; 0 for the rows that a tile lacks, which removes them from every product
+    auto gate = [&](int s) {
+        const int t = t0 + 2 * s + half, r = 32 * t + l32;
+        const bool ok = t < t1 && r < p.rows.n;
+        return ok ? p.R[p.rows.head_major(hk, ok ? r : 0) * E + b.e] : 0.0f;
+    };
+    request(0);
+    float rg = gate(0);
+    Split8 kB[2 * CT], uB[2 * CT], vB[2 * CT];
+    const long wrow = b.wrow + (l32 < b.rows ? l32 : b.rows - 1);
+    {
+        f32x4 x[2][4 * CT];
+        load_row_operand<CT>(x[0], p.K + wrow * DH, g, DH);
+        load_row_operand<CT>(x[1], p.U + wrow * DH, g, DH);
+        __builtin_amdgcn_sched_barrier(0);
+        split_row_operand<CT>(kB, x[0]);
+#pragma unroll
+        for (int ks = 0; ks < 2 * CT; ++ks)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) asm volatile("" : "+a"(kB[ks].p[i]));
+        load_row_operand<CT>(x[0], p.V + wrow * DH, g, DH);
+        __builtin_amdgcn_sched_barrier(0);
+        split_row_operand<CT>(uB, x[1]);
+#pragma unroll
+        for (int ks = 0; ks < 2 * CT; ++ks) asm volatile("" : "+v"(uB[ks].p[0]), "+v"(uB[ks].p[1]), "+a"(uB[ks].p[2]));
+        __builtin_amdgcn_sched_barrier(0);
+        split_row_operand<CT>(vB, x[0]);
+    }
+    const PlaneLane pl(lane);
+    f32x16 dk[CT], du[CT], dv[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) { dk[ct] = zero16(); du[ct] = zero16(); dv[ct] = zero16(); }
+
+    for (int s = 0; s < steps; ++s) {
+        wait_vmcnt<0>();      // this lane's values have landed
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<RAW>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, k = i % CT, h = i / CT % 2;
+            f32x4 x = *reinterpret_cast<const f32x4*>(raw + i * 1024 + lane * 16);
+            if (32 * k + cut.col >= DH) x = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            cut.store(planes + (i < 2 * CT ? 0 : PLANES_B) + h * 16 * TILE_ROW_B, k, x);
+        });
+        if (g == 0) sR[l32] = rg;
+        __syncthreads();      // the planes are there, and this lane's values have been read
+        request(s + 1 < steps ? s + 1 : s);
+        rg = gate(s + 1);
+        f32x16 mna[3];
+        first_split<CT, 3, 2>(mna, planes, {kB, uB, vB}, pl, WeightAcc{}, [](auto) {});
+        f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
+        f32x4 r4[2];
+        auto gates = [&](int h) {
+            r4[0] = *reinterpret_cast<const f32x4*>(sR + split_row(8 * h, g));
+            r4[1] = *reinterpret_cast<const f32x4*>(sR + split_row(8 * h + 4, g));
+        };
+        gates(0);
+        mfma_result_fence(m, n, da);
+        float sg;
+        auto sigma = [&](int i) { sg = sigmoid_exact(m[i]); };
+        auto element = [&](int i) {
+            const float r = r4[(i >> 2) & 1][i & 3], sl = m[i] * sg, ra = r * da[i], nn = n[i];
+            m[i] = ra * nn * fmaf(sl, 1.0f - sg, sg);      // dM
+            n[i] = ra * sl;                                // dN
+            da[i] = r * sl * nn;                           // P
+        };
+        static_for<8>([&](auto ic) {
+            sigma(decltype(ic)::value);
+            element(decltype(ic)::value);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        gates(1);
+        // The second products of the first eight rows; behind their 18 CT matrix instructions the rest of the element-wise code.
+        u32x4 dm[3], dn[3], pp[3];
+        auto pair = [&](auto ic, u32x4(&v)[3], const f32x16& x, int first) {
+            split8_pair<decltype(ic)::value>(v, [&](int j) { return x[first + j]; });
+        };
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        static_for<4>([&](auto ic) { pair(ic, dm, m, 0); });
+        second_split<CT>(dk, planes, 0, split8_of(dm), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 4) pair(ic, dn, n, 0);
+            fence();
+        });
+        second_split<CT>(du, planes, 0, split8_of(dn), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 4) pair(ic, pp, da, 0);
+            fence();
+        });
+        second_split<CT>(dv, planes + PLANES_B, 0, split8_of(pp), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 16) {
+                if constexpr (i & 1) element(8 + i / 2);
+                else sigma(8 + i / 2);
+            }
+            fence();
+        });
+        static_for<16>([&](auto ic) {      // (what d_h < 96 leaves)
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i >= 8 + 3 * CT) {
+                sigma(i);
+                element(i);
+                fence();
+            }
+        });
+        static_for<4>([&](auto ic) { pair(ic, dm, m, 8); });
+        second_split<CT>(dk, planes, 1, split8_of(dm), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 4) pair(ic, dn, n, 8);
+            fence();
+        });
+        second_split<CT>(du, planes, 1, split8_of(dn), pl, [&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i < 4) pair(ic, pp, da, 8);
+            fence();
+        });
+        second_split<CT>(dv, planes + PLANES_B, 1, split8_of(pp), pl, [](auto) {});
+        __syncthreads();      // the planes have been read
+    }
+    add_halves_and_store<CT>(p, lds, dk, du, dv);
 }
 
 // dK, dU, dV.  A wave owns one block of weight rows (B operands and accumulators stay in registers) and every other
@@ -394,62 +933,7 @@ __global__ __launch_bounds__(256, 1) void dkdudv_f32_kernel(F32Args p)
             second_product<CT>(dv, sG, da, l);
         }
     }
-    // The odd tiles' sums to the wave with the even ones, one gradient at a time (64 lanes x 16 CT floats, lane-private).
-    // (This lane's row and the bounds of its columns are worked out again, out of the compiler's sight: kept over the loop they
-    // are the few registers too many that made it spill for d_h > 96.)
-    __syncthreads();
-    int lane = threadIdx.x & 63, DH = p.DH;
-    asm volatile("" : "+v"(lane), "+s"(DH));
-    const int l32 = lane & 31, g = lane >> 5;
-    float* xch = reinterpret_cast<float*>(lds) + bw * (3 * CT * 16 * 64) + lane;
-    if (half == 1) {
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                xch[(ct * 16 + i) * 64] = dk[ct][i];
-                xch[((CT + ct) * 16 + i) * 64] = du[ct][i];
-                xch[((2 * CT + ct) * 16 + i) * 64] = dv[ct][i];
-            }
-    }
-    __syncthreads();
-    if (half == 1 || blk >= nblk || l32 >= b.rows) return;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            dk[ct][i] += xch[(ct * 16 + i) * 64];
-            du[ct][i] += xch[((CT + ct) * 16 + i) * 64];
-            dv[ct][i] += xch[((2 * CT + ct) * 16 + i) * 64];
-        }
-    const long wrow = b.wrow + l32, wsz = (long)p.rows.Hkuv * E * p.de * DH;
-    auto store_bf16 = [&](const f32x16(&acc)[CT], void* out) {
-        bf16_t* dst = static_cast<bf16_t*>(out) + wrow * DH;
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-                if (32 * ct + 8 * a < DH) {
-                    bf16x4 v;
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = (bf16_t)acc[ct][4 * a + x];
-                    *reinterpret_cast<bf16x4*>(dst + 32 * ct + 8 * a + 4 * g) = v;
-                }
-    };
-    if (p.nslice > 1) {
-        float* dst = p.part + (long)z * 3 * wsz + wrow * DH;
-        store_row<CT>(dk, dst, g, DH);
-        store_row<CT>(du, dst + wsz, g, DH);
-        store_row<CT>(dv, dst + 2 * wsz, g, DH);
-    } else if (p.out_f32) {
-        store_row<CT>(dk, static_cast<float*>(p.out[0]) + wrow * DH, g, DH);
-        store_row<CT>(du, static_cast<float*>(p.out[1]) + wrow * DH, g, DH);
-        store_row<CT>(dv, static_cast<float*>(p.out[2]) + wrow * DH, g, DH);
-    } else {
-        store_bf16(dk, p.out[0]);
-        store_bf16(du, p.out[1]);
-        store_bf16(dv, p.out[2]);
-    }
+    add_halves_and_store<CT>(p, lds, dk, du, dv);
 }
 
 // Adds the parts' sums in order: the rows of O or dQ (dst, four columns per lane) and, for blockIdx.x >= row_blocks, the
@@ -510,12 +994,14 @@ F32Args f32_args(const void* Q, const void* K, const void* U, const void* V, con
 template <int CT>
 hipError_t launch_fwd_f32_t(const F32Args& a, const Dims& d, hipStream_t st)
 {
-    const int smem = 5 * Tile<CT>::BYTES;
+    constexpr int GROUPS = CT > 3 ? 1 : 2;
+    const int smem = GROUPS * 3 * PLANES_B;
+    static_assert(GROUPS == 1 || 4 * CT * 16 * 64 * 4 <= GROUPS * 3 * PLANES_B, "the teams' exchange fits the planes");
     static LdsOptIn optin;
-    const hipError_t e = ensure_dynamic_lds(optin, (const void*)fwd_f32_kernel<CT>, smem);
+    const hipError_t e = ensure_dynamic_lds(optin, (const void*)fwd_f32_kernel<CT, GROUPS>, smem);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fwd_f32_kernel<CT>, dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit), dim3(256),
-                       smem, st, a);
+    hipLaunchKernelGGL((fwd_f32_kernel<CT, GROUPS>), dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit),
+                       dim3(256 * GROUPS), smem, st, a);
     if (a.parts.nsplit > 1) {
         const unsigned rb = (unsigned)(((long)a.rows.n * (d.d_h / 4) + 255) / 256);
         hipLaunchKernelGGL(sum_f32_kernel, dim3(rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, a.O, rb);
@@ -528,7 +1014,7 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
 {
     hipError_t err = hipSuccess;
     if (phases & PH_BWD_DQDR) {
-        const int smem = 3 * Tile<CT>::BYTES;
+        const int smem = 6 * PLANES_B;
         static LdsOptIn optin;
         err = ensure_dynamic_lds(optin, (const void*)dqdr_f32_kernel<CT>, smem);
         if (err != hipSuccess) return err;
@@ -543,13 +1029,22 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
         if (err != hipSuccess) return err;
     }
     if (phases & PH_BWD_DKDUDV) {
-        const int smem = 8 * Tile<CT>::BYTES + 2 * 4 * 32 * (int)sizeof(float);
-        static_assert(2 * 3 * CT * 16 * 64 * 4 <= 8 * Tile<CT>::BYTES, "the waves' exchange fits the tile stages");
+        const dim3 grid((unsigned)((d.E * nbe_of(d) + 1) / 2), (unsigned)d.Hkuv, (unsigned)a.nslice);
+        void (*kernel)(F32Args);
+        int smem;
+        if constexpr (CT <= 3) {
+            kernel = dkdudv_split_kernel<CT>;
+            smem = 4 * PLANES_B + 16 * CT * 1024 + 4 * 32 * (int)sizeof(float);
+            static_assert(2 * 3 * CT * 16 * 64 * 4 <= 4 * PLANES_B, "the waves' exchange fits the planes");
+        } else {
+            kernel = dkdudv_f32_kernel<CT>;
+            smem = 8 * Tile<CT>::BYTES + 2 * 4 * 32 * (int)sizeof(float);
+            static_assert(2 * 3 * CT * 16 * 64 * 4 <= 8 * Tile<CT>::BYTES, "the waves' exchange fits the tile stages");
+        }
         static LdsOptIn optin;
-        err = ensure_dynamic_lds(optin, (const void*)dkdudv_f32_kernel<CT>, smem);
+        err = ensure_dynamic_lds(optin, (const void*)kernel, smem);
         if (err != hipSuccess) return err;
-        dim3 grid((unsigned)((d.E * nbe_of(d) + 1) / 2), (unsigned)d.Hkuv, (unsigned)a.nslice);
-        hipLaunchKernelGGL(dkdudv_f32_kernel<CT>, grid, dim3(256), smem, st, a);
+        hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, a);
         err = hipGetLastError();
     }
     return err;
