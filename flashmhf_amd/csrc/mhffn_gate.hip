@@ -103,6 +103,21 @@ __device__ __forceinline__ void stage_router_cols(const T* Wr, int E, unsigned c
     }
 }
 
+// 32 rows of DH values as whole rows between memory and registers or LDS, and as half rows (the 16-byte chunks 2 ks + g of row
+// l32) between LDS and the lanes that compute.  Whole rows: a wave-instruction moves the 64 chunks from 64 i on, counted along
+// the rows; chunk c of row r sits at c ^ swz(r) in LDS, which keeps 16 rows' reads of one chunk in different banks.
+template <int DH>
+struct RowTile {
+    static constexpr int CH = DH / 8, INS = DH / 16;
+    __device__ static int swz(int r)
+    {
+        return DH == 128 ? swz16(r) : DH == 96 ? (r >> 2) & 3 : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+    }
+    __device__ static int row(int i, int lane) { return (i * 64 + lane) / CH; }
+    __device__ static int chunk(int i, int lane) { return (i * 64 + lane) % CH ^ swz(row(i, lane)); }
+    __device__ static int half(int ks, int l32, int g) { return l32 * (2 * DH) + (((2 * ks + g) ^ swz(l32)) << 4); }
+};
+
 // Everything the forward computes for one tile, shared by both kernels.
 template <int DH, int NT, bool NORM>
 struct GateTile {
@@ -188,7 +203,11 @@ struct GateTile {
 // memory) leaves the wave as whole cache lines instead of one scattered dword per lane and expert
 constexpr size_t gate_fwd_smem(int DH, int NT) { return (size_t)2 * NT * (DH / 16) * 1024 + DH * 4 + 4 * TILE_B; }
 
-template <int DH, int NT, bool NORM>
+// WHOLE: the rows move between memory and the wave as whole rows, by way of its LDS; else each lane loads and stores its half row,
+// in 32-byte pieces of 32 rows per instruction.  Pieces keep the path from L2 busy four times as long: 32,768 tokens of 16 heads of
+// 128 take 71.5 us with them and 62.8 with whole rows (5.0 TB/s, what a large copy reaches; loads alone in pieces 65.3), 16,384 of
+// 8 heads 18.3 and 16.9.  Few tokens wait for one tile's chain, which the way through LDS makes longer: 512 of 8 heads 6.0 and 6.3.
+template <int DH, int NT, bool NORM, bool WHOLE>
 __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 {
     constexpr int KS = DH / 16;
@@ -213,9 +232,32 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
         const long row = (((long)b * p.S + (valid ? t : p.S - 1)) * p.H + h) * DH;
         GateTile<DH, NT, NORM> T;
         T.eps_ = p.eps;
-        T.load(p.X + row, g);
+        using Rows = RowTile<DH>;
+        unsigned char* xt = reinterpret_cast<unsigned char*>(rtile);      // the wave's rows of x, then of y, then of R
+        const long row0 = (((long)b * p.S + tile * 32) * p.H + h) * DH, stride = (long)p.H * DH;
+        const int nrow = min(32, p.S - tile * 32);
+        if constexpr (WHOLE) {
+#pragma unroll
+            for (int i = 0; i < Rows::INS; ++i)
+                __builtin_amdgcn_global_load_lds((gptr_t)(p.X + row0 + min(Rows::row(i, lane), nrow - 1) * stride + Rows::chunk(i, lane) * 8),
+                                                 (lptr_t)(xt + i * 1024), 16, 0, 0);
+            wait_vmcnt<0>();
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) T.xr[ks] = *reinterpret_cast<const u32x4*>(xt + Rows::half(ks, l32, g));
+        } else {
+            T.load(p.X + row, g);
+        }
         T.template normalise<false>(sW, g);
-        if constexpr (NORM) {
+        if constexpr (NORM && WHOLE) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<bf16x8*>(xt + Rows::half(ks, l32, g)) = T.y[ks];
+#pragma unroll
+            for (int i = 0; i < Rows::INS; ++i) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(xt + i * 1024 + lane * 16);
+                if (Rows::row(i, lane) < nrow)
+                    *reinterpret_cast<u32x4*>(p.Qn + row0 + Rows::row(i, lane) * stride + Rows::chunk(i, lane) * 8) = v;
+            }
+        } else if constexpr (NORM) {
             if (valid) {
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks)
@@ -248,8 +290,8 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 // time and are added up down the columns (4 values per 64 columns).  What that frees holds the next tile's rows of x, requested
 // behind the contraction, while dR and dQ of a tile are requested at its top and used half a trip later.  One wave per SIMD
 // with all sums in registers, ~2,400 instructions per tile, a quarter of them register moves, took 150 us on 32,768 tokens of
-// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 109 us
-// (4.1 TB/s; 128 us traced).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
+// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 109 us, and 101
+// with dX stored as whole rows (4.4 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
 // More experts (NT = 2) have twice the d_router operands: four waves, one per SIMD, all sums in registers, and the next
 // tile's rows requested before the current tile's arithmetic starts.
 constexpr int GATE_Z_ROW_B = 64;                           // NT = 1: row of the dz tile
@@ -299,7 +341,10 @@ __device__ __forceinline__ bf16x8 z_cols(const unsigned char* tile, int lane, in
     return v;
 }
 
-template <int DH, int NT, bool NORM>
+// WHOLE: dX leaves as whole rows, by way of the y tile, as Q does in the forward.  32,768 tokens of 16 heads of 128 take 104 us this way,
+// 112 in half rows' pieces; with one or two tiles per wave the way through LDS is not hidden (12,288 of 8 heads 35.0 and 34.5).
+// (x and dQ as whole rows, too, take registers: 108 us with a spill, 111 for x alone.)
+template <int DH, int NT, bool NORM, bool WHOLE>
 __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
 {
     const int NW = NT == 1 ? (int)blockDim.x / 64 : 4;
@@ -569,14 +614,27 @@ __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_
                 for (int j = 0; j < 8; ++j)
                     du[ks][j] = T.rstd * (du[ks][j] - bf_at(T.xr[ks], j) * T.rstd * c);
         }
-        if (valid) {
+        auto out = [&](int ks) {
+            bf16x8 o;
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                bf16x8 o;
+            for (int j = 0; j < 8; ++j) o[j] = (bf16_t)du[ks][j];
+            return o;
+        };
+        if constexpr (WHOLE) {
+            using Rows = RowTile<DH>;
+            bf16_t* d0 = p.dX + (((long)b * p.S + tile * 32) * p.H + h) * DH;
+            const int nrow = min(32, p.S - tile * 32);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) o[j] = (bf16_t)du[ks][j];
-                *reinterpret_cast<bf16x8*>(p.dX + row + (2 * ks + g) * 8) = o;
+            for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<bf16x8*>(ytile + Rows::half(ks, l32, g)) = out(ks);
+#pragma unroll
+            for (int i = 0; i < Rows::INS; ++i) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(ytile + i * 1024 + lane * 16);
+                if (Rows::row(i, lane) < nrow)
+                    *reinterpret_cast<u32x4*>(d0 + (long)Rows::row(i, lane) * (p.H * DH) + Rows::chunk(i, lane) * 8) = v;
             }
+        } else if (valid) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<bf16x8*>(p.dX + row + (2 * ks + g) * 8) = out(ks);
         }
     }
 
@@ -696,7 +754,9 @@ __global__ __launch_bounds__(256) void mhffn_gate_sum_kernel(const float* part, 
 namespace {
 
 // Tiles a wave takes.  Forward: several waves per SIMD hide the latency, so a wave only takes several tiles once there
-// are at least 8 waves per SIMD; backward: as many waves (and partial sums) as fill the chip once.
+// are at least 8 waves per SIMD; backward: as many waves (and partial sums) as fill the chip once, but for what is left over in a
+// second round of workgroups (one of eight waves fits a compute unit): a round takes 6 us and 8.5 for each of its waves' tiles (heads of
+// 128).  12,288 tokens of 8 heads: 34.8 us in 384 workgroups of one tile per wave, 29.4 in 192 of two; of 16 heads of 6,144 35.6, 29.6.
 int tiles_per_wave(int B, int H, int S, int waves, long cap)
 {
     const long total = (long)B * H * ((S + 31) / 32);
@@ -712,27 +772,38 @@ int gate_bwd_waves(const Dims& d) { return d.E > 32 || (long)d.B * d.H * ((d.S +
 dim3 gate_bwd_grid(const Dims& d, int& tpw)
 {
     const int nw = gate_bwd_waves(d), ntiles = (d.S + 31) / 32;
+    auto workgroups = [&](int t) { return (ntiles + nw * t - 1) / (nw * t); };
+    auto rounds = [&](int t) { return ((long)d.B * d.H * workgroups(t) + CUS - 1) / CUS; };
     tpw = tiles_per_wave(d.B, d.H, d.S, nw * CUS, 64);
-    return dim3((ntiles + nw * tpw - 1) / (nw * tpw), d.H, d.B);
+    for (int t = tpw + 1; t <= 64 && rounds(t - 1) > 1 && workgroups(t - 1) > 1; ++t)
+        if (rounds(t) * (6 + 8.5 * t) < rounds(tpw) * (6 + 8.5 * tpw)) tpw = t;
+    return dim3(workgroups(tpw), d.H, d.B);
 }
 
 template <int DH, int NT, bool NORM>
 hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
 {
-    static LdsOptIn optin_fwd, optin_bwd;
+    static LdsOptIn optin_fwd[2], optin_bwd[2];
     if (backward) {
         const int most = (int)gate_bwd_smem<NT>(DH, gate_bwd_max_waves<NT>()), waves = gate_bwd_waves(d);
-        const hipError_t e = ensure_dynamic_lds(optin_bwd, (const void*)mhffn_gate_bwd_kernel<DH, NT, NORM>, most);
-        if (e != hipSuccess) return e;
         const dim3 grid = gate_bwd_grid(d, a.tpw);
-        hipLaunchKernelGGL((mhffn_gate_bwd_kernel<DH, NT, NORM>), grid, dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
+        constexpr bool CAN = NT == 1;
+        const bool whole = CAN && a.tpw >= 4;
+        auto* fn = whole ? mhffn_gate_bwd_kernel<DH, NT, NORM, CAN> : mhffn_gate_bwd_kernel<DH, NT, NORM, false>;
+        const hipError_t e = ensure_dynamic_lds(optin_bwd[whole], (const void*)fn, most);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(fn, grid, dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
     } else {
         const size_t smem = gate_fwd_smem(DH, NT);
-        const hipError_t e = ensure_dynamic_lds(optin_fwd, (const void*)mhffn_gate_fwd_kernel<DH, NT, NORM>, (int)smem);
+        // whole rows from six tiles per compute unit on (us in pieces / whole: 1,024 tiles of 8 heads of 128 7.5 / 7.8, 1,536 9.6 / 9.2, 2,048
+        // 11.4 / 10.3; of 96 6.5 / 6.7, 8.6 / 8.4 with 2,048; of 64 6.5 / 6.4 with 2,048)
+        const bool whole = (long)a.B * a.H * ((a.S + 31) / 32) >= 6 * CUS;
+        auto* fn = whole ? mhffn_gate_fwd_kernel<DH, NT, NORM, true> : mhffn_gate_fwd_kernel<DH, NT, NORM, false>;
+        const hipError_t e = ensure_dynamic_lds(optin_fwd[whole], (const void*)fn, (int)smem);
         if (e != hipSuccess) return e;
         a.tpw = tiles_per_wave(a.B, a.H, a.S, 8192, 16);
         const dim3 grid(((a.S + 31) / 32 + 4 * a.tpw - 1) / (4 * a.tpw), a.H, a.B);
-        hipLaunchKernelGGL((mhffn_gate_fwd_kernel<DH, NT, NORM>), grid, dim3(256), smem, st, a);
+        hipLaunchKernelGGL(fn, grid, dim3(256), smem, st, a);
     }
     return hipGetLastError();
 }
