@@ -28,6 +28,7 @@ EXPORTS = (
     "mhffn_fwd_layout", "mhffn_bwd_layout", "mhffn_bwd_static", "mhffn_gate_fwd", "mhffn_gate_bwd",
     "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into", "mhffn_rope_fwd", "mhffn_rope_bwd",
     "mhffn_product_preferred", "mhffn_product_faster", "mhffn_product_tile", "mhffn_product",
+    "mhffn_product_pair_faster", "mhffn_product_pair",
 )
 PRODUCT_NT, PRODUCT_NN, PRODUCT_TN = 0, 1, 2
 TOKENS_BHSD, TOKENS_BSHD = 0, 1     # layout of Q, O, dO, dQ
@@ -86,6 +87,8 @@ def lib():
         L.mhffn_product_faster.argtypes = [ctypes.c_int] * 5
         L.mhffn_product_tile.argtypes = [ctypes.c_int] * 5
         L.mhffn_product.argtypes = [ctypes.c_int] * 2 + [vp] * 3 + [ctypes.c_int] * 3 + [vp]
+        L.mhffn_product_pair_faster.argtypes = [ctypes.c_int] * 4
+        L.mhffn_product_pair.argtypes = [vp] * 5 + [ctypes.c_int] * 3 + [vp]
         _lib = L
     return _lib
 

@@ -379,4 +379,27 @@ int mhffn_product(int form, int in_order, const void* A, const void* B, void* C,
     return mhffn::launch_product(form, in_order != 0, A, B, C, M, N, K, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
 }
 
+static int check_pair(int M, int N, int K)
+{
+    const int rc = check_product(MHFFN_PRODUCT_NN, M, K, N);
+    return rc == MHFFN_OK ? check_product(MHFFN_PRODUCT_TN, N, K, M) : rc;
+}
+
+int mhffn_product_pair_faster(int in_order, int M, int N, int K)
+{
+    return check_pair(M, N, K) == MHFFN_OK && mhffn::product_pair_faster(in_order != 0, M, N, K);
+}
+
+int mhffn_product_pair(const void* dy, const void* w, const void* x, void* dx, void* dw, int M, int N, int K, void* stream)
+{
+    const int rc = check_pair(M, N, K);
+    if (rc != MHFFN_OK) return rc;
+    const void* ptrs[] = {dy, w, x, dx, dw};
+    for (const void* p : ptrs) {
+        if (!p) return MHFFN_ERR_NULL_POINTER;
+        if (!aligned16(p)) return MHFFN_ERR_ALIGNMENT;
+    }
+    return mhffn::launch_product_pair(dy, w, x, dx, dw, M, N, K, (hipStream_t)stream) == hipSuccess ? MHFFN_OK : MHFFN_ERR_LAUNCH;
+}
+
 }  // extern "C"

@@ -26,6 +26,8 @@
 #include "mhffn_common.hpp"
 #include "mhffn_product.hpp"
 
+#include <utility>
+
 namespace mhffn {
 
 constexpr int PROD_UNIT_B = 4096;
@@ -45,10 +47,10 @@ static __device__ __align__(16) const unsigned prod_zeros[4] = {0u, 0u, 0u, 0u};
 
 // Workgroup i runs on XCD i % 8: each XCD takes a run of consecutive tiles, counted in columns four tiles of rows high, so that what
 // it reads fits its L2.
-__device__ __forceinline__ void prod_tile(const ProductArgs& p, int& mt, int& nt)
+__device__ __forceinline__ void prod_tile(const ProductArgs& p, unsigned block, int& mt, int& nt)
 {
-    const unsigned total = p.mtiles * p.ntiles, xcd = blockIdx.x & 7, q = total >> 3, rem = total & 7;
-    const unsigned t = (blockIdx.x >> 3) + xcd * q + (xcd < rem ? xcd : rem);
+    const unsigned total = p.mtiles * p.ntiles, xcd = block & 7, q = total >> 3, rem = total & 7;
+    const unsigned t = (block >> 3) + xcd * q + (xcd < rem ? xcd : rem);
     const unsigned band = t / (4u * p.ntiles), in = t - band * 4u * p.ntiles;
     const unsigned high = min(4u, p.mtiles - 4u * band);
     mt = 4 * band + in % high;
@@ -174,7 +176,7 @@ __device__ __forceinline__ f32x4 prod_mfma(bf16x8 a, bf16x8 b, f32x4 c) { return
 // products behind it (TN of 1,024 x 1,024 x 2,048: 11.1 us with every wave filling, 12.2 with the fills between the products, 9.5
 // with waves of their own for them; all eight waves reading and then multiplying together were between these).
 template <bool ACOLS, bool BCOLS, int BM, int BN, int TH, int WM, int KU, int NST>
-__global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(ProductArgs p)
+__device__ __forceinline__ void product_tile_of(const ProductArgs& p, unsigned block)
 {
     constexpr int TM = BM / WM / TH, TN = BN / (8 / WM) / TH;      // tiles of a wave
     using FA = ProductFill<ACOLS, BM, KU, FILLERS>;
@@ -186,7 +188,7 @@ __global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(Produ
     const int late = wave >> 2, wm = wave % WM, wn = wave / WM;
 
     int mt, nt;
-    prod_tile(p, mt, nt);
+    prod_tile(p, block, mt, nt);
     const int m0 = mt * BM, n0 = nt * BN;
     const int nst = (p.K + 64 * KU - 1) / (64 * KU);
     auto barrier = [&]() {
@@ -313,6 +315,34 @@ __global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(Produ
     }
 }
 
+template <bool ACOLS, bool BCOLS, int BM, int BN, int TH, int WM, int KU, int NST>
+__global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_kernel(ProductArgs p)
+{
+    product_tile_of<ACOLS, BCOLS, BM, BN, TH, WM, KU, NST>(p, blockIdx.x);
+}
+
+// The tiles that every form has, by their place in PRODUCT_VARIANTS.
+template <int V>
+struct Tiles {
+    static constexpr int BM = V ? 128 : 64, BN = V == 2 ? 128 : 64, TH = V ? 32 : 16, WM = 4, KU = V == 2 ? 1 : 2, NST = V == 1 ? 3 : 4;
+    static constexpr int SMEM = (BM + BN) * KU * 128 * NST;      // (holds the tile of C, too)
+    static_assert(BM * BN * 2 <= SMEM && SMEM <= 160 * 1024, "LDS of a compute unit");
+};
+
+// Both products of a linear layer's backward in one launch: dx = dy w (NN, tiles VN) in the workgroups from nn0 on, dw = dy^T x (TN,
+// tiles VT) in those from tn0 on.  Each alone leaves compute units idle, most of them with few tokens, and the second waits for a
+// launch; us for both, two launches / one, in a graph of ten:
+//     hidden 768, 512 tokens 11.0 / 6.6, 2,048 17.5 / 11.3; hidden 1024, 64 tokens 10.3 / 7.3, 512 12.0 / 7.8, 1,024 13.6 / 9.1, 2,048 19.7 / 15.8,
+//     4,096 30.2 / 27.8; 512 of 1024 -> 3072 23.1 / 15.1; hidden 2048, 512 20.0 / 15.5, 2,048 42.4 / 41.5.
+template <int VN, int VT>
+__global__ __launch_bounds__(512 + 64 * FILLERS) void mhffn_product_pair_kernel(ProductArgs nn, unsigned nn0, ProductArgs tn, unsigned tn0)
+{
+    using N = Tiles<VN>;
+    using T = Tiles<VT>;
+    if (blockIdx.x - nn0 < (unsigned)(nn.mtiles * nn.ntiles)) product_tile_of<false, true, N::BM, N::BN, N::TH, N::WM, N::KU, N::NST>(nn, blockIdx.x - nn0);
+    else product_tile_of<true, true, T::BM, T::BN, T::TH, T::WM, T::KU, T::NST>(tn, blockIdx.x - tn0);
+}
+
 // NT with few tiles: 32 TM x 32 TN of C per workgroup.  Its eight waves take every eighth chunk of 64 of the summed index each, through
 // LDS of their own (Q chunks in flight, no barrier before the end), and their sums are added at the end, in the waves' order.
 // (512 x 1,024 x 1,024: 5.1 us with 64 x 32 against 6.0 with 32 x 64 above; 64 x 64 this way 6.7.)
@@ -329,7 +359,7 @@ __global__ __launch_bounds__(512) void mhffn_product_split_kernel(ProductArgs p)
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int mt, nt;
-    prod_tile(p, mt, nt);
+    prod_tile(p, blockIdx.x, mt, nt);
     const int m0 = mt * BM, n0 = nt * BN;
     unsigned char* own = smem + wave * Q * CHUNK_B;
     FA fa;
@@ -425,7 +455,7 @@ __global__ __launch_bounds__(512) void mhffn_product_split_kernel(ProductArgs p)
 template <bool ACOLS, bool BCOLS, int BM, int BN, int TH, int WM, int KU, int NST>
 static hipError_t launch_tiles(ProductArgs a, hipStream_t st)
 {
-    constexpr int smem = (BM + BN) * KU * 128 * NST;      // (holds the tile of C, too)
+    constexpr int smem = (BM + BN) * KU * 128 * NST;
     static_assert(BM * BN * 2 <= smem && smem <= 160 * 1024, "LDS of a compute unit");
     static LdsOptIn optin;
     auto* fn = mhffn_product_kernel<ACOLS, BCOLS, BM, BN, TH, WM, KU, NST>;
@@ -481,6 +511,36 @@ int product_tile(int form, bool in_order, int M, int N, int K)
     const ProductVariant& p = PRODUCT_VARIANTS[product_variant(form, in_order, M, N, K)];
     return 65536 * p.bm + p.bn;
 }
+// Time of a pair's launch in tiles vn and vt, by the same prices: n + t workgroups, those that take longer first, each to the compute unit
+// that is free first.  Over 35 pairs (hidden 512 to 2048, 1 to 8,192 tokens) the fastest by this is the fastest of the nine measured or
+// 2.4 % slower, 0.2 % on average; the tiles that each product alone would take are up to 49 % slower (both then run to a second
+// round, which larger tiles do without: 1,024 tokens of hidden 768 11.4 us, in 128 x 64 and 64 x 64 7.7).
+static double product_pair_us(int vn, int vt, int M, int N, int K, bool& nn_first)
+{
+    const ProductVariant &pn = PRODUCT_VARIANTS[vn], &pt = PRODUCT_VARIANTS[vt];
+    long n = product_tiles(pn, M, K), t = product_tiles(pt, N, K);
+    const long all = n + t;
+    const double load = all <= CUS / 2 ? 0 : all >= CUS ? 1 : (all - CUS / 2) / (double)(CUS / 2);
+    double dn = pn.again + (N + 63) / 64 * pn.step * (1 + pn.full * load), dt = pt.again + (M + 63) / 64 * pt.step * (1 + pt.full * load);
+    nn_first = dn >= dt;
+    const double launch = pn.base - pn.again > pt.base - pt.again ? pn.base - pn.again : pt.base - pt.again;
+    if (all > 16 * CUS) return launch + (n * dn + t * dt) / CUS;
+    if (!nn_first) {
+        std::swap(n, t);
+        std::swap(dn, dt);
+    }
+    // compute units with n / CUS of the longer ones and with one more; the shorter ones to whichever is free first
+    const long more = n % CUS, less = CUS - more;
+    double a = (double)(n / CUS) * dn, b = a + dn, end = more ? b : a;
+    while (t > 0) {
+        double& free = a <= b || !more ? a : b;
+        t -= &free == &a ? less : more;
+        free += dt;
+        if (free > end) end = free;
+    }
+    return launch + end;
+}
+
 // One round of the largest tiles: there these kernels are as fast as the library's or faster (NT of 3,000 x 1,024 x 1,024 11.3 us
 // against 11.7, of 2,048^3 20.3 against 20.4; TN of the latter 21.2 against 25.3); with more its larger tiles win in NT and NN
 // (8,192 x 1,024 x 1,024: 25 against 22).
@@ -505,13 +565,25 @@ bool product_faster(int form, bool in_order, int M, int N, int K)
     return true;
 }
 
+// Both products of a backward in one launch: wherever each is taken here, and where dw is two rounds of the largest tiles, which the
+// library's product beats, but not by the launch and the idle compute units that the pair saves (two launches with the library's dw /
+// one: 512 rows of 1024 -> 8192 49.5 / 33.4, 2,048 84.6 / 81.3; of 768 -> 8192 48.7 / 33.1, 79.8 / 66.4).
+bool product_pair_faster(bool in_order, int M, int N, int K)
+{
+    return product_faster(PRODUCT_NN, in_order, M, K, N) && (product_faster(PRODUCT_TN, in_order, N, K, M) || product_tiles(PRODUCT_VARIANTS[2], N, K) <= 2 * CUS);
+}
+
 template <bool ACOLS, bool BCOLS>
 static hipError_t launch_form(const ProductArgs& a, int variant, hipStream_t st)
 {
+    auto tiles = [&](auto t) {
+        using T = decltype(t);
+        return launch_tiles<ACOLS, BCOLS, T::BM, T::BN, T::TH, T::WM, T::KU, T::NST>(a, st);
+    };
     switch (variant) {
-        case 0: return launch_tiles<ACOLS, BCOLS, 64, 64, 16, 4, 2, 4>(a, st);
-        case 1: return launch_tiles<ACOLS, BCOLS, 128, 64, 32, 4, 2, 3>(a, st);
-        case 2: return launch_tiles<ACOLS, BCOLS, 128, 128, 32, 4, 1, 4>(a, st);
+        case 0: return tiles(Tiles<0>{});
+        case 1: return tiles(Tiles<1>{});
+        case 2: return tiles(Tiles<2>{});
     }
     if constexpr (!ACOLS && !BCOLS) switch (variant) {
         case 3: return launch_tiles<ACOLS, BCOLS, 32, 64, 16, 2, 2, 4>(a, st);
@@ -519,6 +591,41 @@ static hipError_t launch_form(const ProductArgs& a, int variant, hipStream_t st)
         case 5: return launch_split<2, 1, 1>(a, st);
     }
     return hipErrorInvalidValue;
+}
+
+template <int VN, int VT>
+static hipError_t launch_pair_of(ProductArgs nn, ProductArgs tn, bool nn_first, hipStream_t st)
+{
+    constexpr int smem = Tiles<VN>::SMEM > Tiles<VT>::SMEM ? Tiles<VN>::SMEM : Tiles<VT>::SMEM;
+    static LdsOptIn optin;
+    auto* fn = mhffn_product_pair_kernel<VN, VT>;
+    const hipError_t e = ensure_dynamic_lds(optin, (const void*)fn, smem);
+    if (e != hipSuccess) return e;
+    nn.mtiles = (nn.M + Tiles<VN>::BM - 1) / Tiles<VN>::BM;
+    nn.ntiles = (nn.N + Tiles<VN>::BN - 1) / Tiles<VN>::BN;
+    tn.mtiles = (tn.M + Tiles<VT>::BM - 1) / Tiles<VT>::BM;
+    tn.ntiles = (tn.N + Tiles<VT>::BN - 1) / Tiles<VT>::BN;
+    const unsigned n = nn.mtiles * nn.ntiles, t = tn.mtiles * tn.ntiles;
+    hipLaunchKernelGGL(fn, dim3(n + t), dim3(512 + 64 * FILLERS), smem, st, nn, nn_first ? 0u : t, tn, nn_first ? n : 0u);
+    return hipGetLastError();
+}
+hipError_t launch_product_pair(const void* dy, const void* w, const void* x, void* dx, void* dw, int M, int N, int K, hipStream_t st)
+{
+    const ProductArgs nn{(const bf16_t*)dy, (const bf16_t*)w, (bf16_t*)dx, M, K, N, 0, 0};
+    const ProductArgs tn{(const bf16_t*)dy, (const bf16_t*)x, (bf16_t*)dw, N, K, M, 0, 0};
+    using Launch = hipError_t (*)(ProductArgs, ProductArgs, bool, hipStream_t);
+    static constexpr Launch of[3][3] = {{launch_pair_of<0, 0>, launch_pair_of<0, 1>, launch_pair_of<0, 2>},
+                                        {launch_pair_of<1, 0>, launch_pair_of<1, 1>, launch_pair_of<1, 2>},
+                                        {launch_pair_of<2, 0>, launch_pair_of<2, 1>, launch_pair_of<2, 2>}};
+    int best = 0;
+    double best_us = 0;
+    bool best_first = true;
+    for (int v = 0; v < 9; ++v) {
+        bool first;
+        const double us = product_pair_us(v / 3, v % 3, M, N, K, first);
+        if (v == 0 || us < best_us) { best = v; best_us = us; best_first = first; }
+    }
+    return of[best / 3][best % 3](nn, tn, best_first, st);
 }
 
 hipError_t launch_product(int form, bool in_order, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t st)

@@ -348,19 +348,23 @@ bool library_in_order(int form, int64_t M, int64_t N, int64_t K)
     if (form == MHFFN_PRODUCT_TN) return K > 16;
     return M > (form == MHFFN_PRODUCT_NT ? 31 : 16) && (K <= 1024 || M * N > (1 << 18));
 }
-// M x N with inner extent K into `out_sizes`, or an undefined tensor where the product is the library's: where it is
-// faster or outside the kernels' sizes, under a dispatch mode (which is to see the call), or where autograd is to record the call.
+// Whether an M x N product with inner extent K may run in these kernels: not where its bits are to be the library's and are not, not
+// under a dispatch mode (which is to see the call) nor where autograd is to record the call.
+bool own_may(int form, Whose whose, const Tensor& a, const Tensor& b, int64_t M, int64_t N, int64_t K)
+{
+    if (whose == LIBRARY || (whose == OWN_IN_ORDER && !library_in_order(form, M, N, K))) return false;
+    if (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) return false;
+    if (!plain(a) || !plain(b) || a.device() != b.device() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+    return std::max({M, N, K}) <= INT_MAX;
+}
+// That product into `out_sizes`, or an undefined tensor where it is the library's: also where that is faster
 Tensor own_product(int form, Whose whose, const Tensor& a, const Tensor& b, int64_t M, int64_t N, int64_t K, at::IntArrayRef out_sizes)
 {
-    if (whose == LIBRARY || (whose == OWN_IN_ORDER && !library_in_order(form, M, N, K))) return {};
-    if (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) return {};
-    if (!plain(a) || !plain(b) || a.device() != b.device() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return {};
-    const int in_order = whose == OWN_IN_ORDER;
-    if (std::max({M, N, K}) > INT_MAX || !mhffn_product_faster(form, in_order, (int)M, (int)N, (int)K)) return {};
+    if (!own_may(form, whose, a, b, M, N, K) || !mhffn_product_faster(form, whose == OWN_IN_ORDER, (int)M, (int)N, (int)K)) return {};
     RECORD_FUNCTION("mhffn::product", std::vector<c10::IValue>());
     OnDevice on_device(a);
     Tensor c = empty_of(out_sizes, at::kBFloat16, a);
-    raise_for_code(mhffn_product(form, in_order, ptr(a), ptr(b), ptr(c), (int)M, (int)N, (int)K, stream()), "mhffn_product");
+    raise_for_code(mhffn_product(form, whose == OWN_IN_ORDER, ptr(a), ptr(b), ptr(c), (int)M, (int)N, (int)K, stream()), "mhffn_product");
     return c;
 }
 // x w^T, x [.., in], w [out, in]
@@ -386,6 +390,26 @@ Tensor product_tn(const Tensor& a, const Tensor& b, Whose whose)
     return c.defined() ? c : at::mm(a.t(), b);
 }
 
+// Both gradients of a linear layer, {dy w, dy^T x} of matrices: in one launch where that is faster.
+std::pair<Tensor, Tensor> product_pair(const Tensor& dy, const Tensor& w, const Tensor& x, Whose whose)
+{
+    const int64_t M = dy.size(0), N = dy.size(1), K = w.size(1);
+    if (w.size(0) == N && x.size(0) == M && x.size(1) == K && own_may(MHFFN_PRODUCT_NN, whose, dy, w, M, K, N) &&
+        own_may(MHFFN_PRODUCT_TN, whose, dy, x, N, K, M) && mhffn_product_pair_faster(whose == OWN_IN_ORDER, (int)M, (int)N, (int)K)) {
+        OnDevice on_device(dy);
+        Tensor dx, dw;
+        {
+            RECORD_FUNCTION("mhffn::product", std::vector<c10::IValue>());      // (one for each product)
+            dx = empty_of({M, K}, at::kBFloat16, dy);
+        }
+        RECORD_FUNCTION("mhffn::product", std::vector<c10::IValue>());
+        dw = empty_of({N, K}, at::kBFloat16, dy);
+        raise_for_code(mhffn_product_pair(ptr(dy), ptr(w), ptr(x), ptr(dx), ptr(dw), (int)M, (int)N, (int)K, stream()), "mhffn_product_pair");
+        return {dx, dw};
+    }
+    return {product_nn(dy, w, whose), product_tn(dy, x, whose)};
+}
+
 // A linear layer without bias (Projection in mhffn_layer.py).
 struct LinearNode : torch::autograd::Function<LinearNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, int64_t whose)
@@ -402,12 +426,15 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
         const Whose whose = Whose(ctx->saved_data["whose"].toInt());
         const Tensor dy = g[0].reshape({-1, g[0].size(-1)});
         Tensor dx, dw;
-        if (ctx->needs_input_grad(0)) {
+        const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
+        if (need_x && need_w) std::tie(dx, dw) = product_pair(dy, w, x.reshape({-1, x.size(-1)}), whose);
+        else if (need_x) dx = product_nn(dy, w, whose);
+        else if (need_w) dw = product_tn(dy, x.reshape({-1, x.size(-1)}), whose);
+        if (need_x) {
             at::DimVector sizes(g[0].sizes());
             sizes.back() = w.size(1);
-            dx = product_nn(dy, w, whose).view(sizes);
+            dx = dx.view(sizes);
         }
-        if (ctx->needs_input_grad(1)) dw = product_tn(dy, x.reshape({-1, x.size(-1)}), whose);
         return {dx, dw, Tensor()};
     }
 };
@@ -483,21 +510,21 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         variable_list g(5), h(3);
         // (the products of a linear layer's own backward: d_in = d_out w, d_w = d_out^T in)
         const Tensor dY = grads[0].reshape({-1, hid});
-        if (asked(after_nw + 4, after_nw + 5)) {
-            Tensor O4 = s[13];
-            if (at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
-                O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose);
-            dw2 = product_tn(dY, O4.reshape({-1, hid}), whose);
-        }
-        if (prologue || experts) {
-            const Tensor dO = product_nn(dY, w2, whose).view(s[13].sizes());
-            g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.transpose(1, 2), K.scalar_type(), one_part);
-        }
+        auto both = [&](bool need_in, bool need_w, const Tensor& d, const Tensor& w, const Tensor& in) -> std::pair<Tensor, Tensor> {
+            if (need_in && need_w) return product_pair(d, w, in, whose);
+            return {need_in ? product_nn(d, w, whose) : Tensor(), need_w ? product_tn(d, in, whose) : Tensor()};
+        };
+        const bool need_w2 = asked(after_nw + 4, after_nw + 5);
+        Tensor dO, O4 = s[13];
+        if (need_w2 && at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
+            O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose);
+        std::tie(dO, dw2) = both(prologue || experts, need_w2, dY, w2, O4.reshape({-1, hid}));
+        if (prologue || experts)
+            g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.view(s[13].sizes()).transpose(1, 2), K.scalar_type(), one_part);
         if (prologue) {
             h = gate_backward(x4, nw, router, wn, wr, eps, g[0], g[4]);
-            const Tensor dp = h[0].view({-1, hid});
-            if (ctx->needs_input_grad(0)) dx = product_nn(dp, w1, whose).view(x.sizes());
-            if (ctx->needs_input_grad(1)) dw1 = product_tn(dp, x.reshape({-1, hid}), whose);
+            std::tie(dx, dw1) = both(ctx->needs_input_grad(0), ctx->needs_input_grad(1), h[0].view({-1, hid}), w1, x.reshape({-1, hid}));
+            if (dx.defined()) dx = dx.view(x.sizes());
         }
         return {dx, dw1, h[1], h[2], g[1], g[2], g[3], dw2, Tensor(), Tensor(), Tensor()};
     }

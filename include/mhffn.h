@@ -238,6 +238,11 @@ int mhffn_product_preferred(int M, int N);
 int mhffn_product_faster(int form, int in_order, int M, int N, int K);
 int mhffn_product_tile(int form, int in_order, int M, int N, int K);
 int mhffn_product(int form, int in_order, const void* A, const void* B, void* C, int M, int N, int K, void* stream);
+/* The backward of y[M,N] = x[M,K] w[N,K]^T in one launch: dx[M,K] = dy w and dw[N,K] = dy^T x, with the bits of mhffn_product's NN and
+ * TN forms.  M free, N and K multiples of 8, all matrices contiguous on 16-byte boundaries.  mhffn_product_pair_faster() is 1 where
+ * that is faster than two launches, of which the library's may be one (0: slower, or extents refused). */
+int mhffn_product_pair_faster(int in_order, int M, int N, int K);
+int mhffn_product_pair(const void* dy, const void* w, const void* x, void* dx, void* dw, int M, int N, int K, void* stream);
 
 #ifdef __cplusplus
 }

@@ -205,3 +205,23 @@ def test_a_decoder_of_linear_layers_has_the_same_bits(B, S):
         results.append((loss, *torch.autograd.grad(loss, list(m.parameters()))))
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+# (y = x w^T of M x K by N x K.)  Edges of every tile, one workgroup to several rounds, sums shorter than a stage and longer than the ring
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (1, 64, 64), (37, 72, 40), (64, 1096, 264), (129, 136, 1000), (300, 768, 768), (512, 1024, 1024),
+                                   (700, 768, 768), (733, 1032, 1032), (1024, 1024, 1024), (1025, 768, 768), (1500, 1024, 1024),
+                                   (2056, 1544, 520), (4104, 768, 768), (512, 8192, 264), (700, 2048, 2048), (512, 3072, 1024), (512, 2048, 2048)])
+def test_a_pair_has_the_bits_of_its_products(M, N, K):
+    dev = "cuda:0"
+    print(f"M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    nan = torch.full((64,), float("nan"), device=dev, dtype=torch.bfloat16)
+    # (behind the operands lies what must not be read, behind the results what must not be touched)
+    dy, w, x = (torch.cat([torch.randn(n, generator=g, device=dev).bfloat16(), nan]) for n in (M * N, N * K, M * K))
+    out = [torch.full((n + 64,), 7.0, device=dev, dtype=torch.bfloat16) for n in (M * K, N * K, M * K, N * K)]
+    L, st = _capi.lib(), torch.cuda.current_stream().cuda_stream
+    assert L.mhffn_product_pair(dy.data_ptr(), w.data_ptr(), x.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), M, N, K, st) == _capi.OK
+    assert L.mhffn_product(NN, 1, dy.data_ptr(), w.data_ptr(), out[2].data_ptr(), M, K, N, st) == _capi.OK
+    assert L.mhffn_product(TN, 1, dy.data_ptr(), x.data_ptr(), out[3].data_ptr(), N, K, M, st) == _capi.OK
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3]) and all((o[-64:] == 7.0).all() for o in out)
+    assert torch.isfinite(out[0]).all() and torch.isfinite(out[1]).all()
