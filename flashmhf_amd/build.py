@@ -128,11 +128,12 @@ def parse_resource_usage(stderr_text):
 # Kernels whose code assumes that every value stays in registers, as (name fragment, instantiations expected).
 EXPECTED_KERNELS = (
     ("mhffn_fwd_kernel", 3), ("mhffn_bwd_dqdr_kernel", 3), ("mhffn_bwd_dkdudv_kernel", 6),
-    ("mhffn_gate_fwd_kernel", 24), ("mhffn_gate_bwd_kernel", 18),
+    ("mhffn_gate_fwd_kernel", 12), ("mhffn_gate_bwd_kernel", 12),
 )
 # Variants of those kernels for smaller problems and for float32, and the products, under the same rule.
 VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
                    ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 1), ("dkdudv_split_kernelILi", 3),
+                   ("WholeRows", 18),
                    ("mhffn_product_kernel", 10), ("mhffn_product_pair_kernel", 9), ("mhffn_product_split_kernel", 2))
 # The one instantiation known to spill: head prologue backward for d_h = 128 with more than 32 experts and RMSNorm
 # (<128, 2, true>).  It is correct but slow; the block (MHFFNLayer.heads_and_gate) does not route that case to it.
@@ -145,7 +146,7 @@ def check_no_scratch(usage):
     run time.  Fails the build if the compiler reports private (scratch) memory for one of them, and also if the
     resource remarks of an expected kernel are missing (a changed remark format must not pass silently)."""
     for frag, count in EXPECTED_KERNELS:
-        found = [n for n in usage if frag in n and "ScratchSize" in usage[n]]
+        found = [n for n in usage if frag in n and "ScratchSize" in usage[n] and "WholeRows" not in n]
         if len(found) != count:
             raise RuntimeError(f"expected resource-usage remarks for {count} instantiations of {frag}, found {len(found)}")
     for name, u in usage.items():

@@ -106,6 +106,7 @@ __device__ __forceinline__ void stage_router_cols(const T* Wr, int E, unsigned c
 // 32 rows of DH values as whole rows between memory and registers or LDS, and as half rows (the 16-byte chunks 2 ks + g of row
 // l32) between LDS and the lanes that compute.  Whole rows: a wave-instruction moves the 64 chunks from 64 i on, counted along
 // the rows; chunk c of row r sits at c ^ swz(r) in LDS, which keeps 16 rows' reads of one chunk in different banks.
+struct WholeRows {};      // (mode of the kernels below)
 template <int DH>
 struct RowTile {
     static constexpr int CH = DH / 8, INS = DH / 16;
@@ -203,13 +204,14 @@ struct GateTile {
 // memory) leaves the wave as whole cache lines instead of one scattered dword per lane and expert
 constexpr size_t gate_fwd_smem(int DH, int NT) { return (size_t)2 * NT * (DH / 16) * 1024 + DH * 4 + 4 * TILE_B; }
 
-// WHOLE: the rows move between memory and the wave as whole rows, by way of its LDS; else each lane loads and stores its half row,
+// With WholeRows the rows move between memory and the wave as whole rows, by way of its LDS; else each lane loads and stores its half row,
 // in 32-byte pieces of 32 rows per instruction.  Pieces keep the path from L2 busy four times as long: 32,768 tokens of 16 heads of
 // 128 take 71.5 us with them and 62.8 with whole rows (5.0 TB/s, what a large copy reaches; loads alone in pieces 65.3), 16,384 of
 // 8 heads 18.3 and 16.9.  Few tokens wait for one tile's chain, which the way through LDS makes longer: 512 of 8 heads 6.0 and 6.3.
-template <int DH, int NT, bool NORM, bool WHOLE>
+template <int DH, int NT, bool NORM, class... Mode>
 __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 {
+    constexpr bool WHOLE = sizeof...(Mode) > 0;
     constexpr int KS = DH / 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     float* sW = reinterpret_cast<float*>(smem + 2 * NT * KS * 1024);
@@ -341,12 +343,13 @@ __device__ __forceinline__ bf16x8 z_cols(const unsigned char* tile, int lane, in
     return v;
 }
 
-// WHOLE: dX leaves as whole rows, by way of the y tile, as Q does in the forward.  32,768 tokens of 16 heads of 128 take 104 us this way,
+// With WholeRows dX leaves as whole rows, by way of the y tile, as Q does in the forward.  32,768 tokens of 16 heads of 128 take 104 us this way,
 // 112 in half rows' pieces; with one or two tiles per wave the way through LDS is not hidden (12,288 of 8 heads 35.0 and 34.5).
 // (x and dQ as whole rows, too, take registers: 108 us with a spill, 111 for x alone.)
-template <int DH, int NT, bool NORM, bool WHOLE>
+template <int DH, int NT, bool NORM, class... Mode>
 __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
 {
+    constexpr bool WHOLE = sizeof...(Mode) > 0;
     const int NW = NT == 1 ? (int)blockDim.x / 64 : 4;
     constexpr int KS = DH / 16, CT = DH / 32, REGION_B = gate_bwd_region<NT>();
     constexpr bool AHEAD = NT > 1;                              // rows requested one tile ahead; d_norm_weight in registers
@@ -787,9 +790,8 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
     if (backward) {
         const int most = (int)gate_bwd_smem<NT>(DH, gate_bwd_max_waves<NT>()), waves = gate_bwd_waves(d);
         const dim3 grid = gate_bwd_grid(d, a.tpw);
-        constexpr bool CAN = NT == 1;
-        const bool whole = CAN && a.tpw >= 4;
-        auto* fn = whole ? mhffn_gate_bwd_kernel<DH, NT, NORM, CAN> : mhffn_gate_bwd_kernel<DH, NT, NORM, false>;
+        const bool whole = NT == 1 && a.tpw >= 4;
+        auto* fn = whole ? mhffn_gate_bwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_bwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_bwd[whole], (const void*)fn, most);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(fn, grid, dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
@@ -798,7 +800,7 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
         // whole rows from six tiles per compute unit on (us in pieces / whole: 1,024 tiles of 8 heads of 128 7.5 / 7.8, 1,536 9.6 / 9.2, 2,048
         // 11.4 / 10.3; of 96 6.5 / 6.7, 8.6 / 8.4 with 2,048; of 64 6.5 / 6.4 with 2,048)
         const bool whole = (long)a.B * a.H * ((a.S + 31) / 32) >= 6 * CUS;
-        auto* fn = whole ? mhffn_gate_fwd_kernel<DH, NT, NORM, true> : mhffn_gate_fwd_kernel<DH, NT, NORM, false>;
+        auto* fn = whole ? mhffn_gate_fwd_kernel<DH, NT, NORM, WholeRows> : mhffn_gate_fwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_fwd[whole], (const void*)fn, (int)smem);
         if (e != hipSuccess) return e;
         a.tpw = tiles_per_wave(a.B, a.H, a.S, 8192, 16);
