@@ -510,14 +510,13 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
 }
 
 // Adds the parts' sums of dQ (in the order of the parts) and rounds once, four columns per lane; adds the sums of dR over the
-// parts that hold blocks of the expert, one value per lane.  blockIdx.x < dq_blocks: dQ, otherwise dR.
+// parts that hold blocks of the expert, one value per lane.  Workgroup `block` of head hk: below dq_blocks dQ, otherwise dR.
 template <int DH>
-__global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsigned dq_blocks)
+__device__ __forceinline__ void dqdr_sum(const DqArgs& p, int hk, unsigned block, unsigned dq_blocks)
 {
-    const int hk = blockIdx.y;
     const long hrows = (long)p.rows.Hkuv * p.rows.n;
-    if (blockIdx.x < dq_blocks) {
-        const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (block < dq_blocks) {
+        const unsigned i = block * 256 + threadIdx.x;
         const unsigned r = i / (DH / 4), c = (i % (DH / 4)) * 4;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
@@ -528,7 +527,7 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsig
         for (int x = 0; x < 4; ++x) v[x] = (bf16_t)sum[x];
         *reinterpret_cast<bf16x4*>(p.dQ + p.rows.tok(hk, r) * DH + c) = v;
     } else {
-        const unsigned i = (blockIdx.x - dq_blocks) * 256 + threadIdx.x;
+        const unsigned i = (block - dq_blocks) * 256 + threadIdx.x;
         const int E = p.parts.E;
         const unsigned r = i / (unsigned)E;
         const int e = i - r * E;
@@ -537,6 +536,11 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsig
         p.dR[p.rows.gate(hk, r) * E + e] =
             sum_in_order(0.0f, p.parts.part_lo(e), p.parts.part_hi(e), [&](int z) { return src[z * hrows * E]; });
     }
+}
+template <int DH>
+__global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsigned dq_blocks)
+{
+    dqdr_sum<DH>(p, blockIdx.y, blockIdx.x, dq_blocks);
 }
 
 // ------------------------------------------------------------------------------------------------ dK / dU / dV
@@ -1028,15 +1032,13 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     }
 }
 
-// Sums the token-slice partials of dK, dU or dV (blockIdx.y) and converts to the output dtype, four values per lane.
+// Sums the token-slice partials of dK, dU or dV (w = 0, 1, 2) and converts to the output dtype, four values per lane.
 template <typename OutT>
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ part, OutT* dK, OutT* dU, OutT* dV,
-                                                              long wsz, int nslice)
+__device__ __forceinline__ void slice_sum(const float* __restrict__ part, OutT* dK, OutT* dU, OutT* dV, long wsz, int nslice, int w, unsigned block)
 {
     typedef OutT OutT4 __attribute__((ext_vector_type(4)));
-    const long i4 = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+    const long i4 = ((long)block * 256 + threadIdx.x) * 4;
     if (i4 >= wsz) return;
-    const int w = blockIdx.y;
     const float* src = part + w * wsz + i4;
     auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + 3 * z * wsz); };
     const f32x4 sum = sum_in_order(load(0), 1, nslice, load);
@@ -1044,6 +1046,29 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
 #pragma unroll
     for (int x = 0; x < 4; ++x) v[x] = (OutT)sum[x];
     *reinterpret_cast<OutT4*>((w == 0 ? dK : w == 1 ? dU : dV) + i4) = v;
+}
+template <typename OutT>
+__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ part, OutT* dK, OutT* dU, OutT* dV,
+                                                              long wsz, int nslice)
+{
+    slice_sum(part, dK, dU, dV, wsz, nslice, blockIdx.y, blockIdx.x);
+}
+
+// Both sums of a backward in one launch, behind both its kernels: a launch less, and one pass fills the chip where two were
+// latency (2 x 300 tokens of 8 heads of 96, two K/U/V heads: 4.9 + 7.0 us under the profiler, 10.0 in one; the call, bound by the host there, 99 -> 92).  Workgroups: dq_blocks of dQ and
+// r_blocks of dR per head, then w_blocks of each gradient.
+template <int DH, typename OutT>
+__global__ __launch_bounds__(256) void mhffn_bwd_sums_kernel(DqArgs p, unsigned dq_blocks, unsigned head_blocks, const float* __restrict__ part,
+                                                             OutT* dK, OutT* dU, OutT* dV, long wsz, int nslice, unsigned w_blocks)
+{
+    const unsigned heads = head_blocks * p.rows.Hkuv;
+    if (blockIdx.x < heads) {
+        const unsigned hk = blockIdx.x / head_blocks;
+        dqdr_sum<DH>(p, hk, blockIdx.x - hk * head_blocks, dq_blocks);
+    } else {
+        const unsigned b = blockIdx.x - heads, w = b / w_blocks;
+        slice_sum(part, dK, dU, dV, wsz, nslice, w, b - w * w_blocks);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ host side
@@ -1093,13 +1118,13 @@ size_t bwd_min_workspace_bytes_bf16(const Dims& d)
     return ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
 }
 
-// The two kernels run one after the other, so the parts of dQ, dR and the token slices of dK, dU, dV share the workspace.
+// The parts of dQ, dR lie behind the token slices of dK, dU, dV, so that one launch can add up both.  Where they do not fit there
+// they share the workspace, and are added up before the slices are written.
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
     const int nq = dq_pick_bf16(d, ~(size_t)0, 0).nsplit;
     const size_t dw = bwd_min_workspace_bytes_bf16(d);
-    const size_t dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
-    return dw > dq ? dw : dq;
+    return dw + (nq > 1 ? align256(nq * dq_part_bytes(d)) : 0);
 }
 
 template <int DH>
@@ -1109,13 +1134,18 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
 {
     hipError_t err = hipSuccess;
     float* part = reinterpret_cast<float*>(ws);
-    const int nbe = d.d_e / JB, G = d.H / d.Hkuv;
+    const int nbe = d.d_e / JB, G = d.H / d.Hkuv, nslice = dw_slices_bf16(d, ws_bytes);
+    const long wsz = (long)d.Hkuv * d.E * d.d_e * d.d_h;
+    const Pick pick = dq_pick_bf16(d, ws ? ws_bytes : 0, phases);
+    const size_t slices_b = align256((size_t)nslice * 3 * wsz * sizeof(float));
+    constexpr int ALL = PH_BWD_DQDR | PH_BWD_DKDUDV | PH_BWD_REDUCE;
+    const bool together = (phases & ALL) == ALL && nslice > 1 && pick.nsplit > 1 && slices_b + pick.nsplit * dq_part_bytes(d) <= ws_bytes;
+    DqArgs dq{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, (bf16_t*)dQ, dR,
+              together ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + slices_b) : part, RowMap(d), Parts(d.E, nbe, pick.nsplit)};
+    const unsigned qb = (unsigned)(((long)dq.rows.n * (DH / 4) + 255) / 256), rb = (unsigned)(((long)dq.rows.n * d.E + 255) / 256);
 
     if (phases & PH_BWD_DQDR) {
-        const Pick pick = dq_pick_bf16(d, ws ? ws_bytes : 0, phases);
-        DqArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R,
-                 (bf16_t*)dQ, dR, part, RowMap(d),
-                 Parts(d.E, nbe, pick.nsplit)};
+        const DqArgs& a = dq;
         const int tokw = pick.tile_rows;
         const int smem = (tokw == 32 ? DQ32_R0 : DQ_NST * DQ_STAGE_B) +
                          (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
@@ -1127,15 +1157,11 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
         dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
         if (tokw == 32) hipLaunchKernelGGL((mhffn_bwd_dqdr_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
         else hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
-        if (a.parts.nsplit > 1) {
-            const unsigned qb = (unsigned)(((long)a.rows.n * (DH / 4) + 255) / 256);
-            const unsigned rb = (unsigned)(((long)a.rows.n * d.E + 255) / 256);
+        if (a.parts.nsplit > 1 && !together)
             hipLaunchKernelGGL((mhffn_bwd_dqdr_sum_kernel<DH>), dim3(qb + rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, qb);
-        }
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
-    const int nslice = dw_slices_bf16(d, ws_bytes);
     if (phases & PH_BWD_DKDUDV) {
         DwArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, part,
                  {dK, dU, dV}, grad_w_f32, d.B, d.H, G, d.S, d.E, nbe, nslice, d.tokmaj};
@@ -1154,9 +1180,15 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
         if (err != hipSuccess) return err;
     }
     if ((phases & PH_BWD_REDUCE) && nslice > 1) {
-        const long wsz = (long)d.Hkuv * d.E * d.d_e * d.d_h;
         const unsigned rblocks = (unsigned)((wsz / 4 + 255) / 256);
-        if (grad_w_f32)
+        const unsigned all = (qb + rb) * d.Hkuv + 3 * rblocks;
+        if (together && grad_w_f32)
+            hipLaunchKernelGGL((mhffn_bwd_sums_kernel<DH, float>), dim3(all), dim3(256), 0, st, dq, qb, qb + rb, part, (float*)dK, (float*)dU,
+                               (float*)dV, wsz, nslice, rblocks);
+        else if (together)
+            hipLaunchKernelGGL((mhffn_bwd_sums_kernel<DH, bf16_t>), dim3(all), dim3(256), 0, st, dq, qb, qb + rb, part, (bf16_t*)dK, (bf16_t*)dU,
+                               (bf16_t*)dV, wsz, nslice, rblocks);
+        else if (grad_w_f32)
             hipLaunchKernelGGL((reduce_partials_kernel<float>), dim3(rblocks, 3), dim3(256), 0, st, part, (float*)dK,
                                (float*)dU, (float*)dV, wsz, nslice);
         else

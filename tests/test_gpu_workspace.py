@@ -56,3 +56,21 @@ def test_backward_runs_with_less_workspace(shape, dtype):
                 assert all(torch.equal(a, b) for a, b in zip(one, got))
     if need:
         assert _bwd(L, ins, dims, dtype, need - 16)[0] == _capi.ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("shape", [(2, 8, 300, 96, 8, 256, 2), (3, 4, 43, 64, 7, 96, 1), (1, 1, 700, 128, 9, 256, 1)])
+@pytest.mark.parametrize("weights", [torch.bfloat16, torch.float32])
+def test_sums_in_one_launch_have_the_bits_of_two(shape, weights):
+    """With room for the parts of dQ, dR behind the token slices of dK, dU, dV one launch adds up both; with less they take turns."""
+    from flashmhf_amd import _capi
+    print("case", shape, weights, flush=True)
+    L = _capi.lib()
+    B, H, S, dh, E, de, Hk = shape
+    dims, code = _capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_BF16
+    plan = _capi.launch_plan(dims, code)
+    assert plan.dqdr_parts > 1 and plan.dkdudv_slices > 1
+    ins = [t.to(DEV) for t in make_inputs(B, H, S, dh, E, de, Hk, seed=2, dtype=torch.bfloat16)]
+    most = L.mhffn_bwd_workspace_bytes(dims, code)
+    results = [_bwd(L, ins, dims, weights, b) for b in (most, most - 256)]
+    assert [rc for rc, _ in results] == [0, 0]
+    assert all(torch.equal(a, b) for a, b in zip(results[0][1], results[1][1]))
