@@ -290,222 +290,276 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
     }
 }
 
-// 32 rows, four blocks a trip: the same products, element-wise formulas and order of sums as the kernel above.  K and U tiles
-// are read by all waves to the end of a trip, V only by its own wave's first products.  K tiles have two sets; LDS has no
-// room for a second set of U too, whose next tile waits in registers instead.  dR is one running sum over the elements of an
-// expert's blocks: wave k adds those of its block to what wave k - 1 left (an exchange of the terms would take another 32 KB of
-// LDS).  A number in LDS says whose turn it is -- the blocks added so far; a wave looks for its own in front of its second products of
-// its own block, by when the wave before has had the time of one block's products, and nobody else waits: 2.45 us a trip, against
-// 2.7 with a barrier behind each of the four.  (Wave 0's number is there since the trip before, so every wait ends.)
-// A lone wave stands still while the loads that it has issued wait for the path to LDS: the next trip's K and U are requested one
-// instruction of each behind a k-step of the first products, V two behind four elements, instead of in bursts: 2.39 us.
-constexpr int DQ32_U0 = 2 * QUAD * TILE_B, DQ32_V0 = DQ32_U0 + QUAD * TILE_B, DQ32_D0 = DQ32_V0 + QUAD * TILE_B,
-              DQ32_E0 = DQ32_D0 + QUAD * 4096, DQ32_T0 = DQ32_E0 + 256, DQ32_R0 = DQ32_T0 + 256;
+// 32 rows, the blocks in a pipeline: the same products, element-wise formulas and order of sums as the kernel above.  Four waves
+// take the first products and the element-wise work, each of every fourth block, in four phases of about equal length and a
+// phase apart from each other; four more request the tiles, 24 KB a phase, and add one block a phase to dQ, a column tile
+// each.  A SIMD has one wave of either kind.  (Four waves that did all of it for four blocks at a time, products, element-wise code,
+// barrier, sums, barrier, took 0.60 us a block, most of it the chain of these; a phase takes 0.42 us at half a chip, 0.53 where
+// every compute unit has a workgroup.  By s_memtime, of the 870 cycles of a phase a wave works 560 to 720, and none of the four
+// phases and neither kind of wave stands out; without the fills 0.41.  First products in one phase: 0.56.  512 rows of the
+// 370M heads in one part 78.9 -> 52.5 us, of 8 heads of 96 40.1 -> 27.7, of 64 37.5 -> 28.3.)
+// What a phase reads was there before the barrier in front of it wherever it can be: V's and the transposed K and U operands are
+// requested a phase ahead.  dR is one running sum over the elements of an expert's blocks, which the wave of a block hands to the
+// wave of the next through LDS.  Loads go out three phases ahead of their block.
+constexpr int DQ32_A = 4, DQ32_W = DQ32_A + 4;        // waves of the first kind, and all; also a block's phases up to its sums
+constexpr int DQ32_AHEAD = 7 - DQ32_A;                 // phases between the request of a block's tiles and its first products
+constexpr int DQ32_KU = 7, DQ32_V = DQ32_AHEAD + 1;    // tile sets: a block's K and U from the request to its sums, V to its first products
+constexpr int DQ32_V0 = DQ32_KU * 2 * TILE_B, DQ32_D0 = DQ32_V0 + DQ32_V * TILE_B, DQ32_E0 = DQ32_D0 + 2 * 4096, DQ32_SMEM = DQ32_E0 + 256;
 template <int DH>
-__global__ __launch_bounds__(256) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
+__global__ __launch_bounds__(DQ32_W * 64) void mhffn_bwd_dqdr_rows32_kernel(DqArgs p)
 {
     constexpr int KS = DH / 16, CT = DH / 32;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    float* sR = reinterpret_cast<float*>(smem + DQ32_R0);                 // [E][32]
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
     const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
     const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
-    const int nex = p.parts.by_nbe.div(jb0 + nblk + nbe - 1);
     const bf16_t* Kh = p.K + ((long)hk * E * nbe + blk0) * JB * DH;
-    const long offU = p.U - p.K, offV = p.V - p.K;
-    unsigned char *ownU = smem + DQ32_U0 + wave * TILE_B, *ownV = smem + DQ32_V0 + wave * TILE_B;
-    auto row_of = [&](int t) { return tok0 + t < p.rows.n ? tok0 + t : p.rows.n - 1; };
-    auto block = [&](int b0) { return Kh + (long)(b0 + wave < nblk ? b0 + wave : nblk - 1) * JB * DH; };
-    // U through registers, coalesced as the fills are: row lane / 16 of every group of four, 16-byte chunk lane % 16 (a narrow
-    // row's unused chunks take chunk 0)
-    u32x4 un[8];
-    auto load_u = [&](int b0, int i) {
-        const int c = (lane & 15) < DH / 8 ? lane & 15 : 0;
-        un[i] = *reinterpret_cast<const u32x4*>(block(b0) + offU + (lane >> 4) * DH + c * 8 + 4 * i * DH);
-    };
-    auto store_u = [&]() {
-        static_for<8>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            const int r = 4 * i + (lane >> 4);
-            lds_write16<0>(lds_addr(ownU) + r * TILE_ROW_B + (((lane & 15) ^ swz16(r)) << 4), un[i]);
-        });
-    };
+    const unsigned smem0 = lds_addr(smem);
+    const int nphase = nblk + DQ32_A;      // block b: first products in phase b, its sums in phase b + DQ32_A; every phase ends with a barrier
 
-    bf16x8 q[KS], go[KS];
-    {
-        const long row = p.rows.tok(hk, row_of(l32)) * DH + 8 * g;
+    if (wave < DQ32_A) {
+        const int t = tok0 + l32 < p.rows.n ? tok0 + l32 : p.rows.n - 1;
+        const long grow = p.rows.gate(hk, t) * E;
+        bf16x8 q[KS], go[KS];
+        {
+            const long row = p.rows.tok(hk, t) * DH + 8 * g;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            q[ks] = *reinterpret_cast<const bf16x8*>(p.Q + row + ks * 16);
-            go[ks] = *reinterpret_cast<const bf16x8*>(p.dO + row + ks * 16);
+            for (int ks = 0; ks < KS; ++ks) {
+                q[ks] = *reinterpret_cast<const bf16x8*>(p.Q + row + ks * 16);
+                go[ks] = *reinterpret_cast<const bf16x8*>(p.dO + row + ks * 16);
+            }
         }
-    }
-    quad_stage_gates(sR, p.R + ex0, nex, tid, [&](int t) { return p.rows.gate(hk, row_of(t)) * E; });
-    if (tid == 0) *reinterpret_cast<int*>(smem + DQ32_T0) = 0;
-    // (from here to the end of the loop the vmcnt events are the fills, the loads of U and the stores of dR)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]), "+v"(go[ks]));
-    __syncthreads();          // the gate values
-#pragma unroll
-    for (int i = 0; i < 8; ++i) load_u(0, i);
-    quad_fill<DH>(block(0), smem + wave * TILE_B, lane);
-    quad_fill<DH>(block(0) + offV, ownV, lane);
-    float* drow;
-    {
-        const int t = row_of(l32);
+        const float* rrow = p.R + grow + ex0;
         const long hrows = (long)p.rows.Hkuv * p.rows.n;
-        drow = nsplit == 1 ? p.dR + p.rows.gate(hk, t) * E
-                           : p.part + nsplit * hrows * DH + (z * hrows + (long)hk * p.rows.n + t) * E + ex0;
-    }
-    f32x16 dq;
+        float* drow = nsplit == 1 ? p.dR + grow : p.part + nsplit * hrows * DH + (z * hrows + (long)hk * p.rows.n + t) * E + ex0;
+        auto gate = [&](int b) { return rrow[p.parts.by_nbe.div(jb0 + (b < nblk ? b : nblk - 1))]; };
+        float r = 0.0f, rnext = gate(wave);
+        // (these loads end here: waited for in the loop, each trip would also wait for the next gate value)
 #pragma unroll
-    for (int x = 0; x < 16; ++x) dq[x] = 0.0f;
-    const int krow = row_perm32(l32);
+        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]), "+v"(go[ks]));
+        asm volatile("" : "+v"(rnext));
+        const int krow = row_perm32(l32), sw = swz16(krow);
+        unsigned at[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) at[ks] = smem0 + krow * TILE_ROW_B + (((2 * ks + g) ^ sw) << 4);
+        const unsigned sD = smem0 + DQ32_D0 + lane * 16, sE = smem0 + DQ32_E0 + lane * 4;
+
+        f32x16 m, n, da, sg;
+        f32x16 as;                // as, n: the factors of dR's terms
+        bf16x8 dmt[2], dnt[2];
+        QuadRows<KS, 2> a;
+        QuadRows<KS, 1> av;
+        // Phase 1: K1 k-steps of M and N, with the reads of the others and of V between the matrix instructions.
+        constexpr int K1 = KS / 2, FIRST = KS - K1;
+        auto phase1 = [&](int b) {
+            r = rnext;
+            rnext = gate(b + DQ32_A);      // a round ahead of its use
+            const unsigned ku = (b % DQ32_KU) * 2 * TILE_B, v = DQ32_V0 + (b % DQ32_V) * TILE_B;
+            auto request = [&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                const unsigned x = at[ks] + ku;
+                a.template request<0, ks>(x);
+                a.template request<1, ks, TILE_B>(x);
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<FIRST>([&](auto kc) { request(kc); });
+#pragma unroll
+            for (int x = 0; x < 16; ++x) { m[x] = 0.0f; n[x] = 0.0f; }
+            // behind k-step ks: the reads of k-step FIRST + ks and as many of V as leaves none for the last one
+            constexpr int VN = (KS + K1 - 1) / K1;
+            static_for<K1>([&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                constexpr int kus = (FIRST + ks < KS ? FIRST + ks : KS) - (ks + 1), vs = ks * VN < KS ? ks * VN : KS;
+                lds_wait_n<(2 * kus + vs < 15 ? 2 * kus + vs : 15)>();
+                asm volatile("" : "+v"(a.v[0][ks]), "+v"(a.v[1][ks]));
+                m = mfma32(a.get(0, ks), q[ks], m);
+                n = mfma32(a.get(1, ks), q[ks], n);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (FIRST + ks < KS) request(std::integral_constant<int, FIRST + ks>{});
+                static_for<VN>([&](auto vc) {
+                    constexpr int k = ks * VN + decltype(vc)::value;
+                    if constexpr (k < KS) av.template request<0, k>(at[k] + v);
+                });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            static_assert(FIRST + K1 >= KS, "every k-step's operands are requested in phase 1");
+        };
+        // Phase 2: the other k-steps, then dA with the sigmoids of the first elements under its matrix instructions.
+        constexpr int SIG = 6;
+        auto phase2 = [&]() {
+            static_for<KS - K1>([&](auto kc) {
+                constexpr int ks = K1 + decltype(kc)::value;
+                asm volatile("" : "+v"(a.v[0][ks]), "+v"(a.v[1][ks]));       // (returned before the barrier, as V's)
+                m = mfma32(a.get(0, ks), q[ks], m);
+                n = mfma32(a.get(1, ks), q[ks], n);
+            });
+#pragma unroll
+            for (int x = 0; x < 16; ++x) da[x] = 0.0f;
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<KS>([&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                asm volatile("" : "+v"(av.v[0][ks]));
+                da = mfma32(av.get(0, ks), go[ks], da);
+#pragma unroll
+                for (int i = ks * SIG / KS; i < (ks + 1) * SIG / KS; ++i) sg[i] = fast_sigmoid(m[i]);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        auto elements = [&](auto i0_, auto i1_) {
+            constexpr int i0 = decltype(i0_)::value, i1 = decltype(i1_)::value;
+#pragma unroll
+            for (int i = i0 < SIG ? SIG : i0; i < i1; ++i) sg[i] = fast_sigmoid(m[i]);
+#pragma unroll
+            for (int i = i0; i < i1; ++i) {
+                const float x = m[i], nn = n[i], a = da[i];
+                const float sl = x * sg[i];              // silu(m)
+                as[i] = a * sl;
+                const float w = __builtin_fmaf(sl, 1.0f - sg[i], sg[i]);    // silu'(m)
+                dnt[i >> 3][i & 7] = (bf16_t)(r * as[i]);
+                dmt[i >> 3][i & 7] = (bf16_t)((r * a) * (nn * w));
+            }
+        };
+        // The running sum of dR goes from block to block through LDS: the block before has left it a phase ago.
+        auto gate_gradient = [&](int b, const u32x2& in) {
+            const int j = jb0 + b, e = p.parts.by_nbe.div(j), jb = j - e * nbe;
+            const unsigned bits = in[0];
+            float dr = jb == 0 || b == 0 ? 0.0f : __builtin_bit_cast(float, bits);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dr = __builtin_fmaf(as[i], n[i], dr);
+            lds_write4(sE, dr);
+            if (jb == nbe - 1 || b == nblk - 1) {
+                const float tot = dr + __shfl_xor(dr, 32);      // the lane halves hold disjoint j rows of one token column
+                if (g == 0 && tok0 + l32 < p.rows.n) drow[e] = tot;
+            }
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I12 = std::integral_constant<int, 12>;
+        using I16 = std::integral_constant<int, 16>;
+        for (int i = 0; i <= wave; ++i) quad_barrier();      // (the first: block 0 has landed)
+        int phase = wave;
+        for (int b = wave; b < nblk; b += DQ32_A, phase += DQ32_A) {
+            phase1(b);
+            quad_barrier();
+            phase2();
+            quad_barrier();
+            elements(I0{}, I12{});
+            asm volatile("" : "+v"(dmt[0]), "+v"(dnt[0]), "+v"(dmt[1]), "+v"(dnt[1]), "+v"(as));     // (here, not behind the barrier)
+            const unsigned d = sD + (b & 1) * 4096;
+            quad_barrier();
+            u32x2 in = lds_read_apart_async<1>(sE);
+            lds_write16<0>(d, dmt[0]);
+            lds_write16<2048>(d, dnt[0]);
+            elements(I12{}, I16{});
+            lds_write16<1024>(d, dmt[1]);
+            lds_write16<3072>(d, dnt[1]);
+            asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(in));
+            gate_gradient(b, in);
+            quad_barrier();
+        }
+        for (; phase <= nphase; ++phase) quad_barrier();     // (and the one in front of the epilogue)
+        return;
+    }
+
+    // Fills and sums.  Each of these waves requests a quarter of every tile: six vmcnt events a block.
+    const int col = wave - DQ32_A;
+    const long offU = p.U - p.K, offV = p.V - p.K;
+    int ku = 0, v = 0;                     // tile sets of the next block to request
+    // (a lane's place in a row group of the tile as a 32-bit offset to a uniform base; a narrow row's unused chunks take chunk 0)
+    unsigned place[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int row = 4 * (2 * col + i) + (lane >> 4), c = (lane & 15) ^ swz16(row);
+        place[i] = (row * DH + (c < DH / 8 ? c : 0) * 8) * 2;
+    }
+    const char* src;
+    unsigned char *tku, *tv;
+    auto aim = [&](int b) {
+        src = reinterpret_cast<const char*>(Kh + (long)(b < nblk ? b : nblk - 1) * JB * DH);
+        asm("" : "+s"(src));               // (kept apart from the lane's offset: one scalar addition per fill)
+        tku = smem + ku * 2 * TILE_B + 2 * col * 1024;
+        tv = smem + DQ32_V0 + v * TILE_B + 2 * col * 1024;
+        ku = ku + 1 == DQ32_KU ? 0 : ku + 1;
+        v = v + 1 == DQ32_V ? 0 : v + 1;
+    };
+    auto fill = [&](auto tensor_, auto i_) {
+        constexpr int T = decltype(tensor_)::value, i = decltype(i_)::value;
+        const char* from = src + 2 * (T == 0 ? 0 : T == 1 ? offU : offV);
+        unsigned char* to = (T == 2 ? tv : tku + T * TILE_B) + i * 1024;
+        __builtin_amdgcn_global_load_lds((gptr_t)(from + place[i]), (lptr_t)to, 16, 0, 0);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
     const TrLane<CT> trl = make_tr_lane<CT, 8, 4>(lane);
     TrLane<1> tr{};                           // this wave's column tile
 #pragma unroll
     for (int i = 0; i < CT; ++i)
-        if (i == wave) { tr.off[0][0] = trl.off[i][0]; tr.off[0][1] = trl.off[i][1]; }
-    const unsigned smem0 = lds_addr(smem), rowoff = krow * TILE_ROW_B, sw = swz16(krow), ra = lds_addr(sR) + 4 * l32;
-    const unsigned sD = smem0 + DQ32_D0 + lane * 16, sE = smem0 + DQ32_E0 + lane * 4, sT = smem0 + DQ32_T0;
-
-    auto trip = [&](auto set_, int b0) {
-        constexpr int SET = decltype(set_)::value;
-        const unsigned sK = smem0 + SET * QUAD * TILE_B;
-        __builtin_amdgcn_sched_barrier(0);
-        store_u();            // (the barrier before was every wave's last use of the tile)
-        wait_vmcnt<0>();      // this wave's K and V of the trip have landed
-        __builtin_amdgcn_sched_barrier(0);
-        u32x2 rv = lds_read_apart_async<1>(ra + 128 * p.parts.by_nbe.div(jb0 + (b0 + wave < nblk ? b0 + wave : nblk - 1)));
-        const bf16_t* next = block(b0 + QUAD);
-        QuadRows<KS, 3> a;
-        static_for<KS>([&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            const unsigned at = rowoff + (((2 * ks + g) ^ sw) << 4);
-            a.template request<0, ks>(sK + wave * TILE_B + at);
-            a.template request<1, ks>(lds_addr(ownU) + at);
-            a.template request<2, ks>(lds_addr(ownV) + at);
+        if (i == col) { tr.off[0][0] = trl.off[i][0]; tr.off[0][1] = trl.off[i][1]; }
+    f32x16 dq;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) dq[x] = 0.0f;
+    for (int b = 0; b < DQ32_AHEAD; ++b) {
+        aim(b);
+        static_for<3>([&](auto t) {
+            fill(t, I0{});
+            fill(t, I1{});
         });
-        f32x16 m, n, da;
-#pragma unroll
-        for (int x = 0; x < 16; ++x) { m[x] = 0.0f; n[x] = 0.0f; da[x] = 0.0f; }
-        static_for<KS>([&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            a.template wait<ks>();
-            m = mfma32(a.get(0, ks), q[ks], m);
-            n = mfma32(a.get(1, ks), q[ks], n);
-            da = mfma32(a.get(2, ks), go[ks], da);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = ks * 8 / KS; i < (ks + 1) * 8 / KS; ++i) {
-                load_u(b0 + QUAD, i);
-                tile_fill_ins<DH>(next, DH, smem + ((1 - SET) * QUAD + wave) * TILE_B, i, lane);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        asm volatile("" : "+v"(rv));
-        __builtin_amdgcn_sched_barrier(0);
-        bf16x8 dmt[2], dnt[2];
-        f32x16 as;            // the first factors of dR's terms (n holds the second ones)
-        {
-            const unsigned rbits = rv[0];
-            const float r = __builtin_bit_cast(float, rbits);
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-#pragma unroll
-                for (int i = 4 * i4; i < 4 * i4 + 4; ++i) {
-                    const float x = m[i], nn = n[i], a = da[i];
-                    const float sg = fast_sigmoid(x);
-                    const float sl = x * sg;                 // silu(m)
-                    as[i] = a * sl;
-                    const float w = __builtin_fmaf(sl, 1.0f - sg, sg);    // silu'(m)
-                    dnt[i >> 3][i & 7] = (bf16_t)(r * as[i]);
-                    dmt[i >> 3][i & 7] = (bf16_t)((r * a) * (nn * w));
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int k = 2 * i4; k < 2 * i4 + 2; ++k)      // (every read of the tile has returned)
-                    tile_fill_ins<DH>(next + offV, DH, ownV, k, lane);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        lds_write16<0>(sD + wave * 4096, dmt[0]);
-        lds_write16<1024>(sD + wave * 4096, dmt[1]);
-        lds_write16<2048>(sD + wave * 4096, dnt[0]);
-        lds_write16<3072>(sD + wave * 4096, dnt[1]);
-        quad_barrier();       // the four blocks' operands and tiles
-        const int nb = nblk - b0 < QUAD ? nblk - b0 : QUAD;     // (a block that is not there is the last one again, and not used)
-        // a block's operands (twelve LDS operations) are requested one block ahead of their use
-        u32x4 d[2][4];        // dM s 0, 1, dN s 0, 1
-        TrOperand tk[2][2], tu[2][2];
-        auto request = [&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            const unsigned aK = sK + k * TILE_B, aU = smem0 + DQ32_U0 + k * TILE_B;
-            tk[k & 1][0] = tile_read_cols_async<0>(aK, tr, 0);
-            tu[k & 1][0] = tile_read_cols_async<0>(aU, tr, 0);
-            tk[k & 1][1] = tile_read_cols_async<4096>(aK, tr, 0);
-            tu[k & 1][1] = tile_read_cols_async<4096>(aU, tr, 0);
-            d[k & 1][0] = lds_read16_async<k * 4096>(sD);
-            d[k & 1][1] = lds_read16_async<k * 4096 + 1024>(sD);
-            d[k & 1][2] = lds_read16_async<k * 4096 + 2048>(sD);
-            d[k & 1][3] = lds_read16_async<k * 4096 + 3072>(sD);
-        };
-        request(std::integral_constant<int, 0>{});
-        static_for<QUAD>([&](auto kc) {
-            constexpr int k = decltype(kc)::value, c = k & 1;
-            if (k == wave && k < nb) {
-                const int at = jb0 + b0 + k, e = p.parts.by_nbe.div(at), jb = at - e * nbe;
-                u32x2 in;      // (the sum is read behind the number that is checked, and written in front of it)
-                int done;
-                do {
-                    u32x2 tag = lds_read_apart_async<1>(sT);
-                    in = lds_read_apart_async<1>(sE);
-                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tag), "+v"(in));
-                    done = __builtin_amdgcn_readfirstlane((int)tag[0]);
-                } while (done != b0 + k);
-                const unsigned bits = in[0];
-                float dr = jb == 0 || b0 + k == 0 ? 0.0f : __builtin_bit_cast(float, bits);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) dr = __builtin_fmaf(as[i], n[i], dr);
-                lds_write4(sE, dr);
-                lds_write4(sT, __builtin_bit_cast(float, b0 + k + 1));
-                if (jb == nbe - 1 || b0 + k == nblk - 1) {
-                    const float tot = dr + __shfl_xor(dr, 32);      // the lane halves hold disjoint j rows of one token column
-                    if (g == 0 && tok0 + l32 < p.rows.n) drow[e] = tot;
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if constexpr (k + 1 < QUAD) request(std::integral_constant<int, k + 1>{});
-            constexpr int younger = k + 1 < QUAD ? 12 : 0;
-            lds_tr_wait_n<younger>(tk[c][0], tu[c][0]);
-            lds_tr_wait_n<younger>(tk[c][1], tu[c][1]);
-            asm volatile("" : "+v"(d[c][0]), "+v"(d[c][1]), "+v"(d[c][2]), "+v"(d[c][3]));
-            if (k < nb && wave < CT)
-                static_for<2>([&](auto sc) {
-                    constexpr int s = decltype(sc)::value;
-                    dq = mfma32(tr_value(tk[c][s]), __builtin_bit_cast(bf16x8, d[c][s]), dq);
-                    dq = mfma32(tr_value(tu[c][s]), __builtin_bit_cast(bf16x8, d[c][2 + s]), dq);
-                });
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        quad_barrier();       // every wave is done with the tiles and the operands
-    };
-    for (int b0 = 0; b0 < nblk; b0 += 2 * QUAD) {
-        trip(std::integral_constant<int, 0>{}, b0);
-        if (b0 + QUAD < nblk) trip(std::integral_constant<int, 1>{}, b0 + QUAD);
     }
-    wait_vmcnt<0>();          // the fills of blocks that are not there write this wave's tiles, which the epilogue reuses
+    wait_vmcnt<6 * (DQ32_AHEAD - 1)>();
+    quad_barrier();                           // block 0 has landed
+    TrOperand tk[2], tu[2];
+    auto phase_of = [&](auto sums_, int phase) {
+        constexpr bool SUMS = decltype(sums_)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 d[4];                           // dM s 0, 1, dN s 0, 1
+        if constexpr (SUMS) {
+            const unsigned sD = smem0 + DQ32_D0 + ((phase - DQ32_A) & 1) * 4096 + lane * 16;
+            d[0] = lds_read16_async<0>(sD);
+            d[2] = lds_read16_async<2048>(sD);
+            d[1] = lds_read16_async<1024>(sD);
+            d[3] = lds_read16_async<3072>(sD);
+        }
+        aim(phase + DQ32_AHEAD);
+        fill(I0{}, I0{});
+        fill(I0{}, I1{});
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (SUMS) {
+            lds_wait_n<0>();
+            asm volatile("" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]));
+        }
+        // this block's sums, each operand followed by the next block's (from the tile set that the next phase requests into)
+        const unsigned aK = smem0 + ku * 2 * TILE_B;
+        static_for<4>([&](auto kc) {
+            constexpr int k = decltype(kc)::value, half = k >> 1;
+            TrOperand& t = k & 1 ? tu[half] : tk[half];
+            if constexpr (SUMS) dq = mfma32(tr_value(t), __builtin_bit_cast(bf16x8, d[(k & 1) * 2 + half]), dq);
+            __builtin_amdgcn_sched_barrier(0);
+            t = tile_read_cols_async<(k & 1) * TILE_B + half * 4096>(aK, tr, 0);
+            fill(std::integral_constant<int, (k + 2) / 2>{}, std::integral_constant<int, (k & 1)>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        wait_vmcnt<6 * (DQ32_AHEAD - 1)>();   // the next phase's first products have their tiles
+        quad_barrier();
+#pragma unroll
+        for (int s = 0; s < 2; ++s) asm volatile("" : "+v"(tk[s].lo), "+v"(tk[s].hi), "+v"(tu[s].lo), "+v"(tu[s].hi));
+    };
+    int phase = 0;
+    for (const int idle = col < CT ? DQ32_A : nphase; phase < idle; ++phase) phase_of(std::false_type{}, phase);
+    for (; phase < nphase; ++phase) phase_of(std::true_type{}, phase);
+    wait_vmcnt<0>();          // the fills of blocks that are not there write the tiles, which the epilogue reuses
+    __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (wave >= CT) return;
+    if (col >= CT) return;
+    unsigned char* own = smem + col * TILE_B;
     const int nrows = p.rows.n - tok0;
     if (nsplit > 1) {
-        float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH + 32 * wave;
-        quad_store_f32(ownV, dq, nrows, lane, [&](int row) { return prow + row * DH; });
+        float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH + 32 * col;
+        quad_store_f32(own, dq, nrows, lane, [&](int row) { return prow + row * DH; });
     } else {
-        quad_store_bf16(ownV, dq, nrows, lane, [&](int row) { return p.dQ + p.rows.tok(hk, tok0 + row) * DH + 32 * wave; });
+        quad_store_bf16(own, dq, nrows, lane, [&](int row) { return p.dQ + p.rows.tok(hk, tok0 + row) * DH + 32 * col; });
     }
 }
 
@@ -1101,11 +1155,11 @@ int dw_slices_bf16(const Dims& d, size_t ws_bytes)
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
-// Tiles of 256 rows where they fill the chip, of 32 with four blocks a trip below that: a trip takes 2.4 us (four steps of the
-// large tiles 6.6), with an eighth of the rows.  One part of 121 blocks of the 370M heads, 400 rows: 199 us with 256 rows, 77 with
-// 32; 2,048 rows: 202 and (at 2.7 us a trip, two rounds) 173; one row in 32 parts of 32-row tiles 10.1 us.  (Priced at 2.7, as the sweep
-// behind pick_parts measured it: the line between the two kernels lies where it did.)
-constexpr Variant DQ_VARIANTS[] = {{256, 1.6, 0.33, 1}, {32, 2.7, 0.05, QUAD}};
+// Tiles of 256 rows where they fill the chip, of 32 below that: a block of theirs takes a quarter of the time, with an eighth of
+// the rows.  One part of 121 blocks of the 370M heads, 512 rows: 199 us with 256 rows, 48 with 32; 2,048 rows: 200 and (two
+// rounds) 108.  At their best numbers of parts 512 rows take 34.5 us with 32 rows, 36.1 with 256, 733 rows 49.7 and 45.0.  The prices lose
+// 0.3 % on average and 4.8 % at worst over 112 calls (d_h 64, 96, 128; eight layers; 32 to 4,096 rows; up to 40 parts of either kernel).
+constexpr Variant DQ_VARIANTS[] = {{256, 1.7, 0.15, 1}, {32, 0.36, 0.15, 1, DQ32_A + 1}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
     return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
@@ -1147,15 +1201,14 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     if (phases & PH_BWD_DQDR) {
         const DqArgs& a = dq;
         const int tokw = pick.tile_rows;
-        const int smem = (tokw == 32 ? DQ32_R0 : DQ_NST * DQ_STAGE_B) +
-                         (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
+        const int smem = tokw == 32 ? DQ32_SMEM : DQ_NST * DQ_STAGE_B + (d.E < GATE_WIN ? d.E : GATE_WIN) * tokw * (int)sizeof(float);
         if (smem > 160 * 1024) return hipErrorInvalidValue;
         static LdsOptIn optin, optin32;
         err = tokw == 32 ? ensure_dynamic_lds(optin32, (const void*)mhffn_bwd_dqdr_rows32_kernel<DH>, smem)
                          : ensure_dynamic_lds(optin, (const void*)mhffn_bwd_dqdr_kernel<DH>, smem);
         if (err != hipSuccess) return err;
         dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
-        if (tokw == 32) hipLaunchKernelGGL((mhffn_bwd_dqdr_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
+        if (tokw == 32) hipLaunchKernelGGL((mhffn_bwd_dqdr_rows32_kernel<DH>), grid, dim3(DQ32_W * 64), smem, st, a);
         else hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
         if (a.parts.nsplit > 1 && !together)
             hipLaunchKernelGGL((mhffn_bwd_dqdr_sum_kernel<DH>), dim3(qb + rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, qb);

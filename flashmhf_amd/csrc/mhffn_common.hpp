@@ -315,15 +315,15 @@ __device__ __forceinline__ void store_rows_f32(unsigned char* region, float* dst
     });
 }
 
-// ---- tiles of 32 rows, four blocks at a time ------------------------------------------------------------------------
+// ---- tiles of 32 rows, a wave per block -----------------------------------------------------------------------------
 // With few rows the tiles of 128 and 256 rows leave most of the chip idle, and a workgroup walks a head's blocks one after
-// the other.  The rows32 kernels put the four waves of a workgroup on four consecutive blocks of the same 32 rows instead:
+// the other.  The rows32 kernels put four waves of a workgroup on four consecutive blocks of the same 32 rows instead:
 // a wave takes the first products and the element-wise work of its own block, hands the rounded result to the others
-// through LDS, and then adds all four blocks, in their order, to the 32 output columns it owns: the sums are those of the
-// kernels with larger tiles bit for bit.
+// through LDS, and all blocks are added, in their order, by a wave for each 32 output columns (the forward's: the same waves,
+// four blocks at a time; dQ/dR's: four others, one at a time): the sums are those of the kernels with larger tiles bit for bit.
 // Every LDS access of their loops is inline assembly and every wait counted by hand: the compiler would put a wait for all
 // outstanding LDS-direct loads in front of each access.
-constexpr int QUAD = 4;                      // waves of a workgroup = blocks of a trip
+constexpr int QUAD = 4;                      // waves of a workgroup of the forward = blocks of a trip
 
 // Asynchronous fill of one 32-row tile by one wave: eight vmcnt events.
 template <int DH>
@@ -351,15 +351,15 @@ __device__ __forceinline__ void quad_barrier()
 template <int KS, int N>
 struct QuadRows {
     u32x4 v[N][KS];
-    template <int T, int KSI>
+    template <int T, int KSI, int IMM = 0>
     __device__ __forceinline__ void request(unsigned rowaddr)      // address of the row's k-step 0 chunk position
     {
-        v[T][KSI] = lds_read16_async<0>(rowaddr);
+        v[T][KSI] = lds_read16_async<IMM>(rowaddr);
     }
-    template <int KSI>
+    template <int KSI, int MORE = 0>                               // MORE: reads of others requested behind all of these
     __device__ __forceinline__ void wait()
     {
-        constexpr int younger = (KS - 1 - KSI) * N < 15 ? (KS - 1 - KSI) * N : 15;
+        constexpr int younger = (KS - 1 - KSI) * N + MORE < 15 ? (KS - 1 - KSI) * N + MORE : 15;
         lds_wait_n<younger>();
 #pragma unroll
         for (int t = 0; t < N; ++t) asm volatile("" : "+v"(v[t][KSI]));
@@ -584,16 +584,16 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 }
 
 // Into how many parts the forward and the dQ/dR kernel cut the blocks of a head, and which of a kernel's tile heights runs.
-// The steps are times of each kernel on half a chip, two of them of earlier forms of it (at each kernel's variants); a rows32 step is a
-// trip of four blocks.
+// The steps are times of each kernel on half a chip, one of them of an earlier form of it (at each kernel's variants); a step of the
+// rows32 forward is a trip of four blocks.
 // One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute
 // units a part per idle unit shortens the serial walk over the blocks (one token of the 370M layer, 8 tiles of 121 blocks: 46 us
 // in one part, 7.8 in 31), and every part costs a set of fp32 sums that is written and read back.  Time of a launch in us:
 // rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing pass + 0.6 per MB
 // of sums; a step slows by up to `full` as the chip fills (power).  The prices are those of d_h = 128 for every d_h: with it the
-// variants of a kernel get cheaper nearly together.  Against every tile height and 1 to 64 parts, measured on 336 bfloat16 calls
-// (forward and dQ/dR; d_h 64, 96, 128; four layers; 1 to 12,000 rows; profiles/pick_parts_sweep.csv) the pick is 1.5 % slower than
-// the fastest on average and 23 % at worst (forward of 4,096 rows of 8 heads of 64, 45.8 us against 37.3); by d_h at most 23, 21, 18 %.
+// variants of a kernel get cheaper nearly together.  Against every tile height and 1 to 64 parts, measured on 168 bfloat16 calls of the
+// forward (d_h 64, 96, 128; four layers; 1 to 12,000 rows; profiles/pick_parts_sweep.csv) the pick is 1.6 % slower than
+// the fastest on average and 23 % at worst (4,096 rows of 8 heads of 64, 45.8 us against 37.3); dQ/dR: at its variants.
 // Not cut: more experts than one LDS window of gate values holds (bfloat16); and 16,384 rows per head or more, where a head
 // fills a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X
@@ -602,6 +602,7 @@ struct Variant {
     int tile_rows;
     double step, full;
     int unit;             // blocks of a step
+    int ahead = 0;        // steps that a pipeline takes beyond those of its blocks
 };
 struct Pick {
     int tile_rows, nsplit;
@@ -615,13 +616,13 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
     Pick best{variants[0].tile_rows, 1};
     double best_us = 0;
     for (const Variant& v : variants) {
-        if (v.unit > 1 && !may_cut) continue;      // (the rows32 kernels keep all gate values of a tile in LDS)
+        if (v.tile_rows == 32 && !may_cut) continue;      // (the rows32 forward keeps all gate values of a tile in LDS)
         const long tiles = (rows + v.tile_rows - 1) / v.tile_rows * d.Hkuv;
         for (int ns = 1; ns <= most; ++ns) {
             if (ns > 1 && (ns * part_bytes > ws_bytes || tiles * (ns - 1) >= 2 * CUS)) break;
             const long wgs = tiles * ns;
             const double load = wgs <= CUS / 2 ? 0 : wgs >= CUS ? 1 : (wgs - CUS / 2) / (double)(CUS / 2);
-            const double us = (double)((wgs + CUS - 1) / CUS) * (((blocks + ns - 1) / ns + v.unit - 1) / v.unit * v.step * (1 + v.full * load) + 3) +
+            const double us = (double)((wgs + CUS - 1) / CUS) * ((((blocks + ns - 1) / ns + v.unit - 1) / v.unit + v.ahead) * v.step * (1 + v.full * load) + 3) +
                               (ns > 1 ? 2 + ns * part_us : 0);
             if (best_us == 0 || us < best_us) { best_us = us; best = Pick{v.tile_rows, ns}; }
         }
