@@ -465,47 +465,19 @@ __global__ __launch_bounds__(DQ32_W * 64) void mhffn_bwd_dqdr_rows32_kernel(DqAr
 
     // Fills and sums.  Each of these waves requests a quarter of every tile: six vmcnt events a block.
     const int col = wave - DQ32_A;
-    const long offU = p.U - p.K, offV = p.V - p.K;
-    int ku = 0, v = 0;                     // tile sets of the next block to request
-    // (a lane's place in a row group of the tile as a 32-bit offset to a uniform base; a narrow row's unused chunks take chunk 0)
-    unsigned place[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int row = 4 * (2 * col + i) + (lane >> 4), c = (lane & 15) ^ swz16(row);
-        place[i] = (row * DH + (c < DH / 8 ? c : 0) * 8) * 2;
-    }
-    const char* src;
-    unsigned char *tku, *tv;
-    auto aim = [&](int b) {
-        src = reinterpret_cast<const char*>(Kh + (long)(b < nblk ? b : nblk - 1) * JB * DH);
-        asm("" : "+s"(src));               // (kept apart from the lane's offset: one scalar addition per fill)
-        tku = smem + ku * 2 * TILE_B + 2 * col * 1024;
-        tv = smem + DQ32_V0 + v * TILE_B + 2 * col * 1024;
-        ku = ku + 1 == DQ32_KU ? 0 : ku + 1;
-        v = v + 1 == DQ32_V ? 0 : v + 1;
-    };
-    auto fill = [&](auto tensor_, auto i_) {
-        constexpr int T = decltype(tensor_)::value, i = decltype(i_)::value;
-        const char* from = src + 2 * (T == 0 ? 0 : T == 1 ? offU : offV);
-        unsigned char* to = (T == 2 ? tv : tku + T * TILE_B) + i * 1024;
-        __builtin_amdgcn_global_load_lds((gptr_t)(from + place[i]), (lptr_t)to, 16, 0, 0);
-    };
+    QuadFill<DH, DQ32_KU, DQ32_V> fill(Kh, p.U - p.K, p.V - p.K, nblk, smem, smem + DQ32_V0, col, lane);
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
-    const TrLane<CT> trl = make_tr_lane<CT, 8, 4>(lane);
-    TrLane<1> tr{};                           // this wave's column tile
-#pragma unroll
-    for (int i = 0; i < CT; ++i)
-        if (i == col) { tr.off[0][0] = trl.off[i][0]; tr.off[0][1] = trl.off[i][1]; }
+    const TrLane<1> tr = quad_tr_lane<CT>(lane, col);
     f32x16 dq;
 #pragma unroll
     for (int x = 0; x < 16; ++x) dq[x] = 0.0f;
     for (int b = 0; b < DQ32_AHEAD; ++b) {
-        aim(b);
+        fill.aim(b);
         static_for<3>([&](auto t) {
-            fill(t, I0{});
-            fill(t, I1{});
+            fill.request(t, I0{});
+            fill.request(t, I1{});
         });
     }
     wait_vmcnt<6 * (DQ32_AHEAD - 1)>();
@@ -522,23 +494,23 @@ __global__ __launch_bounds__(DQ32_W * 64) void mhffn_bwd_dqdr_rows32_kernel(DqAr
             d[1] = lds_read16_async<1024>(sD);
             d[3] = lds_read16_async<3072>(sD);
         }
-        aim(phase + DQ32_AHEAD);
-        fill(I0{}, I0{});
-        fill(I0{}, I1{});
+        fill.aim(phase + DQ32_AHEAD);
+        fill.request(I0{}, I0{});
+        fill.request(I0{}, I1{});
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (SUMS) {
             lds_wait_n<0>();
             asm volatile("" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]));
         }
         // this block's sums, each operand followed by the next block's (from the tile set that the next phase requests into)
-        const unsigned aK = smem0 + ku * 2 * TILE_B;
+        const unsigned aK = smem0 + fill.ku * 2 * TILE_B;
         static_for<4>([&](auto kc) {
             constexpr int k = decltype(kc)::value, half = k >> 1;
             TrOperand& t = k & 1 ? tu[half] : tk[half];
             if constexpr (SUMS) dq = mfma32(tr_value(t), __builtin_bit_cast(bf16x8, d[(k & 1) * 2 + half]), dq);
             __builtin_amdgcn_sched_barrier(0);
             t = tile_read_cols_async<(k & 1) * TILE_B + half * 4096>(aK, tr, 0);
-            fill(std::integral_constant<int, (k + 2) / 2>{}, std::integral_constant<int, (k & 1)>{});
+            fill.request(std::integral_constant<int, (k + 2) / 2>{}, std::integral_constant<int, (k & 1)>{});
             __builtin_amdgcn_sched_barrier(0);
         });
         wait_vmcnt<6 * (DQ32_AHEAD - 1)>();   // the next phase's first products have their tiles

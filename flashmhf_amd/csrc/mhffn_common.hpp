@@ -319,8 +319,9 @@ __device__ __forceinline__ void store_rows_f32(unsigned char* region, float* dst
 // With few rows the tiles of 128 and 256 rows leave most of the chip idle, and a workgroup walks a head's blocks one after
 // the other.  The rows32 kernels put four waves of a workgroup on four consecutive blocks of the same 32 rows instead:
 // a wave takes the first products and the element-wise work of its own block, hands the rounded result to the others
-// through LDS, and all blocks are added, in their order, by a wave for each 32 output columns (the forward's: the same waves,
-// four blocks at a time; dQ/dR's: four others, one at a time): the sums are those of the kernels with larger tiles bit for bit.
+// through LDS, and all blocks are added, in their order, by a wave for each 32 output columns (the forward of short parts: the same
+// waves, four blocks at a time; the others: four more waves, one block at a time): the sums are those of the kernels with larger
+// tiles bit for bit.
 // Every LDS access of their loops is inline assembly and every wait counted by hand: the compiler would put a wait for all
 // outstanding LDS-direct loads in front of each access.
 constexpr int QUAD = 4;                      // waves of a workgroup of the forward = blocks of a trip
@@ -331,6 +332,56 @@ __device__ __forceinline__ void quad_fill(const bf16_t* src, unsigned char* tile
 {
 #pragma unroll
     for (int i = 0; i < 8; ++i) tile_fill_ins<DH>(src, DH, tile, i, lane);
+}
+// Asynchronous fills of a block's K, U and V tiles by four waves, each a quarter of every tile: two vmcnt events a tile.  A lane's
+// place in a tile is a 32-bit offset to a uniform base (a narrow row's unused chunks take chunk 0).  The tiles go round in KU sets
+// of K | U and in NV sets of V; ku and v are the sets of the block behind the last one aimed at.
+template <int DH, int KU, int NV>
+struct QuadFill {
+    const bf16_t* K;
+    long offU, offV;          // U - K, V - K in bytes
+    unsigned char *ku0, *v0, *to_ku, *to_v;
+    const char* from;
+    unsigned place[2];
+    int nblk, ku, v;
+    __device__ __forceinline__ QuadFill(const bf16_t* K_, long offU_, long offV_, int nblk_, unsigned char* ku0_, unsigned char* v0_, int quarter,
+                                        int lane)
+        : K(K_), offU(2 * offU_), offV(2 * offV_), ku0(ku0_ + 2 * quarter * 1024), v0(v0_ + 2 * quarter * 1024), nblk(nblk_), ku(0), v(0)
+    {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int row = 4 * (2 * quarter + i) + (lane >> 4), c = (lane & 15) ^ swz16(row);
+            place[i] = (row * DH + (c < DH / 8 ? c : 0) * 8) * 2;
+        }
+    }
+    __device__ __forceinline__ void aim(int b)      // (behind the last block: the last one again)
+    {
+        from = reinterpret_cast<const char*>(K + (long)(b < nblk ? b : nblk - 1) * JB * DH);
+        asm("" : "+s"(from));           // (kept apart from the lane's offset: one scalar addition per tile)
+        to_ku = ku0 + ku * 2 * TILE_B;
+        to_v = v0 + v * TILE_B;
+        ku = ku + 1 == KU ? 0 : ku + 1;
+        v = v + 1 == NV ? 0 : v + 1;
+    }
+    template <class T_, class I_>
+    __device__ __forceinline__ void request(T_, I_)     // half I of this wave's part of K, U or V (T = 0, 1, 2)
+    {
+        constexpr int T = T_::value, I = I_::value;
+        const char* src = from + (T == 0 ? 0 : T == 1 ? offU : offV);
+        unsigned char* dst = (T == 2 ? to_v : to_ku + T * TILE_B) + I * 1024;
+        __builtin_amdgcn_global_load_lds((gptr_t)(src + place[I]), (lptr_t)dst, 16, 0, 0);
+    }
+};
+// The transposed operands' places for one column tile.
+template <int CT>
+__device__ __forceinline__ TrLane<1> quad_tr_lane(int lane, int col)
+{
+    const TrLane<CT> all = make_tr_lane<CT, 8, 4>(lane);
+    TrLane<1> t{};
+#pragma unroll
+    for (int i = 0; i < CT; ++i)
+        if (i == col) { t.off[0][0] = all.off[i][0]; t.off[0][1] = all.off[i][1]; }
+    return t;
 }
 template <int IMM, class T>
 __device__ __forceinline__ void lds_write16(unsigned addr, const T& v)
@@ -356,10 +407,10 @@ struct QuadRows {
     {
         v[T][KSI] = lds_read16_async<IMM>(rowaddr);
     }
-    template <int KSI, int MORE = 0>                               // MORE: reads of others requested behind all of these
+    template <int KSI>
     __device__ __forceinline__ void wait()
     {
-        constexpr int younger = (KS - 1 - KSI) * N + MORE < 15 ? (KS - 1 - KSI) * N + MORE : 15;
+        constexpr int younger = (KS - 1 - KSI) * N < 15 ? (KS - 1 - KSI) * N : 15;
         lds_wait_n<younger>();
 #pragma unroll
         for (int t = 0; t < N; ++t) asm volatile("" : "+v"(v[t][KSI]));

@@ -541,6 +541,194 @@ __global__ __launch_bounds__(256) void mhffn_fwd_rows32_kernel(FwdArgs p)
     }
 }
 
+// 32 rows and many blocks: the same products, element-wise formula and order of sums, the blocks in a pipeline as in the 32-row dQ/dR
+// kernel.  Four waves take the first products and the element-wise work, each of every fourth block, in four phases, a phase apart
+// from each other; four more request the tiles, 24 KB a phase, and add one block a phase to O, a column tile each.  A phase takes
+// 0.34 us against the 0.40 of a quarter of a trip above (1,024 rows of 8 heads of 128, 8 experts of 256: 30.0 -> 27.4 us; one part
+// of 512 rows of the 370M heads 48.9 -> 42.0, of 1,024 54.8 -> 47.6, of 512 of 8 heads of 96 24.0 -> 22.7, of 64 21.3 -> 20.8; 100 rows of
+// the 1.3B heads 91.3 -> 75.2).  What bounds it is the issue of the loads to LDS, 65 cycles of a wave each (none of them: 37.1 us for
+// the 512 rows), and the first phase, 570 of 690 cycles.  Three
+// waves in three phases with operands read a phase ahead and a fifth wave for a third of the loads: 44.2.  Its four phases in front of
+// the first sum cost short parts more than it gives: the kernel above takes those.
+constexpr int FWDL_A = 4, FWDL_W = FWDL_A + 4;          // waves of the first kind, and all; also a block's phases up to its sums
+constexpr int FWDL_AHEAD = 4;                             // phases between the request of a block's tiles and its first products
+constexpr int FWDL_KU = FWDL_AHEAD + 1, FWDL_V = FWDL_AHEAD + FWDL_A;      // tile sets: K and U to a block's first phase, V to its sums
+constexpr int FWDL_V0 = FWDL_KU * 2 * TILE_B, FWDL_P0 = FWDL_V0 + FWDL_V * TILE_B, FWDL_SMEM = FWDL_P0 + 2 * 2048;
+template <int DH>
+__global__ __launch_bounds__(FWDL_W * 64) void mhffn_fwd_rows32_long_kernel(FwdArgs p)
+{
+    constexpr int KS = DH / 16, CT = DH / 32;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
+    const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
+    const unsigned smem0 = lds_addr(smem);
+    const int nphase = nblk + FWDL_A;     // block b: first products in phase b, its sums in phase b + FWDL_A; every phase ends with a barrier
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+
+    if (wave < FWDL_A) {
+        const int t = tok0 + l32 < p.rows.n ? tok0 + l32 : p.rows.n - 1;
+        bf16x8 q[KS];
+        {
+            const bf16_t* qr = p.Q + p.rows.tok(hk, t) * DH + 8 * g;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) q[ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16);
+        }
+        const float* rrow = p.R + p.rows.gate(hk, t) * E + ex0;
+        auto gate = [&](int b) { return rrow[p.parts.by_nbe.div(jb0 + (b < nblk ? b : nblk - 1))]; };
+        float rnext = gate(wave), rinv = 0.0f;
+        // (these loads end here: waited for in the loop, each trip would also wait for the next gate value)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(q[ks]));
+        asm volatile("" : "+v"(rnext));
+        const int krow = row_perm32(l32), sw = swz16(krow);
+        unsigned at[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) at[ks] = smem0 + krow * TILE_ROW_B + (((2 * ks + g) ^ sw) << 4);
+        const unsigned sP = smem0 + FWDL_P0 + lane * 16;
+
+        f32x16 m, n;
+        bf16x8 pt[2];
+        QuadRows<KS, 2> a;
+        // Phase 1: half the k-steps of M and N, with the reads of the others between the matrix instructions.
+        constexpr int K1 = KS / 2;
+        auto phase1 = [&](int b) {
+            rinv = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(rnext), -FLT_MAX_F, FLT_MAX_F);
+            rnext = gate(b + FWDL_A);     // a round ahead of its use
+            const unsigned ku = (b % FWDL_KU) * 2 * TILE_B;
+            auto request = [&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                const unsigned x = at[ks] + ku;
+                a.template request<0, ks>(x);
+                a.template request<1, ks, TILE_B>(x);
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<KS - K1>([&](auto kc) { request(kc); });
+#pragma unroll
+            for (int x = 0; x < 16; ++x) { m[x] = 0.0f; n[x] = 0.0f; }
+            static_for<K1>([&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                lds_wait_n<2 * (KS - K1 - 1)>();      // (as many k-steps are requested behind this one)
+                asm volatile("" : "+v"(a.v[0][ks]), "+v"(a.v[1][ks]));
+                m = mfma32(a.get(0, ks), q[ks], m);
+                n = mfma32(a.get(1, ks), q[ks], n);
+                __builtin_amdgcn_sched_barrier(0);
+                request(std::integral_constant<int, KS - K1 + ks>{});
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        auto phase2 = [&]() {
+            static_for<KS - K1>([&](auto kc) {
+                constexpr int ks = K1 + decltype(kc)::value;
+                asm volatile("" : "+v"(a.v[0][ks]), "+v"(a.v[1][ks]));       // (returned before the barrier)
+                m = mfma32(a.get(0, ks), q[ks], m);
+                n = mfma32(a.get(1, ks), q[ks], n);
+            });
+        };
+        auto elements = [&](auto i0_, auto i1_) {
+#pragma unroll
+            for (int i = decltype(i0_)::value; i < decltype(i1_)::value; ++i) {
+                const float ex = __builtin_amdgcn_exp2f(-LOG2E * m[i]);
+                const float xn = m[i] * n[i];
+                pt[i >> 3][i & 7] = (bf16_t)(xn * __builtin_amdgcn_rcpf(__builtin_fmaf(ex, rinv, rinv)));
+            }
+            asm volatile("" : "+v"(pt[0]), "+v"(pt[1]));     // (here, not behind the barrier)
+        };
+        using I4 = std::integral_constant<int, 4>;
+        using I10 = std::integral_constant<int, 10>;
+        using I16 = std::integral_constant<int, 16>;
+        for (int i = 0; i <= wave; ++i) quad_barrier();      // (the first: block 0 has landed)
+        int phase = wave;
+        for (int b = wave; b < nblk; b += FWDL_A, phase += FWDL_A) {
+            phase1(b);
+            quad_barrier();
+            phase2();
+            elements(I0{}, I4{});
+            quad_barrier();
+            elements(I4{}, I10{});
+            quad_barrier();
+            elements(I10{}, I16{});
+            const unsigned d = sP + (b & 1) * 2048;
+            lds_write16<0>(d, pt[0]);
+            lds_write16<1024>(d, pt[1]);
+            quad_barrier();
+        }
+        for (; phase <= nphase; ++phase) quad_barrier();     // (and the one in front of the epilogue)
+        return;
+    }
+
+    // Fills and sums.  Each of these waves requests a quarter of every tile: six vmcnt events a block.
+    const int col = wave - FWDL_A;
+    QuadFill<DH, FWDL_KU, FWDL_V> fill(p.K + ((long)hk * E * nbe + blk0) * JB * DH, p.U - p.K, p.V - p.K, nblk, smem, smem + FWDL_V0, col, lane);
+    const TrLane<1> tr = quad_tr_lane<CT>(lane, col);
+    f32x16 o;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) o[x] = 0.0f;
+    for (int b = 0; b < FWDL_AHEAD; ++b) {
+        fill.aim(b);
+        static_for<3>([&](auto t) {
+            fill.request(t, I0{});
+            fill.request(t, I1{});
+        });
+    }
+    wait_vmcnt<6 * (FWDL_AHEAD - 1)>();
+    quad_barrier();                           // block 0 has landed
+    TrOperand v[2];
+    auto phase_of = [&](auto sums_, int phase) {
+        constexpr bool SUMS = decltype(sums_)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 pv[2];
+        if constexpr (SUMS) {
+            const unsigned sP = smem0 + FWDL_P0 + ((phase - FWDL_A) & 1) * 2048 + lane * 16;
+            pv[0] = lds_read16_async<0>(sP);
+            pv[1] = lds_read16_async<1024>(sP);
+        }
+        fill.aim(phase + FWDL_AHEAD);
+        fill.request(I0{}, I0{});
+        fill.request(I0{}, I1{});
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (SUMS) {
+            lds_wait_n<0>();
+            asm volatile("" : "+v"(pv[0]), "+v"(pv[1]));
+        }
+        // this block's sums, each operand followed by the next block's (from the tile set that the next phase requests into)
+        const unsigned aV = smem0 + FWDL_V0 + fill.v * TILE_B;
+        static_for<2>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            if constexpr (SUMS) o = mfma32(tr_value(v[s]), __builtin_bit_cast(bf16x8, pv[s]), o);
+            __builtin_amdgcn_sched_barrier(0);
+            v[s] = tile_read_cols_async<s * 4096>(aV, tr, 0);
+            fill.request(std::integral_constant<int, 1 + s>{}, I0{});
+            fill.request(std::integral_constant<int, 1 + s>{}, I1{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        wait_vmcnt<6 * (FWDL_AHEAD - 1)>();  // the next phase's first products have their tiles
+        quad_barrier();
+#pragma unroll
+        for (int s = 0; s < 2; ++s) asm volatile("" : "+v"(v[s].lo), "+v"(v[s].hi));
+    };
+    int phase = 0;
+    for (const int idle = col < CT ? FWDL_A : nphase; phase < idle; ++phase) phase_of(std::false_type{}, phase);
+    for (; phase < nphase; ++phase) phase_of(std::true_type{}, phase);
+    wait_vmcnt<0>();          // the fills of blocks that are not there write the tiles, which the epilogue reuses
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (col >= CT) return;
+    unsigned char* own = smem + col * TILE_B;
+    const int nrows = p.rows.n - tok0;
+    if (nsplit > 1) {
+        float* prow = p.part + (((long)z * p.rows.Hkuv + hk) * p.rows.n + tok0) * DH + 32 * col;
+        quad_store_f32(own, o, nrows, lane, [&](int row) { return prow + row * DH; });
+    } else {
+        quad_store_bf16(own, o, nrows, lane, [&](int row) { return p.O + p.rows.tok(hk, tok0 + row) * DH + 32 * col; });
+    }
+}
+
 // Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, four columns per lane.
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
@@ -565,6 +753,9 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // number of parts: one token of the 370M layer 7.8 us against 10.0, 16 tokens of the 1.3B layer 20.3 against 22.5 (95 MB of
 // weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.  (Priced at 0.6 for 128 rows, as
 // before its filling waves: the line between the two kernels lies where it did.)
+// A part of FWDL_FROM blocks or more goes through the pipeline: 15 or 16 blocks a part 14.4 -> 14.0 us (100 rows of the 370M heads) and
+// 19.7 -> 20.4 (16 of the 1.3B heads), 4 blocks 7.6 -> 8.0, 64 blocks as above.
+constexpr int FWDL_FROM = 32;
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
@@ -576,17 +767,21 @@ template <int DH>
 static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, hipStream_t st)
 {
     const int gates = d.E < GATE_WIN ? d.E : GATE_WIN;
-    const int smem = tile_rows == 32 ? FWD32_R0 + gates * 32 * (int)sizeof(float)
+    const bool pipeline = tile_rows == 32 && d.E * (d.d_e / JB) / a.parts.nsplit >= FWDL_FROM;
+    const int smem = pipeline          ? FWDL_SMEM
+                     : tile_rows == 32 ? FWD32_R0 + gates * 32 * (int)sizeof(float)
                                      : FWD_RING_B + gates * 256 * (int)sizeof(float);
     if (smem > 160 * 1024) return hipErrorInvalidValue;
-    static LdsOptIn optin, optin128, optin32;
-    const hipError_t e = tile_rows == 256   ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
+    static LdsOptIn optin, optin128, optin32, optinl;
+    const hipError_t e = pipeline           ? ensure_dynamic_lds(optinl, (const void*)mhffn_fwd_rows32_long_kernel<DH>, smem)
+                         : tile_rows == 256 ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
                          : tile_rows == 128 ? ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem)
                                             : ensure_dynamic_lds(optin32, (const void*)mhffn_fwd_rows32_kernel<DH>, smem);
     if (e != hipSuccess) return e;
     dim3 grid((unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv), (unsigned)a.parts.nsplit);
     if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
     else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(512), smem, st, a);
+    else if (pipeline) hipLaunchKernelGGL((mhffn_fwd_rows32_long_kernel<DH>), grid, dim3(FWDL_W * 64), smem, st, a);
     else hipLaunchKernelGGL((mhffn_fwd_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
         dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 4) + 255) / 256), (unsigned)d.Hkuv);
