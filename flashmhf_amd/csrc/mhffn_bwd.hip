@@ -1131,10 +1131,13 @@ static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d
 // the rows.  One part of 121 blocks of the 370M heads, 512 rows: 199 us with 256 rows, 48 with 32; 2,048 rows: 200 and (two
 // rounds) 108.  At their best numbers of parts 512 rows take 34.5 us with 32 rows, 36.1 with 256, 733 rows 49.7 and 45.0.  The prices lose
 // 0.3 % on average and 4.8 % at worst over 112 calls (d_h 64, 96, 128; eight layers; 32 to 4,096 rows; up to 40 parts of either kernel).
+// Where dK, dU, dV have slices to add up, the parts go along in that launch: whole backward of 2 x 300 tokens of 8 heads of 96 on
+// two 61.7 us with a pass of their own in the price (32 rows, one part), 58.6 without (256 rows, eight parts); 900 of 8 of 128 on four 117.0, 114.6.
 constexpr Variant DQ_VARIANTS[] = {{256, 1.7, 0.15, 1}, {32, 0.36, 0.15, 1, DQ32_A + 1}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
-    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
+    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes,
+                      dw_slices_bf16(d, ws_bytes) > 1 ? 0 : 2);
 }
 
 size_t bwd_min_workspace_bytes_bf16(const Dims& d)

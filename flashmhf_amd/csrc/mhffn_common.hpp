@@ -640,8 +640,9 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 // One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute
 // units a part per idle unit shortens the serial walk over the blocks (one token of the 370M layer, 8 tiles of 121 blocks: 46 us
 // in one part, 7.8 in 31), and every part costs a set of fp32 sums that is written and read back.  Time of a launch in us:
-// rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing pass + 0.6 per MB
-// of sums; a step slows by up to `full` as the chip fills (power).  The prices are those of d_h = 128 for every d_h: with it the
+// rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing pass (dQ/dR: none where
+// the weights' gradients have one, which adds up both) + 0.6 per MB of sums; a step slows by up to `full` as the chip fills
+// (power).  The prices are those of d_h = 128 for every d_h: with it the
 // variants of a kernel get cheaper nearly together.  Against every tile height and 1 to 64 parts, measured on 168 bfloat16 calls of the
 // forward (d_h 64, 96, 128; four layers; 1 to 12,000 rows; profiles/pick_parts_sweep.csv) the pick is 1.3 % slower than
 // the fastest on average and 23 % at worst (4,096 rows of 8 heads of 64, 45.8 us against 37.3); dQ/dR: at its variants.
@@ -659,7 +660,7 @@ struct Pick {
     int tile_rows, nsplit;
 };
 template <int N>
-inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, bool may_cut, size_t part_bytes, size_t ws_bytes)
+inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, bool may_cut, size_t part_bytes, size_t ws_bytes, double sum_us = 2)
 {
     const long rows = (long)(d.H / d.Hkuv) * d.B * d.S;
     const int most = may_cut && rows < SPLIT_ROWS_BELOW && blocks < (1 << 24) ? (blocks < 64 ? blocks : 64) : 1;
@@ -674,7 +675,7 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
             const long wgs = tiles * ns;
             const double load = wgs <= CUS / 2 ? 0 : wgs >= CUS ? 1 : (wgs - CUS / 2) / (double)(CUS / 2);
             const double us = (double)((wgs + CUS - 1) / CUS) * ((((blocks + ns - 1) / ns + v.unit - 1) / v.unit + v.ahead) * v.step * (1 + v.full * load) + 3) +
-                              (ns > 1 ? 2 + ns * part_us : 0);
+                              (ns > 1 ? sum_us + ns * part_us : 0);
             if (best_us == 0 || us < best_us) { best_us = us; best = Pick{v.tile_rows, ns}; }
         }
     }
