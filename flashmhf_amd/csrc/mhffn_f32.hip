@@ -39,12 +39,15 @@ struct F32Args {
 };
 
 __device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-// 1 / (1 + e^-x): the reciprocal with one Newton step (an IEEE division takes three times the instructions), at least 2^-126 (the
-// step would make NaN of an infinite e^-x)
-__device__ __forceinline__ float sigmoid_exact(float x)
+__device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + __expf(-x)); }
+// The same in the kernels that have VALU time to lose: the reciprocal with one Newton step (an IEEE division takes three times the instructions), of a sixteenth of
+// the sum, whose reciprocal is a normal number up to the largest finite e^-x; 0 beyond that, where the step would make NaN of an
+// infinite one.
+__device__ __forceinline__ float sigmoid_newton(float x)
 {
-    const float d = 1.0f + __builtin_amdgcn_exp2f(fminf(-LOG2E * x, 126.0f)), y = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, y, 1.0f), y, y);
+    const float t = -LOG2E * x, d = fmaf(__builtin_amdgcn_exp2f(t), 0.0625f, 0.0625f), y = __builtin_amdgcn_rcpf(d);
+    const float s = fmaf(fmaf(-d, y, 1.0f), y, y) * 0.0625f;
+    return t >= 128.0f ? 0.0f : s;
 }
 __device__ __forceinline__ f32x16 zero16()
 {
@@ -469,7 +472,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS) void fwd_f32_kernel(F32Args p
         f32x16 &m = mn[0], &n = mn[1];
         mfma_result_fence(m, n);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) m[i] *= sigmoid_exact(m[i]) * n[i] * r;
+        for (int i = 0; i < 16; ++i) m[i] *= sigmoid_newton(m[i]) * n[i] * r;
         if (b.rows < JB) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) m[i] = split_row(i, g) < b.rows ? m[i] : 0.0f;
@@ -582,7 +585,7 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
             for (int i = 0; i < 16; ++i) da[i] = split_row(i, g) < b.rows ? da[i] : 0.0f;
         }
         float sg;
-        auto sigma = [&](int i) { sg = sigmoid_exact(m[i]); };
+        auto sigma = [&](int i) { sg = sigmoid_newton(m[i]); };
         auto element = [&](int i) {
             const float sl = m[i] * sg, a = da[i] * sl, ra = r * da[i];
             dr = fmaf(a, n[i], dr);
@@ -796,7 +799,7 @@ __global__ __launch_bounds__(256, 1) void dkdudv_split_kernel(F32Args p)
         gates(0);
         mfma_result_fence(m, n, da);
         float sg;
-        auto sigma = [&](int i) { sg = sigmoid_exact(m[i]); };
+        auto sigma = [&](int i) { sg = sigmoid_newton(m[i]); };
         auto element = [&](int i) {
             const float r = r4[(i >> 2) & 1][i & 3], sl = m[i] * sg, ra = r * da[i], nn = n[i];
             m[i] = ra * nn * fmaf(sl, 1.0f - sg, sg);      // dM

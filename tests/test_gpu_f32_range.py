@@ -1,0 +1,71 @@
+"""The float32 operator at the ends of its range: what a float32 evaluation of the same formulas gives there is also what the kernels
+give, whatever instructions their products run on."""
+import math
+
+import pytest
+import torch
+
+from oracle import mhffn_oracle as orc
+from tests.helpers import make_inputs
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+NAMES = ("O", "dQ", "dK", "dU", "dV", "dR")
+
+
+def _run(Q, K, U, V, R, dO):
+    from flashmhf_amd import mhffn_backward, mhffn_forward
+    ins = [t.to(DEV) for t in (Q, K, U, V, R)]
+    out = (mhffn_forward(*ins), *mhffn_backward(*ins, dO.to(DEV), grad_w_dtype=torch.float32))
+    torch.cuda.synchronize()
+    return [t.cpu() for t in out]
+
+
+def _oracle(*ins):
+    return (orc.mhffn_forward(*ins[:5], compute_dtype=torch.float64), *orc.mhffn_backward(*ins, compute_dtype=torch.float64))
+
+
+def _error(got, want):
+    return ((got.double() - want.double()).norm() / want.double().norm()).item()
+
+
+def _bound(B, H, S, dh, E, de, Hk):
+    """Roundings of 2^-24 of the size of the longest sum, of either sign (see test_gpu_f32_split.py)."""
+    return 2.0 ** -24 * (math.sqrt(6 * (dh + max(E * (de + 31), H // Hk * B * S + 31)) / 16) + 8)
+
+
+@pytest.mark.parametrize("value", [-1e2, -1e10, -1e37, torch.finfo(torch.float32).min])
+@pytest.mark.parametrize("dh", [64, 96, 128])
+def test_silu_goes_to_zero(dh, value):
+    """Rows of K that mask their hidden unit (a constant column of Q times a very negative number): SiLU and its derivative are zero."""
+    shape = B, H, S, dh, E, de, Hk = 1, 2, 70, dh, 2, 64, 2
+    print(f"case d_h={dh} value={value}", flush=True)
+    ins = make_inputs(B, H, S, dh, E, de, Hk, seed=9, dtype=torch.float32)
+    ins[0][..., 3] = 1.0
+    ins[1][:, :, ::5] = 0.0
+    ins[1][:, :, ::5, 3] = value
+    want = _oracle(*ins)
+    for name, got, ref in zip(NAMES, _run(*ins), want):
+        assert torch.isfinite(got).all(), name
+        assert _error(got, ref) <= _bound(*shape), (name, _error(got, ref))
+    got = _run(*ins)
+    assert (got[2][:, :, ::5].abs() <= 1e-30).all() and (got[4][:, :, ::5].abs() <= 1e-30).all()      # (masked rows of dK, dV)
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("dh", [64, 128])
+def test_saturated_preactivations(dh, sign):
+    """Pre-activations of a few hundred of either sign, zero gates and zero rows."""
+    shape = B, H, S, dh, E, de, Hk = 2, 2, 96, dh, 3, 64, 2
+    Q, K, U, V, R, dO = make_inputs(B, H, S, dh, E, de, Hk, seed=5, dtype=torch.float32)
+    Q, K = Q * 12.0 * sign, K * 4.0
+    Q[:, :, 5] = 0
+    R[:, :, ::3, 1] = 0.0
+    R[:, :, 7] = 0.0
+    assert torch.einsum("bhsd,hejd->bhsej", Q, K).abs().max() > 150
+    out = _run(Q, K, U, V, R, dO)
+    assert torch.equal(out[0][:, :, 7], torch.zeros(B, H, dh))
+    # the sigmoid of a pre-activation m is off by |m| times m's own relative rounding: 2^-24 of a few hundred
+    for name, got, ref in zip(NAMES, out, _oracle(Q, K, U, V, R, dO)):
+        assert torch.isfinite(got).all(), name
+        assert _error(got, ref) <= 16 * _bound(*shape), (name, _error(got, ref))
