@@ -184,7 +184,7 @@ __device__ __forceinline__ void store_row(const f32x16 (&acc)[CT], float* dst, i
 // instructions (32 to 1,024 tokens, d_h 24 to 128; O 3.5e-7 -> 2.7e-7, dQ 4.0 -> 3.4, dK, dU, dV 3.4 -> 2.8, dR 3.7 -> 3.0 for
 // 256 tokens of the 128M layer).  The matrix instructions take a plane below 2^-126 for zero, so an operand counts to
 // 2^-126 absolutely (values below 2^-110 lose their last bits).  An infinity or NaN in an operand makes every sum that it enters
-// infinite or NaN; an infinity comes out as NaN where it meets a zero plane.
+// NaN: such rows are taken again (below, "the same on the fp32 matrix instructions").
 constexpr int PLANE_B = TILE_B;                 // one plane of a 32-row tile, in the layout of the bf16 kernels' tiles
 constexpr int PLANES_B = 3 * PLANE_B;
 
@@ -414,6 +414,128 @@ struct Block {
     }
 };
 
+// ---- the same on the fp32 matrix instructions -------------------------------------------------------------------------------
+// What the planes cannot carry comes out as NaN: an infinity in an operand, or a value beyond the largest float32 between the products
+// (infinity minus infinity, in split2).  A row of results that is not finite is therefore taken again on
+// v_mfma_f32_32x32x2_f32, which knows infinities, by the waves of its workgroup together; the workgroup's other rows keep theirs.
+// 256 tokens of the 128M layer: looking for such rows takes 0.1 (forward), 0.4 (dQ/dR) and 0.9 us (dK/dU/dV) of 24.5, 34.3 and 45.1;
+// with one in every workgroup the kernels take 47, 67 and 95 us, alone on these instructions 30, 46 and 61.
+__device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; }
+template <int CT>
+__device__ __forceinline__ bool finite(const f32x16 (&acc)[CT])
+{
+    unsigned most = 0;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) most = max(most, __float_as_uint(acc[ct][i]) & 0x7fffffffu);
+    return most < 0x7f800000u;
+}
+// Whether it holds in this lane or in the one with the other half of its row.
+__device__ __forceinline__ bool in_row(bool here)
+{
+    const int other = __shfl_xor((int)here, 32);      // (read by every lane)
+    return here || other != 0;
+}
+// Whether `here` holds in a lane of the workgroup, which is done with its LDS; word: four bytes of it per wave (of four).
+__device__ __forceinline__ bool anywhere(bool here, unsigned char* words, int wave)
+{
+    volatile unsigned* word = reinterpret_cast<volatile unsigned*>(words);
+    const bool own = __ballot(here) != 0;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) word[wave] = own;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(word[0] | word[1] | word[2] | word[3]) != 0;
+}
+// K, U and V tiles of block b by four waves, waited for.
+template <int CT>
+__device__ __forceinline__ void fill_block(const F32Args& p, const Block& b, unsigned char* lds, int wave)
+{
+    using T = Tile<CT>;
+    constexpr int FI = T::INS / 4 > 0 ? T::INS / 4 : 1;      // fill instructions per wave and tile
+    __syncthreads();      // every wave is done with the block before
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));      // (the fills' addresses are not worth a register each)
+    auto row = [&](const float* W) {
+        return [&, W](int r) { return W + (b.wrow + (r < b.rows ? r : b.rows - 1)) * p.DH; };
+    };
+#pragma unroll
+    for (int k = 0; k < FI; ++k) {
+        T::fill(lds, wave * FI + k, lane, p.DH, row(p.K));
+        T::fill(lds + T::BYTES, wave * FI + k, lane, p.DH, row(p.U));
+        T::fill(lds + 2 * T::BYTES, wave * FI + k, lane, p.DH, row(p.V));
+    }
+    wait_vmcnt<0>();
+    __syncthreads();
+}
+// O of this wave's rows over the part's blocks.
+template <int CT>
+__device__ __forceinline__ void fwd_fp32(const F32Args& p, const Place& w, unsigned char* lds, int wave, f32x16 (&o)[CT])
+{
+    using T = Tile<CT>;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+    f32x4 q[4 * CT];
+    load_row<CT>(q, p.Q + p.rows.tok(w.hk, w.row) * p.DH, g, p.DH);
+    const float* rrow = p.R + p.rows.gate(w.hk, w.row) * p.parts.E;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) o[ct] = zero16();
+    for (int blk = 0; blk < w.nblk; ++blk) {
+        const Block b(p, w.hk, w.blk0 + blk);
+        const float r = rrow[b.e];
+        fill_block<CT>(p, b, lds, wave);
+        f32x16 mn[2];
+        const typename T::Lane l(l32, g);
+        first_products<CT, 2>(mn, {lds, lds + T::BYTES}, {q, q}, l);
+        f32x16 &m = mn[0], &n = mn[1];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float v = m[i] * sigmoid_exact(m[i]) * n[i] * r;
+            asm volatile("" : "+v"(v));      // (or the compiler makes a branch of each element)
+            m[i] = reg_row(i, g) < b.rows ? v : 0.0f;
+        }
+        second_product<CT>(o, lds + 2 * T::BYTES, m, l);
+    }
+}
+// dQ of this wave's rows over the part's blocks, and their dR to drow where `store` holds.
+template <int CT>
+__device__ __forceinline__ void dqdr_fp32(const F32Args& p, const Place& w, unsigned char* lds, int wave, float* drow, bool store, f32x16 (&dq)[CT])
+{
+    using T = Tile<CT>;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+    const long tok = p.rows.tok(w.hk, w.row) * p.DH;
+    f32x4 q[4 * CT], go[4 * CT];
+    load_row<CT>(q, p.Q + tok, g, p.DH);
+    load_row<CT>(go, p.dO + tok, g, p.DH);
+    const float* rrow = p.R + p.rows.gate(w.hk, w.row) * p.parts.E;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) dq[ct] = zero16();
+    float dr = 0.0f;
+    for (int blk = 0; blk < w.nblk; ++blk) {
+        const Block b(p, w.hk, w.blk0 + blk);
+        const float r = rrow[b.e];
+        fill_block<CT>(p, b, lds, wave);
+        f32x16 mna[3];
+        const typename T::Lane l(l32, g);
+        first_products<CT, 3>(mna, {lds, lds + T::BYTES, lds + 2 * T::BYTES}, {q, q, go}, l);
+        f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float sg = sigmoid_exact(m[i]), sl = m[i] * sg;
+            const float a = reg_row(i, g) < b.rows ? da[i] : 0.0f;
+            dr = fmaf(a * sl, n[i], dr);
+            m[i] = r * a * n[i] * (sg + sl * (1.0f - sg));      // dM
+            n[i] = r * a * sl;                                  // dN
+        }
+        second_product<CT>(dq, lds, m, l);
+        second_product<CT>(dq, lds + T::BYTES, n, l);
+        if (blk + 1 == w.nblk || Block(p, w.hk, w.blk0 + blk + 1).e != b.e) {
+            const float tot = dr + __shfl_xor(dr, 32);
+            if (g == 0 && store) drow[b.e] = tot;
+            dr = 0.0f;
+        }
+    }
+}
+
 // Forward: 128 rows, GROUPS teams of four waves that take the blocks of the part in turn, their sums added at the end.  A team's
 // threads take the next block's weights apart on their way from memory to LDS, K and U under the second products, V under the first.
 template <int CT, int GROUPS>
@@ -505,9 +627,16 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS) void fwd_f32_kernel(F32Args p
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[ct][i] += xch[(ct * 16 + i) * 64];
     }
-    if (w.valid)
-        store_row<CT>(o, p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * DH
-                                            : p.O + p.rows.tok(w.hk, w.row) * DH, g, DH);
+    // (the place of a lane's row is worked out anew, out of the compiler's sight, instead of kept)
+    int l32b = l32;
+    asm volatile("" : "+v"(l32b));
+    const Place w2(p, wave, l32b);
+    const bool again = in_row(!finite(o)) && w2.valid;
+    float* dst = p.parts.nsplit > 1 ? p.part + (((long)w2.z * p.rows.Hkuv + w2.hk) * p.rows.n + w2.row) * DH : p.O + p.rows.tok(w2.hk, w2.row) * DH;
+    if (w2.valid && !again) store_row<CT>(o, dst, g, DH);
+    if (!anywhere(again, lds + GROUPS * 3 * PLANES_B - 16, wave)) return;
+    fwd_fp32<CT>(p, w2, lds, wave, o);
+    if (again) store_row<CT>(o, dst, g, DH);
 }
 
 // dQ and dR: four waves of 32 rows, alone on their SIMDs.  LDS: the planes of two blocks; the next block's weights are taken apart
@@ -561,6 +690,7 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) dq[ct] = zero16();
     float dr = 0.0f;
+    bool again = false;      // a result of this row is not finite
     Block b(p, w.hk, w.blk0);
     float r = rrow[b.e];
     for (int blk = 0; blk < w.nblk; ++blk) {
@@ -632,20 +762,28 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
         if (blk + 1 == w.nblk || next.e != b.e) {
             const float tot = dr + __shfl_xor(dr, 32);      // the two lane halves hold different rows j of the same token
             if (g == 0 && w.valid) drow[b.e] = tot;
+            again |= !finite(tot);
             dr = 0.0f;
         }
         b = next;
         r = rnext;
     }
-    if (w.valid)
-        store_row<CT>(dq, p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * DH : p.dQ + tok, g, DH);
+    again |= !finite(dq);
+    again = in_row(again) && w.valid;
+    float* dst = p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * DH : p.dQ + tok;
+    if (w.valid && !again) store_row<CT>(dq, dst, g, DH);
+    if (!anywhere(again, lds + 6 * PLANES_B - 16, wave)) return;
+    dqdr_fp32<CT>(p, w, lds, wave, drow, again, dq);
+    if (again) store_row<CT>(dq, dst, g, DH);
 }
 
-// End of a dK/dU/dV kernel: the odd tiles' sums to the wave with the even ones, one gradient at a time (64 lanes x 16 CT floats,
-// lane-private), then to memory.  (This lane's row and the bounds of its columns are worked out again, out of the compiler's
-// sight: kept over the loop they are the few registers too many that made it spill for d_h > 96.)
-template <int CT>
-__device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned char* lds, f32x16 (&dk)[CT], f32x16 (&du)[CT], f32x16 (&dv)[CT])
+// End of a dK/dU/dV kernel: the odd tiles' sums to the wave with the even ones (64 lanes x 48 CT floats, lane-private), then the
+// rows that `take` picks to memory: take(finite) says whether a row goes, given whether all of it is finite.  (This lane's row and
+// the bounds of its columns are worked out again, out of the compiler's sight: kept over the loop they are the few registers too many
+// that made it spill for d_h > 96.)
+template <int CT, class Take>
+__device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned char* lds, f32x16 (&dk)[CT], f32x16 (&du)[CT], f32x16 (&dv)[CT],
+                                                     Take&& take)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
     const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
@@ -667,7 +805,7 @@ __device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned 
             }
     }
     __syncthreads();
-    if (half == 1 || blk >= nblk || l32 >= b.rows) return;
+    if (half == 1 || blk >= nblk) return;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -676,6 +814,7 @@ __device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned 
             du[ct][i] += xch[((CT + ct) * 16 + i) * 64];
             dv[ct][i] += xch[((2 * CT + ct) * 16 + i) * 64];
         }
+    if (!take([&] { return !in_row(!finite(dk) || !finite(du) || !finite(dv)); }) || l32 >= b.rows) return;
     const long wrow = b.wrow + l32, wsz = (long)p.rows.Hkuv * E * p.de * DH;
     auto store_bf16 = [&](const f32x16(&acc)[CT], void* out) {
         bf16_t* dst = static_cast<bf16_t*>(out) + wrow * DH;
@@ -703,6 +842,78 @@ __device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned 
         store_bf16(dk, p.out[0]);
         store_bf16(du, p.out[1]);
         store_bf16(dv, p.out[2]);
+    }
+}
+
+// dK, dU, dV.  A wave owns one block of weight rows (B operands and accumulators stay in registers) and every other
+// 32-row tile of its slice of the head's rows: waves 0, 1 take the even tiles of two blocks, waves 2, 3 the odd ones, and their
+// sums meet in LDS at the end.  (Halving the tiles inside the workgroup doubles the workgroups of a layer whose blocks are
+// few, without partial sums in memory; LDS is idle, so that each pair of waves has tiles of its own costs nothing.)
+template <int CT>
+__device__ __forceinline__ void dkdudv_fp32(const F32Args& p, unsigned char* lds, f32x16 (&dk)[CT], f32x16 (&du)[CT], f32x16 (&dv)[CT])
+{
+    using T = Tile<CT>;
+    constexpr int FI = T::INS / 2 > 0 ? T::INS / 2 : 1;
+    constexpr int STAGE_B = 2 * T::BYTES;      // Q and dO tile
+    float* sR = reinterpret_cast<float*>(lds + 4 * STAGE_B);      // [stage][wave][32] gate values
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
+    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
+    const int blk = blockIdx.x * 2 + bw;
+    const Block b(p, hk, blk < nblk ? blk : nblk - 1);
+
+    const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5, DH = p.DH;
+    const int ntile = (p.rows.n + 31) / 32;
+    const int t0 = (int)((long)ntile * z / p.nslice), t1 = (int)((long)ntile * (z + 1) / p.nslice);
+    const int steps = (t1 - t0 + 1) / 2;
+    auto fill = [&](int s) {
+        const int t = t0 + 2 * s + half;
+        const int row0 = 32 * (t < ntile ? t : ntile - 1);
+        unsigned char* stage = lds + (half * 2 + (s & 1)) * STAGE_B;
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));      // (the fills' addresses are not worth a register each)
+        auto row = [&](const float* W) {
+            return [&, W](int r) { return W + p.rows.tok_head_major(hk, row0 + r < p.rows.n ? row0 + r : p.rows.n - 1) * DH; };
+        };
+#pragma unroll
+        for (int k = 0; k < FI; ++k) {
+            T::fill(stage, bw * FI + k, lane, DH, row(p.Q));
+            T::fill(stage + T::BYTES, bw * FI + k, lane, DH, row(p.dO));
+        }
+        // gate values of this wave's expert; 0 for the rows that a tile lacks, which removes them from every product
+        if (g == 0) {
+            const bool ok = t < t1 && row0 + l32 < p.rows.n;
+            sR[((s & 1) * 4 + wave) * 32 + l32] = ok ? p.R[p.rows.head_major(hk, ok ? row0 + l32 : 0) * E + b.e] : 0.0f;
+        }
+    };
+    fill(0);
+    f32x4 kB[4 * CT], uB[4 * CT], vB[4 * CT];
+    const long wrow = b.wrow + (l32 < b.rows ? l32 : b.rows - 1);
+    load_row<CT>(kB, p.K + wrow * DH, g, DH);
+    load_row<CT>(uB, p.U + wrow * DH, g, DH);
+    load_row<CT>(vB, p.V + wrow * DH, g, DH);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) { dk[ct] = zero16(); du[ct] = zero16(); dv[ct] = zero16(); }
+
+    for (int s = 0; s < steps; ++s) {
+        const unsigned char *sQ = lds + (half * 2 + (s & 1)) * STAGE_B, *sG = sQ + T::BYTES;
+        wait_vmcnt<0>();
+        __syncthreads();
+        if (s + 1 < steps) fill(s + 1);
+        f32x16 mna[3];
+        const typename T::Lane l(l32, g);
+        first_products<CT, 3>(mna, {sQ, sQ, sG}, {kB, uB, vB}, l);
+        f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
+        const float* rw = sR + ((s & 1) * 4 + wave) * 32;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float r = rw[reg_row(i, g)], sg = sigmoid_exact(m[i]), sl = m[i] * sg, a = da[i], nn = n[i];
+            m[i] = r * a * nn * (sg + sl * (1.0f - sg));      // dM
+            n[i] = r * a * sl;                                // dN
+            da[i] = r * sl * nn;                              // P
+        }
+        second_product<CT>(dk, sQ, m, l);
+        second_product<CT>(du, sQ, n, l);
+        second_product<CT>(dv, sG, da, l);
     }
 }
 
@@ -859,84 +1070,21 @@ __global__ __launch_bounds__(256, 1) void dkdudv_split_kernel(F32Args p)
         second_split<CT>(dv, planes + PLANES_B, 1, split8_of(pp), pl, [](auto) {});
         __syncthreads();      // the planes have been read
     }
-    add_halves_and_store<CT>(p, lds, dk, du, dv);
+    wait_vmcnt<0>();         // what the last step has requested is not used, but lands in LDS
+    bool again = false;      // this lane's row is not finite
+    add_halves_and_store<CT>(p, lds, dk, du, dv, [&](auto all_finite) { return !(again = !all_finite()); });
+    if (!anywhere(again, lds + 4 * PLANES_B + 16 * CT * 1024, wave)) return;
+    dkdudv_fp32<CT>(p, lds, dk, du, dv);
+    add_halves_and_store<CT>(p, lds, dk, du, dv, [&](auto) { return again; });
 }
 
-// dK, dU, dV.  A wave owns one block of weight rows (B operands and accumulators stay in registers) and every other
-// 32-row tile of its slice of the head's rows: waves 0, 1 take the even tiles of two blocks, waves 2, 3 the odd ones, and their
-// sums meet in LDS at the end.  (Halving the tiles inside the workgroup doubles the workgroups of a layer whose blocks are
-// few, without partial sums in memory; LDS is idle, so that each pair of waves has tiles of its own costs nothing.)
 template <int CT>
 __global__ __launch_bounds__(256, 1) void dkdudv_f32_kernel(F32Args p)
 {
-    using T = Tile<CT>;
-    constexpr int FI = T::INS / 2 > 0 ? T::INS / 2 : 1;
-    constexpr int STAGE_B = 2 * T::BYTES;      // Q and dO tile
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    float* sR = reinterpret_cast<float*>(lds + 4 * STAGE_B);      // [stage][wave][32] gate values
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
-    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
-    const int blk = blockIdx.x * 2 + bw;
-    const Block b(p, hk, blk < nblk ? blk : nblk - 1);
-
     f32x16 dk[CT], du[CT], dv[CT];
-    {
-        const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5, DH = p.DH;
-        const int ntile = (p.rows.n + 31) / 32;
-        const int t0 = (int)((long)ntile * z / p.nslice), t1 = (int)((long)ntile * (z + 1) / p.nslice);
-        const int steps = (t1 - t0 + 1) / 2;
-        auto fill = [&](int s) {
-            const int t = t0 + 2 * s + half;
-            const int row0 = 32 * (t < ntile ? t : ntile - 1);
-            unsigned char* stage = lds + (half * 2 + (s & 1)) * STAGE_B;
-            int lane = threadIdx.x & 63;
-            asm volatile("" : "+v"(lane));      // (the fills' addresses are not worth a register each)
-            auto row = [&](const float* W) {
-                return [&, W](int r) { return W + p.rows.tok_head_major(hk, row0 + r < p.rows.n ? row0 + r : p.rows.n - 1) * DH; };
-            };
-#pragma unroll
-            for (int k = 0; k < FI; ++k) {
-                T::fill(stage, bw * FI + k, lane, DH, row(p.Q));
-                T::fill(stage + T::BYTES, bw * FI + k, lane, DH, row(p.dO));
-            }
-            // gate values of this wave's expert; 0 for the rows that a tile lacks, which removes them from every product
-            if (g == 0) {
-                const bool ok = t < t1 && row0 + l32 < p.rows.n;
-                sR[((s & 1) * 4 + wave) * 32 + l32] = ok ? p.R[p.rows.head_major(hk, ok ? row0 + l32 : 0) * E + b.e] : 0.0f;
-            }
-        };
-        fill(0);
-        f32x4 kB[4 * CT], uB[4 * CT], vB[4 * CT];
-        const long wrow = b.wrow + (l32 < b.rows ? l32 : b.rows - 1);
-        load_row<CT>(kB, p.K + wrow * DH, g, DH);
-        load_row<CT>(uB, p.U + wrow * DH, g, DH);
-        load_row<CT>(vB, p.V + wrow * DH, g, DH);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) { dk[ct] = zero16(); du[ct] = zero16(); dv[ct] = zero16(); }
-
-        for (int s = 0; s < steps; ++s) {
-            const unsigned char *sQ = lds + (half * 2 + (s & 1)) * STAGE_B, *sG = sQ + T::BYTES;
-            wait_vmcnt<0>();
-            __syncthreads();
-            if (s + 1 < steps) fill(s + 1);
-            f32x16 mna[3];
-            const typename T::Lane l(l32, g);
-            first_products<CT, 3>(mna, {sQ, sQ, sG}, {kB, uB, vB}, l);
-            f32x16 &m = mna[0], &n = mna[1], &da = mna[2];
-            const float* rw = sR + ((s & 1) * 4 + wave) * 32;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float r = rw[reg_row(i, g)], sg = sigmoid_exact(m[i]), sl = m[i] * sg, a = da[i], nn = n[i];
-                m[i] = r * a * nn * (sg + sl * (1.0f - sg));      // dM
-                n[i] = r * a * sl;                                // dN
-                da[i] = r * sl * nn;                              // P
-            }
-            second_product<CT>(dk, sQ, m, l);
-            second_product<CT>(du, sQ, n, l);
-            second_product<CT>(dv, sG, da, l);
-        }
-    }
-    add_halves_and_store<CT>(p, lds, dk, du, dv);
+    dkdudv_fp32<CT>(p, lds, dk, du, dv);
+    add_halves_and_store<CT>(p, lds, dk, du, dv, [](auto) { return true; });
 }
 
 // Adds the parts' sums in order: the rows of O or dQ (dst, four columns per lane) and, for blockIdx.x >= row_blocks, the

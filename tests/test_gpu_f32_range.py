@@ -69,3 +69,41 @@ def test_saturated_preactivations(dh, sign):
     for name, got, ref in zip(NAMES, out, _oracle(Q, K, U, V, R, dO)):
         assert torch.isfinite(got).all(), name
         assert _error(got, ref) <= 16 * _bound(*shape), (name, _error(got, ref))
+
+
+def _same_with_infinities(name, got, want):
+    """Infinities and NaN in the same places, and the rest alike."""
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(got), kind(want)), (name, kind, kind(got).sum(), kind(want).sum())
+    ok = torch.isfinite(want)
+    if ok.any():
+        assert _error(got[ok], want[ok].double()) <= 1e-5, name
+
+
+def _eager(Q, K, U, V, R, dO):
+    return (orc.mhffn_forward(Q, K, U, V, R, compute_dtype=torch.float32), *orc.mhffn_backward(Q, K, U, V, R, dO, compute_dtype=torch.float32))
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf")])
+@pytest.mark.parametrize("B,H,S,dh,E,de", [(1, 2, 70, 24, 2, 40), (1, 2, 70, 64, 2, 64), (1, 1, 130, 96, 3, 64), (1, 1, 300, 96, 8, 256), (1, 2, 45, 128, 2, 72)])
+def test_an_infinite_weight(B, H, S, dh, E, de, value):
+    """One infinite value of V: infinities of the signs that float32 arithmetic gives in O, dQ and dR, and NaN in its rows of dK and dU."""
+    print(f"case S={S} d_h={dh} E={E} d_e={de} value={value}", flush=True)
+    ins = make_inputs(B, H, S, dh, E, de, H, seed=dh, dtype=torch.float32)
+    ins[3][H - 1, E - 1, 37, dh - 2] = value
+    for name, got, want in zip(NAMES, _run(*ins), _eager(*ins)):
+        _same_with_infinities(name, got, want)
+        assert torch.isfinite(got[:, 0]).all() if H > 1 and name in ("O", "dQ", "dR") else not torch.isfinite(got).all() or name == "dV"
+
+
+@pytest.mark.parametrize("dh", [24, 64, 96, 128])
+def test_products_beyond_the_largest_number(dh):
+    """SiLU(M) N overflows for two tokens, from finite operands: O has their infinities, and the gradients' rows what float32 gives."""
+    Q, K, U, V, R, dO = (t.abs() for t in make_inputs(1, 2, 70, dh, 2, 64, 2, seed=6, dtype=torch.float32))
+    Q[0, 1, 5] *= 1e22
+    Q[0, 1, 40] *= 1e25
+    V[:, :, :, 1] *= -1
+    got, want = _run(Q, K, U, V, R, dO), _eager(Q, K, U, V, R, dO)
+    assert torch.isposinf(want[0][0, 1, 5, 0]) and torch.isneginf(want[0][0, 1, 5, 1])
+    for name, a, b in zip(NAMES, got, want):
+        _same_with_infinities(name, a, b)
