@@ -176,15 +176,16 @@ __device__ __forceinline__ void store_row(const f32x16 (&acc)[CT], float* dst, i
 }
 
 // ---- float32 operands on the bf16 matrix instructions -----------------------------------------------------------------
-// A float32 value is the exact sum of three bfloat16 values (8 + 8 + 8 bits: the upper half of its pattern, then the rest
-// rounded, then what is left).  Of the nine products of two such sums the six of the largest terms run on
-// v_mfma_f32_32x32x16_bf16, which has sixteen times the rate of v_mfma_f32_32x32x2_f32; the three left out are at most 2^-23
-// of the product, 2^-26 on average and of either sign, below what one float32 addition rounds away.  A sum over k then rounds once
+// A float32 value is the exact sum of three bfloat16 values: it rounded to one, the rest rounded, and what is left.  With units of the
+// value's binade these are at most 2, 2^-8 and 2^-17.  Of the nine products of two such sums the six of the largest terms run on
+// v_mfma_f32_32x32x16_bf16, which has sixteen times the rate of v_mfma_f32_32x32x2_f32; the three left out are at most 2^-24
+// of the product (2^-24.06 found by trying), no more than one float32 addition rounds away, and of either sign over mantissas.  (With
+// the largest plane cut off instead of rounded they reach 2^-22.)  A sum over k then rounds once
 // per sixteen terms and plane instead of once per two: against 64 bits the results are 10 to 30 % closer than those of the fp32
-// instructions (32 to 1,024 tokens, d_h 24 to 128; O 3.5e-7 -> 2.7e-7, dQ 4.0 -> 3.4, dK, dU, dV 3.4 -> 2.8, dR 3.7 -> 3.0 for
-// 256 tokens of the 128M layer).  The matrix instructions take a plane below 2^-126 for zero, so an operand counts to
-// 2^-126 absolutely (values below 2^-110 lose their last bits).  An infinity or NaN in an operand makes every sum that it enters
-// NaN: such rows are taken again (below, "the same on the fp32 matrix instructions").
+// instructions (32 to 1,024 tokens, d_h 24 to 128; O 3.5e-7 -> 2.7e-7, dQ 4.0 -> 3.4, dK, dU, dV 3.4 -> 2.8, dR 3.6 -> 3.0
+// for 256 tokens of the 128M layer).  The matrix instructions take a plane below 2^-126 for zero, so an operand counts to
+// 2^-126 absolutely (values below 2^-110 lose their last bits).  An infinity or NaN in an operand, or a value that rounds to an infinite
+// bfloat16, makes every sum that it enters NaN: such rows are taken again (below, "the same on the fp32 matrix instructions").
 constexpr int PLANE_B = TILE_B;                 // one plane of a 32-row tile, in the layout of the bf16 kernels' tiles
 constexpr int PLANES_B = 3 * PLANE_B;
 
@@ -192,11 +193,14 @@ constexpr int PLANES_B = 3 * PLANE_B;
 __device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned& m, unsigned& l)
 {
     typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
-    const unsigned b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
-    h = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-    const float r0 = x0 - __uint_as_float(b0 & 0xffff0000u), r1 = x1 - __uint_as_float(b1 & 0xffff0000u);
-    m = __builtin_bit_cast(unsigned, bf16x2{(bf16_t)r0, (bf16_t)r1});
-    asm("" : "+v"(m));      // (or the compiler rounds r0 a second time instead of shifting the pair)
+    auto round = [](float a, float b) {
+        unsigned v = __builtin_bit_cast(unsigned, bf16x2{(bf16_t)a, (bf16_t)b});
+        asm("" : "+v"(v));      // (or the compiler rounds a second time instead of shifting the pair)
+        return v;
+    };
+    h = round(x0, x1);
+    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+    m = round(r0, r1);
     l = __builtin_bit_cast(unsigned, bf16x2{(bf16_t)(r0 - __uint_as_float(m << 16)), (bf16_t)(r1 - __uint_as_float(m & 0xffff0000u))});
 }
 struct Split8 {
