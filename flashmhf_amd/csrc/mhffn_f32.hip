@@ -40,13 +40,13 @@ struct F32Args {
 
 __device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + __expf(-x)); }
-// The same in the kernels that have VALU time to lose: the reciprocal with one Newton step (an IEEE division takes three times the instructions), of a sixteenth of
-// the sum, whose reciprocal is a normal number up to the largest finite e^-x; 0 beyond that, where the step would make NaN of an
-// infinite one.
-__device__ __forceinline__ float sigmoid_newton(float x)
+// Sixteen times that of x = 2^-48 xs, in the kernels that have VALU time to lose: the reciprocal with one Newton step (an IEEE division
+// takes three times the instructions), a normal number up to the largest finite e^-x; 0 beyond that, where the step would make
+// NaN of an infinite one.
+__device__ __forceinline__ float sigmoid16(float xs)
 {
-    const float t = -LOG2E * x, d = fmaf(__builtin_amdgcn_exp2f(t), 0.0625f, 0.0625f), y = __builtin_amdgcn_rcpf(d);
-    const float s = fmaf(fmaf(-d, y, 1.0f), y, y) * 0.0625f;
+    const float t = -LOG2E * 0x1p-48f * xs, d = fmaf(__builtin_amdgcn_exp2f(t), 0.0625f, 0.0625f), y = __builtin_amdgcn_rcpf(d);
+    const float s = fmaf(fmaf(-d, y, 1.0f), y, y);
     return t >= 128.0f ? 0.0f : s;
 }
 __device__ __forceinline__ f32x16 zero16()
@@ -183,9 +183,14 @@ __device__ __forceinline__ void store_row(const f32x16 (&acc)[CT], float* dst, i
 // the largest plane cut off instead of rounded they reach 2^-22.)  A sum over k then rounds once
 // per sixteen terms and plane instead of once per two: against 64 bits the results are 10 to 30 % closer than those of the fp32
 // instructions (32 to 1,024 tokens, d_h 24 to 128; O 3.5e-7 -> 2.7e-7, dQ 4.0 -> 3.4, dK, dU, dV 3.4 -> 2.8, dR 3.6 -> 3.0
-// for 256 tokens of the 128M layer).  The matrix instructions take a plane below 2^-126 for zero, so an operand counts to
-// 2^-126 absolutely (values below 2^-110 lose their last bits).  An infinity or NaN in an operand, or a value that rounds to an infinite
+// for 256 tokens of the 128M layer).
+// The matrix instructions take a plane below 2^-126 for zero, and the last plane is 2^-23 of a value: operands are taken apart 2^24
+// times as large, which holds every float32 to its last bit.  First products are 2^48 times as large, and so are dM, dN and P (without a
+// multiplication more); the sums of the second products are 2^72 times as large.
+// What is too large for that (products beyond 2^79, P, dM and dN beyond 2^79, results beyond 2^55) overflows.  An infinity or NaN in an operand, or a value that rounds to an infinite
 // bfloat16, makes every sum that it enters NaN: such rows are taken again (below, "the same on the fp32 matrix instructions").
+constexpr float UP = 0x1p24f;                   // of an operand of the first products and of weights
+constexpr float DOWN1 = 0x1p-48f, DOWN2 = 0x1p-72f;      // results of the first and of the second products
 constexpr int PLANE_B = TILE_B;                 // one plane of a 32-row tile, in the layout of the bf16 kernels' tiles
 constexpr int PLANES_B = 3 * PLANE_B;
 
@@ -236,14 +241,14 @@ __device__ __forceinline__ Split8 split8(V&& x)      // x(0) .. x(7)
 // the planes of the six products, smallest terms first
 constexpr int SPLIT_A[6] = {2, 0, 1, 1, 0, 0}, SPLIT_B[6] = {0, 2, 1, 0, 1, 0};
 
-// four values taken apart, two at a time
+// four weights taken apart, two at a time
 struct CutPiece {
     u32x2 h, m, l;
     template <int I>
     __device__ __forceinline__ void half(const f32x4& x)
     {
         unsigned a, b, c;
-        split2(x[2 * I], x[2 * I + 1], a, b, c);
+        split2(UP * x[2 * I], UP * x[2 * I + 1], a, b, c);
         h[I] = a; m[I] = b; l[I] = c;
     }
 };
@@ -386,7 +391,7 @@ template <int CT>
 __device__ __forceinline__ void split_row_operand(Split8 (&v)[2 * CT], const f32x4 (&x)[4 * CT])
 {
 #pragma unroll
-    for (int ks = 0; ks < 2 * CT; ++ks) v[ks] = split8([&](int i) { return x[2 * ks + (i >> 2)][i & 3]; });
+    for (int ks = 0; ks < 2 * CT; ++ks) v[ks] = split8([&](int i) { return UP * x[2 * ks + (i >> 2)][i & 3]; });
 }
 
 // Workgroup of the forward and of dQ/dR: 4 waves of 32 rows of one K/U/V head, one part of the head's blocks.
@@ -434,6 +439,14 @@ __device__ __forceinline__ bool finite(const f32x16 (&acc)[CT])
 #pragma unroll
         for (int i = 0; i < 16; ++i) most = max(most, __float_as_uint(acc[ct][i]) & 0x7fffffffu);
     return most < 0x7f800000u;
+}
+template <int CT>
+__device__ __forceinline__ void scale(f32x16 (&acc)[CT], float by)
+{
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[ct][i] *= by;
 }
 // Whether it holds in this lane or in the one with the other half of its row.
 __device__ __forceinline__ bool in_row(bool here)
@@ -598,7 +611,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS) void fwd_f32_kernel(F32Args p
         f32x16 &m = mn[0], &n = mn[1];
         mfma_result_fence(m, n);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) m[i] *= sigmoid_newton(m[i]) * n[i] * r;
+        for (int i = 0; i < 16; ++i) m[i] = m[i] * sigmoid16(m[i]) * (0.0625f * DOWN1) * n[i] * r;
         if (b.rows < JB) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) m[i] = split_row(i, g) < b.rows ? m[i] : 0.0f;
@@ -636,6 +649,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS) void fwd_f32_kernel(F32Args p
     asm volatile("" : "+v"(l32b));
     const Place w2(p, wave, l32b);
     const bool again = in_row(!finite(o)) && w2.valid;
+    scale(o, DOWN2);
     float* dst = p.parts.nsplit > 1 ? p.part + (((long)w2.z * p.rows.Hkuv + w2.hk) * p.rows.n + w2.row) * DH : p.O + p.rows.tok(w2.hk, w2.row) * DH;
     if (w2.valid && !again) store_row<CT>(o, dst, g, DH);
     if (!anywhere(again, lds + GROUPS * 3 * PLANES_B - 16, wave)) return;
@@ -718,12 +732,12 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
 #pragma unroll
             for (int i = 0; i < 16; ++i) da[i] = split_row(i, g) < b.rows ? da[i] : 0.0f;
         }
-        float sg;
-        auto sigma = [&](int i) { sg = sigmoid_newton(m[i]); };
-        auto element = [&](int i) {
-            const float sl = m[i] * sg, a = da[i] * sl, ra = r * da[i];
-            dr = fmaf(a, n[i], dr);
-            m[i] = ra * n[i] * fmaf(sl, 1.0f - sg, sg);         // dM
+        float sg16;
+        auto sigma = [&](int i) { sg16 = sigmoid16(m[i]); };
+        auto element = [&](int i) {      // (sl and nn as they are; da, dM, dN and dR times 2^48)
+            const float sl = m[i] * sg16 * (0.0625f * DOWN1), sg = 0.0625f * sg16, nn = DOWN1 * n[i], a = da[i] * sl, ra = r * da[i];
+            dr = fmaf(a, nn, dr);
+            m[i] = ra * nn * fmaf(sl, 1.0f - sg, sg);           // dM
             n[i] = r * a;                                       // dN
         };
 #pragma unroll
@@ -765,7 +779,7 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
         second_split<CT>(dq, planes + PLANES_B, 1, split8_of(dn), pl, [](auto) {});
         if (blk + 1 == w.nblk || next.e != b.e) {
             const float tot = dr + __shfl_xor(dr, 32);      // the two lane halves hold different rows j of the same token
-            if (g == 0 && w.valid) drow[b.e] = tot;
+            if (g == 0 && w.valid) drow[b.e] = DOWN1 * tot;
             again |= !finite(tot);
             dr = 0.0f;
         }
@@ -774,6 +788,7 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
     }
     again |= !finite(dq);
     again = in_row(again) && w.valid;
+    scale(dq, DOWN2);
     float* dst = p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * DH : p.dQ + tok;
     if (w.valid && !again) store_row<CT>(dq, dst, g, DH);
     if (!anywhere(again, lds + 6 * PLANES_B - 16, wave)) return;
@@ -1013,13 +1028,13 @@ __global__ __launch_bounds__(256, 1) void dkdudv_split_kernel(F32Args p)
         };
         gates(0);
         mfma_result_fence(m, n, da);
-        float sg;
-        auto sigma = [&](int i) { sg = sigmoid_newton(m[i]); };
-        auto element = [&](int i) {
-            const float r = r4[(i >> 2) & 1][i & 3], sl = m[i] * sg, ra = r * da[i], nn = n[i];
+        float sg16;
+        auto sigma = [&](int i) { sg16 = sigmoid16(m[i]); };
+        auto element = [&](int i) {      // (sl and nn as they are; da, dM, dN and P times 2^48)
+            const float r = r4[(i >> 2) & 1][i & 3], sl = m[i] * sg16 * (0.0625f * DOWN1), sg = 0.0625f * sg16, ra = r * da[i], ns = n[i], nn = DOWN1 * ns;
             m[i] = ra * nn * fmaf(sl, 1.0f - sg, sg);      // dM
             n[i] = ra * sl;                                // dN
-            da[i] = r * sl * nn;                           // P
+            da[i] = r * sl * ns;                           // P
         };
         static_for<8>([&](auto ic) {
             sigma(decltype(ic)::value);
@@ -1075,6 +1090,9 @@ __global__ __launch_bounds__(256, 1) void dkdudv_split_kernel(F32Args p)
         __syncthreads();      // the planes have been read
     }
     wait_vmcnt<0>();         // what the last step has requested is not used, but lands in LDS
+    scale(dk, DOWN2);
+    scale(du, DOWN2);
+    scale(dv, DOWN2);
     bool again = false;      // this lane's row is not finite
     add_halves_and_store<CT>(p, lds, dk, du, dv, [&](auto all_finite) { return !(again = !all_finite()); });
     if (!anywhere(again, lds + 4 * PLANES_B + 16 * CT * 1024, wave)) return;

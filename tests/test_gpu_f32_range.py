@@ -132,3 +132,26 @@ def test_products_are_not_cut_to_one_side(dh):
     off = ((got.double() - want) / want).mean().item() * 2 ** 24
     print("mean error in 2^-24:", off, flush=True)
     assert abs(off) <= 1.5
+
+
+# powers of two that Q, K and U, V, R, dO are multiplied by
+SMALL = [(0, 0, 0, 0, -114), (0, 0, -114, 0, 0), (0, 0, 0, -114, 0), (-114, 90, 0, 0, 0), (90, -114, 0, 0, 0), (0, 0, 0, -100, -14), (-10, 0, -60, 0, -30)]
+
+
+@pytest.mark.parametrize("powers", SMALL)
+@pytest.mark.parametrize("dh", [24, 64, 96, 128])
+def test_small_numbers_keep_their_bits(dh, powers):
+    """Operands, and values between the products, a few powers of two above the smallest normal number: results have the relative error
+    of ordinary ones wherever they are well above that number themselves."""
+    shape = B, H, S, dh, E, de, Hk = 1, 2, 70, dh, 2, 64, 2
+    print(f"case d_h={dh} powers={powers}", flush=True)
+    Q, K, U, V, R, dO = make_inputs(B, H, S, dh, E, de, Hk, seed=8, dtype=torch.float32)
+    q, ku, v, r, do = (2.0 ** p for p in powers)
+    ins = (Q * q, K * ku, U * ku, V * v, R * r, dO * do)
+    checked = 0
+    for name, got, want in zip(NAMES, _run(*ins), _oracle(*ins)):
+        if want.abs().max() < 2.0 ** -117:      # (most of it would be denormal: those have fewer bits)
+            continue
+        checked += 1
+        assert _error(got, want) <= _bound(*shape), (name, _error(got, want), want.abs().max())
+    assert checked >= 3
