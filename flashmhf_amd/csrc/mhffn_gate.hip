@@ -758,8 +758,12 @@ namespace {
 
 // Tiles a wave takes.  Forward: several waves per SIMD hide the latency, so a wave only takes several tiles once there
 // are at least 8 waves per SIMD; backward: as many waves (and partial sums) as fill the chip once, but for what is left over in a
-// second round of workgroups (one of eight waves fits a compute unit): a round takes 6 us and 8.5 for each of its waves' tiles (heads of
-// 128).  12,288 tokens of 8 heads: 34.8 us in 384 workgroups of one tile per wave, 29.4 in 192 of two; of 16 heads of 6,144 35.6, 29.6.
+// second round of workgroups.  A compute unit holds one of eight waves, and one of four with more than 32 experts; with up to
+// 32 it holds two of four (LDS and registers), and those, fewer than 1,024 tiles, never need a second round.  A round is priced at
+// 6 us and 8.5 for each of its waves' tiles (heads of 128, 11 experts).
+// 12,288 tokens of 8 heads of 128: 34.1 us in 384 workgroups of eight waves and one tile per wave, 28.4 in 192 of two; of 64 24.0, 20.5;
+// 9,000 of 16 heads of 96 44.0, 33.0; 8,500 of 8 heads of 128 with 40 experts 129, 102.  Two workgroups per compute unit: 3 x 1,300 tokens of
+// 8 heads of 128 19.6 in 264 workgroups of four waves, 20.8 in 144 of two tiles per wave; of 64 15.1, 15.9.
 int tiles_per_wave(int B, int H, int S, int waves, long cap)
 {
     const long total = (long)B * H * ((S + 31) / 32);
@@ -776,7 +780,8 @@ dim3 gate_bwd_grid(const Dims& d, int& tpw)
 {
     const int nw = gate_bwd_waves(d), ntiles = (d.S + 31) / 32;
     auto workgroups = [&](int t) { return (ntiles + nw * t - 1) / (nw * t); };
-    auto rounds = [&](int t) { return ((long)d.B * d.H * workgroups(t) + CUS - 1) / CUS; };
+    const int at_once = (nw == 4 && d.E <= 32 ? 2 : 1) * CUS;
+    auto rounds = [&](int t) { return ((long)d.B * d.H * workgroups(t) + at_once - 1) / at_once; };
     tpw = tiles_per_wave(d.B, d.H, d.S, nw * CUS, 64);
     for (int t = tpw + 1; t <= 64 && rounds(t - 1) > 1 && workgroups(t - 1) > 1; ++t)
         if (rounds(t) * (6 + 8.5 * t) < rounds(tpw) * (6 + 8.5 * tpw)) tpw = t;

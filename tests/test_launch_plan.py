@@ -107,3 +107,12 @@ def test_each_kernel_matches_the_oracle(dh, dims, want):
 def test_whose_products_are_faster(product, here):
     form = {"NT": _capi.PRODUCT_NT, "NN": _capi.PRODUCT_NN, "TN": _capi.PRODUCT_TN}[product[0]]
     assert bool(_capi.lib().mhffn_product_faster(form, *product[1:])) is here
+
+
+# (B, H, S, E, workgroups): two of four waves share a compute unit, one of eight does, and one of four with more than 32 experts
+@pytest.mark.parametrize("dh", [64, 96, 128])
+@pytest.mark.parametrize("B,H,S,E,workgroups", [(3, 8, 1300, 11, 264), (3, 16, 650, 22, 288), (8, 12, 270, 8, 288), (16, 12, 150, 32, 384), (1, 6, 5392, 11, 258),
+                                                (1, 8, 4064, 11, 256), (1, 8, 12288, 11, 192), (1, 8, 4500, 40, 144)])
+def test_prologue_backward_has_no_second_round_and_no_idle_half(dh, B, H, S, E, workgroups):
+    need = _capi.lib().mhffn_gate_bwd_workspace_bytes(_capi.Dims(B, H, H, S, dh, E, 32))
+    assert need == workgroups * (dh * E + dh) * 4      # (a set of partial sums per workgroup)
