@@ -567,10 +567,14 @@ bool product_faster(int form, bool in_order, int M, int N, int K)
 
 // Both products of a backward in one launch: wherever each is taken here, and where dw is two rounds of the largest tiles, which the
 // library's product beats, but not by the launch and the idle compute units that the pair saves (two launches with the library's dw /
-// one: 512 rows of 1024 -> 8192 49.5 / 33.4, 2,048 84.6 / 81.3; of 768 -> 8192 48.7 / 33.1, 79.8 / 66.4).
+// one: 512 rows of 1024 -> 8192 48.8 / 34.5, 2,048 84.8 / 79.6; of 768 -> 8192 48.0 / 33.3, 77.0 / 66.7, 4,096 127.2 / 115.6).  Where dx
+// leaves few of them idle, or the sums of dw are long, it does (4,096 rows of 1024 -> 8192 142.4 / 147.9, of 1024 -> 5632 111.6 / 119.0; 2,048 of
+// 2048 -> 3072 64.0 / 66.1; 5,400 of 512 -> 16384 214 / 230).
 bool product_pair_faster(bool in_order, int M, int N, int K)
 {
-    return product_faster(PRODUCT_NN, in_order, M, K, N) && (product_faster(PRODUCT_TN, in_order, N, K, M) || product_tiles(PRODUCT_VARIANTS[2], N, K) <= 2 * CUS);
+    if (!product_faster(PRODUCT_NN, in_order, M, K, N)) return false;
+    if (product_faster(PRODUCT_TN, in_order, N, K, M)) return true;
+    return product_tiles(PRODUCT_VARIANTS[2], N, K) <= 2 * CUS && product_tiles(PRODUCT_VARIANTS[2], M, K) <= 3 * CUS / 4 && M <= 4096;
 }
 
 template <bool ACOLS, bool BCOLS>

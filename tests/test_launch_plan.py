@@ -116,3 +116,11 @@ def test_whose_products_are_faster(product, here):
 def test_prologue_backward_has_no_second_round_and_no_idle_half(dh, B, H, S, E, workgroups):
     need = _capi.lib().mhffn_gate_bwd_workspace_bytes(_capi.Dims(B, H, H, S, dh, E, 32))
     assert need == workgroups * (dh * E + dh) * 4      # (a set of partial sums per workgroup)
+
+
+# (y = x w^T of M x K by N x K, one launch for both gradients): both sides of the lines of that rule where dw alone is the library's
+@pytest.mark.parametrize("M,N,K,here", [(512, 8192, 1024, True), (2048, 8192, 1024, True), (3000, 8192, 1024, True), (4096, 8192, 1024, False),
+                                        (4096, 8192, 768, True), (4096, 16384, 512, True), (4104, 16384, 512, False), (2048, 3072, 2048, False),
+                                        (1500, 3072, 2048, True), (512, 8200, 1024, False), (2048, 2048, 2048, True), (8192, 512, 512, True)])
+def test_whose_pairs_are_faster(M, N, K, here):
+    assert bool(_capi.lib().mhffn_product_pair_faster(0, M, N, K)) is here
