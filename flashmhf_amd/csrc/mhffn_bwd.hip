@@ -1133,6 +1133,7 @@ static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d
 // 0.3 % on average and 4.8 % at worst over 112 calls (d_h 64, 96, 128; eight layers; 32 to 4,096 rows; up to 40 parts of either kernel).
 // Where dK, dU, dV have slices to add up, the parts go along in that launch: whole backward of 2 x 300 tokens of 8 heads of 96 on
 // two 61.7 us with a pass of their own in the price (32 rows, one part), 58.6 without (256 rows, eight parts); 900 of 8 of 128 on four 117.0, 114.6.
+// (With no room behind the slices, too, where the pass is there: the choice does not cost more than 1 % then, over 30 calls.)
 constexpr Variant DQ_VARIANTS[] = {{256, 1.7, 0.15, 1}, {32, 0.36, 0.15, 1, DQ32_A + 1}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
@@ -1140,20 +1141,27 @@ Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
                       dw_slices_bf16(d, ws_bytes) > 1 ? 0 : 2);
 }
 
+static size_t dw_slice_bytes(const Dims& d, int nslice) { return align256((size_t)nslice * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float)); }
 size_t bwd_min_workspace_bytes_bf16(const Dims& d)
 {
-    const size_t wsz = (size_t)d.Hkuv * d.E * d.d_e * d.d_h;
     const int ns = dw_slices_bf16(d, ~(size_t)0);
-    return ns > 1 ? align256((size_t)ns * 3 * wsz * sizeof(float)) : 0;
+    return ns > 1 ? dw_slice_bytes(d, ns) : 0;
 }
 
 // The parts of dQ, dR lie behind the token slices of dK, dU, dV, so that one launch can add up both.  Where they do not fit there
-// they share the workspace, and are added up before the slices are written.
+// they share the workspace, and are added up before the slices are written.  So they do where both are more than half of the memory-side
+// cache holds: the parts are still in it then right behind their kernel, and gone behind the next one (training steps in two passes / in
+// one: 84 MB 437.5 us / 435.6, 126 MB 668 / 667, 168 MB 931 / 934, 196 MB 1,094 / 1,098).
+constexpr size_t SUMS_TOGETHER_B = (size_t)128 << 20;
+static bool sums_together(const Dims& d, int nslice, int nsplit)
+{
+    return nslice > 1 && nsplit > 1 && dw_slice_bytes(d, nslice) + nsplit * dq_part_bytes(d) <= SUMS_TOGETHER_B;
+}
 size_t bwd_workspace_bytes_bf16(const Dims& d)
 {
     const int nq = dq_pick_bf16(d, ~(size_t)0, 0).nsplit;
-    const size_t dw = bwd_min_workspace_bytes_bf16(d);
-    return dw + (nq > 1 ? align256(nq * dq_part_bytes(d)) : 0);
+    const size_t dw = bwd_min_workspace_bytes_bf16(d), dq = nq > 1 ? align256(nq * dq_part_bytes(d)) : 0;
+    return sums_together(d, dw_slices_bf16(d, ~(size_t)0), nq) ? dw + dq : dw > dq ? dw : dq;
 }
 
 template <int DH>
@@ -1166,9 +1174,9 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     const int nbe = d.d_e / JB, G = d.H / d.Hkuv, nslice = dw_slices_bf16(d, ws_bytes);
     const long wsz = (long)d.Hkuv * d.E * d.d_e * d.d_h;
     const Pick pick = dq_pick_bf16(d, ws ? ws_bytes : 0, phases);
-    const size_t slices_b = align256((size_t)nslice * 3 * wsz * sizeof(float));
+    const size_t slices_b = dw_slice_bytes(d, nslice);
     constexpr int ALL = PH_BWD_DQDR | PH_BWD_DKDUDV | PH_BWD_REDUCE;
-    const bool together = (phases & ALL) == ALL && nslice > 1 && pick.nsplit > 1 && slices_b + pick.nsplit * dq_part_bytes(d) <= ws_bytes;
+    const bool together = (phases & ALL) == ALL && sums_together(d, nslice, pick.nsplit) && slices_b + pick.nsplit * dq_part_bytes(d) <= ws_bytes;
     DqArgs dq{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, (bf16_t*)dQ, dR,
               together ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + slices_b) : part, RowMap(d), Parts(d.E, nbe, pick.nsplit)};
     const unsigned qb = (unsigned)(((long)dq.rows.n * (DH / 4) + 255) / 256), rb = (unsigned)(((long)dq.rows.n * d.E + 255) / 256);
