@@ -216,8 +216,11 @@ struct Split8 {
 template <int IMM>
 __device__ __forceinline__ void lds_direct16(const float* src, unsigned char* dst)
 {
-    // (the instruction's offset counts at both ends)
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(src), "s"(lds_addr(dst) - IMM), "n"(IMM) : "memory");
+    // (the instruction's offset counts at both ends; m0, where the compiler keeps the base of its own such loads and which a clobber
+    // list cannot name, is left as it was)
+    unsigned m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0) : "v"(src), "s"(lds_addr(dst) - IMM), "n"(IMM) : "memory");
 }
 // pair I of eight values: the planes' registers I
 template <int I, class V>

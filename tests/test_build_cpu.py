@@ -143,3 +143,16 @@ def test_reads_in_flight_are_followed_over_branches(used, wait, target, found):
     """Around a loop and through a jump, forwards and backwards in the text."""
     got = build.reads_touched_in_flight(LOOP.format(used=used, wait=wait, target=target).splitlines())
     assert got == ({} if found is None else {"_Z6kernelv": found})
+
+
+def test_inline_assembly_leaves_m0_as_it_was():
+    """The compiler keeps the LDS base of its own LDS-direct loads there, and takes no clobber of it."""
+    import re
+    found = 0
+    for name in os.listdir(build.CSRC):
+        for asm in re.findall(r'\basm\b[^"]*((?:"[^"]*"\s*)+)', open(os.path.join(build.CSRC, name)).read()):
+            lines = [ln.strip(' "') for ln in re.sub(r'"\s*"', "", asm).strip().split("\\n\\t")]
+            if any(ln.startswith("s_mov_b32 m0,") for ln in lines):
+                found += 1
+                assert lines[0] == "s_mov_b32 %0, m0" and lines[-1] == "s_mov_b32 m0, %0", (name, lines)
+    assert found
