@@ -1134,7 +1134,9 @@ static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d
 // Where dK, dU, dV have slices to add up, the parts go along in that launch: whole backward of 2 x 300 tokens of 8 heads of 96 on
 // two 61.7 us with a pass of their own in the price (32 rows, one part), 58.6 without (256 rows, eight parts); 900 of 8 of 128 on four 117.0, 114.6.
 // (With no room behind the slices, too, where the pass is there: the choice does not cost more than 1 % then, over 30 calls.)
-constexpr Variant DQ_VARIANTS[] = {{256, 1.7, 0.15, 1}, {32, 0.36, 0.15, 1, DQ32_A + 1}};
+// Tiles of 256 rows that are half empty are no choice, whatever the prices of a part of one block say: 64 rows of 6 heads of 64 with 25 blocks
+// 12.1 us in 25 parts, 8.8 in 5 of 32-row tiles; 50 of 4 heads of 128 with 24 blocks 12.5, 10.5; 128 of 2 heads of 128 with 9 blocks 13.2, 8.9.
+constexpr Variant DQ_VARIANTS[] = {{256, 1.7, 0.15, 1, 0, 129}, {32, 0.36, 0.15, 1, DQ32_A + 1}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
     return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes,

@@ -655,6 +655,7 @@ struct Variant {
     double step, full;
     int unit;             // blocks of a step
     int ahead = 0;        // steps that a pipeline takes beyond those of its blocks
+    int rows_from = 0;    // rows of a head from which on it is a choice
 };
 struct Pick {
     int tile_rows, nsplit;
@@ -668,7 +669,7 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
     Pick best{variants[0].tile_rows, 1};
     double best_us = 0;
     for (const Variant& v : variants) {
-        if (v.tile_rows == 32 && !may_cut) continue;      // (the rows32 forward keeps all gate values of a tile in LDS)
+        if (v.tile_rows == 32 ? !may_cut : may_cut && rows < v.rows_from) continue;      // (the rows32 forward keeps all gate values of a tile in LDS)
         const long tiles = (rows + v.tile_rows - 1) / v.tile_rows * d.Hkuv;
         for (int ns = 1; ns <= most; ++ns) {
             if (ns > 1 && (ns * part_bytes > ws_bytes || tiles * (ns - 1) >= 2 * CUS)) break;

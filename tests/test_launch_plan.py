@@ -137,3 +137,10 @@ def test_backward_workspace_holds_both_sums_where_one_launch_adds_them(B, H, S, 
     assert slices == L.mhffn_bwd_workspace_min_bytes(d, 0)
     assert (slices + parts <= 128 << 20) is together
     assert 0 <= L.mhffn_bwd_workspace_bytes(d, 0) - (slices + parts if together else max(slices, parts)) < 256
+
+
+@pytest.mark.parametrize("dh", [64, 96, 128])
+@pytest.mark.parametrize("H,Hk,S,E,de", [(12, 6, 32, 5, 160), (16, 8, 32, 2, 160), (8, 4, 50, 8, 64), (4, 4, 50, 8, 96), (2, 2, 128, 3, 96), (1, 1, 1, 1, 32)])
+def test_dqdr_of_few_rows_has_no_half_empty_large_tiles(dh, H, Hk, S, E, de):
+    assert _capi.launch_plan(_capi.Dims(1, H, Hk, S, dh, E, de), _capi.DTYPE_BF16).dqdr_tile_rows == 32
+    assert _capi.launch_plan(_capi.Dims(1, H, Hk, S, dh, 65, 32), _capi.DTYPE_BF16).dqdr_tile_rows == 256      # (32-row tiles hold the gates of 64 experts)
