@@ -1151,10 +1151,10 @@ size_t bwd_min_workspace_bytes_bf16(const Dims& d)
 }
 
 // The parts of dQ, dR lie behind the token slices of dK, dU, dV, so that one launch can add up both.  Where they do not fit there
-// they share the workspace, and are added up before the slices are written.  So they do where both are more than half of the memory-side
+// they share the workspace, and are added up before the slices are written.  So they do where both are most of what the memory-side
 // cache holds: the parts are still in it then right behind their kernel, and gone behind the next one (training steps in two passes / in
-// one: 84 MB 437.5 us / 435.6, 126 MB 668 / 667, 168 MB 931 / 934, 196 MB 1,094 / 1,098).
-constexpr size_t SUMS_TOGETHER_B = (size_t)128 << 20;
+// one: 84 MB 437.5 us / 435.6, 126 MB 668 / 667, 155 MB 493.8 / 491.6, 168 MB 931 / 934, 196 MB 1,094 / 1,098).
+constexpr size_t SUMS_TOGETHER_B = (size_t)160 << 20;
 static bool sums_together(const Dims& d, int nslice, int nsplit)
 {
     return nslice > 1 && nsplit > 1 && dw_slice_bytes(d, nslice) + nsplit * dq_part_bytes(d) <= SUMS_TOGETHER_B;

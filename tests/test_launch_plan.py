@@ -126,8 +126,8 @@ def test_whose_pairs_are_faster(M, N, K, here):
     assert bool(_capi.lib().mhffn_product_pair_faster(0, M, N, K)) is here
 
 
-# (B, H, S, d_h, E, d_e, Hk, together): parts of dQ, dR and slices of dK, dU, dV of at most 128 MiB lie one behind the other
-@pytest.mark.parametrize("B,H,S,dh,E,de,Hk,together", [(2, 8, 300, 96, 8, 256, 2, True), (8, 8, 512, 128, 11, 352, 4, True), (3, 12, 2500, 64, 12, 256, 6, True),
+# (B, H, S, d_h, E, d_e, Hk, together): parts of dQ, dR and slices of dK, dU, dV of at most 160 MiB lie one behind the other
+@pytest.mark.parametrize("B,H,S,dh,E,de,Hk,together", [(2, 8, 300, 96, 8, 256, 2, True), (8, 8, 512, 128, 11, 352, 4, True), (3, 12, 2500, 64, 12, 256, 6, True), (1, 12, 3000, 128, 9, 384, 6, True),
                                                        (4, 12, 1902, 128, 9, 384, 6, False), (2, 12, 2750, 128, 9, 384, 6, False)])
 def test_backward_workspace_holds_both_sums_where_one_launch_adds_them(B, H, S, dh, E, de, Hk, together):
     L, d = _capi.lib(), _capi.Dims(B, H, Hk, S, dh, E, de)
@@ -135,7 +135,7 @@ def test_backward_workspace_holds_both_sums_where_one_launch_adds_them(B, H, S, 
     assert plan.dqdr_parts > 1 and plan.dkdudv_slices > 1
     slices, parts = plan.dkdudv_slices * 3 * Hk * E * de * dh * 4, plan.dqdr_parts * B * H * S * (dh + E) * 4
     assert slices == L.mhffn_bwd_workspace_min_bytes(d, 0)
-    assert (slices + parts <= 128 << 20) is together
+    assert (slices + parts <= 160 << 20) is together
     assert 0 <= L.mhffn_bwd_workspace_bytes(d, 0) - (slices + parts if together else max(slices, parts)) < 256
 
 
