@@ -132,7 +132,8 @@ EXPECTED_KERNELS = (
 )
 # Variants of those kernels for smaller problems and for float32, and the products, under the same rule.
 VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_fwd_rows32_long_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
-                   ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 1), ("dkdudv_split_kernelILi", 3),
+                   ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 2), ("dkdudv_split_kernelILi", 3),
+                   ("fwd_fp32_kernelILi", 4), ("dqdr_fp32_kernelILi", 4),
                    ("WholeRows", 18),
                    ("mhffn_product_kernel", 10), ("mhffn_product_pair_kernel", 9), ("mhffn_product_split_kernel", 2))
 # The one instantiation known to spill: head prologue backward for d_h = 128 with more than 32 experts and RMSNorm

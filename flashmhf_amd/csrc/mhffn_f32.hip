@@ -462,9 +462,9 @@ __device__ __forceinline__ bool anywhere(bool here, unsigned char* words, int wa
 {
     volatile unsigned* word = reinterpret_cast<volatile unsigned*>(words);
     const bool own = __ballot(here) != 0;
-    __syncthreads();
+    quad_barrier();      // (__syncthreads would wait for the results' stores)
     if ((threadIdx.x & 63) == 0) word[wave] = own;
-    __syncthreads();
+    quad_barrier();
     return __builtin_amdgcn_readfirstlane(word[0] | word[1] | word[2] | word[3]) != 0;
 }
 // K, U and V tiles of block b by four waves, waited for.
@@ -554,6 +554,42 @@ __device__ __forceinline__ void dqdr_fp32(const F32Args& p, const Place& w, unsi
             dr = 0.0f;
         }
     }
+}
+
+// Parts of one block: taking operands apart, a second team and the longer way to the results do not pay there.  Forward of 64 rows of 4
+// heads of 96 in 64 parts 22.5 us, 27.6 with the kernels below; of 32 rows of 4 heads of 64 in 16 parts 10.2, 13.2; of one block of 8 x 8 4.8,
+// 6.9.  dQ/dR: level for d_h > 64, 4 % less time for 64, 7 % below.  From two blocks on the kernels below are level (forward, 266 calls,
+// 0.98 on average) or faster (dQ/dR, 0.86).
+template <int CT>
+__global__ __launch_bounds__(256, 2) void fwd_fp32_kernel(F32Args p)
+{
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const Place w(p, wave, lane & 31);
+    f32x16 o[CT];
+    fwd_fp32<CT>(p, w, lds, wave, o);
+    if (w.valid)
+        store_row<CT>(o, p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * p.DH
+                                            : p.O + p.rows.tok(w.hk, w.row) * p.DH, lane >> 5, p.DH);
+}
+// Where a part leaves the sums of dR of this lane's row.
+__device__ __forceinline__ float* dr_row(const F32Args& p, const Place& w)
+{
+    const long hrows = (long)p.rows.Hkuv * p.rows.n;
+    return p.parts.nsplit > 1 ? p.part + p.parts.nsplit * hrows * p.DH + (w.z * hrows + (long)w.hk * p.rows.n + w.row) * p.parts.E
+                              : p.dR + p.rows.gate(w.hk, w.row) * p.parts.E;
+}
+template <int CT>
+__global__ __launch_bounds__(256, CT > 3 ? 1 : 2) void dqdr_fp32_kernel(F32Args p)
+{
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const Place w(p, wave, lane & 31);
+    f32x16 dq[CT];
+    dqdr_fp32<CT>(p, w, lds, wave, dr_row(p, w), w.valid, dq);
+    if (w.valid)
+        store_row<CT>(dq, p.parts.nsplit > 1 ? p.part + (((long)w.z * p.rows.Hkuv + w.hk) * p.rows.n + w.row) * p.DH
+                                             : p.dQ + p.rows.tok(w.hk, w.row) * p.DH, lane >> 5, p.DH);
 }
 
 // Forward: 128 rows, GROUPS teams of four waves that take the blocks of the part in turn, their sums added at the end.  A team's
@@ -698,9 +734,7 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
             for (int x = 0; x < 3; ++x) asm volatile("" : "+a"(q[ks].p[x]), "+a"(go[ks].p[x]));
     }
     const float* rrow = p.R + p.rows.gate(w.hk, w.row) * E;
-    const long hrows = (long)p.rows.Hkuv * p.rows.n;
-    float* drow = p.parts.nsplit > 1 ? p.part + p.parts.nsplit * hrows * DH + (w.z * hrows + (long)w.hk * p.rows.n + w.row) * E
-                                     : p.dR + p.rows.gate(w.hk, w.row) * E;
+    float* drow = dr_row(p, w);
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
@@ -1171,13 +1205,15 @@ template <int CT>
 hipError_t launch_fwd_f32_t(const F32Args& a, const Dims& d, hipStream_t st)
 {
     constexpr int GROUPS = CT > 3 ? 1 : 2;
-    const int smem = GROUPS * 3 * PLANES_B;
+    const bool one_block = a.parts.nsplit == a.parts.E * a.parts.nbe;
+    const int smem = one_block ? 3 * Tile<CT>::BYTES : GROUPS * 3 * PLANES_B;
     static_assert(GROUPS == 1 || 4 * CT * 16 * 64 * 4 <= GROUPS * 3 * PLANES_B, "the teams' exchange fits the planes");
-    static LdsOptIn optin;
-    const hipError_t e = ensure_dynamic_lds(optin, (const void*)fwd_f32_kernel<CT, GROUPS>, smem);
+    static LdsOptIn optin[2];
+    auto* fn = one_block ? fwd_fp32_kernel<CT> : fwd_f32_kernel<CT, GROUPS>;
+    const hipError_t e = ensure_dynamic_lds(optin[one_block], (const void*)fn, smem);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fwd_f32_kernel<CT, GROUPS>), dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit),
-                       dim3(256 * GROUPS), smem, st, a);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit), dim3(one_block ? 256 : 256 * GROUPS),
+                       smem, st, a);
     if (a.parts.nsplit > 1) {
         const unsigned rb = (unsigned)(((long)a.rows.n * (d.d_h / 4) + 255) / 256);
         hipLaunchKernelGGL(sum_f32_kernel, dim3(rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, a.O, rb);
@@ -1190,11 +1226,13 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
 {
     hipError_t err = hipSuccess;
     if (phases & PH_BWD_DQDR) {
-        const int smem = 6 * PLANES_B;
-        static LdsOptIn optin;
-        err = ensure_dynamic_lds(optin, (const void*)dqdr_f32_kernel<CT>, smem);
+        const bool one_block = a.parts.nsplit == a.parts.E * a.parts.nbe;
+        const int smem = one_block ? 3 * Tile<CT>::BYTES : 6 * PLANES_B;
+        static LdsOptIn optin[2];
+        auto* fn = one_block ? dqdr_fp32_kernel<CT> : dqdr_f32_kernel<CT>;
+        err = ensure_dynamic_lds(optin[one_block], (const void*)fn, smem);
         if (err != hipSuccess) return err;
-        hipLaunchKernelGGL(dqdr_f32_kernel<CT>, dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit),
+        hipLaunchKernelGGL(fn, dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit),
                            dim3(256), smem, st, a);
         if (a.parts.nsplit > 1) {
             const unsigned rb = (unsigned)(((long)a.rows.n * (d.d_h / 4) + 255) / 256);
@@ -1206,19 +1244,15 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
     }
     if (phases & PH_BWD_DKDUDV) {
         const dim3 grid((unsigned)((d.E * nbe_of(d) + 1) / 2), (unsigned)d.Hkuv, (unsigned)a.nslice);
-        void (*kernel)(F32Args);
-        int smem;
-        if constexpr (CT <= 3) {
-            kernel = dkdudv_split_kernel<CT>;
-            smem = 4 * PLANES_B + 16 * CT * 1024 + 4 * 32 * (int)sizeof(float);
-            static_assert(2 * 3 * CT * 16 * 64 * 4 <= 4 * PLANES_B, "the waves' exchange fits the planes");
-        } else {
-            kernel = dkdudv_f32_kernel<CT>;
-            smem = 8 * Tile<CT>::BYTES + 2 * 4 * 32 * (int)sizeof(float);
-            static_assert(2 * 3 * CT * 16 * 64 * 4 <= 8 * Tile<CT>::BYTES, "the waves' exchange fits the tile stages");
-        }
-        static LdsOptIn optin;
-        err = ensure_dynamic_lds(optin, (const void*)kernel, smem);
+        // on the fp32 instructions: d_h > 96, and one step of d_h <= 32 (7.8 of 8.2 us; of d_h 33 to 96 5 % more, two steps 8 to 20 %)
+        constexpr bool EVER = CT == 1 || CT > 3, ALWAYS = CT > 3;
+        const bool plain = ALWAYS || (EVER && (a.rows.n + 31) / 32 <= 2 * a.nslice);
+        auto* kernel = plain ? dkdudv_f32_kernel<EVER ? CT : 1> : dkdudv_split_kernel<ALWAYS ? 1 : CT>;
+        const int smem = plain ? 8 * Tile<CT>::BYTES + 2 * 4 * 32 * (int)sizeof(float) : 4 * PLANES_B + 16 * CT * 1024 + 4 * 32 * (int)sizeof(float);
+        static_assert(!EVER || 2 * 3 * CT * 16 * 64 * 4 <= 8 * Tile<CT>::BYTES, "the waves' exchange fits the tile stages");
+        static_assert(ALWAYS || 2 * 3 * CT * 16 * 64 * 4 <= 4 * PLANES_B, "the waves' exchange fits the planes");
+        static LdsOptIn optin[2];
+        err = ensure_dynamic_lds(optin[plain], (const void*)kernel, smem);
         if (err != hipSuccess) return err;
         hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, a);
         err = hipGetLastError();

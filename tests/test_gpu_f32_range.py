@@ -155,3 +155,21 @@ def test_small_numbers_keep_their_bits(dh, powers):
         checked += 1
         assert _error(got, want) <= _bound(*shape), (name, _error(got, want), want.abs().max())
     assert checked >= 3
+
+
+# (B, H, S, d_h, E, d_e, Hk, parts of one block): such parts run on the fp32 instructions, and dK, dU, dV of d_h <= 32 with one step a slice
+@pytest.mark.parametrize("B,H,S,dh,E,de,Hk,one", [(1, 1, 1, 8, 1, 8, 1, True), (1, 2, 129, 32, 1, 33, 2, True), (1, 8, 63, 96, 8, 256, 4, True), (2, 4, 16, 64, 4, 120, 4, True),
+                                                  (1, 1, 65, 128, 2, 32, 1, True), (1, 8, 65, 96, 8, 256, 8, False), (1, 2, 700, 24, 3, 70, 1, True), (1, 1, 66, 16, 1, 32, 1, True)])
+def test_parts_of_one_block_and_of_more(B, H, S, dh, E, de, Hk, one):
+    from flashmhf_amd import _capi
+    print("case", B, H, S, dh, E, de, Hk, flush=True)
+    plan = _capi.launch_plan(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_F32)
+    assert (plan.fwd_parts == E * ((de + 31) // 32)) is one and (plan.dqdr_parts == plan.fwd_parts or not one)
+    ins = make_inputs(B, H, S, dh, E, de, Hk, seed=S, dtype=torch.float32)
+    bound = 2.0 ** -24 * (math.sqrt((dh + max(E * (de + 31), H // Hk * B * S + 31)) / 2) + 8)      # (_bound, with one rounding per two terms)
+    for name, got, want in zip(NAMES, _run(*ins), _oracle(*ins)):
+        assert _error(got, want) <= bound, (name, _error(got, want))
+    ins[3][0, 0, 3, dh - 2] = float("inf")      # (of d_h that is no multiple of 32 the first four columns stand in for those beyond it, times zero)
+    for name, got, want in zip(NAMES, _run(*ins), _eager(*ins)):
+        if name in ("O", "dQ", "dR"):           # (the rows that a tile lacks are others times zero in dK, dU, dV)
+            _same_with_infinities(name, got, want)
