@@ -804,8 +804,11 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
         const size_t smem = gate_fwd_smem(DH, NT);
         // whole rows from six tiles per compute unit on (us in pieces / whole: 1,024 tiles of 8 heads of 128 7.5 / 7.8, 1,536 9.6 / 9.2, 2,048
         // 11.4 / 10.3; of 96 6.5 / 6.7, 8.6 / 8.4 with 2,048; of 64 6.5 / 6.4 with 2,048)
-        const bool whole = (long)a.B * a.H * ((a.S + 31) / 32) >= 6 * CUS;
-        auto* fn = whole ? mhffn_gate_fwd_kernel<DH, NT, NORM, WholeRows> : mhffn_gate_fwd_kernel<DH, NT, NORM>;
+        // Not with more than 32 experts, whose arithmetic hides the pieces (4,096 tiles of 4 heads of 64 with 40 16.3 / 17.4, of 8 of 128 25.2 / 26.0),
+        // nor with 32 or, below d_h 128, 16: their rows of R share LDS banks, and the way through LDS waits for their writes (16,384 tiles of
+        // 12 heads of 128 with 32 + 9 %, of 96 + 9 %; 12,288 of 96 with 16 35.3 / 36.0).
+        const bool whole = NT == 1 && (a.E % 16 != 0 || (DH == 128 && a.E == 16)) && (long)a.B * a.H * ((a.S + 31) / 32) >= 6 * CUS;
+        auto* fn = whole ? mhffn_gate_fwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_fwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_fwd[whole], (const void*)fn, (int)smem);
         if (e != hipSuccess) return e;
         a.tpw = tiles_per_wave(a.B, a.H, a.S, 8192, 16);

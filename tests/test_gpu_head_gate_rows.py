@@ -30,6 +30,13 @@ def test_forward(B, S, H, dh, E, norm):
             assert torch.equal(Q[b, :, t:t + 500], q[0]) and torch.equal(R[b, :, t:t + 500], r[0])
 
 
+# (32 and more experts, and 16 for heads below 128, stay with pieces: the cases above with 32 and 40)
+@pytest.mark.parametrize("B,S,H,dh,E,norm", [(4, 3072, 4, 64, 31, True), (1, 3041, 16, 96, 17, True), (2, 3050, 8, 128, 16, True), (1, 6200, 8, 64, 8, False),
+                                             (1, 3041, 16, 96, 16, True)])
+def test_forward_around_the_experts_of_that_rule(B, S, H, dh, E, norm):
+    test_forward(B, S, H, dh, E, norm)
+
+
 # 8,192 tiles: four of them per wave, dx whole; 3,104 and 2,080: two per wave instead of a second round of workgroups
 @pytest.mark.parametrize("B,S,H,dh,E,norm", [(1, 16353, 16, 128, 22, True), (2, 16384, 8, 96, 8, True), (1, 32767, 8, 64, 17, True),
                                              (1, 16360, 16, 128, 11, False), (1, 12390, 8, 128, 11, True), (5, 3300, 4, 64, 8, True)])
