@@ -130,7 +130,8 @@ EXPECTED_KERNELS = (
     ("mhffn_fwd_kernel", 3), ("mhffn_bwd_dqdr_kernel", 3), ("mhffn_bwd_dkdudv_kernel", 6),
     ("mhffn_gate_fwd_kernel", 12), ("mhffn_gate_bwd_kernel", 12),
 )
-# Variants of those kernels for smaller problems and for float32, and the products, under the same rule.
+# Variants of those kernels for smaller problems and for float32, and the products, under the same rule.  (The prologue's kernels that move
+# whole rows are told by the mode, a type, that their names end in, and are not counted among the instantiations above.)
 VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_fwd_rows32_long_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
                    ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 2), ("dkdudv_split_kernelILi", 3),
                    ("fwd_fp32_kernelILi", 4), ("dqdr_fp32_kernelILi", 4),

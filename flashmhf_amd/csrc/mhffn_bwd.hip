@@ -1130,7 +1130,9 @@ static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d
 // Tiles of 256 rows where they fill the chip, of 32 below that: a block of theirs takes a quarter of the time, with an eighth of
 // the rows.  One part of 121 blocks of the 370M heads, 512 rows: 199 us with 256 rows, 48 with 32; 2,048 rows: 200 and (two
 // rounds) 108.  At their best numbers of parts 512 rows take 34.5 us with 32 rows, 36.1 with 256, 733 rows 49.7 and 45.0.  The prices lose
-// 0.3 % on average and 4.8 % at worst over 112 calls (d_h 64, 96, 128; eight layers; 32 to 4,096 rows; up to 40 parts of either kernel).
+// 0.6 % on average and 19 % at worst over 112 calls (d_h 64, 96, 128; eight layers; 32 to 4,096 tokens; profiles/pick_parts_sweep.csv: the kernel and
+// a summing pass of its own; in the backward that of 60 of them goes along with another), 2.2 % over 156 of twelve small layers (4 to 26
+// blocks; 1 to 600 tokens).
 // Where dK, dU, dV have slices to add up, the parts go along in that launch: whole backward of 2 x 300 tokens of 8 heads of 96 on
 // two 61.7 us with a pass of their own in the price (32 rows, one part), 58.6 without (256 rows, eight parts); 900 of 8 of 128 on four 117.0, 114.6.
 // (With no room behind the slices, too, where the pass is there: the choice does not cost more than 1 % then, over 30 calls.)

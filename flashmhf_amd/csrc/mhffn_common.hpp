@@ -643,9 +643,10 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 // rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing pass (dQ/dR: none where
 // the weights' gradients have one, which adds up both) + 0.6 per MB of sums; a step slows by up to `full` as the chip fills
 // (power).  The prices are those of d_h = 128 for every d_h: with it the
-// variants of a kernel get cheaper nearly together.  Against every tile height and 1 to 64 parts, measured on 168 bfloat16 calls of the
-// forward (d_h 64, 96, 128; four layers; 1 to 12,000 rows; profiles/pick_parts_sweep.csv) the pick is 1.3 % slower than
-// the fastest on average and 23 % at worst (4,096 rows of 8 heads of 64, 45.8 us against 37.3); dQ/dR: at its variants.
+// variants of a kernel get cheaper nearly together, and that of the 32-row forward is its trips' for its pipeline, too.  Against every
+// tile height and 1 to 64 parts, measured on 168 bfloat16 calls of the forward (d_h 64, 96, 128; four layers; 1 to 12,000 rows;
+// profiles/pick_parts_sweep.csv) the pick is 1.5 % slower than the fastest on average and 24 % at worst (4,096 rows of 8 heads of 64, 46.5 us
+// against 37.5); dQ/dR: at its variants.
 // Not cut: more experts than one LDS window of gate values holds (bfloat16); and 16,384 rows per head or more, where a head
 // fills a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X

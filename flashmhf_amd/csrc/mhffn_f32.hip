@@ -1,13 +1,14 @@
-// fp32 instantiation of the fused multi-head FFN (forward, dQ/dR, dK/dU/dV): operands, products and sums are float32 and the
-// sigmoid is exact, so results track an fp32 eager evaluation to ~1e-6.  Same fusion as the bf16 kernels -- the
+// fp32 instantiation of the fused multi-head FFN (forward, dQ/dR, dK/dU/dV): operands, sums and everything between the products are
+// float32, products are off by 2^-24 at most and the sigmoid by a rounding or two, so results track an fp32 eager evaluation to
+// ~1e-6.  Same fusion as the bf16 kernels -- the
 // [tokens, E*d_e] intermediate exists only in registers.  Generic in d_h (multiple of 8, at most 128; CT = 32-column tiles of
 // it), d_e and E.
 // Formulas: models/flashmhf/modeling_mhffnmoe.py:418-427 (forward), kernels/triton/flash_mlp_moe.py:401-414, 527-542,
 // 720-729 (backward).
 //
 // The products run on v_mfma_f32_32x32x16_bf16 with every operand taken apart into three bfloat16 values ("planes", below);
-// operand layouts are those of mhffn_common.hpp.  dK/dU/dV for d_h > 96, whose planes do not fit a wave's registers, keeps
-// v_mfma_f32_32x32x2_f32, D = A(32x2) * B(2x32) + C, 64 cycles each:
+// operand layouts are those of mhffn_common.hpp.  dK/dU/dV for d_h > 96, whose planes do not fit a wave's registers, parts of one
+// block and rows whose results are not finite run on v_mfma_f32_32x32x2_f32, D = A(32x2) * B(2x32) + C, 64 cycles each:
 //       A: lane l holds row (l % 32), k = l / 32         B: lane l holds col (l % 32), k = l / 32
 //       C/D: lane l holds col (l % 32), register i holds row 8*(i/4) + 4*(l/32) + (i%4)
 // * First products contract over the head dim.  The order of the k index is free as long as A and B agree: with lane group
@@ -19,8 +20,9 @@
 // What bounds them.  256 tokens of the 128M layer took 30 (forward), 45 (dQ/dR) and 61 us (dK/dU/dV) on the fp32 matrix
 // instructions, whose time a kernel's four waves could not go below (15, 26 and 31 us, 153 TFLOP/s over the chip) and under which
 // they issue next to nothing else.  The planes take 2.7 times less matrix time and some VALU instructions per operand and
-// element, put between the matrix instructions where registers allow: 24, 34 and 47 us; per 32 rows of weights (forward, dQ/dR;
-// 128 rows) 5.2 -> 2.2 and 8.2 -> 4.2 us, per 32 tokens (dK/dU/dV, two tiles) 11.2 -> 6.6, the rest is prologue and epilogue.
+// element, put between the matrix instructions where registers allow: 25, 34 and 46 us; per 32 rows of weights (forward, dQ/dR;
+// 128 rows, a part of 64 in one) 5.2 -> 2.3 and 8.2 -> 4.0 us, per 32 tokens (dK/dU/dV, two tiles) 11.2 -> 6.6, the rest is prologue
+// and epilogue.
 #include "mhffn_common.hpp"
 
 namespace mhffn {
@@ -1181,7 +1183,9 @@ __global__ __launch_bounds__(256) void reduce_f32_kernel(const float* __restrict
     }
 }
 
-// Parts of the blocks for the forward and dQ/dR as for bfloat16 (pick_parts).
+// Parts of the blocks for the forward and dQ/dR as for bfloat16 (pick_parts).  A block took 5 us on the fp32 instructions and takes half of it;
+// the choice does not depend on it: with any step from 2 to 5 us it loses 1.7 to 2.1 (forward) and 1.2 to 2.1 % (dQ/dR) to the best number
+// of parts, 28 and 20 % at worst, over 165 calls (twelve layers of d_h 8 to 128; 1 to 1,500 tokens).
 constexpr Variant F32_VARIANTS[] = {{128, 5.0, 0.0, 1}};
 int nbe_of(const Dims& d) { return (d.d_e + JB - 1) / JB; }
 size_t o_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }

@@ -753,8 +753,10 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // number of parts: one token of the 370M layer 7.8 us against 10.0, 16 tokens of the 1.3B layer 20.3 against 22.5 (95 MB of
 // weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.  (Priced at 0.6 for 128 rows, as
 // before its filling waves: the line between the two kernels lies where it did.)
-// A part of FWDL_FROM blocks or more goes through the pipeline: 15 or 16 blocks a part 14.4 -> 14.0 us (100 rows of the 370M heads) and
-// 19.7 -> 20.4 (16 of the 1.3B heads), 4 blocks 7.6 -> 8.0, 64 blocks as above.
+// A part of FWDL_FROM blocks or more goes through the pipeline.  Trips / pipeline, us in one part, 512 rows of 8 heads of 128: 4 blocks 6.1 / 6.6,
+// 12 9.0 / 8.9, 20 11.7 / 11.1, 28 14.5 / 13.3, 32 15.9 / 14.5, 64 27.1 / 23.9; of 96: 16 blocks 9.3 / 9.4, 24 11.6 / 11.4, 32 13.7 / 13.3, 64 23.7 / 22.0;
+// of 64: 16 8.6 / 8.7, 24 10.8 / 10.6, 32 12.9 / 12.7, 64 21.8 / 20.6.  (They meet at 12 to 20 blocks; the line above that is a cautious one, drawn
+// when 16 and 64 were measured.)
 constexpr int FWDL_FROM = 32;
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1}, {128, 0.6, 0.33, 1}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }

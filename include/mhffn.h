@@ -61,7 +61,11 @@ typedef struct mhffn_dims {
 const char* mhffn_strerror(int code);
 
 /* 1 if kernels exist for (d_h, d_e, dtype), else 0.  bf16 (MFMA kernels): d_h in {64, 96, 128}, d_e % 32 == 0, any E.
- * float32 (correctness instantiation, fp32 matrix instructions): d_h a multiple of 8 up to 128, any d_e, any E.
+ * float32 (correctness instantiation): d_h a multiple of 8 up to 128, any d_e, any E.  Its products run on bfloat16 matrix instructions,
+ * every operand as a sum of three bfloat16 values, with at most 2^-24 of a product left out; every finite float32 counts with all its
+ * bits.  A token's row of O or of dQ and dR, or a row of dK, dU, dV, in which a value is not finite on that way -- operands that hold
+ * infinities or NaN; products beyond 2^79, results beyond 2^55 -- is computed again on fp32 matrix instructions, so that it has the
+ * infinities of float32 arithmetic; such calls take up to twice the time.
  * Replaces the reference's shape gates (flash_mlp_moe.py:758, flash_ffn_moe.cu:956-958, 1037). */
 int mhffn_is_supported(int d_h, int d_e, int dtype);
 
@@ -73,10 +77,12 @@ int mhffn_check_dims(const mhffn_dims* dims, int dtype);
  * themselves (e.g. the 370M and 1.3B layers at their benchmark sizes); `workspace` may then be NULL.
  *   - forward: the bytes are those of the fp32 partial sums with which a small number of tokens is computed fastest.  Any
  *     smaller workspace, NULL included, is accepted: the same result (up to fp32 summation order), with less of the GPU busy.
- *   - backward: the bytes are the larger of the partial sums of dQ, dR (few tokens, as in the forward) and those of dK, dU, dV
- *     (token slices).  The second are required and what mhffn_bwd_workspace_min_bytes reports; between the two sizes dQ and dR
- *     are computed with less of the GPU busy, to the same result up to fp32 summation order.  A smaller workspace returns
- *     MHFFN_ERR_WORKSPACE. */
+ *   - backward: the bytes are those of the partial sums of dQ, dR (few tokens, as in the forward) and of dK, dU, dV (token slices):
+ *     in bfloat16 the sum of both up to 160 MiB, so that one launch adds them all up, beyond that and in float32 the larger.
+ *     Those of dK, dU, dV are required and what mhffn_bwd_workspace_min_bytes reports.  With less than the whole the two share the
+ *     bytes and are added up in two launches, to the same bits as long as dQ's and dR's fit by themselves; with less than
+ *     that dQ and dR are computed with less of the GPU busy, to the same result up to fp32 summation order.  A workspace
+ *     below the required one returns MHFFN_ERR_WORKSPACE. */
 size_t mhffn_fwd_workspace_bytes(const mhffn_dims* dims, int dtype);
 size_t mhffn_bwd_workspace_bytes(const mhffn_dims* dims, int dtype);
 size_t mhffn_bwd_workspace_min_bytes(const mhffn_dims* dims, int dtype);
@@ -107,7 +113,8 @@ int mhffn_bwd(const void* Q, const void* K, const void* U, const void* V, const 
  * events on the launch stream; the reference has no counterpart (its kernels are launched one per Python call,
  * flash_mlp_moe.py:832-866).  A mask with a bit outside MHFFN_FWD_ALL / MHFFN_BWD_ALL returns MHFFN_ERR_SHAPE (the bit
  * values are not stable across versions of this header: pass the names, not numbers).  MHFFN_BWD_REDUCE alone needs the last
- * call on the workspace to have run MHFFN_BWD_DKDUDV: the kernels of MHFFN_BWD_DQDR use the same bytes. */
+ * call on the workspace to have run MHFFN_BWD_DKDUDV: the kernels of MHFFN_BWD_DQDR, called without it, use the same bytes.
+ * MHFFN_BWD_DQDR without the others adds up its own partial sums; a full call may leave that to MHFFN_BWD_REDUCE's launch. */
 enum {
     MHFFN_FWD_MAIN = 1, MHFFN_FWD_ALL = 1,
     MHFFN_BWD_DQDR = 1, MHFFN_BWD_DKDUDV = 2, MHFFN_BWD_REDUCE = 4, MHFFN_BWD_ALL = 7,
