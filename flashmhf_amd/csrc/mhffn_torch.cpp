@@ -515,12 +515,14 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
             return {need_in ? product_nn(d, w, whose) : Tensor(), need_w ? product_tn(d, in, whose) : Tensor()};
         };
         const bool need_w2 = asked(after_nw + 4, after_nw + 5);
-        Tensor dO, O4 = s[13];
-        if (need_w2 && at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
-            O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose);
-        std::tie(dO, dw2) = both(prologue || experts, need_w2, dY, w2, O4.reshape({-1, hid}));
-        if (prologue || experts)
-            g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.view(s[13].sizes()).transpose(1, 2), K.scalar_type(), one_part);
+        {
+            Tensor dO, O4 = s[13];      // (dO goes with this scope: the prologue's gradients take its place)
+            if (need_w2 && at::GradMode::is_enabled())      // create_graph: dw2 is a function of O, as a linear layer's own backward has it
+                O4 = stepwise_O4(x, w1, nw, router, K, U, V, eps, one_part, whose);
+            std::tie(dO, dw2) = both(prologue || experts, need_w2, dY, w2, O4.reshape({-1, hid}));
+            if (prologue || experts)
+                g = op_backward(q4.transpose(1, 2), K, U, V, R, dO.view(s[13].sizes()).transpose(1, 2), K.scalar_type(), one_part);
+        }
         if (prologue) {
             h = gate_backward(x4, nw, router, wn, wr, eps, g[0], g[4]);
             std::tie(dx, dw1) = both(ctx->needs_input_grad(0), ctx->needs_input_grad(1), h[0].view({-1, hid}), w1, x.reshape({-1, hid}));
