@@ -587,40 +587,59 @@ struct DwArgs {
 constexpr int DW_NST = 4;                              // LDS stages of the token-tile ring
 constexpr int DW_RTILE_B = 1024;                       // staged gate values: [4 waves][64 lanes] fp32 (each wave: its expert)
 constexpr int DW_STAGE_B = 2 * TILE_B + DW_RTILE_B;    // Q tile | dO tile | gate values
+constexpr int DW_PAIR_STAGE_B = 2 * TILE_B + DW_RTILE_B / 2;
 
-template <int DH, bool TAIL>
+// With TokenHalves (PAIR): two blocks of rows a workgroup, and two waves for each of them: waves 0 and 1 take the first half of the slice's tokens, waves
+// 2 and 3 the second, through a ring of their own, and a block's sums meet in LDS at the end.  Twice the workgroups with half the
+// token tiles each, where the other form leaves compute units idle or takes twice the slices, every one of which is a set of float32
+// sums in memory.  (Four waves on one block would need four rings, 264 KB.)
+struct TokenHalves {};
+template <int DH, bool TAIL, class... Mode>
 __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
 {
+    constexpr bool PAIR = sizeof...(Mode) > 0;
     constexpr int KS = DH / 16, CT = DH / 32;
     constexpr int NCHUNK = DH / 8;                    // 16-byte chunks per token row
+    constexpr int NB = PAIR ? 2 : 4;                  // blocks of the workgroup; waves of a ring
+    constexpr int STAGE_B = PAIR ? DW_PAIR_STAGE_B : DW_STAGE_B, RING_B = DW_NST * STAGE_B;
+    constexpr int FILLS = 8 / NB;                     // a wave's fill instructions per tile
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hk = blockIdx.x, z = blockIdx.z;   // head index fastest: all columns of a head run on one XCD and share its L2
     const int nblk = p.E * p.nbe;
-    const int jblk = blockIdx.y * 4 + wave;
+    const int half = PAIR ? wave >> 1 : 0, wv = PAIR ? wave & 1 : wave;      // which ring, and which block of the workgroup
+    unsigned char* ring = smem_raw + half * RING_B;
+    const int jblk = blockIdx.y * NB + wv;
     const bool active = jblk < nblk;
     const int jb_c = active ? jblk : nblk - 1;        // waves of the last column without a block: addresses stay valid
     const int e_w = jb_c / p.nbe;
     const long wrow = ((long)hk * nblk + jb_c) * JB + l32;      // this lane's row of K/U/V (column j of the products)
 
-    float* sZero = reinterpret_cast<float*>(smem_raw + DW_NST * DW_STAGE_B);   // 32 zero gate values
+    float* sZero = reinterpret_cast<float*>(smem_raw + (PAIR ? 2 : 1) * RING_B);   // 32 zero gate values
     if (tid < 32) sZero[tid] = 0.0f;
     // The first step contracts a tile that does not exist (zero gate values) out of the last stage, which no load has
     // filled yet: clear its Q and dO tiles, or whatever bit patterns the previous kernel left there (possibly NaN or
     // Inf as bf16) would be multiplied by those zeros.
     {
         u32x4 z = {0u, 0u, 0u, 0u};
-        u32x4* last_stage = reinterpret_cast<u32x4*>(smem_raw + (DW_NST - 1) * DW_STAGE_B);
-        for (int i = tid; i < 2 * TILE_B / 16; i += 256) last_stage[i] = z;
+        u32x4* last_stage = reinterpret_cast<u32x4*>(ring + (DW_NST - 1) * STAGE_B);
+        for (int i = tid & (64 * NB - 1); i < 2 * TILE_B / 16; i += 64 * NB) last_stage[i] = z;
     }
     // These clears are ordinary LDS stores that other waves read in step 0, and the barriers of the token loop are bare
     // (no wait on this wave's own LDS stores): one fenced barrier here publishes them, once per workgroup.
     __syncthreads();
     const int nS = (p.S + 31) / 32;
     const int ntile = p.G * p.B * nS;
-    const int t_begin = (int)((long)ntile * z / p.nslice), t_end = (int)((long)ntile * (z + 1) / p.nslice);
+    int t_begin = (int)((long)ntile * z / p.nslice), t_end = (int)((long)ntile * (z + 1) / p.nslice);
+    bool one_less = false;                            // the other waves have a tile, and a barrier, more
+    if constexpr (PAIR) {                             // (the launcher gives every slice two tiles or more)
+        const int mid = t_begin + (t_end - t_begin + 1) / 2;
+        one_less = half && t_end - mid < mid - t_begin;
+        if (half) t_begin = mid;
+        else t_end = mid;
+    }
     const int nt = t_end - t_begin;
 
     // Tile cursor of the prefetcher: tile index -> (q-head of the group, batch, 32-token tile).  It is kept as a running
@@ -639,11 +658,12 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     const int dqrow_s = p.H * p.S - (nS - 1) * 32 * qs;
     const int dqrow_b = (p.tokmaj ? 1 : p.S) - (p.B - 1) * p.H * p.S - (nS - 1) * 32 * qs;
 
-    // per-lane constants of the tile fill: this wave's two 4-row groups of the Q/dO tiles (swizzled source chunk)
+    // per-lane constants of the tile fill: this wave's two 4-row groups of the Q/dO tiles (swizzled source chunk); of the four of PAIR
+    // the first two, the others being 16 rows on, where the swizzle comes round
     int fill_row[2], fill_coff[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        const int ins = wave + 4 * k;
+        const int ins = wv + NB * k;
         const int r = 4 * ins + (lane >> 4);
         int c = (lane & 15) ^ swz16(r);
         c = c < NCHUNK ? c : 0;                       // unused chunk positions of narrow rows load a dummy chunk
@@ -680,26 +700,27 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     };
     auto fire_tile = [&](int sidx) -> int {
         const int last = nx_last;
-        unsigned char* sbase = smem_raw + sidx * DW_STAGE_B;
+        unsigned char* sbase = ring + sidx * STAGE_B;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int row = TAIL ? (fill_row[k] < last ? fill_row[k] : last) : fill_row[k];
-            const unsigned off = (unsigned)(row * qs * (DH * 2) + fill_coff[k]);
-            const int ins = wave + 4 * k;
+        for (int k = 0; k < FILLS; ++k) {
+            const int on = 16 * (k >> 1), r = fill_row[k & 1] + (TAIL ? on : 0);
+            const int row = TAIL ? (r < last ? r : last) : r;
+            const unsigned off = (unsigned)(row * qs * (DH * 2) + fill_coff[k & 1]) + (TAIL ? 0u : (unsigned)(on * qs * (DH * 2)));
+            const int ins = wv + NB * k;
             __builtin_amdgcn_global_load_lds((gptr_t)(nx_qb + off), (lptr_t)(sbase + ins * 1024), 16, 0, 0);
             __builtin_amdgcn_global_load_lds((gptr_t)(nx_gb + off), (lptr_t)(sbase + TILE_B + ins * 1024), 16, 0, 0);
         }
         // gate values of this wave's expert for the 32 token rows (lanes 32..63 repeat them): one 4-byte element per lane
         const int trow = TAIL ? (l32 < last ? l32 : last) : l32;
         __builtin_amdgcn_global_load_lds((gptr_t)(nx_rbp + (unsigned)((trow * p.E + e_w) * 4)),
-                                         (lptr_t)(sbase + 2 * TILE_B + wave * 256), 4, 0, 0);
+                                         (lptr_t)(sbase + 2 * TILE_B + wv * 256), 4, 0, 0);
         return last + 1;
     };
     // Called by every wave after its own loads of stage `sidx` have landed and before the barrier that publishes
     // the stage: zeroes the gate values of the rows a tail tile does not have.
     auto zero_tail = [&](int sidx, int nvalid) {
-        float* sR = reinterpret_cast<float*>(smem_raw + sidx * DW_STAGE_B + 2 * TILE_B);
-        if (l32 >= nvalid) sR[wave * 64 + lane] = 0.0f;
+        float* sR = reinterpret_cast<float*>(ring + sidx * STAGE_B + 2 * TILE_B);
+        if (l32 >= nvalid) sR[wv * 64 + lane] = 0.0f;
     };
 
     // First two tiles of the slice; the third is fired behind the first barrier of the loop.
@@ -728,7 +749,9 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
             }
         }
         wait_vmcnt<0>();
+        if (PAIR && one_less) __builtin_amdgcn_s_barrier();
         __syncthreads();   // the barrier the working waves pass before their epilogue reuses the ring
+        if constexpr (PAIR) __syncthreads();      // ... and the one between its halves
         return;
     }
 
@@ -749,10 +772,16 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
         for (int x = 0; x < 16; ++x) { dk[i][x] = 0.0f; du[i][x] = 0.0f; dv[i][x] = 0.0f; }
 
     const int fr = swz16(l32);
-    const TrLane<CT> trl = make_tr_lane<CT, 4, 8>(lane);
+    TrLane<CT> trl = make_tr_lane<CT, 4, 8>(lane);
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) { trl.off[ct][0] += half * RING_B; trl.off[ct][1] += half * RING_B; }
+    }
     // LDS address of this lane's 16 bytes of k-step 0 in the Q tile of stage 0 (row l32, chunk g ^ swizzle); k-step ks is
     // this address ^ (ks << 5): the ring starts on a 1 KB boundary, so the exclusive-or commutes with the sum
-    const unsigned qaddr = lds_addr(smem_raw) + l32 * 256 + ((g ^ fr) << 4);
+    static_assert(RING_B % 1024 == 0, "the exclusive-or of qaddr");
+    const unsigned qaddr = lds_addr(ring) + l32 * 256 + ((g ^ fr) << 4);
+    const unsigned raddr = lds_addr(ring) + wv * 256;       // the wave's gate values, but for their place in a stage (wave-uniform)
 
     // B operands of the token contraction (P, dM, dN of one tile, bf16).  They live across steps: the element pairs 0 and 1
     // of a tile are converted under the last matrix instructions of the step that computed its first products, the other
@@ -771,23 +800,20 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     auto step = [&](auto st_c, auto sp_c, f32x16& m, f32x16& n, f32x16& da, const f32x16& pm, const f32x16& pn,
                     const f32x16& pda, bool live, int& nv_next) {
         constexpr int ST = decltype(st_c)::value, SP = decltype(sp_c)::value;
-        const unsigned char* sQ = smem_raw + ST * DW_STAGE_B;
-        const unsigned char* sG = sQ + TILE_B;
-        const unsigned char* pQ = smem_raw + SP * DW_STAGE_B;
-        const unsigned char* pG = pQ + TILE_B;
+        const unsigned char* pQ = smem_raw + SP * STAGE_B;       // (trl holds the ring's place)
         // the previous tile's gate values, or zeros when there is no previous tile to contract (first step of a slice,
         // phantom steps that pad the loop): a zero gate makes P, dM and dN exactly zero
-        const float* pR = live ? reinterpret_cast<const float*>(pG + TILE_B) + wave * 64 : sZero;
+        const unsigned rp = live ? raddr + (SP * STAGE_B + 2 * TILE_B) : lds_addr(sZero);
 
         // LDS reads of the first products: the gate values of this tile's first four token rows (for the element pairs
         // converted at the end of this step) and of the previous tile for this lane's 16 token rows (4
         // consecutive rows per 16-byte read), then the operand ring (k-step ks + 2 is requested while ks is consumed).
         // All are issued from inline assembly and waited for by count; the element-wise slices in between are VALU only.
         __builtin_amdgcn_sched_barrier(0);
-        u32x4 rvn = lds_read16_async<0>(lds_addr(smem_raw) + (ST * DW_STAGE_B + 2 * TILE_B) + wave * 256 + 16 * g);
+        u32x4 rvn = lds_read16_async<0>(raddr + (ST * STAGE_B + 2 * TILE_B) + 16 * g);
         u32x4 rvu[4];
         {
-            const unsigned ra = lds_addr(pR) + 16 * g;
+            const unsigned ra = rp + 16 * g;
             rvu[0] = lds_read16_async<0>(ra);
             rvu[1] = lds_read16_async<32>(ra);
             rvu[2] = lds_read16_async<64>(ra);
@@ -797,8 +823,8 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
         auto request = [&](auto kc) {
             constexpr int ks = decltype(kc)::value;
             const unsigned a = qaddr ^ (ks << 5);     // the stage goes into the instruction's immediate offset
-            aq[ks % 3] = lds_read16_async<ST * DW_STAGE_B>(a);
-            ag[ks % 3] = lds_read16_async<ST * DW_STAGE_B + TILE_B>(a);
+            aq[ks % 3] = lds_read16_async<ST * STAGE_B>(a);
+            ag[ks % 3] = lds_read16_async<ST * STAGE_B + TILE_B>(a);
         };
         request(std::integral_constant<int, 0>{});
         request(std::integral_constant<int, 1>{});
@@ -990,7 +1016,49 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
         }
     }
     wait_vmcnt<0>();
+    if (PAIR && one_less) __builtin_amdgcn_s_barrier();
     __syncthreads();      // every wave is done reading the tile ring, which the epilogue reuses
+
+    // PAIR: the first wave of a block takes over the other's sums of dK and dU, the other the first's of dV, each through 16 KB a
+    // gradient that the taker alone reads, and which then serve its stores.
+    unsigned char* region = smem_raw + (PAIR ? wv * 49152 + half * 32768 : wave * 16384);
+    if constexpr (PAIR) {
+        auto leave = [&](const f32x16 (&acc)[CT], unsigned char* to) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    f32x4 v;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = acc[ct][4 * a + x];
+                    *reinterpret_cast<f32x4*>(to + (ct * 4 + a) * 1024 + lane * 16) = v;
+                }
+        };
+        auto take = [&](f32x16 (&acc)[CT], const unsigned char* from) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(from + (ct * 4 + a) * 1024 + lane * 16);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) acc[ct][4 * a + x] += v[x];
+                }
+        };
+        unsigned char* block = smem_raw + wv * 49152;
+        if (half) {
+            leave(dk, block);
+            leave(du, block + 16384);
+        } else {
+            leave(dv, block + 32768);
+        }
+        __syncthreads();
+        if (half) {
+            take(dv, block + 32768);
+        } else {
+            take(dk, block);
+            take(du, block + 16384);
+        }
+    }
 
     // dK^T registers 4a+x of row tile ct: c = 32ct + 8a + 4g + x, column j = l32, i.e. a lane owns runs of 4 c of weight row
     // j.  Stored directly these are 8- or 16-byte pieces scattered over 32 rows per instruction; instead each wave passes
@@ -998,10 +1066,19 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     // c16 ^ r), reads it back row-wise and stores whole rows.  Only this wave touches the region, and LDS operations of
     // one wave complete in order, so no barrier is needed between the three blocks.
     {
-        unsigned char* region = smem_raw + wave * 16384;
         const long wsz = (long)gridDim.x * nblk * JB * DH;   // elements of one weight tensor
         const long row0 = (wrow - l32) * DH;                 // first element of this wave's block of rows
+        // (The addresses are made here, and for PAIR by each store anew: there are no registers to keep them, or parts of them from
+        // before the loop, beside all the sums.)
+        int here = lane;
+        asm volatile("" : "+v"(here));
+        auto own_lane = [&]() {
+            int l = here;
+            if constexpr (PAIR) asm volatile("" : "+v"(l));
+            return l;
+        };
         auto store_f32 = [&](const f32x16 (&acc)[CT], float* dst) {      // rows of DH floats, 512-byte rows in LDS
+            const int lane = own_lane(), l32 = lane & 31, g = lane >> 5;
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -1022,6 +1099,7 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
             }
         };
         auto store_bf16 = [&](const f32x16 (&acc)[CT], bf16_t* dst) {    // rows of DH bf16, 256-byte rows in LDS
+            const int lane = own_lane(), l32 = lane & 31, g = lane >> 5;
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -1041,19 +1119,17 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
                 }
             }
         };
+        const bool ku = !PAIR || !half, v = !PAIR || half;   // the gradients whose sums this wave has
         if (p.nslice > 1) {                                  // fp32 partial sums of this token slice
             float* base = p.part + (long)z * 3 * wsz;
-            store_f32(dk, base);
-            store_f32(du, base + wsz);
-            store_f32(dv, base + 2 * wsz);
+            if (ku) { store_f32(dk, base); store_f32(du, base + wsz); }
+            if (v) store_f32(dv, base + 2 * wsz);
         } else if (p.out_f32) {                              // one slice: the sums are the gradients
-            store_f32(dk, static_cast<float*>(p.out[0]));
-            store_f32(du, static_cast<float*>(p.out[1]));
-            store_f32(dv, static_cast<float*>(p.out[2]));
+            if (ku) { store_f32(dk, static_cast<float*>(p.out[0])); store_f32(du, static_cast<float*>(p.out[1])); }
+            if (v) store_f32(dv, static_cast<float*>(p.out[2]));
         } else {
-            store_bf16(dk, static_cast<bf16_t*>(p.out[0]));
-            store_bf16(du, static_cast<bf16_t*>(p.out[1]));
-            store_bf16(dv, static_cast<bf16_t*>(p.out[2]));
+            if (ku) { store_bf16(dk, static_cast<bf16_t*>(p.out[0])); store_bf16(du, static_cast<bf16_t*>(p.out[1])); }
+            if (v) store_bf16(dv, static_cast<bf16_t*>(p.out[2]));
         }
     }
 }
@@ -1107,23 +1183,40 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // partial sums nor the summing pass exist.  Every further slice adds a set of fp32 partial sums that is written and
 // read back once (priced at the time of a token tile per 2.5 MB: about 4 TB/s against 1.25 us per tile).
 constexpr long DW_FIXED_TILES = 9;      // prologue + epilogue of a workgroup, in token tiles
+// Two blocks a workgroup (PAIR) are the choice between: half the tiles for a wave, in steps that are 8 to 14 % longer (twice the fills a
+// wave) and with two tiles' worth more at the end.  Whole backward, us, before / with it: 512 tokens of 8 heads of 96 with 8 experts of 256 40.8 / 36.2,
+// 1,000 67.8 / 54.0 (two slices / none), 2,048 95.4 / 92.3, 8,192 282.3 / 284.5 (not taken); 600 of 4 heads of 128 with the same experts 47.5 / 40.6, of
+// 12 with 4 of 128 41.9 / 34.9; 2 x 300 of 8 heads of 96 on two, eight slices / four, 54.3 / 51.6; 128 of 8 of 96 22.6 / 22.8 (not taken).
+// Not in two slices: half the partial sums of the other form's four with the longer steps goes either way (1,500 tokens of 4 heads of 128 70.4 / 67.7,
+// in one slice 68.8; 4,000 of 8 on two 333 / 343; 4,000 of 12 with 4 experts of 128 91.9 / 93.8).
+constexpr double DW_PAIR_FIXED_TILES = 10.8, DW_PAIR_STEP = 1.14;
 constexpr long DW_BYTES_PER_TILE_TIME = 2500000;
-int dw_slices_bf16(const Dims& d, size_t ws_bytes)
+struct DwPick {
+    bool pair;
+    int nslice;
+};
+static DwPick dw_pick(const Dims& d, size_t ws_bytes)
 {
     const int nblk = d.E * (d.d_e / JB);
-    const long cols = (long)((nblk + 3) / 4) * d.Hkuv;
     const long ntile = (long)(d.H / d.Hkuv) * d.B * ((d.S + 31) / 32);
     const size_t slice_b = (size_t)3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float);
-    long best = 1, best_cost = -1;
-    for (long ns = 1; ns <= 64 && (ns == 1 || ns <= ntile / 8); ++ns) {
-        if (ns > 1 && align256((size_t)ns * slice_b) > ws_bytes) break;
-        const long rounds = (cols * ns + CUS - 1) / CUS;
-        const long cost = rounds * ((ntile + ns - 1) / ns + DW_FIXED_TILES) +
-                          (ns > 1 ? ns * (long)(slice_b / DW_BYTES_PER_TILE_TIME) : 0);
-        if (best_cost < 0 || cost < best_cost) { best = ns; best_cost = cost; }
+    DwPick best{false, 1};
+    double best_cost = -1;
+    for (int pair = 0; pair < 2; ++pair) {
+        const long cols = (long)((nblk + (pair ? 1 : 3)) / (pair ? 2 : 4)) * d.Hkuv;
+        if (pair && ntile < 2) break;      // (a tile for either half; slices have eight)
+        for (long ns = 1; ns <= 64 && (ns == 1 || ns <= ntile / 8); ++ns) {
+            if (ns > 1 && align256((size_t)ns * slice_b) > ws_bytes) break;
+            if (pair && ns == 2) continue;
+            const long rounds = (cols * ns + CUS - 1) / CUS, tiles = (ntile + ns - 1) / ns;
+            const double cost = rounds * (pair ? (tiles + 1) / 2 * DW_PAIR_STEP + DW_PAIR_FIXED_TILES : tiles + DW_FIXED_TILES) +
+                                (ns > 1 ? ns * (double)slice_b / DW_BYTES_PER_TILE_TIME : 0);
+            if (best_cost < 0 || cost < best_cost) { best = DwPick{pair != 0, (int)ns}; best_cost = cost; }
+        }
     }
-    return (int)best;
+    return best;
 }
+int dw_slices_bf16(const Dims& d, size_t ws_bytes) { return dw_pick(d, ws_bytes).nslice; }
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 
@@ -1205,17 +1298,15 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     if (phases & PH_BWD_DKDUDV) {
         DwArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, part,
                  {dK, dU, dV}, grad_w_f32, d.B, d.H, G, d.S, d.E, nbe, nslice, d.tokmaj};
-        const int smem = DW_NST * DW_STAGE_B + 128;
-        static LdsOptIn optin_full, optin_tail;
-        err = d.S % 32 == 0 ? ensure_dynamic_lds(optin_full, (const void*)mhffn_bwd_dkdudv_kernel<DH, false>, smem)
-                            : ensure_dynamic_lds(optin_tail, (const void*)mhffn_bwd_dkdudv_kernel<DH, true>, smem);
+        const bool pair = dw_pick(d, ws_bytes).pair, tail = d.S % 32 != 0;
+        const int smem = (pair ? 2 * DW_NST * DW_PAIR_STAGE_B : DW_NST * DW_STAGE_B) + 128;
+        static LdsOptIn optin[4];
+        auto* fn = pair ? tail ? mhffn_bwd_dkdudv_kernel<DH, true, TokenHalves> : mhffn_bwd_dkdudv_kernel<DH, false, TokenHalves>
+                        : tail ? mhffn_bwd_dkdudv_kernel<DH, true> : mhffn_bwd_dkdudv_kernel<DH, false>;
+        err = ensure_dynamic_lds(optin[2 * pair + tail], (const void*)fn, smem);
         if (err != hipSuccess) return err;
-        const int nblk = d.E * nbe;
-        dim3 grid((unsigned)d.Hkuv, (unsigned)((nblk + 3) / 4), (unsigned)nslice);
-        if (d.S % 32 == 0)
-            hipLaunchKernelGGL((mhffn_bwd_dkdudv_kernel<DH, false>), grid, dim3(256), smem, st, a);
-        else
-            hipLaunchKernelGGL((mhffn_bwd_dkdudv_kernel<DH, true>), grid, dim3(256), smem, st, a);
+        const int nblk = d.E * nbe, nb = pair ? 2 : 4;
+        hipLaunchKernelGGL(fn, dim3((unsigned)d.Hkuv, (unsigned)((nblk + nb - 1) / nb), (unsigned)nslice), dim3(256), smem, st, a);
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
