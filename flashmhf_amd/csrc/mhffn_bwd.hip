@@ -34,6 +34,7 @@ struct DqArgs {
     float* part;          // [nsplit][Hkuv][rows.n][DH] dQ, then [nsplit][Hkuv][rows.n][E] dR: fp32 partial sums
     RowMap rows;          // rows of Q, dO, dQ, R, dR that meet one K/U/V head
     Parts parts;          // ... and the blocks of that head
+    int tile_rows;
 };
 
 constexpr int DQ_NST = 4;                  // LDS stages (K | U | V tiles each)
@@ -52,6 +53,7 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blockIdx.x = tile * Hkuv + kv-head: the head index runs fastest, so each head's weights stay in one XCD's L2
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    if (tile * BT >= p.rows.n) return;                       // (whole_xcds)
     const int tok0 = tile * BT + wave * 32;                  // this wave's rows of the list (RowMap)
     const int nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;   // blocks of this workgroup, counted from blk0
@@ -314,6 +316,7 @@ __global__ __launch_bounds__(DQ32_W * 64) void mhffn_bwd_dqdr_rows32_kernel(DqAr
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
     const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    if (tok0 >= p.rows.n) return;                            // (whole_xcds)
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
     const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
     const bf16_t* Kh = p.K + ((long)hk * E * nbe + blk0) * JB * DH;
@@ -536,14 +539,16 @@ __global__ __launch_bounds__(DQ32_W * 64) void mhffn_bwd_dqdr_rows32_kernel(DqAr
 }
 
 // Adds the parts' sums of dQ (in the order of the parts) and rounds once, four columns per lane; adds the sums of dR over the
-// parts that hold blocks of the expert, one value per lane.  Workgroup `block` of head hk: below dq_blocks dQ, otherwise dR.
+// parts that hold blocks of the expert, one value per lane.  Workgroup `block` of tile x, counted with the heads as the kernel that left the
+// parts did: below dq_blocks dQ, otherwise dR.
 template <int DH>
-__device__ __forceinline__ void dqdr_sum(const DqArgs& p, int hk, unsigned block, unsigned dq_blocks)
+__device__ __forceinline__ void dqdr_sum(const DqArgs& p, unsigned x, unsigned block, unsigned dq_blocks)
 {
+    const int tile = p.rows.by_hkuv.div(x), hk = x - tile * p.rows.Hkuv;
     const long hrows = (long)p.rows.Hkuv * p.rows.n;
     if (block < dq_blocks) {
         const unsigned i = block * 256 + threadIdx.x;
-        const unsigned r = i / (DH / 4), c = (i % (DH / 4)) * 4;
+        const unsigned r = tile * p.tile_rows + i / (DH / 4), c = (i % (DH / 4)) * 4;
         if (r >= (unsigned)p.rows.n) return;
         const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
         auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + z * hrows * DH); };
@@ -555,9 +560,9 @@ __device__ __forceinline__ void dqdr_sum(const DqArgs& p, int hk, unsigned block
     } else {
         const unsigned i = (block - dq_blocks) * 256 + threadIdx.x;
         const int E = p.parts.E;
-        const unsigned r = i / (unsigned)E;
-        const int e = i - r * E;
-        if (r >= (unsigned)p.rows.n) return;
+        const unsigned row = i / (unsigned)E, r = tile * p.tile_rows + row;
+        const int e = i - row * E;
+        if (row >= (unsigned)p.tile_rows || r >= (unsigned)p.rows.n) return;
         const float* src = p.part + p.parts.nsplit * hrows * DH + ((long)hk * p.rows.n + r) * E + e;
         p.dR[p.rows.gate(hk, r) * E + e] =
             sum_in_order(0.0f, p.parts.part_lo(e), p.parts.part_hi(e), [&](int z) { return src[z * hrows * E]; });
@@ -566,7 +571,7 @@ __device__ __forceinline__ void dqdr_sum(const DqArgs& p, int hk, unsigned block
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_bwd_dqdr_sum_kernel(DqArgs p, unsigned dq_blocks)
 {
-    dqdr_sum<DH>(p, blockIdx.y, blockIdx.x, dq_blocks);
+    dqdr_sum<DH>(p, blockIdx.x, blockIdx.y, dq_blocks);
 }
 
 // ------------------------------------------------------------------------------------------------ dK / dU / dV
@@ -1134,42 +1139,53 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
     }
 }
 
-// Sums the token-slice partials of dK, dU or dV (w = 0, 1, 2) and converts to the output dtype, four values per lane.
+// Sums the token-slice partials of dK, dU and dV and converts to the output dtype, four values per lane.  Workgroups count the columns of
+// the kernel that left them (rows of weights of a head's workgroup) as it did, then 1,024 values of such a column at a time, then the
+// gradients.
+struct WeightSums {
+    const float* part;
+    void* out[3];
+    long size;            // values of a gradient
+    unsigned head;        // ... of a head
+    int nslice, Hkuv, column;      // values of a column
+    unsigned columns, steps;       // workgroups that the kernel's grid has for a slice; workgroups of this pass for a column
+    FastDiv by_columns, by_steps, by_hkuv;
+};
 template <typename OutT>
-__device__ __forceinline__ void slice_sum(const float* __restrict__ part, OutT* dK, OutT* dU, OutT* dV, long wsz, int nslice, int w, unsigned block)
+__device__ __forceinline__ void slice_sum(const WeightSums& p, unsigned block)
 {
     typedef OutT OutT4 __attribute__((ext_vector_type(4)));
-    const long i4 = ((long)block * 256 + threadIdx.x) * 4;
-    if (i4 >= wsz) return;
-    const float* src = part + w * wsz + i4;
-    auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + 3 * z * wsz); };
-    const f32x4 sum = sum_in_order(load(0), 1, nslice, load);
+    const unsigned k = p.by_columns.div(block), u = block - k * p.columns, w = p.by_steps.div(k), step = k - w * p.steps;
+    const unsigned col = p.by_hkuv.div(u), hk = u - col * p.Hkuv, in = col * p.column + step * 1024 + threadIdx.x * 4;
+    if (in >= p.head) return;
+    const long i4 = (long)hk * p.head + in;
+    const float* src = p.part + w * p.size + i4;
+    auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + 3 * z * p.size); };
+    const f32x4 sum = sum_in_order(load(0), 1, p.nslice, load);
     OutT4 v;
 #pragma unroll
     for (int x = 0; x < 4; ++x) v[x] = (OutT)sum[x];
-    *reinterpret_cast<OutT4*>((w == 0 ? dK : w == 1 ? dU : dV) + i4) = v;
+    *reinterpret_cast<OutT4*>(static_cast<OutT*>(w == 0 ? p.out[0] : w == 1 ? p.out[1] : p.out[2]) + i4) = v;
 }
 template <typename OutT>
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ part, OutT* dK, OutT* dU, OutT* dV,
-                                                              long wsz, int nslice)
+__global__ __launch_bounds__(256) void reduce_partials_kernel(WeightSums p)
 {
-    slice_sum(part, dK, dU, dV, wsz, nslice, blockIdx.y, blockIdx.x);
+    slice_sum<OutT>(p, blockIdx.x);
 }
 
 // Both sums of a backward in one launch, behind both its kernels: a launch less, and one pass fills the chip where two were
 // latency (2 x 300 tokens of 8 heads of 96, two K/U/V heads: 4.9 + 7.0 us under the profiler, 10.0 in one; the call, bound by the host there, 99 -> 92).  Workgroups: dq_blocks of dQ and
-// r_blocks of dR per head, then w_blocks of each gradient.
+// r_blocks of dR per tile, then the gradients'.
 template <int DH, typename OutT>
-__global__ __launch_bounds__(256) void mhffn_bwd_sums_kernel(DqArgs p, unsigned dq_blocks, unsigned head_blocks, const float* __restrict__ part,
-                                                             OutT* dK, OutT* dU, OutT* dV, long wsz, int nslice, unsigned w_blocks)
+__global__ __launch_bounds__(256) void mhffn_bwd_sums_kernel(DqArgs p, unsigned dq_blocks, unsigned tile_blocks, unsigned tiles, FastDiv by_tiles,
+                                                             WeightSums w)
 {
-    const unsigned heads = head_blocks * p.rows.Hkuv;
-    if (blockIdx.x < heads) {
-        const unsigned hk = blockIdx.x / head_blocks;
-        dqdr_sum<DH>(p, hk, blockIdx.x - hk * head_blocks, dq_blocks);
+    const unsigned of_tiles = tile_blocks * tiles;
+    if (blockIdx.x < of_tiles) {
+        const unsigned block = by_tiles.div(blockIdx.x);
+        dqdr_sum<DH>(p, blockIdx.x - block * tiles, block, dq_blocks);
     } else {
-        const unsigned b = blockIdx.x - heads, w = b / w_blocks;
-        slice_sum(part, dK, dU, dV, wsz, nslice, w, b - w * w_blocks);
+        slice_sum<OutT>(w, blockIdx.x - of_tiles);
     }
 }
 
@@ -1275,8 +1291,16 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
     constexpr int ALL = PH_BWD_DQDR | PH_BWD_DKDUDV | PH_BWD_REDUCE;
     const bool together = (phases & ALL) == ALL && sums_together(d, nslice, pick.nsplit) && slices_b + pick.nsplit * dq_part_bytes(d) <= ws_bytes;
     DqArgs dq{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, (bf16_t*)dQ, dR,
-              together ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + slices_b) : part, RowMap(d), Parts(d.E, nbe, pick.nsplit)};
-    const unsigned qb = (unsigned)(((long)dq.rows.n * (DH / 4) + 255) / 256), rb = (unsigned)(((long)dq.rows.n * d.E + 255) / 256);
+              together ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + slices_b) : part, RowMap(d), Parts(d.E, nbe, pick.nsplit), pick.tile_rows};
+    // the summing pass's workgroups of a tile for dQ and dR, and the tiles of the grid of dQ/dR
+    const int in_tile = dq.rows.n < pick.tile_rows ? dq.rows.n : pick.tile_rows;
+    const unsigned qb = (unsigned)((in_tile * (DH / 4) + 255) / 256), rb = (unsigned)(((long)in_tile * d.E + 255) / 256);
+    const unsigned tiles = whole_xcds((unsigned)((dq.rows.n + pick.tile_rows - 1) / pick.tile_rows * d.Hkuv), pick.nsplit);
+    static_assert(32 * (DH / 4) % 256 == 0, "a workgroup's rows are of one tile");
+
+    const bool pair = dw_pick(d, ws_bytes).pair;
+    const int nb = pair ? 2 : 4;            // blocks of a workgroup of dK/dU/dV
+    const unsigned columns = (unsigned)((d.E * nbe + nb - 1) / nb * d.Hkuv);
 
     if (phases & PH_BWD_DQDR) {
         const DqArgs& a = dq;
@@ -1287,44 +1311,42 @@ static hipError_t launch_bwd_t(const void* Q, const void* K, const void* U, cons
         err = tokw == 32 ? ensure_dynamic_lds(optin32, (const void*)mhffn_bwd_dqdr_rows32_kernel<DH>, smem)
                          : ensure_dynamic_lds(optin, (const void*)mhffn_bwd_dqdr_kernel<DH>, smem);
         if (err != hipSuccess) return err;
-        dim3 grid((unsigned)((a.rows.n + tokw - 1) / tokw * d.Hkuv), (unsigned)a.parts.nsplit);
+        dim3 grid(tiles, (unsigned)a.parts.nsplit);
         if (tokw == 32) hipLaunchKernelGGL((mhffn_bwd_dqdr_rows32_kernel<DH>), grid, dim3(DQ32_W * 64), smem, st, a);
         else hipLaunchKernelGGL((mhffn_bwd_dqdr_kernel<DH>), grid, dim3(512), smem, st, a);
         if (a.parts.nsplit > 1 && !together)
-            hipLaunchKernelGGL((mhffn_bwd_dqdr_sum_kernel<DH>), dim3(qb + rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, qb);
+            hipLaunchKernelGGL((mhffn_bwd_dqdr_sum_kernel<DH>), dim3(tiles, qb + rb), dim3(256), 0, st, a, qb);
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
     if (phases & PH_BWD_DKDUDV) {
         DwArgs a{(const bf16_t*)Q, (const bf16_t*)dO, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V, R, part,
                  {dK, dU, dV}, grad_w_f32, d.B, d.H, G, d.S, d.E, nbe, nslice, d.tokmaj};
-        const bool pair = dw_pick(d, ws_bytes).pair, tail = d.S % 32 != 0;
+        const bool tail = d.S % 32 != 0;
         const int smem = (pair ? 2 * DW_NST * DW_PAIR_STAGE_B : DW_NST * DW_STAGE_B) + 128;
         static LdsOptIn optin[4];
         auto* fn = pair ? tail ? mhffn_bwd_dkdudv_kernel<DH, true, TokenHalves> : mhffn_bwd_dkdudv_kernel<DH, false, TokenHalves>
                         : tail ? mhffn_bwd_dkdudv_kernel<DH, true> : mhffn_bwd_dkdudv_kernel<DH, false>;
         err = ensure_dynamic_lds(optin[2 * pair + tail], (const void*)fn, smem);
         if (err != hipSuccess) return err;
-        const int nblk = d.E * nbe, nb = pair ? 2 : 4;
-        hipLaunchKernelGGL(fn, dim3((unsigned)d.Hkuv, (unsigned)((nblk + nb - 1) / nb), (unsigned)nslice), dim3(256), smem, st, a);
+        hipLaunchKernelGGL(fn, dim3((unsigned)d.Hkuv, columns / d.Hkuv, (unsigned)nslice), dim3(256), smem, st, a);
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
     if ((phases & PH_BWD_REDUCE) && nslice > 1) {
-        const unsigned rblocks = (unsigned)((wsz / 4 + 255) / 256);
-        const unsigned all = (qb + rb) * d.Hkuv + 3 * rblocks;
+        const int column = nb * JB * DH;
+        static_assert(2 * JB * DH % 1024 == 0, "a workgroup's values are of one column");
+        const WeightSums w{part, {dK, dU, dV}, wsz, (unsigned)(wsz / d.Hkuv), nslice, d.Hkuv, column, columns, (unsigned)column / 1024,
+                           FastDiv(columns), FastDiv(column / 1024), FastDiv(d.Hkuv)};
+        const unsigned wb = 3 * columns * w.steps, tb = together ? (qb + rb) * tiles : 0;
         if (together && grad_w_f32)
-            hipLaunchKernelGGL((mhffn_bwd_sums_kernel<DH, float>), dim3(all), dim3(256), 0, st, dq, qb, qb + rb, part, (float*)dK, (float*)dU,
-                               (float*)dV, wsz, nslice, rblocks);
+            hipLaunchKernelGGL((mhffn_bwd_sums_kernel<DH, float>), dim3(tb + wb), dim3(256), 0, st, dq, qb, qb + rb, tiles, FastDiv(tiles), w);
         else if (together)
-            hipLaunchKernelGGL((mhffn_bwd_sums_kernel<DH, bf16_t>), dim3(all), dim3(256), 0, st, dq, qb, qb + rb, part, (bf16_t*)dK, (bf16_t*)dU,
-                               (bf16_t*)dV, wsz, nslice, rblocks);
+            hipLaunchKernelGGL((mhffn_bwd_sums_kernel<DH, bf16_t>), dim3(tb + wb), dim3(256), 0, st, dq, qb, qb + rb, tiles, FastDiv(tiles), w);
         else if (grad_w_f32)
-            hipLaunchKernelGGL((reduce_partials_kernel<float>), dim3(rblocks, 3), dim3(256), 0, st, part, (float*)dK,
-                               (float*)dU, (float*)dV, wsz, nslice);
+            hipLaunchKernelGGL((reduce_partials_kernel<float>), dim3(wb), dim3(256), 0, st, w);
         else
-            hipLaunchKernelGGL((reduce_partials_kernel<bf16_t>), dim3(rblocks, 3), dim3(256), 0, st, part, (bf16_t*)dK,
-                               (bf16_t*)dU, (bf16_t*)dV, wsz, nslice);
+            hipLaunchKernelGGL((reduce_partials_kernel<bf16_t>), dim3(wb), dim3(256), 0, st, w);
         err = hipGetLastError();
     }
     return err;

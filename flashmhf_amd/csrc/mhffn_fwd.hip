@@ -34,6 +34,7 @@ struct FwdArgs {
     float* part;          // [nsplit][Hkuv][rows.n][DH] fp32 partial sums (more parts than one)
     RowMap rows;          // rows of Q, O, R that meet one K/U/V head
     Parts parts;          // ... and the blocks of that head
+    int tile_rows;
 };
 
 // LDS ring of FWD_NST stages, laid out as three regions (all V tiles, all K tiles, all U tiles).  The block loop is
@@ -91,6 +92,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blockIdx.x = tile * Hkuv + kv-head: the head index runs fastest, so each head's weights stay in one XCD's L2
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
+    if (tile * BT >= p.rows.n) return;                       // (whole_xcds)
     const int tok0 = tile * BT + wave * WT;                  // this wave's rows of the list (RowMap)
     const int nbe = p.parts.nbe, E = p.parts.E;
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;   // blocks of this workgroup, counted from blk0
@@ -423,6 +425,7 @@ __global__ __launch_bounds__(256) void mhffn_fwd_rows32_kernel(FwdArgs p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
     const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    if (tok0 >= p.rows.n) return;                            // (whole_xcds)
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
     const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
     const int nex = p.parts.by_nbe.div(jb0 + nblk + nbe - 1);
@@ -563,6 +566,7 @@ __global__ __launch_bounds__(FWDL_W * 64) void mhffn_fwd_rows32_long_kernel(FwdA
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
     const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
+    if (tok0 >= p.rows.n) return;                            // (whole_xcds)
     const int blk0 = p.parts.first(z), nblk = p.parts.first(z + 1) - blk0;
     const int ex0 = p.parts.by_nbe.div(blk0), jb0 = blk0 - ex0 * nbe;
     const unsigned smem0 = lds_addr(smem);
@@ -729,13 +733,14 @@ __global__ __launch_bounds__(FWDL_W * 64) void mhffn_fwd_rows32_long_kernel(FwdA
     }
 }
 
-// Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, four columns per lane.
+// Adds the parts' sums (in the order of the parts) and rounds once: O row r of kv-head hk, four columns per lane.  blockIdx.x counts tiles
+// and heads as the kernel that left the parts did.
 template <int DH>
 __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 {
-    const unsigned i = blockIdx.x * 256 + threadIdx.x;
-    const unsigned r = i / (DH / 4), c = (i % (DH / 4)) * 4;
-    const int hk = blockIdx.y;
+    const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv;
+    const unsigned i = blockIdx.y * 256 + threadIdx.x;
+    const unsigned r = tile * p.tile_rows + i / (DH / 4), c = (i % (DH / 4)) * 4;
     if (r >= (unsigned)p.rows.n) return;
     const long step = (long)p.rows.Hkuv * p.rows.n * DH;
     const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
@@ -780,13 +785,15 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, h
                          : tile_rows == 128 ? ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem)
                                             : ensure_dynamic_lds(optin32, (const void*)mhffn_fwd_rows32_kernel<DH>, smem);
     if (e != hipSuccess) return e;
-    dim3 grid((unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv), (unsigned)a.parts.nsplit);
+    const unsigned tiles = (unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv);
+    dim3 grid(whole_xcds(tiles, a.parts.nsplit), (unsigned)a.parts.nsplit);
     if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
     else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(512), smem, st, a);
     else if (pipeline) hipLaunchKernelGGL((mhffn_fwd_rows32_long_kernel<DH>), grid, dim3(FWDL_W * 64), smem, st, a);
     else hipLaunchKernelGGL((mhffn_fwd_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
-        dim3 sgrid((unsigned)(((long)a.rows.n * (DH / 4) + 255) / 256), (unsigned)d.Hkuv);
+        static_assert(32 * (DH / 4) % 256 == 0, "a workgroup's rows are of one tile");
+        dim3 sgrid(grid.x, (unsigned)(((a.rows.n < tile_rows ? a.rows.n : tile_rows) * (DH / 4) + 255) / 256));
         hipLaunchKernelGGL((mhffn_fwd_sum_kernel<DH>), sgrid, dim3(256), 0, st, a);
     }
     return hipGetLastError();
@@ -804,7 +811,7 @@ hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const vo
     if (!(phases & PH_FWD_MAIN)) return hipSuccess;
     const Pick pick = fwd_pick_bf16(d, ws ? ws_bytes : 0, phases);
     FwdArgs a{(const bf16_t*)Q, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V,           R,
-              (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, pick.nsplit)};
+              (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, pick.nsplit), pick.tile_rows};
     switch (d.d_h) {
         case 64: return launch_fwd_t<64>(a, d, pick.tile_rows, st);
         case 96: return launch_fwd_t<96>(a, d, pick.tile_rows, st);
