@@ -25,6 +25,8 @@
 // and epilogue.
 #include "mhffn_common.hpp"
 
+#include <utility>
+
 namespace mhffn {
 
 namespace {
@@ -38,6 +40,7 @@ struct F32Args {
     RowMap rows;        // rows of Q, O, dO, dQ, R, dR that meet one K/U/V head
     Parts parts;        // blocks of 32 weight rows of that head, the last of an expert with de % 32 rows if that is not 0
     int DH, de, nslice;
+    int heads_first;    // dK/dU/dV: the head runs fastest over the workgroups
 };
 
 __device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
@@ -400,15 +403,18 @@ __device__ __forceinline__ void split_row_operand(Split8 (&v)[2 * CT], const f32
 }
 
 // Workgroup of the forward and of dQ/dR: 4 waves of 32 rows of one K/U/V head, one part of the head's blocks.
+constexpr int F32_ROWS = 128;
 struct Place {
     int hk, z, row0, row, blk0, nblk;      // row0: this wave's first row of the list, row: this lane's (clamped into the list)
     bool valid;                            // this lane's row exists
+    bool none;                             // no row of the workgroup does (whole_xcds)
     __device__ explicit Place(const F32Args& p, int wave, int l32)
     {
         const int tile = p.rows.by_hkuv.div(blockIdx.x);
         hk = blockIdx.x - tile * p.rows.Hkuv;
         z = blockIdx.y;
-        row0 = tile * 128 + wave * 32;
+        none = tile * F32_ROWS >= p.rows.n;
+        row0 = tile * F32_ROWS + wave * 32;
         valid = row0 + l32 < p.rows.n;
         row = valid ? row0 + l32 : p.rows.n - 1;
         blk0 = p.parts.first(z);
@@ -568,6 +574,7 @@ __global__ __launch_bounds__(256, 2) void fwd_fp32_kernel(F32Args p)
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const Place w(p, wave, lane & 31);
+    if (w.none) return;
     f32x16 o[CT];
     fwd_fp32<CT>(p, w, lds, wave, o);
     if (w.valid)
@@ -587,6 +594,7 @@ __global__ __launch_bounds__(256, CT > 3 ? 1 : 2) void dqdr_fp32_kernel(F32Args 
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const Place w(p, wave, lane & 31);
+    if (w.none) return;
     f32x16 dq[CT];
     dqdr_fp32<CT>(p, w, lds, wave, dr_row(p, w), w.valid, dq);
     if (w.valid)
@@ -603,6 +611,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS) void fwd_f32_kernel(F32Args p
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = wave >> 2;
     const Place w(p, wave & 3, l32);
+    if (w.none) return;
     const int DH = p.DH;
     const Cut<CT> cut(threadIdx.x & 255);
     const PlaneLane pl(lane);
@@ -708,6 +717,7 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Place w(p, wave, l32);
+    if (w.none) return;
     const int DH = p.DH, E = p.parts.E;
     const Cut<CT> cut(threadIdx.x);
     const PlaneLane pl(lane);
@@ -835,6 +845,12 @@ __global__ __launch_bounds__(256, 1) void dqdr_f32_kernel(F32Args p)
     if (again) store_row<CT>(dq, dst, g, DH);
 }
 
+// Head and pair of blocks of a workgroup of dK/dU/dV.  The head runs fastest, so that a head's weights, which dQ/dR has read, are in the L2 of
+// the XCD (both kernels, 256 tokens of the 128M layer 79.2 us in the other order, 77.4; 32 tokens 43.5, 41.5); several slices run in the other
+// order, in which their sums are read faster (500 tokens on four K/U/V heads 131.8, 133.8).
+__device__ __forceinline__ int head_of(const F32Args& p) { return p.heads_first ? blockIdx.x : blockIdx.y; }
+__device__ __forceinline__ int pair_of(const F32Args& p) { return p.heads_first ? blockIdx.y : blockIdx.x; }
+
 // End of a dK/dU/dV kernel: the odd tiles' sums to the wave with the even ones (64 lanes x 48 CT floats, lane-private), then the
 // rows that `take` picks to memory: take(finite) says whether a row goes, given whether all of it is finite.  (This lane's row and
 // the bounds of its columns are worked out again, out of the compiler's sight: kept over the loop they are the few registers too many
@@ -844,8 +860,8 @@ __device__ __forceinline__ void add_halves_and_store(const F32Args& p, unsigned 
                                                      Take&& take)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
-    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
-    const int blk = blockIdx.x * 2 + bw;
+    const int hk = head_of(p), z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
+    const int blk = pair_of(p) * 2 + bw;
     const Block b(p, hk, blk < nblk ? blk : nblk - 1);
     __syncthreads();
     int lane = threadIdx.x & 63, DH = p.DH;
@@ -915,8 +931,8 @@ __device__ __forceinline__ void dkdudv_fp32(const F32Args& p, unsigned char* lds
     constexpr int STAGE_B = 2 * T::BYTES;      // Q and dO tile
     float* sR = reinterpret_cast<float*>(lds + 4 * STAGE_B);      // [stage][wave][32] gate values
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 1, bw = wave & 1;
-    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
-    const int blk = blockIdx.x * 2 + bw;
+    const int hk = head_of(p), z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe;
+    const int blk = pair_of(p) * 2 + bw;
     const Block b(p, hk, blk < nblk ? blk : nblk - 1);
 
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5, DH = p.DH;
@@ -990,8 +1006,8 @@ __global__ __launch_bounds__(256, 1) void dkdudv_split_kernel(F32Args p)
     unsigned char* planes = lds + half * 2 * PLANES_B;                            // Q, dO
     unsigned char* raw = lds + 4 * PLANES_B + wave * RAW * 1024;
     float* sR = reinterpret_cast<float*>(lds + 4 * PLANES_B + 4 * RAW * 1024) + wave * 32;      // gate values of the wave's expert
-    const int hk = blockIdx.y, z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe, DH = p.DH;
-    const int blk = blockIdx.x * 2 + bw;
+    const int hk = head_of(p), z = blockIdx.z, E = p.parts.E, nblk = E * p.parts.nbe, DH = p.DH;
+    const int blk = pair_of(p) * 2 + bw;
     const Block b(p, hk, blk < nblk ? blk : nblk - 1);
     const int ntile = (p.rows.n + 31) / 32;
     const int t0 = (int)((long)ntile * z / p.nslice), t1 = (int)((long)ntile * (z + 1) / p.nslice);
@@ -1148,23 +1164,24 @@ __global__ __launch_bounds__(256, 1) void dkdudv_f32_kernel(F32Args p)
     add_halves_and_store<CT>(p, lds, dk, du, dv, [](auto) { return true; });
 }
 
-// Adds the parts' sums in order: the rows of O or dQ (dst, four columns per lane) and, for blockIdx.x >= row_blocks, the
-// values of dR over the parts that hold blocks of the expert.
-__global__ __launch_bounds__(256) void sum_f32_kernel(F32Args p, float* dst, unsigned row_blocks)
+// Adds the parts' sums in order: the rows of O or dQ (dst, four columns per lane) and, behind a tile's row_blocks, the values of dR over
+// the parts that hold blocks of the expert.  Workgroups count tiles and heads as the kernel that left the parts did (whole_xcds).
+__global__ __launch_bounds__(256) void sum_f32_kernel(F32Args p, float* dst, unsigned row_blocks, unsigned tiles, FastDiv by_tiles)
 {
-    const int hk = blockIdx.y, DH = p.DH, E = p.parts.E;
+    const unsigned block = by_tiles.div(blockIdx.x), x = blockIdx.x - block * tiles;
+    const int tile = p.rows.by_hkuv.div(x), hk = x - tile * p.rows.Hkuv, DH = p.DH, E = p.parts.E;
     const long hrows = (long)p.rows.Hkuv * p.rows.n;
-    if (blockIdx.x < row_blocks) {
-        const unsigned i = blockIdx.x * 256 + threadIdx.x, r = i / (unsigned)(DH / 4);
-        const int c = (i - r * (DH / 4)) * 4;
-        if (r >= (unsigned)p.rows.n) return;
+    if (block < row_blocks) {
+        const unsigned i = block * 256 + threadIdx.x, row = i / (unsigned)(DH / 4), r = tile * F32_ROWS + row;
+        const int c = (i - row * (DH / 4)) * 4;
+        if (row >= (unsigned)F32_ROWS || r >= (unsigned)p.rows.n) return;
         const float* src = p.part + ((long)hk * p.rows.n + r) * DH + c;
         auto load = [&](int z) { return *reinterpret_cast<const f32x4*>(src + z * hrows * DH); };
         *reinterpret_cast<f32x4*>(dst + p.rows.tok(hk, r) * DH + c) = sum_in_order(load(0), 1, p.parts.nsplit, load);
     } else {
-        const unsigned i = (blockIdx.x - row_blocks) * 256 + threadIdx.x, r = i / (unsigned)E;
-        const int e = i - r * E;
-        if (r >= (unsigned)p.rows.n) return;
+        const unsigned i = (block - row_blocks) * 256 + threadIdx.x, row = i / (unsigned)E, r = tile * F32_ROWS + row;
+        const int e = i - row * E;
+        if (row >= (unsigned)F32_ROWS || r >= (unsigned)p.rows.n) return;
         const float* src = p.part + p.parts.nsplit * hrows * DH + ((long)hk * p.rows.n + r) * E + e;
         p.dR[p.rows.gate(hk, r) * E + e] =
             sum_in_order(0.0f, p.parts.part_lo(e), p.parts.part_hi(e), [&](int z) { return src[z * hrows * E]; });
@@ -1205,6 +1222,16 @@ F32Args f32_args(const void* Q, const void* K, const void* U, const void* V, con
     return a;
 }
 
+// Tiles of all heads in the grid of a part, and workgroups of the summing pass for a tile's rows of `width` lanes.
+unsigned tiles_of(const F32Args& a, const Dims& d)
+{
+    return whole_xcds((unsigned)((a.rows.n + F32_ROWS - 1) / F32_ROWS * d.Hkuv), a.parts.nsplit);
+}
+unsigned blocks_of_tile(const F32Args& a, int width)
+{
+    return (unsigned)(((long)(a.rows.n < F32_ROWS ? a.rows.n : F32_ROWS) * width + 255) / 256);
+}
+
 template <int CT>
 hipError_t launch_fwd_f32_t(const F32Args& a, const Dims& d, hipStream_t st)
 {
@@ -1216,11 +1243,11 @@ hipError_t launch_fwd_f32_t(const F32Args& a, const Dims& d, hipStream_t st)
     auto* fn = one_block ? fwd_fp32_kernel<CT> : fwd_f32_kernel<CT, GROUPS>;
     const hipError_t e = ensure_dynamic_lds(optin[one_block], (const void*)fn, smem);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fn, dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit), dim3(one_block ? 256 : 256 * GROUPS),
-                       smem, st, a);
+    const unsigned tiles = tiles_of(a, d);
+    hipLaunchKernelGGL(fn, dim3(tiles, (unsigned)a.parts.nsplit), dim3(one_block ? 256 : 256 * GROUPS), smem, st, a);
     if (a.parts.nsplit > 1) {
-        const unsigned rb = (unsigned)(((long)a.rows.n * (d.d_h / 4) + 255) / 256);
-        hipLaunchKernelGGL(sum_f32_kernel, dim3(rb, (unsigned)d.Hkuv), dim3(256), 0, st, a, a.O, rb);
+        const unsigned rb = blocks_of_tile(a, d.d_h / 4);
+        hipLaunchKernelGGL(sum_f32_kernel, dim3(tiles * rb), dim3(256), 0, st, a, a.O, rb, tiles, FastDiv(tiles));
     }
     return hipGetLastError();
 }
@@ -1236,18 +1263,19 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
         auto* fn = one_block ? dqdr_fp32_kernel<CT> : dqdr_f32_kernel<CT>;
         err = ensure_dynamic_lds(optin[one_block], (const void*)fn, smem);
         if (err != hipSuccess) return err;
-        hipLaunchKernelGGL(fn, dim3((unsigned)(((a.rows.n + 127) / 128) * d.Hkuv), (unsigned)a.parts.nsplit),
-                           dim3(256), smem, st, a);
+        const unsigned tiles = tiles_of(a, d);
+        hipLaunchKernelGGL(fn, dim3(tiles, (unsigned)a.parts.nsplit), dim3(256), smem, st, a);
         if (a.parts.nsplit > 1) {
-            const unsigned rb = (unsigned)(((long)a.rows.n * (d.d_h / 4) + 255) / 256);
-            const unsigned eb = (unsigned)(((long)a.rows.n * d.E + 255) / 256);
-            hipLaunchKernelGGL(sum_f32_kernel, dim3(rb + eb, (unsigned)d.Hkuv), dim3(256), 0, st, a, a.dQ, rb);
+            const unsigned rb = blocks_of_tile(a, d.d_h / 4), eb = blocks_of_tile(a, d.E);
+            hipLaunchKernelGGL(sum_f32_kernel, dim3(tiles * (rb + eb)), dim3(256), 0, st, a, a.dQ, rb, tiles, FastDiv(tiles));
         }
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
     if (phases & PH_BWD_DKDUDV) {
-        const dim3 grid((unsigned)((d.E * nbe_of(d) + 1) / 2), (unsigned)d.Hkuv, (unsigned)a.nslice);
+        dim3 grid((unsigned)((d.E * nbe_of(d) + 1) / 2), (unsigned)d.Hkuv, (unsigned)a.nslice);
+        a.heads_first = a.nslice == 1 && grid.x <= 65535;
+        if (a.heads_first) std::swap(grid.x, grid.y);
         // on the fp32 instructions: d_h > 96, and one step of d_h <= 32 (7.8 of 8.2 us; of d_h 33 to 96 5 % more, two steps 8 to 20 %)
         constexpr bool EVER = CT == 1 || CT > 3, ALWAYS = CT > 3;
         const bool plain = ALWAYS || (EVER && (a.rows.n + 31) / 32 <= 2 * a.nslice);
