@@ -35,8 +35,8 @@ struct GateArgs {
     float* part;         // [H][workgroups of a head][DH * E + DH] sums of d_router, d_norm_weight over a workgroup's tokens
     int B, H, S, E, tpw, dq_tokmaj, wn_bf16, wr_bf16;
     float eps;
-    int wgs;                   // backward: workgroups of a head and batch
-    FastDiv by_h;
+    int wgs, heads_first;      // backward: workgroups of a head and batch; the head runs fastest over the workgroups
+    FastDiv by_fast;           // heads if heads_first, else wgs
 };
 
 __device__ __forceinline__ float param(const void* p, long i, int bf16)
@@ -120,6 +120,11 @@ struct RowTile {
     __device__ static int chunk(int i, int lane) { return (i * 64 + lane) % CH ^ swz(row(i, lane)); }
     __device__ static int half(int ks, int l32, int g) { return l32 * (2 * DH) + (((2 * ks + g) ^ swz(l32)) << 4); }
 };
+
+// Whole rows leave past the caches, room in which they would take from the rows that are being read: 32,768 tokens of 16 heads of 128 forward
+// 59.4 -> 50, backward 103.5 -> 98 us, 8,192 of 8 heads forward 9.7 -> 7.7.  Not so R, whose blocks begin and end inside a line (the same
+// calls 53, 16,384 of 8 heads 16.0 instead of 14.8), nor x on its way in (61).
+__device__ __forceinline__ void store_past(bf16_t* to, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(to)); }
 
 // Everything the forward computes for one tile, shared by both kernels.
 template <int DH, int NT, bool NORM>
@@ -208,8 +213,9 @@ constexpr size_t gate_fwd_smem(int DH, int NT) { return (size_t)2 * NT * (DH / 1
 
 // With WholeRows the rows move between memory and the wave as whole rows, by way of its LDS; else each lane loads and stores its half row,
 // in 32-byte pieces of 32 rows per instruction.  Pieces keep the path from L2 busy four times as long: 32,768 tokens of 16 heads of
-// 128 take 71.5 us with them and 62.8 with whole rows (5.0 TB/s, what a large copy reaches; loads alone in pieces 65.3), 16,384 of
-// 8 heads 18.3 and 16.9.  Few tokens wait for one tile's chain, which the way through LDS makes longer: 512 of 8 heads 6.0 and 6.3.
+// 128 take 71.5 us with them and 62.8 with whole rows (loads alone in pieces 65.3), 16,384 of
+// 8 heads 18.3 and 16.9; with those past the caches (store_past) 59 -> 50 (6.3 TB/s) and 16.3 -> 14.8.
+// Few tokens wait for one tile's chain, which the way through LDS makes longer: 512 of 8 heads 6.0 and 6.3.
 template <int DH, int NT, bool NORM, class... Mode>
 __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 {
@@ -259,7 +265,7 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
             for (int i = 0; i < Rows::INS; ++i) {
                 const u32x4 v = *reinterpret_cast<const u32x4*>(xt + i * 1024 + lane * 16);
                 if (Rows::row(i, lane) < nrow)
-                    *reinterpret_cast<u32x4*>(p.Qn + row0 + Rows::row(i, lane) * stride + Rows::chunk(i, lane) * 8) = v;
+                    store_past(p.Qn + row0 + Rows::row(i, lane) * stride + Rows::chunk(i, lane) * 8, v);
             }
         } else if constexpr (NORM) {
             if (valid) {
@@ -294,8 +300,8 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 // time and are added up down the columns (4 values per 64 columns).  What that frees holds the next tile's rows of x, requested
 // behind the contraction, while dR and dQ of a tile are requested at its top and used half a trip later.  One wave per SIMD
 // with all sums in registers, ~2,400 instructions per tile, a quarter of them register moves, took 150 us on 32,768 tokens of
-// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 109 us, and 101
-// with dX stored as whole rows (4.4 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
+// 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 109 us, 101
+// with dX stored as whole rows and 95 with them past the caches (4.7 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
 // More experts (NT = 2) have twice the d_router operands: four waves, one per SIMD, all sums in registers, and the next
 // tile's rows requested before the current tile's arithmetic starts.
 constexpr int GATE_Z_ROW_B = 64;                           // NT = 1: row of the dz tile
@@ -345,21 +351,22 @@ __device__ __forceinline__ bf16x8 z_cols(const unsigned char* tile, int lane, in
     return v;
 }
 
-// With WholeRows dX leaves as whole rows, by way of the y tile, as Q does in the forward.  32,768 tokens of 16 heads of 128 take 104 us this way,
-// 112 in half rows' pieces; with one or two tiles per wave the way through LDS is not hidden (12,288 of 8 heads 35.0 and 34.5).
-// (x and dQ as whole rows, too, take registers: 108 us with a spill, 111 for x alone.)
+// With WholeRows, workgroups of eight waves, dX leaves as whole rows, by way of the y tile, past the caches (store_past) as Q does in the forward.
+// Both kernels, us, whole rows / half rows' pieces: 32,768 tokens of 16 heads of 128 98 / 112 (104 as whole rows through the caches),
+// 16,384 of 8 30.1 / 31.2, 8,192 18.5 / 20.3, 5,000 17.1 / 18.2, 7,001 of 64 12.9 / 13.3, 4,096 of 96 15.5 / 15.6.  Workgroups of four, one tile a wave, wait for the
+// way through LDS: 3,000 of 8 heads of 128 14.7 / 14.0.  (x and dQ as whole rows, too, take registers: 108 us with a spill, 111 for x alone.)
 template <int DH, int NT, bool NORM, class... Mode>
 __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
 {
     constexpr bool WHOLE = sizeof...(Mode) > 0;
-    const int NW = NT == 1 ? (int)blockDim.x / 64 : 4;
+    constexpr int NW = WHOLE ? 8 : 4;
     constexpr int KS = DH / 16, CT = DH / 32, REGION_B = gate_bwd_region<NT>();
     constexpr bool AHEAD = NT > 1;                              // rows requested one tile ahead; d_norm_weight in registers
     constexpr int NHALF = (DH + 63) / 64;
     // NT = 1: wave w sums column tile w % CT of d_router over the TPG token tiles of its group w / CT of the workgroup's
     // waves (waves beyond GROUPS * CT none); NT = 2: a wave sums all of it over its own tiles
     constexpr int TPG = CT == 2 ? 2 : 4, WCT = AHEAD ? CT : 1;
-    const int GROUPS = NW / TPG;
+    constexpr int GROUPS = NW / TPG;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* sA = smem;                                   // logits operands
     unsigned char* sC = sA + 2 * NT * KS * 1024;                // dy operands
@@ -369,9 +376,8 @@ __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_
     unsigned char* regions = reinterpret_cast<unsigned char*>(sW + DH);
     unsigned char* ytile = regions + wave * REGION_B;
     unsigned char* ztile = ytile + TILE_B;
-    // (with WholeRows the grid is workgroups of a head and batch, heads, batches; else the head runs fastest, see launch_gate)
-    const unsigned wg = WHOLE ? blockIdx.x : p.by_h.div(blockIdx.x), wgs = WHOLE ? gridDim.x : p.wgs;
-    const int h = WHOLE ? blockIdx.y : blockIdx.x - wg * p.H, b = WHOLE ? blockIdx.z : blockIdx.y;
+    const unsigned slow = p.by_fast.div(blockIdx.x), fast = blockIdx.x - slow * (p.heads_first ? p.H : p.wgs);
+    const int wg = p.heads_first ? slow : fast, h = p.heads_first ? fast : slow, b = blockIdx.y;
 
     stage_router_rows<DH, NT>(p.Wr, (long)h * DH * p.E, p.wr_bf16, p.E, sA);
     stage_router_cols<DH, NT>(p.Wr, (long)h * DH * p.E, p.wr_bf16, p.E, sC);
@@ -637,7 +643,7 @@ __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_
             for (int i = 0; i < Rows::INS; ++i) {
                 const u32x4 v = *reinterpret_cast<const u32x4*>(ytile + i * 1024 + lane * 16);
                 if (Rows::row(i, lane) < nrow)
-                    *reinterpret_cast<u32x4*>(d0 + (long)Rows::row(i, lane) * (p.H * DH) + Rows::chunk(i, lane) * 8) = v;
+                    store_past(d0 + (long)Rows::row(i, lane) * (p.H * DH) + Rows::chunk(i, lane) * 8, v);
             }
         } else if (valid) {
 #pragma unroll
@@ -649,7 +655,7 @@ __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_
     // and element --------------------------------------------------------------------------------------------------------
     __syncthreads();   // every wave is past its last tile: the per-wave regions are free
     float* mine = reinterpret_cast<float*>(ytile);
-    float* part = p.part ? p.part + (((long)h * (WHOLE ? gridDim.z : gridDim.y) + b) * wgs + wg) * (DH * p.E + DH) : nullptr;
+    float* part = p.part ? p.part + (((long)h * gridDim.y + b) * p.wgs + wg) * (DH * p.E + DH) : nullptr;
     float* dWr = p.dWr + (long)h * DH * p.E;
     auto put = [&](int nt, int idx, float v) {      // value idx of expert tile nt: lane idx % 64, register idx / 64 % 16, column tile
         const int ln = idx & 63, i = (idx >> 6) & 15, ct = idx >> 10;
@@ -658,9 +664,7 @@ __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_
         if (part) part[col * p.E + e] = v;
         else unsafeAtomicAdd(dWr + (long)col * p.E + e, v);
     };
-    auto leave = [&](auto nw) {      // (for either number of waves: the loops over them are unrolled)
-        constexpr int NW = decltype(nw)::value;
-        [[maybe_unused]] constexpr int GROUPS = NW / TPG;
+    {
         if constexpr (!AHEAD) {
             if constexpr (GROUPS == 1) {      // (a wave's sums are those of the workgroup)
                 if (wave < CT)
@@ -737,9 +741,7 @@ __global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_
                 else unsafeAtomicAdd(p.dWn + h * DH + threadIdx.x, v);
             }
         }
-    };
-    if (NT == 1 && NW == 8) leave(std::integral_constant<int, 8>{});
-    else leave(std::integral_constant<int, 4>{});
+    }
 }
 
 // Adds the workgroups' sums of a head (in order) and writes d_router and d_norm_weight in the parameters' types.  The head runs fastest over
@@ -801,24 +803,25 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
         const int most = (int)gate_bwd_smem<NT>(DH, gate_bwd_max_waves<NT>()), waves = gate_bwd_waves(d);
         const dim3 grid = gate_bwd_grid(d, a.tpw);      // (workgroups of a head and batch, heads, batches)
         a.wgs = grid.x;
-        a.by_h = FastDiv(a.H);
-        const bool whole = NT == 1 && a.tpw >= 4;
+        a.heads_first = NT > 1 || a.tpw < 4;
+        a.by_fast = FastDiv(a.heads_first ? a.H : a.wgs);
+        const bool whole = NT == 1 && waves == 8;
         auto* fn = whole ? mhffn_gate_bwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_bwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_bwd[whole], (const void*)fn, most);
         if (e != hipSuccess) return e;
-        // Without whole rows the workgroups of a head run on one XCD, if heads are a multiple of eight: its sums are still in that L2 when the
-        // pass behind reads them, and dQ, dR where the operator left them.  Both kernels, us, before / so: 16 tokens of 16 heads of 128
-        // 13.6 / 12.4, 512 of 8 13.0 / 12.8, 3,000 14.7 / 14.0, 2,000 of 16 16.2 / 15.2, 4,096 of 8 18.0 / 17.3.  The many rows of the other form are
-        // read faster by the workgroups of a head in turn: 32,768 tokens of 16 heads 103.3, in that order 107.2.
-        hipLaunchKernelGGL(fn, whole ? grid : dim3(grid.x * d.H, d.B), dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
+        // Up to three tiles per wave (and with more than 32 experts) the workgroups of a head run on one XCD, if heads are a multiple of eight: its sums are still in that L2 when the
+        // pass behind reads them, and dQ, dR where the operator left them.  Both kernels, us, head by head / so: 16 tokens of 16 heads of 128
+        // 13.6 / 12.4, 512 of 8 13.0 / 12.8, 3,000 14.7 / 14.0, 5,000 17.8 / 17.1, 7,001 of 64 13.6 / 12.9, 16,384 20.2 / 19.8, of 128 30.0 / 30.1.  Of many rows
+        // a head's workgroups in turn read faster: 32,768 tokens of 16 heads 103.3, in that order 107.2.
+        hipLaunchKernelGGL(fn, dim3(grid.x * d.H, d.B), dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
     } else {
         const size_t smem = gate_fwd_smem(DH, NT);
-        // whole rows from six tiles per compute unit on (us in pieces / whole: 1,024 tiles of 8 heads of 128 7.5 / 7.8, 1,536 9.6 / 9.2, 2,048
-        // 11.4 / 10.3; of 96 6.5 / 6.7, 8.6 / 8.4 with 2,048; of 64 6.5 / 6.4 with 2,048)
+        // whole rows from four tiles per compute unit on (us in pieces / whole: 752 tiles of 8 heads of 128 6.7 / 7.2, 1,256 8.7 / 7.4, 2,000 of 16 9.9 / 8.1;
+        // 1,024 of 8 heads of 96 6.4 / 6.2)
         // Not with more than 32 experts, whose arithmetic hides the pieces (4,096 tiles of 4 heads of 64 with 40 16.3 / 17.4, of 8 of 128 25.2 / 26.0),
         // nor with 32 or, below d_h 128, 16: their rows of R share LDS banks, and the way through LDS waits for their writes (16,384 tiles of
         // 12 heads of 128 with 32 + 9 %, of 96 + 9 %; 12,288 of 96 with 16 35.3 / 36.0).
-        const bool whole = NT == 1 && (a.E % 16 != 0 || (DH == 128 && a.E == 16)) && (long)a.B * a.H * ((a.S + 31) / 32) >= 6 * CUS;
+        const bool whole = NT == 1 && (a.E % 16 != 0 || (DH == 128 && a.E == 16)) && (long)a.B * a.H * ((a.S + 31) / 32) >= 4 * CUS;
         auto* fn = whole ? mhffn_gate_fwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_fwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_fwd[whole], (const void*)fn, (int)smem);
         if (e != hipSuccess) return e;
