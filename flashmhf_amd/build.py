@@ -140,7 +140,7 @@ EXPECTED_KERNELS = (
 # whole rows and the dK/dU/dV kernels with two waves a block are told by the mode, a type, that their names end in, and are not counted
 # among the instantiations above.)
 MODES = ("WholeRows", "TokenHalves")
-VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 3), ("mhffn_fwd_rows32_long_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
+VARIANT_KERNELS = (("mhffn_fwd_rows128_kernel", 3), ("mhffn_fwd_rows32_kernel", 6), ("mhffn_fwd_rows32_long_kernel", 3), ("mhffn_bwd_dqdr_rows32_kernel", 3),
                    ("fwd_f32_kernelILi", 4), ("dqdr_f32_kernelILi", 4), ("dkdudv_f32_kernelILi", 2), ("dkdudv_split_kernelILi", 3),
                    ("fwd_fp32_kernelILi", 4), ("dqdr_fp32_kernelILi", 4),
                    ("WholeRows", 12), ("TokenHalves", 6),

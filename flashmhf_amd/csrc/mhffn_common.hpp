@@ -142,8 +142,8 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 v4bf16_t;
 
 // One wave-instruction of an asynchronous tile fill: 4 rows (ins*4 .. ins*4+3) of a row-major [32][DH] bf16 source
-// tile whose row `r` starts at src_row0 + r * row_stride (elements).  Counts as one vmcnt event.
-template <int DH>
+// tile whose row `r` starts at src_row0 + r * row_stride (elements).  Counts as one vmcnt event.  PAST: the caches need not keep the rows.
+template <int DH, bool PAST = false>
 __device__ __forceinline__ void tile_fill_ins(const bf16_t* src_row0, long row_stride, unsigned char* lds_tile, int ins,
                                               int lane)
 {
@@ -151,7 +151,7 @@ __device__ __forceinline__ void tile_fill_ins(const bf16_t* src_row0, long row_s
     int c = (lane & 15) ^ swz16(r);
     c = c < DH / 8 ? c : 0;   // chunk positions a narrow row does not use receive a dummy chunk
     __builtin_amdgcn_global_load_lds((gptr_t)(src_row0 + r * row_stride + c * 8), (lptr_t)(lds_tile + ins * 1024), 16, 0,
-                                     0);
+                                     PAST ? 2 : 0);      // (the instruction's nt bit)
 }
 
 // A operand (32 rows x 16 k) for k-step ks from a swizzled tile, row-major use: lane holds row `row`, columns
@@ -327,11 +327,11 @@ __device__ __forceinline__ void store_rows_f32(unsigned char* region, float* dst
 constexpr int QUAD = 4;                      // waves of a workgroup of the forward = blocks of a trip
 
 // Asynchronous fill of one 32-row tile by one wave: eight vmcnt events.
-template <int DH>
+template <int DH, bool PAST>
 __device__ __forceinline__ void quad_fill(const bf16_t* src, unsigned char* tile, int lane)
 {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) tile_fill_ins<DH>(src, DH, tile, i, lane);
+    for (int i = 0; i < 8; ++i) tile_fill_ins<DH, PAST>(src, DH, tile, i, lane);
 }
 // Asynchronous fills of a block's K, U and V tiles by four waves, each a quarter of every tile: two vmcnt events a tile.  A lane's
 // place in a tile is a 32-bit offset to a uniform base (a narrow row's unused chunks take chunk 0).  The tiles go round in KU sets

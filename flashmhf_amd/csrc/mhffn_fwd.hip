@@ -413,11 +413,14 @@ __global__ __launch_bounds__(512) void mhffn_fwd_rows128_kernel(FwdArgs p) { fwd
 // 32 rows, four blocks a trip: the same products, element-wise formula and order of sums as fwd_body.  One barrier a trip: P^T
 // operands and V tiles (which all waves read) have two sets, K and U tiles (which only their wave reads) are refilled as
 // soon as the first products have read them.  A trip is 1.43 us, bound by the issue of a lone wave and LDS; with the tiles loaded
-// to registers and written to LDS it was 2.15 (0.58 us of it the writes, 0.45 waiting for the loads).
+// to registers and written to LDS it was 2.15 (0.58 us of it the writes, 0.45 waiting for the loads).  With StreamedWeights the tiles are
+// read past the caches (fwd_streams).
+struct StreamedWeights {};
 constexpr int FWD32_V0 = QUAD * 2 * TILE_B, FWD32_P0 = FWD32_V0 + 2 * QUAD * TILE_B, FWD32_R0 = FWD32_P0 + 2 * QUAD * 2048;
-template <int DH>
+template <int DH, class... Mode>
 __global__ __launch_bounds__(256) void mhffn_fwd_rows32_kernel(FwdArgs p)
 {
+    constexpr bool PAST = sizeof...(Mode) > 0;
     constexpr int KS = DH / 16, CT = DH / 32;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     float* sR = reinterpret_cast<float*>(smem + FWD32_R0);                       // [E][32]
@@ -434,10 +437,10 @@ __global__ __launch_bounds__(256) void mhffn_fwd_rows32_kernel(FwdArgs p)
     unsigned char* own = smem + wave * 2 * TILE_B;      // K | U of this wave's block
     auto row_of = [&](int t) { return tok0 + t < p.rows.n ? tok0 + t : p.rows.n - 1; };
     auto block = [&](int b0) { return Kh + (long)(b0 + wave < nblk ? b0 + wave : nblk - 1) * JB * DH; };
-    auto fill_v = [&](int b0, int set) { quad_fill<DH>(block(b0) + offV, smem + FWD32_V0 + (set * QUAD + wave) * TILE_B, lane); };
+    auto fill_v = [&](int b0, int set) { quad_fill<DH, PAST>(block(b0) + offV, smem + FWD32_V0 + (set * QUAD + wave) * TILE_B, lane); };
     auto fill_ku = [&](int b0) {
-        quad_fill<DH>(block(b0), own, lane);
-        quad_fill<DH>(block(b0) + offU, own + TILE_B, lane);
+        quad_fill<DH, PAST>(block(b0), own, lane);
+        quad_fill<DH, PAST>(block(b0) + offU, own + TILE_B, lane);
     };
 
     bf16x8 q[KS];
@@ -771,6 +774,14 @@ Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
     return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes, SUMS);
 }
 
+// Weights that the eight L2 caches do not hold together are read past them by the trips of the 32-row kernel: each is read by one workgroup
+// or a few at about the same time, and keeping it only pushes out what comes next.  Forward with its sums, us, kept / past, other weights each call:
+// one token of 16 heads of 128 with 95 MB of weights 21.3 / 19.7, with 48 MB 13.6 / 13.0, of 8 heads with 48 MB 14.2 / 13.3, of 64 with 48 MB
+// 14.1 / 12.8, of 96 with 38 MB 13.1 / 12.2; 48 tokens of these 24.6 / 24.0, 16.3 / 15.8, 16.0 / 15.7, 18.1 / 17.4, 14.4 / 13.7.  Below, the caches do
+// help: 28 MB (16 tokens) 11.9 / 12.0, 24 MB (one token) 9.8 / 10.3, 21 MB 9.9 / 10.3.
+constexpr size_t L2_B = (size_t)XCDS * 4 << 20;
+static bool fwd_streams(const Dims& d) { return (size_t)3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(bf16_t) > L2_B; }
+
 template <int DH>
 static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, hipStream_t st)
 {
@@ -780,18 +791,19 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, h
                      : tile_rows == 32 ? FWD32_R0 + gates * 32 * (int)sizeof(float)
                                      : FWD_RING_B + gates * 256 * (int)sizeof(float);
     if (smem > 160 * 1024) return hipErrorInvalidValue;
-    static LdsOptIn optin, optin128, optin32, optinl;
+    auto* rows32 = fwd_streams(d) ? mhffn_fwd_rows32_kernel<DH, StreamedWeights> : mhffn_fwd_rows32_kernel<DH>;
+    static LdsOptIn optin, optin128, optin32[2], optinl;
     const hipError_t e = pipeline           ? ensure_dynamic_lds(optinl, (const void*)mhffn_fwd_rows32_long_kernel<DH>, smem)
                          : tile_rows == 256 ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
                          : tile_rows == 128 ? ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem)
-                                            : ensure_dynamic_lds(optin32, (const void*)mhffn_fwd_rows32_kernel<DH>, smem);
+                                            : ensure_dynamic_lds(optin32[fwd_streams(d)], (const void*)rows32, smem);
     if (e != hipSuccess) return e;
     const unsigned tiles = (unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv);
     dim3 grid(whole_xcds(tiles, a.parts.nsplit), (unsigned)a.parts.nsplit);
     if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
     else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(512), smem, st, a);
     else if (pipeline) hipLaunchKernelGGL((mhffn_fwd_rows32_long_kernel<DH>), grid, dim3(FWDL_W * 64), smem, st, a);
-    else hipLaunchKernelGGL((mhffn_fwd_rows32_kernel<DH>), grid, dim3(256), smem, st, a);
+    else hipLaunchKernelGGL(rows32, grid, dim3(256), smem, st, a);
     if (a.parts.nsplit > 1) {
         static_assert(32 * (DH / 4) % 256 == 0, "a workgroup's rows are of one tile");
         dim3 sgrid(grid.x, (unsigned)(((a.rows.n < tile_rows ? a.rows.n : tile_rows) * (DH / 4) + 255) / 256));
