@@ -1239,18 +1239,19 @@ static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d
 // Tiles of 256 rows where they fill the chip, of 32 below that: a block of theirs takes a quarter of the time, with an eighth of
 // the rows.  One part of 121 blocks of the 370M heads, 512 rows: 199 us with 256 rows, 48 with 32; 2,048 rows: 200 and (two
 // rounds) 108.  At their best numbers of parts 512 rows take 34.5 us with 32 rows, 36.1 with 256, 733 rows 49.7 and 45.0.  The prices lose
-// 0.5 % on average and 12 % at worst over 166 calls (d_h 64, 96, 128; fourteen layers; 48 to 6,000 tokens; profiles/pick_parts_sweep.csv: the kernel and
-// a summing pass of its own; in the backward that of 41 of them goes along with another); those from before the sums ran where their parts are 1.0 and 20 %.
+// 0.7 % on average and 10 % at worst over 160 training calls drawn from layers of 4 to 16 heads and 128 to 16,384 tokens (the whole backward with tile
+// heights and numbers of parts around the pick; profiles/pick_parts_sweep.csv).  Steps of 1.9 and 0.36 with sums at 0.5 us per MB lose 0.6 %, but make parts of more sums
+// (4 x 471 tokens of 8 heads of 96 with 9 blocks 45.4 -> 48.7 us) and with them workspaces larger (2 x 2,568 of 8 of 128 with 90 blocks none -> 67.5 MB).
 // Where dK, dU, dV have slices to add up, the parts go along in that launch: whole backward of 2 x 300 tokens of 8 heads of 96 on
 // two 61.7 us with a pass of their own in the price (32 rows, one part), 58.6 without (256 rows, eight parts); 900 of 8 of 128 on four 117.0, 114.6.
 // (With no room behind the slices, too, where the pass is there: the choice does not cost more than 1 % then, over 30 calls.)
 // Tiles of 256 rows that are half empty are no choice, whatever the prices of a part of one block say: 64 rows of 6 heads of 64 with 25 blocks
 // 12.1 us in 25 parts, 8.8 in 5 of 32-row tiles; 50 of 4 heads of 128 with 24 blocks 12.5, 10.5; 128 of 2 heads of 128 with 9 blocks 13.2, 8.9.
-constexpr Variant DQ_VARIANTS[] = {{256, 1.9, 0.08, 1, 0, 129}, {32, 0.36, 0.17, 1, DQ32_A + 1}};
+constexpr Variant DQ_VARIANTS[] = {{256, 1.7, 0.15, 1, 0, 129}, {32, 0.36, 0.15, 1, DQ32_A + 1}};
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
-    const Sums sums{dw_slices_bf16(d, ws_bytes) > 1 ? 0 : SUMS.pass, SUMS.mb, SUMS.mb_apart};
-    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes, sums);
+    return pick_parts(DQ_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, dq_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes,
+                      dw_slices_bf16(d, ws_bytes) > 1 ? 0 : 2);
 }
 
 static size_t dw_slice_bytes(const Dims& d, int nslice) { return align256((size_t)nslice * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float)); }

@@ -640,13 +640,15 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 // One part needs no partial sums and is what runs where the row tiles alone fill the chip.  With fewer tiles than compute
 // units a part per idle unit shortens the serial walk over the blocks (one token of the 370M layer, 8 tiles of 121 blocks: 46 us
 // in one part, 7.8 in 31), and every part costs a set of fp32 sums that is written and read back.  Time of a launch in us:
-// rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + the prices of the sums, Sums (dQ/dR: no pass
-// where the weights' gradients have one, which adds up both); a step slows by up to `full` as the chip fills
-// (power).  The prices are the same for every d_h: with it the
-// variants of a kernel get cheaper nearly together, and that of the 32-row forward is its trips' for its pipeline, too.  Against every
-// tile height and 1 to 64 parts, measured on 194 bfloat16 calls of the forward (fourteen layers; d_h 64, 96, 128; 1 to 6,000 tokens;
-// profiles/pick_parts_sweep.csv) the pick is 1.5 % slower than the fastest on average and 18 % at worst; with the prices from before
-// the sums ran where their parts are (2 us and 0.6 us per MB) 2.4 and 36 %.  dQ/dR: at its variants.
+// rounds of CUS workgroups x (blocks of a part x step + 3 for prologue and epilogue), + 2 for the summing pass (dQ/dR: none where
+// the weights' gradients have one, which adds up both) + 0.6 per MB of sums; a step slows by up to `full` as the chip fills
+// (power).  The prices are those of d_h = 128 for every d_h: with it the
+// variants of a kernel get cheaper nearly together, and that of the 32-row forward is its trips' for its pipeline, too.  Against tile heights and numbers of
+// parts around the pick, on 300 bfloat16 calls of the forward drawn from layers of 4 to 16 heads and 1 to 16,384 tokens (profiles/pick_parts_sweep.csv), it is
+// 1.9 % slower than the fastest on average and 21 % at worst.  The prices stay above what sums cost since they are added up where they are (whole_xcds):
+// 1.5 us and 0.5 per MB, with steps fitted to them on other calls, come to 1.6 % there, but six of the 300 calls take 3 to 17 % longer with them than with these
+// (47 tokens of 16 heads of 128 on eight 17.4 / 20.4 us, 8 x 449 of 8 heads of 128 91.9 / 101.2; of 520 rows of 6 heads of 128 with 88 blocks 19.5 / 22.1).
+// dQ/dR: at its variants.
 // Not cut: more experts than one LDS window of gate values holds (bfloat16); and 16,384 rows per head or more, where a head
 // fills a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X
@@ -673,15 +675,12 @@ struct Variant {
 struct Pick {
     int tile_rows, nsplit;
 };
-struct Sums {
-    double pass, mb, mb_apart;        // us: the pass, a MB of sums, and one of those that grids put on several XCDs (whole_xcds)
-};
-constexpr Sums SUMS{1.5, 0.5, 0.55}, SUMS_F32{2.0, 0.6, 0.6};
 template <int N>
-inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, bool may_cut, size_t part_bytes, size_t ws_bytes, const Sums& sums)
+inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, bool may_cut, size_t part_bytes, size_t ws_bytes, double sum_us = 2)
 {
     const long rows = (long)(d.H / d.Hkuv) * d.B * d.S;
     const int most = may_cut && rows < SPLIT_ROWS_BELOW && blocks < (1 << 24) ? (blocks < 64 ? blocks : 64) : 1;
+    const double part_us = part_bytes * 0.6e-6;
     Pick best{variants[0].tile_rows, 1};
     double best_us = 0;
     for (const Variant& v : variants) {
@@ -690,10 +689,9 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
         for (int ns = 1; ns <= most; ++ns) {
             if (ns > 1 && (ns * part_bytes > ws_bytes || tiles * (ns - 1) >= 2 * CUS)) break;
             const long wgs = tiles * ns;
-            const double part_us = part_bytes * 1e-6 * (whole_xcds((unsigned)tiles, ns) % XCDS ? sums.mb_apart : sums.mb);
             const double load = wgs <= CUS / 2 ? 0 : wgs >= CUS ? 1 : (wgs - CUS / 2) / (double)(CUS / 2);
             const double us = (double)((wgs + CUS - 1) / CUS) * ((((blocks + ns - 1) / ns + v.unit - 1) / v.unit + v.ahead) * v.step * (1 + v.full * load) + 3) +
-                              (ns > 1 ? sums.pass + ns * part_us : 0);
+                              (ns > 1 ? sum_us + ns * part_us : 0);
             if (best_us == 0 || us < best_us) { best_us = us; best = Pick{v.tile_rows, ns}; }
         }
     }

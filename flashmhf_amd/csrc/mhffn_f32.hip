@@ -1209,7 +1209,7 @@ size_t o_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * si
 size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 Pick pick_f32(const Dims& d, size_t part_bytes, size_t ws_bytes, int phases)
 {
-    return pick_parts(F32_VARIANTS, d, d.E * nbe_of(d), true, part_bytes, phases & PH_ONE_PART ? 0 : ws_bytes, SUMS_F32);
+    return pick_parts(F32_VARIANTS, d, d.E * nbe_of(d), true, part_bytes, phases & PH_ONE_PART ? 0 : ws_bytes);
 }
 
 F32Args f32_args(const void* Q, const void* K, const void* U, const void* V, const float* R, const Dims& d, int nsplit)

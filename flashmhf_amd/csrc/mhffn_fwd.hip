@@ -759,19 +759,20 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // instead of 1.0 (1,500 tokens of the 370M layer in one part: 130 us with 256 rows, 74 with 128; 733 tokens at each one's best number of
 // parts 32.6 and 29.8, of the 128M layer 25.2 and 20.6), and the two are level where every compute unit has one.  Of 32, four blocks a trip of 1.43 us, below that, where 128-row tiles take, at each one's best
 // number of parts: one token of the 370M layer 7.8 us against 10.0, 16 tokens of the 1.3B layer 20.3 against 22.5 (95 MB of
-// weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.  (The prices are fitted to
-// measured calls, together with the other figures of pick_parts: 128 rows' is above a step's own 0.53 to 0.6.)  Up to 32 rows the larger tiles
-// are no choice: four rows of two heads of 96 with 64 blocks 9.7 us in 128-row tiles, 7.2 in 32-row ones.
+// weights); 400 rows in one part 46 against 82.  Rows have the same sums, bit for bit, in all three.  (Priced at 0.6 for 128 rows, as
+// before its filling waves: the line between the two kernels lies where it did.)  Up to 32 rows the larger tiles are no choice, whatever the prices say of
+// parts of one or two blocks: two tokens of 8 heads of 96 on four with 64 blocks 10.3 us in 64 parts of 128-row tiles, 7.2 in 16 of 32-row ones; one of 4 heads of 64
+// with 42 7.9, 6.6; 40 such calls 15 % on average, the worst, of 16 blocks or fewer, 3 to 6 % the other way (6.1 / 6.5).
 // A part of FWDL_FROM blocks or more goes through the pipeline.  Trips / pipeline, us in one part, 512 rows of 8 heads of 128: 4 blocks 6.1 / 6.6,
 // 12 9.0 / 8.9, 20 11.7 / 11.1, 28 14.5 / 13.3, 32 15.9 / 14.5, 64 27.1 / 23.9; of 96: 16 blocks 9.3 / 9.4, 24 11.6 / 11.4, 32 13.7 / 13.3, 64 23.7 / 22.0;
 // of 64: 16 8.6 / 8.7, 24 10.8 / 10.6, 32 12.9 / 12.7, 64 21.8 / 20.6.  (They meet at 12 to 20 blocks; the line above that is a cautious one, drawn
 // when 16 and 64 were measured.)
 constexpr int FWDL_FROM = 32;
-constexpr Variant FWD_VARIANTS[] = {{256, 1.1, 0.25, 1, 0, 33}, {128, 0.65, 0.3, 1, 0, 33}, {32, 1.4, 0.08, QUAD}};
+constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1, 0, 33}, {128, 0.6, 0.33, 1, 0, 33}, {32, 1.45, 0.05, QUAD}};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
-    return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes, SUMS);
+    return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
 }
 
 // Weights that the eight L2 caches do not hold together are read past them by the trips of the 32-row kernel: each is read by one workgroup

@@ -144,3 +144,27 @@ def test_backward_workspace_holds_both_sums_where_one_launch_adds_them(B, H, S, 
 def test_dqdr_of_few_rows_has_no_half_empty_large_tiles(dh, H, Hk, S, E, de):
     assert _capi.launch_plan(_capi.Dims(1, H, Hk, S, dh, E, de), _capi.DTYPE_BF16).dqdr_tile_rows == 32
     assert _capi.launch_plan(_capi.Dims(1, H, Hk, S, dh, 65, 32), _capi.DTYPE_BF16).dqdr_tile_rows == 256      # (32-row tiles hold the gates of 64 experts)
+
+
+# (B, H, Hk, S, d_h, E, d_e, forward, dQ/dR): calls that lower prices of the sums, fitted to others, made slower (tiles of 128 rows in eight parts
+# 22.1 us, in six 19.5; of 32 rows in nine 20.4, of 128 in 22 17.4; dQ/dR in three 48.7, in one 45.4) or gave a workspace that they do not need
+@pytest.mark.parametrize("B,H,Hk,S,dh,E,de,fwd,dq", [(1, 6, 6, 520, 128, 8, 352, (128, 6), (32, 2)), (47, 16, 8, 1, 128, 22, 352, (128, 22), (32, 10)),
+                                                     (36, 16, 8, 1, 128, 22, 352, (128, 22), (32, 10)), (38, 8, 4, 1, 96, 3, 64, (32, 1), (32, 6)),
+                                                     (4, 8, 8, 471, 96, 1, 288, (128, 1), (32, 1)), (2, 8, 8, 2568, 128, 9, 320, (256, 1), (256, 1)),
+                                                     (4, 8, 8, 2686, 128, 9, 224, (256, 1), (256, 1)), (2, 8, 8, 501, 128, 11, 352, (128, 4), (32, 1))])
+def test_parts_only_where_they_pay(B, H, Hk, S, dh, E, de, fwd, dq):
+    d = _capi.Dims(B, H, Hk, S, dh, E, de)
+    p = _capi.launch_plan(d, _capi.DTYPE_BF16)
+    assert (p.fwd_tile_rows, p.fwd_parts) == fwd and (p.dqdr_tile_rows, p.dqdr_parts) == dq
+    L = _capi.lib()
+    assert L.mhffn_fwd_workspace_bytes(d, 0) == (fwd[1] * B * H * S * dh * 4 if fwd[1] > 1 else 0)
+    if dq[1] == 1:
+        assert L.mhffn_bwd_workspace_bytes(d, 0) == L.mhffn_bwd_workspace_min_bytes(d, 0)
+
+
+# rows of a K/U/V head: up to 32 the forward has no choice but its 32-row tiles, whatever the price of a part of one block
+@pytest.mark.parametrize("dh", [64, 96, 128])
+@pytest.mark.parametrize("B,H,Hk,E,de", [(2, 8, 4, 8, 256), (1, 4, 2, 14, 96), (32, 6, 6, 3, 384), (16, 4, 2, 5, 128), (1, 1, 1, 1, 32)])
+def test_forward_of_few_rows_has_no_large_tiles(dh, B, H, Hk, E, de):
+    assert _capi.launch_plan(_capi.Dims(B, H, Hk, 1, dh, E, de), _capi.DTYPE_BF16).fwd_tile_rows == 32
+    assert _capi.launch_plan(_capi.Dims(B, H, Hk, 1, dh, 65, 32), _capi.DTYPE_BF16).fwd_tile_rows != 32      # (32-row tiles hold the gates of 64 experts)
