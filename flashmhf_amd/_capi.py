@@ -23,7 +23,7 @@ OK = 0
 STATIC_SCRATCH_BYTES = 96 << 20
 
 EXPORTS = (
-    "mhffn_strerror", "mhffn_is_supported", "mhffn_check_dims", "mhffn_launch_plan", "mhffn_fwd_workspace_bytes",
+    "mhffn_strerror", "mhffn_is_supported", "mhffn_check_dims", "mhffn_launch_plan", "mhffn_launch_forms", "mhffn_fwd_workspace_bytes",
     "mhffn_bwd_workspace_bytes", "mhffn_bwd_workspace_min_bytes", "mhffn_fwd", "mhffn_bwd", "mhffn_fwd_phases", "mhffn_bwd_phases",
     "mhffn_fwd_layout", "mhffn_bwd_layout", "mhffn_bwd_static", "mhffn_gate_fwd", "mhffn_gate_bwd",
     "mhffn_gate_fwd_typed", "mhffn_gate_bwd_workspace_bytes", "mhffn_gate_bwd_into", "mhffn_rope_fwd", "mhffn_rope_bwd",
@@ -35,6 +35,7 @@ TOKENS_BHSD, TOKENS_BSHD = 0, 1     # layout of Q, O, dO, dQ
 FWD_MAIN, FWD_ALL = 1, 1
 BWD_DQDR, BWD_DKDUDV, BWD_REDUCE, BWD_ALL = 1, 2, 4, 7
 ONE_PART = 256
+FORM_WEIGHTS_PAST_CACHES, FORM_TOKEN_HALVES, FORM_GATE_FWD_WHOLE_ROWS, FORM_GATE_BWD_WHOLE_ROWS = 1, 2, 4, 8
 
 
 class Dims(ctypes.Structure):
@@ -66,6 +67,7 @@ def lib():
             f.restype = ctypes.c_size_t
             f.argtypes = [dp, ctypes.c_int]
         L.mhffn_launch_plan.argtypes = [dp, ctypes.c_int, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int, ctypes.POINTER(Plan)]
+        L.mhffn_launch_forms.argtypes = [dp, ctypes.c_int, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
         L.mhffn_fwd.argtypes = [vp] * 6 + [vp, ctypes.c_size_t, dp, ctypes.c_int, vp]
         L.mhffn_bwd.argtypes = [vp] * 6 + [vp] * 5 + [ctypes.c_int, vp, ctypes.c_size_t, dp, ctypes.c_int, vp]
         L.mhffn_fwd_phases.argtypes = L.mhffn_fwd.argtypes + [ctypes.c_int]
@@ -128,6 +130,15 @@ def launch_plan(dims, dtype, one_part=False):
                                            lib().mhffn_bwd_workspace_bytes(dims, dtype), ONE_PART if one_part else 0, p),
                    "mhffn_launch_plan")
     return p
+
+
+def launch_forms(dims, dtype, one_part=False):
+    """... and the FORM_* bits of its kernels."""
+    L = lib()
+    forms = L.mhffn_launch_forms(dims, dtype, L.mhffn_fwd_workspace_bytes(dims, dtype), L.mhffn_bwd_workspace_bytes(dims, dtype),
+                                 ONE_PART if one_part else 0)
+    raise_for_code(min(forms, OK), "mhffn_launch_forms")
+    return forms
 
 
 def strerror(code):

@@ -1233,6 +1233,7 @@ static DwPick dw_pick(const Dims& d, size_t ws_bytes)
     return best;
 }
 int dw_slices_bf16(const Dims& d, size_t ws_bytes) { return dw_pick(d, ws_bytes).nslice; }
+bool dw_token_halves(const Dims& d, size_t ws_bytes) { return dw_pick(d, ws_bytes).pair; }
 
 static size_t dq_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * (d.d_h + d.E) * sizeof(float); }
 

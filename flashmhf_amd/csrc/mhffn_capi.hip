@@ -124,6 +124,18 @@ int mhffn_launch_plan(const mhffn_dims* dims, int dtype, size_t fwd_workspace_by
     return MHFFN_OK;
 }
 
+int mhffn_launch_forms(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases)
+{
+    mhffn_plan plan;
+    const int rc = mhffn_launch_plan(dims, dtype, fwd_workspace_bytes, bwd_workspace_bytes, phases, &plan);
+    if (rc != MHFFN_OK || dtype != MHFFN_DTYPE_BF16) return rc;
+    const mhffn::Dims d = to_dims(dims);
+    return (mhffn::fwd_reads_past(d, mhffn::Pick{plan.fwd_tile_rows, plan.fwd_parts}) ? MHFFN_FORM_WEIGHTS_PAST_CACHES : 0) |
+           (mhffn::dw_token_halves(d, bwd_workspace_bytes) ? MHFFN_FORM_TOKEN_HALVES : 0) |
+           (mhffn::gate_fwd_whole_rows(d) ? MHFFN_FORM_GATE_FWD_WHOLE_ROWS : 0) |
+           (mhffn::gate_bwd_whole_rows(d) ? MHFFN_FORM_GATE_BWD_WHOLE_ROWS : 0);
+}
+
 int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,
                      void* workspace, size_t workspace_bytes, const mhffn_dims* dims, int dtype, int token_layout,
                      void* stream, int phases)

@@ -702,6 +702,8 @@ inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, 
 Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases);
 Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases);
 int dw_slices_bf16(const Dims& d, size_t ws_bytes);
+bool dw_token_halves(const Dims& d, size_t ws_bytes);      // two waves for a block of rows
+bool fwd_reads_past(const Dims& d, const Pick& pick);      // the weights, past the caches
 Pick fwd_pick_f32(const Dims& d, size_t ws_bytes, int phases);
 Pick dq_pick_f32(const Dims& d, size_t ws_bytes, int phases);
 int dw_slices_f32(const Dims& d);
@@ -734,6 +736,7 @@ hipError_t launch_bwd_f32(const void* Q, const void* K, const void* U, const voi
 hipError_t launch_gate_fwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, void* Qn, float* R,
                            const Dims& d, hipStream_t st);
 size_t gate_bwd_workspace_bytes(const Dims& d);
+bool gate_fwd_whole_rows(const Dims& d), gate_bwd_whole_rows(const Dims& d);      // whether whole rows move (WholeRows)
 hipError_t launch_gate_bwd(const void* X, const void* Wn, int wn_bf16, float eps, const void* Wr, int wr_bf16, const void* dQ,
                            int dq_tokmaj, const float* dR, void* dX, void* dWn, void* dWr, void* ws, const Dims& d, hipStream_t st);
 

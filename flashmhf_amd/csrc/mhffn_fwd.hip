@@ -414,7 +414,7 @@ __global__ __launch_bounds__(512) void mhffn_fwd_rows128_kernel(FwdArgs p) { fwd
 // operands and V tiles (which all waves read) have two sets, K and U tiles (which only their wave reads) are refilled as
 // soon as the first products have read them.  A trip is 1.43 us, bound by the issue of a lone wave and LDS; with the tiles loaded
 // to registers and written to LDS it was 2.15 (0.58 us of it the writes, 0.45 waiting for the loads).  With StreamedWeights the tiles are
-// read past the caches (fwd_streams).
+// read past the caches (fwd_reads_past).
 struct StreamedWeights {};
 constexpr int FWD32_V0 = QUAD * 2 * TILE_B, FWD32_P0 = FWD32_V0 + 2 * QUAD * TILE_B, FWD32_R0 = FWD32_P0 + 2 * QUAD * 2048;
 template <int DH, class... Mode>
@@ -781,23 +781,28 @@ Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 // 14.1 / 12.8, of 96 with 38 MB 13.1 / 12.2; 48 tokens of these 24.6 / 24.0, 16.3 / 15.8, 16.0 / 15.7, 18.1 / 17.4, 14.4 / 13.7.  Below, the caches do
 // help: 28 MB (16 tokens) 11.9 / 12.0, 24 MB (one token) 9.8 / 10.3, 21 MB 9.9 / 10.3.
 constexpr size_t L2_B = (size_t)XCDS * 4 << 20;
-static bool fwd_streams(const Dims& d) { return (size_t)3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(bf16_t) > L2_B; }
+static bool fwd_pipeline(const Dims& d, const Pick& pick) { return pick.tile_rows == 32 && d.E * (d.d_e / JB) / pick.nsplit >= FWDL_FROM; }
+bool fwd_reads_past(const Dims& d, const Pick& pick)
+{
+    return pick.tile_rows == 32 && !fwd_pipeline(d, pick) && (size_t)3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(bf16_t) > L2_B;
+}
 
 template <int DH>
-static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, int tile_rows, hipStream_t st)
+static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, const Pick& pick, hipStream_t st)
 {
+    const int tile_rows = pick.tile_rows;
     const int gates = d.E < GATE_WIN ? d.E : GATE_WIN;
-    const bool pipeline = tile_rows == 32 && d.E * (d.d_e / JB) / a.parts.nsplit >= FWDL_FROM;
+    const bool pipeline = fwd_pipeline(d, pick), past = fwd_reads_past(d, pick);
     const int smem = pipeline          ? FWDL_SMEM
                      : tile_rows == 32 ? FWD32_R0 + gates * 32 * (int)sizeof(float)
                                      : FWD_RING_B + gates * 256 * (int)sizeof(float);
     if (smem > 160 * 1024) return hipErrorInvalidValue;
-    auto* rows32 = fwd_streams(d) ? mhffn_fwd_rows32_kernel<DH, StreamedWeights> : mhffn_fwd_rows32_kernel<DH>;
+    auto* rows32 = past ? mhffn_fwd_rows32_kernel<DH, StreamedWeights> : mhffn_fwd_rows32_kernel<DH>;
     static LdsOptIn optin, optin128, optin32[2], optinl;
     const hipError_t e = pipeline           ? ensure_dynamic_lds(optinl, (const void*)mhffn_fwd_rows32_long_kernel<DH>, smem)
                          : tile_rows == 256 ? ensure_dynamic_lds(optin, (const void*)mhffn_fwd_kernel<DH>, smem)
                          : tile_rows == 128 ? ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem)
-                                            : ensure_dynamic_lds(optin32[fwd_streams(d)], (const void*)rows32, smem);
+                                            : ensure_dynamic_lds(optin32[past], (const void*)rows32, smem);
     if (e != hipSuccess) return e;
     const unsigned tiles = (unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv);
     dim3 grid(whole_xcds(tiles, a.parts.nsplit), (unsigned)a.parts.nsplit);
@@ -827,9 +832,9 @@ hipError_t launch_fwd_bf16(const void* Q, const void* K, const void* U, const vo
     FwdArgs a{(const bf16_t*)Q, (const bf16_t*)K, (const bf16_t*)U, (const bf16_t*)V,           R,
               (bf16_t*)O,       (float*)ws,       RowMap(d),        Parts(d.E, d.d_e / JB, pick.nsplit), pick.tile_rows};
     switch (d.d_h) {
-        case 64: return launch_fwd_t<64>(a, d, pick.tile_rows, st);
-        case 96: return launch_fwd_t<96>(a, d, pick.tile_rows, st);
-        case 128: return launch_fwd_t<128>(a, d, pick.tile_rows, st);
+        case 64: return launch_fwd_t<64>(a, d, pick, st);
+        case 96: return launch_fwd_t<96>(a, d, pick, st);
+        case 128: return launch_fwd_t<128>(a, d, pick, st);
     }
     return hipErrorInvalidValue;
 }

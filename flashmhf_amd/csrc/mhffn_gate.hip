@@ -795,6 +795,21 @@ dim3 gate_bwd_grid(const Dims& d, int& tpw)
     return dim3(workgroups(tpw), d.H, d.B);
 }
 
+}  // namespace
+
+// whole rows from four tiles per compute unit on (us in pieces / whole: 752 tiles of 8 heads of 128 6.7 / 7.2, 1,256 8.7 / 7.4, 2,000 of 16 9.9 / 8.1;
+// 1,024 of 8 heads of 96 6.4 / 6.2)
+// Not with more than 32 experts, whose arithmetic hides the pieces (4,096 tiles of 4 heads of 64 with 40 16.3 / 17.4, of 8 of 128 25.2 / 26.0),
+// nor with 32 or, below d_h 128, 16: their rows of R share LDS banks, and the way through LDS waits for their writes (16,384 tiles of
+// 12 heads of 128 with 32 + 9 %, of 96 + 9 %; 12,288 of 96 with 16 35.3 / 36.0).
+bool gate_fwd_whole_rows(const Dims& d)
+{
+    return d.E <= 32 && (d.E % 16 != 0 || (d.d_h == 128 && d.E == 16)) && (long)d.B * d.H * ((d.S + 31) / 32) >= 4 * CUS;
+}
+bool gate_bwd_whole_rows(const Dims& d) { return gate_bwd_waves(d) == 8; }
+
+namespace {
+
 template <int DH, int NT, bool NORM>
 hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
 {
@@ -805,7 +820,7 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
         a.wgs = grid.x;
         a.heads_first = NT > 1 || a.tpw < 4;
         a.by_fast = FastDiv(a.heads_first ? a.H : a.wgs);
-        const bool whole = NT == 1 && waves == 8;
+        const bool whole = gate_bwd_whole_rows(d);
         auto* fn = whole ? mhffn_gate_bwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_bwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_bwd[whole], (const void*)fn, most);
         if (e != hipSuccess) return e;
@@ -816,12 +831,7 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
         hipLaunchKernelGGL(fn, dim3(grid.x * d.H, d.B), dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
     } else {
         const size_t smem = gate_fwd_smem(DH, NT);
-        // whole rows from four tiles per compute unit on (us in pieces / whole: 752 tiles of 8 heads of 128 6.7 / 7.2, 1,256 8.7 / 7.4, 2,000 of 16 9.9 / 8.1;
-        // 1,024 of 8 heads of 96 6.4 / 6.2)
-        // Not with more than 32 experts, whose arithmetic hides the pieces (4,096 tiles of 4 heads of 64 with 40 16.3 / 17.4, of 8 of 128 25.2 / 26.0),
-        // nor with 32 or, below d_h 128, 16: their rows of R share LDS banks, and the way through LDS waits for their writes (16,384 tiles of
-        // 12 heads of 128 with 32 + 9 %, of 96 + 9 %; 12,288 of 96 with 16 35.3 / 36.0).
-        const bool whole = NT == 1 && (a.E % 16 != 0 || (DH == 128 && a.E == 16)) && (long)a.B * a.H * ((a.S + 31) / 32) >= 4 * CUS;
+        const bool whole = gate_fwd_whole_rows(d);
         auto* fn = whole ? mhffn_gate_fwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_fwd_kernel<DH, NT, NORM>;
         const hipError_t e = ensure_dynamic_lds(optin_fwd[whole], (const void*)fn, (int)smem);
         if (e != hipSuccess) return e;

@@ -143,6 +143,16 @@ typedef struct mhffn_plan {
 } mhffn_plan;
 int mhffn_launch_plan(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases,
                       mhffn_plan* plan);
+/* ... and in which forms the kernels of that plan run (bits of MHFFN_FORM_*, bfloat16; a negative value is an error): the forward's 32-row
+ * tiles read the weights past the caches; dK/dU/dV has two waves for a block of weight rows, each on half of a slice's tokens; the head
+ * prologue's forward moves whole rows; its backward stores whole rows. */
+enum {
+    MHFFN_FORM_WEIGHTS_PAST_CACHES = 1,
+    MHFFN_FORM_TOKEN_HALVES = 2,
+    MHFFN_FORM_GATE_FWD_WHOLE_ROWS = 4,
+    MHFFN_FORM_GATE_BWD_WHOLE_ROWS = 8
+};
+int mhffn_launch_forms(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases);
 
 /* Token-major variants: Q, O, dO, dQ are [B, S, H, d_h] (MHFFN_TOKENS_BSHD) -- the layout the caller's projections
  * produce and consume -- instead of [B, H, S, d_h] (MHFFN_TOKENS_BHSD, what the calls above use).  K, U, V, R, dR and all

@@ -1,5 +1,5 @@
 """The forward of few rows whose weights are larger than the L2 caches together: the 32-row tiles read them past the caches
-(csrc/mhffn_fwd.hip, fwd_streams).  Weights just above and just below that size, rows around a tile, parts that end in the middle of a trip, grouped heads and every head
+(csrc/mhffn_fwd.hip, fwd_reads_past).  Weights just above and just below that size, rows around a tile, parts that end in the middle of a trip, grouped heads and every head
 width, against the fp64 oracle."""
 import pytest
 import torch
@@ -21,6 +21,7 @@ def test_few_rows(H, Hkuv, S, dh, E, de, past):
     plan = _capi.launch_plan(_capi.Dims(1, H, Hkuv, S, dh, E, de), 0)
     assert plan.fwd_tile_rows == 32 and E * de // 32 // plan.fwd_parts < 32
     assert (3 * Hkuv * E * de * dh * 2 > L2) == past
+    assert bool(_capi.launch_forms(_capi.Dims(1, H, Hkuv, S, dh, E, de), 0) & _capi.FORM_WEIGHTS_PAST_CACHES) == past
     ins = make_inputs(1, H, S, dh, E, de, Hkuv, seed=E, dtype=torch.bfloat16)
     O = mhffn_forward(*(t.to(DEV) for t in ins[:5]))
     torch.cuda.synchronize()

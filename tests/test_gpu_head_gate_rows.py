@@ -15,7 +15,7 @@ def _inputs(B, S, H, dh, E, norm):
     return x, wn, 0.1 * torch.randn(H, dh, E, generator=g, device=DEV), g
 
 
-# 1,536 tiles of 32 tokens over all heads and batches and more move whole rows: last tiles of 1, 31 and 32 rows
+# 1,536 tiles of 32 tokens over all heads and batches (from 1,024 on whole rows move): last tiles of 1, 31 and 32 rows
 @pytest.mark.parametrize("B,S,H,dh,E,norm", [(1, 3041, 16, 128, 22, True), (2, 3071, 8, 96, 8, True), (4, 3072, 4, 64, 32, True),
                                              (1, 3050, 16, 128, 11, False), (1, 3041, 16, 96, 40, True)])
 def test_forward(B, S, H, dh, E, norm):

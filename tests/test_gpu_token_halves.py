@@ -8,8 +8,7 @@ from tests.helpers import assert_bf16_parity, make_inputs
 
 DEV = "cuda:0"
 
-# B, H, S, E, de, Hk, token slices of such workgroups.  (With one slice nothing tells this form from the other by its plan: there the cases have
-# few blocks and six tiles or more.)
+# B, H, S, E, de, Hk, token slices of such workgroups
 CASES = [
     (1, 2, 192, 1, 96, 2, 1),       # six tiles; three blocks: the last workgroup of a head has one
     (1, 3, 223, 1, 32, 3, 1),       # four tiles and three; a ragged end; one block
@@ -25,7 +24,16 @@ CASES = [
 @pytest.mark.parametrize("case", CASES)
 def test_slices(case, dh):
     B, H, S, E, de, Hk, slices = case
-    assert _capi.launch_plan(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_BF16).dkdudv_slices == slices
+    d = _capi.Dims(B, H, Hk, S, dh, E, de)
+    assert _capi.launch_forms(d, _capi.DTYPE_BF16) & _capi.FORM_TOKEN_HALVES
+    assert _capi.launch_plan(d, _capi.DTYPE_BF16).dkdudv_slices == slices
+
+
+# columns that fill the chip, few tiles, and longer steps that cost more than half the partial sums save
+@pytest.mark.parametrize("dh", [64, 96, 128])
+@pytest.mark.parametrize("B,H,S,E,de,Hk", [(8, 8, 2048, 11, 352, 8), (1, 2, 32, 1, 96, 2), (1, 1, 64, 1, 32, 1), (4, 1, 8, 3, 64, 1), (1, 8, 128, 8, 256, 8)])
+def test_the_other_form_runs_elsewhere(B, H, S, E, de, Hk, dh):
+    assert not _capi.launch_forms(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_BF16) & _capi.FORM_TOKEN_HALVES
 
 
 @pytest.mark.gpu

@@ -118,7 +118,24 @@ def test_prologue_backward_has_no_second_round_and_no_idle_half(dh, B, H, S, E, 
     assert need == workgroups * (dh * E + dh) * 4      # (a set of partial sums per workgroup)
 
 
-# (y = x w^T of M x K by N x K, one launch for both gradients): both sides of the lines of that rule where dw alone is the library's
+# (B, H, S, d_h, E, whole rows forward, backward): both sides of 1,024 tiles of 32 tokens, and of the experts that keep to pieces
+@pytest.mark.parametrize("B,H,S,dh,E,fwd,bwd", [(1, 8, 4065, 128, 11, True, True), (1, 8, 4064, 128, 11, False, False), (3, 6, 1985, 96, 8, True, True), (2, 4, 4127, 64, 31, True, True),
+                                                (1, 8, 4095, 128, 16, True, True), (1, 8, 4095, 64, 32, False, True), (1, 16, 3041, 96, 16, False, True), (1, 16, 3041, 96, 40, False, False),
+                                                (3, 3, 3777, 96, 8, True, True), (5, 4, 3300, 64, 8, True, True), (1, 8, 500, 128, 11, False, False), (4, 16, 8192, 128, 22, True, True)])
+def test_prologue_moves_whole_rows_of_many_tokens(B, H, S, dh, E, fwd, bwd):
+    forms = _capi.launch_forms(_capi.Dims(B, H, H, S, dh, E, 32), _capi.DTYPE_BF16)
+    assert bool(forms & _capi.FORM_GATE_FWD_WHOLE_ROWS) is fwd and bool(forms & _capi.FORM_GATE_BWD_WHOLE_ROWS) is bwd
+
+
+def test_forms_are_refused_as_plans_are():
+    L, sliced = _capi.lib(), _capi.Dims(2, 8, 2, 300, 96, 8, 256)
+    assert L.mhffn_launch_forms(sliced, 0, 0, 0, 0) == _capi.ERR_WORKSPACE
+    assert L.mhffn_launch_forms(sliced, 0, 0, 1 << 30, 512) == _capi.ERR_SHAPE and L.mhffn_launch_forms(sliced, 7, 0, 0, 0) == _capi.ERR_DTYPE
+    assert L.mhffn_launch_forms(ctypes.POINTER(_capi.Dims)(), 0, 0, 0, 0) == _capi.ERR_NULL_POINTER
+    assert _capi.launch_forms(_capi.Dims(2, 8, 8, 128, 96, 8, 256), _capi.DTYPE_F32) == 0
+
+
+# (y = x w^T of M x K, one launch for both gradients): both sides of the lines of that rule where dw alone is the library's
 @pytest.mark.parametrize("M,N,K,here", [(512, 8192, 1024, True), (2048, 8192, 1024, True), (3000, 8192, 1024, True), (4096, 8192, 1024, False),
                                         (4096, 8192, 768, True), (4096, 16384, 512, True), (4104, 16384, 512, False), (2048, 3072, 2048, False),
                                         (1500, 3072, 2048, True), (512, 8200, 1024, False), (2048, 2048, 2048, True), (8192, 512, 512, True)])
