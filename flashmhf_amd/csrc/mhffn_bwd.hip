@@ -1203,8 +1203,10 @@ constexpr long DW_FIXED_TILES = 9;      // prologue + epilogue of a workgroup, i
 // wave) and with two tiles' worth more at the end.  Whole backward, us, before / with it: 512 tokens of 8 heads of 96 with 8 experts of 256 40.8 / 36.2,
 // 1,000 67.8 / 54.0 (two slices / none), 2,048 95.4 / 92.3, 8,192 282.3 / 284.5 (not taken); 600 of 4 heads of 128 with the same experts 47.5 / 40.6, of
 // 12 with 4 of 128 41.9 / 34.9; 2 x 300 of 8 heads of 96 on two, eight slices / four, 54.3 / 51.6; 128 of 8 of 96 22.6 / 22.8 (not taken).
-// Not in two slices: half the partial sums of the other form's four with the longer steps goes either way (1,500 tokens of 4 heads of 128 70.4 / 67.7,
-// in one slice 68.8; 4,000 of 8 on two 333 / 343; 4,000 of 12 with 4 experts of 128 91.9 / 93.8).
+// In two slices they run instead of one, or of the other form's two or three, but not of its four and more, with which they are level.  The whole backward in two such
+// slices over what the price takes without them, 100 calls drawn from layers of 4 to 16 heads that it would send there: instead of two 0.86 to 0.93 (136 tokens twice of 4 heads
+// of 96 on two with 12 blocks 26.9 / 23.2), of three 0.94 to 0.96, of one 0.90 to 1.00 (409 of 8 of 128 on two with 121 82.6 / 74.0); instead of four or five 0.95 to 1.03,
+// 0.99 on average (2 x 716 of 8 of 96 on four with 64 87.5 / 90.1, 2 x 376 64.7 / 61.9).
 constexpr double DW_PAIR_FIXED_TILES = 10.8, DW_PAIR_STEP = 1.14;
 constexpr long DW_BYTES_PER_TILE_TIME = 2500000;
 struct DwPick {
@@ -1223,7 +1225,7 @@ static DwPick dw_pick(const Dims& d, size_t ws_bytes)
         if (pair && ntile < 2) break;      // (a tile for either half; slices have eight)
         for (long ns = 1; ns <= 64 && (ns == 1 || ns <= ntile / 8); ++ns) {
             if (ns > 1 && align256((size_t)ns * slice_b) > ws_bytes) break;
-            if (pair && ns == 2) continue;
+            if (pair && ns == 2 && !best.pair && best.nslice >= 4) continue;
             const long rounds = (cols * ns + CUS - 1) / CUS, tiles = (ntile + ns - 1) / ns;
             const double cost = rounds * (pair ? (tiles + 1) / 2 * DW_PAIR_STEP + DW_PAIR_FIXED_TILES : tiles + DW_FIXED_TILES) +
                                 (ns > 1 ? ns * (double)slice_b / DW_BYTES_PER_TILE_TIME : 0);

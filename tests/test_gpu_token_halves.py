@@ -16,6 +16,9 @@ CASES = [
     (3, 4, 40, 2, 96, 2, 1),        # 12 tiles of two heads and three sequences
     (1, 8, 1000, 8, 256, 8, 1),     # the other form would take two slices
     (2, 8, 300, 8, 256, 2, 4),      # 80 tiles in slices of 20
+    (3, 4, 170, 3, 96, 4, 2),       # 18 tiles in slices of nine, five of them and four; the last workgroup of a head has one block
+    (2, 3, 288, 5, 96, 3, 2),       # whole tiles, 18 in slices of nine; 15 blocks
+    (2, 4, 136, 1, 384, 2, 2),      # a ragged end, 20 tiles in slices of ten
     (3, 6, 210, 3, 96, 3, 5),       # 42 tiles in slices of eight and nine, the latter five tiles and four; nine blocks
 ]
 
