@@ -35,7 +35,7 @@ TOKENS_BHSD, TOKENS_BSHD = 0, 1     # layout of Q, O, dO, dQ
 FWD_MAIN, FWD_ALL = 1, 1
 BWD_DQDR, BWD_DKDUDV, BWD_REDUCE, BWD_ALL = 1, 2, 4, 7
 ONE_PART = 256
-FORM_WEIGHTS_PAST_CACHES, FORM_TOKEN_HALVES, FORM_GATE_FWD_WHOLE_ROWS, FORM_GATE_BWD_WHOLE_ROWS = 1, 2, 4, 8
+FORM_WEIGHTS_PAST_CACHES, FORM_TOKEN_HALVES, FORM_GATE_FWD_WHOLE_ROWS, FORM_GATE_BWD_WHOLE_ROWS, FORM_FWD_PADDED, FORM_DQDR_PADDED = 1, 2, 4, 8, 16, 32
 
 
 class Dims(ctypes.Structure):

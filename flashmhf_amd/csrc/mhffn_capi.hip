@@ -128,12 +128,18 @@ int mhffn_launch_forms(const mhffn_dims* dims, int dtype, size_t fwd_workspace_b
 {
     mhffn_plan plan;
     const int rc = mhffn_launch_plan(dims, dtype, fwd_workspace_bytes, bwd_workspace_bytes, phases, &plan);
-    if (rc != MHFFN_OK || dtype != MHFFN_DTYPE_BF16) return rc;
+    if (rc != MHFFN_OK) return rc;
     const mhffn::Dims d = to_dims(dims);
-    return (mhffn::fwd_reads_past(d, mhffn::Pick{plan.fwd_tile_rows, plan.fwd_parts}) ? MHFFN_FORM_WEIGHTS_PAST_CACHES : 0) |
-           (mhffn::dw_token_halves(d, bwd_workspace_bytes) ? MHFFN_FORM_TOKEN_HALVES : 0) |
-           (mhffn::gate_fwd_whole_rows(d) ? MHFFN_FORM_GATE_FWD_WHOLE_ROWS : 0) |
-           (mhffn::gate_bwd_whole_rows(d) ? MHFFN_FORM_GATE_BWD_WHOLE_ROWS : 0);
+    const mhffn::Pick f{plan.fwd_tile_rows, plan.fwd_parts}, q{plan.dqdr_tile_rows, plan.dqdr_parts};
+    const bool f32 = dtype == MHFFN_DTYPE_F32;
+    auto padded = [&](const mhffn::Pick& p) { return (f32 ? mhffn::grid_of_part_f32(d, p) : mhffn::whole_xcds(d, p, 2)) != mhffn::tiles_of(d, p); };
+    int forms = (padded(f) ? MHFFN_FORM_FWD_PADDED : 0) | (padded(q) ? MHFFN_FORM_DQDR_PADDED : 0);
+    if (f32) return forms;
+    if (mhffn::fwd_reads_past(d, f)) forms |= MHFFN_FORM_WEIGHTS_PAST_CACHES;
+    if (mhffn::dw_token_halves(d, bwd_workspace_bytes)) forms |= MHFFN_FORM_TOKEN_HALVES;
+    if (mhffn::gate_fwd_whole_rows(d)) forms |= MHFFN_FORM_GATE_FWD_WHOLE_ROWS;
+    if (mhffn::gate_bwd_whole_rows(d)) forms |= MHFFN_FORM_GATE_BWD_WHOLE_ROWS;
+    return forms;
 }
 
 int mhffn_fwd_layout(const void* Q, const void* K, const void* U, const void* V, const float* R, void* O,

@@ -652,18 +652,7 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 // Not cut: more experts than one LDS window of gate values holds (bfloat16); and 16,384 rows per head or more, where a head
 // fills a quarter of the chip alone and its results do not depend on how many other heads run beside it.
 constexpr int CUS = 256;                     // compute units of an MI355X
-// Workgroup i of a launch runs on XCD i % 8, and what it writes stays in that XCD's L2 for the next kernel.  A pass that adds up what several
-// workgroups left therefore runs where they did: launches that leave parts are padded (whole_xcds; workgroups with nothing to do return
-// at once), so that the parts of a tile are written on one XCD, and the pass counts its workgroups the same way.  Only time depends on it.
-// 733 tokens of the 128M layer, forward, us: sums by rows on any XCD 19.4, here 16.0; 2,048 33.2, 29.0; 512 of the 370M layer 26.2, 24.1.
 constexpr int XCDS = 8;
-// `workgroups` in each of `parts`, padded to a multiple of XCDS; as they are where that would put more on one XCD than its share of the
-// rounds that the launch takes.
-inline unsigned whole_xcds(unsigned workgroups, unsigned parts)
-{
-    const unsigned most = (workgroups + XCDS - 1) / XCDS * parts, rounds = (unsigned)(((long)workgroups * parts + CUS - 1) / CUS);
-    return parts < 2 || most > rounds * (CUS / XCDS) ? workgroups : (workgroups + XCDS - 1) / XCDS * XCDS;
-}
 constexpr long SPLIT_ROWS_BELOW = 16384;
 struct Variant {
     int tile_rows;
@@ -675,6 +664,35 @@ struct Variant {
 struct Pick {
     int tile_rows, nsplit;
 };
+// Workgroup i of a launch runs on XCD i % 8, and what it writes stays in that XCD's L2 for the next kernel.  A pass that adds up what several
+// workgroups left therefore runs where they did: launches that leave parts are padded (workgroups with nothing to do return
+// at once), so that the parts of a tile are written on one XCD, and the pass counts its workgroups the same way.  Only time depends on it.
+// 733 tokens of the 128M layer, forward, us: sums by rows on any XCD 19.4, here 16.0; 2,048 33.2, 29.0; 512 of the 370M layer 26.2, 24.1.
+// Padding puts more workgroups on some XCDs than an even share, and where those work longer for it than the sums save, the grid stays as it is.  150 forwards and 100 training
+// calls drawn from layers of 4 to 16 heads, us, as it is / padded:
+// * more workgroups than the launch's rounds hold on an XCD: never padded;
+// * tiles of 256 rows of weights above PAD_WEIGHTS (their steps are bound by the tile fills of the XCD's workgroups): 2 x 3,200 rows of 6 heads of 128 with 26 MB 105.8 / 107.7,
+//   4 x 346 tokens of 8 heads of 128 on four, backward, 149.3 / 152.7; below it the sums count for more (8 x 459 of 4 heads of 64 on two with 3 MB 36.7 / 33.6,
+//   8 x 348 of 4 of 96, backward, 53.8 / 49.5; 6 to 9 MB go either way by 1 %);
+// * smaller tiles, which are few where it matters and read all weights once: an XCD reads more of them, a microsecond for every MB.  One to eight tokens of 8 heads of 128 on
+//   two, whose 31 parts would all run on two XCDs, 8.3 / 8.9 to 9.5 / 10.4, 39 of 6 heads of 128 with 26 MB 14.6 / 15.6; with less than PAD_MORE
+//   more (270 of 8 of 96 on two 14.8 / 12.9, one of 6 of 64 on three 7.2 / 6.6) the sums save half a microsecond and more.
+// Padded by this rule, 2 of the 150 forwards and 2 of the 100 training calls are slower than as they are by 1.5 to 3 %; always padded 17 and 7, by up to 10 %.
+constexpr double PAD_WEIGHTS = 6e6, PAD_MORE = 0.6e6;      // bytes
+inline unsigned tiles_of(const Dims& d, const Pick& pick)
+{
+    return (unsigned)(((long)(d.H / d.Hkuv) * d.B * d.S + pick.tile_rows - 1) / pick.tile_rows * d.Hkuv);
+}
+// the workgroups of a part
+inline unsigned whole_xcds(const Dims& d, const Pick& pick, size_t element)
+{
+    const unsigned tiles = tiles_of(d, pick), parts = pick.nsplit, padded = (tiles + XCDS - 1) / XCDS * XCDS;
+    const unsigned most = padded / XCDS * parts, share = (unsigned)(((long)tiles * parts + XCDS - 1) / XCDS);
+    const unsigned rounds = (unsigned)(((long)tiles * parts + CUS - 1) / CUS);
+    const double weights = 3.0 * d.Hkuv * d.E * d.d_e * d.d_h * element;
+    if (parts < 2 || most > rounds * (CUS / XCDS)) return tiles;
+    return (pick.tile_rows == 256 ? weights <= PAD_WEIGHTS : weights / XCDS * (most - share) <= PAD_MORE * share) ? padded : tiles;
+}
 template <int N>
 inline Pick pick_parts(const Variant (&variants)[N], const Dims& d, int blocks, bool may_cut, size_t part_bytes, size_t ws_bytes, double sum_us = 2)
 {
@@ -704,6 +722,7 @@ Pick dq_pick_bf16(const Dims& d, size_t ws_bytes, int phases);
 int dw_slices_bf16(const Dims& d, size_t ws_bytes);
 bool dw_token_halves(const Dims& d, size_t ws_bytes);      // two waves for a block of rows
 bool fwd_reads_past(const Dims& d, const Pick& pick);      // the weights, past the caches
+unsigned grid_of_part_f32(const Dims& d, const Pick& pick);      // workgroups (whole_xcds)
 Pick fwd_pick_f32(const Dims& d, size_t ws_bytes, int phases);
 Pick dq_pick_f32(const Dims& d, size_t ws_bytes, int phases);
 int dw_slices_f32(const Dims& d);

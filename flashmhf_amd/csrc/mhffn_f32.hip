@@ -1222,11 +1222,7 @@ F32Args f32_args(const void* Q, const void* K, const void* U, const void* V, con
     return a;
 }
 
-// Tiles of all heads in the grid of a part, and workgroups of the summing pass for a tile's rows of `width` lanes.
-unsigned tiles_of(const F32Args& a, const Dims& d)
-{
-    return whole_xcds((unsigned)((a.rows.n + F32_ROWS - 1) / F32_ROWS * d.Hkuv), a.parts.nsplit);
-}
+// Workgroups of the summing pass for a tile's rows of `width` lanes.
 unsigned blocks_of_tile(const F32Args& a, int width)
 {
     return (unsigned)(((long)(a.rows.n < F32_ROWS ? a.rows.n : F32_ROWS) * width + 255) / 256);
@@ -1243,7 +1239,7 @@ hipError_t launch_fwd_f32_t(const F32Args& a, const Dims& d, hipStream_t st)
     auto* fn = one_block ? fwd_fp32_kernel<CT> : fwd_f32_kernel<CT, GROUPS>;
     const hipError_t e = ensure_dynamic_lds(optin[one_block], (const void*)fn, smem);
     if (e != hipSuccess) return e;
-    const unsigned tiles = tiles_of(a, d);
+    const unsigned tiles = grid_of_part_f32(d, Pick{F32_ROWS, a.parts.nsplit});
     hipLaunchKernelGGL(fn, dim3(tiles, (unsigned)a.parts.nsplit), dim3(one_block ? 256 : 256 * GROUPS), smem, st, a);
     if (a.parts.nsplit > 1) {
         const unsigned rb = blocks_of_tile(a, d.d_h / 4);
@@ -1263,7 +1259,7 @@ hipError_t launch_bwd_f32_t(F32Args a, const Dims& d, hipStream_t st, int phases
         auto* fn = one_block ? dqdr_fp32_kernel<CT> : dqdr_f32_kernel<CT>;
         err = ensure_dynamic_lds(optin[one_block], (const void*)fn, smem);
         if (err != hipSuccess) return err;
-        const unsigned tiles = tiles_of(a, d);
+        const unsigned tiles = grid_of_part_f32(d, Pick{F32_ROWS, a.parts.nsplit});
         hipLaunchKernelGGL(fn, dim3(tiles, (unsigned)a.parts.nsplit), dim3(256), smem, st, a);
         if (a.parts.nsplit > 1) {
             const unsigned rb = blocks_of_tile(a, d.d_h / 4), eb = blocks_of_tile(a, d.E);
@@ -1316,6 +1312,13 @@ size_t fwd_workspace_bytes_f32(const Dims& d)
 
 // (at least one copy of dK, dU, dV, which the launch needs only where it slices the tokens: what callers of earlier versions
 // reserve)
+// Float32 kernels work longer for a row, so that an XCD's even share counts for more beside the sums: padded up to three tiles an XCD (us, as it is / padded: 268 tokens of the
+// 128M layer on four heads 98.7 / 97.7 with gradients), not above (44 tiles 48.8 / 49.1 forward, 28 153.7 / 156.9 and 60 261.2 / 264.0 with gradients).
+unsigned grid_of_part_f32(const Dims& d, const Pick& pick)
+{
+    return tiles_of(d, pick) <= 3 * XCDS ? whole_xcds(d, pick, sizeof(float)) : tiles_of(d, pick);
+}
+
 size_t bwd_min_workspace_bytes_f32(const Dims& d)
 {
     return (size_t)dw_slices_f32(d) * 3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(float);

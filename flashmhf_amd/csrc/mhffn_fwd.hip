@@ -804,8 +804,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, const Dims& d, const Pick& pick
                          : tile_rows == 128 ? ensure_dynamic_lds(optin128, (const void*)mhffn_fwd_rows128_kernel<DH>, smem)
                                             : ensure_dynamic_lds(optin32[past], (const void*)rows32, smem);
     if (e != hipSuccess) return e;
-    const unsigned tiles = (unsigned)((a.rows.n + tile_rows - 1) / tile_rows * d.Hkuv);
-    dim3 grid(whole_xcds(tiles, a.parts.nsplit), (unsigned)a.parts.nsplit);
+    dim3 grid(whole_xcds(d, pick, sizeof(bf16_t)), (unsigned)pick.nsplit);
     if (tile_rows == 256) hipLaunchKernelGGL((mhffn_fwd_kernel<DH>), grid, dim3(256), smem, st, a);
     else if (tile_rows == 128) hipLaunchKernelGGL((mhffn_fwd_rows128_kernel<DH>), grid, dim3(512), smem, st, a);
     else if (pipeline) hipLaunchKernelGGL((mhffn_fwd_rows32_long_kernel<DH>), grid, dim3(FWDL_W * 64), smem, st, a);

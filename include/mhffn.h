@@ -143,14 +143,17 @@ typedef struct mhffn_plan {
 } mhffn_plan;
 int mhffn_launch_plan(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases,
                       mhffn_plan* plan);
-/* ... and in which forms the kernels of that plan run (bits of MHFFN_FORM_*, bfloat16; a negative value is an error): the forward's 32-row
- * tiles read the weights past the caches; dK/dU/dV has two waves for a block of weight rows, each on half of a slice's tokens; the head
- * prologue's forward moves whole rows; its backward stores whole rows. */
+/* ... and in which forms the kernels of that plan run (bits of MHFFN_FORM_*, float32 the last two; a negative value is an error): the forward's
+ * 32-row tiles read the weights past the caches; dK/dU/dV has two waves for a block of weight rows, each on half of a slice's tokens; the head
+ * prologue's forward moves whole rows; its backward stores whole rows; a part's workgroups of the forward, of dQ/dR, are padded to a multiple of
+ * the chip's eight XCDs. */
 enum {
     MHFFN_FORM_WEIGHTS_PAST_CACHES = 1,
     MHFFN_FORM_TOKEN_HALVES = 2,
     MHFFN_FORM_GATE_FWD_WHOLE_ROWS = 4,
-    MHFFN_FORM_GATE_BWD_WHOLE_ROWS = 8
+    MHFFN_FORM_GATE_BWD_WHOLE_ROWS = 8,
+    MHFFN_FORM_FWD_PADDED = 16,
+    MHFFN_FORM_DQDR_PADDED = 32
 };
 int mhffn_launch_forms(const mhffn_dims* dims, int dtype, size_t fwd_workspace_bytes, size_t bwd_workspace_bytes, int phases);
 

@@ -9,8 +9,8 @@ from tests.helpers import make_inputs
 DEV = "cuda:0"
 
 # B, H, S, dh, E, de, Hk; padded grid, several token slices
-CASES = [((1, 3, 129, 40, 5, 37, 3), True, True), ((2, 10, 150, 72, 3, 64, 5), True, True), ((1, 4, 300, 96, 6, 33, 2), True, True),
-         ((1, 1, 40, 8, 70, 31, 1), False, False), ((1, 8, 32, 64, 10, 224, 8), False, False), ((1, 33, 70, 24, 8, 65, 33), True, False)]
+CASES = [((1, 3, 129, 40, 5, 37, 3), True, True), ((2, 10, 150, 72, 3, 64, 5), False, True), ((1, 4, 300, 96, 6, 33, 2), True, True),
+         ((1, 1, 40, 8, 70, 31, 1), False, False), ((1, 8, 32, 64, 10, 224, 8), False, False), ((1, 33, 70, 24, 8, 65, 33), False, False)]
 
 
 @pytest.mark.parametrize("dims,padded,slices", CASES)
@@ -19,7 +19,8 @@ def test_what_the_cases_cover(dims, padded, slices):
     p = _capi.launch_plan(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_F32)
     tiles, parts = -(-B * S * H // Hk // 128) * Hk, p.fwd_parts
     assert parts > 1 and p.dqdr_parts > 1 and (p.dkdudv_slices > 1) is slices
-    assert (tiles % 8 != 0 and -(-tiles // 8) * parts <= 32 * -(-tiles * parts // 256)) is padded
+    assert bool(_capi.launch_forms(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_F32) & _capi.FORM_FWD_PADDED) is padded
+    assert not padded or (tiles % 8 != 0 and tiles <= 24 and -(-tiles // 8) * parts <= 32 * -(-tiles * parts // 256))
 
 
 @pytest.mark.gpu
