@@ -775,16 +775,17 @@ Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
     return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
 }
 
-// Weights that the eight L2 caches do not hold together are read past them by the trips of the 32-row kernel: each is read by one workgroup
-// or a few at about the same time, and keeping it only pushes out what comes next.  Forward with its sums, us, kept / past, other weights each call:
-// one token of 16 heads of 128 with 95 MB of weights 21.3 / 19.7, with 48 MB 13.6 / 13.0, of 8 heads with 48 MB 14.2 / 13.3, of 64 with 48 MB
-// 14.1 / 12.8, of 96 with 38 MB 13.1 / 12.2; 48 tokens of these 24.6 / 24.0, 16.3 / 15.8, 16.0 / 15.7, 18.1 / 17.4, 14.4 / 13.7.  Below, the caches do
-// help: 28 MB (16 tokens) 11.9 / 12.0, 24 MB (one token) 9.8 / 10.3, 21 MB 9.9 / 10.3.
-constexpr size_t L2_B = (size_t)XCDS * 4 << 20;
+// Large weights are read past the caches by the trips of the 32-row kernel: each is read by one workgroup or a few at about the same time, and keeping it only pushes out
+// what comes next.  Forward with its sums, us, kept / past, twelve sets of weights in turn: one token of 16 heads of 128 with 95 MB 23.1 / 21.3, with 74 MB 19.1 / 17.8,
+// 32 tokens 24.2 / 23.0 and 20.5 / 19.7; the block 40.5 / 38.2 and 36.9 / 35.5 for one token.  Three sets in turn stay in the memory-side cache of 256 MB where they are
+// smaller, and then the caches do help: the block with 48 MB (16 heads of 128 on eight) of 9 tokens 30.0 / 31.4, of 21 30.7 / 33.1, with 53 MB (12 heads of 96) of 16
+// 27.8 / 29.1; twelve such sets 34.7 / 33.4, 36.8 / 35.5, 31.4 / 30.8.  The line lies where neither way loses: with 74 MB three sets in turn 33.4 / 33.7 to 36.9 / 35.7,
+// with 95 MB 39.7 / 36.7.
+constexpr size_t PAST_FROM_B = (size_t)64 << 20;
 static bool fwd_pipeline(const Dims& d, const Pick& pick) { return pick.tile_rows == 32 && d.E * (d.d_e / JB) / pick.nsplit >= FWDL_FROM; }
 bool fwd_reads_past(const Dims& d, const Pick& pick)
 {
-    return pick.tile_rows == 32 && !fwd_pipeline(d, pick) && (size_t)3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(bf16_t) > L2_B;
+    return pick.tile_rows == 32 && !fwd_pipeline(d, pick) && (size_t)3 * d.Hkuv * d.E * d.d_e * d.d_h * sizeof(bf16_t) > PAST_FROM_B;
 }
 
 template <int DH>
