@@ -307,8 +307,6 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 constexpr int GATE_Z_ROW_B = 64;                           // NT = 1: row of the dz tile
 constexpr int GATE_WAVE_REGION_B = 2 * TILE_B + 1024;      // NT = 2: also a 64 x 65 float transpose
 template <int NT>
-constexpr int gate_bwd_max_waves() { return NT == 1 ? 8 : 4; }
-template <int NT>
 constexpr int gate_bwd_region() { return NT == 1 ? TILE_B + 32 * 32 * 4 : GATE_WAVE_REGION_B; }      // (dR passes through the dz tile as fp32)
 template <int NT>
 constexpr size_t gate_bwd_smem(int DH, int waves)
@@ -356,7 +354,7 @@ __device__ __forceinline__ bf16x8 z_cols(const unsigned char* tile, int lane, in
 // 16,384 of 8 30.1 / 31.2, 8,192 18.5 / 20.3, 5,000 17.1 / 18.2, 7,001 of 64 12.9 / 13.3, 4,096 of 96 15.5 / 15.6.  Workgroups of four, one tile a wave, wait for the
 // way through LDS: 3,000 of 8 heads of 128 14.7 / 14.0.  (x and dQ as whole rows, too, take registers: 108 us with a spill, 111 for x alone.)
 template <int DH, int NT, bool NORM, class... Mode>
-__global__ __launch_bounds__(64 * gate_bwd_max_waves<NT>()) void mhffn_gate_bwd_kernel(GateArgs p)
+__global__ __launch_bounds__(sizeof...(Mode) > 0 ? 512 : 256, NT == 1 ? 2 : 1) void mhffn_gate_bwd_kernel(GateArgs p)      // (two waves per SIMD up to 32 experts)
 {
     constexpr bool WHOLE = sizeof...(Mode) > 0;
     constexpr int NW = WHOLE ? 8 : 4;
@@ -815,20 +813,20 @@ hipError_t launch_gate(GateArgs a, const Dims& d, bool backward, hipStream_t st)
 {
     static LdsOptIn optin_fwd[2], optin_bwd[2];
     if (backward) {
-        const int most = (int)gate_bwd_smem<NT>(DH, gate_bwd_max_waves<NT>()), waves = gate_bwd_waves(d);
+        const int waves = gate_bwd_waves(d), smem = (int)gate_bwd_smem<NT>(DH, waves);
         const dim3 grid = gate_bwd_grid(d, a.tpw);      // (workgroups of a head and batch, heads, batches)
         a.wgs = grid.x;
         a.heads_first = NT > 1 || a.tpw < 4;
         a.by_fast = FastDiv(a.heads_first ? a.H : a.wgs);
         const bool whole = gate_bwd_whole_rows(d);
         auto* fn = whole ? mhffn_gate_bwd_kernel<DH, 1, NORM, WholeRows> : mhffn_gate_bwd_kernel<DH, NT, NORM>;
-        const hipError_t e = ensure_dynamic_lds(optin_bwd[whole], (const void*)fn, most);
+        const hipError_t e = ensure_dynamic_lds(optin_bwd[whole], (const void*)fn, smem);
         if (e != hipSuccess) return e;
         // Up to three tiles per wave (and with more than 32 experts) the workgroups of a head run on one XCD, if heads are a multiple of eight: its sums are still in that L2 when the
         // pass behind reads them, and dQ, dR where the operator left them.  Both kernels, us, head by head / so: 16 tokens of 16 heads of 128
         // 13.6 / 12.4, 512 of 8 13.0 / 12.8, 3,000 14.7 / 14.0, 5,000 17.8 / 17.1, 7,001 of 64 13.6 / 12.9, 16,384 20.2 / 19.8, of 128 30.0 / 30.1.  Of many rows
         // a head's workgroups in turn read faster: 32,768 tokens of 16 heads 103.3, in that order 107.2.
-        hipLaunchKernelGGL(fn, dim3(grid.x * d.H, d.B), dim3(64 * waves), gate_bwd_smem<NT>(DH, waves), st, a);
+        hipLaunchKernelGGL(fn, dim3(grid.x * d.H, d.B), dim3(64 * waves), smem, st, a);
     } else {
         const size_t smem = gate_fwd_smem(DH, NT);
         const bool whole = gate_fwd_whole_rows(d);
