@@ -645,7 +645,7 @@ __device__ __forceinline__ T sum_in_order(T acc, int z0, int z1, Load&& load)
 // (power).  The prices are those of d_h = 128 for every d_h: with it the
 // variants of a kernel get cheaper nearly together, and that of the 32-row forward is its trips' for its pipeline, too.  Against tile heights and numbers of
 // parts around the pick, on 300 bfloat16 calls of the forward drawn from layers of 4 to 16 heads and 1 to 16,384 tokens (profiles/pick_parts_sweep.csv), it is
-// 1.9 % slower than the fastest on average and 21 % at worst.  The prices stay above what sums cost since they are added up where they are (whole_xcds):
+// 1.8 % slower than the fastest on average and 21 % at worst.  The prices stay above what sums cost since they are added up where they are (whole_xcds):
 // 1.5 us and 0.5 per MB, with steps fitted to them on other calls, come to 1.6 % there, but six of the 300 calls take 3 to 17 % longer with them than with these
 // (47 tokens of 16 heads of 128 on eight 17.4 / 20.4 us, 8 x 449 of 8 heads of 128 91.9 / 101.2; of 520 rows of 6 heads of 128 with 88 blocks 19.5 / 22.1).
 // dQ/dR: at its variants.

@@ -769,10 +769,18 @@ __global__ __launch_bounds__(256) void mhffn_fwd_sum_kernel(FwdArgs p)
 // when 16 and 64 were measured.)
 constexpr int FWDL_FROM = 32;
 constexpr Variant FWD_VARIANTS[] = {{256, 1.0, 0.2, 1, 0, 33}, {128, 0.6, 0.33, 1, 0, 33}, {32, 1.45, 0.05, QUAD}};
+// A call in one part has its tile height by a step of 256 rows that is 8 % dearer on a full chip: three rounds of 128-row tiles are faster than two of 256-row ones, and rows have the same
+// sums in both.  120 calls of 16,384 to 65,000 rows per head drawn from layers of 4 to 16 heads, us, 256 rows / 128: 37 of them with one and a half rounds or less of the larger 0.88 to 0.95
+// (20,664 rows of 4 heads of 128 with 121 blocks 292 / 266, 41,160 of 2 of 96 with 64 142 / 125, 21,936 of 3 of 64 with 65 117 / 103); over all of them 3.0 % over the faster one on average with
+// the step above, 0.03 % with this.  Calls that might be cut keep the step above beside their parts (2 x 1,571 tokens of 8 heads of 128 with 140 blocks in two parts of 256-row tiles 106,
+// in one of 128 114).
+constexpr Variant FWD_ONE_PART[] = {{256, 1.0, 0.3, 1, 0, 33}, FWD_VARIANTS[1], FWD_VARIANTS[2]};
 static size_t fwd_part_bytes(const Dims& d) { return (size_t)d.B * d.H * d.S * d.d_h * sizeof(float); }
 Pick fwd_pick_bf16(const Dims& d, size_t ws_bytes, int phases)
 {
-    return pick_parts(FWD_VARIANTS, d, d.E * (d.d_e / JB), d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
+    const int blocks = d.E * (d.d_e / JB);
+    const Pick pick = pick_parts(FWD_VARIANTS, d, blocks, d.E <= GATE_WIN, fwd_part_bytes(d), phases & PH_ONE_PART ? 0 : ws_bytes);
+    return pick.nsplit > 1 ? pick : pick_parts(FWD_ONE_PART, d, blocks, d.E <= GATE_WIN, fwd_part_bytes(d), 0);
 }
 
 // Large weights are read past the caches by the trips of the 32-row kernel: each is read by one workgroup or a few at about the same time, and keeping it only pushes out

@@ -168,7 +168,7 @@ def test_dqdr_of_few_rows_has_no_half_empty_large_tiles(dh, H, Hk, S, E, de):
 @pytest.mark.parametrize("B,H,Hk,S,dh,E,de,fwd,dq", [(1, 6, 6, 520, 128, 8, 352, (128, 6), (32, 2)), (47, 16, 8, 1, 128, 22, 352, (128, 22), (32, 10)),
                                                      (36, 16, 8, 1, 128, 22, 352, (128, 22), (32, 10)), (38, 8, 4, 1, 96, 3, 64, (32, 1), (32, 6)),
                                                      (4, 8, 8, 471, 96, 1, 288, (128, 1), (32, 1)), (2, 8, 8, 2568, 128, 9, 320, (256, 1), (256, 1)),
-                                                     (4, 8, 8, 2686, 128, 9, 224, (256, 1), (256, 1)), (2, 8, 8, 501, 128, 11, 352, (128, 4), (32, 1))])
+                                                     (4, 8, 8, 2686, 128, 9, 224, (128, 1), (256, 1)), (2, 8, 8, 501, 128, 11, 352, (128, 4), (32, 1))])
 def test_parts_only_where_they_pay(B, H, Hk, S, dh, E, de, fwd, dq):
     d = _capi.Dims(B, H, Hk, S, dh, E, de)
     p = _capi.launch_plan(d, _capi.DTYPE_BF16)
@@ -177,6 +177,14 @@ def test_parts_only_where_they_pay(B, H, Hk, S, dh, E, de, fwd, dq):
     assert L.mhffn_fwd_workspace_bytes(d, 0) == (fwd[1] * B * H * S * dh * 4 if fwd[1] > 1 else 0)
     if dq[1] == 1:
         assert L.mhffn_bwd_workspace_bytes(d, 0) == L.mhffn_bwd_workspace_min_bytes(d, 0)
+
+
+# (B, H, Hk, S, d_h, E, d_e, rows of a tile) of calls in one part: three rounds of 128-row tiles instead of two of 256, but not four instead of two, nor two instead of one
+@pytest.mark.parametrize("B,H,Hk,S,dh,E,de,rows", [(4, 8, 4, 2064, 128, 11, 352, 128), (1, 6, 3, 15528, 64, 11, 320, 128), (8, 8, 8, 1367, 96, 8, 256, 128), (2, 8, 8, 4796, 96, 8, 256, 128),
+                                                   (8, 8, 8, 2048, 128, 11, 352, 256), (1, 8, 8, 16384, 96, 8, 256, 256), (4, 16, 16, 8192, 128, 22, 352, 256), (1, 8, 8, 8192, 128, 11, 352, 256)])
+def test_forward_in_one_part_has_the_height_with_the_shorter_rounds(B, H, Hk, S, dh, E, de, rows):
+    p = _capi.launch_plan(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_BF16)
+    assert (p.fwd_tile_rows, p.fwd_parts) == (rows, 1)
 
 
 # rows of a K/U/V head: up to 32 the forward has no choice but its 32-row tiles, whatever the price of a part of one block
