@@ -834,7 +834,7 @@ __global__ __launch_bounds__(256) void mhffn_bwd_dkdudv_kernel(DwArgs p)
         request(std::integral_constant<int, 0>{});
         request(std::integral_constant<int, 1>{});
         // The fill of the stage that came free at the barrier (tile k + 2) is issued behind the first reads: its five
-        // instructions and their address arithmetic pass while those reads are on their way.
+        // instructions (nine with TokenHalves) and their address arithmetic pass while those reads are on their way.
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (TAIL) prepare_tile();     // (the tail instantiation has no registers to spare for the early call)
         nv_next = fire_tile((ST + 2) % DW_NST);

@@ -121,9 +121,10 @@ struct RowTile {
     __device__ static int half(int ks, int l32, int g) { return l32 * (2 * DH) + (((2 * ks + g) ^ swz(l32)) << 4); }
 };
 
-// Whole rows leave past the caches, room in which they would take from the rows that are being read: 32,768 tokens of 16 heads of 128 forward
-// 59.4 -> 50, backward 103.5 -> 98 us, 8,192 of 8 heads forward 9.7 -> 7.7.  Not so R, whose blocks begin and end inside a line (the same
-// calls 53, 16,384 of 8 heads 16.0 instead of 14.8), nor x on its way in (61).
+// Whole rows leave past the caches, room in which they would take from the rows that are being read.  us through them / past, four inputs in turn: 8,192 tokens of 8 heads of 128
+// forward 12.1 / 10.5, backward 22.9 / 21.2, 16,384 18.3 / 17.0 and 36.3 / 33.5, 32,768 of 16 heads 62.4 / 62.2 and 109.6 / 105.7.  Where x is in the memory-side cache already, it
+// stays there: the last on one input again and again 66.6 / 54.3 forward; both passes behind each other 169 / 161.  Not so R, whose blocks begin and end inside a line (16,384 of
+// 8 heads 16.0 instead of 14.8, one input), nor x on its way in (32,768 of 16 61 instead of 50).
 __device__ __forceinline__ void store_past(bf16_t* to, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(to)); }
 
 // Everything the forward computes for one tile, shared by both kernels.
@@ -214,7 +215,7 @@ constexpr size_t gate_fwd_smem(int DH, int NT) { return (size_t)2 * NT * (DH / 1
 // With WholeRows the rows move between memory and the wave as whole rows, by way of its LDS; else each lane loads and stores its half row,
 // in 32-byte pieces of 32 rows per instruction.  Pieces keep the path from L2 busy four times as long: 32,768 tokens of 16 heads of
 // 128 take 71.5 us with them and 62.8 with whole rows (loads alone in pieces 65.3), 16,384 of
-// 8 heads 18.3 and 16.9; with those past the caches (store_past) 59 -> 50 (6.3 TB/s) and 16.3 -> 14.8.
+// 8 heads 18.3 and 16.9 (those past the caches: store_past; 5.1 TB/s for the former, what a large copy reaches).
 // Few tokens wait for one tile's chain, which the way through LDS makes longer: 512 of 8 heads 6.0 and 6.3.
 template <int DH, int NT, bool NORM, class... Mode>
 __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(256) void mhffn_gate_fwd_kernel(GateArgs p)
 // behind the contraction, while dR and dQ of a tile are requested at its top and used half a trip later.  One wave per SIMD
 // with all sums in registers, ~2,400 instructions per tile, a quarter of them register moves, took 150 us on 32,768 tokens of
 // 16 heads of 128 with 22 experts; two waves with the d_router sums in registers and no rows ahead 145; this 109 us, 101
-// with dX stored as whole rows and 95 with them past the caches (4.7 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
+// with dX stored as whole rows; past the caches 105.7 with its sums where it was 109.6, four inputs in turn (4.2 TB/s).  What is left is latency inside a tile (LDS operands, the chains over a row) at two waves per SIMD.
 // More experts (NT = 2) have twice the d_router operands: four waves, one per SIMD, all sums in registers, and the next
 // tile's rows requested before the current tile's arithmetic starts.
 constexpr int GATE_Z_ROW_B = 64;                           // NT = 1: row of the dz tile
@@ -350,7 +351,7 @@ __device__ __forceinline__ bf16x8 z_cols(const unsigned char* tile, int lane, in
 }
 
 // With WholeRows, workgroups of eight waves, dX leaves as whole rows, by way of the y tile, past the caches (store_past) as Q does in the forward.
-// Both kernels, us, whole rows / half rows' pieces: 32,768 tokens of 16 heads of 128 98 / 112 (104 as whole rows through the caches),
+// Both kernels, us, whole rows / half rows' pieces, one input again and again: 32,768 tokens of 16 heads of 128 98 / 112 (104 as whole rows through the caches),
 // 16,384 of 8 30.1 / 31.2, 8,192 18.5 / 20.3, 5,000 17.1 / 18.2, 7,001 of 64 12.9 / 13.3, 4,096 of 96 15.5 / 15.6.  Workgroups of four, one tile a wave, wait for the
 // way through LDS: 3,000 of 8 heads of 128 14.7 / 14.0.  (x and dQ as whole rows, too, take registers: 108 us with a spill, 111 for x alone.)
 template <int DH, int NT, bool NORM, class... Mode>
