@@ -673,12 +673,12 @@ struct Pick {
 // * more workgroups than the launch's rounds hold on an XCD: never padded;
 // * tiles of 256 rows of weights above PAD_WEIGHTS (their steps are bound by the tile fills of the XCD's workgroups): 2 x 3,200 rows of 6 heads of 128 with 26 MB 105.8 / 107.7,
 //   4 x 346 tokens of 8 heads of 128 on four, backward, 149.3 / 152.7; below it the sums count for more (8 x 459 of 4 heads of 64 on two with 3 MB 36.7 / 33.6,
-//   8 x 348 of 4 of 96, backward, 53.8 / 49.5; 6 to 9 MB go either way by 1 %);
+//   8 x 348 of 4 of 96, backward, 53.8 / 49.5; 5 to 9 MB go either way by 2 %: 8 x 171 tokens of 8 heads of 128 on two 193 / 198 forward and backward);
 // * smaller tiles, which are few where it matters and read all weights once: an XCD reads more of them, a microsecond for every MB.  One to eight tokens of 8 heads of 128 on
 //   two, whose 31 parts would all run on two XCDs, 8.3 / 8.9 to 9.5 / 10.4, 39 of 6 heads of 128 with 26 MB 14.6 / 15.6; with less than PAD_MORE
 //   more (270 of 8 of 96 on two 14.8 / 12.9, one of 6 of 64 on three 7.2 / 6.6) the sums save half a microsecond and more.
 // Padded by this rule, 2 of the 150 forwards and 2 of the 100 training calls are slower than as they are by 1.5 to 3 %; always padded 17 and 7, by up to 10 %.
-constexpr double PAD_WEIGHTS = 6e6, PAD_MORE = 0.6e6;      // bytes
+constexpr double PAD_WEIGHTS = 5e6, PAD_MORE = 0.6e6;      // bytes
 inline unsigned tiles_of(const Dims& d, const Pick& pick)
 {
     return (unsigned)(((long)(d.H / d.Hkuv) * d.B * d.S + pick.tile_rows - 1) / pick.tile_rows * d.Hkuv);

@@ -31,7 +31,7 @@ def test_the_cases_cover_padded_grids_and_others():
 # B, H, Hk, S, dh, E, de, padded: both sides of the lines (weights for 256-row tiles; what an XCD reads more for smaller ones)
 @pytest.mark.parametrize("B,H,Hk,S,dh,E,de,fwd,dq", [(8, 8, 2, 1, 128, 11, 352, False, False), (1, 8, 2, 270, 96, 8, 256, True, True), (1, 6, 6, 39, 128, 16, 352, False, False),
                                                      (1, 6, 3, 1, 64, 4, 384, True, False), (2, 6, 6, 1600, 128, 16, 352, False, False), (4, 8, 4, 346, 128, 11, 352, False, False),
-                                                     (8, 4, 2, 459, 64, 13, 256, True, True), (8, 8, 8, 64, 128, 11, 352, False, False), (1, 8, 8, 2048, 128, 11, 352, False, False)])
+                                                     (8, 4, 2, 459, 64, 13, 256, True, True), (8, 8, 8, 64, 128, 11, 352, False, False), (8, 8, 2, 171, 128, 11, 352, False, False), (1, 8, 8, 2048, 128, 11, 352, False, False)])
 def test_grids_are_padded_where_the_sums_save_more(B, H, Hk, S, dh, E, de, fwd, dq):
     forms = _capi.launch_forms(_capi.Dims(B, H, Hk, S, dh, E, de), _capi.DTYPE_BF16)
     assert (bool(forms & _capi.FORM_FWD_PADDED), bool(forms & _capi.FORM_DQDR_PADDED)) == (fwd, dq)
