@@ -52,6 +52,7 @@ __global__ __launch_bounds__(512) void mhffn_bwd_dqdr_kernel(DqArgs p)
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blockIdx.x = tile * Hkuv + kv-head: the head index runs fastest, so each head's weights stay in one XCD's L2
+    arguments_first(p);
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
     if (tile * BT >= p.rows.n) return;                       // (whole_xcds)
     const int tok0 = tile * BT + wave * 32;                  // this wave's rows of the list (RowMap)
@@ -314,6 +315,7 @@ __global__ __launch_bounds__(DQ32_W * 64) void mhffn_bwd_dqdr_rows32_kernel(DqAr
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    arguments_first(p);
     const int tile = p.rows.by_hkuv.div(blockIdx.x), hk = blockIdx.x - tile * p.rows.Hkuv, z = blockIdx.y;
     const int tok0 = tile * 32, nbe = p.parts.nbe, E = p.parts.E, nsplit = p.parts.nsplit;
     if (tok0 >= p.rows.n) return;                            // (whole_xcds)
